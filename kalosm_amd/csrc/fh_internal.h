@@ -49,9 +49,11 @@ struct fh_device {
     size_t part_cap = 0;
     float *ksplit_buf = nullptr; // partial planes of a k-split prefill matmul
     size_t ksplit_cap = 0;
+    void *frag_buf = nullptr;    // weights of a prompt's product in fragment order, at most 512 MB and their scales
+    size_t frag_cap = 0;
     // 64 KB that never moves: partial results of small reductions (argmax)
     void *small_buf = nullptr;
-    // Counts the reallocations of act_buf / part_buf / ksplit_buf.  A captured graph holds their addresses as
+    // Counts the reallocations of act_buf / part_buf / ksplit_buf / frag_buf.  A captured graph holds their addresses as
     // kernel arguments, so whoever keeps a graph records the value at capture and must not replay it after
     // the value has changed.
     uint64_t scratch_gen = 0;

@@ -9,6 +9,7 @@
 // v_mfma_f32_32x32x16_f16 as  w_hi*x_hi + w_lo*x_hi (+ w_hi*x_lo)  with f32 accumulation, so the only
 // deviation from the f32 reference is the summation order and the 2^-22 residues.
 #include "fh_blocks.h"
+#include "fh_qmm_frag.h"
 #include <type_traits>
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -1792,6 +1793,9 @@ fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf
         FH_FAIL(FH_ERR_UNSUPPORTED, "type %u with k = %lld has no matrix-core matmul (it runs through fh_qmatmul)", q->type,
                 (long long)K);
     FH_REQUIRE((m + 127) / 128 <= 65535, "m = %d too large for one launch", m);
+    const int64_t mk = dev->opt_matmul_kernel;
+    if (((uintptr_t)x & 15) == 0 && (mk == 0 ? fh_qmm_frag_pays(q, x_is_bf16, m) : mk == 13 && fh_qmm_frag_supports(q)))
+        return fh_launch_qmm_frag(q, x, x_is_bf16, m, y);
     // planes: xh | xl | rs | (Q4_K: sums of the 32-groups, hi and lo)
     const size_t plane = ((size_t)m * K * 2 + 255) & ~(size_t)255;
     const size_t rs_bytes = ((size_t)m * 4 + 255) & ~(size_t)255;

@@ -1,0 +1,86 @@
+"""GPU parity: the prompt matmul on fragment-ordered operands (csrc/fh_qmm_frag.hip) against a float64 product of the checker's
+dequantised weights.
+
+Bound: the operands are exact up to 2^-22 of each activation and each product is added in f32, k / 16 * 3 additions in a
+chain at most, whose rounding errors (2^-24 each, of either sign) grow with the root of their number: 2e-6 of the result's
+root mean square covers k = 14336 with the cancellation of the offsets (a factor of about two) included.  The largest single
+difference is held to ten times that (ten standard deviations)."""
+import numpy as np
+import pytest
+
+from kalosm_amd import synth
+from kalosm_amd.fusor import QMatrix, Tensor
+
+pytestmark = pytest.mark.gpu
+TYPES = [synth.Q4_0, synth.Q5_0, synth.Q8_0, synth.Q4_K, synth.Q5_K, synth.Q6_K]
+
+
+def product(dev, oracle, ty, m, n, k, act, option, x=None, seed=1):
+    raw = synth.random_weight(ty, n, k, seed=seed + n, sigma=2e-3)
+    x = synth.random_activation(m, k, seed=seed + m) if x is None else x
+    bits = synth.to_bf16_bits(x) if act == "bf16" else None
+    if bits is not None:
+        x = synth.from_bf16_bits(bits)
+    q = QMatrix.from_raw_bytes(dev, (n, k), raw, ty)
+    xt = Tensor.from_slice(dev, x) if bits is None else Tensor.from_slice(dev, bits, dtype="bf16")
+    out = Tensor.filled_bytes(dev, (m, n), 0xFF)  # poisoned: unwritten elements show as NaN
+    dev.set_option("matmul_kernel", option)
+    try:
+        got = xt.q_mat_mul(q, out=out).as_slice().astype(np.float64)
+    finally:
+        dev.set_option("matmul_kernel", 0)
+    w = oracle.dequantize(ty, raw).reshape(n, k).astype(np.float64)
+    return got, x.astype(np.float64) @ w.T
+
+
+@pytest.mark.parametrize("act", ["f32", "bf16"])
+@pytest.mark.parametrize("ty", TYPES, ids=lambda t: synth.TYPE_NAMES[t])
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 256),        # one row, one output
+    (64, 256, 512),     # exactly a tile of the small form
+    (65, 257, 768),     # one past it; three scales of 256
+    (127, 100, 1024),
+    (129, 513, 2048),   # one past 128 activation and 512 weight rows; k split over workgroups
+    (300, 40, 14336),   # long k
+])
+def test_product(dev, oracle, ty, act, m, n, k):
+    got, want = product(dev, oracle, ty, m, n, k, act, 13)
+    rms = np.sqrt(np.mean(want * want))
+    assert np.isfinite(got).all()
+    assert np.sqrt(np.mean((got - want) ** 2)) <= 2e-6 * rms
+    assert np.abs(got - want).max() <= 2e-5 * rms
+
+
+@pytest.mark.parametrize("ty", [synth.Q4_0, synth.Q8_0, synth.Q5_0], ids=lambda t: synth.TYPE_NAMES[t])
+@pytest.mark.parametrize("k", [128, 384, 640])
+def test_odd_multiples_of_128(dev, oracle, ty, k):
+    """Formats with a scale per 32: the last 128 of k are a half round of the loop."""
+    got, want = product(dev, oracle, ty, 70, 130, k, "f32", 13)
+    assert np.sqrt(np.mean((got - want) ** 2)) <= 2e-6 * np.sqrt(np.mean(want * want))
+
+
+@pytest.mark.parametrize("act", ["f32", "bf16"])
+@pytest.mark.parametrize("ty,m,n,k", [(synth.Q4_K, 17, 272, 2048), (synth.Q6_K, 64, 300, 512), (synth.Q4_K, 1025, 512, 512),
+                                      (synth.Q6_K, 513, 512, 512), (synth.Q8_0, 513, 130, 4096), (synth.Q5_K, 129, 512, 1024)])
+def test_default_dispatch(dev, oracle, ty, m, n, k, act):
+    """Sizes at the lines of the dispatch rule, whichever kernel they take."""
+    got, want = product(dev, oracle, ty, m, n, k, act, 0)
+    assert np.sqrt(np.mean((got - want) ** 2)) <= 2e-6 * np.sqrt(np.mean(want * want))
+
+
+@pytest.mark.parametrize("ty", [synth.Q4_K, synth.Q6_K, synth.Q8_0], ids=lambda t: synth.TYPE_NAMES[t])
+def test_rows_are_independent(dev, oracle, ty):
+    """Zeros stay zero, a power of two passes through exactly, and an infinity or a NaN stays in its row."""
+    m, n, k = 80, 96, 1024
+    x = synth.random_activation(m, k, seed=5)
+    base, _ = product(dev, oracle, ty, m, n, k, "f32", 13, x=x.copy(), seed=9)
+    x[3] = 0.0
+    x[4] *= np.float32(2.0 ** 20)
+    x[5, 7] = np.inf
+    x[6, 9] = np.nan
+    got, _ = product(dev, oracle, ty, m, n, k, "f32", 13, x=x, seed=9)
+    assert not got[3].any()
+    assert np.array_equal(got[4], base[4] * 2.0 ** 20)
+    assert not np.isfinite(got[5]).any() and np.isnan(got[6]).all()
+    rest = [r for r in range(m) if r not in (3, 4, 5, 6)]
+    assert np.array_equal(got[rest], base[rest])

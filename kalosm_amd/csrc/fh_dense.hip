@@ -156,6 +156,186 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(FhGemm g) {
     }
 }
 
+// Large products: 256 weight rows x 256 or 128 activation rows per workgroup of eight wavefronts, on v_mfma_f32_32x32x16_bf16.
+// What bounds the 128 x 128 kernel above is what a compute unit gets from its L2 - 32 KB per 64 of k and 128 x 128 outputs, 78 B/ns
+// at the rate of the matrix cores - and that every step waits for the step just requested.  256 x 256 halves the bytes, and
+// the clock, which the matrix cores bring down to 1.7 GHz, becomes the bound: 2048 x 14336 x 4096 in 231 us (1.04 PFLOP/s, 331 us
+// before), 2048 x 4096 x 14336 with 128 rows per tile in 211 us (1.14 PFLOP/s).  Products grouped by expert stay bound by their
+// weights: 32 experts of 4096 x 4096 and 8192 rows 417 us (454 before; reading 1.07 GB takes 230 us).
+// 64 of k (a slab) per barrier; the barrier sits ahead of the slab's last quarter, whose operands are in registers already, so
+// the next slab's first operands are read and the requests of the slab after it go out while that quarter is multiplied.
+// SLABS buffers: two of 64 KB, or three of 48 KB with 128 activation rows (groups of rows, fewer rows).
+template <int TX>
+struct WideTile {
+    static constexpr int TW = 256, WGX = TX == 256 ? 4 : 2, FW = TX == 256 ? 4 : 2, FX = 2; // a wavefront: FW x FX tiles of 32 x 32
+    static constexpr int NLW = TW / 64, NLX = TX / 64, NL = NLW + NLX;                      // requests of a wavefront per slab
+    static constexpr int SLAB = (TW + TX) * 128, SLABS = TX == 256 ? 2 : 3;
+};
+
+template <int TX, int EPI>
+__global__ __launch_bounds__(512) void k_gemm_bf16_wide(FhGemm g) {
+    typedef WideTile<TX> Tile;
+    typedef float f16v __attribute__((ext_vector_type(16)));
+    constexpr int TW = Tile::TW, WGX = Tile::WGX, FW = Tile::FW, FX = Tile::FX, SLAB = Tile::SLAB, SLABS = Tile::SLABS;
+    constexpr bool W_ROWS = EPI == FH_GEMM_SWIGLU || EPI == FH_GEMM_ACT_T; // weight rows along the registers of the result, else along its lanes
+    extern __shared__ __attribute__((aligned(16))) uint8_t wide_smem[];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31;
+    const int ww = wave / WGX, wx = wave % WGX;
+    // The eight dies take runs of tiles.  Without groups: eight weight tiles by all row tiles, weight tiles first; with groups all
+    // weight tiles of a row tile first: a group's rows and weights meet in one die's L2.
+    const int tn = (g.n + TW - 1) / TW, ty = g.tiles ? *g.n_tiles : (g.m + TX - 1) / TX;
+    const int total = tn * ty, per = total >> 3, more = total & 7, die = (int)blockIdx.x & 7, idx = (int)blockIdx.x >> 3;
+    if (idx >= per + (die < more ? 1 : 0)) return;
+    const int lin = idx + die * per + (die < more ? die : more);
+    int row0, m_end, n0;
+    const uint16_t *w = g.w;
+    if (g.tiles) {
+        const FhTile t = g.tiles[lin / tn];
+        n0 = lin % tn * TW;
+        row0 = t.row0;
+        m_end = t.row0 + t.rows;
+        w += (int64_t)t.group * g.w_group;
+    } else {
+        const int grp = lin / (8 * ty), in = lin - grp * 8 * ty, gw = tn - grp * 8 < 8 ? tn - grp * 8 : 8;
+        n0 = (grp * 8 + in % gw) * TW;
+        row0 = in / gw * TX;
+        m_end = g.m;
+    }
+    // LDS-direct loads: a wavefront's request fills eight rows of 128 bytes; lane l supplies row l / 8, position l % 8 (swizzle
+    // as above, on the memory side)
+    const uint16_t *wp[Tile::NLW], *xp[Tile::NLX];
+    const int rl = tid >> 3, piece = ((tid & 7) ^ gemm_sw(rl)) * 8;
+#pragma unroll
+    for (int i = 0; i < Tile::NLW; i++) {
+        const int n = n0 + rl + 64 * i < g.n ? n0 + rl + 64 * i : g.n - 1; // rows past the end repeat the last one, never stored
+        wp[i] = w + (int64_t)n * g.kp + piece;
+    }
+#pragma unroll
+    for (int i = 0; i < Tile::NLX; i++) {
+        int m = row0 + rl + 64 * i < m_end ? row0 + rl + 64 * i : m_end - 1;
+        if (g.gather) m = g.gather[m];
+        xp[i] = (const uint16_t *)g.x + (int64_t)m * g.kp + piece;
+    }
+    const int slabs = g.kp / 64;
+    auto fetch = [&](int s, int at) { // slab s into the buffer at byte `at`; past the end a repeat, so that the counts stay equal
+        const int64_t o = (int64_t)(s < slabs ? s : slabs - 1) * 64;
+        uint8_t *dst = wide_smem + at + wave * 1024;
+#pragma unroll
+        for (int i = 0; i < Tile::NLW; i++)
+            __builtin_amdgcn_global_load_lds((const uint32_t *)(wp[i] + o),
+                                             (__attribute__((address_space(3))) uint32_t *)(dst + i * 8192), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < Tile::NLX; i++)
+            __builtin_amdgcn_global_load_lds((const uint32_t *)(xp[i] + o),
+                                             (__attribute__((address_space(3))) uint32_t *)(dst + (Tile::NLW + i) * 8192), 16, 0, 0);
+    };
+    fh_bf8 fw[2][FW], fx[2][FX];
+    const int sw = gemm_sw(li), rw = (ww * FW * 32 + li) * 128, rx = (TW + wx * FX * 32 + li) * 128; // (tiles start at multiples of 32 rows)
+    auto read = [&](int set, int at, int q) { // quarter q (16 of k) of the slab at byte `at`
+        const uint8_t *b = wide_smem + at + ((2 * q + (lane >> 5)) ^ sw) * 16;
+#pragma unroll
+        for (int a = 0; a < FW; a++) fw[set][a] = *(const fh_bf8 *)(b + rw + a * 4096);
+#pragma unroll
+        for (int c = 0; c < FX; c++) fx[set][c] = *(const fh_bf8 *)(b + rx + c * 4096);
+    };
+    f16v acc[FW][FX];
+#pragma unroll
+    for (int a = 0; a < FW; a++)
+#pragma unroll
+        for (int c = 0; c < FX; c++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[a][c][r] = 0.f;
+    auto mul = [&](int set) {
+#pragma unroll
+        for (int a = 0; a < FW; a++)
+#pragma unroll
+            for (int c = 0; c < FX; c++)
+                acc[a][c] = W_ROWS ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[set][a], fx[set][c], acc[a][c], 0, 0, 0)
+                                   : __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[set][c], fw[set][a], acc[a][c], 0, 0, 0);
+    };
+#pragma unroll
+    for (int i = 0; i < SLABS; i++) fetch(i, i * SLAB);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SLABS - 1) * Tile::NL) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, 0, 0);
+    int cur = 0;
+    for (int s = 0; s < slabs; s++) {
+        const int nxt = cur + SLAB == SLABS * SLAB ? 0 : cur + SLAB;
+        read(1, cur, 1);
+        mul(0);
+        __builtin_amdgcn_sched_barrier(0);
+        read(0, cur, 2);
+        mul(1);
+        __builtin_amdgcn_sched_barrier(0);
+        read(1, cur, 3);
+        mul(0);
+        __builtin_amdgcn_sched_barrier(0);
+        // the last quarter's operands are here: this wavefront is done with the slab's buffer; and slab s + 1 has landed
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((SLABS - 2) * Tile::NL) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        read(0, nxt, 0);
+        fetch(s + SLABS, cur);
+        mul(1);
+        __builtin_amdgcn_sched_barrier(0);
+        cur = nxt;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // no LDS-direct load outlives the workgroup's LDS
+    const int nb = n0 + ww * FW * 32, mb = row0 + wx * FX * 32, h4 = 4 * (lane >> 5);
+#pragma unroll
+    for (int a = 0; a < FW; a++)
+#pragma unroll
+        for (int c = 0; c < FX; c++) {
+            if (EPI == FH_GEMM_SWIGLU) { // rows 0 .. 15 of a tile are gates, 16 .. 31 the same outputs' up rows
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    fh_f4 v;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) v[r] = fh_silu_f(acc[a][c][4 * q + r]) * acc[a][c][8 + 4 * q + r];
+                    gemm_store<FH_GEMM_ACT, uint16_t>(g.y, g.ldy, mb + c * 32 + li, (nb + a * 32) / 2 + 8 * q + h4, v, m_end, g.n / 2);
+                }
+            } else {
+                const int nl = nb + a * 32, ml = mb + c * 32;
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int o = 8 * (r >> 2) + h4 + (r & 3);
+                    const int n = W_ROWS ? nl + o : nl + li, m = W_ROWS ? ml + li : ml + o;
+                    if (n >= g.n || m >= m_end) continue;
+                    const float v = acc[a][c][r];
+                    if (EPI == FH_GEMM_F32) ((float *)g.y)[(int64_t)m * g.ldy + n] = v;
+                    else if (EPI == FH_GEMM_ACT_T) ((uint16_t *)g.y)[(int64_t)n * g.ldy + m] = fh_to<uint16_t>(v);
+                    else if (EPI == FH_GEMM_RELU2) ((uint16_t *)g.y)[(int64_t)m * g.ldy + n] = fh_to<uint16_t>(fmaxf(v, 0.f) * fmaxf(v, 0.f));
+                    else ((uint16_t *)g.y)[(int64_t)m * g.ldy + n] = fh_to<uint16_t>(v);
+                }
+            }
+        }
+}
+
+template <int TX>
+static fh_status gemm_wide(fh_device *dev, int epi, const FhGemm &g) {
+    constexpr int LDS = WideTile<TX>::SLAB * WideTile<TX>::SLABS;
+    const int64_t ty = g.tiles ? g.max_tiles : (g.m + TX - 1) / TX, total = (g.n + 255) / 256 * ty;
+    FH_REQUIRE(total <= 0x7FFFFF00, "product too large for one launch");
+    const dim3 grid((unsigned)((total + 7) / 8 * 8));
+#define WIDE_GO(E_)                                                                           \
+    do {                                                                                      \
+        FH_TRY(fh_kernel_lds(dev, (const void *)k_gemm_bf16_wide<TX, E_>, (size_t)LDS));      \
+        k_gemm_bf16_wide<TX, E_><<<grid, 512, LDS, dev->stream>>>(g);                         \
+    } while (0)
+    switch (epi) {
+    case FH_GEMM_F32: WIDE_GO(FH_GEMM_F32); break;
+    case FH_GEMM_ACT: WIDE_GO(FH_GEMM_ACT); break;
+    case FH_GEMM_ACT_T: WIDE_GO(FH_GEMM_ACT_T); break;
+    case FH_GEMM_RELU2: WIDE_GO(FH_GEMM_RELU2); break;
+    default: WIDE_GO(FH_GEMM_SWIGLU); break;
+    }
+#undef WIDE_GO
+    FH_HIP(hipGetLastError());
+    return FH_OK;
+}
+
 // f32 activations: 64 x 64 outputs per workgroup, 32 of k per step, true f32 products (v_mfma_f32_16x16x4_f32) of the
 // widened weights.
 template <int EPI>
@@ -256,6 +436,16 @@ fh_status fh_gemm(fh_device *dev, int dtype, int epi, const FhGemm &g) {
         FH_GEMM_EPI(FH_K_, grid)
 #undef FH_K_
     } else {
+        const int64_t cus = dev->compute_units, wn = (g.n + 255) / 256;
+        // The wide kernel from three quarters of a workgroup per compute unit on (below, the 128 x 128 and 128 x 64 tiles have more of
+        // them): prompts of 2048 / 1000 / 512 tokens through the four Zovovik layers of width 4096 took 5.9 / 4.3 / 3.2 ms with
+        // this line and 7.2 / 4.7 / 3.4 ms without the kernel.  matmul_kernel = 3: never, 4: always where its row tiles fit.
+        const int64_t opt = dev->opt_matmul_kernel;
+        if (opt != 3) {
+            if (!g.tiles && (opt == 4 || wn * ((g.m + 255) / 256) * 4 >= cus * 3)) return gemm_wide<256>(dev, epi, g);
+            if (g.tiles ? g.tile_rows == 128 && (opt == 4 || wn * g.max_tiles >= cus) : wn * ((g.m + 127) / 128) * 4 >= cus * 3)
+                return gemm_wide<128>(dev, epi, g);
+        }
         const int tn = (g.n + 127) / 128;
         // small row tiles where the large ones would leave compute units without work
         const bool big = g.tiles ? g.tile_rows == 128 : (int64_t)tn * ((g.m + 127) / 128) >= dev->compute_units;

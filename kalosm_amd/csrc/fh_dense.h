@@ -64,6 +64,56 @@ __device__ __forceinline__ fh_f4 fh_mma32(const fh_f8 &a, const fh_f8 &b, fh_f4 
     return c;
 }
 
+// ROWS weight rows of one wavefront, streamed in pieces of 512 (a lane: eight values, 16 bytes) with AHEAD pieces on their way.
+// No request is under a condition - a lane past the end of the rows repeats the last eight values, and a piece past the last one
+// is not requested: with a branch around a request the compiler can no longer count what is younger and waits for everything.
+template <int ROWS, int AHEAD>
+struct FhRowStream {
+    const uint16_t *w[ROWS];
+    uint4 u[AHEAD][ROWS];
+    int kp, pieces, lane8;
+    __device__ __forceinline__ void fetch(int slot, int piece) {
+        const int c = piece * 512 + lane8, at = c < kp ? c : kp - 8;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) u[slot][r] = *(const uint4 *)(w[r] + at);
+    }
+    __device__ __forceinline__ void start(int kp_) {
+        kp = kp_, pieces = (kp + 511) / 512, lane8 = (threadIdx.x & 63) * 8;
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) fetch(i, i < pieces ? i : pieces - 1);
+    }
+    __device__ __forceinline__ void use(int slot, int piece, const float *x, float *acc) const {
+        const int c = piece * 512 + lane8;
+        if (c >= kp) return;
+        const float4 a = *(const float4 *)(x + c), b = *(const float4 *)(x + c + 4);
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            acc[r] = fmaf(fh_bf_lo(u[slot][r].x), a.x, acc[r]);
+            acc[r] = fmaf(fh_bf_hi(u[slot][r].x), a.y, acc[r]);
+            acc[r] = fmaf(fh_bf_lo(u[slot][r].y), a.z, acc[r]);
+            acc[r] = fmaf(fh_bf_hi(u[slot][r].y), a.w, acc[r]);
+            acc[r] = fmaf(fh_bf_lo(u[slot][r].z), b.x, acc[r]);
+            acc[r] = fmaf(fh_bf_hi(u[slot][r].z), b.y, acc[r]);
+            acc[r] = fmaf(fh_bf_lo(u[slot][r].w), b.z, acc[r]);
+            acc[r] = fmaf(fh_bf_hi(u[slot][r].w), b.w, acc[r]);
+        }
+    }
+    // acc[r] += rows . x (x: kp values in the LDS), not yet summed over the lanes
+    __device__ __forceinline__ void run(const float *x, float *acc) {
+        int p = 0;
+        for (; p + AHEAD < pieces; p += AHEAD) {
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) {
+                use(i, p + i, x, acc);
+                fetch(i, p + i + AHEAD < pieces ? p + i + AHEAD : pieces - 1);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++)
+            if (p + i < pieces) use(i, p + i, x, acc);
+    }
+};
+
 // ---------------------------------------------------------------- host launchers
 // Storage of activations between kernels: FH_F32, or FH_BF16_ACT for decoders that serve in bf16.
 enum { FH_BF16_ACT = 2 };

@@ -503,6 +503,10 @@ fh_status fh_rows_to_act(fh_device *dev, int dtype, const float *x, int64_t ldx,
 // ------------------------------------------------------------------------------ decode matvec
 // One wavefront per ROWS weight rows; a lane takes eight consecutive weights (16 bytes) of every 512.  The input is
 // normed once per workgroup into the LDS; f32 products and sums.
+// What bounds the decode products: a plain read of 117 MB takes 19 us on this device, the product 27 us (14336 x 4096) and 22 us
+// (4096 x 14336), 29 and 25 us while the requests were under conditions (which emptied the pipeline every AHEAD pieces).  The rest
+// is the input every workgroup stages: without it the same loops take 5 us less, whether it is requested first, last, behind a
+// barrier, rotated or from copies of its own, with 2 to 16 pieces ahead, and with one workgroup per compute unit.
 struct MvSegs { FhMvSeg s[3]; int tiles[3]; int n; };
 
 template <int ROWS>
@@ -515,36 +519,58 @@ __global__ __launch_bounds__(256) void k_matvec_norm(const float *__restrict__ x
     while (si + 1 < segs.n && tile >= segs.tiles[si]) tile -= segs.tiles[si++];
     const FhMvSeg seg = segs.s[si];
     const int row0 = (tile * 4 + wave) * ROWS;
-    const uint16_t *wr[ROWS];
+    FhRowStream<ROWS, 16 / ROWS < 8 ? 16 / ROWS : 8> rows;
 #pragma unroll
-    for (int r = 0; r < ROWS; r++) wr[r] = seg.w + (int64_t)(row0 + r < seg.n ? row0 + r : seg.n - 1) * kp + lane * 8;
-    // the first weights are requested before the norm
-    uint4 cur[ROWS];
-    const bool in0 = lane * 8 < kp;
+    for (int r = 0; r < ROWS; r++) rows.w[r] = seg.w + (int64_t)(row0 + r < seg.n ? row0 + r : seg.n - 1) * kp;
+    // The input is requested first (it comes out of the L2 while the weights are on their way: requests are waited for in order),
+    // then the first weights, then the input is normed.
+    if (!(k & 3) && k <= 4096) {
+        float4 v[4], w[4];
+        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int r = 0; r < ROWS; r++) cur[r] = in0 ? *(const uint4 *)wr[r] : uint4{0, 0, 0, 0};
-    float ss = 0.f;
-    if ((k & 3) == 0) {
-#pragma unroll 4
-        for (int i = tid * 4; i < kp; i += 1024) {
-            const float4 v = i < k ? *(const float4 *)(x + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-            ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
-            *(float4 *)(xs + i) = v;
+        for (int j = 0; j < 4; j++) {
+            const int i = (tid + 256 * j) * 4, at = i < k ? i : 0;
+            v[j] = *(const float4 *)(x + at);
+            w[j] = nw ? *(const float4 *)(nw + at) : zero;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        rows.start(kp);
+        __builtin_amdgcn_sched_barrier(0);
+        float inv = 1.f;
+        if (nw) {
+            float ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if ((tid + 256 * j) * 4 < k) ss = fmaf(v[j].x, v[j].x, fmaf(v[j].y, v[j].y, fmaf(v[j].z, v[j].z, fmaf(v[j].w, v[j].w, ss))));
+            ss = fh_wave_sum(ss);
+            if (lane == 0) red[wave] = ss;
+            __syncthreads();
+            inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int i = (tid + 256 * j) * 4;
+            if (i >= kp) continue;
+            float4 o = i < k ? v[j] : zero;
+            if (nw && i < k) o = make_float4(o.x * inv * w[j].x, o.y * inv * w[j].y, o.z * inv * w[j].z, o.w * inv * w[j].w);
+            *(float4 *)(xs + i) = o;
         }
     } else {
+        rows.start(kp);
+        float ss = 0.f;
         for (int i = tid; i < kp; i += 256) {
             const float v = i < k ? x[i] : 0.f;
             ss = fmaf(v, v, ss);
             xs[i] = v;
         }
-    }
-    if (nw) {
-        ss = fh_wave_sum(ss);
-        if (lane == 0) red[wave] = ss;
-        __syncthreads();
-        const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
+        if (nw) {
+            ss = fh_wave_sum(ss);
+            if (lane == 0) red[wave] = ss;
+            __syncthreads();
+            const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
 #pragma unroll 4
-        for (int i = tid; i < k; i += 256) xs[i] = xs[i] * inv * nw[i];
+            for (int i = tid; i < k; i += 256) xs[i] = xs[i] * inv * nw[i];
+        }
     }
     __syncthreads();
     if (norm_out && blockIdx.x == 0)
@@ -552,25 +578,7 @@ __global__ __launch_bounds__(256) void k_matvec_norm(const float *__restrict__ x
     float acc[ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; r++) acc[r] = 0.f;
-    for (int c = lane * 8; c < kp; c += 512) {
-        uint4 nxt[ROWS];
-        const bool more = c + 512 < kp;
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) nxt[r] = more ? *(const uint4 *)(wr[r] + (c - lane * 8) + 512) : uint4{0, 0, 0, 0};
-        const float4 a = *(const float4 *)(xs + c), b = *(const float4 *)(xs + c + 4);
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) {
-            acc[r] = fmaf(fh_bf_lo(cur[r].x), a.x, acc[r]);
-            acc[r] = fmaf(fh_bf_hi(cur[r].x), a.y, acc[r]);
-            acc[r] = fmaf(fh_bf_lo(cur[r].y), a.z, acc[r]);
-            acc[r] = fmaf(fh_bf_hi(cur[r].y), a.w, acc[r]);
-            acc[r] = fmaf(fh_bf_lo(cur[r].z), b.x, acc[r]);
-            acc[r] = fmaf(fh_bf_hi(cur[r].z), b.y, acc[r]);
-            acc[r] = fmaf(fh_bf_lo(cur[r].w), b.z, acc[r]);
-            acc[r] = fmaf(fh_bf_hi(cur[r].w), b.w, acc[r]);
-            cur[r] = nxt[r];
-        }
-    }
+    rows.run(xs, acc);
 #pragma unroll
     for (int r = 0; r < ROWS; r++) acc[r] = fh_wave_sum(acc[r]);
     if (lane == 0)
@@ -768,7 +776,10 @@ __device__ __forceinline__ float mv_sum8(const float *red) {
 }
 
 // x' into the LDS, mixed with the token before it where the matrix wants that.
-__device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int k, int kp, float *xs, float *red) {
+// The input is requested ahead of the first weights (`start`): requests are waited for in order, and the input comes out of the
+// L2 while the weights are on their way.
+template <typename F>
+__device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int k, int kp, float *xs, float *red, F start) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int pos = in.state ? *in.pos_dev : 0;
     const float *before = in.state + ((pos - 1) & 1) * k;
@@ -780,14 +791,19 @@ __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int
         float ss = 0.f;
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const int i = (tid + 512 * j) * 4;
-            const bool ok = i < k;
-            x[j] = ok ? *(const float4 *)(in.x + i) : zero;
-            y[j] = ok && in.y ? *(const float4 *)(in.y + i) : zero;
-            w[j] = ok && in.y ? *(const float4 *)(in.w + i) : zero;
-            m[j] = ok && mu ? *(const float4 *)(mu + i) : zero;
-            b[j] = ok && shift ? *(const float4 *)(before + i) : zero;
+            const int i = (tid + 512 * j) * 4, at = i < k ? i : 0; // (past the end: the first values again, dropped below)
+            x[j] = *(const float4 *)(in.x + at);
+            y[j] = in.y ? *(const float4 *)(in.y + at) : zero;
+            w[j] = in.y ? *(const float4 *)(in.w + at) : zero;
+            m[j] = mu ? *(const float4 *)(mu + at) : zero;
+            b[j] = shift ? *(const float4 *)(before + at) : zero;
         }
+        __builtin_amdgcn_sched_barrier(0);
+        start();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            if ((tid + 512 * j) * 4 >= k) x[j] = y[j] = w[j] = m[j] = b[j] = zero;
         float inv = 0.f;
         if (in.y) {
 #pragma unroll
@@ -814,6 +830,26 @@ __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int
         }
         return;
     }
+    if (!in.y && !(k & 3) && !in.x_out && !in.state && !mu && k <= 16384) { // a plain copy
+        float4 v[8];
+        const int n = (k + 2047) / 2048;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = (tid + 512 * j) * 4;
+            v[j] = *(const float4 *)(in.x + (i < k ? i : 0));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        start();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = (tid + 512 * j) * 4;
+            if (j < n && i < kp) *(float4 *)(xs + i) = i < k ? v[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        for (int i = k + tid; i < kp; i += 512) xs[i] = 0.f;
+        return;
+    }
+    start();
     float inv = 0.f;
     if (in.y) {
         float ss = 0.f;
@@ -823,10 +859,6 @@ __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int
         if (lane == 0) red[wave] = ss;
         __syncthreads();
         inv = 1.0f / sqrtf(mv_sum8(red) / (float)k + in.eps);
-    } else if (!(k & 3) && !in.x_out && !in.state && !mu) { // a plain copy
-#pragma unroll 4
-        for (int i = tid * 4; i < kp; i += 2048) *(float4 *)(xs + i) = i < k ? *(const float4 *)(in.x + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-        return;
     }
     for (int i = tid; i < kp; i += 512) {
         float v = 0.f;
@@ -865,55 +897,29 @@ __device__ __forceinline__ void mv_gated(const FhMvAdd &in, int k, int kp, float
 }
 
 template <int ROWS, bool GATED>
-__global__ __launch_bounds__(512) void k_matvec_mix(FhMvAdd in, int k, int kp, MvMixes segs) {
-    constexpr int AHEAD = ROWS == 4 ? 3 : 8 / ROWS;
+__global__ __launch_bounds__(512, 4) void k_matvec_mix(FhMvAdd in, int k, int kp, MvMixes segs) {
+    constexpr int AHEAD = ROWS == 1 ? 8 : 16 / ROWS;
     extern __shared__ __attribute__((aligned(16))) float xs[]; // [kp | groups]
     __shared__ float red[8];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     int tile = blockIdx.x, si = 0;
     while (si + 1 < segs.n && tile >= segs.tiles[si]) tile -= segs.tiles[si++];
     const FhMvMix seg = segs.s[si];
-    const int row0 = (tile * 8 + wave) * ROWS, pieces = (kp + 511) / 512;
-    const uint16_t *wr[ROWS];
+    const int row0 = (tile * 8 + wave) * ROWS;
+    FhRowStream<ROWS, AHEAD> rows;
 #pragma unroll
-    for (int r = 0; r < ROWS; r++) wr[r] = seg.w + (int64_t)(row0 + r < seg.n ? row0 + r : seg.n - 1) * kp + lane * 8;
-    uint4 u[AHEAD][ROWS];
-    auto fetch = [&](int i, uint4 *v) {
-        const bool ok = i * 512 + lane * 8 < kp;
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) v[r] = ok ? *(const uint4 *)(wr[r] + i * 512) : uint4{0, 0, 0, 0};
-    };
-#pragma unroll
-    for (int i = 0; i < AHEAD; i++) fetch(i, u[i]);
-    if (GATED) mv_gated(in, k, kp, xs, xs + kp);
-    else mv_input(in, seg.mu, k, kp, xs, red);
+    for (int r = 0; r < ROWS; r++) rows.w[r] = seg.w + (int64_t)(row0 + r < seg.n ? row0 + r : seg.n - 1) * kp;
+    if (GATED) {
+        rows.start(kp);
+        mv_gated(in, k, kp, xs, xs + kp);
+    } else {
+        mv_input(in, seg.mu, k, kp, xs, red, [&]() { rows.start(kp); });
+    }
     __syncthreads();
     float acc[ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; r++) acc[r] = 0.f;
-    for (int p = 0; p < pieces; p += AHEAD) {
-#pragma unroll
-        for (int i = 0; i < AHEAD; i++) {
-            uint4 cur[ROWS];
-#pragma unroll
-            for (int r = 0; r < ROWS; r++) cur[r] = u[i][r];
-            fetch(p + i + AHEAD, u[i]);
-            const int c = (p + i) * 512 + lane * 8;
-            if (c >= kp) continue;
-            const float4 a = *(const float4 *)(xs + c), b = *(const float4 *)(xs + c + 4);
-#pragma unroll
-            for (int r = 0; r < ROWS; r++) {
-                acc[r] = fmaf(fh_bf_lo(cur[r].x), a.x, acc[r]);
-                acc[r] = fmaf(fh_bf_hi(cur[r].x), a.y, acc[r]);
-                acc[r] = fmaf(fh_bf_lo(cur[r].y), a.z, acc[r]);
-                acc[r] = fmaf(fh_bf_hi(cur[r].y), a.w, acc[r]);
-                acc[r] = fmaf(fh_bf_lo(cur[r].z), b.x, acc[r]);
-                acc[r] = fmaf(fh_bf_hi(cur[r].z), b.y, acc[r]);
-                acc[r] = fmaf(fh_bf_lo(cur[r].w), b.z, acc[r]);
-                acc[r] = fmaf(fh_bf_hi(cur[r].w), b.w, acc[r]);
-            }
-        }
-    }
+    rows.run(xs, acc);
 #pragma unroll
     for (int r = 0; r < ROWS; r++) acc[r] = fh_wave_sum(acc[r]);
     if (lane == 0)

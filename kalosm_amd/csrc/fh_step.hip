@@ -162,22 +162,17 @@ __device__ __forceinline__ void expert_step(const FhStep &st, int b, float *lds)
     for (int i = tid * 4; i < st.kp; i += 1024) *(float4 *)(lds + i) = *(const float4 *)(st.hn + i);
     __syncthreads();
     const uint16_t *w = m.gate_up + (int64_t)*who * m.gu_stride;
-    const uint16_t *row[4];
+    FhRowStream<4, 4> rows;
     const int p0 = tile * 8 + wave * 2;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         const int p = p0 + i < m.ff ? p0 + i : m.ff - 1;
-        row[2 * i] = w + (int64_t)(p / 16 * 32 + p % 16) * st.kp;
-        row[2 * i + 1] = row[2 * i] + (int64_t)16 * st.kp;
+        rows.w[2 * i] = w + (int64_t)(p / 16 * 32 + p % 16) * st.kp;
+        rows.w[2 * i + 1] = rows.w[2 * i] + (int64_t)16 * st.kp;
     }
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int c = lane * 8; c < st.kp; c += 512) {
-        uint4 u[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) u[i] = *(const uint4 *)(row[i] + c);
-#pragma unroll
-        for (int i = 0; i < 4; i++) acc[i] = dot8(u[i], lds + c, acc[i]);
-    }
+    rows.start(st.kp);
+    rows.run(lds, acc);
 #pragma unroll
     for (int i = 0; i < 4; i++) acc[i] = fh_wave_sum(acc[i]);
     if (lane == 0)
@@ -233,20 +228,43 @@ fh_status fh_step_middle(fh_device *dev, int dtype, const FhStep &st, fh_kvcache
 // ------------------------------------------------------------------------------ output launch
 // One wavefront per row of the residual stream, eight rows per workgroup.  A row's weights - of the output projection, of
 // the chosen experts and of the always-on one - are one list of pieces of 512; a table in the LDS says where each
-// piece lies.  The first pieces are requested before the inputs are staged (the recurrent mixers' gate and norm are
-// applied on the way into the LDS), later ones while earlier ones are multiplied.
+// piece lies.  The inputs are requested beside the experts' numbers, so that they are there when the first pieces go out, and
+// reach the LDS (gate and norm of the recurrent mixers applied on the way) while those are on theirs.  No request is under a
+// condition (FhRowStream).
 struct OutPiece { const uint16_t *w; int kp, len, in; };
 enum { FH_OUT_AHEAD = 8 };
 
-__global__ __launch_bounds__(512) void k_step_out(FhStep st, int n_pieces) {
+__global__ __launch_bounds__(512, 4) void k_step_out(FhStep st, int n_pieces) {
     extern __shared__ __attribute__((aligned(16))) float in[]; // [kpo | top * ffp | sffp | norm groups | pieces]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const FhMoe &m = st.moe;
     const int n_e = m.experts ? m.top : 0, n_s = m.sff ? m.sffp : 0, n_in = st.kpo + n_e * m.ffp + n_s;
-    const int n_g = st.kind == FH_MIX_RECURRENT ? (st.rec.norm_groups + 3) / 4 * 4 : 0;
+    const bool recurrent = st.kind == FH_MIX_RECURRENT;
+    const int n_g = recurrent ? (st.rec.norm_groups + 3) / 4 * 4 : 0;
     float *ie = in + st.kpo, *is = ie + n_e * m.ffp, *ginv = in + n_in;
     OutPiece *pt = (OutPiece *)(ginv + n_g);
     const int po = (st.kpo + 511) / 512, pe = (m.ffp + 511) / 512;
+    const int inner = recurrent ? st.rec.heads * st.rec.vdim : st.lat.heads * st.lat.dv;
+    const float *gate = recurrent ? st.proj + st.rec.col_g : st.o;
+    // up to 4096 values of the mixer and 8192 of the experts in registers (more are read when they are staged)
+    constexpr int NO = 8, NE = 4;
+    const bool early = st.kpo <= 512 * NO && n_e * m.ffp <= 2048 * NE;
+    float ov[NO], gv[NO];
+    float4 ev[NE];
+    if (early) {
+#pragma unroll
+        for (int j = 0; j < NO; j++) {
+            const int i = tid + 512 * j, at = i < inner ? i : inner - 1;
+            ov[j] = st.o[at];
+            gv[j] = gate[at];
+        }
+        if (n_e)
+#pragma unroll
+            for (int j = 0; j < NE; j++) {
+                const int i = (tid + 512 * j) * 4;
+                ev[j] = *(const float4 *)(st.act + (i < n_e * m.ffp ? i : 0));
+            }
+    }
     for (int i = tid; i < n_pieces; i += 512) {
         OutPiece p;
         int k;
@@ -262,23 +280,49 @@ __global__ __launch_bounds__(512) void k_step_out(FhStep st, int n_pieces) {
     __syncthreads();
     const int row = (int)blockIdx.x * 8 + wave, r = row < st.width ? row : st.width - 1;
     uint4 u[FH_OUT_AHEAD];
-    auto fetch = [&](int i) -> uint4 {
-        if (i >= n_pieces) return uint4{0, 0, 0, 0};
-        const OutPiece p = pt[i];
-        return lane * 8 < p.len ? *(const uint4 *)(p.w + (int64_t)r * p.kp + lane * 8) : uint4{0, 0, 0, 0};
+    auto fetch = [&](int i) -> uint4 { // (a lane past the end of a short piece repeats its last eight values)
+        const OutPiece p = pt[i < n_pieces ? i : n_pieces - 1];
+        return *(const uint4 *)(p.w + (int64_t)r * p.kp + (lane * 8 < p.len ? lane * 8 : p.len - 8));
     };
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < FH_OUT_AHEAD; i++) u[i] = fetch(i);
-    if (st.kind == FH_MIX_RECURRENT) {
-        const FhRecurrent &rc = st.rec;
-        const float *gate = st.proj + rc.col_g;
-        const int inner = rc.heads * rc.vdim, gl = inner / rc.norm_groups;
+    __builtin_amdgcn_sched_barrier(0);
+    const bool gate_first = recurrent && st.rec.gate_first;
+    if (early) {
+#pragma unroll
+        for (int j = 0; j < NO; j++) {
+            const int i = tid + 512 * j;
+            if (i < st.kpo) in[i] = i < inner ? (gate_first ? ov[j] * fh_silu_f(gv[j]) : ov[j]) : 0.f;
+        }
+    } else {
         for (int i = tid; i < st.kpo; i += 512) {
             float v = i < inner ? st.o[i] : 0.f;
-            if (rc.gate_first && i < inner) v *= fh_silu_f(gate[i]);
+            if (gate_first && i < inner) v *= fh_silu_f(gate[i]);
             in[i] = v;
         }
-        __syncthreads();
+    }
+    auto put = [&](int i, const float4 &v) {
+        const int j = i / m.ffp, c = i % m.ffp;
+        const float w = st.wts[j];
+        *(float4 *)(ie + i) = make_float4(c < m.ff ? w * v.x : 0.f, c + 1 < m.ff ? w * v.y : 0.f, c + 2 < m.ff ? w * v.z : 0.f,
+                                          c + 3 < m.ff ? w * v.w : 0.f);
+    };
+    if (early) {
+#pragma unroll
+        for (int j = 0; j < NE; j++)
+            if ((tid + 512 * j) * 4 < n_e * m.ffp) put((tid + 512 * j) * 4, ev[j]);
+    } else {
+        for (int i = tid * 4; i < n_e * m.ffp; i += 2048) put(i, *(const float4 *)(st.act + i));
+    }
+    for (int i = tid; i < n_s; i += 512) {
+        const int g = i / 16 * 32 + i % 16;
+        is[i] = fh_silu_f(st.s_gu[g]) * st.s_gu[g + 16];
+    }
+    __syncthreads();
+    if (recurrent) {
+        const FhRecurrent &rc = st.rec;
+        const int gl = inner / rc.norm_groups;
         for (int g = wave; g < rc.norm_groups; g += 8) {
             float ss = 0.f;
             for (int i = lane; i < gl; i += 64) ss = fmaf(in[g * gl + i], in[g * gl + i], ss);
@@ -286,37 +330,40 @@ __global__ __launch_bounds__(512) void k_step_out(FhStep st, int n_pieces) {
             if (lane == 0) ginv[g] = 1.0f / sqrtf(ss / (float)gl + rc.eps);
         }
         __syncthreads();
-        for (int i = tid; i < inner; i += 512) {
-            float v = in[i] * ginv[i / gl] * rc.norm[rc.norm_len == inner ? i : i % rc.norm_len];
-            if (!rc.gate_first) v *= fh_silu_f(gate[i]);
-            in[i] = v;
+        if (early) {
+#pragma unroll
+            for (int j = 0; j < NO; j++) {
+                const int i = tid + 512 * j;
+                if (i >= inner) continue;
+                float v = in[i] * ginv[i / gl] * rc.norm[rc.norm_len == inner ? i : i % rc.norm_len];
+                if (!gate_first) v *= fh_silu_f(gv[j]);
+                in[i] = v;
+            }
+        } else {
+            for (int i = tid; i < inner; i += 512) {
+                float v = in[i] * ginv[i / gl] * rc.norm[rc.norm_len == inner ? i : i % rc.norm_len];
+                if (!gate_first) v *= fh_silu_f(gate[i]);
+                in[i] = v;
+            }
         }
-    } else {
-        const int inner = st.lat.heads * st.lat.dv;
-        for (int i = tid; i < st.kpo; i += 512) in[i] = i < inner ? st.o[i] : 0.f;
+        __syncthreads();
     }
-#pragma unroll 4
-    for (int i = tid * 4; i < n_e * m.ffp; i += 2048) {
-        const int j = i / m.ffp, c = i % m.ffp;
-        const float w = st.wts[j];
-        const float4 v = *(const float4 *)(st.act + i);
-        *(float4 *)(ie + i) = make_float4(c < m.ff ? w * v.x : 0.f, c + 1 < m.ff ? w * v.y : 0.f, c + 2 < m.ff ? w * v.z : 0.f,
-                                          c + 3 < m.ff ? w * v.w : 0.f);
-    }
-    for (int i = tid; i < n_s; i += 512) {
-        const int g = i / 16 * 32 + i % 16;
-        is[i] = fh_silu_f(st.s_gu[g]) * st.s_gu[g + 16];
-    }
-    __syncthreads();
     float acc = 0.f;
-    for (int b = 0; b < n_pieces; b += FH_OUT_AHEAD) {
+    auto use = [&](int slot, int i) {
+        const OutPiece &p = pt[i];
+        if (lane * 8 < p.len) acc = dot8(u[slot], in + p.in + lane * 8, acc);
+    };
+    int b = 0;
+    for (; b + FH_OUT_AHEAD < n_pieces; b += FH_OUT_AHEAD) {
 #pragma unroll
         for (int i = 0; i < FH_OUT_AHEAD; i++) {
-            const uint4 w = u[i];
+            use(i, b + i);
             u[i] = fetch(b + i + FH_OUT_AHEAD);
-            if (b + i < n_pieces && lane * 8 < pt[b + i].len) acc = dot8(w, in + pt[b + i].in + lane * 8, acc);
         }
     }
+#pragma unroll
+    for (int i = 0; i < FH_OUT_AHEAD; i++)
+        if (b + i < n_pieces) use(i, b + i);
     acc = fh_wave_sum(acc);
     if (lane == 0 && row < st.width) st.x[row] += acc;
 }

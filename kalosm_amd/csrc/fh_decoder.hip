@@ -165,31 +165,13 @@ fh_status fh_decoder::decode_greedy(uint32_t first_token, int steps, uint32_t *o
 // Sampled decode (models/kalosm-llama/src/model/inference.rs:38-173, forward.rs:346-404): the sampled id stays in
 // device memory and feeds the next step; it also joins the window of previous ids that the repetition penalty
 // looks at (membership only, so the window is a ring).
-__global__ void k_store_sampled(const uint32_t *result, uint32_t *ids, uint32_t *out, int *step, uint32_t *prev,
-                                uint32_t range, int *kv_len) {
-    *kv_len = *kv_len + 1;
-    const uint32_t t = result[0] == FH_SAMPLE_STATUS_SAMPLED ? result[1] : 0xFFFFFFFFu;
-    const uint32_t next = t == 0xFFFFFFFFu ? 0u : t;
-    ids[0] = next;
-    out[*step] = t;
-    *step = *step + 1;
-    if (range) {
-        const uint32_t slot = prev[65];
-        prev[slot] = next;
-        prev[65] = slot + 1 == range ? 0u : slot + 1;
-        if (prev[64] < range) prev[64] = prev[64] + 1;
-    }
-}
-
 fh_status fh_decoder::sampled_step() {
     FH_TRY(layers(1, true));
     FH_TRY(head(0, logits));
     uint32_t *sd = samp_dev;
+    const FhSampleStore store = {ids, out_tok_dev, step_dev, sd, samp_range, len_dev()};
     FH_TRY(fh_sample_token_dev(dev, logits, vocab, &samp_params, sd, sd + 64, 0, (const float *)(sd + 128),
-                               step_dev, (float *)(sd + 66), sd + 68, nullptr, nullptr));
-    k_store_sampled<<<1, 1, 0, dev->stream>>>(sd + 68, ids, out_tok_dev, step_dev, sd, samp_range,
-                                                len_dev());
-    FH_HIP(hipGetLastError());
+                               step_dev, (float *)(sd + 66), sd + 68, nullptr, nullptr, &store));
     return FH_OK;
 }
 

@@ -282,9 +282,19 @@ struct FhStepTail {
     int *kv_len = nullptr;          // KV cache length
 };
 fh_status fh_argmax_step(fh_device *dev, const float *x_dev, int64_t count, uint32_t *id_dev, FhStepTail tail);
+// Bookkeeping of a sampled step (models/kalosm-llama/src/model/inference.rs:38-173, forward.rs:346-404), done by the sampler's
+// last workgroup: the id is the next step's input, joins the output list and the window of previous ids that the repetition
+// penalty looks at (membership only, so the window is a ring: 64 ids, their count, the next slot).
+struct FhSampleStore {
+    uint32_t *ids = nullptr, *out = nullptr;
+    int *step = nullptr;
+    uint32_t *prev = nullptr;
+    uint32_t range = 0;
+    int *kv_len = nullptr;
+};
 // Sampler with every per-step input in device memory (fh_elementwise.hip); fh_sample_token is its host-input form.
 fh_status fh_sample_token_dev(fh_device *dev, const float *logits_dev, int64_t count, const fh_sampler_params *p,
                               const uint32_t *prev_dev, const uint32_t *prev_len_dev, uint32_t n_prev,
                               const float *randoms_dev, const int *step_dev, float *mu_dev, uint32_t *result_dev,
-                              uint32_t *ids_dev, float *values_dev);
+                              uint32_t *ids_dev, float *values_dev, const FhSampleStore *store);
 

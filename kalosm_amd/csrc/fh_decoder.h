@@ -46,6 +46,8 @@ struct fh_decoder {
     virtual fh_status layers(int s, bool dev_pos) = 0;
     // Final norm and output matrix on row `row` of the last portion: out [vocab]; hidden() is the normed row.
     virtual fh_status head(int row, float *out) = 0;
+    // head() of `n` rows: rows[i] of the last portion into place places[i] of `logits`, in order.
+    virtual fh_status heads(const int *rows, const int *places, int n);
     virtual const float *hidden() const = 0;
     // Cache storage for `positions` positions of the sequence; capacity() changes when a captured step no longer fits it.
     virtual fh_status reserve(int positions) = 0;

@@ -47,6 +47,11 @@ fh_status fh_decoder::reset() {
     return set_len(0, true);
 }
 
+fh_status fh_decoder::heads(const int *rows, const int *places, int n) {
+    for (int i = 0; i < n; i++) FH_TRY(head(rows[i], logits + (size_t)places[i] * vocab));
+    return FH_OK;
+}
+
 fh_status fh_decoder::forward(const uint32_t *tokens, int count, const int32_t *want, int n_want, float *logits_host,
                               float *hidden_host) {
     FH_REQUIRE(finalized && tokens, "decoder not finalized or NULL tokens");
@@ -76,6 +81,7 @@ fh_status fh_decoder::forward(const uint32_t *tokens, int count, const int32_t *
     }
     FH_TRY(ensure_logits(std::max(n_want, 1)));
     FH_TRY(forward_begin());
+    std::vector<int> rows, places;
     const int portion = std::min(count, max_portion());
     FH_TRY(ensure_steps(portion));
     FH_TRY(reserve(pos + count));
@@ -83,10 +89,12 @@ fh_status fh_decoder::forward(const uint32_t *tokens, int count, const int32_t *
         const int n = std::min(portion, count - at);
         FH_TRY(fh_upload(dev, ids, tokens + at, (size_t)n * 4));
         FH_TRY(layers(n, false));
+        rows.clear(), places.clear();
         for (int i = 0; i < n_want; i++) {
             const int row = want[i] + skip - at;
-            if (row >= 0 && row < n) FH_TRY(head(row, logits + (size_t)i * vocab));
+            if (row >= 0 && row < n) rows.push_back(row), places.push_back(i);
         }
+        FH_TRY(heads(rows.data(), places.data(), (int)rows.size()));
         // all layers appended: advance the caches
         history.insert(history.end(), tokens + at, tokens + at + n);
         pos += n;

@@ -613,6 +613,132 @@ fh_status fh_matvec_norm(fh_device *dev, const float *x, int k, const float *w, 
     return FH_OK;
 }
 
+// ------------------------------------------------------------------------------ the output matrix for several rows
+// Bound by the weights, which the matvec reads again for every row (16 rows of 4096 and a matrix of 32768: 16 x 45 us), so up to 16
+// rows share one pass over them on the matrix cores.  The rows stay f32: each value is cut into three bf16 numbers of 8 bits (24
+// in all: without a remainder), whose products with a bf16 weight are exact.  Each of the four wavefronts of a workgroup takes every fourth 64 of k and
+// sums the first terms of even and odd steps and the others apart, so a sum has an eighth of the chain: against 64 bits 1.4e-7 of the root
+// mean square at k = 4096, the matvec 1.6e-7.  With the launch that norms and cuts the rows 14 + 70 us at the size above.
+enum { HEAD_ROWS = 16 };
+struct HeadRows { int row[HEAD_ROWS], place[HEAD_ROWS], n; };
+
+// Final norm of the rows (the arithmetic of k_matvec_norm) and their three terms in the order of the MFMA operand: 64 of k: two
+// steps of 32: three terms: lane l (row l % 16, k = 8 (l / 16) .. + 7): 16 bytes.  Rows that are not there are zeros.
+__global__ __launch_bounds__(256) void k_head_x(const float *__restrict__ x, int k, int kp, const float *__restrict__ nw, float eps,
+                                                HeadRows rows, uint16_t *__restrict__ xf, float *__restrict__ norm_out) {
+    __shared__ float red[4];
+    const int tid = threadIdx.x, r = blockIdx.x;
+    const bool there = r < rows.n;
+    const float *xr = x + (int64_t)rows.row[there ? r : 0] * k;
+    float ss = 0.f;
+    for (int i = tid; i < k; i += 256) ss = fmaf(xr[i], xr[i], ss);
+    ss = fh_wave_sum(ss);
+    if ((tid & 63) == 0) red[tid >> 6] = ss;
+    __syncthreads();
+    const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
+    for (int i = tid; i < kp; i += 256) {
+        const float v = there && i < k ? xr[i] * inv * nw[i] : 0.f;
+        if (r == rows.n - 1) norm_out[i] = v;
+        // cut, not rounded: nothing overflows; an infinity or a NaN is the first term's alone
+        const uint32_t u = __float_as_uint(v);
+        const bool finite = (u & 0x7F800000u) != 0x7F800000u;
+        uint16_t t[3] = {(uint16_t)(u >> 16), 0, 0};
+        if (finite) {
+            const float v1 = v - __uint_as_float(u & 0xFFFF0000u);
+            const uint32_t u1 = __float_as_uint(v1);
+            t[1] = (uint16_t)(u1 >> 16);
+            t[2] = (uint16_t)(__float_as_uint(v1 - __uint_as_float(u1 & 0xFFFF0000u)) >> 16);
+        } else if (u & 0x007FFFFFu)
+            t[0] |= 0x40u;
+        const int step = i >> 5, lane = (i >> 3 & 3) * 16 + r;
+#pragma unroll
+        for (int e = 0; e < 3; e++) xf[(((int64_t)step * 3 + e) * 64 + lane) * 8 + (i & 7)] = t[e];
+    }
+}
+
+__global__ __launch_bounds__(256, 2) void k_head_rows(const uint16_t *__restrict__ w, int n, int kp, const uint16_t *__restrict__ xf,
+                                                      HeadRows rows, float *__restrict__ y, int64_t ldy) {
+    constexpr int STAGES = 3; // 64 of k each: 8 KB of weights and 6 KB of rows a wavefront
+    __shared__ fh_f4 red[4][4][64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row0 = blockIdx.x * 64;
+    const int blocks = kp >> 6, mine = (blocks - wave + 3) >> 2;
+    const uint16_t *wp[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int row = row0 + 16 * t + (lane & 15);
+        wp[t] = w + (int64_t)(row < n ? row : n - 1) * kp + (lane >> 4) * 8;
+    }
+    fh_bf8 a[STAGES][2][4], b[STAGES][2][3];
+    const auto fetch = [&](int s, int i) { // (no request under a condition; past the end the last block again)
+        const int blk = min(4 * min(i, mine - 1) + wave, blocks - 1);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) fh_frag_load(a[s][h][t], wp[t] + blk * 64 + h * 32);
+#pragma unroll
+            for (int e = 0; e < 3; e++) fh_frag_load(b[s][h][e], xf + (((int64_t)blk * 2 + h) * 3 + e) * 512 + lane * 8);
+        }
+    };
+    fh_f4 acc[4][3] = {}; // of the first term in the even and the odd steps, of the two others
+    const auto use = [&](int s) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int e = 0; e < 3; e++) acc[t][e ? 2 : h] = fh_mma32(a[s][h][t], b[s][h][e], acc[t][e ? 2 : h]);
+    };
+    if (mine > 0) {
+#pragma unroll
+        for (int s = 0; s < STAGES; s++) fetch(s, s);
+        int i = 0;
+        for (; i + STAGES < mine; i += STAGES) {
+#pragma unroll
+            for (int s = 0; s < STAGES; s++) {
+                use(s);
+                fetch(s, i + s + STAGES);
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < STAGES; s++)
+            if (i + s < mine) use(s);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        fh_f4 v;
+#pragma unroll
+        for (int e = 0; e < 4; e++) { // (a weight that is infinite leaves a NaN in the terms that are 0)
+            const float hi = acc[t][0][e] + acc[t][1][e];
+            v[e] = (__float_as_uint(hi) & 0x7F800000u) != 0x7F800000u ? hi + acc[t][2][e] : hi;
+        }
+        red[wave][t][lane] = v;
+    }
+    __syncthreads();
+    const fh_f4 v = (red[0][wave][lane] + red[1][wave][lane]) + (red[2][wave][lane] + red[3][wave][lane]);
+    const int r = lane & 15, at = row0 + 16 * wave + 4 * (lane >> 4);
+    if (r >= rows.n) return;
+    float *yr = y + rows.place[r] * ldy;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (at + e < n) yr[at + e] = v[e];
+}
+
+fh_status fh_head_rows(fh_device *dev, const float *x, int k, const float *w, float eps, const uint16_t *out, int n, const int *row,
+                       const int *place, int count, float *y, int64_t ldy, float *norm_out) {
+    const int kp = (int)fh_pad64(k);
+    FH_TRY(fh_dev_scratch(dev, (void **)&dev->ksplit_buf, &dev->ksplit_cap, (size_t)kp * 3 * HEAD_ROWS * 2));
+    uint16_t *xf = (uint16_t *)dev->ksplit_buf;
+    for (int at = 0; at < count; at += HEAD_ROWS) {
+        HeadRows rows = {};
+        rows.n = std::min<int>(count - at, HEAD_ROWS);
+        for (int i = 0; i < rows.n; i++) rows.row[i] = row[at + i], rows.place[i] = place[at + i];
+        k_head_x<<<dim3(HEAD_ROWS), 256, 0, dev->stream>>>(x, k, kp, w, eps, rows, xf, norm_out);
+        k_head_rows<<<dim3((unsigned)((n + 63) / 64)), 256, 0, dev->stream>>>(out, n, kp, xf, rows, y, ldy);
+        FH_HIP(hipGetLastError());
+    }
+    return FH_OK;
+}
+
 // ------------------------------------------------------------------------------ residual streams normed at a sublayer's end
 __global__ void k_group_tiles(int groups, int s, int tile_rows, FhTile *tiles, int *n_tiles) {
     const int per = (s + tile_rows - 1) / tile_rows;

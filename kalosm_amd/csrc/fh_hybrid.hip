@@ -113,6 +113,7 @@ struct Hybrid : fh_decoder {
     FhMvAdd take();
     fh_status step_layer(Layer &l);
     fh_status head(int row, float *dst) override;
+    fh_status heads(const int *rows, const int *places, int n) override;
     const float *hidden() const override { return normed; }
     fh_status reserve(int positions) override;
     int64_t capacity() const override {
@@ -922,6 +923,11 @@ fh_status Hybrid::layers(int s, bool dev_pos) {
 fh_status Hybrid::head(int row, float *dst) {
     const FhMvSeg seg{(const uint16_t *)out->data, dst, vocab};
     return fh_matvec_norm(dev, x + (size_t)row * d_model, d_model, out_norm, eps, &seg, 1, normed);
+}
+
+fh_status Hybrid::heads(const int *rows, const int *places, int n) {
+    if (n < 2) return fh_decoder::heads(rows, places, n); // one row: the matvec, 45 us against 84 for 2 to 16 (4096 x 32768)
+    return fh_head_rows(dev, x, d_model, out_norm, eps, (const uint16_t *)out->data, vocab, rows, places, n, logits, vocab, normed);
 }
 
 fh_status Hybrid::layer_output(int li, float *dst, int64_t count) {

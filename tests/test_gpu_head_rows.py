@@ -1,0 +1,34 @@
+"""GPU parity: the output matrix for several rows in one pass (csrc/fh_dense.hip: k_head_x, k_head_rows) against float64.
+
+Bound: a row's three bf16 terms hold its 24 bits and multiply exactly, so what is left is the rounding of the f32 sums: k errors of
+2^-24 of either sign, 1e-6 of the root mean square for k up to 1000, and ten times that for the largest single difference."""
+import numpy as np
+import pytest
+
+import hybridgen as G
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("width,vocab,count", [(20, 30, 2), (64, 64, 16), (72, 65, 17), (256, 130, 33), (1000, 333, 5)])
+def test_rows(dev, width, vocab, count):
+    """Fewer blocks of 64 than wavefronts, k and n that fill no tile, one row more than a pass takes, places in any order and
+    twice; the normed row that is given back is the last one's."""
+    cfg = G.config([G.with_mlp(G.delta(1, 1, 16, 16, 4), None)], width, vocab)
+    w = G.weights(cfg)
+    m = G.build(dev, cfg, w)
+    rng = np.random.default_rng(width)
+    toks = rng.integers(0, vocab, 40)
+    places = [int(p) for p in rng.integers(0, 40, count)]
+    places[1] = places[0]
+    got, last = m.forward(toks, want_hidden=True, want=places)
+    head = G.round_bf16(w["head"]).astype(np.float64)
+    for i, place in enumerate(places):
+        m.reset()
+        alone, hidden = m.forward(toks, want_hidden=True, want=[place])
+        want = head @ hidden.astype(np.float64)
+        rms = np.sqrt(np.mean(want * want))
+        for y in (got[i], alone[0]):
+            assert np.sqrt(np.mean((y - want) ** 2)) <= 1e-6 * rms
+            assert np.abs(y - want).max() <= 1e-5 * rms
+    assert np.abs(last - hidden).max() <= 1e-6 * np.abs(hidden).max()

@@ -4,6 +4,7 @@
 // raw/rope.rs:87-112 (interleaved RoPE for the llama architecture), model/inference.rs:11-396
 // (decode loop, here greedy).
 #include "fh_decoder.h"
+#include "fh_qmm_frag.h"
 
 #include <algorithm>
 #include <cstdarg>
@@ -480,9 +481,13 @@ fh_status fh_llama::layers(int s, bool dev_pos) {
         } else if (l.gate_up && s <= 2) {
             FH_TRY(fh_qmatmul_swiglu(l.gate_up, m->xn, s, m->act));
         } else if (l.gate_up) {
-            FH_TRY(fh_qmatmul(l.gate_up, m->xn, s, m->gu)); // [s, 2F]: gate | up per row
-            // split the halves: silu(gate) * up with row stride 2F
-            FH_TRY(fh_swiglu_rows(dev, m->gu, s, F, m->act));
+            fh_status st = fh_qmm_frag_swiglu(l.gate_up, m->xn, s, m->act);
+            if (st == FH_ERR_UNSUPPORTED) {
+                FH_TRY(fh_qmatmul(l.gate_up, m->xn, s, m->gu)); // [s, 2F]: gate | up per row
+                // split the halves: silu(gate) * up with row stride 2F
+                st = fh_swiglu_rows(dev, m->gu, s, F, m->act);
+            }
+            FH_TRY(st);
         } else {
             FH_TRY(fh_qmatmul(l.gate, m->xn, s, m->gu));
             FH_TRY(fh_qmatmul(l.up, m->xn, s, m->gu + (size_t)s * F));

@@ -163,12 +163,17 @@ __device__ __forceinline__ void frag_store(uint8_t *p, const _Float16 *h) {
 // One workgroup: a tile of 16 rows of the tiled layout, its wavefronts share out the 256-runs of k; lane = (lane group g, row j)
 // of the layout.  `d` receives the scales [k / 256 (+ 1)] (formats with one per 256; the last one belongs to the offsets) or
 // [k / 32], n_pad apart.  ext columns as in k_frag_x; plane: distance of the second weight plane (Q6_K).
+// half > 0 (a multiple of 32): rows i and half + i belong together (gate and up); their groups of 32 are stored in turn, so that a
+// wavefront of the product holds both.
 template <int T>
 __global__ __launch_bounds__(512) void k_frag_w(QView q, int64_t tile0, int ext, int xplanes, uint8_t *__restrict__ out,
-                                                 int64_t plane, float *__restrict__ d, int64_t n_pad) {
+                                                 int64_t plane, float *__restrict__ d, int64_t n_pad, int half) {
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, j = lane & 15, g = lane >> 4;
     const int64_t tile = tile0 + blockIdx.x;
-    const int k = (int)q.k, kf = (k + ext) >> 4, row = (int)blockIdx.x * 16 + j;
+    const int k = (int)q.k, kf = (k + ext) >> 4;
+    int row = (int)blockIdx.x * 16;
+    if (half) row = row < half ? (row & ~31) * 2 + (row & 31) : ((row - half) & ~31) * 2 + 32 + ((row - half) & 31);
+    row += j;
     uint8_t *dst = out + ((int64_t)(row >> 5) * kf) * 1024 + (row & 31) * 16;
     const uint8_t *recs = q.data + tile * q.recs * q.rec_bytes;
     const int runs = (k + 255) >> 8;
@@ -313,6 +318,7 @@ struct FragArgs {
     int m, n, n0;    // rows, weight rows of this launch, first of them in y
     int kf, tiles_w, tiles_x, parts;
     int64_t part_stride; // floats between the partial planes of a split k
+    int half;            // > 0: y[:, i] = silu(row i) * (row half + i)
 };
 
 // NW / NX: weight and activation planes; SC: k per scale (32 or 256); a wavefront owns FW x FX tiles of 32 x 32, the eight
@@ -484,6 +490,20 @@ __global__ __launch_bounds__(512) void k_qmm_frag(FragArgs g) {
     if (SC == 32) scale(3, FW / 2, FW); // (a multiple of four 32s: the last one's scale is in the last place)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // no LDS-direct load outlives the workgroup's LDS
     float *y = g.y + part * g.part_stride;
+    if (g.half) { // (FW is 2: gate and up)
+        const int nn = (tw * (TW / 64) + ww) * 32 + li;
+        if (nn >= g.half) return;
+#pragma unroll
+        for (int c = 0; c < FX; c++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int mm = tx * TX + (wx * FX + c) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                if (mm >= g.m) continue;
+                const float gate = acc[0][c][r] * g.rs[mm], up = acc[1][c][r] * g.rs[mm];
+                y[(int64_t)mm * g.ldy + nn] = (gate / (expf(-gate) + 1.0f)) * up;
+            }
+        return;
+    }
 #pragma unroll
     for (int a = 0; a < FW; a++) {
         const int nn = tw * TW + (ww * FW + a) * 32 + li;
@@ -519,7 +539,7 @@ __global__ void k_frag_sum(const float *__restrict__ part, int parts, int64_t st
 
 // ------------------------------------------------------------------------------ launches
 template <int NW, int NX, int SC, int FW, int FX, int WGX>
-static fh_status frag_product(fh_device *dev, FragArgs g) {
+static fh_status frag_product(fh_device *dev, FragArgs g, bool ask) { // ask: is k in one part?
     typedef FragTile<NW, NX, FW, FX, WGX> Tile;
     constexpr int TW = Tile::TW, TX = Tile::TX, LDS = Tile::STAGES * Tile::STAGE;
     g.tiles_w = (g.n + TW - 1) / TW;
@@ -530,13 +550,14 @@ static fh_status frag_product(fh_device *dev, FragArgs g) {
     const int64_t tiles = (int64_t)g.tiles_w * g.tiles_x;
     double best = 1e30;
     int parts = 1;
-    const int most = g.n == g.ldy ? 8 : 1; // (weight rows in several launches: whole)
+    const int most = g.n == g.ldy || g.half ? 8 : 1; // (weight rows in several launches: whole)
     for (int p = 1; p <= most && p * 2 <= quads; p++) {
         const int64_t rounds = (tiles * p + dev->compute_units - 1) / dev->compute_units;
         double t = (double)rounds * ((double)((quads + p - 1) / p) + 1.5) * 2.5;
         if (p > 1) t += 4.0 + (2.0 * p + 1.0) * g.m * (double)g.n * 4.0 / 4e6;
         if (t < best * 0.97) best = t, parts = p;
     }
+    if (ask || (g.half && parts > 1)) return parts == 1 ? FH_OK : FH_ERR_UNSUPPORTED;
     g.parts = parts;
     float *y = g.y;
     if (parts > 1) { // whole planes [m][n] of this launch's weight rows
@@ -584,11 +605,32 @@ bool fh_qmm_frag_pays(const fh_qmatrix *q, int x_is_bf16, int m) {
     return !x_is_bf16 && m > 512;
 }
 
-fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y) {
+#define FRAG_GO(NW_, NX_, SC_, WGX_) \
+    (m <= 64 ? frag_product<NW_, NX_, SC_, 2, 1, 2>(dev, g, ask) : frag_product<NW_, NX_, SC_, 2, 2, WGX_>(dev, g, ask))
+static fh_status frag_go(fh_device *dev, const FragArgs &g, int sc, int wp, int xp, bool ask) {
+    const int m = g.m;
+    if (sc == 32) return xp == 2 ? FRAG_GO(1, 2, 32, 2) : FRAG_GO(1, 1, 32, 2);
+    if (wp == 2) return xp == 2 ? FRAG_GO(2, 2, 256, 4) : FRAG_GO(2, 1, 256, 4);
+    return xp == 2 ? FRAG_GO(1, 2, 256, 2) : FRAG_GO(1, 1, 256, 2);
+}
+#undef FRAG_GO
+
+static fh_status qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, int half) {
     fh_device *dev = q->dev;
     const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2, wp = q->type == FH_Q6_K ? 2 : 1;
     const int ext = q->type == FH_Q4_K || q->type == FH_Q5_K ? frag_ext(k, xp) : 0, kf = (k + ext) / 16;
     const int sc = fh_block_elems(q->type);
+    // weights: as many rows at a time as 512 MB of fragments hold
+    const int64_t rows_all = (q->n + 255) / 256 * 256;
+    int64_t rows = (int64_t)(512 << 20) / ((int64_t)kf * 32 * wp) / 256 * 256;
+    rows = rows < 256 ? 256 : (rows > rows_all ? rows_all : rows);
+    if (half) { // all rows at once, k in one part
+        if (rows < q->n) return FH_ERR_UNSUPPORTED;
+        FragArgs g{};
+        g.m = m, g.n = (int)q->n, g.kf = kf, g.half = half;
+        const fh_status st = frag_go(dev, g, sc, wp, xp, true);
+        if (st != FH_OK) return st;
+    }
     // activations: rows up to a multiple of the largest tile (rows past m are multiplied and never stored)
     const int64_t mp = ((int64_t)m + 255) / 256 * 256, xplane = mp * kf * 32;
     FH_TRY(fh_dev_scratch(dev, &dev->act_buf, &dev->act_cap, (size_t)(xplane * xp + mp * 4)));
@@ -606,10 +648,6 @@ fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, 
         k_frag_x<0><<<dim3((unsigned)((m + 7) / 8), (unsigned)runs), 512, lds, dev->stream>>>(x, m, k, ext, xf, xplane, rs);
     }
     FH_HIP(hipGetLastError());
-    // weights: as many rows at a time as 512 MB of fragments hold
-    const int64_t rows_all = (q->n + 255) / 256 * 256;
-    int64_t rows = (int64_t)(512 << 20) / ((int64_t)kf * 32 * wp) / 256 * 256;
-    rows = rows < 256 ? 256 : (rows > rows_all ? rows_all : rows);
     const int64_t wplane = rows * kf * 32, scales = sc == 32 ? k / 32 : k / 256 + (ext ? (ext + 255) / 256 : 0);
     const size_t need = (size_t)(wplane * wp + scales * rows * 4);
     FH_TRY(fh_dev_scratch(dev, &dev->frag_buf, &dev->frag_cap, need));
@@ -619,7 +657,7 @@ fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, 
     for (int64_t n0 = 0; n0 < q->n; n0 += rows) {
         const int64_t n = q->n - n0 < rows ? q->n - n0 : rows;
         const dim3 grid((unsigned)((n + 15) / 16));
-#define FRAG_W(T_) k_frag_w<T_><<<grid, 512, 0, dev->stream>>>(v, n0 / 16, ext, xp, wf, wplane, d, rows)
+#define FRAG_W(T_) k_frag_w<T_><<<grid, 512, 0, dev->stream>>>(v, n0 / 16, ext, xp, wf, wplane, d, rows, half)
         switch (q->type) {
         case FH_Q4_0: FRAG_W(FH_Q4_0); break;
         case FH_Q8_0: FRAG_W(FH_Q8_0); break;
@@ -632,14 +670,20 @@ fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, 
 #undef FRAG_W
         FH_HIP(hipGetLastError());
         FragArgs g{};
-        g.w = wf, g.x = xf, g.w_plane = wplane, g.x_plane = xplane, g.d = d, g.n_pad = rows, g.rs = rs, g.y = y, g.ldy = q->n;
+        g.w = wf, g.x = xf, g.w_plane = wplane, g.x_plane = xplane, g.d = d, g.n_pad = rows, g.rs = rs, g.y = y, g.ldy = half ? half : q->n, g.half = half;
         g.m = m, g.n = (int)n, g.n0 = (int)n0, g.kf = kf;
-#define FRAG_GO(NW_, NX_, SC_, WGX_) \
-    (m <= 64 ? frag_product<NW_, NX_, SC_, 2, 1, 2>(dev, g) : frag_product<NW_, NX_, SC_, 2, 2, WGX_>(dev, g))
-        if (sc == 32) FH_TRY((xp == 2 ? FRAG_GO(1, 2, 32, 2) : FRAG_GO(1, 1, 32, 2)));
-        else if (wp == 2) FH_TRY((xp == 2 ? FRAG_GO(2, 2, 256, 4) : FRAG_GO(2, 1, 256, 4)));
-        else FH_TRY((xp == 2 ? FRAG_GO(1, 2, 256, 2) : FRAG_GO(1, 1, 256, 2)));
-#undef FRAG_GO
+        FH_TRY(frag_go(dev, g, sc, wp, xp, false));
     }
     return FH_OK;
+}
+
+fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y) { return qmm_frag(q, x, x_is_bf16, m, y, 0); }
+
+// In the epilogue of the product SwiGLU saves writing and reading 2 n floats a row and a launch: 2048 rows of a 28672 x 4096 matrix
+// take 835 us and no 77 of a SwiGLU launch (7 % of a layer was writing and reading what one store now holds).
+fh_status fh_qmm_frag_swiglu(const fh_qmatrix *q, const float *x, int m, float *y) {
+    const int64_t opt = q->dev->opt_matmul_kernel;
+    if (q->n % 64 || ((uintptr_t)x & 15) || m <= 16 || !(opt == 0 ? fh_qmm_frag_pays(q, 0, m) : opt == 13 && fh_qmm_frag_supports(q)))
+        return FH_ERR_UNSUPPORTED;
+    return qmm_frag(q, x, 0, m, y, (int)(q->n / 2));
 }

@@ -84,3 +84,23 @@ def test_rows_are_independent(dev, oracle, ty):
     assert not np.isfinite(got[5]).any() and np.isnan(got[6]).all()
     rest = [r for r in range(m) if r not in (3, 4, 5, 6)]
     assert np.array_equal(got[rest], base[rest])
+
+
+@pytest.mark.parametrize("m", [17, 64, 65, 257])
+@pytest.mark.parametrize("ffn", [256, 768])
+def test_swiglu_epilogue(dev, m, ffn):
+    """gate | up of one launch, SwiGLU at the store, against the two halves as matrices of their own: the same sums and the same
+    formula, so the logits are the same bits."""
+    from kalosm_amd.llama import Model
+
+    cfg = dict(n_layers=2, d_model=256, n_heads=2, n_kv_heads=1, head_dim=128, ffn=ffn, vocab=320, ctx=512, eps=1e-5, theta=1e4)
+    tokens = np.random.default_rng(m).integers(0, 320, m)
+    got = []
+    for fuse in (True, False):
+        model = Model.random_init(dev, cfg, seed=2, sigma=2e-3, fuse_gate_up=fuse)
+        dev.set_option("matmul_kernel", 13)
+        try:
+            got.append(model.forward(tokens))
+        finally:
+            dev.set_option("matmul_kernel", 0)
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])

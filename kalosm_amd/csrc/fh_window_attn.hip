@@ -8,7 +8,12 @@ static constexpr float FH_LOG2E = 1.4426950408889634f;
 // softmax statistics are per-lane scalars.  MFMA row i of half hf of a 32-key group reads key 8 (i / 4) + 4 hf + i % 4:
 // with that order the accumulators of a lane are keys 8 g .. 8 g + 7 (g = lane / 16), the k-slots of its P^T operand.
 // Key tiles of 64 go through the LDS (K as [key][dq], V transposed as [value][key]); the next tile is requested into
-// registers while the current one is multiplied.
+// registers while the current one is multiplied.  No request is under a condition: rows and columns past the end are read from
+// the last one and dropped (keys by the mask, the rest when they are stored to the LDS) - a branch with a request in it and a use of
+// it behind it makes the wavefront wait for that request alone, four times a tile.  Tiles that every query of the wavefront sees
+// whole, all but the first and the last ones of a block, take no mask.
+// 2048 queries, window 1024: 32 heads of 192 / 128 124 us (255 before), 128 / 128 119 us (237); two wavefronts a SIMD (512 registers
+// were one).  What bounds it: the softmax between two products on the matrix cores.
 // P^T operands: bf16 as hi + lo
 __device__ __forceinline__ void fh_pv(fh_f4 &acc, const fh_bf8 &v, const float *p) {
     fh_bf8 hi, lo;
@@ -28,7 +33,7 @@ __device__ __forceinline__ void fh_pv(fh_f4 &acc, const fh_f8 &v, const float *p
 }
 
 template <typename T, int DQS, int DVT, int QF>
-__global__ __launch_bounds__(256) void k_window_attn(FhWindowAttn a, const T *__restrict__ q, const T *__restrict__ kn,
+__global__ __launch_bounds__(256, sizeof(T) == 2 && DQS * DVT < 64 ? 2 : 1) void k_window_attn(FhWindowAttn a, const T *__restrict__ q, const T *__restrict__ kn,
                                                      const T *__restrict__ kr, const T *__restrict__ vt, int64_t ldt, int s,
                                                      int keys, T *__restrict__ o, int ldo, int kp) {
     typedef typename FhFrag<T>::type Frag;
@@ -66,42 +71,56 @@ __global__ __launch_bounds__(256) void k_window_attn(FhWindowAttn a, const T *__
     const int j1 = a.pos + last - a.gap + 1;                         // one past the last visible key
     const int nk = a.keep < keys ? a.keep : keys;
     auto next = [&](int j) { return j + 64 >= nk && j + 64 < j0 ? j0 : j + 64; };
+    // Eight threads a row: keys r0 and r0 + 32, pieces p0, p0 + 8, ...; value rows r0, r0 + 32, ..., keys 8 p0 .. + 7.
+    // (worked out anew for every tile: as values kept over the loop they spill)
+    auto place = [&](int &r0, int &p0) {
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        r0 = t >> 3, p0 = t & 7;
+    };
+    static_assert(DQ % 64 == 0, "eight threads share a key's pieces evenly");
     FhPiece<T> pk[NK], pv[NV];
     auto fetch = [&](int j) {
+        int r0, p0;
+        place(r0, p0);
+        // scalar bases, offsets within the tile in 32 bits (addresses of 64 bits kept over the loop do not fit the registers)
+        const T *nope = kn + (int64_t)j * kvh * a.dnp, *rope = kr + (int64_t)j * a.drp, *val = vt + (int64_t)hk * a.dv * ldt + j;
+        const int end = keys - 1 - j; // the tile's last key that is there
 #pragma unroll
         for (int i = 0; i < NK; i++) {
-            const int x = tid + 256 * i, r = x / (DQ / 8), c = x % (DQ / 8);
-            const int key = j + r;
-            if (key < keys && c < npk) pk[i] = fh_ld_piece(kn + ((int64_t)key * kvh + hk) * a.dnp + c * 8);
-            else if (key < keys && c - npk < nrk && c >= npk) pk[i] = fh_ld_piece(kr + (int64_t)key * a.drp + (c - npk) * 8);
-            else pk[i] = fh_zero_piece<T>();
+            const int row = r0 + 32 * (i & 1), key = row < end ? row : end, c = p0 + 8 * (i >> 1);
+            const bool r = c >= npk && nrk;
+            const int cn = c < npk ? c : npk - 1, cr = c - npk < nrk ? c - npk : nrk - 1;
+            pk[i] = fh_ld_piece((r ? rope : nope) + (uint32_t)(r ? key * a.drp + cr * 8 : (key * kvh + hk) * a.dnp + cn * 8));
         }
 #pragma unroll
         for (int i = 0; i < NV; i++) {
-            const int x = tid + 256 * i, r = x >> 3, c = (x & 7) * 8;
-            if (dv0 + r < a.dv && j + c < keys) {
-                pv[i] = fh_ld_piece(vt + (int64_t)(hk * a.dv + dv0 + r) * ldt + j + c);
-                if (j + c + 8 > keys)
-#pragma unroll
-                    for (int e = 0; e < 8; e++)
-                        if (j + c + e >= keys) pv[i].v[e] = 0;
-            } else pv[i] = fh_zero_piece<T>();
+            const int r = r0 + 32 * i, row = dv0 + r < a.dv ? dv0 + r : a.dv - 1;
+            pv[i] = fh_ld_piece(val + (uint32_t)(row * (int)ldt + (8 * p0 < end ? 8 * p0 : end & ~7)));
         }
     };
+    const bool padded = (npk + nrk) * 8 < DQ;
     const int first = nk > 0 ? 0 : j0;
     fetch(first);
     for (int j = first; j < j1; j = next(j)) {
         __syncthreads(); // the previous tile has been read
+        int r0, p0;
+        place(r0, p0);
 #pragma unroll
         for (int i = 0; i < NK; i++) {
-            const int x = tid + 256 * i, r = x / (DQ / 8), c = x % (DQ / 8);
-            fh_st_piece(sk + r * KS + c * 8, pk[i]);
+            const int c = p0 + 8 * (i >> 1);
+            if (padded && c >= npk + nrk) pk[i] = fh_zero_piece<T>();
+            fh_st_piece(sk + (r0 + 32 * (i & 1)) * KS + c * 8, pk[i]);
+        }
+        if (j + 64 > keys) { // values past the end: zeros
+#pragma unroll
+            for (int i = 0; i < NV; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (j + 8 * p0 + e >= keys) pv[i].v[e] = 0;
         }
 #pragma unroll
-        for (int i = 0; i < NV; i++) {
-            const int x = tid + 256 * i, r = x >> 3, c = (x & 7) * 8;
-            fh_st_piece(sv + r * VS + c, pv[i]);
-        }
+        for (int i = 0; i < NV; i++) fh_st_piece(sv + (r0 + 32 * i) * VS + 8 * p0, pv[i]);
         __syncthreads();
         if (next(j) < j1) fetch(next(j));
         fh_f4 S[4][QF];
@@ -119,9 +138,23 @@ __global__ __launch_bounds__(256) void k_window_attn(FhWindowAttn a, const T *__
             }
         }
         float p[QF][2][8];
+        // positions of the tile's first and last row; the first and the last query of the wavefront
+        const int lo = j + (j >= a.kept ? a.gap : 0), hi = j + 63 + (j + 63 >= a.kept ? a.gap : 0);
+        const int q0 = a.pos + qb + wave * 16 * QF, q1 = q0 + 16 * QF - 1;
+        const bool whole = hi <= q0 && (!a.window || q1 - lo < a.window);
 #pragma unroll
         for (int f = 0; f < QF; f++) {
             float tm = -INFINITY;
+            if (whole) {
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float v = S[t][f][r] * sc;
+                        p[f][t >> 1][4 * (t & 1) + r] = v;
+                        tm = fmaxf(tm, v);
+                    }
+            } else
 #pragma unroll
             for (int t = 0; t < 4; t++)
 #pragma unroll
@@ -137,13 +170,13 @@ __global__ __launch_bounds__(256) void k_window_attn(FhWindowAttn a, const T *__
             tm = fmaxf(tm, __shfl_xor(tm, 16, 64));
             tm = fmaxf(tm, __shfl_xor(tm, 32, 64));
             const float mn = fmaxf(mx[f], tm), mb = mn == -INFINITY ? 0.f : mn;
-            const float resc = exp2f(mx[f] - mb);
+            const float resc = __builtin_amdgcn_exp2f(mx[f] - mb); // (below 2^-126: 0)
             float sum = 0.f;
 #pragma unroll
             for (int u = 0; u < 2; u++)
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-                    const float w = exp2f(p[f][u][e] - mb);
+                    const float w = __builtin_amdgcn_exp2f(p[f][u][e] - mb);
                     p[f][u][e] = w;
                     sum += w;
                 }

@@ -3,35 +3,46 @@
 #include "fh_recurrent.h"
 
 // ------------------------------------------------------------------------------ inputs of the recurrence
-// One workgroup per token.
-__global__ __launch_bounds__(256) void k_rec_prep(FhRecurrent r, const float *__restrict__ proj, int64_t ldp, int pos,
+// One workgroup per T tokens.  Bound by memory: with one token a workgroup a thread read the same column of four rows, one after the
+// other, for every token; with four it has seven rows on their way and uses each up to four times
+// (2048 tokens, 16 + 16 heads of 128 and 32 of 128: 133 -> 79 us; with a quarter of the threads 104).
+template <int T>
+__global__ __launch_bounds__(T * 256) void k_rec_prep(FhRecurrent r, const float *__restrict__ proj, int64_t ldp, int s, int pos,
                                                   const float *__restrict__ ring, FhRecWork w, int dp) {
-    extern __shared__ float qk[]; // [2 * kv_heads * dim]
-    const int t = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    extern __shared__ float qk[]; // [T][2 * kv_heads * dim]
+    const int t0 = (int)blockIdx.x * T, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, nt = s - t0 < T ? s - t0 : T;
     const int nq = r.kv_heads * r.dim, inner = r.heads * r.vdim, channels = 2 * nq + inner;
-    for (int ch = tid; ch < channels; ch += 256) {
-        const float v = fh_rec_conv(r, ch, proj, ldp, t, pos, ring, channels);
-        if (ch < 2 * nq) qk[ch] = v;
-        else w.v[(int64_t)t * inner + ch - 2 * nq] = v;
+    for (int ch = tid; ch < channels; ch += 256 * T) {
+        float v[T];
+        if (T > 1) fh_rec_conv_rows<T>(r, ch, proj, ldp, t0, s, pos, ring, channels, v);
+        else v[0] = fh_rec_conv(r, ch, proj, ldp, t0, pos, ring, channels);
+#pragma unroll
+        for (int i = 0; i < T; i++) {
+            if (i >= nt) break;
+            if (ch < 2 * nq) qk[i * 2 * nq + ch] = v[i];
+            else w.v[(int64_t)(t0 + i) * inner + ch - 2 * nq] = v[i];
+        }
     }
-    for (int h = tid; h < r.heads; h += 256) {
+    for (int x = tid; x < nt * r.heads; x += 256 * T) {
+        const int t = t0 + x / r.heads, h = x % r.heads;
         const float *row = proj + (int64_t)t * ldp;
         const float sp = fh_softplus_f(row[r.col_a + h] + r.dt_bias[h]);
         w.la[(int64_t)t * r.heads + h] = -expf(r.a_log[h]) * sp;
         w.beta[(int64_t)t * r.heads + h] = r.delta() ? fh_sigmoid_f(row[r.col_b + h]) : sp;
     }
     __syncthreads();
-    for (int h = wave; h < 2 * r.kv_heads; h += 4) {
-        const float *x = qk + h * r.dim;
+    for (int y = wave; y < nt * 2 * r.kv_heads; y += 4 * T) {
+        const int i = y / (2 * r.kv_heads), h = y % (2 * r.kv_heads);
+        const float *x = qk + i * 2 * nq + h * r.dim;
         float f = 1.f;
         if (r.delta()) {
             float ss = 0.f;
-            for (int i = lane; i < r.dim; i += 64) ss = fmaf(x[i], x[i], ss);
+            for (int e = lane; e < r.dim; e += 64) ss = fmaf(x[e], x[e], ss);
             f = 1.0f / sqrtf(fh_wave_sum(ss) + 1e-6f);
         }
         if (h < r.kv_heads) f *= r.q_scale;
-        float *dst = (h < r.kv_heads ? w.q : w.k) + ((int64_t)t * r.kv_heads + h % r.kv_heads) * dp;
-        for (int i = lane; i < dp; i += 64) dst[i] = i < r.dim ? x[i] * f : 0.f;
+        float *dst = (h < r.kv_heads ? w.q : w.k) + ((int64_t)(t0 + i) * r.kv_heads + h % r.kv_heads) * dp;
+        for (int e = lane; e < dp; e += 64) dst[e] = e < r.dim ? x[e] * f : 0.f;
     }
 }
 
@@ -649,8 +660,15 @@ fh_status fh_recurrent_prefill(fh_device *dev, int dtype, const FhRecurrent &r, 
         const int nq = r.kv_heads * r.dim, channels = fh_rec_channels(r);
         const size_t lds = (size_t)2 * nq * 4;
         FH_REQUIRE(lds <= 150 * 1024, "recurrent layer of %d channels is too wide", channels);
-        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_rec_prep, lds));
-        k_rec_prep<<<dim3((unsigned)s), 256, lds, str>>>(r, proj, ldp, pos, st.conv, w, dp);
+        // four tokens a workgroup where there are enough of them for the compute units (fewer leave some idle), their queries and
+        // keys fit the LDS twice and the taps reach no further back than the rows a thread holds
+        if (r.taps <= FH_REC_TAPS && s >= 4 * dev->compute_units && 4 * lds <= 80 * 1024) {
+            if (4 * lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_rec_prep<4>, 4 * lds));
+            k_rec_prep<4><<<dim3((unsigned)((s + 3) / 4)), 1024, 4 * lds, str>>>(r, proj, ldp, s, pos, st.conv, w, dp);
+        } else {
+            if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_rec_prep<1>, lds));
+            k_rec_prep<1><<<dim3((unsigned)s), 256, lds, str>>>(r, proj, ldp, s, pos, st.conv, w, dp);
+        }
         const int ty = s < r.taps ? s : r.taps;
         k_rec_tail<<<dim3((unsigned)((channels + 255) / 256), (unsigned)ty), 256, 0, str>>>(r, proj, ldp, s, pos, st.conv);
     }

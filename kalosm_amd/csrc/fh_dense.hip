@@ -509,7 +509,10 @@ fh_status fh_rows_to_act(fh_device *dev, int dtype, const float *x, int64_t ldx,
 // barrier, rotated or from copies of its own, with 2 to 16 pieces ahead, and with one workgroup per compute unit.
 struct MvSegs { FhMvSeg s[3]; int tiles[3]; int n; };
 
-template <int ROWS>
+// XV: 16-byte pieces of the input a thread holds.  Inputs of at most 2048 take two of them and four pieces of the weights ahead:
+// with the four and eight of longer ones, requests past the end repeat the last piece: a matrix of 32768 x 2048 takes 30.2
+// us for 31.2, the four matrices ahead of a layer's mixer 8.7 - 13.8 for 9.6 - 14.4.
+template <int ROWS, int XV>
 __global__ __launch_bounds__(256) void k_matvec_norm(const float *__restrict__ x, int k, int kp, const float *__restrict__ nw,
                                                      float eps, MvSegs segs, float *__restrict__ norm_out) {
     extern __shared__ __attribute__((aligned(16))) float xs[]; // [kp]
@@ -519,16 +522,16 @@ __global__ __launch_bounds__(256) void k_matvec_norm(const float *__restrict__ x
     while (si + 1 < segs.n && tile >= segs.tiles[si]) tile -= segs.tiles[si++];
     const FhMvSeg seg = segs.s[si];
     const int row0 = (tile * 4 + wave) * ROWS;
-    FhRowStream<ROWS, 16 / ROWS < 8 ? 16 / ROWS : 8> rows;
+    FhRowStream<ROWS, 16 / ROWS < 2 * XV ? 16 / ROWS : 2 * XV> rows;
 #pragma unroll
     for (int r = 0; r < ROWS; r++) rows.w[r] = seg.w + (int64_t)(row0 + r < seg.n ? row0 + r : seg.n - 1) * kp;
     // The input is requested first (it comes out of the L2 while the weights are on their way: requests are waited for in order),
     // then the first weights, then the input is normed.
-    if (!(k & 3) && k <= 4096) {
-        float4 v[4], w[4];
+    if (!(k & 3) && k <= 1024 * XV) {
+        float4 v[XV], w[XV];
         const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < XV; j++) {
             const int i = (tid + 256 * j) * 4, at = i < k ? i : 0;
             v[j] = *(const float4 *)(x + at);
             w[j] = nw ? *(const float4 *)(nw + at) : zero;
@@ -540,7 +543,7 @@ __global__ __launch_bounds__(256) void k_matvec_norm(const float *__restrict__ x
         if (nw) {
             float ss = 0.f;
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < XV; j++)
                 if ((tid + 256 * j) * 4 < k) ss = fmaf(v[j].x, v[j].x, fmaf(v[j].y, v[j].y, fmaf(v[j].z, v[j].z, fmaf(v[j].w, v[j].w, ss))));
             ss = fh_wave_sum(ss);
             if (lane == 0) red[wave] = ss;
@@ -548,7 +551,7 @@ __global__ __launch_bounds__(256) void k_matvec_norm(const float *__restrict__ x
             inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < XV; j++) {
             const int i = (tid + 256 * j) * 4;
             if (i >= kp) continue;
             float4 o = i < k ? v[j] : zero;
@@ -604,11 +607,19 @@ fh_status fh_matvec_norm(fh_device *dev, const float *x, int k, const float *w, 
     }
     const size_t lds = (size_t)kp * 4;
     FH_REQUIRE(lds <= 120 * 1024, "k = %d too long for the matvec", k);
-    const void *fn = rows == 4 ? (const void *)k_matvec_norm<4> : rows == 2 ? (const void *)k_matvec_norm<2> : (const void *)k_matvec_norm<1>;
-    if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, fn, lds));
-    if (rows == 4) k_matvec_norm<4><<<dim3((unsigned)tiles), 256, lds, dev->stream>>>(x, k, kp, w, eps, ms, norm_out);
-    else if (rows == 2) k_matvec_norm<2><<<dim3((unsigned)tiles), 256, lds, dev->stream>>>(x, k, kp, w, eps, ms, norm_out);
-    else k_matvec_norm<1><<<dim3((unsigned)tiles), 256, lds, dev->stream>>>(x, k, kp, w, eps, ms, norm_out);
+#define MV_NORM(ROWS_, XV_)                                                                                               \
+    do {                                                                                                                  \
+        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_matvec_norm<ROWS_, XV_>, lds));                    \
+        k_matvec_norm<ROWS_, XV_><<<dim3((unsigned)tiles), 256, lds, dev->stream>>>(x, k, kp, w, eps, ms, norm_out);      \
+    } while (0)
+    if (k <= 2048) {
+        if (rows == 4) MV_NORM(4, 2);
+        else if (rows == 2) MV_NORM(2, 2);
+        else MV_NORM(1, 2);
+    } else if (rows == 4) MV_NORM(4, 4);
+    else if (rows == 2) MV_NORM(2, 4);
+    else MV_NORM(1, 4);
+#undef MV_NORM
     FH_HIP(hipGetLastError());
     return FH_OK;
 }

@@ -47,7 +47,7 @@ __global__ __launch_bounds__(1024) void k_moe_sort(FhMoe m, const int *__restric
 }
 
 // x += mix + the token's weighted expert rows + its row of the always-on expert.  Bound by memory (top + 4 rows of f32): a thread
-// takes V neighbouring columns, so that a wavefront has whole kilobytes of every row on their way: 2048 rows of 4096, top 2 47 us (one column 72).
+// takes V neighbouring columns, so that a wavefront has whole kilobytes of every row on their way: 2048 rows of 4096, top 4 47 us (one column 72).
 template <int V>
 __global__ __launch_bounds__(256) void k_moe_combine(FhMoe m, const float *__restrict__ mix, const float *__restrict__ y,
                                                      const float *__restrict__ sy, const int *__restrict__ inv,

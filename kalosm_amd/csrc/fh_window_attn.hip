@@ -12,8 +12,8 @@ static constexpr float FH_LOG2E = 1.4426950408889634f;
 // the last one and dropped (keys by the mask, the rest when they are stored to the LDS) - a branch with a request in it and a use of
 // it behind it makes the wavefront wait for that request alone, four times a tile.  Tiles that every query of the wavefront sees
 // whole, all but the first and the last ones of a block, take no mask.
-// 2048 queries, window 1024: 32 heads of 192 / 128 124 us (255 before), 128 / 128 119 us (237); two wavefronts a SIMD (512 registers
-// were one).  What bounds it: the softmax between two products on the matrix cores.
+// 2048 queries that see all before them, 32 heads of 192 / 128: 124 us (255 before), 128 / 128: 119 us (237); two wavefronts a SIMD
+// (with 346 registers it was one).  What bounds it: the softmax between two products on the matrix cores.
 // P^T operands: bf16 as hi + lo
 __device__ __forceinline__ void fh_pv(fh_f4 &acc, const fh_bf8 &v, const float *p) {
     fh_bf8 hi, lo;

@@ -1,4 +1,4 @@
-"""GPU parity: the prompt matmul on fragment-ordered operands (csrc/fh_qmm_frag.hip) against a float64 product of the checker's
+"""GPU parity: the prompt matmul on fragment-ordered operands (csrc/fh_qmm_frag.hip) against a float64 product of the oracle's
 dequantised weights.
 
 Bound: the operands are exact up to 2^-22 of each activation and each product is added in f32, k / 16 * 3 additions in a

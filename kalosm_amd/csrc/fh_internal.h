@@ -205,7 +205,10 @@ bool fh_qmatvec_batch_supports(const fh_qmatrix *q, int m, int epi);
 fh_status fh_launch_qmatvec_batch(const fh_qmatrix *q, const float *x, int m, float *y, int epi, const float *a,
                                   const float *b);
 fh_status fh_launch_qmm_q8_mfma(const fh_qmatrix *q, const float *x, int m, float *y);
-fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y);
+// fragments: whether the rule of fh_qmm_frag.hip may take the product
+fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, bool fragments = true);
+// fh_qmatmul of a decoder's prompt: short ones keep the sums of the tile kernels (fh_qmm_frag.h, FH_SHORT_PROMPT).
+fh_status fh_qmatmul_prompt(const fh_qmatrix *q, const float *x, int m, float *y);
 // power of two for fh_qmatrix::wscale from the largest |w| of `count` f32 values on the device (blocking)
 fh_status fh_dense_wscale(fh_device *dev, const float *w_dev, int64_t count, float *wscale);
 enum { FH_EPI_NONE = 0, FH_EPI_ADD2 = 1, FH_EPI_SWIGLU = 2, FH_EPI_ROPEKV = 3, FH_EPI_ACC = 4 };

@@ -389,16 +389,16 @@ fh_status fh_llama::layers(int s, bool dev_pos) {
         const float *qp, *kp, *vp;
         int64_t row;
         if (l.qkv) {
-            if (!qkv_done) FH_TRY(fh_qmatmul(l.qkv, m->xn, s, m->qkv));
+            if (!qkv_done) FH_TRY(fh_qmatmul_prompt(l.qkv, m->xn, s, m->qkv));
             row = QD + 2 * KD;
             qp = m->qkv;
             kp = m->qkv + QD;
             vp = m->qkv + QD + KD;
         } else {
             float *qb = m->qkv, *kb2 = m->qkv + (size_t)s * QD, *vb = kb2 + (size_t)s * KD;
-            FH_TRY(fh_qmatmul(l.wq, m->xn, s, qb));
-            FH_TRY(fh_qmatmul(l.wk, m->xn, s, kb2));
-            FH_TRY(fh_qmatmul(l.wv, m->xn, s, vb));
+            FH_TRY(fh_qmatmul_prompt(l.wq, m->xn, s, qb));
+            FH_TRY(fh_qmatmul_prompt(l.wk, m->xn, s, kb2));
+            FH_TRY(fh_qmatmul_prompt(l.wv, m->xn, s, vb));
             row = 0; // per-tensor strides below
             qp = qb; kp = kb2; vp = vb;
         }
@@ -454,7 +454,7 @@ fh_status fh_llama::layers(int s, bool dev_pos) {
             FH_TRY(fh_transpose_shd(dev, m->att, H, s, hd, m->att_t));
             att_in = m->att_t;
         }
-        if (!wo_done) FH_TRY(fh_qmatmul(l.wo, att_in, s, m->attn_out));
+        if (!wo_done) FH_TRY(fh_qmatmul_prompt(l.wo, att_in, s, m->attn_out));
         if (trace) {
             FH_TRY(trace_probe(m, m->attn_out, s, D, li, "attn_out"));
             FH_TRY(trace_mark(m, 2, li, "wo"));
@@ -483,14 +483,14 @@ fh_status fh_llama::layers(int s, bool dev_pos) {
         } else if (l.gate_up) {
             fh_status st = fh_qmm_frag_swiglu(l.gate_up, m->xn, s, m->act);
             if (st == FH_ERR_UNSUPPORTED) {
-                FH_TRY(fh_qmatmul(l.gate_up, m->xn, s, m->gu)); // [s, 2F]: gate | up per row
+                FH_TRY(fh_qmatmul_prompt(l.gate_up, m->xn, s, m->gu)); // [s, 2F]: gate | up per row
                 // split the halves: silu(gate) * up with row stride 2F
                 st = fh_swiglu_rows(dev, m->gu, s, F, m->act);
             }
             FH_TRY(st);
         } else {
-            FH_TRY(fh_qmatmul(l.gate, m->xn, s, m->gu));
-            FH_TRY(fh_qmatmul(l.up, m->xn, s, m->gu + (size_t)s * F));
+            FH_TRY(fh_qmatmul_prompt(l.gate, m->xn, s, m->gu));
+            FH_TRY(fh_qmatmul_prompt(l.up, m->xn, s, m->gu + (size_t)s * F));
             FH_TRY(fh_swiglu(dev, m->gu, m->gu + (size_t)s * F, m->act, (int64_t)s * F));
         }
         if (trace) FH_TRY(trace_mark(m, 2, li, "ffn_norm+gate_up+swiglu"));
@@ -510,7 +510,7 @@ fh_status fh_llama::layers(int s, bool dev_pos) {
             }
             FH_TRY(st);
         } else {      // raw/mod.rs:1036
-            FH_TRY(fh_qmatmul(l.down, m->act, s, m->ff));
+            FH_TRY(fh_qmatmul_prompt(l.down, m->act, s, m->ff));
             FH_TRY(fh_add3(dev, m->ff, m->attn_out, m->x, m->x, (int64_t)s * D));
         }
         if (trace) {

@@ -12,6 +12,7 @@
 //                  the 16x16 accumulator whose columns are the lane's own weight row.  The min term
 //                  of Q4_K uses the factorisation  y = d*sum_j sc_j*(q.x)_j - dmin*sum_j m_j*(sum x)_j.
 #include "fh_blocks.h"
+#include "fh_qmm_frag.h"
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -398,7 +399,7 @@ static fh_status qmm_check(const fh_qmatrix *q, const void *x, int m, const void
     return FH_OK;
 }
 
-extern "C" fh_status fh_qmatmul(const fh_qmatrix *q, const float *x_dev, int32_t m, float *y_dev) {
+static fh_status qmatmul(const fh_qmatrix *q, const float *x_dev, int32_t m, float *y_dev, bool fragments) {
     FH_TRY(qmm_check(q, x_dev, m, y_dev));
     const int64_t mk = q->dev->opt_matmul_kernel;
     if (q->type == FH_BF16 && mk != 1 && q->dev->opt_matvec_kernel != 1) return fh_launch_bf16_matmul(q, x_dev, 0, m, y_dev);
@@ -407,8 +408,16 @@ extern "C" fh_status fh_qmatmul(const fh_qmatrix *q, const float *x_dev, int32_t
     const bool dense = (q->type == FH_W_F16 || q->type == FH_W_F32) && q->k % 32 == 0;
     // (the 5-bit formats have no batch kernel for 2 .. 16 rows: rows are a launch each up to 12, tiles above)
     const int tile_from = (q->type == FH_Q5_K || q->type == FH_Q5_0) && q->k % 256 == 0 ? 12 : 16;
-    if (((m > tile_from && mk != 1) || mk >= 2) && (!fh_is_plain(q->type) || dense)) return fh_launch_qmatmul_tile(q, x_dev, 0, m, y_dev);
+    if (((m > tile_from && mk != 1) || mk >= 2) && (!fh_is_plain(q->type) || dense)) return fh_launch_qmatmul_tile(q, x_dev, 0, m, y_dev, fragments);
     return fh_launch_qmatvec(q, x_dev, m, y_dev, FH_EPI_NONE, nullptr, nullptr);
+}
+
+extern "C" fh_status fh_qmatmul(const fh_qmatrix *q, const float *x_dev, int32_t m, float *y_dev) {
+    return qmatmul(q, x_dev, m, y_dev, true);
+}
+
+fh_status fh_qmatmul_prompt(const fh_qmatrix *q, const float *x_dev, int m, float *y_dev) {
+    return qmatmul(q, x_dev, m, y_dev, m > FH_SHORT_PROMPT);
 }
 
 extern "C" fh_status fh_qmatmul_add2(const fh_qmatrix *q, const float *x_dev, int32_t m, const float *a_dev,

@@ -1785,7 +1785,7 @@ static fh_status qmm_launch_dense(const fh_qmatrix *q, const _Float16 *xh, const
     return FH_OK;
 }
 
-fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y) {
+fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, bool fragments) {
     fh_device *dev = q->dev;
     const int64_t K = q->k;
     if (q->type == FH_BF16) return fh_launch_bf16_matmul(q, x, x_is_bf16, m, y);
@@ -1794,7 +1794,7 @@ fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf
                 (long long)K);
     FH_REQUIRE((m + 127) / 128 <= 65535, "m = %d too large for one launch", m);
     const int64_t mk = dev->opt_matmul_kernel;
-    if (((uintptr_t)x & 15) == 0 && (mk == 0 ? fh_qmm_frag_pays(q, x_is_bf16, m) : mk == 13 && fh_qmm_frag_supports(q)))
+    if (((uintptr_t)x & 15) == 0 && (mk == 0 ? fragments && fh_qmm_frag_pays(q, x_is_bf16, m) : mk == 13 && fh_qmm_frag_supports(q)))
         return fh_launch_qmm_frag(q, x, x_is_bf16, m, y);
     // planes: xh | xl | rs | (Q4_K: sums of the 32-groups, hi and lo)
     const size_t plane = ((size_t)m * K * 2 + 255) & ~(size_t)255;

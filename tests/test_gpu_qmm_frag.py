@@ -104,3 +104,23 @@ def test_swiglu_epilogue(dev, m, ffn):
         finally:
             dev.set_option("matmul_kernel", 0)
     assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("tokens", [17, 37, 64])
+def test_short_prompts_keep_the_tile_sums(dev, tokens):
+    """What a sampled answer draws follows from the last bits of the cache that its prompt left, so a decoder's short prompts stay
+    on the tile kernels (option 11 takes the fragments nowhere and is the default in all else at these sizes): the same bits."""
+    from kalosm_amd.llama import Model
+
+    cfg = dict(n_layers=2, d_model=512, n_heads=4, n_kv_heads=2, head_dim=128, ffn=1024, vocab=320, ctx=128, eps=1e-5, theta=1e4)
+    model = Model.random_init(dev, cfg, seed=2, sigma=2e-3)
+    prompt = np.random.default_rng(tokens).integers(0, 320, tokens)
+    got = []
+    for option in (0, 11):
+        dev.set_option("matmul_kernel", option)
+        try:
+            got.append(model.forward(prompt, want_hidden=True)[1])
+        finally:
+            dev.set_option("matmul_kernel", 0)
+        model.reset()
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))

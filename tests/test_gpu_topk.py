@@ -37,3 +37,32 @@ def test_layouts(dev, oracle, n, layout):
         got, want = t.top_k_pairs(k), oracle.top_k(x, k)
         assert [g[0] for g in got] == [w[0] for w in want], (k, len(got), len(want))
         assert np.array_equal(np.float32([g[1] for g in got]).view(np.uint32), np.float32([w[1] for w in want]).view(np.uint32))
+
+
+@pytest.mark.parametrize("kind", ["standard", "mirostat2"])
+def test_continuation(dev, oracle, kind):
+    """64 draws in a row on given logits, the state and a window of 20 previous ids (which moves on three times) carried over: the
+    oracle's token at each step whose deciding comparison is not closer than exp and log2 of the two sides differ."""
+    from kalosm_amd.fusor import GpuMirostat2Sampler, GpuMirostat2SamplerParams, GpuStandardSamplerParams
+
+    rng, n = np.random.default_rng(64), 32768
+    sampler, mu, history, near = GpuMirostat2Sampler(dev, 10.0), 10.0, rng.integers(0, n, 20).tolist(), 0
+    for _ in range(64):
+        x = (2.0 * rng.standard_normal(n)).astype(np.float32)
+        x[history[-30:]] += 8.0  # (so that the ids of the window, and some that left it, are candidates)
+        t, u, prev = Tensor.from_slice(dev, x), float(rng.random(dtype=np.float32)), np.array(history[-20:])
+        if kind == "standard":
+            got = t.sample_standard_token(prev, GpuStandardSamplerParams(64, 0.8, 1.3, 0.95, 0.01, u))
+            want = oracle.sample_token(x, 0, 64, 0.8, 1.3, 0.95, 0.01, random=u, previous=prev)
+        else:
+            got = t.sample_mirostat2_token(sampler, prev, GpuMirostat2SamplerParams(64, 0.8, 1.3, 5.0, 0.1, u))
+            want = oracle.sample_token(x, 1, 64, 0.8, 1.3, tau=5.0, eta=0.1, random=u, previous=prev, mu=mu)
+        if want["margin"] > 1e-4:
+            assert got == want["token"]
+        near += want["margin"] <= 1e-4
+        if kind == "mirostat2":
+            if got == want["token"]:
+                assert sampler.mu == pytest.approx(want["mu"], rel=1e-5, abs=1e-5)
+            mu = sampler.mu
+        history.append(got)
+    assert near <= 6

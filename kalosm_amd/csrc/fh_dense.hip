@@ -503,17 +503,24 @@ fh_status fh_rows_to_act(fh_device *dev, int dtype, const float *x, int64_t ldx,
 // ------------------------------------------------------------------------------ decode matvec
 // One wavefront per ROWS weight rows; a lane takes eight consecutive weights (16 bytes) of every 512.  The input is
 // normed once per workgroup into the LDS; f32 products and sums.
-// What bounds the decode products: a plain read of 117 MB takes 19 us on this device, the product 27 us (14336 x 4096) and 22 us
-// (4096 x 14336), 29 and 25 us while the requests were under conditions (which emptied the pipeline every AHEAD pieces).  The rest
-// is the input every workgroup stages: without it the same loops take 5 us less, whether it is requested first, last, behind a
+// What bounds the decode products: a plain read of 117 MB takes 19 us on this device, the product 24 us (14336 x 4096) and 23 us
+// (4096 x 14336).  No request is under a condition, which would empty the pipeline every AHEAD pieces (FhRowStream).  The rest is the
+// input every workgroup stages: without it the same loops take 5 us less, whether it is requested first, last, behind a
 // barrier, rotated or from copies of its own, with 2 to 16 pieces ahead, and with one workgroup per compute unit.
 struct MvSegs { FhMvSeg s[3]; int tiles[3]; int n; };
 
-// XV: 16-byte pieces of the input a thread holds.  Inputs of at most 2048 take two of them and four pieces of the weights ahead:
-// with the four and eight of longer ones, requests past the end repeat the last piece: a matrix of 32768 x 2048 takes 30.2
-// us for 31.2, the four matrices ahead of a layer's mixer 8.7 - 13.8 for 9.6 - 14.4.
+// XV: 16-byte pieces of the input a thread holds, requested ahead of the first weights; 0: the input goes to the LDS in a loop ahead
+// of them.  How much each way has on its way, and which one, is a matter of how many wavefronts there are on a compute unit:
+//   four rows a wavefront (8192 rows of the matrices or more): all workgroups of a matrix of 32768 rows fit the device at once if a
+//     wavefront takes at most 64 registers, so XV = 0 and two pieces of the weights: 32768 x 1024 / 2048 / 4096 in 13.2 / 27.6 /
+//     48.7 us; with the input in registers and four pieces (104 - 122 registers) 17.4 / 30.5 / 54.2.
+//   two rows (from 2048): XV = 0 and four pieces for inputs of 1025 to 4096 - 7000 x 4096 13.3 us, 4096 x 4096 9.1, in registers 15.9
+//     and 10.6.  Shorter ones are a piece a thread (7000 x 1000 4.8 us, the loop 5.1); longer ones leave room for few workgroups
+//     beside their LDS, so registers are free (7000 x 14336 39 us, 4096 x 14336 23; the loop 45 and 27).
+//   one row: in registers (1024 x 4096 5.3 us, 1024 x 14336 7.7), and two pieces of the weights for each of the input's, up to
+//     eight.  Requests past the end repeat the last piece, so more pieces than there are cost time (128 x 1024: 2.1 us, with four 2.5).
 template <int ROWS, int XV>
-__global__ __launch_bounds__(256) void k_matvec_norm(const float *__restrict__ x, int k, int kp, const float *__restrict__ nw,
+__global__ __launch_bounds__(256, XV ? 1 : 8) void k_matvec_norm(const float *__restrict__ x, int k, int kp, const float *__restrict__ nw,
                                                      float eps, MvSegs segs, float *__restrict__ norm_out) {
     extern __shared__ __attribute__((aligned(16))) float xs[]; // [kp]
     __shared__ float red[4];
@@ -522,57 +529,75 @@ __global__ __launch_bounds__(256) void k_matvec_norm(const float *__restrict__ x
     while (si + 1 < segs.n && tile >= segs.tiles[si]) tile -= segs.tiles[si++];
     const FhMvSeg seg = segs.s[si];
     const int row0 = (tile * 4 + wave) * ROWS;
-    FhRowStream<ROWS, 16 / ROWS < 2 * XV ? 16 / ROWS : 2 * XV> rows;
+    FhRowStream<ROWS, XV == 0 ? 8 / ROWS : XV < 4 ? 2 * XV : 8> rows;
 #pragma unroll
     for (int r = 0; r < ROWS; r++) rows.w[r] = seg.w + (int64_t)(row0 + r < seg.n ? row0 + r : seg.n - 1) * kp;
-    // The input is requested first (it comes out of the L2 while the weights are on their way: requests are waited for in order),
-    // then the first weights, then the input is normed.
-    if (!(k & 3) && k <= 1024 * XV) {
-        float4 v[XV], w[XV];
+    float ss = 0.f;
+    const auto scale = [&]() { // of the norm, from the threads' sums of squares
+        ss = fh_wave_sum(ss);
+        if (lane == 0) red[wave] = ss;
+        __syncthreads();
+        return 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
+    };
+    if (XV && !(k & 3)) { // (k is at most 1024 XV)
+        constexpr int NX = XV ? XV : 1, NW = XV <= 4 ? NX : 1; // (long inputs read the norm's weights when they are used)
+        float4 v[NX], w[NW];
         const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int j = 0; j < XV; j++) {
+        for (int j = 0; j < NX; j++) {
             const int i = (tid + 256 * j) * 4, at = i < k ? i : 0;
             v[j] = *(const float4 *)(x + at);
-            w[j] = nw ? *(const float4 *)(nw + at) : zero;
+            if (NW == NX) w[j] = nw ? *(const float4 *)(nw + at) : zero;
         }
         __builtin_amdgcn_sched_barrier(0);
         rows.start(kp);
         __builtin_amdgcn_sched_barrier(0);
         float inv = 1.f;
         if (nw) {
-            float ss = 0.f;
 #pragma unroll
-            for (int j = 0; j < XV; j++)
+            for (int j = 0; j < NX; j++)
                 if ((tid + 256 * j) * 4 < k) ss = fmaf(v[j].x, v[j].x, fmaf(v[j].y, v[j].y, fmaf(v[j].z, v[j].z, fmaf(v[j].w, v[j].w, ss))));
-            ss = fh_wave_sum(ss);
-            if (lane == 0) red[wave] = ss;
-            __syncthreads();
-            inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
+            inv = scale();
         }
 #pragma unroll
-        for (int j = 0; j < XV; j++) {
+        for (int j = 0; j < NX; j++) {
             const int i = (tid + 256 * j) * 4;
             if (i >= kp) continue;
             float4 o = i < k ? v[j] : zero;
-            if (nw && i < k) o = make_float4(o.x * inv * w[j].x, o.y * inv * w[j].y, o.z * inv * w[j].z, o.w * inv * w[j].w);
+            if (nw && i < k) {
+                const float4 m = NW == NX ? w[j % NW] : *(const float4 *)(nw + i);
+                o = make_float4(o.x * inv * m.x, o.y * inv * m.y, o.z * inv * m.z, o.w * inv * m.w);
+            }
             *(float4 *)(xs + i) = o;
         }
     } else {
-        rows.start(kp);
-        float ss = 0.f;
-        for (int i = tid; i < kp; i += 256) {
-            const float v = i < k ? x[i] : 0.f;
-            ss = fmaf(v, v, ss);
-            xs[i] = v;
+        if (!(k & 3)) {
+#pragma unroll 8
+            for (int i = tid * 4; i < kp; i += 1024) {
+                const float4 v = i < k ? *(const float4 *)(x + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+                ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
+                *(float4 *)(xs + i) = v;
+            }
+        } else {
+#pragma unroll 8
+            for (int i = tid; i < kp; i += 256) {
+                const float v = i < k ? x[i] : 0.f;
+                ss = fmaf(v, v, ss);
+                xs[i] = v;
+            }
         }
+        rows.start(kp);
         if (nw) {
-            ss = fh_wave_sum(ss);
-            if (lane == 0) red[wave] = ss;
-            __syncthreads();
-            const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
+            const float inv = scale();
+            if (!(k & 3))
+#pragma unroll 2
+                for (int i = tid * 4; i < k; i += 1024) {
+                    const float4 v = *(const float4 *)(xs + i), m = *(const float4 *)(nw + i);
+                    *(float4 *)(xs + i) = make_float4(v.x * inv * m.x, v.y * inv * m.y, v.z * inv * m.z, v.w * inv * m.w);
+                }
+            else
 #pragma unroll 4
-            for (int i = tid; i < k; i += 256) xs[i] = xs[i] * inv * nw[i];
+                for (int i = tid; i < k; i += 256) xs[i] = xs[i] * inv * nw[i];
         }
     }
     __syncthreads();
@@ -612,13 +637,16 @@ fh_status fh_matvec_norm(fh_device *dev, const float *x, int k, const float *w, 
         if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_matvec_norm<ROWS_, XV_>, lds));                    \
         k_matvec_norm<ROWS_, XV_><<<dim3((unsigned)tiles), 256, lds, dev->stream>>>(x, k, kp, w, eps, ms, norm_out);      \
     } while (0)
-    if (k <= 2048) {
-        if (rows == 4) MV_NORM(4, 2);
-        else if (rows == 2) MV_NORM(2, 2);
-        else MV_NORM(1, 2);
-    } else if (rows == 4) MV_NORM(4, 4);
-    else if (rows == 2) MV_NORM(2, 4);
-    else MV_NORM(1, 4);
+    if (rows == 4) MV_NORM(4, 0);
+    else if (rows == 2) {
+        if (k <= 1024) MV_NORM(2, 1);
+        else if (k <= 4096 || k > 16384) MV_NORM(2, 0);
+        else MV_NORM(2, 16);
+    } else if (k <= 1024) MV_NORM(1, 1);
+    else if (k <= 2048) MV_NORM(1, 2);
+    else if (k <= 4096) MV_NORM(1, 4);
+    else if (k <= 16384) MV_NORM(1, 16);
+    else MV_NORM(1, 0);
 #undef MV_NORM
     FH_HIP(hipGetLastError());
     return FH_OK;
@@ -987,6 +1015,11 @@ __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int
         return;
     }
     start();
+    if (!in.y && !(k & 3) && !in.x_out && !in.state && !mu) { // a longer one
+#pragma unroll 8
+        for (int i = tid * 4; i < kp; i += 2048) *(float4 *)(xs + i) = i < k ? *(const float4 *)(in.x + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+        return;
+    }
     float inv = 0.f;
     if (in.y) {
         float ss = 0.f;

@@ -584,25 +584,51 @@ bool fh_qmm_frag_supports(const fh_qmatrix *q) {
     return false;
 }
 
-// Where the fragments pay for being written, against the tile kernels that decode inside the product (us, fragments / tiles):
-//   up to 64 rows those have too few workgroups and decode for few rows: Q4_K f32 4096 x 4096, 32 rows 42 / 150, 28672 x 4096,
-//     64 rows 139 / 173, Q6_K 4096 x 14336, 32 rows 147 / 580, bf16 38 / 140
-//   above, writing the fragments (250 MB for a 28672 x 4096 matrix: 52 us) is the price whatever the rows:
-//     Q4_K f32, 28672 x 4096: 128 rows 160 / 166, 256 rows 195 / 166, 320 rows 280 / 295, 768 rows 427 / 483, 2048 rows 895 / 1189;
-//     4096 x 4096: 256 rows 53 / 48, 320 rows 60 / 63, 768 rows 83 / 116
-//     Q6_K f32, 4096 x 14336: 320 rows 227 / 218, 512 rows 238 / 238, 768 rows 324 / 428, 2048 rows 626 / 891
-//     Q8_0 f32, 14336 x 4096: 512 rows 172 / 179, 768 rows 278 / 283, 2048 rows 539 / 674
-//     the 5-bit formats, which the tiles multiply as split f32 values: Q5_K f32, 4096 x 14336: 128 rows 100 / 106, 512 rows 186 / 249
-//     one activation plane halves the products but not the fragments: Q4_K bf16, 14336 x 4096: 512 rows 113 / 113, 768 rows
-//     184 / 179, 1024 rows 188 / 219, 2048 rows 349 / 415; Q6_K 463 / 480 and Q8_0 (bound by its scaling) 475 / 364 stay
+// Where the fragments pay for being written, against the tile kernels that decode inside the product.  Both were timed for 13 - 64
+// rows of 12 matrices and 129 - 3000 rows of 23, in every format; us, fragments / tiles, at the lines:
+//   Up to 64 rows a tile kernel takes the same time for any matrix whose tiles of 128 rows fit the device at once (32768 rows), the
+//     fragments as long as they are: Q4_K f32, 32 rows, 11008 x 4096 55 / 150, 32768 x 4096 145 / 158, 128256 x 4096 595 / 294;
+//     Q4_0 22528 x 4096 97 / 142, 28672 x 4096 160 / 141; Q6_K, two planes, 16384 x 4096 128 / 166, 28672 x 4096 232 / 166.
+//   Above, they cost 52 us for a 28672 x 4096 matrix whatever the rows (250 MB), and two launches more: narrow matrices need rows
+//     for that (640 rows, Q8_0 f32, 512 x 2048 39 / 33, 1024 x 4096 53 / 59, 2048 x 2048 45 / 55), unless their n is no multiple of
+//     four, which the tile kernels cannot split k for (Q4_0 130 x 14336: 117 / 434).
+//   Few rows (Q4_K f32 257 - 512, Q5_0 129 - 256) are worth it where the tiles leave the device idle: `fill` is what they keep busy
+//     of it, with what they spend on rows past m against tiles of 128.  Q4_K f32, 512 rows: 14336 x 4096 150 / 166,
+//     4096 x 14336 190 / 172; Q5_0 f32, 192 rows: 6144 x 4096 69 / 89, 4096 x 14336 131 / 128.
+//   The 5-bit formats, which the tiles multiply as split f32 values, gain most (Q5_K f32, 4096 x 14336, 512 rows: 190 / 255); one activation
+//     plane halves the products but not the fragments (Q4_K bf16, 14336 x 4096: 768 rows 182 / 180, 2048 rows 369 / 415).
+//   Left on the tiles although the fragments are up to 1.8 times as fast there: 129 - 512 rows of Q4_0, Q8_0 and Q6_K, f32 (6144 x 4096;
+//     4096 x 14336 0.75 - 1.3), 129 - 256 of Q4_K (0.75 - 1.4).  bf16 rows of Q6_K (2048 x 4096 x 14336: 463 / 480, too little) and of
+//     Q8_0 (bound by its scaling, 475 / 364) stay there as well.
+static double tile_fill(const fh_qmatrix *q, int m) {
+    const int64_t cus = q->dev->compute_units, rows = (m + 255) / 256;
+    int64_t tiles = (q->n + 127) / 128 * rows, parts = 1, steps = q->k / 32;
+    while (tiles * parts * 5 < cus * 4 && parts < 8 && steps % (parts * 4) == 0 && steps / (parts * 2) >= 16) parts *= 2; // (as qmm_launch_t)
+    tiles *= parts;
+    return (double)tiles / (double)((tiles + cus - 1) / cus * cus) * (double)((m + 127) / 128) / (double)(2 * rows);
+}
+
 bool fh_qmm_frag_pays(const fh_qmatrix *q, int x_is_bf16, int m) {
     if (!fh_qmm_frag_supports(q)) return false;
-    if (m <= 64) return m > 12 && q->k >= 512;
-    switch (q->type) {
-    case FH_Q5_0: case FH_Q5_K: return m > 128;
-    case FH_Q4_K: return m > (x_is_bf16 ? 768 : 256);
+    const int64_t n = q->n, k = q->k, fits = (int64_t)q->dev->compute_units * 128;
+    const bool four = q->type == FH_Q4_K || q->type == FH_Q5_K; // one plane, a scale per 256
+    if (m <= 64) {
+        if (m <= 12 || k < 512) return false;
+        if (four) return n <= fits;
+        return q->type == FH_Q6_K ? n <= fits * 9 / 16 : n <= (k <= 2048 ? fits : fits * 11 / 16);
     }
-    return !x_is_bf16 && m > 512;
+    const bool any = n % 4 != 0, wide = n >= 2048 || (n >= 1024 && k >= 4096), rows = m > 1024 && (n >= 1024 || (n >= 512 && k >= 4096));
+    switch (q->type) {
+    case FH_Q5_K: return m > 128 && (any || n >= 3072 || (m > 256 && n >= 1024) || (m > 512 && n >= 512) || m > 1024);
+    case FH_Q5_0:
+        if (m <= 256) return m > 128 && (any || (n >= 3072 && n <= fits / 2 && tile_fill(q, m) < 0.9));
+        return any || (m <= 512 ? n >= 3072 : wide || rows);
+    case FH_Q4_K:
+        if (x_is_bf16) return m > 768 && (any || (m <= 1024 ? n >= 2048 && n <= fits / 2 : n >= 512));
+        if (m <= 512) return m > 256 && (any || (n >= 2048 && tile_fill(q, m) < 0.9));
+        return any || n >= (m <= 1024 ? 1024 : 512);
+    }
+    return !x_is_bf16 && m > 512 && (any || wide || rows);
 }
 
 #define FRAG_GO(NW_, NX_, SC_, WGX_) \

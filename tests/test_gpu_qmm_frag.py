@@ -68,6 +68,33 @@ def test_default_dispatch(dev, oracle, ty, m, n, k, act):
     assert np.sqrt(np.mean((got - want) ** 2)) <= 2e-6 * np.sqrt(np.mean(want * want))
 
 
+@pytest.mark.parametrize("ty,act,m,n,k,fragments", [
+    (synth.Q4_K, "f32", 32, 4096, 512, True), (synth.Q4_K, "f32", 32, 32784, 512, False),        # more tiles than fit at once
+    (synth.Q6_K, "bf16", 64, 18432, 512, True), (synth.Q6_K, "bf16", 64, 18448, 512, False),
+    (synth.Q8_0, "f32", 17, 32768, 512, True), (synth.Q8_0, "f32", 17, 22544, 2176, False),
+    (synth.Q8_0, "f32", 600, 512, 2048, False), (synth.Q8_0, "f32", 600, 2048, 512, True),       # narrow matrices
+    (synth.Q8_0, "f32", 600, 130, 2048, True), (synth.Q4_0, "f32", 1100, 1024, 512, True),
+    (synth.Q5_0, "f32", 200, 3072, 512, True), (synth.Q5_0, "f32", 200, 8192, 2048, False),      # few rows, tiles that fill the device
+    (synth.Q4_K, "f32", 300, 2048, 512, True), (synth.Q4_K, "f32", 512, 8192, 2048, False),
+    (synth.Q4_K, "bf16", 800, 1024, 512, False), (synth.Q4_K, "bf16", 800, 2048, 512, True),
+    (synth.Q5_K, "bf16", 200, 2048, 512, False), (synth.Q5_K, "bf16", 200, 3072, 512, True),
+])
+def test_rule(dev, ty, act, m, n, k, fragments):
+    """Both sides of the dispatch's lines: the bits of the fragments (option 13) or those of the tiles (11), which are different."""
+    q = QMatrix.from_raw_bytes(dev, (n, k), synth.random_weight(ty, n, k, seed=n, sigma=2e-3), ty)
+    x = synth.random_activation(m, k, seed=m)
+    xt = Tensor.from_slice(dev, x) if act == "f32" else Tensor.from_slice(dev, synth.to_bf16_bits(x), dtype="bf16")
+    got = {}
+    for option in (0, 11, 13):
+        dev.set_option("matmul_kernel", option)
+        try:
+            got[option] = xt.q_mat_mul(q).as_slice().view(np.uint32)
+        finally:
+            dev.set_option("matmul_kernel", 0)
+    assert not np.array_equal(got[11], got[13])
+    assert np.array_equal(got[0], got[13 if fragments else 11])
+
+
 @pytest.mark.parametrize("ty", [synth.Q4_K, synth.Q6_K, synth.Q8_0], ids=lambda t: synth.TYPE_NAMES[t])
 def test_rows_are_independent(dev, oracle, ty):
     """Zeros stay zero, a power of two passes through exactly, and an infinity or a NaN stays in its row."""

@@ -597,16 +597,15 @@ __device__ __forceinline__ void topk_sample(const uint64_t *s, const float *w, i
 // Bitonic sort, descending, of the 1024 keys of a workgroup of 512: thread t holds those at
 // positions 2t and 2t + 1 (which input lands where does not matter).  Partners at distance 1 are in its own registers, up to
 // distance 64 in its wavefront (lane exchange), beyond that in another wavefront (through the LDS, two buffers of 1024 in turn
-// so that one barrier per stage is enough).  The sorted keys end in s.
+// so that one barrier per stage is enough).  The sorted keys end in s.  Written out (55 stages): 1048577 logits and 64 candidates
+// take 81 us with the launches of the call, as loops 91.
 __device__ __forceinline__ void topk_sort(uint64_t (&kk)[2], uint64_t *s) {
     const int tid = threadIdx.x;
     int flip = 0;
-    // loops, not 55 stages written out: a kernel that runs once a step finds no instruction in the cache, and fetching straight
-    // code takes longer than running it
-#pragma unroll 1
+#pragma unroll
     for (int size = 2; size <= 1024; size <<= 1) {
         const bool down = ((2 * tid) & size) == 0; // this run is sorted descending
-#pragma unroll 1
+#pragma unroll
         for (int m = size >> 2; m > 0; m >>= 1) { // distance in threads
             uint64_t o[2];
             if (m <= 32) {
@@ -718,7 +717,9 @@ __global__ __launch_bounds__(512) void k_topk_pass(const float *__restrict__ x, 
 // What is left are chains of memory and LDS latencies.  k_topk_keys writes the keys and the largest key of every 64.
 // The k-th largest of those maxima bounds the k-th largest key from below, since k lists hold one at least as large, so one
 // workgroup finds (nearly) that maximum by counting, gathers the keys above it from the lists whose maximum is - about k for
-// logits in any order - and sorts only them.
+// logits in any order - and sorts only them.  Where that leaves more than 1024 (not many more lists than candidates, or logits in rising
+// order), it counts the keys of those lists in the same way: 256 candidates of 20000 / 32768 logits take 69 / 71 us with the launches
+// of the call, the three sorts 80 / 79.  Slower than those are 256 candidates of sorted logits (32768: 90 / 79) and equal ones.
 __global__ __launch_bounds__(1024) void k_topk_keys(const float *__restrict__ x, int64_t n, TopkProc proc, uint64_t *__restrict__ keys,
                                                      uint64_t *__restrict__ list_max) {
     __shared__ uint32_t s_prev[64];
@@ -734,33 +735,33 @@ __global__ __launch_bounds__(1024) void k_topk_keys(const float *__restrict__ x,
     if ((threadIdx.x & 63) == 0) list_max[idx >> 6] = key;
 }
 
-__global__ __launch_bounds__(512) void k_topk_pick(const float *__restrict__ x, const uint64_t *__restrict__ keys,
-                                                   const uint64_t *list_max, int lists, int k, uint32_t *__restrict__ ids_out,
-                                                   float *__restrict__ vals_out, uint32_t *__restrict__ found_out, TopkProc proc,
-                                                   TopkSample samp) {
-    __shared__ uint64_t s[2048];
-    __shared__ uint32_t hist[2048];
-    __shared__ float s_w[256];
-    __shared__ uint32_t s_sum[8], s_bin, s_above, s_lists, s_count;
+// A bound that at least k of the n values at(0) .. reach and, unless equal ones do, at most `limit` (of k or more; 0 where there
+// are no more than that).  Eleven bits a round from the top: `prefix` holds the bits so far, `above` values are above all that
+// start with it, `in` start with it.  A round that tells none of them apart (equal logits: keys that differ in the id) is followed by
+// a pass that finds the next bit in which they differ.
+template <typename F>
+__device__ __forceinline__ uint64_t topk_bound(F at, int n, uint32_t k, uint32_t limit, uint32_t *hist, uint32_t *s_sum, uint32_t *s_at) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const TopkState state = topk_state(samp);
-    // the threshold, eleven bits a round from the top: `prefix` holds the bits so far, `above` maxima are above all that start
-    // with it, `in` start with it; done once the maxima at or above the prefix are at most 2 k (or the bits are used up)
     uint64_t prefix = 0;
-    uint32_t above = 0, in = (uint32_t)lists;
+    uint32_t above = 0, in = (uint32_t)n;
     int shift = 64;
-    while (shift > 0 && above + in > 2u * (uint32_t)k) {
+    while (shift > 0 && above + in > limit) {
         const int bits = shift < 11 ? shift : 11;
 #pragma unroll 1
         for (int i = tid; i < 2048; i += 512) hist[i] = 0;
         __syncthreads();
 #pragma unroll 1
-        for (int i = tid; i < lists; i += 512) {
-            const uint64_t m = list_max[i];
-            if (shift == 64 || (m >> shift) == (prefix >> shift)) atomicAdd(&hist[(m >> (shift - bits)) & ((1u << bits) - 1)], 1u);
+        for (int i0 = tid; i0 < n; i0 += 2048) { // (four on their way)
+            uint64_t m[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) m[j] = at(i0 + 512 * j < n ? i0 + 512 * j : i0);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (i0 + 512 * j < n && (shift == 64 || (m[j] >> shift) == (prefix >> shift)))
+                    atomicAdd(&hist[(m[j] >> (shift - bits)) & ((1u << bits) - 1)], 1u);
         }
         __syncthreads();
-        // thread t owns the bins 2047 - 4t .. 2044 - 4t: how many maxima lie above them
+        // thread t owns the bins 2047 - 4t .. 2044 - 4t: how many values lie above them
         uint32_t own[4], sum = 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) sum += own[j] = hist[2047 - 4 * tid - j];
@@ -771,96 +772,132 @@ __global__ __launch_bounds__(512) void k_topk_pick(const float *__restrict__ x, 
             if (lane >= o) run += v;
         }
         if (lane == 63) s_sum[wave] = run;
-        if (tid == 0) s_bin = 0xFFFFFFFFu;
         __syncthreads();
         uint32_t before = above + run - sum;
 #pragma unroll 1
         for (int w = 0; w < wave; w++) before += s_sum[w];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            if (before < (uint32_t)k && before + own[j] >= (uint32_t)k) s_bin = 2047 - 4 * tid - j, s_above = before; // one thread at most
+            if (before < k && before + own[j] >= k) s_at[0] = 2047 - 4 * tid - j, s_at[1] = before; // one thread: limit is k or more
             before += own[j];
         }
         __syncthreads();
-        // (there are more than 2 k maxima at or above the prefix, so the k-th is in one of the bins)
-        prefix |= (uint64_t)s_bin << (shift - bits);
-        above = s_above;
-        in = hist[s_bin];
+        const bool none = hist[s_at[0]] == in;
+        prefix |= (uint64_t)s_at[0] << (shift - bits);
+        above = s_at[1];
+        in = hist[s_at[0]];
         shift -= bits;
         __syncthreads();
+        if (none && shift > 0 && above + in > limit) {
+            uint64_t some = 0, all = ~0ull; // bits of any and of all of them
+            if (tid < 4) hist[tid] = tid < 2 ? 0u : ~0u;
+            __syncthreads();
+#pragma unroll 4
+            for (int i = tid; i < n; i += 512) {
+                const uint64_t m = at(i);
+                if ((m >> shift) == (prefix >> shift)) some |= m, all &= m;
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) some |= __shfl_xor(some, o), all &= __shfl_xor(all, o);
+            if (lane == 0) {
+                atomicOr(&hist[0], (uint32_t)some), atomicOr(&hist[1], (uint32_t)(some >> 32));
+                atomicAnd(&hist[2], (uint32_t)all), atomicAnd(&hist[3], (uint32_t)(all >> 32));
+            }
+            __syncthreads();
+            some = hist[0] | (uint64_t)hist[1] << 32, all = hist[2] | (uint64_t)hist[3] << 32;
+            shift = some == all ? 0 : 64 - __clzll((long long)(some ^ all));
+            prefix = some >> (shift & 63) << (shift & 63); // (shift is 53 at most)
+            __syncthreads();
+        }
     }
-    const uint64_t least = prefix > 1 ? prefix : 1; // 0: no key
-    if (tid == 0) s_lists = s_count = 0;
+    return prefix;
+}
+
+__global__ __launch_bounds__(512) void k_topk_pick(const float *__restrict__ x, const uint64_t *__restrict__ keys,
+                                                   const uint64_t *list_max, int lists, int k, uint32_t *__restrict__ ids_out,
+                                                   float *__restrict__ vals_out, uint32_t *__restrict__ found_out, TopkProc proc,
+                                                   TopkSample samp) {
+    __shared__ uint64_t s[2048];
+    __shared__ uint32_t hist[2048], which[512];
+    __shared__ float s_w[256];
+    __shared__ uint32_t s_sum[8], s_at[2], s_lists, s_count;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const TopkState state = topk_state(samp);
+    // the maxima that count: at most 2 k, a good half of them where there are few (fewer keys are above the larger ones)
+    const uint32_t limit = max(k, min(2 * k, lists / 2));
+    uint64_t least = topk_bound([&](int i) { return list_max[i]; }, lists, (uint32_t)k, limit, hist, s_sum, s_at);
+    if (least == 0) least = 1; // 0: no key
+    if (tid == 0) s_lists = 0;
     __syncthreads();
-    // the lists that count (at most 2 k = 512: their numbers take the place of the histogram) and their keys
+    // the lists that count (at most 2 k = 512) and their keys
 #pragma unroll 1
     for (int i = tid; i < lists; i += 512)
-        if (list_max[i] >= least) hist[atomicAdd(&s_lists, 1u)] = (uint32_t)i;
+        if (list_max[i] >= least) which[atomicAdd(&s_lists, 1u)] = (uint32_t)i;
     __syncthreads();
     const int n_lists = (int)s_lists;
-    // (twelve lists a wavefront in flight: one after the other, the gather of 64 candidates took 4 us)
+    const auto gather = [&]() { // (twelve lists a wavefront in flight: one after the other, the gather of 64 candidates took 4 us)
+        if (tid == 0) s_count = 0;
+        __syncthreads();
 #pragma unroll 1
-    for (int j0 = 12 * wave; j0 < n_lists; j0 += 96) {
-        uint64_t key[12], in[12];
-        uint32_t total = 0;
+        for (int j0 = 12 * wave; j0 < n_lists; j0 += 96) {
+            uint64_t key[12], in[12];
+            uint32_t total = 0;
 #pragma unroll
-        for (int j = 0; j < 12; j++) key[j] = keys[(int64_t)hist[j0 + j < n_lists ? j0 + j : j0] * 64 + lane];
+            for (int j = 0; j < 12; j++) key[j] = keys[(int64_t)which[j0 + j < n_lists ? j0 + j : j0] * 64 + lane];
 #pragma unroll
-        for (int j = 0; j < 12; j++) {
-            in[j] = __ballot(key[j] >= least && j0 + j < n_lists);
-            total += (uint32_t)__popcll(in[j]);
+            for (int j = 0; j < 12; j++) {
+                in[j] = __ballot(key[j] >= least && j0 + j < n_lists);
+                total += (uint32_t)__popcll(in[j]);
+            }
+            uint32_t at = 0;
+            if (lane == 0) at = atomicAdd(&s_count, total);
+            at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+            for (int j = 0; j < 12; j++) {
+                const uint32_t mine = at + (uint32_t)__popcll(in[j] & ((1ull << lane) - 1));
+                if ((in[j] >> lane & 1) && mine < 1024) s[mine] = key[j];
+                at += (uint32_t)__popcll(in[j]);
+            }
         }
-        uint32_t at = 0;
-        if (lane == 0) at = atomicAdd(&s_count, total);
-        at = __builtin_amdgcn_readfirstlane(at);
-#pragma unroll
-        for (int j = 0; j < 12; j++) {
-            const uint32_t mine = at + (uint32_t)__popcll(in[j] & ((1ull << lane) - 1));
-            if ((in[j] >> lane & 1) && mine < 1024) s[mine] = key[j];
-            at += (uint32_t)__popcll(in[j]);
-        }
+        __syncthreads();
+        return (int)s_count;
+    };
+    int count = least > 1 || n_lists <= 16 ? gather() : n_lists * 64; // (all lists are there: more than 1024)
+    if (count > 1024) { // (no two keys are equal, so the second bound leaves 1024 at most)
+        least = topk_bound([&](int i) { return keys[(int64_t)which[i >> 6] * 64 + (i & 63)]; }, n_lists * 64, (uint32_t)k, 1024u, hist, s_sum, s_at);
+        if (least == 0) least = 1;
+        count = gather();
+    }
+    // A key's place is the number of larger ones: counted by several threads a key where there are few.  For 128 keys 0.6 us (the
+    // 28 stages of a sort 4.3), for 1024 40, so what is far more than k is cut down first.
+    uint64_t *from = s, *to = s + 1024;
+    const uint32_t most = max(k + k / 4, 160);
+    if (2 * count > 3 * (int)most) {
+        const uint64_t bound = topk_bound([&](int i) { return s[i]; }, count, (uint32_t)k, most, hist, s_sum, s_at);
+        if (tid == 0) s_count = 0;
+        __syncthreads();
+        for (int i = tid; i < count; i += 512)
+            if (s[i] >= bound) s[1024 + atomicAdd(&s_count, 1u)] = s[i];
+        __syncthreads();
+        count = (int)s_count, from = s + 1024, to = s;
+    }
+    int per = 64; // keys side by side
+    while (per < count && per < 512) per <<= 1;
+    const int parts = 512 / per, part = tid / per;
+    for (int i = tid; i < 1024; i += 512) hist[i] = 0, to[i] = 0;
+    __syncthreads();
+#pragma unroll 1
+    for (int i = tid & (per - 1); i < count; i += per) {
+        const uint64_t mine = from[i];
+        uint32_t larger = 0;
+#pragma unroll 4
+        for (int j = part; j < count; j += parts) larger += from[j] > mine;
+        atomicAdd(&hist[i], larger);
     }
     __syncthreads();
-    const int count = (int)s_count;
-    if (count <= 1024) {
-        // A key's place is the number of larger ones (no two are equal): counted by several threads a key where there are few.
-        // For 128 keys 0.6 us, the 28 stages of the sort 4.3.
-        int per = 64; // keys side by side
-        while (per < count && per < 512) per <<= 1;
-        const int parts = 512 / per, part = tid / per;
-        for (int i = tid; i < 1024; i += 512) hist[i] = 0, s[1024 + i] = 0;
-        __syncthreads();
-#pragma unroll 1
-        for (int i = tid & (per - 1); i < count; i += per) {
-            const uint64_t mine = s[i];
-            uint32_t larger = 0;
-#pragma unroll 4
-            for (int j = part; j < count; j += parts) larger += s[j] > mine;
-            atomicAdd(&hist[i], larger);
-        }
-        __syncthreads();
-        for (int i = tid; i < count; i += 512) s[1024 + hist[i]] = s[i];
-        __syncthreads();
-        topk_finish(s + 1024, s_w, k, x, ids_out, vals_out, found_out, proc, samp, state);
-        return;
-    }
-    // logits in rising order, or equal: the best k so far and twelve lists at a time
-#pragma unroll 1
-    for (int j0 = 0; j0 < n_lists; j0 += 12) {
-        uint64_t kk[2];
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int i = 2 * tid + h, j = j0 + ((i - 256) >> 6);
-            kk[h] = 0;
-            if (i < 256) {
-                if (j0 > 0 && i < k) kk[h] = s[i];
-            } else if (j < n_lists)
-                kk[h] = keys[(int64_t)hist[j] * 64 + ((i - 256) & 63)];
-        }
-        __syncthreads();
-        topk_sort(kk, s);
-    }
-    topk_finish(s, s_w, k, x, ids_out, vals_out, found_out, proc, samp, state);
+    for (int i = tid; i < count; i += 512) to[hist[i]] = from[i];
+    __syncthreads();
+    topk_finish(to, s_w, k, x, ids_out, vals_out, found_out, proc, samp, state);
 }
 
 static fh_status topk_run(fh_device *dev, const float *x_dev, int64_t count, int32_t k, uint32_t *ids_dev,

@@ -28,9 +28,10 @@ def _logits(layout, n, rng):
     return x
 
 
-@pytest.mark.parametrize("n", [1025, 4097, 32768, 131073, 1 << 20, (1 << 20) + 1])
+@pytest.mark.parametrize("n", [1025, 4097, 8192, 16385, 20000, 32768, 131073, 1 << 20, (1 << 20) + 1])
 @pytest.mark.parametrize("layout", ["rising", "one_list", "spread", "equal", "few", "none", "close"])
 def test_layouts(dev, oracle, n, layout):
+    """Up to 256 candidates of 32 lists or more: fewer lists than candidates, as many, a few more, far more."""
     x = _logits(layout, n, np.random.default_rng(n))
     t = Tensor.from_slice(dev, x)
     for k in (1, 2, 63, 200, 256):

@@ -439,11 +439,16 @@ fh_status fh_gemm(fh_device *dev, int dtype, int epi, const FhGemm &g) {
         const int64_t cus = dev->compute_units, wn = (g.n + 255) / 256;
         // The wide kernel from three quarters of a workgroup per compute unit on (below, the 128 x 128 and 128 x 64 tiles have more of
         // them): prompts of 2048 / 1000 / 512 tokens through the four Zovovik layers of width 4096 took 5.9 / 4.3 / 3.2 ms with
-        // this line and 7.2 / 4.7 / 3.4 ms without the kernel.  matmul_kernel = 3: never, 4: always where its row tiles fit.
+        // this line and 7.2 / 4.7 / 3.4 ms without the kernel.  matmul_kernel = 3: never, 4: always where its row tiles fit, 14: the form with
+        // 128 activation rows.
         const int64_t opt = dev->opt_matmul_kernel;
         if (opt != 3) {
-            if (!g.tiles && (opt == 4 || wn * ((g.m + 255) / 256) * 4 >= cus * 3)) return gemm_wide<256>(dev, epi, g);
-            if (g.tiles ? g.tile_rows == 128 && (opt == 4 || wn * g.max_tiles >= cus) : wn * ((g.m + 127) / 128) * 4 >= cus * 3)
+            // A round of workgroups with 128 activation rows takes two thirds of one with 256 (67 / 101 us at 4096 columns), so they
+            // are the better ones where the tiles of 256 just miss a round: 14336 x 4096, 1025 rows 139 / 202 us (128 x 128: 156).
+            const int64_t t256 = wn * ((g.m + 255) / 256), t128 = wn * ((g.m + 127) / 128);
+            const bool tall = t256 * 4 >= cus * 3 && (t128 + cus - 1) / cus * 2 >= (t256 + cus - 1) / cus * 3;
+            if (!g.tiles && opt != 14 && (opt == 4 || tall)) return gemm_wide<256>(dev, epi, g);
+            if (g.tiles ? g.tile_rows == 128 && (opt == 4 || opt == 14 || wn * g.max_tiles >= cus) : opt == 14 || t128 * 4 >= cus * 3)
                 return gemm_wide<128>(dev, epi, g);
         }
         const int tn = (g.n + 127) / 128;

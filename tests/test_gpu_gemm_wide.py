@@ -11,17 +11,18 @@ from kalosm_amd.fusor import QMatrix, Tensor
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 1, 64), (256, 256, 64), (257, 255, 128), (300, 513, 192), (511, 272, 1024), (40, 1030, 4096),
+@pytest.mark.parametrize("option", [4, 14])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 64), (128, 256, 128), (129, 257, 192), (256, 256, 64), (257, 255, 128), (300, 513, 192), (511, 272, 1024), (40, 1030, 4096),
                                    (700, 600, 1000)])
-def test_wide_product(dev, m, n, k):
-    """Tiles exactly full and one row or column past that, one slab of k, k that is not a multiple of 64; option 4 takes the
-    kernel whatever the size."""
+def test_wide_product(dev, m, n, k, option):
+    """Tiles exactly full and one row or column past that, fewer slabs of k than buffers, k that is not a multiple of 64; options 4 and
+    14 take the forms with 256 and 128 activation rows whatever the size."""
     rng = np.random.default_rng(m + n + k)
     w = synth.to_bf16_bits(rng.standard_normal((n, k)).astype(np.float32))
     x = synth.to_bf16_bits(rng.standard_normal((m, k)).astype(np.float32))
     q = QMatrix.from_raw_bytes(dev, (n, k), w, synth.W_BF16)
     out = Tensor.filled_bytes(dev, (m, n), 0xFF)
-    dev.set_option("matmul_kernel", 4)
+    dev.set_option("matmul_kernel", option)
     try:
         got = Tensor.from_slice(dev, x, dtype="bf16").q_mat_mul(q, out=out).as_slice().astype(np.float64)
     finally:

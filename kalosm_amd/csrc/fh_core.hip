@@ -104,7 +104,7 @@ extern "C" fh_status fh_malloc(fh_device *dev, size_t bytes, void **out_dev) {
     *out_dev = nullptr;
     if (bytes == 0) bytes = 16;
     FH_HIP(hipSetDevice(dev->ordinal));
-    FH_HIP(hipMalloc(out_dev, bytes));
+    FH_HIP(fh_dev_malloc(dev, out_dev, bytes));
     return FH_OK;
 }
 
@@ -170,22 +170,55 @@ extern "C" fh_status fh_timer_stop(fh_device *dev, float *elapsed_ms) {
     return FH_OK;
 }
 
+hipError_t fh_dev_malloc(fh_device *dev, void **ptr, size_t bytes) {
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e == hipErrorOutOfMemory && dev->frag_buf && !dev->capturing) {
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(dev->stream);
+        (void)hipFree(dev->frag_buf);
+        dev->frag_buf = nullptr;
+        dev->frag_cap = 0;
+        dev->frag_gen++;
+        e = hipMalloc(ptr, bytes);
+    }
+    if (e != hipSuccess) (void)hipGetLastError(); // the caller has it; the next launch is not to find it
+    return e;
+}
+
+// What could not be allocated leaves the buffer empty (the graphs that hold its address are void either way).
+static hipError_t scratch_grow(fh_device *dev, void **buf, size_t *cap, size_t need) {
+    if (dev->opt_scratch_limit > 0 && need > (size_t)dev->opt_scratch_limit) return hipErrorOutOfMemory;
+    if (*buf) {
+        hipError_t e = hipStreamSynchronize(dev->stream);
+        if (e == hipSuccess) e = hipFree(*buf);
+        if (e != hipSuccess) return e;
+        *buf = nullptr;
+        *cap = 0;
+    }
+    if (buf == &dev->frag_buf) dev->frag_gen++;
+    else dev->scratch_gen++;
+    const size_t want = need < (1u << 20) ? (1u << 20) : need;
+    const hipError_t e = fh_dev_malloc(dev, buf, want);
+    if (e == hipSuccess) *cap = want;
+    else *buf = nullptr;
+    return e;
+}
+
 fh_status fh_dev_scratch(fh_device *dev, void **buf, size_t *cap, size_t need) {
     if (*cap >= need) return FH_OK;
     if (dev->capturing)
         FH_FAIL(FH_ERR_INVALID, "a captured call needs %zu bytes of scratch but only %zu are allocated: run the "
                                 "sequence once eagerly before capturing it", need, *cap);
-    if (*buf) {
-        FH_HIP(hipStreamSynchronize(dev->stream));
-        FH_HIP(hipFree(*buf));
-        *buf = nullptr;
-        *cap = 0;
-    }
-    size_t want = need < (1u << 20) ? (1u << 20) : need;
-    FH_HIP(hipMalloc(buf, want));
-    *cap = want;
-    dev->scratch_gen++;
+    FH_HIP(scratch_grow(dev, buf, cap, need));
     return FH_OK;
+}
+
+bool fh_dev_scratch_try(fh_device *dev, void **buf, size_t *cap, size_t need) {
+    if (*cap >= need) return true;
+    if (dev->capturing) return false;
+    if (scratch_grow(dev, buf, cap, need) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
 }
 
 fh_status fh_kernel_lds(fh_device *dev, const void *kernel, size_t bytes) {
@@ -223,6 +256,7 @@ extern "C" fh_status fh_set_option(fh_device *dev, const char *key, int64_t valu
     else if (!strcmp(key, "down_tiles")) dev->opt_down_tiles = value;
     else if (!strcmp(key, "deterministic")) dev->opt_deterministic = value;
     else if (!strcmp(key, "recurrent_kernel")) dev->opt_recurrent_kernel = value;
+    else if (!strcmp(key, "scratch_limit")) dev->opt_scratch_limit = value;
     else if (!strcmp(key, "step_eager")) dev->opt_step_eager = value;
     else if (!strcmp(key, "trace_nan")) dev->opt_trace_nan = value;
     else if (!strcmp(key, "trace_timing")) dev->opt_trace_timing = value;
@@ -236,7 +270,8 @@ struct fh_graph {
     fh_device *dev = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    uint64_t scratch_gen = 0; // dev->scratch_gen when the capture ended
+    uint64_t scratch_gen = 0, frag_gen = 0; // the device's when the capture ended
+    bool frag = false;                      // a kernel of it holds the address of frag_buf
 };
 
 extern "C" fh_status fh_graph_begin(fh_device *dev) {
@@ -245,6 +280,7 @@ extern "C" fh_status fh_graph_begin(fh_device *dev) {
     FH_HIP(hipStreamSynchronize(dev->stream));
     FH_HIP(hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
     dev->capturing = true;
+    dev->frag_captured = false;
     return FH_OK;
 }
 
@@ -266,13 +302,15 @@ extern "C" fh_status fh_graph_end(fh_device *dev, fh_graph **out) {
     r->graph = g;
     r->exec = ex;
     r->scratch_gen = dev->scratch_gen;
+    r->frag_gen = dev->frag_gen;
+    r->frag = dev->frag_captured;
     *out = r;
     return FH_OK;
 }
 
 extern "C" fh_status fh_graph_launch(fh_graph *g) {
     FH_REQUIRE(g && g->exec, "NULL graph");
-    if (g->scratch_gen != g->dev->scratch_gen)
+    if (g->scratch_gen != g->dev->scratch_gen || (g->frag && g->frag_gen != g->dev->frag_gen))
         FH_FAIL(FH_ERR_INVALID, "the device's scratch buffers were reallocated by a larger call since this graph was "
                                 "captured; its kernels hold the old addresses: capture it again");
     FH_HIP(hipGraphLaunch(g->exec, g->dev->stream));

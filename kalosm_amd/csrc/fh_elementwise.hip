@@ -1010,7 +1010,7 @@ extern "C" fh_status fh_kvcache_create(fh_device *dev, int32_t layers, int32_t k
     c->head_dim = head_dim;
     c->max_len = max_len;
     c->dtype = dtype;
-    hipError_t e = hipMalloc((void **)&c->len_dev, 256);
+    hipError_t e = fh_dev_malloc(dev, (void **)&c->len_dev, 256);
     if (e != hipSuccess) {
         delete c;
         FH_FAIL(FH_ERR_OOM, "hipMalloc failed: %s", hipGetErrorString(e));
@@ -1068,8 +1068,8 @@ fh_status fh_kvcache_reserve(fh_kvcache *c, int required) {
     size_t es = fh_dtype_size(c->dtype);
     size_t bytes = (size_t)c->layers * c->kv_heads * cap * c->head_dim * es;
     void *nk = nullptr, *nv = nullptr;
-    FH_HIP(hipMalloc(&nk, bytes));
-    hipError_t e = c->has_v ? hipMalloc(&nv, bytes) : hipSuccess;
+    FH_HIP(fh_dev_malloc(c->dev, &nk, bytes));
+    hipError_t e = c->has_v ? fh_dev_malloc(c->dev, &nv, bytes) : hipSuccess;
     if (e != hipSuccess) {
         (void)hipFree(nk);
         FH_FAIL(FH_ERR_OOM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));

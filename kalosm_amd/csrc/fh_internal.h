@@ -49,11 +49,14 @@ struct fh_device {
     size_t part_cap = 0;
     float *ksplit_buf = nullptr; // partial planes of a k-split prefill matmul
     size_t ksplit_cap = 0;
-    void *frag_buf = nullptr;    // weights of a prompt's product in fragment order, at most 512 MB and their scales
+    // weights of a prompt's product in fragment order and their scales, at most 512 MB; given back when memory runs out
+    void *frag_buf = nullptr;
     size_t frag_cap = 0;
+    uint64_t frag_gen = 0;      // counts its reallocations: graphs that hold its address are few, so it is not part of scratch_gen
+    bool frag_captured = false; // used since fh_graph_begin
     // 64 KB that never moves: partial results of small reductions (argmax)
     void *small_buf = nullptr;
-    // Counts the reallocations of act_buf / part_buf / ksplit_buf / frag_buf.  A captured graph holds their addresses as
+    // Counts the reallocations of act_buf / part_buf / ksplit_buf.  A captured graph holds their addresses as
     // kernel arguments, so whoever keeps a graph records the value at capture and must not replay it after
     // the value has changed.
     uint64_t scratch_gen = 0;
@@ -83,6 +86,7 @@ struct fh_device {
     int64_t opt_fuse_norm = 0;       // 0: decode steps fold rms_norm into the consuming matvec, 1: separate launches
     int64_t opt_deterministic = 0;   // 1: decode steps never accumulate k-split partial sums with float atomics (run-to-run bit-equal)
     int64_t opt_recurrent_kernel = 0; // 0 auto, 1 token by token, 2 chunks of 64 tokens for every portion
+    int64_t opt_scratch_limit = 0;   // > 0: no scratch buffer grows beyond so many bytes (growth fails as without memory)
     int64_t opt_step_eager = 0;      // 1: decode loops launch their steps on the stream (kernel tracers), never a captured graph
     int64_t opt_trace_nan = 0;       // 1: fh_llama_forward probes the residual stream of every layer for NaN / inf
     int64_t opt_trace_timing = 0;    // 1: fh_llama_forward times its layer loop, 2: and every stage of every layer
@@ -91,7 +95,11 @@ struct fh_device {
     int64_t opt_matmul_kernel = 0;   // 0 auto, 1 generic for every m, 2 MFMA tile kernels for every m, 3 / 4 and never / always the 128 x 256 one
 };
 
+// hipMalloc, once more without frag_buf where there is not enough memory
+hipError_t fh_dev_malloc(fh_device *dev, void **ptr, size_t bytes);
 fh_status fh_dev_scratch(fh_device *dev, void **buf, size_t *cap, size_t need);
+// The same for callers that can do without: false, and no error, where `need` bytes cannot be had (or not while capturing).
+bool fh_dev_scratch_try(fh_device *dev, void **buf, size_t *cap, size_t need);
 // Allows the kernel `bytes` of dynamic LDS on this device (hipFuncSetAttribute, once per kernel and device).
 fh_status fh_kernel_lds(fh_device *dev, const void *kernel, size_t bytes);
 fh_status fh_static_scratch_init(fh_device *dev); // with dev->ordinal current

@@ -132,7 +132,7 @@ static fh_status qm_alloc(fh_device *dev, uint32_t type, int64_t n, int64_t k, f
             q->bytes = (size_t)q->n_pad * (size_t)q->recs * 2;
         }
     }
-    hipError_t err = hipMalloc((void **)&q->data, q->bytes + 256); // slack: kernels may prefetch one record ahead
+    hipError_t err = fh_dev_malloc(dev, (void **)&q->data, q->bytes + 256); // slack: kernels may prefetch one record ahead
     if (err != hipSuccess) {
         delete q;
         FH_FAIL(err == hipErrorOutOfMemory ? FH_ERR_OOM : FH_ERR_HIP, "hipMalloc(%zu) failed: %s", q->bytes,
@@ -180,7 +180,7 @@ extern "C" fh_status fh_qmatrix_from_gguf_bytes(fh_device *dev, uint32_t ggml_ty
         return FH_OK;
     }
     uint8_t *staging = nullptr;
-    hipError_t err = hipMalloc((void **)&staging, len);
+    hipError_t err = fh_dev_malloc(dev, (void **)&staging, len);
     if (err != hipSuccess) {
         fh_qmatrix_free(q);
         FH_FAIL(FH_ERR_OOM, "hipMalloc(%zu) for staging failed: %s", len, hipGetErrorString(err));

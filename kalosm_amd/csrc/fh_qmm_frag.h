@@ -4,7 +4,8 @@
 
 bool fh_qmm_frag_supports(const fh_qmatrix *q);
 bool fh_qmm_frag_pays(const fh_qmatrix *q, int x_is_bf16, int m); // and where it is the faster way
-// y[m, n] = x[m, k] . deq(q)^T; x f32 or bf16, rows contiguous and 16-byte aligned.
+// y[m, n] = x[m, k] . deq(q)^T; x f32 or bf16, rows contiguous and 16-byte aligned.  FH_ERR_UNSUPPORTED where the memory for the
+// fragments cannot be had.
 fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y);
 // A decoder's prompts of up to this many tokens stay on the tile kernels.  The fragments are the faster way there (37 tokens and 64
 // sampled ones through four layers of width 2048: 9.4 ms for 11.1) and the closer one (against 64 bits 4e-6 of the logits, the

@@ -539,7 +539,7 @@ __global__ void k_frag_sum(const float *__restrict__ part, int parts, int64_t st
 
 // ------------------------------------------------------------------------------ launches
 template <int NW, int NX, int SC, int FW, int FX, int WGX>
-static fh_status frag_product(fh_device *dev, FragArgs g, bool ask) { // ask: is k in one part?
+static fh_status frag_product(fh_device *dev, FragArgs g, int *ask) { // ask: only into how many parts of k
     typedef FragTile<NW, NX, FW, FX, WGX> Tile;
     constexpr int TW = Tile::TW, TX = Tile::TX, LDS = Tile::STAGES * Tile::STAGE;
     g.tiles_w = (g.n + TW - 1) / TW;
@@ -557,11 +557,13 @@ static fh_status frag_product(fh_device *dev, FragArgs g, bool ask) { // ask: is
         if (p > 1) t += 4.0 + (2.0 * p + 1.0) * g.m * (double)g.n * 4.0 / 4e6;
         if (t < best * 0.97) best = t, parts = p;
     }
-    if (ask || (g.half && parts > 1)) return parts == 1 ? FH_OK : FH_ERR_UNSUPPORTED;
+    if (ask) {
+        *ask = parts;
+        return FH_OK;
+    }
     g.parts = parts;
     float *y = g.y;
-    if (parts > 1) { // whole planes [m][n] of this launch's weight rows
-        FH_TRY(fh_dev_scratch(dev, (void **)&dev->ksplit_buf, &dev->ksplit_cap, (size_t)parts * g.m * g.n * 4));
+    if (parts > 1) { // whole planes [m][n] of this launch's weight rows (qmm_frag has the memory)
         g.y = dev->ksplit_buf;
         g.part_stride = (int64_t)g.m * g.n;
     }
@@ -633,7 +635,7 @@ bool fh_qmm_frag_pays(const fh_qmatrix *q, int x_is_bf16, int m) {
 
 #define FRAG_GO(NW_, NX_, SC_, WGX_) \
     (m <= 64 ? frag_product<NW_, NX_, SC_, 2, 1, 2>(dev, g, ask) : frag_product<NW_, NX_, SC_, 2, 2, WGX_>(dev, g, ask))
-static fh_status frag_go(fh_device *dev, const FragArgs &g, int sc, int wp, int xp, bool ask) {
+static fh_status frag_go(fh_device *dev, const FragArgs &g, int sc, int wp, int xp, int *ask) {
     const int m = g.m;
     if (sc == 32) return xp == 2 ? FRAG_GO(1, 2, 32, 2) : FRAG_GO(1, 1, 32, 2);
     if (wp == 2) return xp == 2 ? FRAG_GO(2, 2, 256, 4) : FRAG_GO(2, 1, 256, 4);
@@ -646,20 +648,24 @@ static fh_status qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int
     const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2, wp = q->type == FH_Q6_K ? 2 : 1;
     const int ext = q->type == FH_Q4_K || q->type == FH_Q5_K ? frag_ext(k, xp) : 0, kf = (k + ext) / 16;
     const int sc = fh_block_elems(q->type);
-    // weights: as many rows at a time as 512 MB of fragments hold
-    const int64_t rows_all = (q->n + 255) / 256 * 256;
-    int64_t rows = (int64_t)(512 << 20) / ((int64_t)kf * 32 * wp) / 256 * 256;
+    // weights: as many rows at a time as 512 MB of fragments and their scales hold (less where the device's scratch is bounded)
+    const int64_t rows_all = (q->n + 255) / 256 * 256, scales = sc == 32 ? k / 32 : k / 256 + (ext ? (ext + 255) / 256 : 0);
+    const int64_t row_bytes = (int64_t)kf * 32 * wp + scales * 4, bound = dev->opt_scratch_limit;
+    int64_t rows = (bound > 0 && bound < (512 << 20) ? bound : 512 << 20) / row_bytes / 256 * 256;
     rows = rows < 256 ? 256 : (rows > rows_all ? rows_all : rows);
-    if (half) { // all rows at once, k in one part
-        if (rows < q->n) return FH_ERR_UNSUPPORTED;
-        FragArgs g{};
-        g.m = m, g.n = (int)q->n, g.kf = kf, g.half = half;
-        const fh_status st = frag_go(dev, g, sc, wp, xp, true);
-        if (st != FH_OK) return st;
-    }
+    FragArgs g{};
+    g.m = m, g.n = (int)(rows < q->n ? rows : q->n), g.ldy = half ? half : q->n, g.kf = kf, g.half = half;
+    int parts = 1;
+    FH_TRY(frag_go(dev, g, sc, wp, xp, &parts));
+    if (half && (rows < q->n || parts > 1)) return FH_ERR_UNSUPPORTED; // all rows at once, k in one part
     // activations: rows up to a multiple of the largest tile (rows past m are multiplied and never stored)
-    const int64_t mp = ((int64_t)m + 255) / 256 * 256, xplane = mp * kf * 32;
-    FH_TRY(fh_dev_scratch(dev, &dev->act_buf, &dev->act_cap, (size_t)(xplane * xp + mp * 4)));
+    const int64_t mp = ((int64_t)m + 255) / 256 * 256, xplane = mp * kf * 32, wplane = rows * kf * 32;
+    // The tile kernels need less, so what cannot be had is no error.  (frag_buf last: the others' growth may give it back.)
+    if (!fh_dev_scratch_try(dev, &dev->act_buf, &dev->act_cap, (size_t)(xplane * xp + mp * 4)) ||
+        (parts > 1 && !fh_dev_scratch_try(dev, (void **)&dev->ksplit_buf, &dev->ksplit_cap, (size_t)parts * m * g.n * 4)) ||
+        !fh_dev_scratch_try(dev, &dev->frag_buf, &dev->frag_cap, (size_t)(rows * row_bytes)))
+        return FH_ERR_UNSUPPORTED;
+    dev->frag_captured |= dev->capturing;
     uint8_t *xf = (uint8_t *)dev->act_buf;
     float *rs = (float *)(xf + xplane * xp);
     int runs = 1;
@@ -674,9 +680,6 @@ static fh_status qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int
         k_frag_x<0><<<dim3((unsigned)((m + 7) / 8), (unsigned)runs), 512, lds, dev->stream>>>(x, m, k, ext, xf, xplane, rs);
     }
     FH_HIP(hipGetLastError());
-    const int64_t wplane = rows * kf * 32, scales = sc == 32 ? k / 32 : k / 256 + (ext ? (ext + 255) / 256 : 0);
-    const size_t need = (size_t)(wplane * wp + scales * rows * 4);
-    FH_TRY(fh_dev_scratch(dev, &dev->frag_buf, &dev->frag_cap, need));
     uint8_t *wf = (uint8_t *)dev->frag_buf;
     float *d = (float *)(wf + wplane * wp);
     QView v = fh_view(q);
@@ -695,10 +698,8 @@ static fh_status qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int
         }
 #undef FRAG_W
         FH_HIP(hipGetLastError());
-        FragArgs g{};
-        g.w = wf, g.x = xf, g.w_plane = wplane, g.x_plane = xplane, g.d = d, g.n_pad = rows, g.rs = rs, g.y = y, g.ldy = half ? half : q->n, g.half = half;
-        g.m = m, g.n = (int)n, g.n0 = (int)n0, g.kf = kf;
-        FH_TRY(frag_go(dev, g, sc, wp, xp, false));
+        g.w = wf, g.x = xf, g.w_plane = wplane, g.x_plane = xplane, g.d = d, g.n_pad = rows, g.rs = rs, g.y = y, g.n = (int)n, g.n0 = (int)n0;
+        FH_TRY(frag_go(dev, g, sc, wp, xp, nullptr));
     }
     return FH_OK;
 }

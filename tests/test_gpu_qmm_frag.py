@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from kalosm_amd import synth
-from kalosm_amd.fusor import QMatrix, Tensor
+from kalosm_amd.fusor import Device, FusorHipError, QMatrix, Tensor
 
 pytestmark = pytest.mark.gpu
 TYPES = [synth.Q4_0, synth.Q5_0, synth.Q8_0, synth.Q4_K, synth.Q5_K, synth.Q6_K]
@@ -151,3 +151,82 @@ def test_short_prompts_keep_the_tile_sums(dev, tokens):
             dev.set_option("matmul_kernel", 0)
         model.reset()
     assert np.isfinite(got[0]).all() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
+def bits(dev, q, x, option):
+    dev.set_option("matmul_kernel", option)
+    try:
+        return x.q_mat_mul(q).as_slice().view(np.uint32)
+    finally:
+        dev.set_option("matmul_kernel", 0)
+
+
+@pytest.mark.parametrize("ty", [synth.Q8_0, synth.Q4_K, synth.Q6_K], ids=lambda t: synth.TYPE_NAMES[t])
+def test_weights_in_several_launches(oracle, ty):
+    """Scratch of 3.5 MB holds the fragments of 768 to 1536 of the 3000 rows."""
+    dev = Device.gpu(0)
+    dev.set_option("scratch_limit", 3500000)
+    try:
+        got, want = product(dev, oracle, ty, 70, 3000, 1024, "f32", 13)
+        tiles, _ = product(dev, oracle, ty, 70, 3000, 1024, "f32", 11)
+    finally:
+        dev.close()
+    assert np.sqrt(np.mean((got - want) ** 2)) <= 2e-6 * np.sqrt(np.mean(want * want))
+    assert not np.array_equal(got, tiles)
+
+
+def test_without_memory_for_the_fragments():
+    """The tile kernels, which need less, take the product."""
+    dev = Device.gpu(0)
+    try:
+        q = QMatrix.from_raw_bytes(dev, (512, 512), synth.random_weight(synth.Q4_K, 512, 512, seed=1, sigma=2e-3), synth.Q4_K)
+        x = Tensor.from_slice(dev, synth.random_activation(40, 512, seed=2))
+        dev.set_option("scratch_limit", 300000)
+        refused = bits(dev, q, x, 0)
+        dev.set_option("scratch_limit", 0)
+        assert np.array_equal(refused, bits(dev, q, x, 11))
+        assert np.array_equal(bits(dev, q, x, 0), bits(dev, q, x, 13)) and not np.array_equal(bits(dev, q, x, 0), refused)
+    finally:
+        dev.close()
+
+
+def test_fragments_and_graphs():
+    """A captured product takes the fragments if their memory is there, and the tiles if not; growth of that memory ends the graphs
+    that use it and no others; an allocation that fails has asked for it first."""
+    dev = Device.gpu(0)
+    try:
+        x = Tensor.from_slice(dev, synth.random_activation(40, 512, seed=2))
+        q = {n: QMatrix.from_raw_bytes(dev, (n, 512), synth.random_weight(synth.Q8_0, n, 512, seed=n, sigma=2e-3), synth.Q8_0)
+             for n in (64, 2048, 8192)}
+        out = Tensor(dev, (40, 2048))
+
+        def capture():
+            dev.graph_begin()
+            x.q_mat_mul(q[2048], out=out)
+            return dev.graph_end()
+
+        def replay(graph):
+            graph.launch()
+            return out.as_slice().view(np.uint32)
+
+        bits(dev, q[64], x, 13)                       # 1 MB of each buffer
+        tiles = bits(dev, q[2048], x, 11)
+        on_tiles = capture()                          # 2 MB of fragments
+        assert np.array_equal(replay(on_tiles), tiles)
+        fragments = bits(dev, q[2048], x, 0)
+        assert not np.array_equal(fragments, tiles)
+        on_fragments = capture()
+        for _ in range(3):
+            assert np.array_equal(replay(on_fragments), fragments)
+            assert np.array_equal(replay(on_tiles), tiles)
+        bits(dev, q[8192], x, 0)
+        with pytest.raises(FusorHipError, match="capture it again"):
+            on_fragments.launch()
+        assert np.array_equal(replay(on_tiles), tiles)
+        with pytest.raises(FusorHipError):
+            dev.alloc(1 << 42)
+        assert np.array_equal(replay(capture()), tiles)
+        assert np.array_equal(bits(dev, q[2048], x, 0), fragments)
+        del on_tiles, on_fragments
+    finally:
+        dev.close()

@@ -666,7 +666,8 @@ fh_status fh_matvec_norm(fh_device *dev, const float *x, int k, const float *w, 
 enum { HEAD_ROWS = 16 };
 struct HeadRows { int row[HEAD_ROWS], place[HEAD_ROWS], n; };
 
-// Final norm of the rows (the arithmetic of k_matvec_norm) and their three terms in the order of the MFMA operand: 64 of k: two
+// Final norm of the rows (the arithmetic of k_matvec_norm, addition for addition: the normed row that a pass gives back has the same
+// bits however many rows it has) and their three terms in the order of the MFMA operand: 64 of k: two
 // steps of 32: three terms: lane l (row l % 16, k = 8 (l / 16) .. + 7): 16 bytes.  Rows that are not there are zeros.
 __global__ __launch_bounds__(256) void k_head_x(const float *__restrict__ x, int k, int kp, const float *__restrict__ nw, float eps,
                                                 HeadRows rows, uint16_t *__restrict__ xf, float *__restrict__ norm_out) {
@@ -675,7 +676,13 @@ __global__ __launch_bounds__(256) void k_head_x(const float *__restrict__ x, int
     const bool there = r < rows.n;
     const float *xr = x + (int64_t)rows.row[there ? r : 0] * k;
     float ss = 0.f;
-    for (int i = tid; i < k; i += 256) ss = fmaf(xr[i], xr[i], ss);
+    if (!(k & 3))
+        for (int i = tid * 4; i < k; i += 1024) {
+            const float4 v = *(const float4 *)(xr + i);
+            ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
+        }
+    else
+        for (int i = tid; i < k; i += 256) ss = fmaf(xr[i], xr[i], ss);
     ss = fh_wave_sum(ss);
     if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();

@@ -1,7 +1,7 @@
 """GPU parity: the output matrix for several rows in one pass (csrc/fh_dense.hip: k_head_x, k_head_rows) against float64.
 
 Bound: a row's three bf16 terms hold its 24 bits and multiply exactly, so what is left is the rounding of the f32 sums: k errors of
-2^-24 of either sign, 1e-6 of the root mean square for k up to 1000, and ten times that for the largest single difference."""
+2^-24 of either sign, 1e-6 of the root mean square for k up to 2060, and ten times that for the largest single difference."""
 import numpy as np
 import pytest
 
@@ -10,7 +10,7 @@ import hybridgen as G
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("width,vocab,count", [(20, 30, 2), (64, 64, 16), (72, 65, 17), (256, 130, 33), (1000, 333, 5)])
+@pytest.mark.parametrize("width,vocab,count", [(20, 30, 2), (64, 64, 16), (72, 65, 17), (256, 130, 33), (1000, 333, 5), (1001, 70, 3), (2060, 40, 2)])
 def test_rows(dev, width, vocab, count):
     """Fewer blocks of 64 than wavefronts, k and n that fill no tile, one row more than a pass takes, places in any order and
     twice; the normed row that is given back is the last one's."""
@@ -31,4 +31,4 @@ def test_rows(dev, width, vocab, count):
         for y in (got[i], alone[0]):
             assert np.sqrt(np.mean((y - want) ** 2)) <= 1e-6 * rms
             assert np.abs(y - want).max() <= 1e-5 * rms
-    assert np.abs(last - hidden).max() <= 1e-6 * np.abs(hidden).max()
+    assert np.array_equal(last.view(np.uint32), hidden.view(np.uint32))  # of one place and of several: the same bits

@@ -32,6 +32,10 @@ __device__ __forceinline__ void fh_pv(fh_f4 &acc, const fh_f8 &v, const float *p
     acc = fh_mma32(v, b, acc);
 }
 
+// Weights below 2^-126 are 0 where they are multiplied as bf16 terms; f32 keeps them (four instructions more).
+template <typename T>
+__device__ __forceinline__ float window_exp2(float x) { return sizeof(T) == 4 ? exp2f(x) : __builtin_amdgcn_exp2f(x); }
+
 template <typename T, int DQS, int DVT, int QF>
 __global__ __launch_bounds__(256, sizeof(T) == 2 && DQS * DVT < 64 ? 2 : 1) void k_window_attn(FhWindowAttn a, const T *__restrict__ q, const T *__restrict__ kn,
                                                      const T *__restrict__ kr, const T *__restrict__ vt, int64_t ldt, int s,
@@ -170,13 +174,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 && DQS * DVT < 64 ? 2 : 1) void
             tm = fmaxf(tm, __shfl_xor(tm, 16, 64));
             tm = fmaxf(tm, __shfl_xor(tm, 32, 64));
             const float mn = fmaxf(mx[f], tm), mb = mn == -INFINITY ? 0.f : mn;
-            const float resc = __builtin_amdgcn_exp2f(mx[f] - mb); // (below 2^-126: 0)
+            const float resc = window_exp2<T>(mx[f] - mb);
             float sum = 0.f;
 #pragma unroll
             for (int u = 0; u < 2; u++)
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-                    const float w = __builtin_amdgcn_exp2f(p[f][u][e] - mb);
+                    const float w = window_exp2<T>(p[f][u][e] - mb);
                     p[f][u][e] = w;
                     sum += w;
                 }

@@ -65,8 +65,8 @@ __device__ __forceinline__ fh_f4 fh_mma32(const fh_f8 &a, const fh_f8 &b, fh_f4 
 }
 
 // ROWS weight rows of one wavefront, streamed in pieces of 512 (a lane: eight values, 16 bytes) with AHEAD pieces on their way.
-// No request is under a condition - a lane past the end of the rows repeats the last eight values, and a piece past the last one
-// is not requested: with a branch around a request the compiler can no longer count what is younger and waits for everything.
+// No request is under a condition - a lane past the end of the rows repeats the last eight values, a piece past the last one the
+// last piece: with a branch around a request the compiler can no longer count what is younger and waits for everything.
 template <int ROWS, int AHEAD>
 struct FhRowStream {
     const uint16_t *w[ROWS];

@@ -69,23 +69,29 @@ def test_tile_matmul_five_bit_formats(dev, oracle, ty, m, n, k):
 @pytest.mark.parametrize("ty", ALL, ids=lambda t: NAMES[t])
 @pytest.mark.parametrize("m,n,k", [(200, 384, 4096), (70, 132, 8192), (512, 4096, 2048), (512, 4096, 4096)])
 def test_tile_matmul_split_k(dev, oracle, ty, m, n, k):
-    """Few output tiles for the device and a long k: the default dispatch splits k over workgroups and sums the
-    partial planes in a second launch (on 256 compute units: 64-row tiles four- and eight-fold, 128-row tiles
-    two-fold, 256-row tiles four-fold); f32 and bf16 activations.  The sum is in plane order, so two runs agree bit
-    for bit.  The large cases are checked on the activation rows around the tile edges."""
+    """Few output tiles for the device and a long k: the tile kernels (option 2: they alone, by their own rule) split k over
+    workgroups and sum the partial planes in a second launch (on 256 compute units: 64-row tiles four- and eight-fold,
+    128-row tiles two-fold, 256-row tiles four-fold); f32 and bf16 activations.  The sum is in plane order, so two runs
+    agree bit for bit.  The default dispatch, which may take other kernels, gives the same.  The large cases are checked
+    on the activation rows around the tile edges."""
     raw = synth.random_weight(ty, n, k, seed=150 + ty)
     x = synth.random_activation(m, k, seed=160 + m)
     q = QMatrix.from_raw_bytes(dev, (n, k), raw, ty)
     rows = np.arange(m) if m * n * k < 2 ** 30 else np.array([0, 63, 64, 127, 128, 255, 256, m - 1])
-    got = tile_matmul(dev, x, q, 0)
-    assert_close(got[rows], oracle.q_mat_mul(ty, x[rows], raw, n, fast=True), what=f"{NAMES[ty]} {n}x{k} m={m} split k")
-    assert np.array_equal(got.view(np.uint32), tile_matmul(dev, x, q, 0).view(np.uint32))
     bits, xb = bf16_round(x)
-    out = Tensor.filled_bytes(dev, (m, n), 0xFF)
-    gb = Tensor.from_slice(dev, bits, dtype="bf16").q_mat_mul(q, out=out).as_slice()
-    assert_close(gb[rows], oracle.q_mat_mul(ty, xb[rows], raw, n, fast=True),
-                 what=f"{NAMES[ty]} {n}x{k} m={m} split k, bf16")
-    assert not np.isnan(gb).any() and not np.isnan(got).any()
+    for option in (2, 0):
+        got = tile_matmul(dev, x, q, option)
+        assert_close(got[rows], oracle.q_mat_mul(ty, x[rows], raw, n, fast=True), what=f"{NAMES[ty]} {n}x{k} m={m} split k")
+        assert np.array_equal(got.view(np.uint32), tile_matmul(dev, x, q, option).view(np.uint32))
+        out = Tensor.filled_bytes(dev, (m, n), 0xFF)
+        dev.set_option("matmul_kernel", option)
+        try:
+            gb = Tensor.from_slice(dev, bits, dtype="bf16").q_mat_mul(q, out=out).as_slice()
+        finally:
+            dev.set_option("matmul_kernel", 0)
+        assert_close(gb[rows], oracle.q_mat_mul(ty, xb[rows], raw, n, fast=True),
+                     what=f"{NAMES[ty]} {n}x{k} m={m} split k, bf16")
+        assert not np.isnan(gb).any() and not np.isnan(got).any()
 
 
 @pytest.mark.parametrize("ty", ALL, ids=lambda t: NAMES[t])
@@ -248,19 +254,25 @@ def test_tile_kernels_split_last_round(dev, oracle, ty, act, n):
     are split; ragged in both directions, n a multiple of four or odd) - in every kernel with 256 x 128 tiles: integer
     codes with 64 and 32 of k per step (Q8_0 / Q4_0), Q6_K on two integer terms (bf16) and on the split form (f32), Q4_K
     on integer codes with one and two activation planes.  Against the checker on sampled columns, and against the same
-    product with the split switched off (matmul_kernel = 11), which must agree to the rounding of one addition."""
+    product with the split switched off (matmul_kernel = 11), which must agree to the rounding of one addition - and, in the
+    tiles of the last round, differ by it.  (Option 2: the tile kernels by their own rule; the default takes some of these
+    products to others.)"""
     m, k = 3333, 512
     raw = synth.random_weight(ty, n, k, seed=77)
     xb, xf = bf16_round(synth.random_activation(m, k, seed=78))
     q = QMatrix.from_raw_bytes(dev, (n, k), raw, ty)
     x = Tensor.from_slice(dev, xb, dtype="bf16") if act == "bf16" else Tensor.from_slice(dev, xf)
-    got = x.q_mat_mul(q).as_slice()
-    dev.set_option("matmul_kernel", 11)
+    auto = x.q_mat_mul(q).as_slice()
+    dev.set_option("matmul_kernel", 2)
     try:
+        got = x.q_mat_mul(q).as_slice()
+        dev.set_option("matmul_kernel", 11)
         whole = x.q_mat_mul(q).as_slice()
     finally:
         dev.set_option("matmul_kernel", 0)
     assert np.abs(got - whole).max() <= 1e-5 * np.abs(whole).max()
+    assert not np.array_equal(got, whole)
+    assert np.abs(auto - whole).max() <= 1e-5 * np.abs(whole).max()
     rows = (np.arange(96) * 53 + 7) % n
     bpr = len(raw) // n
     sub = np.concatenate([raw[r * bpr:(r + 1) * bpr] for r in rows])

@@ -114,13 +114,15 @@ def test_rows_are_independent(dev, oracle, ty):
 
 
 @pytest.mark.parametrize("m", [17, 64, 65, 257])
-@pytest.mark.parametrize("ffn", [256, 768])
-def test_swiglu_epilogue(dev, m, ffn):
+@pytest.mark.parametrize("ffn,d_model", [(256, 256), (768, 256), (1280, 256), (256, 2048), (512, 4096)])
+def test_swiglu_epilogue(dev, m, ffn, d_model):
     """gate | up of one launch, SwiGLU at the store, against the two halves as matrices of their own: the same sums and the same
-    formula, so the logits are the same bits."""
+    formula, so the logits are the same bits.  (Halves that end within a tile of 512 weight rows; with a long d_model k is in
+    several parts, so SwiGLU is a launch of its own and the sums of one matrix and of two are parted differently: each within the
+    2e-6 of above, in two layers, is 8e-6 between them.)"""
     from kalosm_amd.llama import Model
 
-    cfg = dict(n_layers=2, d_model=256, n_heads=2, n_kv_heads=1, head_dim=128, ffn=ffn, vocab=320, ctx=512, eps=1e-5, theta=1e4)
+    cfg = dict(n_layers=2, d_model=d_model, n_heads=d_model // 128, n_kv_heads=d_model // 256, head_dim=128, ffn=ffn, vocab=320, ctx=512, eps=1e-5, theta=1e4)
     tokens = np.random.default_rng(m).integers(0, 320, m)
     got = []
     for fuse in (True, False):
@@ -130,7 +132,10 @@ def test_swiglu_epilogue(dev, m, ffn):
             got.append(model.forward(tokens))
         finally:
             dev.set_option("matmul_kernel", 0)
-    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])
+    assert np.isfinite(got[0]).all()
+    if d_model == 256:
+        assert np.array_equal(got[0], got[1])
+    assert np.sqrt(np.mean((got[0] - got[1]) ** 2)) <= 1e-5 * np.sqrt(np.mean(got[1] ** 2))
 
 
 @pytest.mark.parametrize("tokens", [17, 37, 64])

@@ -8,7 +8,8 @@
 //                  k.  The 4-bit codes are turned into f16 SUBNORMAL integers (code * 2^-24) with
 //                  one AND per two codes and fed to v_mfma_f32_16x16x32_f16 as the B operand; the A
 //                  operand holds the activations as an exact two-term f16 split (hi + lo) of the
-//                  block-normalised f32 values.  Products are exact; scales are applied in f32 on
+//                  block-normalised f32 values.  Products of such codes lose up to 1.3e-6 (measured; those
+//                  of normal f16 values nothing); scales are applied in f32 on
 //                  the 16x16 accumulator whose columns are the lane's own weight row.  The min term
 //                  of Q4_K uses the factorisation  y = d*sum_j sc_j*(q.x)_j - dmin*sum_j m_j*(sum x)_j.
 #include "fh_blocks.h"

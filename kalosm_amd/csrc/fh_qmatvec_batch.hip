@@ -7,7 +7,7 @@
 //
 // Exactness: a weight code c (4, 6 or 8 bits) is used as the f16 subnormal c * 2^-24 straight from a mask of the
 // packed bytes; each 256-element chunk of an activation row is scaled by a power of two into the f16 range and
-// split into f16 hi + lo, so code * activation products are exact and accumulate in f32.  The block scale
+// split into f16 hi + lo; code * activation products (of subnormals, to 1.3e-6) accumulate in f32.  The block scale
 // (d * sc, d) multiplies the per-block MFMA result, the block offset (dmin * m, 32 * d * sc, 8 * d, 128 * d)
 // multiplies the f32 sum of the block's activations: the same algebra as GgufBlock::dequantize followed by the
 // dot product, re-associated.

@@ -270,8 +270,7 @@ struct fh_graph {
     fh_device *dev = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    uint64_t scratch_gen = 0, frag_gen = 0; // the device's when the capture ended
-    bool frag = false;                      // a kernel of it holds the address of frag_buf
+    FhScratchStamp stamp;
 };
 
 extern "C" fh_status fh_graph_begin(fh_device *dev) {
@@ -280,7 +279,7 @@ extern "C" fh_status fh_graph_begin(fh_device *dev) {
     FH_HIP(hipStreamSynchronize(dev->stream));
     FH_HIP(hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
     dev->capturing = true;
-    dev->frag_captured = false;
+    FhScratchStamp::begin(dev);
     return FH_OK;
 }
 
@@ -301,16 +300,14 @@ extern "C" fh_status fh_graph_end(fh_device *dev, fh_graph **out) {
     r->dev = dev;
     r->graph = g;
     r->exec = ex;
-    r->scratch_gen = dev->scratch_gen;
-    r->frag_gen = dev->frag_gen;
-    r->frag = dev->frag_captured;
+    r->stamp.end(dev);
     *out = r;
     return FH_OK;
 }
 
 extern "C" fh_status fh_graph_launch(fh_graph *g) {
     FH_REQUIRE(g && g->exec, "NULL graph");
-    if (g->scratch_gen != g->dev->scratch_gen || (g->frag && g->frag_gen != g->dev->frag_gen))
+    if (!g->stamp.valid(g->dev))
         FH_FAIL(FH_ERR_INVALID, "the device's scratch buffers were reallocated by a larger call since this graph was "
                                 "captured; its kernels hold the old addresses: capture it again");
     FH_HIP(hipGraphLaunch(g->exec, g->dev->stream));

@@ -25,7 +25,7 @@ struct fh_decoder {
     hipGraphExec_t graph_exec = nullptr;
     hipGraph_t graph = nullptr;
     int64_t captured_capacity = -1;
-    uint64_t captured_gen = 0, samp_gen = 0; // dev->scratch_gen at the captures
+    FhScratchStamp captured_stamp, samp_stamp;
     uint64_t captured_opt = 0, samp_opt = 0; // dev->opt_gen at the captures (options pick the kernels of a step)
     // sampled decode state: [0..63] previous ids, [64] their count, [65] next slot, [66] Mirostat mu (f32),
     // [68..69] status and token of the last step, [128..] one random number per step

@@ -134,7 +134,7 @@ fh_status fh_decoder::decode_greedy(uint32_t first_token, int steps, uint32_t *o
         // One eager step sizes every scratch buffer and sets kernel attributes; the capture then
         // records launches only.  The graph depends on the cache capacity (strides), so it is
         // rebuilt when the capacity changed since the last capture.
-        if (!graph_exec || captured_capacity != capacity() || captured_gen != dev->scratch_gen ||
+        if (!graph_exec || captured_capacity != capacity() || !captured_stamp.valid(dev) ||
             captured_opt != dev->opt_gen) {
             FH_TRY(fh_timer_start(dev));
             FH_TRY(greedy_step());
@@ -142,6 +142,7 @@ fh_status fh_decoder::decode_greedy(uint32_t first_token, int steps, uint32_t *o
             FH_HIP(hipStreamSynchronize(s));
             if (graph_exec) { (void)hipGraphExecDestroy(graph_exec); graph_exec = nullptr; }
             if (graph) { (void)hipGraphDestroy(graph); graph = nullptr; }
+            FhScratchStamp::begin(dev);
             FH_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             fh_status st = greedy_step();
             hipError_t e = hipStreamEndCapture(s, &graph);
@@ -149,7 +150,7 @@ fh_status fh_decoder::decode_greedy(uint32_t first_token, int steps, uint32_t *o
             FH_HIP(e);
             FH_HIP(hipGraphInstantiate(&graph_exec, graph, nullptr, nullptr, 0));
             captured_capacity = capacity();
-            captured_gen = dev->scratch_gen;
+            captured_stamp.end(dev);
             captured_opt = dev->opt_gen;
         } else {
             FH_TRY(fh_timer_start(dev));
@@ -220,7 +221,7 @@ fh_status fh_decoder::decode_sampled(uint32_t first_token, int steps, const fh_s
         fh_sampler_params want = *params;
         want.random = 0.f; // every step takes its number from randoms_host
         const bool same = samp_exec && samp_capacity == capacity() && samp_range == range &&
-                          samp_gen == dev->scratch_gen && samp_opt == dev->opt_gen &&
+                          samp_stamp.valid(dev) && samp_opt == dev->opt_gen &&
                           memcmp(&samp_params, &want, sizeof(want)) == 0;
         samp_params = want;
         samp_range = range;
@@ -232,6 +233,7 @@ fh_status fh_decoder::decode_sampled(uint32_t first_token, int steps, const fh_s
             if (samp_exec) { (void)hipGraphExecDestroy(samp_exec); samp_exec = nullptr; }
             if (samp_graph) { (void)hipGraphDestroy(samp_graph); samp_graph = nullptr; }
             samp_capacity = -1;
+            FhScratchStamp::begin(dev);
             FH_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             fh_status st = sampled_step();
             hipError_t e = hipStreamEndCapture(s, &samp_graph);
@@ -239,7 +241,7 @@ fh_status fh_decoder::decode_sampled(uint32_t first_token, int steps, const fh_s
             FH_HIP(e);
             FH_HIP(hipGraphInstantiate(&samp_exec, samp_graph, nullptr, nullptr, 0));
             samp_capacity = capacity();
-            samp_gen = dev->scratch_gen;
+            samp_stamp.end(dev);
             samp_opt = dev->opt_gen;
         } else {
             FH_TRY(fh_timer_start(dev));

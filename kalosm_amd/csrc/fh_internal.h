@@ -53,7 +53,7 @@ struct fh_device {
     void *frag_buf = nullptr;
     size_t frag_cap = 0;
     uint64_t frag_gen = 0;      // counts its reallocations: graphs that hold its address are few, so it is not part of scratch_gen
-    bool frag_captured = false; // used since fh_graph_begin
+    bool frag_used = false;     // by a call since the last capture began
     // 64 KB that never moves: partial results of small reductions (argmax)
     void *small_buf = nullptr;
     // Counts the reallocations of act_buf / part_buf / ksplit_buf.  A captured graph holds their addresses as
@@ -93,6 +93,15 @@ struct fh_device {
     int64_t opt_trace_stderr = 0;    // 1: trace lines go to stderr as well as into the decoder's trace text
     uint64_t opt_gen = 0;            // bumped by every fh_set_option: captured decode steps are recorded again after a change
     int64_t opt_matmul_kernel = 0;   // 0 auto, 1 generic for every m, 2 MFMA tile kernels for every m, 3 / 4 and never / always the 128 x 256 one
+};
+
+// Which scratch memory the kernels of a captured graph hold the addresses of: begin ahead of the capture, end behind it.
+struct FhScratchStamp {
+    uint64_t scratch = 0, frag = 0;
+    bool frag_used = false;
+    static void begin(fh_device *dev) { dev->frag_used = false; }
+    void end(const fh_device *dev) { scratch = dev->scratch_gen, frag = dev->frag_gen, frag_used = dev->frag_used; }
+    bool valid(const fh_device *dev) const { return scratch == dev->scratch_gen && (!frag_used || frag == dev->frag_gen); }
 };
 
 // hipMalloc, once more without frag_buf where there is not enough memory

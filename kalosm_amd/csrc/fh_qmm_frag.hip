@@ -665,7 +665,7 @@ static fh_status qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int
         (parts > 1 && !fh_dev_scratch_try(dev, (void **)&dev->ksplit_buf, &dev->ksplit_cap, (size_t)parts * m * g.n * 4)) ||
         !fh_dev_scratch_try(dev, &dev->frag_buf, &dev->frag_cap, (size_t)(rows * row_bytes)))
         return FH_ERR_UNSUPPORTED;
-    dev->frag_captured |= dev->capturing;
+    dev->frag_used = true;
     uint8_t *xf = (uint8_t *)dev->act_buf;
     float *rs = (float *)(xf + xplane * xp);
     int runs = 1;

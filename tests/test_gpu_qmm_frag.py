@@ -235,3 +235,24 @@ def test_fragments_and_graphs():
         del on_tiles, on_fragments
     finally:
         dev.close()
+
+
+def test_fragments_in_a_captured_step():
+    """Option 13 takes a decoder's one-row products there as well: a step that was captured with them is captured again when a
+    larger product moves their memory."""
+    from kalosm_amd.llama import Model
+
+    dev = Device.gpu(0)
+    dev.set_option("matmul_kernel", 13)
+    try:
+        cfg = dict(n_layers=1, d_model=512, n_heads=4, n_kv_heads=2, head_dim=128, ffn=1024, vocab=320, ctx=64, eps=1e-5, theta=1e4)
+        model = Model.random_init(dev, cfg, seed=2, sigma=2e-3, fuse_qkv=False)
+        want = model.decode_greedy(5, 8)[0].tolist()
+        x = Tensor.from_slice(dev, synth.random_activation(40, 512, seed=2))
+        large = QMatrix.from_raw_bytes(dev, (16384, 512), synth.random_weight(synth.Q8_0, 16384, 512, seed=3, sigma=2e-3), synth.Q8_0)
+        for _ in range(2):
+            x.q_mat_mul(large).as_slice()
+            model.reset()
+            assert model.decode_greedy(5, 8)[0].tolist() == want
+    finally:
+        dev.close()

@@ -777,8 +777,8 @@ __global__ __launch_bounds__(256, 2) void k_head_rows(const uint16_t *__restrict
 fh_status fh_head_rows(fh_device *dev, const float *x, int k, const float *w, float eps, const uint16_t *out, int n, const int *row,
                        const int *place, int count, float *y, int64_t ldy, float *norm_out) {
     const int kp = (int)fh_pad64(k);
-    FH_TRY(fh_dev_scratch(dev, (void **)&dev->ksplit_buf, &dev->ksplit_cap, (size_t)kp * 3 * HEAD_ROWS * 2));
-    uint16_t *xf = (uint16_t *)dev->ksplit_buf;
+    FH_REQUIRE((size_t)kp * 3 * HEAD_ROWS * 2 <= FH_FIXED_BYTES, "k = %d too long for the output matrix", k);
+    uint16_t *xf = (uint16_t *)dev->fixed_buf;
     for (int at = 0; at < count; at += HEAD_ROWS) {
         HeadRows rows = {};
         rows.n = std::min<int>(count - at, HEAD_ROWS);

@@ -906,8 +906,8 @@ static fh_status topk_run(fh_device *dev, const float *x_dev, int64_t count, int
     // One workgroup walks the 64-key maxima twice: 2 x 1.4 us at 128256 logits; past 2^20 the passes spread that over many.
     if (blocks > 1 && count <= (1 << 20)) {
         const int lists = (int)(blocks * 16);
-        FH_TRY(fh_dev_scratch(dev, (void **)&dev->ksplit_buf, &dev->ksplit_cap, (size_t)blocks * 1024 * 8 + (size_t)lists * 8));
-        uint64_t *keys = (uint64_t *)dev->ksplit_buf, *list_max = keys + blocks * 1024;
+        static_assert((1 << 20) * 8 + (1 << 14) * 8 <= FH_FIXED_BYTES, "keys and maxima of 2^20 logits");
+        uint64_t *keys = (uint64_t *)dev->fixed_buf, *list_max = keys + blocks * 1024;
         k_topk_keys<<<dim3((unsigned)blocks), dim3(1024), 0, dev->stream>>>(x_dev, count, proc, keys, list_max);
         k_topk_pick<<<dim3(1), dim3(512), 0, dev->stream>>>(x_dev, keys, list_max, lists, k, ids_dev, values_dev, found_dev, proc, samp);
         FH_HIP(hipGetLastError());

@@ -56,6 +56,9 @@ struct fh_device {
     bool frag_used = false;     // by a call since the last capture began
     // 64 KB that never moves: partial results of small reductions (argmax)
     void *small_buf = nullptr;
+    // 9 MB that never move (FH_FIXED_BYTES): the keys of a top-k over up to 2^20 logits, the rows of the output matrix's one pass.  In
+    // buffers that grow they would end the graphs of other calls, and a captured call would need an eager one of its size.
+    void *fixed_buf = nullptr;
     // Counts the reallocations of act_buf / part_buf / ksplit_buf.  A captured graph holds their addresses as
     // kernel arguments, so whoever keeps a graph records the value at capture and must not replay it after
     // the value has changed.
@@ -94,6 +97,8 @@ struct fh_device {
     uint64_t opt_gen = 0;            // bumped by every fh_set_option: captured decode steps are recorded again after a change
     int64_t opt_matmul_kernel = 0;   // 0 auto, 1 generic for every m, 2 MFMA tile kernels for every m, 3 / 4 and never / always the 128 x 256 one
 };
+
+enum { FH_FIXED_BYTES = 9 << 20 };
 
 // Which scratch memory the kernels of a captured graph hold the addresses of: begin ahead of the capture, end behind it.
 struct FhScratchStamp {

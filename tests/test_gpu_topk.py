@@ -67,3 +67,37 @@ def test_continuation(dev, oracle, kind):
             mu = sampler.mu
         history.append(got)
     assert near <= 6
+
+
+def test_graphs_outlive_a_larger_vocabulary():
+    """The keys of 151936 logits lie in memory that never moves, and so do the rows of an output matrix of width 12288: a graph
+    that was captured before them is still launched."""
+    import hybridgen as G
+    from kalosm_amd import synth
+    from kalosm_amd.fusor import Device, QMatrix
+
+    dev = Device.gpu(0)
+    try:
+        rng = np.random.default_rng(3)
+        q = QMatrix.from_raw_bytes(dev, (64, 512), synth.random_weight(synth.Q8_0, 64, 512, 1), synth.Q8_0)
+        x, y = Tensor.from_slice(dev, synth.random_activation(16, 512, 2)), Tensor.zeros(dev, (16, 64))
+        cfg = G.config([G.with_mlp(G.delta(1, 1, 16, 16, 4), None)], 12288, 40)
+        model = G.build(dev, cfg, G.weights(cfg))
+        alone = model.forward([3, 1, 2])
+        Tensor.from_slice(dev, rng.standard_normal((1 << 20) + 1).astype(np.float32)).top_k_pairs(1)  # the passes' scratch: 1 MB
+        x.q_mat_mul(q, out=y)
+        want = y.as_slice()
+        dev.graph_begin()
+        x.q_mat_mul(q, out=y)
+        graph = dev.graph_end()
+        logits = rng.standard_normal(151936).astype(np.float32)
+        assert [p[0] for p in Tensor.from_slice(dev, logits).top_k_pairs(64)] == np.argsort(-logits, kind="stable")[:64].tolist()
+        model.reset()
+        several = model.forward([3, 1, 2], want=[0, 1, 2])
+        assert np.sqrt(np.mean((several[2] - alone) ** 2)) <= 2e-6 * np.sqrt(np.mean(alone ** 2))
+        for _ in range(2):
+            graph.launch()
+            assert np.array_equal(y.as_slice(), want)
+        del graph
+    finally:
+        dev.close()

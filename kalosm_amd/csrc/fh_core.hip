@@ -75,6 +75,7 @@ extern "C" fh_status fh_device_destroy(fh_device *dev) {
     if (dev->part_buf) (void)hipFree(dev->part_buf);
     if (dev->ksplit_buf) (void)hipFree(dev->ksplit_buf);
     if (dev->frag_buf) (void)hipFree(dev->frag_buf);
+    if (dev->frag_x) (void)hipFree(dev->frag_x);
     if (dev->small_buf) (void)hipFree(dev->small_buf);
     if (dev->fixed_buf) (void)hipFree(dev->fixed_buf);
     (void)hipEventDestroy(dev->ev_start);
@@ -174,12 +175,13 @@ extern "C" fh_status fh_timer_stop(fh_device *dev, float *elapsed_ms) {
 
 hipError_t fh_dev_malloc(fh_device *dev, void **ptr, size_t bytes) {
     hipError_t e = hipMalloc(ptr, bytes);
-    if (e == hipErrorOutOfMemory && dev->frag_buf && !dev->capturing) {
+    if (e == hipErrorOutOfMemory && (dev->frag_buf || dev->frag_x) && !dev->capturing) {
         (void)hipGetLastError();
         (void)hipStreamSynchronize(dev->stream);
-        (void)hipFree(dev->frag_buf);
-        dev->frag_buf = nullptr;
-        dev->frag_cap = 0;
+        if (dev->frag_buf) (void)hipFree(dev->frag_buf);
+        if (dev->frag_x) (void)hipFree(dev->frag_x);
+        dev->frag_buf = dev->frag_x = nullptr;
+        dev->frag_cap = dev->frag_x_cap = 0;
         dev->frag_gen++;
         e = hipMalloc(ptr, bytes);
     }
@@ -197,7 +199,7 @@ static hipError_t scratch_grow(fh_device *dev, void **buf, size_t *cap, size_t n
         *buf = nullptr;
         *cap = 0;
     }
-    if (buf == &dev->frag_buf) dev->frag_gen++;
+    if (buf == &dev->frag_buf || buf == &dev->frag_x) dev->frag_gen++;
     else dev->scratch_gen++;
     const size_t want = need < (1u << 20) ? (1u << 20) : need;
     const hipError_t e = fh_dev_malloc(dev, buf, want);

@@ -49,10 +49,11 @@ struct fh_device {
     size_t part_cap = 0;
     float *ksplit_buf = nullptr; // partial planes of a k-split prefill matmul
     size_t ksplit_cap = 0;
-    // weights of a prompt's product in fragment order and their scales, at most 512 MB; given back when memory runs out
-    void *frag_buf = nullptr;
-    size_t frag_cap = 0;
-    uint64_t frag_gen = 0;      // counts its reallocations: graphs that hold its address are few, so it is not part of scratch_gen
+    // A prompt's product in fragment order: weights and their scales, at most 512 MB; activations and the partial planes of a split k.
+    // Given back when memory runs out.
+    void *frag_buf = nullptr, *frag_x = nullptr;
+    size_t frag_cap = 0, frag_x_cap = 0;
+    uint64_t frag_gen = 0;      // counts their reallocations: graphs that hold their addresses are few, so it is not part of scratch_gen
     bool frag_used = false;     // by a call since the last capture began
     // 64 KB that never moves: partial results of small reductions (argmax)
     void *small_buf = nullptr;
@@ -109,7 +110,7 @@ struct FhScratchStamp {
     bool valid(const fh_device *dev) const { return scratch == dev->scratch_gen && (!frag_used || frag == dev->frag_gen); }
 };
 
-// hipMalloc, once more without frag_buf where there is not enough memory
+// hipMalloc, once more without frag_buf and frag_x where there is not enough memory
 hipError_t fh_dev_malloc(fh_device *dev, void **ptr, size_t bytes);
 fh_status fh_dev_scratch(fh_device *dev, void **buf, size_t *cap, size_t need);
 // The same for callers that can do without: false, and no error, where `need` bytes cannot be had (or not while capturing).
@@ -229,6 +230,7 @@ fh_status fh_launch_qmatvec_batch(const fh_qmatrix *q, const float *x, int m, fl
 fh_status fh_launch_qmm_q8_mfma(const fh_qmatrix *q, const float *x, int m, float *y);
 // fragments: whether the rule of fh_qmm_frag.hip may take the product
 fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, bool fragments = true);
+size_t fh_qmatmul_tile_planes(const fh_qmatrix *q, int x_is_bf16, int m); // what it takes of act_buf
 // fh_qmatmul of a decoder's prompt: short ones keep the sums of the tile kernels (fh_qmm_frag.h, FH_SHORT_PROMPT).
 fh_status fh_qmatmul_prompt(const fh_qmatrix *q, const float *x, int m, float *y);
 // power of two for fh_qmatrix::wscale from the largest |w| of `count` f32 values on the device (blocking)

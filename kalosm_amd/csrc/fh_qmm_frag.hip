@@ -317,7 +317,8 @@ struct FragArgs {
     int64_t ldy;     // outputs of a row of y
     int m, n, n0;    // rows, weight rows of this launch, first of them in y
     int kf, tiles_w, tiles_x, parts;
-    int64_t part_stride; // floats between the partial planes of a split k
+    float *part;         // partial planes of a split k,
+    int64_t part_stride; // so many floats apart
     int half;            // > 0: y[:, i] = silu(row i) * (row half + i)
 };
 
@@ -563,8 +564,8 @@ static fh_status frag_product(fh_device *dev, FragArgs g, int *ask) { // ask: on
     }
     g.parts = parts;
     float *y = g.y;
-    if (parts > 1) { // whole planes [m][n] of this launch's weight rows (qmm_frag has the memory)
-        g.y = dev->ksplit_buf;
+    if (parts > 1) { // whole planes [m][n] of this launch's weight rows
+        g.y = g.part;
         g.part_stride = (int64_t)g.m * g.n;
     }
     FH_TRY(fh_kernel_lds(dev, (const void *)k_qmm_frag<NW, NX, SC, FW, FX, WGX>, (size_t)LDS));
@@ -572,7 +573,7 @@ static fh_status frag_product(fh_device *dev, FragArgs g, int *ask) { // ask: on
     FH_HIP(hipGetLastError());
     if (parts > 1) {
         const int64_t count = (int64_t)g.m * g.n;
-        k_frag_sum<<<dim3((unsigned)((count + 1023) / 1024)), 256, 0, dev->stream>>>(dev->ksplit_buf, parts, g.part_stride, count, y);
+        k_frag_sum<<<dim3((unsigned)((count + 1023) / 1024)), 256, 0, dev->stream>>>(g.part, parts, g.part_stride, count, y);
         FH_HIP(hipGetLastError());
     }
     return FH_OK;
@@ -660,14 +661,17 @@ static fh_status qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int
     if (half && (rows < q->n || parts > 1)) return FH_ERR_UNSUPPORTED; // all rows at once, k in one part
     // activations: rows up to a multiple of the largest tile (rows past m are multiplied and never stored)
     const int64_t mp = ((int64_t)m + 255) / 256 * 256, xplane = mp * kf * 32, wplane = rows * kf * 32;
-    // The tile kernels need less, so what cannot be had is no error.  (frag_buf last: the others' growth may give it back.)
-    if (!fh_dev_scratch_try(dev, &dev->act_buf, &dev->act_cap, (size_t)(xplane * xp + mp * 4)) ||
-        (parts > 1 && !fh_dev_scratch_try(dev, (void **)&dev->ksplit_buf, &dev->ksplit_cap, (size_t)parts * m * g.n * 4)) ||
-        !fh_dev_scratch_try(dev, &dev->frag_buf, &dev->frag_cap, (size_t)(rows * row_bytes)))
+    const size_t part_at = ((size_t)(xplane * xp + mp * 4) + 255) & ~(size_t)255, x_bytes = part_at + (parts > 1 ? (size_t)parts * m * g.n * 4 : 0);
+    // The tile kernels need less, so what cannot be had is no error.  Their planes are there too: a captured product takes them where the
+    // fragments do not fit.  (The growth of one of frag_x and frag_buf may give the other back.)
+    (void)fh_dev_scratch_try(dev, &dev->act_buf, &dev->act_cap, fh_qmatmul_tile_planes(q, x_is_bf16, m));
+    if (!fh_dev_scratch_try(dev, &dev->frag_x, &dev->frag_x_cap, x_bytes) ||
+        !fh_dev_scratch_try(dev, &dev->frag_buf, &dev->frag_cap, (size_t)(rows * row_bytes)) || dev->frag_x_cap < x_bytes)
         return FH_ERR_UNSUPPORTED;
     dev->frag_used = true;
-    uint8_t *xf = (uint8_t *)dev->act_buf;
+    uint8_t *xf = (uint8_t *)dev->frag_x;
     float *rs = (float *)(xf + xplane * xp);
+    g.part = (float *)(xf + part_at);
     int runs = 1;
     while (runs < 8 && (m + 7) / 8 * runs < dev->compute_units && k / (runs * 2) >= 1024) runs *= 2;
     while (ext && ((k + runs - 1) / runs + 511) / 512 * 512 > 32768) runs *= 2; // the sums of a run: at most 32 KB of LDS

@@ -1785,6 +1785,22 @@ static fh_status qmm_launch_dense(const fh_qmatrix *q, const _Float16 *xh, const
     return FH_OK;
 }
 
+// planes: xh | xl | rs | (Q4_K: sums of the 32-groups, hi and lo)
+struct TilePlanes {
+    size_t plane, rs_bytes, bytes;
+    bool sums;
+};
+static TilePlanes tile_planes(const fh_qmatrix *q, int x_is_bf16, int m) {
+    const int64_t K = q->k;
+    TilePlanes p;
+    p.plane = ((size_t)m * K * 2 + 255) & ~(size_t)255;
+    p.rs_bytes = ((size_t)m * 4 + 255) & ~(size_t)255;
+    p.sums = q->type == FH_Q4_K && K % 256 == 0;
+    p.bytes = p.plane * (x_is_bf16 ? 1 : 2) + p.rs_bytes + (p.sums ? 2 * (size_t)m * (K / 32) * 2 : 0) + 256;
+    return p;
+}
+size_t fh_qmatmul_tile_planes(const fh_qmatrix *q, int x_is_bf16, int m) { return tile_planes(q, x_is_bf16, m).bytes; }
+
 fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, bool fragments) {
     fh_device *dev = q->dev;
     const int64_t K = q->k;
@@ -1798,12 +1814,10 @@ fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf
         const fh_status st = fh_launch_qmm_frag(q, x, x_is_bf16, m, y);
         if (st != FH_ERR_UNSUPPORTED) return st; // (no memory for the fragments)
     }
-    // planes: xh | xl | rs | (Q4_K: sums of the 32-groups, hi and lo)
-    const size_t plane = ((size_t)m * K * 2 + 255) & ~(size_t)255;
-    const size_t rs_bytes = ((size_t)m * 4 + 255) & ~(size_t)255;
-    const bool sums = q->type == FH_Q4_K && K % 256 == 0;
-    const size_t need = plane * (x_is_bf16 ? 1 : 2) + rs_bytes + (sums ? 2 * (size_t)m * (K / 32) * 2 : 0) + 256;
-    FH_TRY(fh_dev_scratch(dev, &dev->act_buf, &dev->act_cap, need));
+    const TilePlanes planes = tile_planes(q, x_is_bf16, m);
+    const size_t plane = planes.plane, rs_bytes = planes.rs_bytes;
+    const bool sums = planes.sums;
+    FH_TRY(fh_dev_scratch(dev, &dev->act_buf, &dev->act_cap, planes.bytes));
     _Float16 *xh = (_Float16 *)dev->act_buf;
     _Float16 *xl = x_is_bf16 ? nullptr : (_Float16 *)((uint8_t *)dev->act_buf + plane);
     float *rs = (float *)((uint8_t *)dev->act_buf + plane * (x_is_bf16 ? 1 : 2));

@@ -256,3 +256,36 @@ def test_fragments_in_a_captured_step():
             assert model.decode_greedy(5, 8)[0].tolist() == want
     finally:
         dev.close()
+
+
+def test_graphs_of_other_calls_outlive_fragments():
+    """A product on fragments takes more memory than on the tiles (activations for whole tiles, here 2.2 MB for 0.3), all of it its
+    own: a graph that was captured on the tiles is still launched after it, and one that holds fragments until they move."""
+    dev = Device.gpu(0)
+    try:
+        q = QMatrix.from_raw_bytes(dev, (1024, 2048), synth.random_weight(synth.Q4_K, 1024, 2048, seed=1, sigma=2e-3), synth.Q4_K)
+        x = Tensor.from_slice(dev, synth.random_activation(32, 2048, seed=2))
+        few, out = Tensor.from_slice(dev, synth.random_activation(8, 2048, seed=3)), Tensor(dev, (8, 1024))
+        tiles = bits(dev, q, x, 11)
+        want = few.q_mat_mul(q, out=out).as_slice()
+        dev.graph_begin()
+        few.q_mat_mul(q, out=out)
+        graph = dev.graph_end()
+        fragments = bits(dev, q, x, 0)
+        assert not np.array_equal(fragments, tiles)
+        graph.launch()
+        assert np.array_equal(out.as_slice(), want)
+        result = Tensor(dev, (32, 1024))
+        dev.graph_begin()
+        x.q_mat_mul(q, out=result)
+        on_fragments = dev.graph_end()
+        on_fragments.launch()
+        assert np.array_equal(result.as_slice().view(np.uint32), fragments)
+        many = Tensor.from_slice(dev, synth.random_activation(2000, 2048, seed=4))
+        many.q_mat_mul(q).as_slice()
+        with pytest.raises(FusorHipError, match="capture it again"):
+            on_fragments.launch()
+        assert np.array_equal(bits(dev, q, x, 0), fragments)
+        del graph, on_fragments
+    finally:
+        dev.close()

@@ -100,8 +100,8 @@ __device__ __forceinline__ float fh_rec_conv(const FhRecurrent &r, int ch, const
     if (b) acc += b[c];
     return fh_silu_f(acc);
 }
-// The same for T tokens t0 .. of the portion (the ones from s on are not read and their results not used), with up to FH_REC_TAPS
-// taps: a row is read once for all the tokens that it reaches, and all rows are on their way together.
+// The same for T tokens t0 .. of the portion (the ones from s on are not read and their results not used), with FH_REC_TAPS taps: a
+// row is read once for all the tokens that it reaches, and all rows are on their way together.
 enum { FH_REC_TAPS = 4 };
 template <int T>
 __device__ __forceinline__ void fh_rec_conv_rows(const FhRecurrent &r, int ch, const float *proj, int64_t ldp, int t0, int s, int pos,
@@ -113,24 +113,23 @@ __device__ __forceinline__ void fh_rec_conv_rows(const FhRecurrent &r, int ch, c
     else if (c < 2 * nq) c -= nq, w = r.conv_k, b = r.bias_k, col = r.col_k + c;
     else c -= 2 * nq, w = r.conv_v, b = r.bias_v, col = r.col_v + c;
     constexpr int B = FH_REC_TAPS - 1;
-    const int skip = FH_REC_TAPS - r.taps; // places of the window in front of the first tap
     float x[T + B], tap[FH_REC_TAPS];
 #pragma unroll
     for (int j = 0; j < T + B; j++) { // row t0 - B + j
         const int tt = t0 - B + j;
         const float *p = tt >= 0 ? proj + (int64_t)(tt < s ? tt : s - 1) * ldp + col
-                                 : ring + (int64_t)((pos + tt > 0 ? pos + tt : 0) % r.taps) * channels + ch;
+                                 : ring + (int64_t)((pos + tt > 0 ? pos + tt : 0) % FH_REC_TAPS) * channels + ch;
         x[j] = *p;
     }
 #pragma unroll
-    for (int i = 0; i < FH_REC_TAPS; i++) tap[i] = w[c * r.taps + (i >= skip ? i - skip : 0)];
+    for (int i = 0; i < FH_REC_TAPS; i++) tap[i] = w[c * FH_REC_TAPS + i];
     const float bias = b ? b[c] : 0.f;
 #pragma unroll
     for (int o = 0; o < T; o++) {
         float acc = 0.f;
 #pragma unroll
         for (int i = 0; i < FH_REC_TAPS; i++)
-            if (i >= skip && pos + t0 + o - B + i >= 0) acc = fmaf(x[o + i], tap[i], acc);
+            if (pos + t0 + o - B + i >= 0) acc = fmaf(x[o + i], tap[i], acc);
         if (b) acc += bias;
         out[o] = fh_silu_f(acc);
     }

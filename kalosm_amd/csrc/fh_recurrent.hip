@@ -5,7 +5,7 @@
 // ------------------------------------------------------------------------------ inputs of the recurrence
 // One workgroup per T tokens.  Bound by memory: with one token a workgroup a thread read the same column of four rows, one after the
 // other, for every token; with four it has seven rows on their way and uses each up to four times
-// (2048 tokens, 16 + 16 heads of 128 and 32 of 128: 133 -> 79 us; with a quarter of the threads 104).
+// (2048 tokens, 16 + 16 heads of 128 and 32 of 128: 85 -> 53 us; with a quarter of the threads a third longer).
 template <int T>
 __global__ __launch_bounds__(T * 256) void k_rec_prep(FhRecurrent r, const float *__restrict__ proj, int64_t ldp, int s, int pos,
                                                   const float *__restrict__ ring, FhRecWork w, int dp) {
@@ -18,21 +18,21 @@ __global__ __launch_bounds__(T * 256) void k_rec_prep(FhRecurrent r, const float
         else v[0] = fh_rec_conv(r, ch, proj, ldp, t0, pos, ring, channels);
 #pragma unroll
         for (int i = 0; i < T; i++) {
-            if (i >= nt) break;
+            if (T > 1 && i >= nt) break;
             if (ch < 2 * nq) qk[i * 2 * nq + ch] = v[i];
             else w.v[(int64_t)(t0 + i) * inner + ch - 2 * nq] = v[i];
         }
     }
-    for (int x = tid; x < nt * r.heads; x += 256 * T) {
-        const int t = t0 + x / r.heads, h = x % r.heads;
+    for (int x = tid; x < (T == 1 ? 1 : nt) * r.heads; x += 256 * T) {
+        const int t = T == 1 ? t0 : t0 + x / r.heads, h = T == 1 ? x : x % r.heads;
         const float *row = proj + (int64_t)t * ldp;
         const float sp = fh_softplus_f(row[r.col_a + h] + r.dt_bias[h]);
         w.la[(int64_t)t * r.heads + h] = -expf(r.a_log[h]) * sp;
         w.beta[(int64_t)t * r.heads + h] = r.delta() ? fh_sigmoid_f(row[r.col_b + h]) : sp;
     }
     __syncthreads();
-    for (int y = wave; y < nt * 2 * r.kv_heads; y += 4 * T) {
-        const int i = y / (2 * r.kv_heads), h = y % (2 * r.kv_heads);
+    for (int y = wave; y < (T == 1 ? 1 : nt) * 2 * r.kv_heads; y += 4 * T) {
+        const int i = T == 1 ? 0 : y / (2 * r.kv_heads), h = T == 1 ? y : y % (2 * r.kv_heads);
         const float *x = qk + i * 2 * nq + h * r.dim;
         float f = 1.f;
         if (r.delta()) {
@@ -660,9 +660,12 @@ fh_status fh_recurrent_prefill(fh_device *dev, int dtype, const FhRecurrent &r, 
         const int nq = r.kv_heads * r.dim, channels = fh_rec_channels(r);
         const size_t lds = (size_t)2 * nq * 4;
         FH_REQUIRE(lds <= 150 * 1024, "recurrent layer of %d channels is too wide", channels);
-        // four tokens a workgroup where there are enough of them for the compute units (fewer leave some idle), their queries and
-        // keys fit the LDS twice and the taps reach no further back than the rows a thread holds
-        if (r.taps <= FH_REC_TAPS && s >= 4 * dev->compute_units && 4 * lds <= 80 * 1024) {
+        // Four tokens a workgroup where there are enough of them for the compute units (fewer leave some idle), their queries and
+        // keys fit the LDS twice, the taps are as many as the rows a thread holds, and the channels give a thread of 1024 work of
+        // its own, the more so where queries and keys are normed behind them.  us, four / one, 1280 tokens: delta rule, 8192
+        // channels 47 / 71, 2048 17 / 21; state space, 1280 11 / 15.  With the number of taps as a variable (a sixth slower) 1024 channels
+        // of the delta rule took 13.5 / 12.1, 640 of the state space 11 / 9.4, three taps 58 / 52 (6144 channels), two 28 / 21 (4096).
+        if (r.taps == FH_REC_TAPS && channels >= (r.delta() ? 2048 : 1280) && s >= 4 * dev->compute_units && 4 * lds <= 80 * 1024) {
             if (4 * lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_rec_prep<4>, 4 * lds));
             k_rec_prep<4><<<dim3((unsigned)((s + 3) / 4)), 1024, 4 * lds, str>>>(r, proj, ldp, s, pos, st.conv, w, dp);
         } else {

@@ -147,7 +147,12 @@ __device__ __forceinline__ void latent_step(const FhStep &st, T *ring, int cap, 
         }
 }
 
-// Gate and up products of the chosen experts: a workgroup takes 8 activations of one of them, two per wavefront.
+// Gate and up products of the chosen experts: a workgroup takes 8 activations of one of them, two per wavefront, with AHEAD pieces of
+// their rows on their way.  Four (100 registers) where all workgroups of the launch are on the device at once with them, four a
+// compute unit, and the rows are longer than two; else two (62 registers, eight a compute unit): us of the launch, two / four / one
+// in a loop, width 2048 with a state space of 4096, top 6 of 1024 14.4 / 14.0 / 14.8, top 8 of 1024 17.1 / 22.6 / 17.6; width 512 and
+// top 8 of 2048 16.3 / 22.3 / 16.3.
+template <int AHEAD>
 __device__ __forceinline__ void expert_step(const FhStep &st, int b, float *lds) {
     const FhMoe &m = st.moe;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, tiles = (m.ff + 7) / 8, slot = b / tiles, tile = b % tiles;
@@ -162,7 +167,7 @@ __device__ __forceinline__ void expert_step(const FhStep &st, int b, float *lds)
     for (int i = tid * 4; i < st.kp; i += 1024) *(float4 *)(lds + i) = *(const float4 *)(st.hn + i);
     __syncthreads();
     const uint16_t *w = m.gate_up + (int64_t)*who * m.gu_stride;
-    FhRowStream<4, 4> rows;
+    FhRowStream<4, AHEAD> rows;
     const int p0 = tile * 8 + wave * 2;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
@@ -181,17 +186,17 @@ __device__ __forceinline__ void expert_step(const FhStep &st, int b, float *lds)
             if (p0 + i < m.ff) st.act[(int64_t)slot * m.ffp + p0 + i] = fh_silu_f(acc[2 * i]) * acc[2 * i + 1];
 }
 
-template <int RPT>
+template <int RPT, int AHEAD>
 __global__ __launch_bounds__(256) void k_step_recurrent(FhStep st, int n_mix) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     if ((int)blockIdx.x < n_mix) rec_step<RPT>(st, blockIdx.x, lds);
-    else expert_step(st, (int)blockIdx.x - n_mix, lds);
+    else expert_step<AHEAD>(st, (int)blockIdx.x - n_mix, lds);
 }
-template <typename T>
+template <typename T, int AHEAD>
 __global__ __launch_bounds__(256) void k_step_latent(FhStep st, T *ring, int cap, int n_mix) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     if ((int)blockIdx.x < n_mix) latent_step<T>(st, ring, cap, blockIdx.x, lds);
-    else expert_step(st, (int)blockIdx.x - n_mix, lds);
+    else expert_step<AHEAD>(st, (int)blockIdx.x - n_mix, lds);
 }
 
 fh_status fh_step_middle(fh_device *dev, int dtype, const FhStep &st, fh_kvcache *cache) {
@@ -202,24 +207,37 @@ fh_status fh_step_middle(fh_device *dev, int dtype, const FhStep &st, fh_kvcache
         const int n_mix = st.rec.heads * ((st.rec.vdim + 15) / 16), rpt = (st.rec.dim + 15) / 16;
         const size_t need = (size_t)(2 * st.rec.dim + 32) * 4;
         lds = lds > need ? lds : need;
-        const void *fn = rpt <= 2 ? (const void *)k_step_recurrent<2> : rpt <= 4 ? (const void *)k_step_recurrent<4>
-                         : rpt <= 8 ? (const void *)k_step_recurrent<8> : (const void *)k_step_recurrent<16>;
         FH_REQUIRE(rpt <= 16, "recurrent state of %d rows (at most 256)", st.rec.dim);
-        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, fn, lds));
         const dim3 grid((unsigned)(n_mix + n_exp));
-        if (rpt <= 2) k_step_recurrent<2><<<grid, 256, lds, dev->stream>>>(st, n_mix);
-        else if (rpt <= 4) k_step_recurrent<4><<<grid, 256, lds, dev->stream>>>(st, n_mix);
-        else if (rpt <= 8) k_step_recurrent<8><<<grid, 256, lds, dev->stream>>>(st, n_mix);
-        else k_step_recurrent<16><<<grid, 256, lds, dev->stream>>>(st, n_mix);
+        const bool four = st.kp > 1024 && n_mix + n_exp <= 4 * dev->compute_units;
+#define STEP_RECURRENT(RPT_)                                                                                                      \
+    do {                                                                                                                          \
+        const void *fn = four ? (const void *)k_step_recurrent<RPT_, 4> : (const void *)k_step_recurrent<RPT_, 2>;                \
+        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, fn, lds));                                                                 \
+        if (four) k_step_recurrent<RPT_, 4><<<grid, 256, lds, dev->stream>>>(st, n_mix);                                          \
+        else k_step_recurrent<RPT_, 2><<<grid, 256, lds, dev->stream>>>(st, n_mix);                                               \
+    } while (0)
+        if (rpt <= 2) STEP_RECURRENT(2);
+        else if (rpt <= 4) STEP_RECURRENT(4);
+        else if (rpt <= 8) STEP_RECURRENT(8);
+        else STEP_RECURRENT(16);
+#undef STEP_RECURRENT
     } else {
         const int n_mix = st.lat.heads * ((st.lat.r8 + 127) / 128) + 1;
         const size_t need = (size_t)16 * 128 * 4;
         lds = lds > need ? lds : need;
         const dim3 grid((unsigned)(n_mix + n_exp));
-        if (lds > 48 * 1024)
-            FH_TRY(fh_kernel_lds(dev, dtype == FH_F32 ? (const void *)k_step_latent<float> : (const void *)k_step_latent<uint16_t>, lds));
-        if (dtype == FH_F32) k_step_latent<float><<<grid, 256, lds, dev->stream>>>(st, (float *)cache->k, cache->capacity, n_mix);
-        else k_step_latent<uint16_t><<<grid, 256, lds, dev->stream>>>(st, (uint16_t *)cache->k, cache->capacity, n_mix);
+        const bool four = st.kp > 1024 && n_mix + n_exp <= 4 * dev->compute_units;
+#define STEP_LATENT(T_)                                                                                                           \
+    do {                                                                                                                          \
+        const void *fn = four ? (const void *)k_step_latent<T_, 4> : (const void *)k_step_latent<T_, 2>;                          \
+        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, fn, lds));                                                                 \
+        if (four) k_step_latent<T_, 4><<<grid, 256, lds, dev->stream>>>(st, (T_ *)cache->k, cache->capacity, n_mix);              \
+        else k_step_latent<T_, 2><<<grid, 256, lds, dev->stream>>>(st, (T_ *)cache->k, cache->capacity, n_mix);                   \
+    } while (0)
+        if (dtype == FH_F32) STEP_LATENT(float);
+        else STEP_LATENT(uint16_t);
+#undef STEP_LATENT
     }
     FH_HIP(hipGetLastError());
     return FH_OK;

@@ -147,6 +147,7 @@ fh_status fh_gemm(fh_device *dev, int dtype, int epi, const FhGemm &g);
 struct FhMvSeg { const uint16_t *w; float *y; int n; };
 fh_status fh_matvec_norm(fh_device *dev, const float *x, int k, const float *w, float eps, const FhMvSeg *segs, int n_segs,
                          float *norm_out);
+int fh_head_rows_from(int k, int n); // from how many rows on the pass below is faster than a matvec for each
 // y[place[i]] [n] = W . n(x row row[i]) for `count` rows that share the pass over the weights; norm_out: n(the last row), kp values.
 fh_status fh_head_rows(fh_device *dev, const float *x, int k, const float *w, float eps, const uint16_t *out, int n, const int *row,
                        const int *place, int count, float *y, int64_t ldy, float *norm_out);

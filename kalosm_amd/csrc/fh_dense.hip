@@ -664,6 +664,15 @@ fh_status fh_matvec_norm(fh_device *dev, const float *x, int k, const float *w, 
 // sums the first terms of even and odd steps and the others apart, so a sum has an eighth of the chain: against 64 bits 1.4e-7 of the root
 // mean square at k = 4096, the matvec 1.6e-7.  With the launch that norms and cuts the rows 14 + 70 us at the size above.
 enum { HEAD_ROWS = 16 };
+
+// A small matrix is a few workgroups' work here, one after the other through its k, whatever the rows, and a matvec of it is short.  Both
+// launches here / one matvec, us (k x n): 1024 x 512 12.7 / 3.4, 2048 x 512 17.5 / 4.4, 2048 x 4096 17.4 / 4.8, 2048 x 16384 20 / 18, 4096 x 512
+// 28 / 5.5, 4096 x 4096 30 / 8.3, 4096 x 8192 31 / 14, 4096 x 12000 32 / 18, 8192 x 512 49 / 6.8, 8192 x 4096 53 / 14, 8192 x 6144 53 / 19.
+int fh_head_rows_from(int k, int n) {
+    if (n >= 6000) return n >= 12000 ? 2 : 3;
+    if (n >= 3500) return k < 2048 ? 3 : 4;
+    return 3 + std::min((k + 1024) / 2048, n >= 2048 ? 2 : 4);
+}
 struct HeadRows { int row[HEAD_ROWS], place[HEAD_ROWS], n; };
 
 // Final norm of the rows (the arithmetic of k_matvec_norm, addition for addition: the normed row that a pass gives back has the same

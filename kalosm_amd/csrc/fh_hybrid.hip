@@ -926,7 +926,7 @@ fh_status Hybrid::head(int row, float *dst) {
 }
 
 fh_status Hybrid::heads(const int *rows, const int *places, int n) {
-    if (n < 2) return fh_decoder::heads(rows, places, n); // one row: the matvec, 45 us against 84 for 2 to 16 (4096 x 32768)
+    if (n < fh_head_rows_from(d_model, vocab)) return fh_decoder::heads(rows, places, n);
     return fh_head_rows(dev, x, d_model, out_norm, eps, (const uint16_t *)out->data, vocab, rows, places, n, logits, vocab, normed);
 }
 

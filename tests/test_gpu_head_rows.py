@@ -32,3 +32,21 @@ def test_rows(dev, width, vocab, count):
             assert np.sqrt(np.mean((y - want) ** 2)) <= 1e-6 * rms
             assert np.abs(y - want).max() <= 1e-5 * rms
     assert np.array_equal(last.view(np.uint32), hidden.view(np.uint32))  # of one place and of several: the same bits
+
+
+@pytest.mark.parametrize("width,vocab,matvecs", [(1000, 40, 2), (1024, 40, 3), (2048, 40, 3), (4100, 40, 4), (4100, 2050, 4), (100, 3500, 2), (2100, 3510, 3), (64, 6000, 2), (64, 12010, 1)])
+def test_few_rows(dev, width, vocab, matvecs):
+    """Up to so many places of a small matrix take a matvec each, the same bits as alone; one more and they share a pass."""
+    cfg = G.config([G.with_mlp(G.delta(1, 1, 16, 16, 4), None)], width, vocab)
+    m = G.build(dev, cfg, G.weights(cfg))
+    toks = np.random.default_rng(width).integers(0, vocab, 8)
+    alone = []
+    for place in range(matvecs + 1):
+        m.reset()
+        alone.append(m.forward(toks, want=[place])[0])
+    for count in (matvecs, matvecs + 1):
+        m.reset()
+        got = m.forward(toks, want=list(range(count)))
+        want = np.array(alone[:count])
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)) == (count == matvecs)
+        assert np.sqrt(np.mean((got - want) ** 2)) <= 2e-6 * np.sqrt(np.mean(want ** 2))

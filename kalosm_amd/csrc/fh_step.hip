@@ -253,7 +253,7 @@ struct OutPiece { const uint16_t *w; int kp, len, in; };
 enum { FH_OUT_AHEAD = 8 };
 
 // NO, NE: 512 values of the mixer and 2048 of the experts a thread holds in registers (more are read when they are staged).  Requests past
-// the end repeat a value, so a thread holds no more than the size needs: a mixer of 512 without experts 4.9 us, with NO = 8 5.5.
+// the end repeat a value, so a thread holds no more than the size needs: a mixer of 512 without experts 4.4 us, with NO = 8 5.4 (read as it is staged 4.8).
 template <int NO, int NE>
 __global__ __launch_bounds__(512, 4) void k_step_out(FhStep st, int n_pieces) {
     extern __shared__ __attribute__((aligned(16))) float in[]; // [kpo | top * ffp | sffp | norm groups | pieces]

@@ -5,6 +5,13 @@
 #pragma once
 #include "fh_internal.h"
 
+// 16 bytes a lane from base[0, bytes) at offset + at into 1 KB of LDS; base, lds and at are the wavefront's.  The compiler waits for
+// all requests at the first use of any loaded register behind a global_load_lds; behind a buffer load it counts them.
+__device__ __forceinline__ void fh_buffer_to_lds(const void *base, int bytes, void *lds, int offset, int at) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void *)base, 0, bytes, 0x00027000),
+                                             (__attribute__((address_space(3))) uint32_t *)lds, 16, offset, at, 0, 0);
+}
+
 typedef _Float16 fh_half;
 
 __device__ __forceinline__ float fh_h2f(uint16_t bits) {

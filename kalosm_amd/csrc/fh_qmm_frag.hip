@@ -367,15 +367,14 @@ __global__ __launch_bounds__(512) void k_qmm_frag(FragArgs g) {
         const uint8_t *base = u < UW ? g.w + (u / (TW / 32)) * g.w_plane + ((int64_t)(tw * (TW / 32) + u % (TW / 32)) * g.kf) * 1024
                                      : g.x + ((u - UW) / (TX / 32)) * g.x_plane +
                                            ((int64_t)(tx * (TX / 32) + (u - UW) % (TX / 32)) * g.kf) * 1024;
-        src[i] = base + lane * 16;
+        src[i] = base;
         at[i] = u * 1024;
     }
     auto fetch = [&](int s, int buf) { // step s into the buffer at byte `buf`; past the end a repeat, so that the counts stay equal
-        const int64_t o = (int64_t)(s < s1 ? s : s1 - 1) * 1024;
+        const int o = (s < s1 ? s : s1 - 1) * 1024;
 #pragma unroll
         for (int i = 0; i < PW; i++)
-            __builtin_amdgcn_global_load_lds((const uint32_t *)(src[i] + o),
-                                             (__attribute__((address_space(3))) uint32_t *)(smem + buf + at[i]), 16, 0, 0);
+            fh_buffer_to_lds(src[i], g.kf * 1024, smem + buf + at[i], lane * 16, o);
     };
     half8 fw[2][NW][FW], fx[2][NX][FX];
     auto read = [&](int set, int buf) {
@@ -490,6 +489,15 @@ __global__ __launch_bounds__(512) void k_qmm_frag(FragArgs g) {
     }
     if (SC == 32) scale(3, FW / 2, FW); // (a multiple of four 32s: the last one's scale is in the last place)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // no LDS-direct load outlives the workgroup's LDS
+    // The rows' factors ahead of all stores: a load between them would wait for the stores before it (one counter for both).
+    float rs[FX][16];
+#pragma unroll
+    for (int c = 0; c < FX; c++)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+            const float4 v = *(const float4 *)(g.rs + tx * TX + (wx * FX + c) * 32 + 2 * r + 4 * (lane >> 5));
+            rs[c][r] = v.x, rs[c][r + 1] = v.y, rs[c][r + 2] = v.z, rs[c][r + 3] = v.w;
+        }
     float *y = g.y + part * g.part_stride;
     if (g.half) { // (FW is 2: gate and up)
         const int nn = (tw * (TW / 64) + ww) * 32 + li;
@@ -500,7 +508,7 @@ __global__ __launch_bounds__(512) void k_qmm_frag(FragArgs g) {
             for (int r = 0; r < 16; r++) {
                 const int mm = tx * TX + (wx * FX + c) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                 if (mm >= g.m) continue;
-                const float gate = acc[0][c][r] * g.rs[mm], up = acc[1][c][r] * g.rs[mm];
+                const float gate = acc[0][c][r] * rs[c][r], up = acc[1][c][r] * rs[c][r];
                 y[(int64_t)mm * g.ldy + nn] = (gate / (expf(-gate) + 1.0f)) * up;
             }
         return;
@@ -514,7 +522,7 @@ __global__ __launch_bounds__(512) void k_qmm_frag(FragArgs g) {
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int mm = tx * TX + (wx * FX + c) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (mm < g.m) y[(int64_t)mm * g.ldy + g.n0 + nn] = acc[a][c][r] * g.rs[mm];
+                if (mm < g.m) y[(int64_t)mm * g.ldy + g.n0 + nn] = acc[a][c][r] * rs[c][r];
             }
     }
 }

@@ -530,7 +530,7 @@ __global__ __launch_bounds__(512) void k_qmm_frag(FragArgs g) {
 __global__ void k_frag_sum(const float *__restrict__ part, int parts, int64_t stride, int64_t count, float *__restrict__ y) {
     const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (i >= count) return;
-    if (i + 3 < count && (stride & 3) == 0) {
+    if (i + 3 < count && (stride & 3) == 0 && ((uintptr_t)y & 15) == 0) {
         float4 a = *(const float4 *)(part + i);
         for (int p = 1; p < parts; p++) {
             const float4 b = *(const float4 *)(part + p * stride + i);
@@ -547,6 +547,12 @@ __global__ void k_frag_sum(const float *__restrict__ part, int parts, int64_t st
 }
 
 // ------------------------------------------------------------------------------ launches
+fh_status fh_frag_sum(fh_device *dev, const float *part, int parts, int64_t stride, int64_t count, float *y) {
+    k_frag_sum<<<dim3((unsigned)((count + 1023) / 1024)), 256, 0, dev->stream>>>(part, parts, stride, count, y);
+    FH_HIP(hipGetLastError());
+    return FH_OK;
+}
+
 template <int NW, int NX, int SC, int FW, int FX, int WGX>
 static fh_status frag_product(fh_device *dev, FragArgs g, int *ask) { // ask: only into how many parts of k
     typedef FragTile<NW, NX, FW, FX, WGX> Tile;
@@ -579,12 +585,7 @@ static fh_status frag_product(fh_device *dev, FragArgs g, int *ask) { // ask: on
     FH_TRY(fh_kernel_lds(dev, (const void *)k_qmm_frag<NW, NX, SC, FW, FX, WGX>, (size_t)LDS));
     k_qmm_frag<NW, NX, SC, FW, FX, WGX><<<dim3((unsigned)(tiles * parts)), 512, LDS, dev->stream>>>(g);
     FH_HIP(hipGetLastError());
-    if (parts > 1) {
-        const int64_t count = (int64_t)g.m * g.n;
-        k_frag_sum<<<dim3((unsigned)((count + 1023) / 1024)), 256, 0, dev->stream>>>(g.part, parts, g.part_stride, count, y);
-        FH_HIP(hipGetLastError());
-    }
-    return FH_OK;
+    return parts > 1 ? fh_frag_sum(dev, g.part, parts, g.part_stride, (int64_t)g.m * g.n, y) : FH_OK;
 }
 
 bool fh_qmm_frag_supports(const fh_qmatrix *q) {
@@ -722,6 +723,8 @@ fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, 
 // take 835 us and no 77 of a SwiGLU launch (7 % of a layer was writing and reading what one store now holds).
 fh_status fh_qmm_frag_swiglu(const fh_qmatrix *q, const float *x, int m, float *y) {
     const int64_t opt = q->dev->opt_matmul_kernel;
+    if (q->n % 64 == 0 && ((uintptr_t)x & 15) == 0 && (opt == 0 ? m > FH_SHORT_PROMPT && fh_qmm_reg_pays(q, 0, m) : opt == 14 && fh_qmm_reg_supports(q)))
+        return fh_qmm_reg_swiglu(q, x, m, y);
     if (q->n % 64 || ((uintptr_t)x & 15) || m <= 16 || !(opt == 0 ? m > FH_SHORT_PROMPT && fh_qmm_frag_pays(q, 0, m) : opt == 13 && fh_qmm_frag_supports(q)))
         return FH_ERR_UNSUPPORTED;
     return qmm_frag(q, x, 0, m, y, (int)(q->n / 2));

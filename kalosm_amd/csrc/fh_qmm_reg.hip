@@ -1,0 +1,689 @@
+// Quantized matmul for a small prompt (17 to some hundred rows; bf16 from one row on), weights decoded in registers:
+// Y[m, n] = X[m, k] . deq(W)[n, k]^T.
+//
+// The tiled layout holds a lane's codes in the order in which v_mfma_f32_16x16x32_f16 takes them, so a wavefront loads 16 bytes a lane
+// and turns them into operands by itself: no pass over memory that writes f16 weights (products on fragments write and read 4 bytes
+// a weight, 52 us for 14336 x 4096 whatever the rows), no LDS or barrier for them (the tile kernels, 128 rows of weights a workgroup
+// one slab after the other).  Only the activations, laid out once per call, come through the LDS.
+//
+// Codes are exact in f16, products add up in f32:
+//   Q4_K / Q5_K  sc * q, d per 256; the offsets dmin * m: one product of the integers m with the sums of 32 activations / 64 (hi + lo)
+//   Q6_K         sc * (q - 32) = its f16 rounding and what that leaves (-1, 0, 1)
+//   Q8_0, Q4_0, Q5_0   the code, d per 32, a sum of its own per 256
+// Activations: a power of two per row, hi + lo (f32 input) or one exact term (bf16).  With f32 input Q6_K drops lo * lo.
+//
+// What bounds it: 17 rows of 14336 x 4096 in Q4_K take 21 us (59 on fragments), 64 rows 32 (67), 192 rows 70 (102), 512 rows 140
+// (153); in Q6_K 26 (118), 38 (124), 90 (139), 180 (247); bf16 rows of Q8_0: one row 16 (140), 33 rows 22 (74), 512 rows 110 (120).  Up
+// to 64 rows that is three launches and, in the middle one, two or three memory round trips; from some hundred rows on the matrix
+// cores and the vector ALU beside them (a 16 x 16 x 32 product hides two vector instructions, a block of 32 has 2.2 a product).
+// Against 64 bits: 1.6e-7 (Q4_K), 1.1e-7 (Q8_0), 1.7e-7 (Q6_K); the tiles 2.6e-7 - 7e-7, the fragments 1.3e-7 - 1.8e-7.
+#include "fh_blocks.h"
+#include "fh_qmm_frag.h"
+
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+// ------------------------------------------------------------------------------ activations
+// Stored [row tile of 16][256 of k]: eight (hi plane) and eight (lo plane, f32 input) operands of 1 KB, one of the sums if there are offsets.
+static constexpr __host__ __device__ bool reg_sums(int t) { return t == FH_Q4_K || t == FH_Q5_K; }
+// order of the eight k of a lane: 0 ascending, 1 (0 2 1 3, 4 6 5 7), 2 the same of 4 g .. and 16 + 4 g ..
+static constexpr __host__ __device__ int reg_order(int t) { return reg_sums(t) ? 1 : t == FH_Q4_0 || t == FH_Q5_0 ? 2 : 0; }
+
+template <int IN, int ORDER>
+__device__ __forceinline__ void reg_x_read(const void *xin, int64_t row, int k, int gi, float v[8]) {
+    const int sb = gi >> 2, g = gi & 3;
+    const int64_t a = row * k + (ORDER == 2 ? sb * 32 + 4 * g : gi * 8), b = a + (ORDER == 2 ? 16 : 4);
+    float4 p, q;
+    if (IN == 1) {
+        const uint2 u = *(const uint2 *)((const uint16_t *)xin + a), w = *(const uint2 *)((const uint16_t *)xin + b);
+        p = make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xFFFF0000u), __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xFFFF0000u));
+        q = make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xFFFF0000u), __uint_as_float(w.y << 16), __uint_as_float(w.y & 0xFFFF0000u));
+    } else {
+        p = *(const float4 *)((const float *)xin + a);
+        q = *(const float4 *)((const float *)xin + b);
+    }
+    if (ORDER == 0) v[0] = p.x, v[1] = p.y, v[2] = p.z, v[3] = p.w, v[4] = q.x, v[5] = q.y, v[6] = q.z, v[7] = q.w;
+    else v[0] = p.x, v[1] = p.z, v[2] = p.y, v[3] = p.w, v[4] = q.x, v[5] = q.z, v[6] = q.y, v[7] = q.w;
+}
+
+// One workgroup: a row, G groups of eight a thread in registers between the maximum and the conversion.
+template <int IN, int ORDER, int G>
+__global__ __launch_bounds__(1024) void k_reg_x(const void *__restrict__ xin, int k, uint8_t *__restrict__ out, float *__restrict__ rs) {
+    constexpr bool SUMS = ORDER == 1;
+    constexpr int CH = (IN == 1 ? 8 : 16) * 1024 + (SUMS ? 1024 : 0);
+    __shared__ float s_max[16], sums[SUMS ? G * 256 : 1];
+    const int tid = threadIdx.x, row = (int)blockIdx.x, groups = k >> 3;
+    float v[G][8], amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < G; i++) {
+        const int gi = tid + i * (int)blockDim.x;
+        reg_x_read<IN, ORDER>(xin, row, k, gi < groups ? gi : groups - 1, v[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < G; i++)
+#pragma unroll
+        for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(v[i][j]));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    if ((tid & 63) == 0) s_max[tid >> 6] = amax;
+    __syncthreads();
+    for (int i = 0; i < (int)blockDim.x >> 6; i++) amax = fmaxf(amax, s_max[i]);
+    int e = 141 - (int)((__float_as_uint(amax) >> 23) & 0xFFu); // 14 - floor(log2 amax); zero / inf / nan clamp
+    e = e > 100 ? 100 : (e < -100 ? -100 : e);
+    const bool infrow = amax == INFINITY; // finite values vanish next to an infinity, which is carried as +-32768
+    const float sc = __uint_as_float((uint32_t)(e + 127) << 23);
+    if (tid == 0) rs[row] = infrow ? INFINITY : __uint_as_float((uint32_t)(127 - e) << 23);
+    uint8_t *dst = out + (int64_t)(row >> 4) * (k >> 8) * CH + (row & 15) * 16;
+#pragma unroll
+    for (int i = 0; i < G; i++) {
+        const int gi = tid + i * (int)blockDim.x;
+        _Float16 h[8], l[8];
+        float t = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            float w = v[i][j] * sc;
+            if (infrow && fabsf(w) == INFINITY) w = copysignf(32768.f, w);
+            h[j] = (_Float16)w;
+            const float d = w - (float)h[j];
+            l[j] = (_Float16)(d == d ? d : 0.f); // a NaN stays in the hi plane alone
+            t += w;
+        }
+        if (SUMS) { // of 32: four threads
+            t += __shfl_xor(t, 1, 64);
+            t += __shfl_xor(t, 2, 64);
+            if ((gi & 3) == 0 && gi < groups) sums[gi >> 2] = t * 0.015625f;
+        }
+        if (gi < groups) {
+            uint8_t *p = dst + (int64_t)(gi >> 5) * CH + ((gi >> 2) & 7) * 1024 + (gi & 3) * 256;
+            uint4 u;
+            __builtin_memcpy(&u, h, 16);
+            *(uint4 *)p = u;
+            if (IN != 1) {
+                __builtin_memcpy(&u, l, 16);
+                *(uint4 *)(p + 8192) = u;
+            }
+        }
+    }
+    if (!SUMS) return;
+    __syncthreads();
+    // a 256's sums: hi in lane group 0, lo in 1, zeros in 2 and 3
+    for (int i = tid; i < (k >> 6); i += (int)blockDim.x) {
+        const int c = i >> 2, g = i & 3;
+        _Float16 h[8];
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const float s = sums[c * 8 + b];
+            const _Float16 sh = (_Float16)s;
+            h[b] = g == 0 ? sh : g == 1 ? (_Float16)(s - (float)sh) : (_Float16)0.f;
+        }
+        uint4 u;
+        __builtin_memcpy(&u, h, 16);
+        *(uint4 *)(dst + (int64_t)c * CH + CH - 1024 + g * 256) = u;
+    }
+}
+
+// ------------------------------------------------------------------------------ weights
+__device__ __forceinline__ half2v reg_h2(uint32_t u) {
+    half2v h;
+    __builtin_memcpy(&h, &u, 4);
+    return h;
+}
+__device__ __forceinline__ half2v reg_splat(float v) { return half2v{(_Float16)v, (_Float16)v}; }
+
+__device__ __forceinline__ half8 reg_cat(const half2v (&r)[4]) {
+    half8 out;
+#pragma unroll
+    for (int i = 0; i < 4; i++) out[2 * i] = r[i][0], out[2 * i + 1] = r[i][1];
+    return out;
+}
+// bytes B and B + 1 (or B twice) of w under the byte 0x64: the f16 pair 1024 + byte
+template <int A, int B>
+__device__ __forceinline__ half2v reg_bytes(uint32_t w) {
+    return reg_h2(__builtin_amdgcn_perm(0x64646464u, w, 0x04000400u | A | B << 16));
+}
+
+// A row tile's 256 of k as a wavefront holds them, lane = (lane group g, row j) of the layout: what is asked for with the first half
+// (ask_a, for the next 256 while this one's second half is multiplied) and with the second (ask_b), begin() in between.
+// get: block sb's operands, one = 0x64006400 in a vector register; scale: of block sb (formats with one per 32), of the 256.
+template <int T>
+struct RegW;
+
+template <int T>
+struct RegK { // Q4_K, Q5_K
+    static constexpr int REC = T == FH_Q5_K ? 2816 : 2304, QA = T == FH_Q5_K ? 3 : 2, QB = 1, NW = 1;
+    uint4 next, cod[2];
+    uint2 next5, five;
+    uint32_t dm, sc[2], mn[2];
+    __device__ __forceinline__ void ask_a(const uint8_t *rec, int lane) {
+        next = *(const uint4 *)(rec + (lane & 15) * 16);
+        cod[0] = *(const uint4 *)(rec + 256 + lane * 16);
+        if (T == FH_Q5_K) next5 = *(const uint2 *)(rec + 2304 + lane * 8);
+    }
+    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { cod[1] = *(const uint4 *)(rec + 1280 + lane * 16); }
+    __device__ __forceinline__ void begin() {
+        dm = next.x, five = next5;
+        sc[0] = next.y & 0x3F3F3F3Fu, sc[1] = (next.w & 0x0F0F0F0Fu) | ((next.y >> 2) & 0x30303030u);
+        mn[0] = next.z & 0x3F3F3F3Fu, mn[1] = ((next.w >> 4) & 0x0F0F0F0Fu) | ((next.z >> 2) & 0x30303030u);
+    }
+    // sc q, exact: a nibble (and its fifth bit) under the byte 0x64 is the f16 1024 + q, high nibbles 1024 + 16 q; one fma per two
+    __device__ __forceinline__ void get(int sb, uint32_t one, half8 (&out)[1]) const {
+        const int p = sb >> 2, u = (sb >> 1) & 1, hn = sb & 1;
+        const uint4 c = cod[p];
+        const uint32_t w[2] = {u ? c.z : c.x, u ? c.w : c.y}, h[2] = {five.x, five.y};
+        const half2v s = reg_h2(__builtin_amdgcn_perm(0x64646464u, sc[p], 0x04000400u + (uint32_t)(sb & 3) * 0x00010001u)) - reg_splat(1024.f);
+        const half2v a = hn ? s * reg_splat(0.0625f) : s, b = s * reg_splat(hn ? -64.f : -1024.f);
+        half2v r[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            uint32_t v = (((i & 1) ? w[i >> 1] >> 8 : w[i >> 1]) & (hn ? 0x00F000F0u : 0x000F000Fu)) | one;
+            if (T == FH_Q5_K) {
+                const int from = sb + 8 * (i & 1), to = hn ? 8 : 4;
+                v |= (from > to ? h[i >> 1] >> (from - to) : h[i >> 1] << (to - from)) & (hn ? 0x01000100u : 0x00100010u);
+            }
+            r[i] = __builtin_elementwise_fma(reg_h2(v), a, b);
+        }
+        out[0] = reg_cat(r);
+    }
+    __device__ __forceinline__ float scale(int) const { return fh_h2f((uint16_t)(dm & 0xFFFFu)); }
+    __device__ __forceinline__ float offset() const { return -64.f * fh_h2f((uint16_t)(dm >> 16)); }
+    __device__ __forceinline__ half8 offsets() const {
+        const half2v k = reg_splat(1024.f), r[4] = {reg_bytes<0, 1>(mn[0]) - k, reg_bytes<2, 3>(mn[0]) - k, reg_bytes<0, 1>(mn[1]) - k, reg_bytes<2, 3>(mn[1]) - k};
+        return reg_cat(r);
+    }
+};
+template <>
+struct RegW<FH_Q4_K> : RegK<FH_Q4_K> {};
+template <>
+struct RegW<FH_Q5_K> : RegK<FH_Q5_K> {};
+
+template <>
+struct RegW<FH_Q6_K> {
+    static constexpr int REC = 3360, QA = 4, QB = 1, NW = 2;
+    uint4 lo[2], next_hi, hi;
+    uint32_t next_sc, sc[4], at;
+    uint16_t next_d, dv;
+    __device__ __forceinline__ void ask_a(const uint8_t *rec, int lane) {
+        lo[0] = *(const uint4 *)(rec + lane * 16);
+        next_hi = *(const uint4 *)(rec + 2048 + lane * 16);
+        next_sc = *(const uint32_t *)(rec + 3072 + lane * 4);
+        next_d = fh_ld16(rec + 3328 + (lane & 15) * 2);
+    }
+    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { lo[1] = *(const uint4 *)(rec + 1024 + lane * 16); }
+    __device__ __forceinline__ void begin() {
+        hi = next_hi, dv = next_d;
+        const int lane = (int)threadIdx.x & 63;
+#pragma unroll
+        for (int q = 0; q < 4; q++) // groups 2 q, 2 q + 1 of both halves are in lane group q; bytes 0 and 2: the one of this lane's k
+            sc[q] = ((uint32_t)__builtin_amdgcn_ds_bpermute((q * 16 + (lane & 15)) * 4, (int)next_sc) ^ 0x80808080u) >> ((lane >> 5) * 8);
+    }
+    // sc (q - 32) = its f16 rounding and what that leaves (-1, 0 or 1)
+    __device__ __forceinline__ void get(int sb, uint32_t one, half8 (&out)[2]) const {
+        const uint4 l4 = lo[sb >> 2];
+        const uint32_t l = (sb & 3) == 0 ? l4.x : (sb & 3) == 1 ? l4.y : (sb & 3) == 2 ? l4.z : l4.w;
+        const uint32_t h = (sb >> 1) == 0 ? hi.x : (sb >> 1) == 1 ? hi.y : (sb >> 1) == 2 ? hi.z : hi.w;
+        const half2v s = (sb < 4 ? reg_bytes<0, 0>(sc[sb & 3]) : reg_bytes<2, 2>(sc[sb & 3])) - reg_splat(1152.f);
+        half2v a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int from = q6k_hbit(sb, i);
+            const uint32_t v = (((l >> (4 * i)) & 0x000F000Fu) | one) | ((from > 4 ? h >> (from - 4) : h << (4 - from)) & 0x00300030u);
+            const half2v q = reg_h2(v) - reg_splat(1056.f);
+            a[i] = q * s;
+            b[i] = __builtin_elementwise_fma(q, s, -a[i]);
+        }
+        out[0] = reg_cat(a), out[1] = reg_cat(b);
+    }
+    __device__ __forceinline__ float scale(int) const { return fh_h2f(dv); }
+};
+
+template <>
+struct RegW<FH_Q8_0> {
+    static constexpr int REC = 4352, QA = 4, QB = 4, NW = 1;
+    uint4 cod[2][2];
+    uint32_t dd[2][2];
+    __device__ __forceinline__ void ask(int p, const uint8_t *rec, int lane) {
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            cod[p][r] = *(const uint4 *)(rec + (2 * p + r) * 1088 + lane * 16);
+            dd[p][r] = *(const uint32_t *)(rec + (2 * p + r) * 1088 + 1024 + (lane & 15) * 4);
+        }
+    }
+    __device__ __forceinline__ void ask_a(const uint8_t *rec, int lane) { ask(0, rec, lane); }
+    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { ask(1, rec, lane); }
+    __device__ __forceinline__ void begin() {}
+    __device__ __forceinline__ void get(int sb, uint32_t, half8 (&out)[1]) const {
+        const uint4 c = cod[sb >> 2][(sb >> 1) & 1];
+        const uint32_t x = (sb & 1 ? c.z : c.x) ^ 0x80808080u, y = (sb & 1 ? c.w : c.y) ^ 0x80808080u;
+        const half2v k = reg_splat(1152.f), r[4] = {reg_bytes<0, 1>(x) - k, reg_bytes<2, 3>(x) - k, reg_bytes<0, 1>(y) - k, reg_bytes<2, 3>(y) - k};
+        out[0] = reg_cat(r);
+    }
+    __device__ __forceinline__ float scale(int sb) const { return fh_h2f((uint16_t)(dd[sb >> 2][(sb >> 1) & 1] >> (16 * (sb & 1)))); }
+};
+
+template <int T>
+struct Reg4 { // Q4_0, Q5_0
+    static constexpr int HALF = T == FH_Q5_0 ? 1408 : 1152, REC = 2 * HALF, QA = T == FH_Q5_0 ? 3 : 2, QB = QA, NW = 1;
+    uint4 cod[2];
+    uint2 dd[2];
+    uint32_t five[2];
+    __device__ __forceinline__ void ask(int p, const uint8_t *rec, int lane) {
+        cod[p] = *(const uint4 *)(rec + p * HALF + lane * 16);
+        dd[p] = *(const uint2 *)(rec + p * HALF + 1024 + (lane & 15) * 8);
+        if (T == FH_Q5_0) five[p] = *(const uint32_t *)(rec + p * HALF + 1152 + lane * 4);
+    }
+    __device__ __forceinline__ void ask_a(const uint8_t *rec, int lane) { ask(0, rec, lane); }
+    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { ask(1, rec, lane); }
+    __device__ __forceinline__ void begin() {}
+    // q - 8 (q - 16) from 1024 + q, high nibbles from 1024 + 16 q
+    __device__ __forceinline__ void get(int sb, uint32_t one, half8 (&out)[1]) const {
+        const int p = sb >> 2, u = sb & 3;
+        const uint4 c = cod[p];
+        const uint32_t w = u == 0 ? c.x : u == 1 ? c.y : u == 2 ? c.z : c.w, lo5 = (five[p] >> (8 * u)) & 15u, hi5 = (five[p] >> (8 * u + 4)) & 15u;
+        const float off = T == FH_Q5_0 ? 16.f : 8.f;
+        half2v r[4];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            uint32_t a = ((i ? w >> 8 : w) & 0x000F000Fu) | one, b = ((i ? w >> 8 : w) & 0x00F000F0u) | one;
+            if (T == FH_Q5_0) { // bits i and i + 2 of four
+                a |= (lo5 * (i ? 0x20008u : 0x40010u)) & 0x00100010u;
+                b |= (hi5 * (i ? 0x200080u : 0x400100u)) & 0x01000100u;
+            }
+            r[i] = reg_h2(a) - reg_splat(1024.f + off);
+            r[2 + i] = __builtin_elementwise_fma(reg_h2(b), reg_splat(0.0625f), reg_splat(-64.f - off));
+        }
+        out[0] = reg_cat(r);
+    }
+    __device__ __forceinline__ float scale(int sb) const { return fh_h2f((uint16_t)((sb & 2 ? dd[sb >> 2].y : dd[sb >> 2].x) >> (16 * (sb & 1)))); }
+};
+template <>
+struct RegW<FH_Q4_0> : Reg4<FH_Q4_0> {};
+template <>
+struct RegW<FH_Q5_0> : Reg4<FH_Q5_0> {};
+
+// ------------------------------------------------------------------------------ product
+struct RegArgs {
+    QView q;
+    const uint8_t *x;
+    const float *rs;
+    float *y;
+    int64_t ldy;
+    int m, n, chunks, wtiles; // 256s of k, row tiles of the matrix
+    int tiles_w, tiles_x, parts;
+    int64_t part_stride;
+    int half; // > 0: y[:, i] = silu(row i) * (row half + i)
+};
+
+// NX planes of activations, MT row tiles of 16 of them; the eight wavefronts are WW along the weight rows, TW row tiles each, times KW
+// along k (added up in LDS at the end).  KW is what a small product needs: with 2 x 4 wavefronts 1024 x 4096 is 16 workgroups whose
+// wavefronts multiply four 256s, with 8 x 1 it is four whose wavefronts multiply 16.
+// A stage is SB blocks of 32 of k: one barrier, in front of it the wait for the stage after.  TW is 2: with 4, half the LDS reads a
+// product, 17 rows took 15 - 25 % longer and 512 rows the same.
+template <int T, int NX, int TW, int MT, int WW, int KW>
+struct RegTile {
+    static constexpr int SB = KW == 1 ? 4 : KW == 2 ? 2 : 1; // blocks of 32 in a stage
+    static constexpr int PIECES = NX * MT * SB, FR = (PIECES + WW - 1) / WW, STAGE = PIECES * KW * 1024;
+    static constexpr int FIT = 163840 / STAGE, ST = FIT > 8 ? 8 : FIT;
+    static constexpr int RED = (KW - 1) * WW * TW * MT * 1024, LDS = ST * STAGE > RED ? ST * STAGE : RED;
+    static constexpr int CH = NX * 8192 + (reg_sums(T) ? 1024 : 0);
+    static_assert(ST >= 4, "four stages at least");
+    // requests for weights (and sums) at block e of a 256
+    static constexpr int wreq(int e) { return e == 0 ? TW * RegW<T>::QB : e == 4 ? TW * RegW<T>::QA : e == 6 && reg_sums(T) ? MT : 0; }
+    // requests younger than those of stage s + 1 at the start of stage s, which begins at block e of a 256.  (In its own stage the
+    // pieces of a stage come behind the first block's requests; those of its other blocks are not counted.)
+    static constexpr int younger(int e) {
+        int n = 0;
+        for (int b = 1; b <= (ST - 3) * SB; b++) n += (b % SB == 0 ? FR : 0) + wreq((e + 64 - b) & 7);
+        return n > 63 ? 63 : n;
+    }
+};
+
+template <int T, int NX, int TW, int MT, int WW, int KW>
+__global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
+    typedef RegTile<T, NX, TW, MT, WW, KW> Tile;
+    constexpr int FR = Tile::FR, PIECES = Tile::PIECES, STAGE = Tile::STAGE, ST = Tile::ST, CH = Tile::CH, SB = Tile::SB;
+    constexpr bool SUMS = reg_sums(T), PER32 = !SUMS && T != FH_Q6_K;
+    constexpr int NW = RegW<T>::NW, NP = NW == 2 ? NX + 1 : NX; // products of a weight operand and 16 rows
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int ww = wave % WW, kw = wave / WW;
+    // workgroups go to the eight dies in turn: a die takes a run of tiles, those of the same weights together
+    const int total = g.tiles_w * g.tiles_x * g.parts, per = total >> 3, more = total & 7, die = (int)blockIdx.x & 7;
+    int lin = ((int)blockIdx.x >> 3) + die * per + (die < more ? die : more);
+    const int tx = lin % g.tiles_x;
+    lin /= g.tiles_x;
+    const int tw = lin % g.tiles_w, part = lin / g.tiles_w;
+    // 256s of this group of wavefronts: first .. first + mine, and the most that one has
+    const int P = g.parts * KW, run = part * KW + kw;
+    const int first = g.chunks * run / P, mine = g.chunks * (run + 1) / P - first;
+    int most = 0;
+#pragma unroll
+    for (int i = 0; i < KW; i++) {
+        const int a = g.chunks * (part * KW + i) / P, b = g.chunks * (part * KW + i + 1) / P;
+        most = b - a > most ? b - a : most;
+    }
+    auto chunk = [&](int i) { const int c = first + (i < most ? i : most - 1); return c < g.chunks ? c : g.chunks - 1; };
+    int tile[TW];
+    const uint8_t *recs[TW];
+#pragma unroll
+    for (int t = 0; t < TW; t++) {
+        const int w = tw * WW + ww;
+        int at = g.half ? (t < TW / 2 ? w * (TW / 2) + t : (g.half >> 4) + w * (TW / 2) + t - TW / 2) : w * TW + t;
+        tile[t] = at;
+        at = at < g.wtiles ? at : g.wtiles - 1;
+        recs[t] = g.q.data + (int64_t)at * g.chunks * RegW<T>::REC;
+    }
+    const uint8_t *xt = g.x + (int64_t)tx * MT * g.chunks * CH;
+    auto fetch = [&](int c, int sb, int buf) { // the stage from block sb of the 256 c on into the buffer at byte `buf`
+#pragma unroll
+        for (int i = 0; i < FR; i++) {
+            const int u = ww + WW * i < PIECES ? ww + WW * i : PIECES - 1; // (past the last one: the same bytes to the same place)
+            const int v = u / (NX * MT), p = u / MT % NX, mt = u % MT;
+            fh_buffer_to_lds(xt, MT * g.chunks * CH, smem + buf + (kw * PIECES + u) * 1024, lane * 16, (mt * g.chunks + c) * CH + (p * 8 + sb + v) * 1024);
+        }
+    };
+    RegW<T> w[TW];
+    floatx4 acc[TW][MT], sum[TW][MT], part256[TW][MT]; // of all, of a scale, of a 256 (formats with a scale per 32)
+    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < TW; t++)
+#pragma unroll
+        for (int c = 0; c < MT; c++) acc[t][c] = zero;
+    half8 xs[MT];
+    int cur = 0;
+#pragma unroll
+    for (int t = 0; t < TW; t++) w[t].ask_a(recs[t] + (int64_t)chunk(0) * RegW<T>::REC, lane);
+#pragma unroll
+    for (int i = 0; i < ST - 1; i++) fetch(chunk(i * SB >> 3), i * SB & 7, i * STAGE);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (the counts of the first steps are those of later ones, with more requests)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    half8 xv[MT * NX], wv[2][NW];
+    float d32 = 0.f;
+#pragma unroll
+    for (int u = 0; u < MT * NX; u++) xv[u] = *(const half8 *)(smem + (kw * PIECES + u) * 1024 + lane * 16);
+    uint32_t one;
+    asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(one));
+    for (int i = 0; i < most; i++) {
+        const int c0 = chunk(i), c1 = chunk(i + 1);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            if (e % SB == 0) {
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Tile::younger(e)) : "memory"); // stage s + 1 has landed (and stage s) ...
+                __builtin_amdgcn_s_barrier();                                           // ... everywhere; the buffer of s - 1 is free
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (e == 0) {
+#pragma unroll
+                for (int t = 0; t < TW; t++) w[t].ask_b(recs[t] + (int64_t)c0 * RegW<T>::REC, lane);
+#pragma unroll
+                for (int t = 0; t < TW; t++) w[t].begin();
+            }
+            if (e == 4)
+#pragma unroll
+                for (int t = 0; t < TW; t++) w[t].ask_a(recs[t] + (int64_t)c1 * RegW<T>::REC, lane);
+            if (SUMS && e == 6)
+#pragma unroll
+                for (int m = 0; m < MT; m++) xs[m] = *(const half8 *)(xt + (m * g.chunks + c0) * CH + CH - 1024 + lane * 16);
+            __builtin_amdgcn_sched_barrier(0);
+            if (e % SB == 0) {
+                constexpr int AHEAD = (ST - 1) * SB; // blocks
+                fetch(chunk(i + (e + AHEAD) / 8), (e + AHEAD) & 7, cur == 0 ? (ST - 1) * STAGE : cur - STAGE);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the next block's activations, each behind its last use here
+            const int nb = e % SB == SB - 1 ? (cur + STAGE == ST * STAGE ? 0 : cur + STAGE) : cur;
+            const uint8_t *b = smem + nb + (kw * PIECES + (e + 1) % SB * NX * MT) * 1024 + lane * 16;
+            if (e == 0) w[0].get(0, one, wv[0]);
+#pragma unroll
+            for (int t = 0; t < TW; t++) { // the next tile's (block's) weights are decoded while this one's are multiplied
+                const int now = t & 1;
+                if (e < 7 || t < TW - 1) w[(t + 1) % TW].get(t == TW - 1 ? e + 1 : e, one, wv[now ^ 1]);
+#pragma unroll
+                for (int u = 0; u < MT * NP; u++) { // (plane by plane, so that neighbours are of different sums)
+                    const int m = u % MT, p = u / MT;
+                    sum[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[p < NX ? u : m], wv[now][p < NX ? 0 : NW - 1],
+                                                                       (PER32 || e == 0) && p == 0 ? zero : sum[t][m], 0, 0, 0);
+                }
+                if (t == TW - 1)
+#pragma unroll
+                    for (int u = 0; u < MT * NX; u++) xv[u] = *(const half8 *)(b + u * 1024);
+                if (PER32) {
+                    if (e + t > 0) { // the sums before these
+                        const int pe = t ? e : e - 1, pt = t ? t - 1 : TW - 1;
+#pragma unroll
+                        for (int m = 0; m < MT; m++)
+#pragma unroll
+                            for (int r = 0; r < 4; r++) part256[pt][m][r] = pe ? fmaf(sum[pt][m][r], d32, part256[pt][m][r]) : sum[pt][m][r] * d32;
+                    }
+                    d32 = i < mine ? w[t].scale(e) : 0.f; // (before the next half's scales are asked for into their place)
+                }
+#pragma unroll
+                for (int u = 0; u < MT * NP; u++) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, (16 * NW + (PER32 ? 4 * MT : 0)) / (MT * NP), 0);
+                    if (t == TW - 1 && u >= MT * (NP - NX)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
+            }
+            if (e % SB == SB - 1) cur = cur + STAGE == ST * STAGE ? 0 : cur + STAGE;
+        }
+        // a 256's own sum first (with its offsets, which all but cancel it): the long sum takes one rounding for it
+#pragma unroll
+        for (int t = 0; t < TW; t++) {
+            const float d = PER32 ? d32 : i < mine ? w[t].scale(0) : 0.f;
+            if constexpr (SUMS) {
+                const float o = i < mine ? w[t].offset() : 0.f;
+                const half8 ov = w[t].offsets();
+#pragma unroll
+                for (int m = 0; m < MT; m++) {
+                    const floatx4 so = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs[m], ov, zero, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[t][m][r] += fmaf(sum[t][m][r], d, so[r] * o);
+                }
+            } else
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        acc[t][m][r] = PER32 ? acc[t][m][r] + (t == TW - 1 ? fmaf(sum[t][m][r], d, part256[t][m][r]) : part256[t][m][r])
+                                             : fmaf(sum[t][m][r], d, acc[t][m][r]);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // no LDS-direct load outlives its buffer
+    if (KW > 1) { // the groups' sums through LDS, in their order
+        __syncthreads();
+        float *red = (float *)smem + lane * 4;
+        if (kw > 0)
+#pragma unroll
+            for (int t = 0; t < TW; t++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) *(floatx4 *)(red + (((kw - 1) * WW + ww) * TW * MT + t * MT + m) * 256) = acc[t][m];
+        __syncthreads();
+        if (kw > 0) return;
+#pragma unroll
+        for (int i = 0; i < KW - 1; i++)
+#pragma unroll
+            for (int t = 0; t < TW; t++)
+#pragma unroll
+                for (int m = 0; m < MT; m++) acc[t][m] += *(const floatx4 *)(red + ((i * WW + ww) * TW * MT + t * MT + m) * 256);
+    }
+    float rs[MT][4]; // ahead of all stores: a load between them would wait for the stores before it
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+        const float4 v = *(const float4 *)(g.rs + (tx * MT + m) * 16 + 4 * (lane >> 4));
+        rs[m][0] = v.x, rs[m][1] = v.y, rs[m][2] = v.z, rs[m][3] = v.w;
+    }
+    float *y = g.y + part * g.part_stride;
+    if (g.half) {
+#pragma unroll
+        for (int t = 0; t < TW / 2; t++) {
+            const int nn = tile[t] * 16 + (lane & 15);
+            if (nn >= g.half) continue;
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int mm = (tx * MT + m) * 16 + 4 * (lane >> 4) + r;
+                    const float gate = acc[t][m][r] * rs[m][r], up = acc[t + TW / 2][m][r] * rs[m][r];
+                    if (mm < g.m) y[mm * g.ldy + nn] = (gate / (expf(-gate) + 1.0f)) * up;
+                }
+        }
+        return;
+    }
+#pragma unroll
+    for (int t = 0; t < TW; t++) {
+        const int nn = tile[t] * 16 + (lane & 15);
+        if (nn >= g.n) continue;
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int mm = (tx * MT + m) * 16 + 4 * (lane >> 4) + r;
+                if (mm < g.m) y[mm * g.ldy + nn] = acc[t][m][r] * rs[m][r];
+            }
+    }
+}
+
+// ------------------------------------------------------------------------------ launches
+template <int T, int NX, int TW, int MT, int WW, int KW>
+static fh_status reg_product(fh_device *dev, RegArgs g, float *part) {
+    typedef RegTile<T, NX, TW, MT, WW, KW> Tile;
+    g.tiles_w = (g.wtiles + TW * WW - 1) / (TW * WW);
+    g.tiles_x = (g.m + MT * 16 - 1) / (MT * 16);
+    float *y = g.y;
+    if (g.parts > 1) {
+        g.y = part;
+        g.part_stride = (int64_t)g.m * g.n;
+    }
+    FH_TRY(fh_kernel_lds(dev, (const void *)k_qmm_reg<T, NX, TW, MT, WW, KW>, (size_t)Tile::LDS));
+    k_qmm_reg<T, NX, TW, MT, WW, KW><<<dim3((unsigned)(g.tiles_w * g.tiles_x * g.parts)), 512, Tile::LDS, dev->stream>>>(g);
+    FH_HIP(hipGetLastError());
+    if (g.parts > 1) return fh_frag_sum(dev, part, g.parts, g.part_stride, g.part_stride, y);
+    return FH_OK;
+}
+
+template <int T, int NX>
+static fh_status reg_go(fh_device *dev, const RegArgs &g, float *part, int mt, int kw) {
+#define GO(MT_)                                                                                                  \
+    return kw == 1 ? reg_product<T, NX, 2, MT_, 8, 1>(dev, g, part) : kw == 2 ? reg_product<T, NX, 2, MT_, 4, 2>(dev, g, part) \
+                                                                              : reg_product<T, NX, 2, MT_, 2, 4>(dev, g, part)
+    switch (mt) {
+    case 1: GO(1);
+    case 2: GO(2);
+    case 3: GO(3);
+    default: GO(4);
+    }
+#undef GO
+}
+
+bool fh_qmm_reg_supports(const fh_qmatrix *q) {
+    switch (q->type) {
+    case FH_Q4_0: case FH_Q5_0: case FH_Q8_0: case FH_Q4_K: case FH_Q5_K: case FH_Q6_K: return q->k % 256 == 0 && q->k <= 16384;
+    }
+    return false;
+}
+
+// Where it is the better way, by timing 17 - 2048 rows of five matrices (14336 x 4096, 4096 x 14336, 4096 x 4096, 1024 x 4096, 5632 x 2048)
+// in six formats and both activation types against the fragments and the tiles; us, this / the others, at the lines:
+//   Q4_K f32   512 rows 140 / 153, 152 / 180, 52 / 76, 32 / 47, 44 / 54; 768 rows 193 / 236, 218 / 245, 70 / 82, 37 / 45, 71 / 66
+//   Q4_K bf16  768 rows 133 / 185, 150 / 209, 50 / 93, 28 / 53, 55 / 91; 1024 rows 186 / 182, 168 / 191, 56 / 69, 30 / 46, 58 / 54
+//   Q5_K f32   512 rows 150 / 156, 159 / 185, 56 / 66, 33 / 46, 47 / 54; 768 rows 224 / 238, 260 / 249; bf16 384 rows 103 / 109,
+//              108 / 112, 512 rows 120 / 117
+//   Q6_K f32   512 rows 175 / 247, 178 / 250, 59 / 91, 33 / 44, 51 / 100; 768 rows 264 / 319 but 87 / 78; bf16 768 rows 205 / 212, 207 / 240,
+//              73 / 100, 1024 rows 278 / 257
+//   Q8_0 f32   512 rows 146 / 194, 153 / 238, 52 / 93, 32 / 44, 43 / 97; 768 rows 218 / 257 but 75 / 69; bf16 768 rows 161 / 178, 180 / 279,
+//              59 / 111, 1024 rows 216 / 212 but 190 / 349, 62 / 123, 31 / 56, 64 / 107 for the smaller n.  Q4_0 as Q8_0.
+//   Q5_0 bf16  512 rows 122 / 136, 118 / 166; 768 rows 71 / 59 for 5632 x 2048
+// Left on the tiles though slower: Q4_K and Q5_0, f32, of rows (from 512, above 192) and matrices for which the tiles win over the fragments
+// (tile_fill; 8192 x 2048).  Fewer than 1024 columns: four 256s are the least that a workgroup's wavefronts share out.
+bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m) {
+    if (!fh_qmm_reg_supports(q) || q->k < 1024) return false;
+    const int64_t n = q->n, k = q->k;
+    switch (q->type) {
+    case FH_Q4_K:
+        if (x_is_bf16) return m <= 768;
+        return m < 512 || (m <= 640 && (k > n || fh_qmm_frag_pays(q, 0, m)));
+    case FH_Q5_K: return m <= (x_is_bf16 ? 448 : 512);
+    case FH_Q5_0:
+        if (x_is_bf16) return m <= 512;
+        return m <= 192 || (m <= 512 && fh_qmm_frag_pays(q, 0, m));
+    case FH_Q6_K: return m <= (x_is_bf16 ? 768 : 512);
+    }
+    return m <= (x_is_bf16 ? (n <= 8192 ? 1280 : 768) : 512); // Q8_0, Q4_0
+}
+
+// How a product is cut: row tiles of activations a workgroup takes (as even as they come out, four at most: registers), groups of
+// wavefronts and workgroups that share out k.  The least of a model fitted to 17 - 192 rows of four matrices: a round of workgroups
+// costs 5 us and, per 256 of k, 1 us (Q6_K 2) and 0.28 us a row tile and product, more of it the fewer wavefronts share their
+// activations; partial planes a launch and their bytes.  whole: k in one part.
+struct RegCut {
+    int mt, kw, parts;
+};
+static RegCut reg_cut(const fh_qmatrix *q, int x_is_bf16, int m, bool whole) {
+    const int chunks = (int)(q->k / 256), tiles = (m + 15) / 16, tx = (tiles + 3) / 4;
+    const int np = (x_is_bf16 ? 1 : 2) + (q->type == FH_Q6_K ? 1 : 0);
+    RegCut best{(tiles + tx - 1) / tx, 1, 1};
+    const double block = (q->type == FH_Q6_K ? 2.0 : 1.0) + 0.28 * best.mt * np; // us of 256 of k
+    double least = 1e30;
+    for (int kw = 1; kw <= 4; kw *= 2)
+        for (int parts = 1; parts <= (whole ? 1 : 16) && parts * kw <= chunks; parts++) {
+            const int64_t groups = (q->n + 16 * 16 / kw - 1) / (16 * 16 / kw) * tx * parts;
+            const int64_t rounds = (groups + q->dev->compute_units - 1) / q->dev->compute_units;
+            const int run = (chunks + parts * kw - 1) / (parts * kw);
+            double t = (double)rounds * (5.0 + run * block * (kw == 1 ? 1.0 : kw == 2 ? 1.13 : 1.4));
+            if (parts > 1) t += 3.4 + (2.0 * parts + 1.0) * m * (double)q->n * 4.0 / 4e6;
+            if (t < least * 0.98) least = t, best.kw = kw, best.parts = parts;
+        }
+    return best;
+}
+
+static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, int half) {
+    fh_device *dev = q->dev;
+    const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2;
+    const RegCut cut = reg_cut(q, x_is_bf16, m, half > 0);
+    RegArgs g{};
+    g.q = fh_view(q);
+    g.m = m, g.n = (int)q->n, g.ldy = half ? half : q->n, g.chunks = k / 256, g.wtiles = (int)((q->n + 15) / 16), g.parts = cut.parts, g.half = half;
+    // activations: up to four row tiles past the last one (rows past m are multiplied and never stored)
+    const int64_t ch = xp * 8192 + (reg_sums(q->type) ? 1024 : 0), xbytes = (((int64_t)m + 15) / 16 + 4) * g.chunks * ch;
+    const size_t part_at = ((size_t)xbytes + ((size_t)m + 80) * 4 + 255) & ~(size_t)255;
+    const size_t bytes = part_at + (cut.parts > 1 ? (size_t)cut.parts * m * q->n * 4 : 0);
+    // as products on fragments do it: what cannot be had is no error, and the tile kernels' planes are there too
+    (void)fh_dev_scratch_try(dev, &dev->act_buf, &dev->act_cap, fh_qmatmul_tile_planes(q, x_is_bf16, m));
+    if (!fh_dev_scratch_try(dev, &dev->frag_x, &dev->frag_x_cap, bytes)) return FH_ERR_UNSUPPORTED;
+    dev->frag_used = true;
+    uint8_t *xf = (uint8_t *)dev->frag_x;
+    float *rs = (float *)(xf + xbytes), *part = (float *)(xf + part_at);
+    g.x = xf, g.rs = rs, g.y = y;
+    const unsigned threads = k / 8 >= 1024 ? 1024 : (unsigned)(k / 8 + 63) / 64 * 64;
+#define REG_X(IN_, O_)                                                                                      \
+    if (k > 8192) k_reg_x<IN_, O_, 2><<<dim3((unsigned)m), threads, 0, dev->stream>>>(x, k, xf, rs);        \
+    else k_reg_x<IN_, O_, 1><<<dim3((unsigned)m), threads, 0, dev->stream>>>(x, k, xf, rs);                 \
+    break
+    switch (reg_order(q->type) + (x_is_bf16 ? 3 : 0)) {
+    case 0: REG_X(0, 0);
+    case 1: REG_X(0, 1);
+    case 2: REG_X(0, 2);
+    case 3: REG_X(1, 0);
+    case 4: REG_X(1, 1);
+    case 5: REG_X(1, 2);
+    }
+#undef REG_X
+    FH_HIP(hipGetLastError());
+#define REG_GO(T_) return x_is_bf16 ? reg_go<T_, 1>(dev, g, part, cut.mt, cut.kw) : reg_go<T_, 2>(dev, g, part, cut.mt, cut.kw)
+    switch (q->type) {
+    case FH_Q4_0: REG_GO(FH_Q4_0);
+    case FH_Q5_0: REG_GO(FH_Q5_0);
+    case FH_Q8_0: REG_GO(FH_Q8_0);
+    case FH_Q4_K: REG_GO(FH_Q4_K);
+    case FH_Q5_K: REG_GO(FH_Q5_K);
+    case FH_Q6_K: REG_GO(FH_Q6_K);
+    }
+#undef REG_GO
+    FH_FAIL(FH_ERR_UNSUPPORTED, "unsupported type %u", q->type);
+}
+
+fh_status fh_launch_qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y) { return qmm_reg(q, x, x_is_bf16, m, y, 0); }
+fh_status fh_qmm_reg_swiglu(const fh_qmatrix *q, const float *x, int m, float *y) { return qmm_reg(q, x, 0, m, y, (int)(q->n / 2)); }

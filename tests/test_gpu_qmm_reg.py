@@ -1,0 +1,102 @@
+"""GPU parity: the matmul that decodes weights in registers (csrc/fh_qmm_reg.hip) against a float64 product of the oracle's
+dequantised weights.
+
+Bound: the operands are exact up to 2^-22 of each activation; products are added in f32, sixteen times 2 or 3 in a chain within a 256,
+then k / 256 of those (each with its offsets, which cancel most of it), and rounding errors (2^-24 each, of either sign) grow with the
+root of their number: 1e-6 of the root of the sum of the squared products (the result's root mean square where there are many of
+them; one result alone may be next to nothing by cancellation) covers k = 16384.  The largest single difference is held to ten
+times that (ten standard deviations)."""
+import numpy as np
+import pytest
+
+from kalosm_amd import synth
+from kalosm_amd.fusor import QMatrix, Tensor
+
+pytestmark = pytest.mark.gpu
+TYPES = [synth.Q4_0, synth.Q5_0, synth.Q8_0, synth.Q4_K, synth.Q5_K, synth.Q6_K]
+
+
+def operands(dev, ty, m, n, k, act, x=None):
+    raw = synth.random_weight(ty, n, k, seed=n + k, sigma=2e-3)
+    x = synth.random_activation(m, k, seed=m) if x is None else x
+    q = QMatrix.from_raw_bytes(dev, (n, k), raw, ty)
+    if act == "f32":
+        return q, Tensor.from_slice(dev, x), x, raw
+    bits = synth.to_bf16_bits(x)
+    return q, Tensor.from_slice(dev, bits, dtype="bf16"), synth.from_bf16_bits(bits), raw
+
+
+def run(dev, q, xt, option):
+    out = Tensor.filled_bytes(dev, (xt.shape[0], q.shape()[0]), 0xFF)  # poisoned: unwritten elements show as NaN
+    dev.set_option("matmul_kernel", option)
+    try:
+        return xt.q_mat_mul(q, out=out).as_slice()
+    finally:
+        dev.set_option("matmul_kernel", 0)
+
+
+@pytest.mark.parametrize("act", ["f32", "bf16"])
+@pytest.mark.parametrize("ty", TYPES, ids=lambda t: synth.TYPE_NAMES[t])
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 256),       # one row, one output, one 256: most wavefronts have nothing of k
+    (17, 33, 1280),    # five 256s over four groups of wavefronts; a second row tile of one row
+    (48, 272, 2304),   # three row tiles; nine 256s
+    (65, 96, 4096),    # five row tiles in two workgroups of three
+    (130, 520, 1024),  # nine row tiles in three workgroups
+    (33, 40, 16384),   # the longest k, in parts
+])
+def test_product(dev, oracle, ty, act, m, n, k):
+    q, xt, x, raw = operands(dev, ty, m, n, k, act)
+    got = run(dev, q, xt, 14).astype(np.float64)
+    x, w = x.astype(np.float64), oracle.dequantize(ty, raw).reshape(n, k).astype(np.float64)
+    want, rms = x @ w.T, np.sqrt(np.mean((x * x) @ (w * w).T))
+    assert np.isfinite(got).all()
+    assert np.sqrt(np.mean((got - want) ** 2)) <= 1e-6 * rms
+    assert np.abs(got - want).max() <= 1e-5 * rms
+
+
+@pytest.mark.parametrize("ty,act,m,n,k,taken", [
+    (synth.Q8_0, "bf16", 1, 64, 1024, True), (synth.Q8_0, "bf16", 1, 64, 768, False),
+    (synth.Q4_K, "f32", 17, 64, 1024, True), (synth.Q4_K, "f32", 16, 64, 1024, False),
+    (synth.Q4_K, "f32", 511, 8192, 2048, True), (synth.Q4_K, "f32", 512, 8192, 2048, False), (synth.Q4_K, "f32", 640, 64, 2048, True),
+    (synth.Q5_0, "f32", 192, 8192, 2048, True), (synth.Q5_0, "f32", 193, 8192, 2048, False),
+    (synth.Q8_0, "bf16", 1280, 64, 1024, True), (synth.Q8_0, "bf16", 769, 8208, 1024, False), (synth.Q6_K, "f32", 513, 64, 1024, False),
+])
+def test_rule(dev, ty, act, m, n, k, taken):
+    """Both sides of the dispatch's lines: the bits of this kernel (option 14) or others."""
+    q, xt, _, _ = operands(dev, ty, m, n, k, act)
+    assert np.array_equal(run(dev, q, xt, 0).view(np.uint32), run(dev, q, xt, 14).view(np.uint32)) == taken
+
+
+@pytest.mark.parametrize("ty", [synth.Q4_K, synth.Q6_K, synth.Q8_0], ids=lambda t: synth.TYPE_NAMES[t])
+def test_rows_are_independent(dev, ty):
+    """Zeros stay zero, a power of two passes through exactly, and an infinity or a NaN stays in its row - also where a group of
+    wavefronts has fewer 256s than others (five over four)."""
+    m, n, k = 40, 96, 1280
+    x = synth.random_activation(m, k, seed=5)
+    q, xt, _, _ = operands(dev, ty, m, n, k, "f32", x.copy())
+    base = run(dev, q, xt, 14)
+    x[3] = 0.0
+    x[4] *= np.float32(2.0 ** 20)
+    x[5, 7] = np.inf
+    x[6, 9] = np.nan
+    got = run(dev, q, Tensor.from_slice(dev, x), 14)
+    assert not got[3].any()
+    assert np.array_equal(got[4], base[4] * np.float32(2.0 ** 20))
+    assert not np.isfinite(got[5]).any() and np.isnan(got[6]).all()
+    rest = [r for r in range(m) if r not in (3, 4, 5, 6)]
+    assert np.array_equal(got[rest], base[rest])
+
+
+@pytest.mark.parametrize("m", [65, 100])
+@pytest.mark.parametrize("ffn", [256, 1280])
+def test_swiglu_epilogue(dev, m, ffn):
+    """gate | up of one launch, SwiGLU at the store, against the two halves as matrices of their own, whose k may be in other
+    parts: each product within 1e-6 of the exact one, so two layers of three products within 1e-5 of each other."""
+    from kalosm_amd.llama import Model
+
+    cfg = dict(n_layers=2, d_model=1024, n_heads=8, n_kv_heads=4, head_dim=128, ffn=ffn, vocab=320, ctx=256, eps=1e-5, theta=1e4)
+    tokens = np.random.default_rng(m).integers(0, 320, m)
+    got = [Model.random_init(dev, cfg, seed=2, sigma=2e-3, fuse_gate_up=fuse).forward(tokens) for fuse in (True, False)]
+    assert np.isfinite(got[0]).all()
+    assert np.sqrt(np.mean((got[0] - got[1]) ** 2)) <= 1e-5 * np.sqrt(np.mean(got[1] ** 2))

@@ -723,7 +723,7 @@ fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, 
 // take 835 us and no 77 of a SwiGLU launch (7 % of a layer was writing and reading what one store now holds).
 fh_status fh_qmm_frag_swiglu(const fh_qmatrix *q, const float *x, int m, float *y) {
     const int64_t opt = q->dev->opt_matmul_kernel;
-    if (q->n % 64 == 0 && ((uintptr_t)x & 15) == 0 && (opt == 0 ? m > FH_SHORT_PROMPT && fh_qmm_reg_pays(q, 0, m) : opt == 14 && fh_qmm_reg_supports(q)))
+    if (q->n % 64 == 0 && ((uintptr_t)x & 15) == 0 && (opt == 0 ? m > FH_SHORT_PROMPT && fh_qmm_reg_pays(q, 0, m) : opt >= 14 && opt <= 16 && fh_qmm_reg_supports(q)))
         return fh_qmm_reg_swiglu(q, x, m, y);
     if (q->n % 64 || ((uintptr_t)x & 15) || m <= 16 || !(opt == 0 ? m > FH_SHORT_PROMPT && fh_qmm_frag_pays(q, 0, m) : opt == 13 && fh_qmm_frag_supports(q)))
         return FH_ERR_UNSUPPORTED;

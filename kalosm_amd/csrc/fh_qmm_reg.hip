@@ -47,42 +47,53 @@ __device__ __forceinline__ void reg_x_read(const void *xin, int64_t row, int k, 
     else v[0] = p.x, v[1] = p.z, v[2] = p.y, v[3] = p.w, v[4] = q.x, v[5] = q.z, v[6] = q.y, v[7] = q.w;
 }
 
-// One workgroup: a row, G groups of eight a thread in registers between the maximum and the conversion.
-template <int IN, int ORDER, int G>
-__global__ __launch_bounds__(1024) void k_reg_x(const void *__restrict__ xin, int k, uint8_t *__restrict__ out, float *__restrict__ rs) {
+// One workgroup: ROWS rows (1, or 8 for whole 128-byte pieces of the operands), G groups of eight a thread in registers between the
+// maximum and the conversion; G = 0: read twice.  WIDE: operands of 32 rows and 16 of k instead (k_qmm_wide).
+template <int IN, int ORDER, int G, bool WIDE, int ROWS>
+__global__ __launch_bounds__(1024) void k_reg_x(const void *__restrict__ xin, int m, int k, uint8_t *__restrict__ out, float *__restrict__ rs) {
     constexpr bool SUMS = ORDER == 1;
-    constexpr int CH = (IN == 1 ? 8 : 16) * 1024 + (SUMS ? 1024 : 0);
-    __shared__ float s_max[16], sums[SUMS ? G * 256 : 1];
-    const int tid = threadIdx.x, row = (int)blockIdx.x, groups = k >> 3;
-    float v[G][8], amax = 0.f;
+    constexpr int CH = (IN == 1 ? 8 : 16) * (WIDE ? 2048 : 1024) + (SUMS ? 1024 : 0);
+    __shared__ float s_max[16][ROWS], sums[SUMS ? 512 * ROWS : 1]; // k <= 16384
+    const int tid = threadIdx.x, r = tid % ROWS, row = (int)blockIdx.x * ROWS + r, groups = k >> 3, step = (int)blockDim.x / ROWS;
+    const int from = row < m ? row : m - 1;
+    float v[G ? G : 1][8], amax = 0.f;
+    auto most = [&](const float (&w)[8]) {
 #pragma unroll
-    for (int i = 0; i < G; i++) {
-        const int gi = tid + i * (int)blockDim.x;
-        reg_x_read<IN, ORDER>(xin, row, k, gi < groups ? gi : groups - 1, v[i]);
+        for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(w[j]));
+    };
+    if (G) {
+#pragma unroll
+        for (int i = 0; i < G; i++) {
+            const int gi = tid / ROWS + i * step;
+            reg_x_read<IN, ORDER>(xin, from, k, gi < groups ? gi : groups - 1, v[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < G; i++) most(v[i]);
+    } else {
+#pragma unroll 4
+        for (int gi = tid / ROWS; gi < groups; gi += step) {
+            float w[8];
+            reg_x_read<IN, ORDER>(xin, from, k, gi, w);
+            most(w);
+        }
     }
 #pragma unroll
-    for (int i = 0; i < G; i++)
-#pragma unroll
-        for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(v[i][j]));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
-    if ((tid & 63) == 0) s_max[tid >> 6] = amax;
+    for (int o = 32; o >= ROWS; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    if ((tid & 63) < ROWS) s_max[tid >> 6][r] = amax;
     __syncthreads();
-    for (int i = 0; i < (int)blockDim.x >> 6; i++) amax = fmaxf(amax, s_max[i]);
+    for (int i = 0; i < (int)blockDim.x >> 6; i++) amax = fmaxf(amax, s_max[i][r]);
     int e = 141 - (int)((__float_as_uint(amax) >> 23) & 0xFFu); // 14 - floor(log2 amax); zero / inf / nan clamp
     e = e > 100 ? 100 : (e < -100 ? -100 : e);
     const bool infrow = amax == INFINITY; // finite values vanish next to an infinity, which is carried as +-32768
     const float sc = __uint_as_float((uint32_t)(e + 127) << 23);
-    if (tid == 0) rs[row] = infrow ? INFINITY : __uint_as_float((uint32_t)(127 - e) << 23);
-    uint8_t *dst = out + (int64_t)(row >> 4) * (k >> 8) * CH + (row & 15) * 16;
-#pragma unroll
-    for (int i = 0; i < G; i++) {
-        const int gi = tid + i * (int)blockDim.x;
+    if (tid < ROWS && row < m) rs[row] = infrow ? INFINITY : __uint_as_float((uint32_t)(127 - e) << 23);
+    uint8_t *dst = WIDE ? out + (int64_t)(row >> 5) * (k >> 8) * CH + (row & 31) * 16 : out + (int64_t)(row >> 4) * (k >> 8) * CH + (row & 15) * 16;
+    auto put = [&](int gi, const float (&x)[8]) {
         _Float16 h[8], l[8];
         float t = 0.f;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            float w = v[i][j] * sc;
+            float w = x[j] * sc;
             if (infrow && fabsf(w) == INFINITY) w = copysignf(32768.f, w);
             h[j] = (_Float16)w;
             const float d = w - (float)h[j];
@@ -90,37 +101,50 @@ __global__ __launch_bounds__(1024) void k_reg_x(const void *__restrict__ xin, in
             t += w;
         }
         if (SUMS) { // of 32: four threads
-            t += __shfl_xor(t, 1, 64);
-            t += __shfl_xor(t, 2, 64);
-            if ((gi & 3) == 0 && gi < groups) sums[gi >> 2] = t * 0.015625f;
+            t += __shfl_xor(t, ROWS, 64);
+            t += __shfl_xor(t, 2 * ROWS, 64);
+            if ((gi & 3) == 0 && gi < groups) sums[(gi >> 2) * ROWS + r] = t * 0.015625f;
         }
-        if (gi < groups) {
-            uint8_t *p = dst + (int64_t)(gi >> 5) * CH + ((gi >> 2) & 7) * 1024 + (gi & 3) * 256;
+        if (gi < groups && row < m) {
+            // a block's eights 0 and 2 are the halves of one wide operand, 1 and 3 of the other
+            uint8_t *p = dst + (int64_t)(gi >> 5) * CH + (WIDE ? ((gi >> 2) & 7) * 2048 + (gi & 1) * 1024 + (gi & 2) * 256 : ((gi >> 2) & 7) * 1024 + (gi & 3) * 256);
             uint4 u;
             __builtin_memcpy(&u, h, 16);
             *(uint4 *)p = u;
             if (IN != 1) {
                 __builtin_memcpy(&u, l, 16);
-                *(uint4 *)(p + 8192) = u;
+                *(uint4 *)(p + (WIDE ? 16384 : 8192)) = u;
             }
         }
-    }
+    };
+    if (G) {
+#pragma unroll
+        for (int i = 0; i < G; i++) put(tid / ROWS + i * step, v[i]);
+    } else
+        for (int at = 0; at < groups; at += step) { // (all threads together: the sums go through their neighbours)
+            const int gi = at + tid / ROWS;
+            float w[8];
+            reg_x_read<IN, ORDER>(xin, from, k, gi < groups ? gi : groups - 1, w);
+            put(gi, w);
+        }
     if (!SUMS) return;
     __syncthreads();
     // a 256's sums: hi in lane group 0, lo in 1, zeros in 2 and 3
-    for (int i = tid; i < (k >> 6); i += (int)blockDim.x) {
-        const int c = i >> 2, g = i & 3;
-        _Float16 h[8];
+    if (row < m)
+        for (int i = tid / ROWS; i < (k >> 6); i += step) {
+            const int c = i >> 2, g = i & 3;
+            _Float16 h[8];
 #pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const float s = sums[c * 8 + b];
-            const _Float16 sh = (_Float16)s;
-            h[b] = g == 0 ? sh : g == 1 ? (_Float16)(s - (float)sh) : (_Float16)0.f;
+            for (int b = 0; b < 8; b++) {
+                const float s = sums[(c * 8 + b) * ROWS + r];
+                const _Float16 sh = (_Float16)s;
+                h[b] = g == 0 ? sh : g == 1 ? (_Float16)(s - (float)sh) : (_Float16)0.f;
+            }
+            uint4 u;
+            __builtin_memcpy(&u, h, 16);
+            if (!WIDE) *(uint4 *)(dst + (int64_t)c * CH + CH - 1024 + g * 256) = u;
+            else if (g < 2) *(uint4 *)(dst + (int64_t)c * CH + CH - 1024 + g * 512) = u;
         }
-        uint4 u;
-        __builtin_memcpy(&u, h, 16);
-        *(uint4 *)(dst + (int64_t)c * CH + CH - 1024 + g * 256) = u;
-    }
 }
 
 // ------------------------------------------------------------------------------ weights
@@ -546,6 +570,359 @@ __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
     }
 }
 
+// ------------------------------------------------------------------------------ wide product
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+// Two row tiles' (32 rows') 256 of k for v_mfma_f32_32x32x16_f16.  The tiles' registers [A0 A1 A2 A3], [B0 B1 B2 B3] (16 lanes each, k in
+// eights) become [A0 B0 A2 B2], [A1 B1 A3 B3] by one v_permlane16_swap each: operands of 32 rows with eights 0 and 2, 1 and 3 of a block.
+// Slots are what a request brings: SL of them are a 256, two are held.  A lane's row is lane % 32, its header, scales and sums that row's.
+__device__ __forceinline__ void reg_swap(uint32_t &a, uint32_t &b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+__device__ __forceinline__ void reg_swap(uint4 &a, uint4 &b) { reg_swap(a.x, b.x), reg_swap(a.y, b.y), reg_swap(a.z, b.z), reg_swap(a.w, b.w); }
+
+template <int T>
+struct WideW {
+    static constexpr bool K4 = T == FH_Q4_K || T == FH_Q5_K, Q6 = T == FH_Q6_K, Q8 = T == FH_Q8_0;
+    static constexpr int REC = T == FH_Q4_K ? 2304 : T == FH_Q5_K ? 2816 : Q6 ? 3360 : Q8 ? 4352 : T == FH_Q5_0 ? 2816 : 2304;
+    static constexpr int SL = Q8 ? 4 : 2, NW = Q6 ? 2 : 1; // slots of a 256
+    static constexpr int SLOT = K4 || Q6 ? 0 : REC / SL;   // bytes of one (formats with a scale per 32)
+    // requests of a slot, and those of a 256's header
+    static constexpr int QS = K4 || Q6 ? 2 : T == FH_Q5_0 ? 5 : 3, QH = T == FH_Q4_K ? 1 : T == FH_Q5_K ? 3 : Q6 ? 7 : 0;
+    uint4 cod[2][2];
+    uint32_t five[2][2]; // Q5_0: a slot's fifth bits
+    uint2 dd[2];         // scales of a slot's blocks
+    uint4 head, hi[2], next_hi[2];
+    uint2 five_k[2], next5[2]; // Q5_K: a 256's
+    uint32_t dm, sc[4], next_sc[4], mn[2];
+    uint16_t next_d;
+
+    // a, b: the tiles' records of a 256, own: the one of this lane's row
+    __device__ __forceinline__ void ask(int s, const uint8_t *a, const uint8_t *b, int lane) {
+        const int o = K4 ? 256 + s * 1024 : Q6 ? s * 1024 : s * SLOT;
+        cod[s & 1][0] = *(const uint4 *)(a + o + lane * 16);
+        cod[s & 1][1] = *(const uint4 *)(b + o + lane * 16);
+        if (K4 || Q6) return;
+        if (T == FH_Q5_0) {
+            five[s & 1][0] = *(const uint32_t *)(a + o + 1152 + lane * 4);
+            five[s & 1][1] = *(const uint32_t *)(b + o + 1152 + lane * 4);
+        }
+        const uint8_t *own = (lane & 16 ? b : a) + o + 1024;
+        if (Q8) dd[s & 1].x = *(const uint32_t *)(own + (lane & 15) * 4);
+        else dd[s & 1] = *(const uint2 *)(own + (lane & 15) * 8);
+    }
+    __device__ __forceinline__ void ask_head(const uint8_t *a, const uint8_t *b, int lane) {
+        const uint8_t *own = lane & 16 ? b : a;
+        if (K4) head = *(const uint4 *)(own + (lane & 15) * 16);
+        if (T == FH_Q5_K) next5[0] = *(const uint2 *)(a + 2304 + lane * 8), next5[1] = *(const uint2 *)(b + 2304 + lane * 8);
+        if (Q6) {
+            next_hi[0] = *(const uint4 *)(a + 2048 + lane * 16), next_hi[1] = *(const uint4 *)(b + 2048 + lane * 16);
+#pragma unroll
+            for (int q = 0; q < 4; q++) next_sc[q] = *(const uint32_t *)(own + 3072 + (q * 16 + (lane & 15)) * 4);
+            next_d = fh_ld16(own + 3328 + (lane & 15) * 2);
+        }
+    }
+    __device__ __forceinline__ void begin_head(int lane) {
+        if (K4) {
+            dm = head.x;
+            sc[0] = head.y & 0x3F3F3F3Fu, sc[1] = (head.w & 0x0F0F0F0Fu) | ((head.y >> 2) & 0x30303030u);
+            mn[0] = head.z & 0x3F3F3F3Fu, mn[1] = ((head.w >> 4) & 0x0F0F0F0Fu) | ((head.z >> 2) & 0x30303030u);
+        }
+        if (T == FH_Q5_K) {
+            five_k[0] = next5[0], five_k[1] = next5[1];
+            reg_swap(five_k[0].x, five_k[1].x), reg_swap(five_k[0].y, five_k[1].y);
+        }
+        if (Q6) {
+            hi[0] = next_hi[0], hi[1] = next_hi[1], dm = next_d;
+            reg_swap(hi[0], hi[1]);
+#pragma unroll
+            for (int q = 0; q < 4; q++) sc[q] = (next_sc[q] ^ 0x80808080u) >> ((lane >> 5) * 8); // bytes 0 and 2: the one of this lane's k
+        }
+    }
+    __device__ __forceinline__ void begin(int s) {
+        reg_swap(cod[s & 1][0], cod[s & 1][1]);
+        if (T == FH_Q5_0) reg_swap(five[s & 1][0], five[s & 1][1]);
+    }
+    // block e's operand h (eights 0 and 2, or 1 and 3)
+    __device__ __forceinline__ void get(int e, int h, uint32_t one, half8 (&out)[NW]) const {
+        const int s = e * SL / 8, u = e % (8 / SL);
+        const uint4 c = cod[s & 1][h];
+        half2v r[4], r2[4];
+        if (K4) {
+            const int hn = e & 1;
+            const uint32_t w[2] = {e & 2 ? c.z : c.x, e & 2 ? c.w : c.y}, f[2] = {five_k[h].x, five_k[h].y};
+            const half2v k = reg_h2(__builtin_amdgcn_perm(0x64646464u, sc[e >> 2], 0x04000400u + (uint32_t)(e & 3) * 0x00010001u)) - reg_splat(1024.f);
+            const half2v a = hn ? k * reg_splat(0.0625f) : k, b = k * reg_splat(hn ? -64.f : -1024.f);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint32_t v = (((i & 1) ? w[i >> 1] >> 8 : w[i >> 1]) & (hn ? 0x00F000F0u : 0x000F000Fu)) | one;
+                if (T == FH_Q5_K) {
+                    const int from = e + 8 * (i & 1), to = hn ? 8 : 4;
+                    v |= (from > to ? f[i >> 1] >> (from - to) : f[i >> 1] << (to - from)) & (hn ? 0x01000100u : 0x00100010u);
+                }
+                r[i] = __builtin_elementwise_fma(reg_h2(v), a, b);
+            }
+        } else if (Q6) {
+            const uint32_t l = (e & 3) == 0 ? c.x : (e & 3) == 1 ? c.y : (e & 3) == 2 ? c.z : c.w;
+            const uint32_t t = (e >> 1) == 0 ? hi[h].x : (e >> 1) == 1 ? hi[h].y : (e >> 1) == 2 ? hi[h].z : hi[h].w;
+            const half2v k = (e < 4 ? reg_bytes<0, 0>(sc[e & 3]) : reg_bytes<2, 2>(sc[e & 3])) - reg_splat(1152.f);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int from = q6k_hbit(e, i);
+                const uint32_t v = (((l >> (4 * i)) & 0x000F000Fu) | one) | ((from > 4 ? t >> (from - 4) : t << (4 - from)) & 0x00300030u);
+                const half2v q = reg_h2(v) - reg_splat(1056.f);
+                r[i] = q * k;
+                r2[i] = __builtin_elementwise_fma(q, k, -r[i]);
+            }
+            out[NW - 1] = reg_cat(r2);
+        } else if (Q8) {
+            const uint32_t x = (u ? c.z : c.x) ^ 0x80808080u, y = (u ? c.w : c.y) ^ 0x80808080u;
+            const half2v k = reg_splat(1152.f);
+            r[0] = reg_bytes<0, 1>(x) - k, r[1] = reg_bytes<2, 3>(x) - k, r[2] = reg_bytes<0, 1>(y) - k, r[3] = reg_bytes<2, 3>(y) - k;
+        } else {
+            const uint32_t w = u == 0 ? c.x : u == 1 ? c.y : u == 2 ? c.z : c.w, f = five[s & 1][h];
+            const uint32_t lo5 = (f >> (8 * u)) & 15u, hi5 = (f >> (8 * u + 4)) & 15u;
+            const float off = T == FH_Q5_0 ? 16.f : 8.f;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                uint32_t a = ((i ? w >> 8 : w) & 0x000F000Fu) | one, b = ((i ? w >> 8 : w) & 0x00F000F0u) | one;
+                if (T == FH_Q5_0) {
+                    a |= (lo5 * (i ? 0x20008u : 0x40010u)) & 0x00100010u;
+                    b |= (hi5 * (i ? 0x200080u : 0x400100u)) & 0x01000100u;
+                }
+                r[i] = reg_h2(a) - reg_splat(1024.f + off);
+                r[2 + i] = __builtin_elementwise_fma(reg_h2(b), reg_splat(0.0625f), reg_splat(-64.f - off));
+            }
+        }
+        out[0] = reg_cat(r);
+    }
+    __device__ __forceinline__ float scale(int e) const { // of block e (formats with one per 32), of the 256
+        if (K4 || Q6) return fh_h2f((uint16_t)(dm & 0xFFFFu));
+        const int s = e * SL / 8, u = e % (8 / SL);
+        return fh_h2f((uint16_t)((u & 2 ? dd[s & 1].y : dd[s & 1].x) >> (16 * (u & 1))));
+    }
+    __device__ __forceinline__ float offset() const { return -64.f * fh_h2f((uint16_t)(dm >> 16)); }
+    __device__ __forceinline__ half8 offsets() const {
+        const half2v k = reg_splat(1024.f), r[4] = {reg_bytes<0, 1>(mn[0]) - k, reg_bytes<2, 3>(mn[0]) - k, reg_bytes<0, 1>(mn[1]) - k, reg_bytes<2, 3>(mn[1]) - k};
+        return reg_cat(r);
+    }
+};
+
+// A wavefront: two pairs of row tiles (64 rows, for SwiGLU 32 of gate and 32 of up) by MX groups of 32 rows of activations; four
+// wavefronts side by side along the weight rows, 256 x 32 MX a workgroup, two of which share a compute unit.  What bounds it is the vector
+// ALU beside the matrix cores (Q8_0, one plane: 7.4 vector instructions for the work of a 16 x 16 x 32 product, of which two hide), so
+//   products are the 32 x 32 x 16 ones, which leave it more room (16 of their half-size and 128 vector instructions of two wavefronts
+//   take 307 ns, as 16 x 16 x 32 ones 370);
+//   the two workgroups drift apart, and one decodes while the other multiplies: as one of eight wavefronts, in step at every barrier, 2048
+//   rows of 14336 x 4096 took 393 us in Q8_0 (333 so), 332 in Q4_K (289), bf16;
+//   the tiles that run together on a die are eight weight tiles by eight of activations (as two by 32: 358 and 304).
+template <int T, int NX, int MX>
+struct WideTile {
+    static constexpr int SB = 2, PIECES = NX * MX * 2 * SB, FR = PIECES / 4, STAGE = PIECES * 1024;
+    static constexpr int FIT = 81920 / STAGE, ST = FIT > 6 ? 6 : FIT, LDS = ST * STAGE;
+    static constexpr int CH = NX * 16384 + (reg_sums(T) ? 1024 : 0);
+    static_assert(ST >= 4 && PIECES % 4 == 0, "four stages at least");
+    typedef WideW<T> W;
+    static constexpr int wreq(int e) {
+        return (e % (8 / W::SL) == 0 ? 2 * W::QS : 0) + (e == 8 - 8 / W::SL ? 2 * W::QH : 0) + (e == 6 && reg_sums(T) ? MX : 0);
+    }
+    static constexpr int younger(int e) { // as RegTile::younger
+        int n = 0;
+        for (int b = 1; b <= (ST - 3) * SB; b++) n += (b % SB == 0 ? FR : 0) + wreq((e + 64 - b) & 7);
+        return n > 63 ? 63 : n;
+    }
+};
+
+template <int T, int NX, int MX>
+__global__ __launch_bounds__(256, 2) void k_qmm_wide(RegArgs g) {
+    typedef WideTile<T, NX, MX> Tile;
+    typedef WideW<T> W;
+    constexpr int FR = Tile::FR, STAGE = Tile::STAGE, ST = Tile::ST, CH = Tile::CH, SB = Tile::SB, SL = W::SL;
+    constexpr bool SUMS = reg_sums(T), PER32 = !SUMS && T != FH_Q6_K;
+    constexpr int NW = W::NW, NP = NW == 2 ? NX + 1 : NX, XB = NX * MX * 2; // operands of a block: [plane][eights][group]
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int total = g.tiles_w * g.tiles_x, per = total >> 3, more = total & 7, die = (int)blockIdx.x & 7;
+    const int lin = ((int)blockIdx.x >> 3) + die * per + (die < more ? die : more);
+    const int group = lin / (8 * g.tiles_x), in = lin - group * 8 * g.tiles_x; // eight weight tiles by all others, weight tiles first
+    const int gw = g.tiles_w - group * 8 < 8 ? g.tiles_w - group * 8 : 8;
+    const int tw = group * 8 + in % gw, tx = in / gw;
+    const int most = g.chunks;
+    auto chunk = [&](int i) { return i < most ? i : most - 1; };
+    int row0[2];
+    const uint8_t *ra[2], *rb[2];
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        const int w = tw * 4 + wave;
+        row0[p] = g.half ? p * g.half + w * 32 : w * 64 + p * 32;
+        const int a = row0[p] >> 4, b = a + 1;
+        ra[p] = g.q.data + (int64_t)(a < g.wtiles ? a : g.wtiles - 1) * g.chunks * W::REC;
+        rb[p] = g.q.data + (int64_t)(b < g.wtiles ? b : g.wtiles - 1) * g.chunks * W::REC;
+    }
+    const uint8_t *xt = g.x + (int64_t)tx * MX * g.chunks * CH;
+    auto fetch = [&](int c, int e, int buf) { // the stage from block e of the 256 c on into the buffer at byte `buf`
+#pragma unroll
+        for (int i = 0; i < FR; i++) {
+            const int u = wave + 4 * i, v = u / XB, p = u % XB / (2 * MX), h = u / MX % 2, m = u % MX;
+            fh_buffer_to_lds(xt, MX * g.chunks * CH, smem + buf + u * 1024, lane * 16, (m * g.chunks + c) * CH + p * 16384 + (e + v) * 2048 + h * 1024);
+        }
+    };
+    W w[2];
+    floatx16 acc[2][MX], sum[PER32 ? 1 : 2][PER32 ? 2 : MX];
+    const floatx16 zero = {0.f};
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+        for (int m = 0; m < MX; m++) acc[p][m] = zero;
+    half8 xs[MX];
+    int cur = 0;
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        w[p].ask_head(ra[p] + (int64_t)chunk(0) * W::REC, rb[p] + (int64_t)chunk(0) * W::REC, lane);
+        w[p].ask(0, ra[p] + (int64_t)chunk(0) * W::REC, rb[p] + (int64_t)chunk(0) * W::REC, lane);
+    }
+#pragma unroll
+    for (int i = 0; i < ST - 1; i++) fetch(chunk(i * SB >> 3), i * SB & 7, i * STAGE);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (the counts of the first steps are those of later ones, with more requests)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    half8 xv[XB], wv[2][2][NW];
+#pragma unroll
+    for (int u = 0; u < XB; u++) xv[u] = *(const half8 *)(smem + u * 1024 + lane * 16);
+    uint32_t one;
+    asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(one));
+    float d32 = 0.f;
+    if (PER32) sum[0][1] = zero;
+    for (int i = 0; i < most; i++) {
+        const int c0 = chunk(i), c1 = chunk(i + 1);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            constexpr int PER = 8 / SL; // blocks of a slot
+            if (e % SB == 0) {
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Tile::younger(e)) : "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (e % PER == 0) {
+                const int s = e / PER, c = s + 1 < SL ? c0 : c1;
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    if (s == 0) w[p].begin_head(lane);
+                    w[p].begin(s);
+                }
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    if (s == SL - 1) w[p].ask_head(ra[p] + (int64_t)c * W::REC, rb[p] + (int64_t)c * W::REC, lane);
+                    w[p].ask((s + 1) % SL, ra[p] + (int64_t)c * W::REC, rb[p] + (int64_t)c * W::REC, lane);
+                }
+            }
+            if (SUMS && e == 6)
+#pragma unroll
+                for (int m = 0; m < MX; m++) xs[m] = *(const half8 *)(xt + (m * g.chunks + c0) * CH + CH - 1024 + lane * 16);
+            __builtin_amdgcn_sched_barrier(0);
+            if (e % SB == 0) {
+                constexpr int AHEAD = (ST - 1) * SB; // blocks
+                fetch(chunk(i + (e + AHEAD) / 8), (e + AHEAD) & 7, cur == 0 ? (ST - 1) * STAGE : cur - STAGE);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const int nb = e % SB == SB - 1 ? (cur + STAGE == ST * STAGE ? 0 : cur + STAGE) : cur;
+            const uint8_t *b = smem + nb + (e + 1) % SB * XB * 1024 + lane * 16; // the next block's activations
+            if (PER32 && e % PER == 0) w[0].get(e, 0, one, wv[0][0]), w[0].get(e, 1, one, wv[0][1]);
+#pragma unroll
+            for (int p = 0; p < 2; p++) { // the next pair's (block's) weights are decoded while this one's are multiplied
+                if (!PER32) w[p].get(e, 0, one, wv[p][0]), w[p].get(e, 1, one, wv[p][1]);
+                else if (p == 0 || (e + 1) % PER) w[p ^ 1].get(e + p, 0, one, wv[p ^ 1][0]), w[p ^ 1].get(e + p, 1, one, wv[p ^ 1][1]);
+                if (PER32) {
+                    float d = w[p].scale(e);
+                    asm volatile("" : "+v"(d)); // (an f32 of its own: fused into the multiply-adds the conversion makes them the slow mixed ones)
+#pragma unroll
+                    for (int m = 0; m < MX; m++) { // a finished sum is scaled while the next is multiplied
+                        const int at = (p * MX + m) & 1;
+#pragma unroll
+                        for (int v = 0; v < NX * 2; v++)
+                            sum[0][at] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xv[(v >> 1) * 2 * MX + (v & 1) * MX + m], wv[p][v & 1][0], v ? sum[0][at] : zero, 0, 0, 0);
+                        const int pp = m ? p : p ^ 1, pm = m ? m - 1 : MX - 1;
+#pragma unroll
+                        for (int r = 0; r < 16; r++) acc[pp][pm][r] = fmaf(sum[0][at ^ 1][r], d32, acc[pp][pm][r]);
+                        d32 = d;
+                        if (p)
+#pragma unroll
+                            for (int v = 0; v < NX * 2; v++) {
+                                const int u = (v >> 1) * 2 * MX + (v & 1) * MX + m;
+                                xv[u] = *(const half8 *)(b + u * 1024);
+                            }
+#pragma unroll
+                        for (int v = 0; v < NX * 2; v++) {
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x002, (16 + 44 / MX) / (NX * 2), 0);
+                            if (p) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < MX * NP * 2; j++) {
+                        const int m = j % MX, v = j / MX, h = v & 1, q = v >> 1;
+                        sum[p][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xv[(q < NX ? q : 0) * 2 * MX + h * MX + m], wv[p][h][q < NX ? 0 : NW - 1],
+                                                                           e == 0 && v == 0 ? zero : sum[p][m], 0, 0, 0);
+                    }
+                    if (p)
+#pragma unroll
+                        for (int u = 0; u < XB; u++) xv[u] = *(const half8 *)(b + u * 1024);
+                }
+            }
+            if (e % SB == SB - 1) cur = cur + STAGE == ST * STAGE ? 0 : cur + STAGE;
+        }
+        if (!PER32)
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const float d = w[p].scale(0);
+                if constexpr (SUMS) {
+                    const float o = w[p].offset();
+                    const half8 ov = w[p].offsets();
+#pragma unroll
+                    for (int m = 0; m < MX; m++) {
+                        const floatx16 so = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs[m], ov, zero, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 16; r++) acc[p][m][r] += fmaf(sum[p][m][r], d, so[r] * o);
+                    }
+                } else
+#pragma unroll
+                    for (int m = 0; m < MX; m++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++) acc[p][m][r] = fmaf(sum[p][m][r], d, acc[p][m][r]);
+            }
+    }
+    if (PER32)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[1][MX - 1][r] = fmaf(sum[0][1][r], d32, acc[1][MX - 1][r]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // no LDS-direct load outlives its buffer
+    float *y = g.y;
+#pragma unroll
+    for (int m = 0; m < MX; m++) {
+        float rs[16]; // ahead of the stores: a load between them would wait for the stores before it
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+            const float4 v = *(const float4 *)(g.rs + (tx * MX + m) * 32 + 2 * r + 4 * (lane >> 5));
+            rs[r] = v.x, rs[r + 1] = v.y, rs[r + 2] = v.z, rs[r + 3] = v.w;
+        }
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const int nn = row0[p] + (lane & 31);
+            if (nn >= (g.half ? g.half : g.n) || (g.half && p)) continue;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int mm = (tx * MX + m) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                float v = acc[p][m][r] * rs[r];
+                if (g.half) v = (v / (expf(-v) + 1.0f)) * (acc[1][m][r] * rs[r]);
+                if (mm < g.m) y[mm * g.ldy + nn] = v;
+            }
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------ launches
 template <int T, int NX, int TW, int MT, int WW, int KW>
 static fh_status reg_product(fh_device *dev, RegArgs g, float *part) {
@@ -578,6 +955,17 @@ static fh_status reg_go(fh_device *dev, const RegArgs &g, float *part, int mt, i
 #undef GO
 }
 
+template <int T, int NX, int MX>
+static fh_status wide_product(fh_device *dev, RegArgs g) {
+    typedef WideTile<T, NX, MX> Tile;
+    const int n = g.half ? g.half * 2 : g.n;
+    g.tiles_w = (n + 255) / 256;
+    g.tiles_x = (g.m + MX * 32 - 1) / (MX * 32);
+    FH_TRY(fh_kernel_lds(dev, (const void *)k_qmm_wide<T, NX, MX>, (size_t)Tile::LDS));
+    k_qmm_wide<T, NX, MX><<<dim3((unsigned)(g.tiles_w * g.tiles_x)), 256, Tile::LDS, dev->stream>>>(g);
+    FH_HIP(hipGetLastError());
+    return FH_OK;
+}
 bool fh_qmm_reg_supports(const fh_qmatrix *q) {
     switch (q->type) {
     case FH_Q4_0: case FH_Q5_0: case FH_Q8_0: case FH_Q4_K: case FH_Q5_K: case FH_Q6_K: return q->k % 256 == 0 && q->k <= 16384;
@@ -585,21 +973,50 @@ bool fh_qmm_reg_supports(const fh_qmatrix *q) {
     return false;
 }
 
-// Where it is the better way, by timing 17 - 2048 rows of five matrices (14336 x 4096, 4096 x 14336, 4096 x 4096, 1024 x 4096, 5632 x 2048)
+// How a product is cut: row tiles of activations a workgroup takes (as even as they come out, four at most: registers), groups of
+// wavefronts and workgroups that share out k.  The least of a model fitted to 17 - 192 rows of four matrices: a round of workgroups
+// costs 5 us and, per 256 of k, 1 us (Q6_K 2) and 0.28 us a row tile and product, more of it the fewer wavefronts share their
+// activations; partial planes a launch and their bytes.  whole: k in one part.
+struct RegCut {
+    int mt, kw, parts;
+    double us;
+};
+static RegCut reg_cut(const fh_qmatrix *q, int x_is_bf16, int m, bool whole) {
+    const int chunks = (int)(q->k / 256), tiles = (m + 15) / 16, tx = (tiles + 3) / 4;
+    const int np = (x_is_bf16 ? 1 : 2) + (q->type == FH_Q6_K ? 1 : 0);
+    RegCut best{(tiles + tx - 1) / tx, 1, 1, 0.0};
+    const double block = (q->type == FH_Q6_K ? 2.0 : 1.0) + 0.28 * best.mt * np; // us of 256 of k
+    double least = 1e30;
+    for (int kw = 1; kw <= 4; kw *= 2)
+        for (int parts = 1; parts <= (whole ? 1 : 16) && parts * kw <= chunks; parts++) {
+            if (x_is_bf16 && q->k >= 8192 && parts * kw < 2) continue; // (one chain along a long k is less exact than the tiles' parted ones)
+            const int64_t groups = (q->n + 16 * 16 / kw - 1) / (16 * 16 / kw) * tx * parts;
+            const int64_t rounds = (groups + q->dev->compute_units - 1) / q->dev->compute_units;
+            const int run = (chunks + parts * kw - 1) / (parts * kw);
+            double t = (double)rounds * (5.0 + run * block * (kw == 1 ? 1.0 : kw == 2 ? 1.13 : 1.4));
+            if (parts > 1) t += 3.4 + (2.0 * parts + 1.0) * m * (double)q->n * 4.0 / 4e6;
+            if (t < least * 0.98) least = t, best.kw = kw, best.parts = parts;
+        }
+    const bool five = q->type == FH_Q5_0 || q->type == FH_Q5_K;
+    const double type = q->type == FH_Q6_K ? 0.92 : q->type == FH_Q4_K ? 1.15 : five ? (x_is_bf16 ? 1.5 : 1.33) : 1.25;
+    best.us = 8.0 + m * (double)q->k / 1e6 * 1.6 + type * least; // (with the activations' launch; from 320 rows on, where there is a choice)
+    return best;
+}
+
+// Few rows: where k_qmm_reg is the better way, by timing 17 - 2048 rows of five matrices (14336 x 4096, 4096 x 14336, 4096 x 4096, 1024 x 4096, 5632 x 2048)
 // in six formats and both activation types against the fragments and the tiles; us, this / the others, at the lines:
 //   Q4_K f32   512 rows 140 / 153, 152 / 180, 52 / 76, 32 / 47, 44 / 54; 768 rows 193 / 236, 218 / 245, 70 / 82, 37 / 45, 71 / 66
 //   Q4_K bf16  768 rows 133 / 185, 150 / 209, 50 / 93, 28 / 53, 55 / 91; 1024 rows 186 / 182, 168 / 191, 56 / 69, 30 / 46, 58 / 54
 //   Q5_K f32   512 rows 150 / 156, 159 / 185, 56 / 66, 33 / 46, 47 / 54; 768 rows 224 / 238, 260 / 249; bf16 384 rows 103 / 109,
 //              108 / 112, 512 rows 120 / 117
 //   Q6_K f32   512 rows 175 / 247, 178 / 250, 59 / 91, 33 / 44, 51 / 100; 768 rows 264 / 319 but 87 / 78; bf16 768 rows 205 / 212, 207 / 240,
-//              73 / 100, 1024 rows 278 / 257
+//              73 / 100, 1024 rows 278 / 257; of 14336 columns 400 rows 148 / 145, 512 152 / 148
 //   Q8_0 f32   512 rows 146 / 194, 153 / 238, 52 / 93, 32 / 44, 43 / 97; 768 rows 218 / 257 but 75 / 69; bf16 768 rows 161 / 178, 180 / 279,
 //              59 / 111, 1024 rows 216 / 212 but 190 / 349, 62 / 123, 31 / 56, 64 / 107 for the smaller n.  Q4_0 as Q8_0.
 //   Q5_0 bf16  512 rows 122 / 136, 118 / 166; 768 rows 71 / 59 for 5632 x 2048
 // Left on the tiles though slower: Q4_K and Q5_0, f32, of rows (from 512, above 192) and matrices for which the tiles win over the fragments
 // (tile_fill; 8192 x 2048).  Fewer than 1024 columns: four 256s are the least that a workgroup's wavefronts share out.
-bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m) {
-    if (!fh_qmm_reg_supports(q) || q->k < 1024) return false;
+static bool reg_few(const fh_qmatrix *q, int x_is_bf16, int m) {
     const int64_t n = q->n, k = q->k;
     switch (q->type) {
     case FH_Q4_K:
@@ -609,46 +1026,59 @@ bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m) {
     case FH_Q5_0:
         if (x_is_bf16) return m <= 512;
         return m <= 192 || (m <= 512 && fh_qmm_frag_pays(q, 0, m));
-    case FH_Q6_K: return m <= (x_is_bf16 ? 768 : 512);
+    case FH_Q6_K: return x_is_bf16 ? m <= 768 && (k <= 8192 || m <= 256 || m > 512) : m <= 512;
     }
     return m <= (x_is_bf16 ? (n <= 8192 ? 1280 : 768) : 512); // Q8_0, Q4_0
 }
 
-// How a product is cut: row tiles of activations a workgroup takes (as even as they come out, four at most: registers), groups of
-// wavefronts and workgroups that share out k.  The least of a model fitted to 17 - 192 rows of four matrices: a round of workgroups
-// costs 5 us and, per 256 of k, 1 us (Q6_K 2) and 0.28 us a row tile and product, more of it the fewer wavefronts share their
-// activations; partial planes a launch and their bytes.  whole: k in one part.
-struct RegCut {
-    int mt, kw, parts;
-};
-static RegCut reg_cut(const fh_qmatrix *q, int x_is_bf16, int m, bool whole) {
-    const int chunks = (int)(q->k / 256), tiles = (m + 15) / 16, tx = (tiles + 3) / 4;
-    const int np = (x_is_bf16 ? 1 : 2) + (q->type == FH_Q6_K ? 1 : 0);
-    RegCut best{(tiles + tx - 1) / tx, 1, 1};
-    const double block = (q->type == FH_Q6_K ? 2.0 : 1.0) + 0.28 * best.mt * np; // us of 256 of k
-    double least = 1e30;
-    for (int kw = 1; kw <= 4; kw *= 2)
-        for (int parts = 1; parts <= (whole ? 1 : 16) && parts * kw <= chunks; parts++) {
-            const int64_t groups = (q->n + 16 * 16 / kw - 1) / (16 * 16 / kw) * tx * parts;
-            const int64_t rounds = (groups + q->dev->compute_units - 1) / q->dev->compute_units;
-            const int run = (chunks + parts * kw - 1) / (parts * kw);
-            double t = (double)rounds * (5.0 + run * block * (kw == 1 ? 1.0 : kw == 2 ? 1.13 : 1.4));
-            if (parts > 1) t += 3.4 + (2.0 * parts + 1.0) * m * (double)q->n * 4.0 / 4e6;
-            if (t < least * 0.98) least = t, best.kw = kw, best.parts = parts;
-        }
-    return best;
+// k_qmm_wide: us, model fitted to 14 matrices, nine row counts from 320 to 2048, four formats and both activation types (within 3 - 5 %
+// of all of them): 256 of k of a tile take so long alone on its compute unit and so long for two that share one.
+static double wide_us(const fh_qmatrix *q, int x_is_bf16, int m) {
+    const int64_t tiles = (q->n + 255) / 256 * ((m + 63) / 64), each = (tiles + q->dev->compute_units - 1) / q->dev->compute_units;
+    double one, two;
+    switch (q->type) {
+    case FH_Q4_K: one = x_is_bf16 ? 2.3 : 3.8, two = x_is_bf16 ? 4.2 : 6.8; break;
+    case FH_Q6_K: one = x_is_bf16 ? 3.75 : 5.55, two = x_is_bf16 ? 6.8 : 9.7; break;
+    case FH_Q5_K: case FH_Q5_0: one = x_is_bf16 ? 3.4 : 4.1, two = x_is_bf16 ? 5.6 : 7.5; break;
+    default: one = x_is_bf16 ? 3.1 : 4.3, two = x_is_bf16 ? 5.0 : 7.5;
+    }
+    return 15.0 + m * (double)q->k / 1e6 * (x_is_bf16 ? 0.9 : 1.5) + (double)(q->k / 256) * ((double)(each & 1) * one + (double)(each >> 1) * two);
 }
+
+// Which of the two, if any.  Both where few rows take k_qmm_reg: the one that is quicker by the models.  Above, k_qmm_wide where its
+// tiles keep the device busy (us, wide / others: Q4_K bf16, 2048 rows, 14336 x 4096 276 / 315, 8192 x 3072 130 / 135, 5632 x 2048 74 / 89;
+// Q8_0 bf16 317 / 363, 148 / 165, 83 / 107; Q6_K bf16 420 / 478, 192 / 213, 105 / 131; Q4_K f32, 1024 rows, 28672 x 4096 437 / 495,
+// 14336 x 4096, five eighths full, 248 / 245), with f32 rows only for matrices of
+// 8192 rows and more (4096 x 4096, 2048 rows: 146 / 143) and not for Q6_K (2048 rows, 8192 x 3072 298 / 278).  Its
+// sums are one chain along k, less exact than those of products that are parted along k: k to 8192 only, and not where the tiles part it
+// (qmm_launch_t).  bf16 rows of the formats whose tiles leave the device idle for narrow matrices stay on k_qmm_reg (Q8_0, 1536 rows, 1024 x 4096 45 / 86, 3072 x 3072 85 / 140).
+enum { REG_NONE, REG_NARROW, REG_WIDE };
+static int reg_way(const fh_qmatrix *q, int x_is_bf16, int m) {
+    if (!fh_qmm_reg_supports(q) || q->k < 1024) return REG_NONE;
+    const int64_t n = q->n, tiles = (n + 255) / 256 * ((m + 63) / 64), cus = q->dev->compute_units;
+    const bool can = q->k <= 8192 && (x_is_bf16 || n >= 8192) && (n + 127) / 128 * ((m + 255) / 256) * 5 >= cus * 4, few = reg_few(q, x_is_bf16, m);
+    const bool narrow = few || (x_is_bf16 && n <= 3072 && (q->type == FH_Q8_0 || q->type == FH_Q4_0 || q->type == FH_Q6_K));
+    const double fill = (double)tiles / (double)((tiles + cus - 1) / cus * cus);
+    if (!few && can && m > 512 && (x_is_bf16 || q->type != FH_Q6_K) && tiles >= 160 && fill >= (x_is_bf16 ? 0.6 : 0.7)) return REG_WIDE;
+    if (!narrow) return REG_NONE;
+    return can && wide_us(q, x_is_bf16, m) < 0.97 * reg_cut(q, x_is_bf16, m, false).us ? REG_WIDE : REG_NARROW;
+}
+bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m) { return reg_way(q, x_is_bf16, m) != REG_NONE; }
 
 static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, int half) {
     fh_device *dev = q->dev;
     const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2;
-    const RegCut cut = reg_cut(q, x_is_bf16, m, half > 0);
+    RegCut cut = reg_cut(q, x_is_bf16, m, half > 0);
+    const int64_t opt = dev->opt_matmul_kernel; // 15: always the wide one, 16: never
+    const bool wide = opt == 15 || (opt != 16 && reg_way(q, x_is_bf16, m) == REG_WIDE);
+    if (wide) cut.parts = 1;
     RegArgs g{};
     g.q = fh_view(q);
     g.m = m, g.n = (int)q->n, g.ldy = half ? half : q->n, g.chunks = k / 256, g.wtiles = (int)((q->n + 15) / 16), g.parts = cut.parts, g.half = half;
     // activations: up to four row tiles past the last one (rows past m are multiplied and never stored)
-    const int64_t ch = xp * 8192 + (reg_sums(q->type) ? 1024 : 0), xbytes = (((int64_t)m + 15) / 16 + 4) * g.chunks * ch;
-    const size_t part_at = ((size_t)xbytes + ((size_t)m + 80) * 4 + 255) & ~(size_t)255;
+    const int rows = wide ? 32 : 16;
+    const int64_t ch = xp * 512 * rows + (reg_sums(q->type) ? 1024 : 0), xbytes = (((int64_t)m + rows - 1) / rows + 4) * g.chunks * ch;
+    const size_t part_at = ((size_t)xbytes + ((size_t)m + 160) * 4 + 255) & ~(size_t)255;
     const size_t bytes = part_at + (cut.parts > 1 ? (size_t)cut.parts * m * q->n * 4 : 0);
     // as products on fragments do it: what cannot be had is no error, and the tile kernels' planes are there too
     (void)fh_dev_scratch_try(dev, &dev->act_buf, &dev->act_cap, fh_qmatmul_tile_planes(q, x_is_bf16, m));
@@ -657,10 +1087,18 @@ static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int 
     uint8_t *xf = (uint8_t *)dev->frag_x;
     float *rs = (float *)(xf + xbytes), *part = (float *)(xf + part_at);
     g.x = xf, g.rs = rs, g.y = y;
-    const unsigned threads = k / 8 >= 1024 ? 1024 : (unsigned)(k / 8 + 63) / 64 * 64;
-#define REG_X(IN_, O_)                                                                                      \
-    if (k > 8192) k_reg_x<IN_, O_, 2><<<dim3((unsigned)m), threads, 0, dev->stream>>>(x, k, xf, rs);        \
-    else k_reg_x<IN_, O_, 1><<<dim3((unsigned)m), threads, 0, dev->stream>>>(x, k, xf, rs);                 \
+    const bool many = m >= 1024 || (m >= 512 && k <= 8192);
+    const unsigned threads = many || k / 8 >= 1024 ? 1024 : (unsigned)(k / 8 + 63) / 64 * 64;
+#define REG_X3(IN_, O_, G_, W_, R_) k_reg_x<IN_, O_, G_, W_, R_><<<dim3((unsigned)((m + R_ - 1) / R_)), threads, 0, dev->stream>>>(x, m, k, xf, rs)
+#define REG_X2(IN_, O_, W_)                          \
+    if (!many && k > 8192) REG_X3(IN_, O_, 2, W_, 1); \
+    else if (!many) REG_X3(IN_, O_, 1, W_, 1);       \
+    else if (k > 8192) REG_X3(IN_, O_, 0, W_, 8);    \
+    else if (k > 4096) REG_X3(IN_, O_, 8, W_, 8);    \
+    else REG_X3(IN_, O_, 4, W_, 8)
+#define REG_X(IN_, O_)                    \
+    if (wide) { REG_X2(IN_, O_, true); } \
+    else { REG_X2(IN_, O_, false); }      \
     break
     switch (reg_order(q->type) + (x_is_bf16 ? 3 : 0)) {
     case 0: REG_X(0, 0);
@@ -671,8 +1109,12 @@ static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int 
     case 5: REG_X(1, 2);
     }
 #undef REG_X
+#undef REG_X2
+#undef REG_X3
     FH_HIP(hipGetLastError());
-#define REG_GO(T_) return x_is_bf16 ? reg_go<T_, 1>(dev, g, part, cut.mt, cut.kw) : reg_go<T_, 2>(dev, g, part, cut.mt, cut.kw)
+#define REG_GO(T_)                                                                                              \
+    if (wide) return x_is_bf16 ? wide_product<T_, 1, 2>(dev, g) : wide_product<T_, 2, 2>(dev, g); \
+    return x_is_bf16 ? reg_go<T_, 1>(dev, g, part, cut.mt, cut.kw) : reg_go<T_, 2>(dev, g, part, cut.mt, cut.kw)
     switch (q->type) {
     case FH_Q4_0: REG_GO(FH_Q4_0);
     case FH_Q5_0: REG_GO(FH_Q5_0);

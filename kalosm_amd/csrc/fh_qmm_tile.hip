@@ -1810,7 +1810,7 @@ fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf
                 (long long)K);
     FH_REQUIRE((m + 127) / 128 <= 65535, "m = %d too large for one launch", m);
     const int64_t mk = dev->opt_matmul_kernel;
-    if (((uintptr_t)x & 15) == 0 && (mk == 0 ? fragments && fh_qmm_reg_pays(q, x_is_bf16, m) : mk == 14 && fh_qmm_reg_supports(q))) {
+    if (((uintptr_t)x & 15) == 0 && (mk == 0 ? fragments && fh_qmm_reg_pays(q, x_is_bf16, m) : mk >= 14 && mk <= 16 && fh_qmm_reg_supports(q))) {
         const fh_status st = fh_launch_qmm_reg(q, x, x_is_bf16, m, y);
         if (st != FH_ERR_UNSUPPORTED) return st;
     }

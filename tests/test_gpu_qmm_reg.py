@@ -2,7 +2,8 @@
 dequantised weights.
 
 Bound: the operands are exact up to 2^-22 of each activation; products are added in f32, sixteen times 2 or 3 in a chain within a 256,
-then k / 256 of those (each with its offsets, which cancel most of it), and rounding errors (2^-24 each, of either sign) grow with the
+then k / 256 of those (each with its offsets, which cancel most of it; the wide products of
+formats with a scale per 32 k / 32 of those), and rounding errors (2^-24 each, of either sign) grow with the
 root of their number: 1e-6 of the root of the sum of the squared products (the result's root mean square where there are many of
 them; one result alone may be next to nothing by cancellation) covers k = 16384.  The largest single difference is held to ten
 times that (ten standard deviations)."""
@@ -37,17 +38,23 @@ def run(dev, q, xt, option):
 
 @pytest.mark.parametrize("act", ["f32", "bf16"])
 @pytest.mark.parametrize("ty", TYPES, ids=lambda t: synth.TYPE_NAMES[t])
-@pytest.mark.parametrize("m,n,k", [
-    (1, 1, 256),       # one row, one output, one 256: most wavefronts have nothing of k
-    (17, 33, 1280),    # five 256s over four groups of wavefronts; a second row tile of one row
-    (48, 272, 2304),   # three row tiles; nine 256s
-    (65, 96, 4096),    # five row tiles in two workgroups of three
-    (130, 520, 1024),  # nine row tiles in three workgroups
-    (33, 40, 16384),   # the longest k, in parts
+@pytest.mark.parametrize("m,n,k,option", [
+    (1, 1, 256, 16),       # one row, one output, one 256: most wavefronts have nothing of k
+    (17, 33, 1280, 16),    # five 256s over four groups of wavefronts; a second row tile of one row
+    (48, 272, 2304, 16),   # three row tiles; nine 256s
+    (65, 96, 4096, 16),    # five row tiles in two workgroups of three
+    (130, 520, 1024, 16),  # nine row tiles in three workgroups
+    (33, 40, 16384, 16),   # the longest k, in parts
+    (1, 1, 256, 15),       # the wide products (option 15): the same
+    (64, 256, 512, 15),    # exactly a tile
+    (65, 257, 768, 15),    # one past it; three 256s
+    (515, 80, 4096, 15),   # activations laid out eight rows a workgroup, half of k held by a thread, ...
+    (513, 48, 8192, 15),   # ... all of it, ...
+    (1027, 33, 8448, 15),  # ... read twice; rows past the last eight
 ])
-def test_product(dev, oracle, ty, act, m, n, k):
+def test_product(dev, oracle, ty, act, m, n, k, option):
     q, xt, x, raw = operands(dev, ty, m, n, k, act)
-    got = run(dev, q, xt, 14).astype(np.float64)
+    got = run(dev, q, xt, option).astype(np.float64)
     x, w = x.astype(np.float64), oracle.dequantize(ty, raw).reshape(n, k).astype(np.float64)
     want, rms = x @ w.T, np.sqrt(np.mean((x * x) @ (w * w).T))
     assert np.isfinite(got).all()
@@ -60,7 +67,9 @@ def test_product(dev, oracle, ty, act, m, n, k):
     (synth.Q4_K, "f32", 17, 64, 1024, True), (synth.Q4_K, "f32", 16, 64, 1024, False),
     (synth.Q4_K, "f32", 511, 8192, 2048, True), (synth.Q4_K, "f32", 512, 8192, 2048, False), (synth.Q4_K, "f32", 640, 64, 2048, True),
     (synth.Q5_0, "f32", 192, 8192, 2048, True), (synth.Q5_0, "f32", 193, 8192, 2048, False),
-    (synth.Q8_0, "bf16", 1280, 64, 1024, True), (synth.Q8_0, "bf16", 769, 8208, 1024, False), (synth.Q6_K, "f32", 513, 64, 1024, False),
+    (synth.Q8_0, "bf16", 1280, 64, 1024, True), (synth.Q6_K, "f32", 513, 64, 1024, False),
+    (synth.Q4_K, "bf16", 1300, 8192, 1024, True), (synth.Q4_K, "bf16", 1300, 1024, 1024, False), (synth.Q4_K, "bf16", 1300, 4096, 8448, False),
+    (synth.Q4_K, "f32", 1000, 8192, 1024, True), (synth.Q4_K, "f32", 1000, 8176, 1024, False),
 ])
 def test_rule(dev, ty, act, m, n, k, taken):
     """Both sides of the dispatch's lines: the bits of this kernel (option 14) or others."""
@@ -68,19 +77,20 @@ def test_rule(dev, ty, act, m, n, k, taken):
     assert np.array_equal(run(dev, q, xt, 0).view(np.uint32), run(dev, q, xt, 14).view(np.uint32)) == taken
 
 
+@pytest.mark.parametrize("option", [15, 16])
 @pytest.mark.parametrize("ty", [synth.Q4_K, synth.Q6_K, synth.Q8_0], ids=lambda t: synth.TYPE_NAMES[t])
-def test_rows_are_independent(dev, ty):
+def test_rows_are_independent(dev, ty, option):
     """Zeros stay zero, a power of two passes through exactly, and an infinity or a NaN stays in its row - also where a group of
     wavefronts has fewer 256s than others (five over four)."""
     m, n, k = 40, 96, 1280
     x = synth.random_activation(m, k, seed=5)
     q, xt, _, _ = operands(dev, ty, m, n, k, "f32", x.copy())
-    base = run(dev, q, xt, 14)
+    base = run(dev, q, xt, option)
     x[3] = 0.0
     x[4] *= np.float32(2.0 ** 20)
     x[5, 7] = np.inf
     x[6, 9] = np.nan
-    got = run(dev, q, Tensor.from_slice(dev, x), 14)
+    got = run(dev, q, Tensor.from_slice(dev, x), option)
     assert not got[3].any()
     assert np.array_equal(got[4], base[4] * np.float32(2.0 ** 20))
     assert not np.isfinite(got[5]).any() and np.isnan(got[6]).all()
@@ -88,15 +98,21 @@ def test_rows_are_independent(dev, ty):
     assert np.array_equal(got[rest], base[rest])
 
 
+@pytest.mark.parametrize("option", [15, 16])
 @pytest.mark.parametrize("m", [65, 100])
 @pytest.mark.parametrize("ffn", [256, 1280])
-def test_swiglu_epilogue(dev, m, ffn):
+def test_swiglu_epilogue(dev, m, ffn, option):
     """gate | up of one launch, SwiGLU at the store, against the two halves as matrices of their own, whose k may be in other
     parts: each product within 1e-6 of the exact one, so two layers of three products within 1e-5 of each other."""
     from kalosm_amd.llama import Model
 
     cfg = dict(n_layers=2, d_model=1024, n_heads=8, n_kv_heads=4, head_dim=128, ffn=ffn, vocab=320, ctx=256, eps=1e-5, theta=1e4)
     tokens = np.random.default_rng(m).integers(0, 320, m)
-    got = [Model.random_init(dev, cfg, seed=2, sigma=2e-3, fuse_gate_up=fuse).forward(tokens) for fuse in (True, False)]
+    models = [Model.random_init(dev, cfg, seed=2, sigma=2e-3, fuse_gate_up=fuse) for fuse in (True, False)]
+    dev.set_option("matmul_kernel", option)
+    try:
+        got = [model.forward(tokens) for model in models]
+    finally:
+        dev.set_option("matmul_kernel", 0)
     assert np.isfinite(got[0]).all()
     assert np.sqrt(np.mean((got[0] - got[1]) ** 2)) <= 1e-5 * np.sqrt(np.mean(got[1] ** 2))

@@ -201,13 +201,98 @@ __global__ __launch_bounds__(256) void k_dense_rows(const void *__restrict__ bin
 }
 
 // ------------------------------------------------------------------------------ weight slab decode
-// Eight dequantised weights of row (tile16*16 + j), lane group g, k-step ks (32 wide).  pos[i] is the position
-// of w[i] inside the step.  Arithmetic as in fh_blocks.h (bit-exact f32 decode).
+// Eight weights of row (tile16*16 + j), lane group g, k-step ks (32 wide) of a block format, as they lie in memory.
+struct Raw8 {
+    uint4 h;      // header of a 256
+    uint2 c, hb;  // codes, high bits
+    uint32_t d;   // scale (Q6_K: and the group's, above it)
+};
+template <int T>
+__device__ __forceinline__ Raw8 load8(const QView &q, int64_t tile16, int j, int g, int ks) {
+    Raw8 r;
+    if (T == FH_Q8_0) {
+        const uint8_t *rec = q.data + (tile16 * q.recs + (ks >> 1)) * 1088;
+        r.c = *(const uint2 *)(rec + (g * 16 + j) * 16 + 8 * (ks & 1));
+        r.d = fh_ld16(rec + 1024 + 4 * j + 2 * (ks & 1));
+    } else if (T == FH_Q4_0 || T == FH_Q5_0) {
+        const uint8_t *rec = q.data + (tile16 * q.recs + (ks >> 2)) * (T == FH_Q5_0 ? 1408 : 1152);
+        r.c.x = *(const uint32_t *)(rec + (g * 16 + j) * 16 + 4 * (ks & 3));
+        if (T == FH_Q5_0) r.hb.x = rec[q50_qh_off(j, ks & 3, g)];
+        r.d = fh_ld16(rec + 1024 + 8 * j + 2 * (ks & 3));
+    } else if (T == FH_Q4_K || T == FH_Q5_K) { // Q5_K: the Q4_K record plus the lane's eight qh bytes
+        const uint8_t *rec = q.data + (tile16 * q.recs + (ks >> 3)) * (T == FH_Q5_K ? 2816 : 2304);
+        r.c = *(const uint2 *)(rec + 256 + ((ks & 7) >> 2) * 1024 + (g * 16 + j) * 16 + 8 * ((ks >> 1) & 1));
+        if (T == FH_Q5_K) r.hb = *(const uint2 *)(rec + 2304 + (g * 16 + j) * 8);
+        r.h = *(const uint4 *)(rec + 16 * j);
+    } else { // FH_Q6_K
+        const uint8_t *rec = q.data + (tile16 * q.recs + (ks >> 3)) * 3360;
+        const int t = ks & 7;
+        r.c.x = *(const uint32_t *)(rec + q6k_lword_off(j, t, g));
+        r.c.y = *(const uint32_t *)(rec + q6k_hword_off(j, t, g));
+        r.d = fh_ld16(rec + q6k_d_off(j)) | (uint32_t)rec[q6k_sc_off(j, 2 * t + (g >> 1))] << 16;
+    }
+    return r;
+}
+// Their values; w[0 .. 3] and w[4 .. 7] stand at p0 and p1 inside the step.  Arithmetic as in fh_blocks.h (bit-exact f32 decode).
+template <int T>
+__device__ __forceinline__ void conv8(const Raw8 &r, int g, int ks, float *w, int &p0, int &p1) {
+    p0 = 8 * g;
+    p1 = 8 * g + 4;
+    if (T == FH_Q8_0) {
+        const float d = fh_h2f((uint16_t)r.d);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            w[i] = (float)(int)(int8_t)(r.c.x >> (8 * i)) * d;
+            w[4 + i] = (float)(int)(int8_t)(r.c.y >> (8 * i)) * d;
+        }
+    } else if (T == FH_Q4_0 || T == FH_Q5_0) { // Q5_0: one byte of fifth bits per lane and block; d * (code - 16)
+        const float d = fh_h2f((uint16_t)r.d);
+        const uint32_t c = r.c.x;
+        p0 = 4 * g;
+        p1 = 16 + 4 * g;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            uint32_t a = (c >> (8 * i)) & 15u, b = (c >> (8 * i + 4)) & 15u;
+            if (T == FH_Q5_0) a |= ((r.hb.x >> i) & 1u) << 4, b |= ((r.hb.x >> (4 + i)) & 1u) << 4;
+            w[i] = (float)((int)a - (T == FH_Q5_0 ? 16 : 8)) * d;
+            w[4 + i] = (float)((int)b - (T == FH_Q5_0 ? 16 : 8)) * d;
+        }
+    } else if (T == FH_Q4_K || T == FH_Q5_K) {
+        const int sb = ks & 7, sh = 4 * (sb & 1);
+        const uint4 h = r.h;
+        const uint2 c = r.c;
+        uint2 hb = make_uint2(0, 0);
+        if (T == FH_Q5_K) hb = r.hb;
+        const float d = fh_h2f((uint16_t)(h.x & 0xFFFF)), dmin = fh_h2f((uint16_t)(h.x >> 16));
+        const uint32_t scw = sb < 4 ? (h.y & 0x3F3F3F3Fu) : ((h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u));
+        const uint32_t mnw = sb < 4 ? (h.z & 0x3F3F3F3Fu) : (((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u));
+        const float scale = (float)((scw >> (8 * (sb & 3))) & 0xFFu) * d;
+        const float off = (float)((mnw >> (8 * (sb & 3))) & 0xFFu) * dmin;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float a = scale * (float)(((c.x >> (8 * i + sh)) & 15u) + (((hb.x >> (8 * i + sb)) & 1u) << 4));
+            const float b = scale * (float)(((c.y >> (8 * i + sh)) & 15u) + (((hb.y >> (8 * i + sb)) & 1u) << 4));
+            w[i] = a - off;
+            w[4 + i] = b - off;
+        }
+    } else { // FH_Q6_K
+        const int t = ks & 7;
+        const float ds = fh_h2f((uint16_t)(r.d & 0xFFFFu)) * (float)(int)(int8_t)(r.d >> 16);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int pp = i >> 1, odd = i & 1;
+            const int nib = (int)((r.c.x >> (4 * (pp + 4 * odd))) & 15u);
+            const int hb = (int)((r.c.y >> (q6k_hbit(t, pp) + 16 * odd)) & 3u);
+            w[i] = ds * (float)(((hb << 4) | nib) - 32);
+        }
+    }
+}
+// Eight dequantised weights, dense rows too.
 template <int T>
 __device__ __forceinline__ void decode8(const QView &q, int64_t tile16, int j, int g, int ks, float *w, int &p0, int &p1) {
-    p0 = 8 * g;     // position of w[0..3]
-    p1 = 8 * g + 4; // position of w[4..7]
     if (T == FH_W_F32 || T == FH_W_F16) { // dense rows [n][k]: row-major, no blocks
+        p0 = 8 * g;
+        p1 = 8 * g + 4;
         int64_t row = tile16 * 16 + j;
         if (row >= q.n) row = q.n - 1; // rows past the end repeat the last one and are never stored
         const int64_t at = row * q.k + (int64_t)ks * 32 + 8 * g;
@@ -222,76 +307,7 @@ __device__ __forceinline__ void decode8(const QView &q, int64_t tile16, int j, i
 #pragma unroll
             for (int i = 0; i < 8; i++) w[i] = (float)h[i];
         }
-    } else if (T == FH_Q8_0) {
-        const uint8_t *rec = q.data + (tile16 * q.recs + (ks >> 1)) * 1088;
-        const int u = ks & 1;
-        const uint2 c = *(const uint2 *)(rec + (g * 16 + j) * 16 + 8 * u);
-        const float d = fh_h2f(fh_ld16(rec + 1024 + 4 * j + 2 * u));
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            w[i] = (float)(int)(int8_t)(c.x >> (8 * i)) * d;
-            w[4 + i] = (float)(int)(int8_t)(c.y >> (8 * i)) * d;
-        }
-    } else if (T == FH_Q4_0) {
-        const uint8_t *rec = q.data + (tile16 * q.recs + (ks >> 2)) * 1152;
-        const int u = ks & 3;
-        const uint32_t c = *(const uint32_t *)(rec + (g * 16 + j) * 16 + 4 * u);
-        const float d = fh_h2f(fh_ld16(rec + 1024 + 8 * j + 2 * u));
-        p0 = 4 * g;
-        p1 = 16 + 4 * g;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            w[i] = (float)((int)((c >> (8 * i)) & 15u) - 8) * d;
-            w[4 + i] = (float)((int)((c >> (8 * i + 4)) & 15u) - 8) * d;
-        }
-    } else if (T == FH_Q5_0) { // the Q4_0 record plus one byte of fifth bits per lane and block; d * (code - 16)
-        const uint8_t *rec = q.data + (tile16 * q.recs + (ks >> 2)) * 1408;
-        const int u = ks & 3;
-        const uint32_t c = *(const uint32_t *)(rec + (g * 16 + j) * 16 + 4 * u);
-        const uint32_t hb = rec[q50_qh_off(j, u, g)];
-        const float d = fh_h2f(fh_ld16(rec + 1024 + 8 * j + 2 * u));
-        p0 = 4 * g;
-        p1 = 16 + 4 * g;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            w[i] = (float)((int)(((c >> (8 * i)) & 15u) | (((hb >> i) & 1u) << 4)) - 16) * d;
-            w[4 + i] = (float)((int)(((c >> (8 * i + 4)) & 15u) | (((hb >> (4 + i)) & 1u) << 4)) - 16) * d;
-        }
-    } else if (T == FH_Q4_K || T == FH_Q5_K) { // Q5_K: the Q4_K record plus the lane's eight qh bytes
-        const uint8_t *rec = q.data + (tile16 * q.recs + (ks >> 3)) * (T == FH_Q5_K ? 2816 : 2304);
-        const int sb = ks & 7, p = sb >> 2, u = (sb >> 1) & 1, hn = sb & 1;
-        const uint2 c = *(const uint2 *)(rec + 256 + p * 1024 + (g * 16 + j) * 16 + 8 * u);
-        uint2 hb = make_uint2(0, 0);
-        if (T == FH_Q5_K) hb = *(const uint2 *)(rec + 2304 + (g * 16 + j) * 8);
-        const uint4 h = *(const uint4 *)(rec + 16 * j);
-        const float d = fh_h2f((uint16_t)(h.x & 0xFFFF)), dmin = fh_h2f((uint16_t)(h.x >> 16));
-        const uint32_t scw = sb < 4 ? (h.y & 0x3F3F3F3Fu) : ((h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u));
-        const uint32_t mnw = sb < 4 ? (h.z & 0x3F3F3F3Fu) : (((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u));
-        const float scale = (float)((scw >> (8 * (sb & 3))) & 0xFFu) * d;
-        const float off = (float)((mnw >> (8 * (sb & 3))) & 0xFFu) * dmin;
-        const int sh = 4 * hn;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float a = scale * (float)(((c.x >> (8 * i + sh)) & 15u) + (((hb.x >> (8 * i + sb)) & 1u) << 4));
-            const float b = scale * (float)(((c.y >> (8 * i + sh)) & 15u) + (((hb.y >> (8 * i + sb)) & 1u) << 4));
-            w[i] = a - off;
-            w[4 + i] = b - off;
-        }
-    } else { // FH_Q6_K
-        const uint8_t *rec = q.data + (tile16 * q.recs + (ks >> 3)) * 3360;
-        const int t = ks & 7;
-        const uint32_t lw = *(const uint32_t *)(rec + q6k_lword_off(j, t, g));
-        const uint32_t hw = *(const uint32_t *)(rec + q6k_hword_off(j, t, g));
-        const int sc = (int)(int8_t)rec[q6k_sc_off(j, 2 * t + (g >> 1))];
-        const float ds = fh_h2f(fh_ld16(rec + q6k_d_off(j))) * (float)sc;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int pp = i >> 1, odd = i & 1;
-            const int nib = (int)((lw >> (4 * (pp + 4 * odd))) & 15u);
-            const int hb = (int)((hw >> (q6k_hbit(t, pp) + 16 * odd)) & 3u);
-            w[i] = ds * (float)(((hb << 4) | nib) - 32);
-        }
-    }
+    } else conv8<T>(load8<T>(q, tile16, j, g, ks), g, ks, w, p0, p1);
 }
 
 // ------------------------------------------------------------------------------ tile kernel
@@ -426,6 +442,123 @@ __global__ __launch_bounds__(64 * WGN * WGM) void k_qmm_tile(QView q, const _Flo
                     if (nn + 3 < q.n) dst[3] = v.w;
                 }
             }
+        }
+    }
+}
+
+// k_qmm_tile's sums for at most 64 rows, bit by bit (the same operands, the same products in the same order along k, one chain an output),
+// from 32 weight rows a workgroup instead of 128: what bounds a short prompt is the chain, three products of 32 x 32 x 16 for every 16 of k,
+// and the tiles of 128 rows decode, wait and multiply in turn around it, in few workgroups (37 rows, 2048 x 5632, Q6_K: 16 of them, 317 us, 54 here;
+// 3072 x 2048 and 14336 x 2048, Q4_K: 85 us, 16 and 32 here).  2 us for 256 of k, of which the chain is 0.64; the activations come in pieces of 32
+// bytes a row, 64 KB a workgroup and 256 of k.
+// Here eight wavefronts decode the next 256 of k into LDS in operand order, their bytes requested a 256 earlier, while one wavefront per
+// 32 rows of activations multiplies this one's, its activations requested eight products of 16 earlier.
+template <int T, int NTERM, int FM>
+__global__ __launch_bounds__(64 * (8 + FM)) void k_qmm_short(QView q, const _Float16 *__restrict__ xh, const _Float16 *__restrict__ xl,
+                                                              const float *__restrict__ rs, int m, float *__restrict__ y) {
+    // [buffer][hi, lo][16 of k][lane][8]
+    __shared__ __attribute__((aligned(16))) _Float16 s_w[2][2][16][64 * 8];
+    constexpr int AHEAD = 8;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int64_t tiles16 = (q.n + 15) / 16;
+    const int K = (int)q.k, chunks = K >> 8;
+    auto meet = [] { // (no wait for requests on their way, as __syncthreads has)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (wave < 8) { // a wavefront decodes step `wave` of the 256, both row tiles
+        const int g = lane >> 4, j = lane & 15;
+        Raw8 raw[2];
+        auto ask = [&](int c) {
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                int64_t tile = (int64_t)blockIdx.x * 2 + t;
+                if (tile >= tiles16) tile = tiles16 - 1; // rows past the end decode a valid tile and are never stored
+                raw[t] = load8<T>(q, tile, j, g, (c < chunks ? c : chunks - 1) * 8 + wave);
+            }
+        };
+        auto put = [&](int buf) {
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                float w[8];
+                int p0, p1;
+                conv8<T>(raw[t], g, wave, w, p0, p1);
+                _Float16 hi[8], lo[8];
+#pragma unroll
+                for (int c = 0; c < 8; c++) hi[c] = (_Float16)w[c], lo[c] = (_Float16)(w[c] - (float)hi[c]);
+                const int row = t * 16 + j;
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const int p = e ? p1 : p0, at = (32 * ((p >> 3) & 1) + row) * 8 + (p & 7);
+                    uint2 u;
+                    __builtin_memcpy(&u, hi + 4 * e, 8);
+                    *(uint2 *)(&s_w[buf][0][2 * wave + (p >> 4)][at]) = u;
+                    __builtin_memcpy(&u, lo + 4 * e, 8);
+                    *(uint2 *)(&s_w[buf][1][2 * wave + (p >> 4)][at]) = u;
+                }
+            }
+        };
+        ask(0);
+        put(0);
+        ask(1);
+        meet();
+        for (int c = 0; c < chunks; c++) {
+            put((c + 1) & 1); // (behind the last one: once more the last, which nobody reads)
+            ask(c + 2);
+            meet();
+        }
+        return;
+    }
+    const int mm = (wave - 8) * 32 + (lane & 31);
+    const int64_t at = (int64_t)(mm < m ? mm : m - 1) * K + 8 * (lane >> 5);
+    half8 bh[AHEAD], bl[AHEAD];
+    auto ask = [&](int slot, int s) {
+        const int64_t o = at + (s * 16 < K ? s * 16 : K - 16);
+        bh[slot] = *(const half8 *)(xh + o);
+        if (NTERM == 2) bl[slot] = *(const half8 *)(xl + o);
+    };
+    floatx16 acc = {0.f};
+#pragma unroll
+    for (int s = 0; s < AHEAD; s++) ask(s, s);
+    meet();
+    for (int c = 0; c < chunks; c++) {
+        const int buf = c & 1;
+        half8 ah[4], al[4]; // three steps ahead
+        auto read = [&](int s) {
+            ah[s & 3] = *(const half8 *)(&s_w[buf][0][s][lane * 8]);
+            al[s & 3] = *(const half8 *)(&s_w[buf][1][s][lane * 8]);
+        };
+#pragma unroll
+        for (int s = 0; s < 3; s++) read(s);
+#pragma unroll
+        for (int s = 0; s < 16; s++) {
+            if (s + 3 < 16) read(s + 3);
+            __builtin_amdgcn_sched_barrier(0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s & 3], bh[s % AHEAD], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[s & 3], bh[s % AHEAD], acc, 0, 0, 0);
+            if (NTERM == 2) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s & 3], bl[s % AHEAD], acc, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            ask(s % AHEAD, c * 16 + s + AHEAD);
+        }
+        meet();
+    }
+    if (mm >= m) return;
+    const bool vec = (q.n & 3) == 0;
+    const float s = rs[mm] * q.winv;
+    const int64_t nb = (int64_t)blockIdx.x * 32 + 4 * (lane >> 5);
+#pragma unroll
+    for (int r4 = 0; r4 < 4; r4++) {
+        const int64_t nn = nb + 8 * r4;
+        const float4 v = make_float4(acc[4 * r4] * s, acc[4 * r4 + 1] * s, acc[4 * r4 + 2] * s, acc[4 * r4 + 3] * s);
+        float *dst = y + (int64_t)mm * q.n + nn;
+        if (vec && nn + 3 < q.n) {
+            *(float4 *)dst = v;
+        } else {
+            if (nn < q.n) dst[0] = v.x;
+            if (nn + 1 < q.n) dst[1] = v.y;
+            if (nn + 2 < q.n) dst[2] = v.z;
+            if (nn + 3 < q.n) dst[3] = v.w;
         }
     }
 }
@@ -1751,9 +1884,10 @@ static fh_status qmm_launch_t(const fh_qmatrix *q, const _Float16 *xh, const _Fl
         if (tn * ((m + 127) / 128) * ks * 5 >= cus * 4) return qmm_launch_tile2<T, NTERM, 2, 2, 1>(q, xh, xl, rs, m, y, ks);
         return qmm_launch_tile2<T, NTERM, 4, 1, 1>(q, xh, xl, rs, m, y, split_for(tn * ((m + 63) / 64)));
     }
-    if (m <= 32) {
-        dim3 grid((unsigned)((q->n + 127) / 128), 1);
-        k_qmm_tile<T, NTERM, 4, 1, 1, 1><<<grid, 256, 0, s>>>(v, xh, xl, rs, m, y);
+    if (m <= 64 && q->k % 256 == 0 && mk != 3 && mk != 5) {
+        const dim3 grid((unsigned)((q->n + 31) / 32));
+        if (m <= 32) k_qmm_short<T, NTERM, 1><<<grid, 576, 0, s>>>(v, xh, xl, rs, m, y);
+        else k_qmm_short<T, NTERM, 2><<<grid, 640, 0, s>>>(v, xh, xl, rs, m, y);
     } else if (m <= 64) {
         dim3 grid((unsigned)((q->n + 127) / 128), 1);
         k_qmm_tile<T, NTERM, 2, 2, 2, 1><<<grid, 256, 0, s>>>(v, xh, xl, rs, m, y);

@@ -30,7 +30,10 @@
 // Inputs may be f32 or f16; operands are rounded to f16, all accumulation and the softmax are f32.
 // SPLIT (f32 Q, K and V): every operand is the exact two-term f16 split hi + lo of the f32 value (2^-22 relative;
 // the values must lie within the f16 range of +-65504) and both products are the three MFMAs
-// hi.hi + lo.hi + hi.lo, so the result keeps f32 accuracy at three times the matrix-core work.
+// hi.hi + lo.hi + hi.lo, so the result keeps f32 accuracy at three times the matrix-core work.  Its tiles fill the LDS: one workgroup a
+// compute unit, for head_dim 128 one wavefront a SIMD, which nothing covers while it waits for an operand - so pairs are requested
+// four ahead (head_dim 64, two wavefronts: two) and the wavefront may have all registers (32 / 8 heads, 2048 tokens, causal: 139 us,
+// 180 with each pair requested in front of its products; 16 / 4 heads of 64, 3000 tokens 94 / 98).
 #include "fh_internal.h"
 
 typedef _Float16 fh_half;
@@ -86,7 +89,7 @@ __device__ __forceinline__ half8 ap_vt8(const fh_half *p, int row_stride) {
 }
 
 template <typename TQ, typename TKV, int D, bool SPLIT = false, int HW = 1, int KS = 1, int QW = 4>
-__global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_eu(QW == 4 ? 2 : 1, 2))) void k_attn_prefill(const TQ *__restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_st,
+__global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_eu(QW == 4 && !(SPLIT && D == 128) ? 2 : 1, SPLIT && D == 128 ? 1 : 2))) void k_attn_prefill(const TQ *__restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_st,
                                                        const TKV *__restrict__ k, const TKV *__restrict__ v,
                                                        int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int hq, int hkv,
                                                        int sq, int skv, float scale, int causal, TQ *__restrict__ out) {
@@ -242,18 +245,30 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
             }
             __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
         } else {
+            // three products an operand pair (hi.hi, lo.hi, hi.lo); pairs are requested four ahead
+            const fh_half *ap = sK + prow * KS_ + 8 * g;
+            constexpr int NI = 2 * KSTEPS, AHEAD = D == 128 ? 4 : 2;
+            half8 kh_[AHEAD], kl_[AHEAD];
+            auto read = [&](int i) {
+                kh_[i % AHEAD] = *(const half8 *)(ap + (i & 1) * 32 * KS_ + 16 * (i >> 1));
+                kl_[i % AHEAD] = *(const half8 *)(ap + (BN + (i & 1) * 32) * KS_ + 16 * (i >> 1));
+            };
 #pragma unroll
-            for (int kt = 0; kt < 2; kt++) {
-                const fh_half *ap = sK + (kt * 32 + prow) * KS_ + 8 * g;
+            for (int i = 0; i < AHEAD; i++) read(i);
 #pragma unroll
-                for (int ks = 0; ks < KSTEPS; ks++) {
-                    const half8 a = *(const half8 *)(ap + 16 * ks);
-                    st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qf[ks], st[kt], 0, 0, 0);
-                    const half8 al = *(const half8 *)(ap + BN * KS_ + 16 * ks);
-                    st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, qf[ks], st[kt], 0, 0, 0);
-                    st[kt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ql[ks], st[kt], 0, 0, 0);
-                }
+            for (int i = 0; i < NI; i++) {
+                st[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh_[i % AHEAD], qf[i >> 1], st[i & 1], 0, 0, 0);
+                st[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl_[i % AHEAD], qf[i >> 1], st[i & 1], 0, 0, 0);
+                st[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh_[i % AHEAD], ql[i >> 1], st[i & 1], 0, 0, 0);
+                if (i + AHEAD < NI) read(i + AHEAD);
             }
+            __builtin_amdgcn_sched_group_barrier(0x100, 2 * AHEAD, 0);
+#pragma unroll
+            for (int i = 0; i < NI - AHEAD; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 3 * AHEAD, 0);
         }
         // ---- tile t+1 goes into the other buffer (last read before the barrier that ended the previous tile) and
         // tile t+2 is requested: the LDS writes and the loads run under the softmax arithmetic
@@ -338,20 +353,30 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
             }
             __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
         } else {
+            const fh_half *vp = sV + vt_off;
+            constexpr int NJ = 4 * DT, AHEAD = D == 128 ? 4 : 2;
+            half8 vh_[AHEAD], vl_[AHEAD];
+            auto read = [&](int j) {
+                vh_[j % AHEAD] = ap_vt8(vp + 32 * (j % DT) + 16 * (j / DT) * VS, VS);
+                vl_[j % AHEAD] = ap_vt8(vp + BN * VS + 32 * (j % DT) + 16 * (j / DT) * VS, VS);
+            };
 #pragma unroll
-            for (int dt = 0; dt < DT; dt++) {
-                const fh_half *vp = sV + vt_off + 32 * dt;
+            for (int j = 0; j < AHEAD; j++) read(j);
 #pragma unroll
-                for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                    for (int s2 = 0; s2 < 2; s2++) {
-                        const half8 a = ap_vt8(vp + (32 * kt + 16 * s2) * VS, VS);
-                        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[kt][s2], acc[dt], 0, 0, 0);
-                        const half8 al = ap_vt8(vp + BN * VS + (32 * kt + 16 * s2) * VS, VS);
-                        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, pb[kt][s2], acc[dt], 0, 0, 0);
-                        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl[kt][s2], acc[dt], 0, 0, 0);
-                    }
+            for (int j = 0; j < NJ; j++) {
+                const int c = j / DT, dt = j % DT;
+                acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh_[j % AHEAD], pb[c >> 1][c & 1], acc[dt], 0, 0, 0);
+                acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl_[j % AHEAD], pb[c >> 1][c & 1], acc[dt], 0, 0, 0);
+                acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh_[j % AHEAD], pl[c >> 1][c & 1], acc[dt], 0, 0, 0);
+                if (j + AHEAD < NJ) read(j + AHEAD);
             }
+            __builtin_amdgcn_sched_group_barrier(0x100, 4 * AHEAD, 0);
+#pragma unroll
+            for (int j = 0; j < NJ - AHEAD; j++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 3 * AHEAD, 0);
         }
         __syncthreads(); // tile t+1 is staged, and nobody reads this tile's buffer any more
     }

@@ -65,6 +65,7 @@ def test_product(dev, oracle, ty, act, m, n, k, option):
 @pytest.mark.parametrize("ty,act,m,n,k,taken", [
     (synth.Q8_0, "bf16", 1, 64, 1024, True), (synth.Q8_0, "bf16", 1, 64, 768, False),
     (synth.Q4_K, "f32", 17, 64, 1024, True), (synth.Q4_K, "f32", 16, 64, 1024, False),
+    (synth.Q5_K, "f32", 5, 64, 1024, True), (synth.Q5_0, "f32", 4, 64, 1024, False), (synth.Q5_0, "f32", 12, 64, 768, False),
     (synth.Q4_K, "f32", 511, 8192, 2048, True), (synth.Q4_K, "f32", 512, 8192, 2048, False), (synth.Q4_K, "f32", 640, 64, 2048, True),
     (synth.Q5_0, "f32", 192, 8192, 2048, True), (synth.Q5_0, "f32", 193, 8192, 2048, False),
     (synth.Q8_0, "bf16", 1280, 64, 1024, True), (synth.Q6_K, "f32", 513, 64, 1024, False),

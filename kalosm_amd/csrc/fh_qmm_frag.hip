@@ -32,7 +32,8 @@ static int frag_ext(int k, int planes) { return (k / 32 * (planes == 2 ? 2 : 3) 
 
 // One workgroup: eight rows, one of gridDim.y runs of k.  IN: 0 f32, 1 bf16.  A wavefront finds the maximum of one row; then a
 // thread converts eight consecutive values of row t % 8, so that a wavefront reads 256 bytes of each row and writes whole
-// 128-byte runs.  sums: [8][run / 32] floats of dynamic LDS when ext > 0.
+// 128-byte runs.  sums: [8][run / 32] floats of dynamic LDS when ext > 0.  Eight requests of a row on their way: 2048 rows of an 8B prompt's
+// widths take 29.9 us a call (34.3 with the loops as they come).
 template <int IN>
 __global__ __launch_bounds__(512) void k_frag_x(const void *__restrict__ xin, int m, int k, int ext, uint8_t *__restrict__ out,
                                                  int64_t plane, float *__restrict__ rs) {
@@ -45,6 +46,7 @@ __global__ __launch_bounds__(512) void k_frag_x(const void *__restrict__ xin, in
         float amax = 0.f;
         if (IN == 1) {
             const uint16_t *p = (const uint16_t *)xin + (int64_t)row * k;
+#pragma unroll 8
             for (int c = lane * 8; c < k; c += 512) {
                 const uint4 u = *(const uint4 *)(p + c);
                 const uint32_t w[4] = {u.x, u.y, u.z, u.w};
@@ -54,6 +56,7 @@ __global__ __launch_bounds__(512) void k_frag_x(const void *__restrict__ xin, in
             }
         } else {
             const float *p = (const float *)xin + (int64_t)row * k;
+#pragma unroll 8
             for (int c = lane * 4; c < k; c += 256) {
                 const float4 a = *(const float4 *)(p + c);
                 amax = fmaxf(amax, fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))));
@@ -77,6 +80,7 @@ __global__ __launch_bounds__(512) void k_frag_x(const void *__restrict__ xin, in
     uint8_t *dst = out + ((int64_t)(row >> 5) * kf) * 1024 + (row & 31) * 16;
     const int parts = (int)gridDim.y, span = ((k + parts - 1) / parts + 511) / 512 * 512, ns = k >> 5;
     const int from = (int)blockIdx.y * span, to = from + span < k ? from + span : k; // (whole 512s, so whole runs of 8 sums)
+#pragma unroll 2
     for (int at = from; at < to; at += 512) {
         const int c = at + (tid >> 3) * 8;
         float v[8];
@@ -596,7 +600,8 @@ bool fh_qmm_frag_supports(const fh_qmatrix *q) {
     return false;
 }
 
-// Where the fragments pay for being written, against the tile kernels that decode inside the product.  Both were timed for 13 - 64
+// Where the fragments pay for being written, against the tile kernels that decode inside the product (the rows and matrices that
+// fh_qmm_reg.hip takes are not asked about: of those up to 64, only k below 1024 or no multiple of 256 is left).  Both were timed for 13 - 64
 // rows of 12 matrices and 129 - 3000 rows of 23, in every format; us, fragments / tiles, at the lines:
 //   Up to 64 rows a tile kernel takes the same time for any matrix whose tiles of 128 rows fit the device at once (32768 rows), the
 //     fragments as long as they are: Q4_K f32, 32 rows, 11008 x 4096 55 / 150, 32768 x 4096 145 / 158, 128256 x 4096 595 / 294;

@@ -7,10 +7,10 @@ bool fh_qmm_frag_pays(const fh_qmatrix *q, int x_is_bf16, int m); // and where i
 // y[m, n] = x[m, k] . deq(q)^T; x f32 or bf16, rows contiguous and 16-byte aligned.  FH_ERR_UNSUPPORTED where the memory for the
 // fragments cannot be had.
 fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y);
-// A decoder's prompts of up to this many tokens stay on the tile kernels.  The fragments are the faster way there (37 tokens and 64
-// sampled ones through four layers of width 2048: 9.4 ms for 11.1) and the closer one (against 64 bits 4e-6 of the logits, the
-// tiles 1e-5), but the cache they leave differs in its last bits: of 1200 sampled continuations of 64 tokens two came to a draw
-// that those bits decide and went another way from there.
+// A decoder's prompts of up to this many tokens keep the sums of the tile kernels (k_qmm_short: 37 tokens and 64 sampled ones through four
+// layers of width 2048 in 9.3 ms, the tiles 11.1).  The fragments are closer (against 64 bits 4e-6 of the logits, the tiles 1e-5),
+// but the cache they leave differs in its last bits: of 1200 sampled continuations of 64 tokens two came to a draw that those bits
+// decide and went another way from there.
 enum { FH_SHORT_PROMPT = 64 };
 // (More than FH_SHORT_PROMPT rows.)  y[m, n / 2] = silu(x . deq(rows 0 ..)^T) * (x . deq(rows n / 2 ..)^T); FH_ERR_UNSUPPORTED where two launches are the faster way.
 fh_status fh_qmm_frag_swiglu(const fh_qmatrix *q, const float *x, int m, float *y);

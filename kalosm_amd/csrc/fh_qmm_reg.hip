@@ -1015,13 +1015,13 @@ static RegCut reg_cut(const fh_qmatrix *q, int x_is_bf16, int m, bool whole) {
 //              59 / 111, 1024 rows 216 / 212 but 190 / 349, 62 / 123, 31 / 56, 64 / 107 for the smaller n.  Q4_0 as Q8_0.
 //   Q5_0 bf16  512 rows 122 / 136, 118 / 166; 768 rows 71 / 59 for 5632 x 2048
 // Left on the tiles though slower: Q4_K and Q5_0, f32, of rows (from 512, above 192) and matrices for which the tiles win over the fragments
-// (tile_fill; 8192 x 2048).  Fewer than 1024 columns: four 256s are the least that a workgroup's wavefronts share out.
+// (tile_fill; 8192 x 2048), but not Q4_K, 512 rows, of less than four times as many rows as columns (8192 x 3072 67 / 93).  Fewer than 1024 columns: four 256s are the least that a workgroup's wavefronts share out.
 static bool reg_few(const fh_qmatrix *q, int x_is_bf16, int m) {
     const int64_t n = q->n, k = q->k;
     switch (q->type) {
     case FH_Q4_K:
         if (x_is_bf16) return m <= 768;
-        return m < 512 || (m <= 640 && (k > n || fh_qmm_frag_pays(q, 0, m)));
+        return m < 512 || (m == 512 && n < 4 * k) || (m <= 640 && (k > n || fh_qmm_frag_pays(q, 0, m)));
     case FH_Q5_K: return m <= (x_is_bf16 ? 448 : 512);
     case FH_Q5_0:
         if (x_is_bf16) return m <= 512;

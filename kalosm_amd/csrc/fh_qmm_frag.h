@@ -17,8 +17,9 @@ fh_status fh_qmm_frag_swiglu(const fh_qmatrix *q, const float *x, int m, float *
 // y[i] = part[i] + part[stride + i] + .., count of them
 fh_status fh_frag_sum(fh_device *dev, const float *part, int parts, int64_t stride, int64_t count, float *y);
 
-// The same for fewer rows, weights decoded in registers (fh_qmm_reg.hip); memory and results as above.
+// The same for fewer rows, weights decoded in registers (fh_qmm_reg.hip); memory and results as above.  planes: the tile kernels, which take
+// the call where the memory cannot be had, find theirs.
 bool fh_qmm_reg_supports(const fh_qmatrix *q);
 bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m);
-fh_status fh_launch_qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y);
+fh_status fh_launch_qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, bool planes);
 fh_status fh_qmm_reg_swiglu(const fh_qmatrix *q, const float *x, int m, float *y);

@@ -1065,7 +1065,7 @@ static int reg_way(const fh_qmatrix *q, int x_is_bf16, int m) {
 }
 bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m) { return reg_way(q, x_is_bf16, m) != REG_NONE; }
 
-static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, int half) {
+static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, int half, bool planes) {
     fh_device *dev = q->dev;
     const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2;
     RegCut cut = reg_cut(q, x_is_bf16, m, half > 0);
@@ -1081,7 +1081,7 @@ static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int 
     const size_t part_at = ((size_t)xbytes + ((size_t)m + 160) * 4 + 255) & ~(size_t)255;
     const size_t bytes = part_at + (cut.parts > 1 ? (size_t)cut.parts * m * q->n * 4 : 0);
     // as products on fragments do it: what cannot be had is no error, and the tile kernels' planes are there too
-    (void)fh_dev_scratch_try(dev, &dev->act_buf, &dev->act_cap, fh_qmatmul_tile_planes(q, x_is_bf16, m));
+    if (planes) (void)fh_dev_scratch_try(dev, &dev->act_buf, &dev->act_cap, fh_qmatmul_tile_planes(q, x_is_bf16, m));
     if (!fh_dev_scratch_try(dev, &dev->frag_x, &dev->frag_x_cap, bytes)) return FH_ERR_UNSUPPORTED;
     dev->frag_used = true;
     uint8_t *xf = (uint8_t *)dev->frag_x;
@@ -1127,5 +1127,7 @@ static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int 
     FH_FAIL(FH_ERR_UNSUPPORTED, "unsupported type %u", q->type);
 }
 
-fh_status fh_launch_qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y) { return qmm_reg(q, x, x_is_bf16, m, y, 0); }
-fh_status fh_qmm_reg_swiglu(const fh_qmatrix *q, const float *x, int m, float *y) { return qmm_reg(q, x, 0, m, y, (int)(q->n / 2)); }
+fh_status fh_launch_qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, bool planes) {
+    return qmm_reg(q, x, x_is_bf16, m, y, 0, planes);
+}
+fh_status fh_qmm_reg_swiglu(const fh_qmatrix *q, const float *x, int m, float *y) { return qmm_reg(q, x, 0, m, y, (int)(q->n / 2), true); }

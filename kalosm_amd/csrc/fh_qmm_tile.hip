@@ -1945,7 +1945,7 @@ fh_status fh_launch_qmatmul_tile(const fh_qmatrix *q, const void *x, int x_is_bf
     FH_REQUIRE((m + 127) / 128 <= 65535, "m = %d too large for one launch", m);
     const int64_t mk = dev->opt_matmul_kernel;
     if (((uintptr_t)x & 15) == 0 && (mk == 0 ? fragments && fh_qmm_reg_pays(q, x_is_bf16, m) : mk >= 14 && mk <= 16 && fh_qmm_reg_supports(q))) {
-        const fh_status st = fh_launch_qmm_reg(q, x, x_is_bf16, m, y);
+        const fh_status st = fh_launch_qmm_reg(q, x, x_is_bf16, m, y, true);
         if (st != FH_ERR_UNSUPPORTED) return st;
     }
     if (((uintptr_t)x & 15) == 0 && (mk == 0 ? fragments && fh_qmm_frag_pays(q, x_is_bf16, m) : mk == 13 && fh_qmm_frag_supports(q))) {

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from kalosm_amd import synth
-from kalosm_amd.fusor import QMatrix, Tensor
+from kalosm_amd.fusor import Device, QMatrix, Tensor
 
 pytestmark = pytest.mark.gpu
 TYPES = [synth.Q4_0, synth.Q5_0, synth.Q8_0, synth.Q4_K, synth.Q5_K, synth.Q6_K]
@@ -117,3 +117,30 @@ def test_swiglu_epilogue(dev, m, ffn, option):
         dev.set_option("matmul_kernel", 0)
     assert np.isfinite(got[0]).all()
     assert np.sqrt(np.mean((got[0] - got[1]) ** 2)) <= 1e-5 * np.sqrt(np.mean(got[1] ** 2))
+
+
+@pytest.mark.parametrize("ty", [synth.Q5_0, synth.Q5_K], ids=lambda t: synth.TYPE_NAMES[t])
+def test_five_bit_rows_without_memory(ty):
+    """5 to 12 rows of the 5-bit formats: where the memory for their activations cannot be had (a bound, a capture ahead of any eager
+    call) they are a launch each, which needs none, and with it they leave the graphs of other calls alone."""
+    dev = Device.gpu(0)
+    try:
+        raw = synth.random_weight(ty, 64, 1024, seed=1, sigma=2e-3)
+        q = QMatrix.from_raw_bytes(dev, (64, 1024), raw, ty)
+        x = synth.random_activation(12, 1024, seed=2)
+        xt, out = Tensor.from_slice(dev, x), Tensor(dev, (12, 64))
+        rows = np.concatenate([Tensor.from_slice(dev, x[r:r + 1]).q_mat_mul(q).as_slice() for r in range(12)])
+        dev.set_option("scratch_limit", 1)
+        assert np.array_equal(run(dev, q, xt, 0).view(np.uint32), rows.view(np.uint32))
+        dev.set_option("scratch_limit", 0)
+        dev.graph_begin()
+        xt.q_mat_mul(q, out=out)
+        graph = dev.graph_end()
+        for _ in range(2):
+            in_one = run(dev, q, xt, 0)
+            graph.launch()
+            assert np.array_equal(out.as_slice().view(np.uint32), rows.view(np.uint32))
+        assert not np.array_equal(in_one, rows)
+        del graph
+    finally:
+        dev.close()

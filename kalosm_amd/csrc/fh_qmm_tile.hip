@@ -247,13 +247,13 @@ __device__ __forceinline__ void conv8(const Raw8 &r, int g, int ks, float *w, in
         }
     } else if (T == FH_Q4_0 || T == FH_Q5_0) { // Q5_0: one byte of fifth bits per lane and block; d * (code - 16)
         const float d = fh_h2f((uint16_t)r.d);
-        const uint32_t c = r.c.x;
+        const uint32_t c = r.c.x, hb = r.hb.x;
         p0 = 4 * g;
         p1 = 16 + 4 * g;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            uint32_t a = (c >> (8 * i)) & 15u, b = (c >> (8 * i + 4)) & 15u;
-            if (T == FH_Q5_0) a |= ((r.hb.x >> i) & 1u) << 4, b |= ((r.hb.x >> (4 + i)) & 1u) << 4;
+            const uint32_t a = ((c >> (8 * i)) & 15u) | (T == FH_Q5_0 ? ((hb >> i) & 1u) << 4 : 0u);
+            const uint32_t b = ((c >> (8 * i + 4)) & 15u) | (T == FH_Q5_0 ? ((hb >> (4 + i)) & 1u) << 4 : 0u);
             w[i] = (float)((int)a - (T == FH_Q5_0 ? 16 : 8)) * d;
             w[4 + i] = (float)((int)b - (T == FH_Q5_0 ? 16 : 8)) * d;
         }

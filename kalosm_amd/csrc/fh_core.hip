@@ -249,6 +249,7 @@ extern "C" fh_status fh_set_option(fh_device *dev, const char *key, int64_t valu
     else if (!strcmp(key, "attn_splits")) dev->opt_attn_splits = value;
     else if (!strcmp(key, "attn_kernel")) dev->opt_attn_kernel = value;
     else if (!strcmp(key, "matmul_kernel")) dev->opt_matmul_kernel = value;
+    else if (!strcmp(key, "matmul_cut")) dev->opt_matmul_cut = value;
     else if (!strcmp(key, "fuse_norm")) dev->opt_fuse_norm = value;
     else if (!strcmp(key, "down_splitk")) dev->opt_down_splitk = value;
     else if (!strcmp(key, "wo_acc")) dev->opt_wo_acc = value;

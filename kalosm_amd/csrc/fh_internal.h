@@ -97,6 +97,7 @@ struct fh_device {
     int64_t opt_trace_stderr = 0;    // 1: trace lines go to stderr as well as into the decoder's trace text
     uint64_t opt_gen = 0;            // bumped by every fh_set_option: captured decode steps are recorded again after a change
     int64_t opt_matmul_kernel = 0;   // 0 auto, 1 generic for every m, 2 MFMA tile kernels for every m, 3 / 4 and never / always the 128 x 256 one
+    int64_t opt_matmul_cut = 0;      // > 0: mt + 16 kw + 256 parts, how the products that decode in registers are cut (tests)
 };
 
 enum { FH_FIXED_BYTES = 9 << 20 };

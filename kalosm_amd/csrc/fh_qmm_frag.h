@@ -14,7 +14,7 @@ fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, 
 enum { FH_SHORT_PROMPT = 64 };
 // (More than FH_SHORT_PROMPT rows.)  y[m, n / 2] = silu(x . deq(rows 0 ..)^T) * (x . deq(rows n / 2 ..)^T); FH_ERR_UNSUPPORTED where two launches are the faster way.
 fh_status fh_qmm_frag_swiglu(const fh_qmatrix *q, const float *x, int m, float *y);
-// y[i] = part[i] + part[stride + i] + .., count of them
+// y[i] = part[i] + part[stride + i] + .., count of them, 16 planes at most, added in pairs
 fh_status fh_frag_sum(fh_device *dev, const float *part, int parts, int64_t stride, int64_t count, float *y);
 
 // The same for fewer rows, weights decoded in registers (fh_qmm_reg.hip); memory and results as above.  planes: the tile kernels, which take

@@ -1072,6 +1072,12 @@ static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int 
     const int64_t opt = dev->opt_matmul_kernel; // 15: always the wide one, 16: never
     const bool wide = opt == 15 || (opt != 16 && reg_way(q, x_is_bf16, m) == REG_WIDE);
     if (wide) cut.parts = 1;
+    else if (dev->opt_matmul_cut > 0) { // tests: row tiles, groups of wavefronts and workgroups along k as asked for
+        const int c = (int)dev->opt_matmul_cut, mt = c & 15, kw = (c >> 4) & 15, parts = c >> 8;
+        FH_REQUIRE(mt >= 1 && mt <= 4 && (kw == 1 || kw == 2 || kw == 4) && parts >= 1 && parts <= (half ? 1 : 16) && parts * kw <= k / 256,
+                   "matmul_cut = %d for k = %d", c, k);
+        cut.mt = mt, cut.kw = kw, cut.parts = parts;
+    }
     RegArgs g{};
     g.q = fh_view(q);
     g.m = m, g.n = (int)q->n, g.ldy = half ? half : q->n, g.chunks = k / 256, g.wtiles = (int)((q->n + 15) / 16), g.parts = cut.parts, g.half = half;

@@ -144,3 +144,26 @@ def test_five_bit_rows_without_memory(ty):
         del graph
     finally:
         dev.close()
+
+
+def long_sum(dev, ty, option, cut, chunks, act="bf16", m=1):
+    """2^24 from the first 256 of k and 1 from each other one: an addition of 1 to a sum of 2^24 leaves it as it is."""
+    k, ones = 256 * chunks, np.zeros((m, 256 * chunks), np.float32)
+    ones[:, ::256] = 1.0
+    ones[:, 0] = 2.0 ** 24
+    raw = np.zeros((16, k // 32, 34), np.uint8)  # Q8_0: scale 1, every 256's first code 1
+    raw[:, :, 0:2] = np.array([1.0], np.float16).view(np.uint8)
+    raw[:, ::8, 2] = 1
+    q = QMatrix.from_raw_bytes(dev, (16, k), raw.reshape(-1), ty)
+    bits = synth.to_bf16_bits(ones)
+    xt = Tensor.from_slice(dev, bits, dtype="bf16") if act == "bf16" else Tensor.from_slice(dev, ones)
+    dev.set_option("matmul_cut", cut)
+    try:
+        return run(dev, q, xt, option).astype(np.float64) - 2.0 ** 24
+    finally:
+        dev.set_option("matmul_cut", 0)
+
+
+def test_partial_planes_are_added_in_pairs(dev):
+    """16 planes of one 256 each: one pair loses its 1, the 14 others arrive.  (One after the other: all 15 are lost.)"""
+    assert (long_sum(dev, synth.Q8_0, 16, 1 + 16 * 1 + 256 * 16, 16) == 14).all()

@@ -407,12 +407,13 @@ __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
         }
     };
     RegW<T> w[TW];
-    floatx4 acc[TW][MT], sum[TW][MT], part256[TW][MT]; // of all, of a scale, of a 256 (formats with a scale per 32)
+    floatx4 acc[TW][MT], sum[TW][MT], part256[TW][MT]; // of up to eight 256s, of a scale, of a 256 (formats with a scale per 32)
+    floatx4 all[TW][MT];                               // of the eights before (formats with a scale per 256)
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < TW; t++)
 #pragma unroll
-        for (int c = 0; c < MT; c++) acc[t][c] = zero;
+        for (int c = 0; c < MT; c++) acc[t][c] = all[t][c] = zero;
     half8 xs[MT];
     int cur = 0;
 #pragma unroll
@@ -428,92 +429,103 @@ __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
     for (int u = 0; u < MT * NX; u++) xv[u] = *(const half8 *)(smem + (kw * PIECES + u) * 1024 + lane * 16);
     uint32_t one;
     asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(one));
-    for (int i = 0; i < most; i++) {
-        const int c0 = chunk(i), c1 = chunk(i + 1);
+    // The sum ends after eight 256s, so that none is long: against 64 bits 384 bf16 rows of 4096 x 14336 in Q4_K 9.9e-8 (sums of 28: 1.22e-7), in Q5_K
+    // 1.08e-7 (1.30e-7), for a hundredth of the time.  (With a scale per 32 there are no registers for it, and the tiles added 32s.)
+    for (int from = 0; from < most;) {
+        const int to = PER32 || from + 8 > most ? most : from + 8;
+        for (int i = from; i < to; i++) {
+            const int c0 = chunk(i), c1 = chunk(i + 1);
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            if (e % SB == 0) {
-                __builtin_amdgcn_sched_barrier(0);
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Tile::younger(e)) : "memory"); // stage s + 1 has landed (and stage s) ...
-                __builtin_amdgcn_s_barrier();                                           // ... everywhere; the buffer of s - 1 is free
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if (e == 0) {
-#pragma unroll
-                for (int t = 0; t < TW; t++) w[t].ask_b(recs[t] + (int64_t)c0 * RegW<T>::REC, lane);
-#pragma unroll
-                for (int t = 0; t < TW; t++) w[t].begin();
-            }
-            if (e == 4)
-#pragma unroll
-                for (int t = 0; t < TW; t++) w[t].ask_a(recs[t] + (int64_t)c1 * RegW<T>::REC, lane);
-            if (SUMS && e == 6)
-#pragma unroll
-                for (int m = 0; m < MT; m++) xs[m] = *(const half8 *)(xt + (m * g.chunks + c0) * CH + CH - 1024 + lane * 16);
-            __builtin_amdgcn_sched_barrier(0);
-            if (e % SB == 0) {
-                constexpr int AHEAD = (ST - 1) * SB; // blocks
-                fetch(chunk(i + (e + AHEAD) / 8), (e + AHEAD) & 7, cur == 0 ? (ST - 1) * STAGE : cur - STAGE);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            // the next block's activations, each behind its last use here
-            const int nb = e % SB == SB - 1 ? (cur + STAGE == ST * STAGE ? 0 : cur + STAGE) : cur;
-            const uint8_t *b = smem + nb + (kw * PIECES + (e + 1) % SB * NX * MT) * 1024 + lane * 16;
-            if (e == 0) w[0].get(0, one, wv[0]);
-#pragma unroll
-            for (int t = 0; t < TW; t++) { // the next tile's (block's) weights are decoded while this one's are multiplied
-                const int now = t & 1;
-                if (e < 7 || t < TW - 1) w[(t + 1) % TW].get(t == TW - 1 ? e + 1 : e, one, wv[now ^ 1]);
-#pragma unroll
-                for (int u = 0; u < MT * NP; u++) { // (plane by plane, so that neighbours are of different sums)
-                    const int m = u % MT, p = u / MT;
-                    sum[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[p < NX ? u : m], wv[now][p < NX ? 0 : NW - 1],
-                                                                       (PER32 || e == 0) && p == 0 ? zero : sum[t][m], 0, 0, 0);
+            for (int e = 0; e < 8; e++) {
+                if (e % SB == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Tile::younger(e)) : "memory"); // stage s + 1 has landed (and stage s) ...
+                    __builtin_amdgcn_s_barrier();                                           // ... everywhere; the buffer of s - 1 is free
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                if (t == TW - 1)
+                if (e == 0) {
 #pragma unroll
-                    for (int u = 0; u < MT * NX; u++) xv[u] = *(const half8 *)(b + u * 1024);
-                if (PER32) {
-                    if (e + t > 0) { // the sums before these
-                        const int pe = t ? e : e - 1, pt = t ? t - 1 : TW - 1;
+                    for (int t = 0; t < TW; t++) w[t].ask_b(recs[t] + (int64_t)c0 * RegW<T>::REC, lane);
 #pragma unroll
-                        for (int m = 0; m < MT; m++)
+                    for (int t = 0; t < TW; t++) w[t].begin();
+                }
+                if (e == 4)
 #pragma unroll
-                            for (int r = 0; r < 4; r++) part256[pt][m][r] = pe ? fmaf(sum[pt][m][r], d32, part256[pt][m][r]) : sum[pt][m][r] * d32;
+                    for (int t = 0; t < TW; t++) w[t].ask_a(recs[t] + (int64_t)c1 * RegW<T>::REC, lane);
+                if (SUMS && e == 6)
+#pragma unroll
+                    for (int m = 0; m < MT; m++) xs[m] = *(const half8 *)(xt + (m * g.chunks + c0) * CH + CH - 1024 + lane * 16);
+                __builtin_amdgcn_sched_barrier(0);
+                if (e % SB == 0) {
+                    constexpr int AHEAD = (ST - 1) * SB; // blocks
+                    fetch(chunk(i + (e + AHEAD) / 8), (e + AHEAD) & 7, cur == 0 ? (ST - 1) * STAGE : cur - STAGE);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // the next block's activations, each behind its last use here
+                const int nb = e % SB == SB - 1 ? (cur + STAGE == ST * STAGE ? 0 : cur + STAGE) : cur;
+                const uint8_t *b = smem + nb + (kw * PIECES + (e + 1) % SB * NX * MT) * 1024 + lane * 16;
+                if (e == 0) w[0].get(0, one, wv[0]);
+#pragma unroll
+                for (int t = 0; t < TW; t++) { // the next tile's (block's) weights are decoded while this one's are multiplied
+                    const int now = t & 1;
+                    if (e < 7 || t < TW - 1) w[(t + 1) % TW].get(t == TW - 1 ? e + 1 : e, one, wv[now ^ 1]);
+#pragma unroll
+                    for (int u = 0; u < MT * NP; u++) { // (plane by plane, so that neighbours are of different sums)
+                        const int m = u % MT, p = u / MT;
+                        sum[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[p < NX ? u : m], wv[now][p < NX ? 0 : NW - 1],
+                                                                           (PER32 || e == 0) && p == 0 ? zero : sum[t][m], 0, 0, 0);
                     }
-                    d32 = i < mine ? w[t].scale(e) : 0.f; // (before the next half's scales are asked for into their place)
-                }
+                    if (t == TW - 1)
 #pragma unroll
-                for (int u = 0; u < MT * NP; u++) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, (16 * NW + (PER32 ? 4 * MT : 0)) / (MT * NP), 0);
-                    if (t == TW - 1 && u >= MT * (NP - NX)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        for (int u = 0; u < MT * NX; u++) xv[u] = *(const half8 *)(b + u * 1024);
+                    if (PER32) {
+                        if (e + t > 0) { // the sums before these
+                            const int pe = t ? e : e - 1, pt = t ? t - 1 : TW - 1;
+#pragma unroll
+                            for (int m = 0; m < MT; m++)
+#pragma unroll
+                                for (int r = 0; r < 4; r++) part256[pt][m][r] = pe ? fmaf(sum[pt][m][r], d32, part256[pt][m][r]) : sum[pt][m][r] * d32;
+                        }
+                        d32 = i < mine ? w[t].scale(e) : 0.f; // (before the next half's scales are asked for into their place)
+                    }
+#pragma unroll
+                    for (int u = 0; u < MT * NP; u++) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, (16 * NW + (PER32 ? 4 * MT : 0)) / (MT * NP), 0);
+                        if (t == TW - 1 && u >= MT * (NP - NX)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    }
                 }
+                if (e % SB == SB - 1) cur = cur + STAGE == ST * STAGE ? 0 : cur + STAGE;
             }
-            if (e % SB == SB - 1) cur = cur + STAGE == ST * STAGE ? 0 : cur + STAGE;
+            // a 256's own sum first (with its offsets, which all but cancel it): the long sum takes one rounding for it
+#pragma unroll
+            for (int t = 0; t < TW; t++) {
+                const float d = PER32 ? d32 : i < mine ? w[t].scale(0) : 0.f;
+                if constexpr (SUMS) {
+                    const float o = i < mine ? w[t].offset() : 0.f;
+                    const half8 ov = w[t].offsets();
+#pragma unroll
+                    for (int m = 0; m < MT; m++) {
+                        const floatx4 so = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs[m], ov, zero, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; r++) acc[t][m][r] += fmaf(sum[t][m][r], d, so[r] * o);
+                    }
+                } else
+#pragma unroll
+                    for (int m = 0; m < MT; m++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+                            acc[t][m][r] = PER32 ? acc[t][m][r] + (t == TW - 1 ? fmaf(sum[t][m][r], d, part256[t][m][r]) : part256[t][m][r])
+                                                 : fmaf(sum[t][m][r], d, acc[t][m][r]);
+            }
         }
-        // a 256's own sum first (with its offsets, which all but cancel it): the long sum takes one rounding for it
+        from = to;
+        if (!PER32)
 #pragma unroll
-        for (int t = 0; t < TW; t++) {
-            const float d = PER32 ? d32 : i < mine ? w[t].scale(0) : 0.f;
-            if constexpr (SUMS) {
-                const float o = i < mine ? w[t].offset() : 0.f;
-                const half8 ov = w[t].offsets();
+            for (int t = 0; t < TW; t++)
 #pragma unroll
-                for (int m = 0; m < MT; m++) {
-                    const floatx4 so = __builtin_amdgcn_mfma_f32_16x16x32_f16(xs[m], ov, zero, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 4; r++) acc[t][m][r] += fmaf(sum[t][m][r], d, so[r] * o);
-                }
-            } else
-#pragma unroll
-                for (int m = 0; m < MT; m++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        acc[t][m][r] = PER32 ? acc[t][m][r] + (t == TW - 1 ? fmaf(sum[t][m][r], d, part256[t][m][r]) : part256[t][m][r])
-                                             : fmaf(sum[t][m][r], d, acc[t][m][r]);
-        }
+                for (int m = 0; m < MT; m++) all[t][m] += acc[t][m], acc[t][m] = to < most ? zero : all[t][m];
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // no LDS-direct load outlives its buffer
     if (KW > 1) { // the groups' sums through LDS, in their order

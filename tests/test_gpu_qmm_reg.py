@@ -146,17 +146,22 @@ def test_five_bit_rows_without_memory(ty):
         dev.close()
 
 
-def long_sum(dev, ty, option, cut, chunks, act="bf16", m=1):
+def long_sum(dev, ty, option, cut, chunks):
     """2^24 from the first 256 of k and 1 from each other one: an addition of 1 to a sum of 2^24 leaves it as it is."""
-    k, ones = 256 * chunks, np.zeros((m, 256 * chunks), np.float32)
-    ones[:, ::256] = 1.0
-    ones[:, 0] = 2.0 ** 24
-    raw = np.zeros((16, k // 32, 34), np.uint8)  # Q8_0: scale 1, every 256's first code 1
-    raw[:, :, 0:2] = np.array([1.0], np.float16).view(np.uint8)
-    raw[:, ::8, 2] = 1
-    q = QMatrix.from_raw_bytes(dev, (16, k), raw.reshape(-1), ty)
-    bits = synth.to_bf16_bits(ones)
-    xt = Tensor.from_slice(dev, bits, dtype="bf16") if act == "bf16" else Tensor.from_slice(dev, ones)
+    x = np.zeros((1, 256 * chunks), np.float32)
+    x[:, ::256] = 1.0
+    x[:, 0] = 2.0 ** 24
+    raw = np.zeros((16, chunks, 210 if ty == synth.Q6_K else 8 * 34), np.uint8)  # a 256's first weight 1, the others 0
+    if ty == synth.Q6_K:
+        raw[..., 128:192] = 0xAA  # code 32 for all: 0
+        raw[..., 0] = 1
+        raw[..., 192:208] = 1
+        raw[..., 208:210] = np.array([1.0], np.float16).view(np.uint8)
+    else:  # Q8_0
+        raw[..., 0:2] = np.array([1.0], np.float16).view(np.uint8)
+        raw[..., 2] = 1
+    q = QMatrix.from_raw_bytes(dev, (16, 256 * chunks), raw.reshape(-1), ty)
+    xt = Tensor.from_slice(dev, synth.to_bf16_bits(x), dtype="bf16")
     dev.set_option("matmul_cut", cut)
     try:
         return run(dev, q, xt, option).astype(np.float64) - 2.0 ** 24
@@ -164,6 +169,14 @@ def long_sum(dev, ty, option, cut, chunks, act="bf16", m=1):
         dev.set_option("matmul_cut", 0)
 
 
-def test_partial_planes_are_added_in_pairs(dev):
+@pytest.mark.parametrize("ty", [synth.Q8_0, synth.Q6_K], ids=lambda t: synth.TYPE_NAMES[t])
+def test_partial_planes_are_added_in_pairs(dev, ty):
     """16 planes of one 256 each: one pair loses its 1, the 14 others arrive.  (One after the other: all 15 are lost.)"""
-    assert (long_sum(dev, synth.Q8_0, 16, 1 + 16 * 1 + 256 * 16, 16) == 14).all()
+    assert (long_sum(dev, ty, 16, 1 + 16 * 1 + 256 * 16, 16) == 14).all()
+
+
+@pytest.mark.parametrize("kw", [1, 4])
+def test_no_sum_is_long(dev, kw):
+    """64 times 256, scale per 256: the ones beside 2^24 in its first eight are lost, the 56 others arrive (of four groups of 16 each too).
+    One sum along k loses all 63, four of them 15."""
+    assert (long_sum(dev, synth.Q6_K, 16, 1 + 16 * kw + 256 * 1, 64) == 56).all()

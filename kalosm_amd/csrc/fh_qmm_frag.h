@@ -4,6 +4,7 @@
 
 bool fh_qmm_frag_supports(const fh_qmatrix *q);
 bool fh_qmm_frag_pays(const fh_qmatrix *q, int x_is_bf16, int m); // and where it is the faster way
+int fh_qmm_frag_parts(const fh_qmatrix *q, int x_is_bf16, int m); // parts of k it would take
 // y[m, n] = x[m, k] . deq(q)^T; x f32 or bf16, rows contiguous and 16-byte aligned.  FH_ERR_UNSUPPORTED where the memory for the
 // fragments cannot be had.
 fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y);

@@ -674,20 +674,36 @@ static fh_status frag_go(fh_device *dev, const FragArgs &g, int sc, int wp, int 
 }
 #undef FRAG_GO
 
-static fh_status qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, int half) {
-    fh_device *dev = q->dev;
-    const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2, wp = q->type == FH_Q6_K ? 2 : 1;
+struct FragPlan {
+    FragArgs g;
+    int ext, parts;          // columns of offsets; parts of k
+    int64_t rows, row_bytes; // weight rows of a launch
+};
+static fh_status frag_plan(const fh_qmatrix *q, int x_is_bf16, int m, int half, FragPlan *p) {
+    const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2, wp = q->type == FH_Q6_K ? 2 : 1, sc = fh_block_elems(q->type);
     const int ext = q->type == FH_Q4_K || q->type == FH_Q5_K ? frag_ext(k, xp) : 0, kf = (k + ext) / 16;
-    const int sc = fh_block_elems(q->type);
     // weights: as many rows at a time as 512 MB of fragments and their scales hold (less where the device's scratch is bounded)
     const int64_t rows_all = (q->n + 255) / 256 * 256, scales = sc == 32 ? k / 32 : k / 256 + (ext ? (ext + 255) / 256 : 0);
-    const int64_t row_bytes = (int64_t)kf * 32 * wp + scales * 4, bound = dev->opt_scratch_limit;
+    const int64_t row_bytes = (int64_t)kf * 32 * wp + scales * 4, bound = q->dev->opt_scratch_limit;
     int64_t rows = (bound > 0 && bound < (512 << 20) ? bound : 512 << 20) / row_bytes / 256 * 256;
     rows = rows < 256 ? 256 : (rows > rows_all ? rows_all : rows);
-    FragArgs g{};
-    g.m = m, g.n = (int)(rows < q->n ? rows : q->n), g.ldy = half ? half : q->n, g.kf = kf, g.half = half;
-    int parts = 1;
-    FH_TRY(frag_go(dev, g, sc, wp, xp, &parts));
+    p->g = FragArgs{};
+    p->g.m = m, p->g.n = (int)(rows < q->n ? rows : q->n), p->g.ldy = half ? half : q->n, p->g.kf = kf, p->g.half = half;
+    p->ext = ext, p->rows = rows, p->row_bytes = row_bytes, p->parts = 1;
+    return frag_go(q->dev, p->g, sc, wp, xp, &p->parts);
+}
+int fh_qmm_frag_parts(const fh_qmatrix *q, int x_is_bf16, int m) {
+    FragPlan p;
+    return frag_plan(q, x_is_bf16, m, 0, &p) == FH_OK ? p.parts : 1;
+}
+
+static fh_status qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, int half) {
+    fh_device *dev = q->dev;
+    FragPlan plan;
+    FH_TRY(frag_plan(q, x_is_bf16, m, half, &plan));
+    FragArgs &g = plan.g;
+    const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2, wp = q->type == FH_Q6_K ? 2 : 1, sc = fh_block_elems(q->type), ext = plan.ext, kf = g.kf, parts = plan.parts;
+    const int64_t rows = plan.rows, row_bytes = plan.row_bytes;
     if (half && (rows < q->n || parts > 1)) return FH_ERR_UNSUPPORTED; // all rows at once, k in one part
     // activations: rows up to a multiple of the largest tile (rows past m are multiplied and never stored)
     const int64_t mp = ((int64_t)m + 255) / 256 * 256, xplane = mp * kf * 32, wplane = rows * kf * 32;

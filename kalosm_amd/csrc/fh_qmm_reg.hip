@@ -732,9 +732,11 @@ struct WideW {
 template <int T, int NX, int MX>
 struct WideTile {
     static constexpr int SB = 2, PIECES = NX * MX * 2 * SB, FR = PIECES / 4, STAGE = PIECES * 1024;
-    static constexpr int FIT = 81920 / STAGE, ST = FIT > 6 ? 6 : FIT, LDS = ST * STAGE;
+    // A scale per 32 and one plane: k in two halves, the first one's sums in LDS and registers meanwhile.
+    static constexpr bool HALVES = NX == 1 && !reg_sums(T) && T != FH_Q6_K;
+    static constexpr int FIT = 81920 / STAGE, ST = FIT > 6 ? 6 : FIT, LDS = ST * STAGE + (HALVES ? MX * 16384 : 0);
     static constexpr int CH = NX * 16384 + (reg_sums(T) ? 1024 : 0);
-    static_assert(ST >= 4 && PIECES % 4 == 0, "four stages at least");
+    static_assert(ST >= 4 && PIECES % 4 == 0 && LDS <= 81920, "four stages at least, two workgroups a compute unit");
     typedef WideW<T> W;
     static constexpr int wreq(int e) {
         return (e % (8 / W::SL) == 0 ? 2 * W::QS : 0) + (e == 8 - 8 / W::SL ? 2 * W::QH : 0) + (e == 6 && reg_sums(T) ? MX : 0);
@@ -806,111 +808,141 @@ __global__ __launch_bounds__(256, 2) void k_qmm_wide(RegArgs g) {
     asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(one));
     float d32 = 0.f;
     if (PER32) sum[0][1] = zero;
-    for (int i = 0; i < most; i++) {
-        const int c0 = chunk(i), c1 = chunk(i + 1);
+    // k in two halves: against 64 bits 2048 rows of 14336 x 4096 in Q8_0 1.45e-7 (one sum 2.04e-7, the tiles, which part k in their last round, 1.97e-7),
+    // for one to two hundredths of the time.  (The first half's sums through y: half as long again, all workgroups write and read them at once.)
+    floatx16 held[MX];
+    float4 *const held_lds = (float4 *)(smem + ST * STAGE) + tid;
+    if (Tile::HALVES)
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            constexpr int PER = 8 / SL; // blocks of a slot
-            if (e % SB == 0) {
-                __builtin_amdgcn_sched_barrier(0);
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Tile::younger(e)) : "memory");
-                __builtin_amdgcn_s_barrier();
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if (e % PER == 0) {
-                const int s = e / PER, c = s + 1 < SL ? c0 : c1;
+        for (int m = 0; m < MX; m++) held[m] = zero;
+    for (int from = 0; from < most;) {
+        const int to = Tile::HALVES && from == 0 && most > 1 ? most >> 1 : most;
+        for (int i = from; i < to; i++) {
+            const int c0 = chunk(i), c1 = chunk(i + 1);
 #pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    if (s == 0) w[p].begin_head(lane);
-                    w[p].begin(s);
+            for (int e = 0; e < 8; e++) {
+                constexpr int PER = 8 / SL; // blocks of a slot
+                if (e % SB == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Tile::younger(e)) : "memory");
+                    __builtin_amdgcn_s_barrier();
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
                 }
+                if (e % PER == 0) {
+                    const int s = e / PER, c = s + 1 < SL ? c0 : c1;
 #pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    if (s == SL - 1) w[p].ask_head(ra[p] + (int64_t)c * W::REC, rb[p] + (int64_t)c * W::REC, lane);
-                    w[p].ask((s + 1) % SL, ra[p] + (int64_t)c * W::REC, rb[p] + (int64_t)c * W::REC, lane);
+                    for (int p = 0; p < 2; p++) {
+                        if (s == 0) w[p].begin_head(lane);
+                        w[p].begin(s);
+                    }
+#pragma unroll
+                    for (int p = 0; p < 2; p++) {
+                        if (s == SL - 1) w[p].ask_head(ra[p] + (int64_t)c * W::REC, rb[p] + (int64_t)c * W::REC, lane);
+                        w[p].ask((s + 1) % SL, ra[p] + (int64_t)c * W::REC, rb[p] + (int64_t)c * W::REC, lane);
+                    }
                 }
-            }
-            if (SUMS && e == 6)
+                if (SUMS && e == 6)
 #pragma unroll
-                for (int m = 0; m < MX; m++) xs[m] = *(const half8 *)(xt + (m * g.chunks + c0) * CH + CH - 1024 + lane * 16);
-            __builtin_amdgcn_sched_barrier(0);
-            if (e % SB == 0) {
-                constexpr int AHEAD = (ST - 1) * SB; // blocks
-                fetch(chunk(i + (e + AHEAD) / 8), (e + AHEAD) & 7, cur == 0 ? (ST - 1) * STAGE : cur - STAGE);
+                    for (int m = 0; m < MX; m++) xs[m] = *(const half8 *)(xt + (m * g.chunks + c0) * CH + CH - 1024 + lane * 16);
                 __builtin_amdgcn_sched_barrier(0);
-            }
-            const int nb = e % SB == SB - 1 ? (cur + STAGE == ST * STAGE ? 0 : cur + STAGE) : cur;
-            const uint8_t *b = smem + nb + (e + 1) % SB * XB * 1024 + lane * 16; // the next block's activations
-            if (PER32 && e % PER == 0) w[0].get(e, 0, one, wv[0][0]), w[0].get(e, 1, one, wv[0][1]);
+                if (e % SB == 0) {
+                    constexpr int AHEAD = (ST - 1) * SB; // blocks
+                    fetch(chunk(i + (e + AHEAD) / 8), (e + AHEAD) & 7, cur == 0 ? (ST - 1) * STAGE : cur - STAGE);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                const int nb = e % SB == SB - 1 ? (cur + STAGE == ST * STAGE ? 0 : cur + STAGE) : cur;
+                const uint8_t *b = smem + nb + (e + 1) % SB * XB * 1024 + lane * 16; // the next block's activations
+                if (PER32 && e % PER == 0) w[0].get(e, 0, one, wv[0][0]), w[0].get(e, 1, one, wv[0][1]);
 #pragma unroll
-            for (int p = 0; p < 2; p++) { // the next pair's (block's) weights are decoded while this one's are multiplied
-                if (!PER32) w[p].get(e, 0, one, wv[p][0]), w[p].get(e, 1, one, wv[p][1]);
-                else if (p == 0 || (e + 1) % PER) w[p ^ 1].get(e + p, 0, one, wv[p ^ 1][0]), w[p ^ 1].get(e + p, 1, one, wv[p ^ 1][1]);
-                if (PER32) {
-                    float d = w[p].scale(e);
-                    asm volatile("" : "+v"(d)); // (an f32 of its own: fused into the multiply-adds the conversion makes them the slow mixed ones)
+                for (int p = 0; p < 2; p++) { // the next pair's (block's) weights are decoded while this one's are multiplied
+                    if (!PER32) w[p].get(e, 0, one, wv[p][0]), w[p].get(e, 1, one, wv[p][1]);
+                    else if (p == 0 || (e + 1) % PER) w[p ^ 1].get(e + p, 0, one, wv[p ^ 1][0]), w[p ^ 1].get(e + p, 1, one, wv[p ^ 1][1]);
+                    if (PER32) {
+                        float d = w[p].scale(e);
+                        asm volatile("" : "+v"(d)); // (an f32 of its own: fused into the multiply-adds the conversion makes them the slow mixed ones)
 #pragma unroll
-                    for (int m = 0; m < MX; m++) { // a finished sum is scaled while the next is multiplied
-                        const int at = (p * MX + m) & 1;
+                        for (int m = 0; m < MX; m++) { // a finished sum is scaled while the next is multiplied
+                            const int at = (p * MX + m) & 1;
 #pragma unroll
-                        for (int v = 0; v < NX * 2; v++)
-                            sum[0][at] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xv[(v >> 1) * 2 * MX + (v & 1) * MX + m], wv[p][v & 1][0], v ? sum[0][at] : zero, 0, 0, 0);
-                        const int pp = m ? p : p ^ 1, pm = m ? m - 1 : MX - 1;
+                            for (int v = 0; v < NX * 2; v++)
+                                sum[0][at] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xv[(v >> 1) * 2 * MX + (v & 1) * MX + m], wv[p][v & 1][0], v ? sum[0][at] : zero, 0, 0, 0);
+                            const int pp = m ? p : p ^ 1, pm = m ? m - 1 : MX - 1;
 #pragma unroll
-                        for (int r = 0; r < 16; r++) acc[pp][pm][r] = fmaf(sum[0][at ^ 1][r], d32, acc[pp][pm][r]);
-                        d32 = d;
-                        if (p)
+                            for (int r = 0; r < 16; r++) acc[pp][pm][r] = fmaf(sum[0][at ^ 1][r], d32, acc[pp][pm][r]);
+                            d32 = d;
+                            if (p)
+#pragma unroll
+                                for (int v = 0; v < NX * 2; v++) {
+                                    const int u = (v >> 1) * 2 * MX + (v & 1) * MX + m;
+                                    xv[u] = *(const half8 *)(b + u * 1024);
+                                }
 #pragma unroll
                             for (int v = 0; v < NX * 2; v++) {
-                                const int u = (v >> 1) * 2 * MX + (v & 1) * MX + m;
-                                xv[u] = *(const half8 *)(b + u * 1024);
+                                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                                __builtin_amdgcn_sched_group_barrier(0x002, (16 + 44 / MX) / (NX * 2), 0);
+                                if (p) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                             }
-#pragma unroll
-                        for (int v = 0; v < NX * 2; v++) {
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x002, (16 + 44 / MX) / (NX * 2), 0);
-                            if (p) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                         }
-                    }
-                } else {
+                    } else {
 #pragma unroll
-                    for (int j = 0; j < MX * NP * 2; j++) {
-                        const int m = j % MX, v = j / MX, h = v & 1, q = v >> 1;
-                        sum[p][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xv[(q < NX ? q : 0) * 2 * MX + h * MX + m], wv[p][h][q < NX ? 0 : NW - 1],
-                                                                           e == 0 && v == 0 ? zero : sum[p][m], 0, 0, 0);
-                    }
-                    if (p)
+                        for (int j = 0; j < MX * NP * 2; j++) {
+                            const int m = j % MX, v = j / MX, h = v & 1, q = v >> 1;
+                            sum[p][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xv[(q < NX ? q : 0) * 2 * MX + h * MX + m], wv[p][h][q < NX ? 0 : NW - 1],
+                                                                               e == 0 && v == 0 ? zero : sum[p][m], 0, 0, 0);
+                        }
+                        if (p)
 #pragma unroll
-                        for (int u = 0; u < XB; u++) xv[u] = *(const half8 *)(b + u * 1024);
+                            for (int u = 0; u < XB; u++) xv[u] = *(const half8 *)(b + u * 1024);
+                    }
                 }
+                if (e % SB == SB - 1) cur = cur + STAGE == ST * STAGE ? 0 : cur + STAGE;
             }
-            if (e % SB == SB - 1) cur = cur + STAGE == ST * STAGE ? 0 : cur + STAGE;
+            if (!PER32)
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    const float d = w[p].scale(0);
+                    if constexpr (SUMS) {
+                        const float o = w[p].offset();
+                        const half8 ov = w[p].offsets();
+#pragma unroll
+                        for (int m = 0; m < MX; m++) {
+                            const floatx16 so = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs[m], ov, zero, 0, 0, 0);
+#pragma unroll
+                            for (int r = 0; r < 16; r++) acc[p][m][r] += fmaf(sum[p][m][r], d, so[r] * o);
+                        }
+                    } else
+#pragma unroll
+                        for (int m = 0; m < MX; m++)
+#pragma unroll
+                            for (int r = 0; r < 16; r++) acc[p][m][r] = fmaf(sum[p][m][r], d, acc[p][m][r]);
+                }
         }
-        if (!PER32)
+        if (Tile::HALVES && to < most)
 #pragma unroll
-            for (int p = 0; p < 2; p++) {
-                const float d = w[p].scale(0);
-                if constexpr (SUMS) {
-                    const float o = w[p].offset();
-                    const half8 ov = w[p].offsets();
+            for (int m = 0; m < MX; m++) {
+                held[m] = acc[1][m], acc[1][m] = zero;
 #pragma unroll
-                    for (int m = 0; m < MX; m++) {
-                        const floatx16 so = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs[m], ov, zero, 0, 0, 0);
-#pragma unroll
-                        for (int r = 0; r < 16; r++) acc[p][m][r] += fmaf(sum[p][m][r], d, so[r] * o);
-                    }
-                } else
-#pragma unroll
-                    for (int m = 0; m < MX; m++)
-#pragma unroll
-                        for (int r = 0; r < 16; r++) acc[p][m][r] = fmaf(sum[p][m][r], d, acc[p][m][r]);
+                for (int r = 0; r < 16; r += 4)
+                    held_lds[(m * 4 + r / 4) * 256] = make_float4(acc[0][m][r], acc[0][m][r + 1], acc[0][m][r + 2], acc[0][m][r + 3]);
+                acc[0][m] = zero;
             }
+        from = to;
     }
     if (PER32)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[1][MX - 1][r] = fmaf(sum[0][1][r], d32, acc[1][MX - 1][r]);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // no LDS-direct load outlives its buffer
+    if (Tile::HALVES && most > 1)
+#pragma unroll
+        for (int m = 0; m < MX; m++) {
+            acc[1][m] += held[m];
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) {
+                const float4 v = held_lds[(m * 4 + r / 4) * 256];
+                acc[0][m][r] += v.x, acc[0][m][r + 1] += v.y, acc[0][m][r + 2] += v.z, acc[0][m][r + 3] += v.w;
+            }
+        }
     float *y = g.y;
 #pragma unroll
     for (int m = 0; m < MX; m++) {
@@ -1061,19 +1093,28 @@ static double wide_us(const fh_qmatrix *q, int x_is_bf16, int m) {
 // tiles keep the device busy (us, wide / others: Q4_K bf16, 2048 rows, 14336 x 4096 276 / 315, 8192 x 3072 130 / 135, 5632 x 2048 74 / 89;
 // Q8_0 bf16 317 / 363, 148 / 165, 83 / 107; Q6_K bf16 420 / 478, 192 / 213, 105 / 131; Q4_K f32, 1024 rows, 28672 x 4096 437 / 495,
 // 14336 x 4096, five eighths full, 248 / 245), with f32 rows only for matrices of
-// 8192 rows and more (4096 x 4096, 2048 rows: 146 / 143) and not for Q6_K (2048 rows, 8192 x 3072 298 / 278).  Its
-// sums are one chain along k, less exact than those of products that are parted along k: k to 8192 only, and not where the tiles part it
-// (qmm_launch_t).  bf16 rows of the formats whose tiles leave the device idle for narrow matrices stay on k_qmm_reg (Q8_0, 1536 rows, 1024 x 4096 45 / 86, 3072 x 3072 85 / 140).
+// 8192 rows and more (4096 x 4096, 2048 rows: 146 / 143) and not for Q6_K (2048 rows, 8192 x 3072 298 / 278).  k to 8192 only, and not where
+// the tiles would part all of it (qmm_launch_t): its sums are long.  f32 rows and a scale per 32: one sum along k, so that k_qmm_reg, whose 256s add up
+// by themselves, takes what the others would part (reg_parted; 750 rows of 14336 x 8192, Q8_0, against 64 bits 1.4e-7, fragments 2.2e-7, wide
+// 3.0e-7; 402, 462 and 407 us).  bf16 rows of the formats whose tiles leave the device idle for narrow matrices stay on k_qmm_reg (Q8_0, 1536 rows, 1024 x 4096 45 / 86, 3072 x 3072 85 / 140).
 enum { REG_NONE, REG_NARROW, REG_WIDE };
+// f32 rows, a scale per 32: whether the fragments, or the tiles in their last round, take k in parts.  (The tiles of Q5_0 multiply f32 values and
+// are the least exact.)
+static bool reg_parted(const fh_qmatrix *q, int m) {
+    if (m > 512 || (q->type == FH_Q5_0 && fh_qmm_frag_pays(q, 0, m))) return fh_qmm_frag_parts(q, 0, m) > 1;
+    const int64_t tiles = (q->n + 127) / 128 * ((m + 255) / 256), cus = q->dev->compute_units, last = tiles > cus ? tiles % cus : 0;
+    return q->type != FH_Q5_0 && last > 0 && last * 2 <= cus;
+}
 static int reg_way(const fh_qmatrix *q, int x_is_bf16, int m) {
     if (!fh_qmm_reg_supports(q) || q->k < 1024) return REG_NONE;
     const int64_t n = q->n, tiles = (n + 255) / 256 * ((m + 63) / 64), cus = q->dev->compute_units;
     const bool can = q->k <= 8192 && (x_is_bf16 || n >= 8192) && (n + 127) / 128 * ((m + 255) / 256) * 5 >= cus * 4, few = reg_few(q, x_is_bf16, m);
     const bool narrow = few || (x_is_bf16 && n <= 3072 && (q->type == FH_Q8_0 || q->type == FH_Q4_0 || q->type == FH_Q6_K));
     const double fill = (double)tiles / (double)((tiles + cus - 1) / cus * cus);
-    if (!few && can && m > 512 && (x_is_bf16 || q->type != FH_Q6_K) && tiles >= 160 && fill >= (x_is_bf16 ? 0.6 : 0.7)) return REG_WIDE;
+    const bool parted = can && !x_is_bf16 && !reg_sums(q->type) && q->type != FH_Q6_K && reg_parted(q, m);
+    if (!few && can && m > 512 && (x_is_bf16 || q->type != FH_Q6_K) && tiles >= 160 && fill >= (x_is_bf16 ? 0.6 : 0.7)) return parted ? REG_NARROW : REG_WIDE;
     if (!narrow) return REG_NONE;
-    return can && wide_us(q, x_is_bf16, m) < 0.97 * reg_cut(q, x_is_bf16, m, false).us ? REG_WIDE : REG_NARROW;
+    return can && !parted && wide_us(q, x_is_bf16, m) < 0.97 * reg_cut(q, x_is_bf16, m, false).us ? REG_WIDE : REG_NARROW;
 }
 bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m) { return reg_way(q, x_is_bf16, m) != REG_NONE; }
 

@@ -180,3 +180,23 @@ def test_no_sum_is_long(dev, kw):
     """64 times 256, scale per 256: the ones beside 2^24 in its first eight are lost, the 56 others arrive (of four groups of 16 each too).
     One sum along k loses all 63, four of them 15."""
     assert (long_sum(dev, synth.Q6_K, 16, 1 + 16 * kw + 256 * 1, 64) == 56).all()
+
+
+@pytest.mark.parametrize("chunks,kept", [(1, 0), (2, 0), (8, 4), (9, 4), (32, 16)])
+def test_wide_products_in_two_halves(dev, chunks, kept):
+    """Scale per 32, bf16: the ones beside 2^24 in the first half of k are lost, those of the second arrive, up to the last one
+    of an odd number.  (One sum along k: none does.)"""
+    assert (long_sum(dev, synth.Q8_0, 15, 0, chunks) == kept).all()
+
+
+@pytest.mark.parametrize("m,n,k,parted", [
+    (1040, 8192, 8192, True), (600, 24576, 2048, False),  # the fragments in two parts, in one
+    (200, 49152, 2048, True), (200, 32768, 2048, False),  # 384 tiles, the last 128 of them in two parts; 256 tiles
+])
+def test_f32_products_that_others_part(dev, m, n, k, parted):
+    """f32, scale per 32: what the fragments, or the tiles in their last round, would part takes k_qmm_reg (option 16), other products
+    k_qmm_wide (15)."""
+    q, xt, _, _ = operands(dev, synth.Q4_0, m, n, k, "f32")
+    got = {option: run(dev, q, xt, option).view(np.uint32) for option in (0, 15, 16)}
+    assert not np.array_equal(got[15], got[16])
+    assert np.array_equal(got[0], got[16 if parted else 15])

@@ -408,9 +408,10 @@ static fh_status qmatmul(const fh_qmatrix *q, const float *x_dev, int32_t m, flo
     // the matrix-core tiles as well once there are rows to fill them
     const bool dense = (q->type == FH_W_F16 || q->type == FH_W_F32) && q->k % 32 == 0;
     // The 5-bit formats have no batch kernel for 2 .. 16 rows: rows are a launch each up to four, the kernel of small prompts takes them
-    // from there (us, Q5_0, launches / that: 14336 x 4096 four rows 34 / 21, 12 rows 100 / 21; 4096 x 4096 15.6 / 16.0 and 45 / 15; 512 x 2048
-    // 14 / 13 and 34 / 13).  Where it does not (few columns, short prompts of a decoder, no memory for its activations) they stay a launch
-    // each up to 12, which needs none; the tiles take them above.
+    // from there, with a power of two per 32 activations as they have it (us, launches / that: 12 rows of 14336 x 4096 in Q5_0 97 / 23, in Q5_K
+    // 100 / 25, of 4096 x 4096 46 / 14 and 46 / 15, of 512 x 2048 40 / 14 and 40 / 16; four rows of the latter two take 16 and 14 as launches).
+    // Where it does not (few columns, short prompts of a decoder, no memory for its activations) they stay a launch each up to 12, which
+    // needs none; the tiles take them above.
     const bool five = (q->type == FH_Q5_K || q->type == FH_Q5_0) && q->k % 256 == 0;
     if (five && m > 4 && m <= 12 && mk == 0 && q->dev->opt_matvec_kernel == 0 && fragments && ((uintptr_t)x_dev & 15) == 0 && fh_qmm_reg_pays(q, 0, m)) {
         const fh_status st = fh_launch_qmm_reg(q, x_dev, 0, m, y_dev, false);

@@ -48,15 +48,16 @@ __device__ __forceinline__ void reg_x_read(const void *xin, int64_t row, int k, 
 }
 
 // One workgroup: ROWS rows (1, or 8 for whole 128-byte pieces of the operands), G groups of eight a thread in registers between the
-// maximum and the conversion; G = 0: read twice.  WIDE: operands of 32 rows and 16 of k instead (k_qmm_wide).
-template <int IN, int ORDER, int G, bool WIDE, int ROWS>
+// maximum and the conversion; G = 0: read twice.  WIDE: operands of 32 rows and 16 of k instead (k_qmm_wide).  OWN: a power of two per 32
+// values instead of one per row, [8][16 rows] floats of a 256 in the place of its sums (k_qmm_reg, OWN; ROWS 1, G > 0).
+template <int IN, int ORDER, int G, bool WIDE, int ROWS, bool OWN = false>
 __global__ __launch_bounds__(1024) void k_reg_x(const void *__restrict__ xin, int m, int k, uint8_t *__restrict__ out, float *__restrict__ rs) {
-    constexpr bool SUMS = ORDER == 1;
-    constexpr int CH = (IN == 1 ? 8 : 16) * (WIDE ? 2048 : 1024) + (SUMS ? 1024 : 0);
+    constexpr bool SUMS = ORDER == 1 && !OWN;
+    constexpr int CH = (IN == 1 ? 8 : 16) * (WIDE ? 2048 : 1024) + (SUMS || OWN ? 1024 : 0);
     __shared__ float s_max[16][ROWS], sums[SUMS ? 512 * ROWS : 1]; // k <= 16384
     const int tid = threadIdx.x, r = tid % ROWS, row = (int)blockIdx.x * ROWS + r, groups = k >> 3, step = (int)blockDim.x / ROWS;
     const int from = row < m ? row : m - 1;
-    float v[G ? G : 1][8], amax = 0.f;
+    float v[G ? G : 1][8], amax = 0.f, own[OWN ? G : 1] = {0.f};
     auto most = [&](const float (&w)[8]) {
 #pragma unroll
         for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(w[j]));
@@ -68,7 +69,14 @@ __global__ __launch_bounds__(1024) void k_reg_x(const void *__restrict__ xin, in
             reg_x_read<IN, ORDER>(xin, from, k, gi < groups ? gi : groups - 1, v[i]);
         }
 #pragma unroll
-        for (int i = 0; i < G; i++) most(v[i]);
+        for (int i = 0; i < G; i++) {
+            most(v[i]);
+            if (OWN) { // of four threads
+                amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
+                own[i] = fmaxf(amax, __shfl_xor(amax, 2, 64));
+                amax = 0.f;
+            }
+        }
     } else {
 #pragma unroll 4
         for (int gi = tid / ROWS; gi < groups; gi += step) {
@@ -77,16 +85,24 @@ __global__ __launch_bounds__(1024) void k_reg_x(const void *__restrict__ xin, in
             most(w);
         }
     }
+    bool inf; // finite values vanish next to an infinity, which is carried as +-32768
+    float sc;
+    auto normal = [&](float a) { // the power of two, and what it takes back
+        int e = 141 - (int)((__float_as_uint(a) >> 23) & 0xFFu); // 14 - floor(log2 a); zero / inf / nan clamp
+        e = e > 100 ? 100 : (e < -100 ? -100 : e);
+        inf = a == INFINITY;
+        sc = __uint_as_float((uint32_t)(e + 127) << 23);
+        return inf ? INFINITY : __uint_as_float((uint32_t)(127 - e) << 23);
+    };
+    if (!OWN) {
 #pragma unroll
-    for (int o = 32; o >= ROWS; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
-    if ((tid & 63) < ROWS) s_max[tid >> 6][r] = amax;
-    __syncthreads();
-    for (int i = 0; i < (int)blockDim.x >> 6; i++) amax = fmaxf(amax, s_max[i][r]);
-    int e = 141 - (int)((__float_as_uint(amax) >> 23) & 0xFFu); // 14 - floor(log2 amax); zero / inf / nan clamp
-    e = e > 100 ? 100 : (e < -100 ? -100 : e);
-    const bool infrow = amax == INFINITY; // finite values vanish next to an infinity, which is carried as +-32768
-    const float sc = __uint_as_float((uint32_t)(e + 127) << 23);
-    if (tid < ROWS && row < m) rs[row] = infrow ? INFINITY : __uint_as_float((uint32_t)(127 - e) << 23);
+        for (int o = 32; o >= ROWS; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+        if ((tid & 63) < ROWS) s_max[tid >> 6][r] = amax;
+        __syncthreads();
+        for (int i = 0; i < (int)blockDim.x >> 6; i++) amax = fmaxf(amax, s_max[i][r]);
+    }
+    const float back = normal(amax);
+    if (tid < ROWS && row < m) rs[row] = OWN ? 1.f : back;
     uint8_t *dst = WIDE ? out + (int64_t)(row >> 5) * (k >> 8) * CH + (row & 31) * 16 : out + (int64_t)(row >> 4) * (k >> 8) * CH + (row & 15) * 16;
     auto put = [&](int gi, const float (&x)[8]) {
         _Float16 h[8], l[8];
@@ -94,7 +110,7 @@ __global__ __launch_bounds__(1024) void k_reg_x(const void *__restrict__ xin, in
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             float w = x[j] * sc;
-            if (infrow && fabsf(w) == INFINITY) w = copysignf(32768.f, w);
+            if (inf && fabsf(w) == INFINITY) w = copysignf(32768.f, w);
             h[j] = (_Float16)w;
             const float d = w - (float)h[j];
             l[j] = (_Float16)(d == d ? d : 0.f); // a NaN stays in the hi plane alone
@@ -119,7 +135,14 @@ __global__ __launch_bounds__(1024) void k_reg_x(const void *__restrict__ xin, in
     };
     if (G) {
 #pragma unroll
-        for (int i = 0; i < G; i++) put(tid / ROWS + i * step, v[i]);
+        for (int i = 0; i < G; i++) {
+            const int gi = tid / ROWS + i * step;
+            if (OWN) {
+                const float b = normal(own[i]);
+                if ((gi & 3) == 0 && gi < groups) *(float *)(out + ((int64_t)(row >> 4) * (k >> 8) + (gi >> 5)) * CH + CH - 1024 + ((gi >> 2) & 7) * 64 + (row & 15) * 4) = b;
+            }
+            put(gi, v[i]);
+        }
     } else
         for (int at = 0; at < groups; at += step) { // (all threads together: the sums go through their neighbours)
             const int gi = at + tid / ROWS;
@@ -213,6 +236,10 @@ struct RegK { // Q4_K, Q5_K
     __device__ __forceinline__ float offset() const { return -64.f * fh_h2f((uint16_t)(dm >> 16)); }
     __device__ __forceinline__ half8 offsets() const {
         const half2v k = reg_splat(1024.f), r[4] = {reg_bytes<0, 1>(mn[0]) - k, reg_bytes<2, 3>(mn[0]) - k, reg_bytes<0, 1>(mn[1]) - k, reg_bytes<2, 3>(mn[1]) - k};
+        return reg_cat(r);
+    }
+    __device__ __forceinline__ half8 block_offset(int sb) const { // m of block sb, for all of its k
+        const half2v h = reg_h2(__builtin_amdgcn_perm(0x64646464u, mn[sb >> 2], 0x04000400u + (uint32_t)(sb & 3) * 0x00010001u)) - reg_splat(1024.f), r[4] = {h, h, h, h};
         return reg_cat(r);
     }
 };
@@ -343,16 +370,19 @@ struct RegArgs {
 // wavefronts multiply four 256s, with 8 x 1 it is four whose wavefronts multiply 16.
 // A stage is SB blocks of 32 of k: one barrier, in front of it the wait for the stage after.  TW is 2: with 4, half the LDS reads a
 // product, 17 rows took 15 - 25 % longer and 512 rows the same.
-template <int T, int NX, int TW, int MT, int WW, int KW>
+// OWN: activations with a power of two per 32 (one row tile of f32), so every block's sum is scaled by itself, in Q5_K with the block's offset,
+// two more products with its m (12 rows of 14336 x 4096, one power of two per row / per 32: Q5_0 20.5 / 22.7 us, Q5_K 20.4 / 25.4).
+template <int T, int NX, int TW, int MT, int WW, int KW, bool OWN>
 struct RegTile {
     static constexpr int SB = KW == 1 ? 4 : KW == 2 ? 2 : 1; // blocks of 32 in a stage
     static constexpr int PIECES = NX * MT * SB, FR = (PIECES + WW - 1) / WW, STAGE = PIECES * KW * 1024;
     static constexpr int FIT = 163840 / STAGE, ST = FIT > 8 ? 8 : FIT;
     static constexpr int RED = (KW - 1) * WW * TW * MT * 1024, LDS = ST * STAGE > RED ? ST * STAGE : RED;
-    static constexpr int CH = NX * 8192 + (reg_sums(T) ? 1024 : 0);
+    static constexpr int CH = NX * 8192 + (reg_sums(T) || OWN ? 1024 : 0);
     static_assert(ST >= 4, "four stages at least");
-    // requests for weights (and sums) at block e of a 256
-    static constexpr int wreq(int e) { return e == 0 ? TW * RegW<T>::QB : e == 4 ? TW * RegW<T>::QA : e == 6 && reg_sums(T) ? MT : 0; }
+    static_assert(!OWN || (MT == 1 && NX == 2), "one row tile of f32");
+    // requests for weights (and sums, or powers of two) at block e of a 256
+    static constexpr int wreq(int e) { return e == 0 ? TW * RegW<T>::QB : e == 4 ? TW * RegW<T>::QA + (OWN ? 8 : 0) : e == 6 && reg_sums(T) && !OWN ? MT : 0; }
     // requests younger than those of stage s + 1 at the start of stage s, which begins at block e of a 256.  (In its own stage the
     // pieces of a stage come behind the first block's requests; those of its other blocks are not counted.)
     static constexpr int younger(int e) {
@@ -362,11 +392,11 @@ struct RegTile {
     }
 };
 
-template <int T, int NX, int TW, int MT, int WW, int KW>
+template <int T, int NX, int TW, int MT, int WW, int KW, bool OWN>
 __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
-    typedef RegTile<T, NX, TW, MT, WW, KW> Tile;
+    typedef RegTile<T, NX, TW, MT, WW, KW, OWN> Tile;
     constexpr int FR = Tile::FR, PIECES = Tile::PIECES, STAGE = Tile::STAGE, ST = Tile::ST, CH = Tile::CH, SB = Tile::SB;
-    constexpr bool SUMS = reg_sums(T), PER32 = !SUMS && T != FH_Q6_K;
+    constexpr bool SUMS = reg_sums(T) && !OWN, PER32 = OWN || (!SUMS && T != FH_Q6_K), MINS = OWN && reg_sums(T);
     constexpr int NW = RegW<T>::NW, NP = NW == 2 ? NX + 1 : NX; // products of a weight operand and 16 rows
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -418,6 +448,13 @@ __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
     int cur = 0;
 #pragma unroll
     for (int t = 0; t < TW; t++) w[t].ask_a(recs[t] + (int64_t)chunk(0) * RegW<T>::REC, lane);
+    floatx4 pw[OWN ? 8 : 1], next_pw[OWN ? 8 : 1]; // powers of two of a 256's blocks, of the next
+    floatx4 off[TW], off256[TW], own = zero;       // sums with m, of a block and of a 256; the powers of two that go with the sums before
+    auto ask_pw = [&](int c) {
+#pragma unroll
+        for (int b = 0; b < 8; b++) next_pw[b] = *(const floatx4 *)(xt + (int64_t)c * CH + CH - 1024 + b * 64 + (lane >> 4) * 16);
+    };
+    if constexpr (OWN) ask_pw(chunk(0));
 #pragma unroll
     for (int i = 0; i < ST - 1; i++) fetch(chunk(i * SB >> 3), i * SB & 7, i * STAGE);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (the counts of the first steps are those of later ones, with more requests)
@@ -449,10 +486,15 @@ __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
                     for (int t = 0; t < TW; t++) w[t].ask_b(recs[t] + (int64_t)c0 * RegW<T>::REC, lane);
 #pragma unroll
                     for (int t = 0; t < TW; t++) w[t].begin();
+                    if constexpr (OWN)
+#pragma unroll
+                        for (int b = 0; b < 8; b++) pw[b] = next_pw[b];
                 }
-                if (e == 4)
+                if (e == 4) {
 #pragma unroll
                     for (int t = 0; t < TW; t++) w[t].ask_a(recs[t] + (int64_t)c1 * RegW<T>::REC, lane);
+                    if constexpr (OWN) ask_pw(c1);
+                }
                 if (SUMS && e == 6)
 #pragma unroll
                     for (int m = 0; m < MT; m++) xs[m] = *(const half8 *)(xt + (m * g.chunks + c0) * CH + CH - 1024 + lane * 16);
@@ -476,6 +518,12 @@ __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
                         sum[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[p < NX ? u : m], wv[now][p < NX ? 0 : NW - 1],
                                                                            (PER32 || e == 0) && p == 0 ? zero : sum[t][m], 0, 0, 0);
                     }
+                    floatx4 off_now;
+                    if constexpr (MINS) {
+                        const half8 ov = w[t].block_offset(e);
+                        off_now = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[0], ov, zero, 0, 0, 0);
+                        off_now = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[1], ov, off_now, 0, 0, 0);
+                    }
                     if (t == TW - 1)
 #pragma unroll
                         for (int u = 0; u < MT * NX; u++) xv[u] = *(const half8 *)(b + u * 1024);
@@ -485,15 +533,21 @@ __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
 #pragma unroll
                             for (int m = 0; m < MT; m++)
 #pragma unroll
-                                for (int r = 0; r < 4; r++) part256[pt][m][r] = pe ? fmaf(sum[pt][m][r], d32, part256[pt][m][r]) : sum[pt][m][r] * d32;
+                                for (int r = 0; r < 4; r++) {
+                                    const float d = OWN ? own[r] : d32;
+                                    part256[pt][m][r] = pe ? fmaf(sum[pt][m][r], d, part256[pt][m][r]) : sum[pt][m][r] * d;
+                                    if constexpr (MINS) off256[pt][r] = pe ? fmaf(off[pt][r], d, off256[pt][r]) : off[pt][r] * d;
+                                }
                         }
                         d32 = i < mine ? w[t].scale(e) : 0.f; // (before the next half's scales are asked for into their place)
+                        if constexpr (MINS) off[t] = off_now, own = pw[e]; // (the scale is the 256's)
+                        else if constexpr (OWN) own = pw[e] * d32;
                     }
 #pragma unroll
-                    for (int u = 0; u < MT * NP; u++) {
+                    for (int u = 0; u < MT * NP + (MINS ? 2 : 0); u++) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x002, (16 * NW + (PER32 ? 4 * MT : 0)) / (MT * NP), 0);
-                        if (t == TW - 1 && u >= MT * (NP - NX)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, (16 * NW + (MINS ? 28 : OWN ? 8 : PER32 ? 4 * MT : 0)) / (MT * NP + (MINS ? 2 : 0)), 0);
+                        if (t == TW - 1 && u >= MT * (NP - NX) + (MINS ? 2 : 0)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                     }
                 }
                 if (e % SB == SB - 1) cur = cur + STAGE == ST * STAGE ? 0 : cur + STAGE;
@@ -511,6 +565,17 @@ __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
 #pragma unroll
                         for (int r = 0; r < 4; r++) acc[t][m][r] += fmaf(sum[t][m][r], d, so[r] * o);
                     }
+                } else if constexpr (MINS) {
+                    const float d256 = i < mine ? w[t].scale(0) : 0.f, o256 = i < mine ? w[t].offset() * 0.015625f : 0.f;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float s = t == TW - 1 ? fmaf(sum[t][0][r], own[r], part256[t][0][r]) : part256[t][0][r];
+                        const float o = t == TW - 1 ? fmaf(off[t][r], own[r], off256[t][r]) : off256[t][r];
+                        acc[t][0][r] += fmaf(s, d256, o * o256);
+                    }
+                } else if constexpr (OWN) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[t][0][r] += t == TW - 1 ? fmaf(sum[t][0][r], own[r], part256[t][0][r]) : part256[t][0][r];
                 } else
 #pragma unroll
                     for (int m = 0; m < MT; m++)
@@ -808,7 +873,7 @@ __global__ __launch_bounds__(256, 2) void k_qmm_wide(RegArgs g) {
     asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(one));
     float d32 = 0.f;
     if (PER32) sum[0][1] = zero;
-    // k in two halves: against 64 bits 2048 rows of 14336 x 4096 in Q8_0 1.45e-7 (one sum 2.04e-7, the tiles, which part k in their last round, 1.97e-7),
+    // k in two halves: against 64 bits 2048 rows of 14336 x 4096 in Q8_0 1.47e-7 (one sum 2.04e-7, the tiles, which part k in their last round, 1.97e-7),
     // for one to two hundredths of the time.  (The first half's sums through y: half as long again, all workgroups write and read them at once.)
     floatx16 held[MX];
     float4 *const held_lds = (float4 *)(smem + ST * STAGE) + tid;
@@ -968,9 +1033,9 @@ __global__ __launch_bounds__(256, 2) void k_qmm_wide(RegArgs g) {
 }
 
 // ------------------------------------------------------------------------------ launches
-template <int T, int NX, int TW, int MT, int WW, int KW>
+template <int T, int NX, int TW, int MT, int WW, int KW, bool OWN = false>
 static fh_status reg_product(fh_device *dev, RegArgs g, float *part) {
-    typedef RegTile<T, NX, TW, MT, WW, KW> Tile;
+    typedef RegTile<T, NX, TW, MT, WW, KW, OWN> Tile;
     g.tiles_w = (g.wtiles + TW * WW - 1) / (TW * WW);
     g.tiles_x = (g.m + MT * 16 - 1) / (MT * 16);
     float *y = g.y;
@@ -978,15 +1043,18 @@ static fh_status reg_product(fh_device *dev, RegArgs g, float *part) {
         g.y = part;
         g.part_stride = (int64_t)g.m * g.n;
     }
-    FH_TRY(fh_kernel_lds(dev, (const void *)k_qmm_reg<T, NX, TW, MT, WW, KW>, (size_t)Tile::LDS));
-    k_qmm_reg<T, NX, TW, MT, WW, KW><<<dim3((unsigned)(g.tiles_w * g.tiles_x * g.parts)), 512, Tile::LDS, dev->stream>>>(g);
+    FH_TRY(fh_kernel_lds(dev, (const void *)k_qmm_reg<T, NX, TW, MT, WW, KW, OWN>, (size_t)Tile::LDS));
+    k_qmm_reg<T, NX, TW, MT, WW, KW, OWN><<<dim3((unsigned)(g.tiles_w * g.tiles_x * g.parts)), 512, Tile::LDS, dev->stream>>>(g);
     FH_HIP(hipGetLastError());
     if (g.parts > 1) return fh_frag_sum(dev, part, g.parts, g.part_stride, g.part_stride, y);
     return FH_OK;
 }
 
 template <int T, int NX>
-static fh_status reg_go(fh_device *dev, const RegArgs &g, float *part, int mt, int kw) {
+static fh_status reg_go(fh_device *dev, const RegArgs &g, float *part, int mt, int kw, bool own) {
+    if constexpr ((T == FH_Q5_0 || T == FH_Q5_K) && NX == 2)
+        if (own) return kw == 1 ? reg_product<T, NX, 2, 1, 8, 1, true>(dev, g, part) : kw == 2 ? reg_product<T, NX, 2, 1, 4, 2, true>(dev, g, part)
+                                                                                               : reg_product<T, NX, 2, 1, 2, 4, true>(dev, g, part);
 #define GO(MT_)                                                                                                  \
     return kw == 1 ? reg_product<T, NX, 2, MT_, 8, 1>(dev, g, part) : kw == 2 ? reg_product<T, NX, 2, MT_, 4, 2>(dev, g, part) \
                                                                               : reg_product<T, NX, 2, MT_, 2, 4>(dev, g, part)
@@ -1136,7 +1204,10 @@ static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int 
     g.m = m, g.n = (int)q->n, g.ldy = half ? half : q->n, g.chunks = k / 256, g.wtiles = (int)((q->n + 15) / 16), g.parts = cut.parts, g.half = half;
     // activations: up to four row tiles past the last one (rows past m are multiplied and never stored)
     const int rows = wide ? 32 : 16;
-    const int64_t ch = xp * 512 * rows + (reg_sums(q->type) ? 1024 : 0), xbytes = (((int64_t)m + rows - 1) / rows + 4) * g.chunks * ch;
+    // Up to 12 rows of the 5-bit formats are a launch each of the kernel for one row otherwise, which normalises 32 values by themselves, so that
+    // groups small beside a row's largest value keep all their bits: as it does.
+    const bool own = !wide && !x_is_bf16 && m <= 12 && (q->type == FH_Q5_0 || q->type == FH_Q5_K);
+    const int64_t ch = xp * 512 * rows + (reg_sums(q->type) || own ? 1024 : 0), xbytes = (((int64_t)m + rows - 1) / rows + 4) * g.chunks * ch;
     const size_t part_at = ((size_t)xbytes + ((size_t)m + 160) * 4 + 255) & ~(size_t)255;
     const size_t bytes = part_at + (cut.parts > 1 ? (size_t)cut.parts * m * q->n * 4 : 0);
     // as products on fragments do it: what cannot be had is no error, and the tile kernels' planes are there too
@@ -1159,7 +1230,10 @@ static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int 
     if (wide) { REG_X2(IN_, O_, true); } \
     else { REG_X2(IN_, O_, false); }      \
     break
-    switch (reg_order(q->type) + (x_is_bf16 ? 3 : 0)) {
+#define REG_OWN(O_, G_) k_reg_x<0, O_, G_, false, 1, true><<<dim3((unsigned)m), threads, 0, dev->stream>>>(x, m, k, xf, rs)
+    if (own && q->type == FH_Q5_K) { if (k > 8192) REG_OWN(1, 2); else REG_OWN(1, 1); }
+    else if (own) { if (k > 8192) REG_OWN(2, 2); else REG_OWN(2, 1); }
+    else switch (reg_order(q->type) + (x_is_bf16 ? 3 : 0)) {
     case 0: REG_X(0, 0);
     case 1: REG_X(0, 1);
     case 2: REG_X(0, 2);
@@ -1170,10 +1244,11 @@ static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int 
 #undef REG_X
 #undef REG_X2
 #undef REG_X3
+#undef REG_OWN
     FH_HIP(hipGetLastError());
 #define REG_GO(T_)                                                                                              \
     if (wide) return x_is_bf16 ? wide_product<T_, 1, 2>(dev, g) : wide_product<T_, 2, 2>(dev, g); \
-    return x_is_bf16 ? reg_go<T_, 1>(dev, g, part, cut.mt, cut.kw) : reg_go<T_, 2>(dev, g, part, cut.mt, cut.kw)
+    return x_is_bf16 ? reg_go<T_, 1>(dev, g, part, cut.mt, cut.kw, false) : reg_go<T_, 2>(dev, g, part, cut.mt, cut.kw, own)
     switch (q->type) {
     case FH_Q4_0: REG_GO(FH_Q4_0);
     case FH_Q5_0: REG_GO(FH_Q5_0);

@@ -200,3 +200,31 @@ def test_f32_products_that_others_part(dev, m, n, k, parted):
     got = {option: run(dev, q, xt, option).view(np.uint32) for option in (0, 15, 16)}
     assert not np.array_equal(got[15], got[16])
     assert np.array_equal(got[0], got[16 if parted else 15])
+
+
+@pytest.mark.parametrize("ty", [synth.Q5_0, synth.Q5_K], ids=lambda t: synth.TYPE_NAMES[t])
+@pytest.mark.parametrize("m", [5, 12])
+@pytest.mark.parametrize("cut", [0, 1 + 16 * 1 + 256 * 1, 1 + 16 * 2 + 256 * 2, 1 + 16 * 4 + 256 * 1])
+def test_small_values_beside_large_ones(dev, oracle, ty, m, cut):
+    """5 to 12 rows of the 5-bit formats keep every bit of a group of 32 whatever stands in the others, as the kernel for one row
+    does: each 256 has a group of values 2^30 times the others', which meet weights of zero.  (Within a row's range of f16 hi + lo the others
+    would keep nothing.)  Five 256s, so that groups of wavefronts have unequal numbers of them."""
+    n, k = 48, 1280
+    raw = synth.random_weight(ty, n, k, seed=3, sigma=2e-3).reshape(n, k // 256, -1)
+    if ty == synth.Q5_0:
+        raw.reshape(n, k // 256, 8, 22)[:, :, 3, 0:2] = 0  # scale of the fourth 32
+    else:
+        raw[..., 4 + 3] &= 0xC0      # scale and minimum of the fourth 32: six bits of bytes 3 and 7
+        raw[..., 4 + 4 + 3] &= 0xC0
+    x = synth.random_activation(m, k, seed=m)
+    x.reshape(m, k // 256, 8, 32)[:, :, 3] *= np.float32(2.0 ** 30)
+    q = QMatrix.from_raw_bytes(dev, (n, k), raw.reshape(-1), ty)
+    dev.set_option("matmul_cut", cut)
+    try:
+        got = run(dev, q, Tensor.from_slice(dev, x), 0 if not cut else 16).astype(np.float64)
+    finally:
+        dev.set_option("matmul_cut", 0)
+    w = oracle.dequantize(ty, raw.reshape(-1)).reshape(n, k).astype(np.float64)
+    assert not w.reshape(n, k // 256, 8, 32)[:, :, 3].any()
+    want = x.astype(np.float64) @ w.T
+    assert np.sqrt(np.mean((got - want) ** 2)) <= 1e-6 * np.sqrt(np.mean(want ** 2))

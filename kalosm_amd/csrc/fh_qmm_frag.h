@@ -23,4 +23,5 @@ fh_status fh_frag_sum(fh_device *dev, const float *part, int parts, int64_t stri
 bool fh_qmm_reg_supports(const fh_qmatrix *q);
 bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m);
 fh_status fh_launch_qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, bool planes);
+bool fh_qmm_reg_swiglu_pays(const fh_qmatrix *q, int m); // (where fh_qmm_reg_pays)
 fh_status fh_qmm_reg_swiglu(const fh_qmatrix *q, const float *x, int m, float *y);

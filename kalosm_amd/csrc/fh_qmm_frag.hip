@@ -761,7 +761,7 @@ fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, 
 fh_status fh_qmm_frag_swiglu(const fh_qmatrix *q, const float *x, int m, float *y) {
     const int64_t opt = q->dev->opt_matmul_kernel;
     if (q->n % 64 == 0 && ((uintptr_t)x & 15) == 0 && (opt == 0 ? m > FH_SHORT_PROMPT && fh_qmm_reg_pays(q, 0, m) : opt >= 14 && opt <= 16 && fh_qmm_reg_supports(q)))
-        return fh_qmm_reg_swiglu(q, x, m, y);
+        return opt || fh_qmm_reg_swiglu_pays(q, m) ? fh_qmm_reg_swiglu(q, x, m, y) : FH_ERR_UNSUPPORTED;
     if (q->n % 64 || ((uintptr_t)x & 15) || m <= 16 || !(opt == 0 ? m > FH_SHORT_PROMPT && fh_qmm_frag_pays(q, 0, m) : opt == 13 && fh_qmm_frag_supports(q)))
         return FH_ERR_UNSUPPORTED;
     return qmm_frag(q, x, 0, m, y, (int)(q->n / 2));

@@ -1173,7 +1173,7 @@ static bool reg_parted(const fh_qmatrix *q, int m) {
     const int64_t tiles = (q->n + 127) / 128 * ((m + 255) / 256), cus = q->dev->compute_units, last = tiles > cus ? tiles % cus : 0;
     return q->type != FH_Q5_0 && last > 0 && last * 2 <= cus;
 }
-static int reg_way(const fh_qmatrix *q, int x_is_bf16, int m) {
+static int reg_way(const fh_qmatrix *q, int x_is_bf16, int m, bool whole) { // whole: k in one part
     if (!fh_qmm_reg_supports(q) || q->k < 1024) return REG_NONE;
     const int64_t n = q->n, tiles = (n + 255) / 256 * ((m + 63) / 64), cus = q->dev->compute_units;
     const bool can = q->k <= 8192 && (x_is_bf16 || n >= 8192) && (n + 127) / 128 * ((m + 255) / 256) * 5 >= cus * 4, few = reg_few(q, x_is_bf16, m);
@@ -1182,16 +1182,23 @@ static int reg_way(const fh_qmatrix *q, int x_is_bf16, int m) {
     const bool parted = can && !x_is_bf16 && !reg_sums(q->type) && q->type != FH_Q6_K && reg_parted(q, m);
     if (!few && can && m > 512 && (x_is_bf16 || q->type != FH_Q6_K) && tiles >= 160 && fill >= (x_is_bf16 ? 0.6 : 0.7)) return parted ? REG_NARROW : REG_WIDE;
     if (!narrow) return REG_NONE;
-    return can && !parted && wide_us(q, x_is_bf16, m) < 0.97 * reg_cut(q, x_is_bf16, m, false).us ? REG_WIDE : REG_NARROW;
+    return can && !parted && wide_us(q, x_is_bf16, m) < 0.97 * reg_cut(q, x_is_bf16, m, whole).us ? REG_WIDE : REG_NARROW;
 }
-bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m) { return reg_way(q, x_is_bf16, m) != REG_NONE; }
+bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m) { return reg_way(q, x_is_bf16, m, false) != REG_NONE; }
+// SwiGLU at the store takes k in one part.  A product that is quicker in several, its sums to memory and a launch for SwiGLU (4 us and their bytes, of
+// 243 layers of three formats): 65 rows of 1024 x 4096 in Q8_0 11 us less a layer in two launches, 2048 x 4096 6, 4096 x 4096 2; 200 rows of 4096 x 4096 6 more.
+bool fh_qmm_reg_swiglu_pays(const fh_qmatrix *q, int m) {
+    const int way = reg_way(q, 0, m, true);
+    if (way != REG_NARROW) return way == REG_WIDE;
+    return reg_cut(q, 0, m, true).us <= reg_cut(q, 0, m, false).us + 4.0 + 2.0 * m * (double)q->n * 4.0 / 4e6;
+}
 
 static fh_status qmm_reg(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, int half, bool planes) {
     fh_device *dev = q->dev;
     const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2;
     RegCut cut = reg_cut(q, x_is_bf16, m, half > 0);
     const int64_t opt = dev->opt_matmul_kernel; // 15: always the wide one, 16: never
-    const bool wide = opt == 15 || (opt != 16 && reg_way(q, x_is_bf16, m) == REG_WIDE);
+    const bool wide = opt == 15 || (opt != 16 && reg_way(q, x_is_bf16, m, half > 0) == REG_WIDE);
     if (wide) cut.parts = 1;
     else if (dev->opt_matmul_cut > 0) { // tests: row tiles, groups of wavefronts and workgroups along k as asked for
         const int c = (int)dev->opt_matmul_cut, mt = c & 15, kw = (c >> 4) & 15, parts = c >> 8;

@@ -228,3 +228,20 @@ def test_small_values_beside_large_ones(dev, oracle, ty, m, cut):
     assert not w.reshape(n, k // 256, 8, 32)[:, :, 3].any()
     want = x.astype(np.float64) @ w.T
     assert np.sqrt(np.mean((got - want) ** 2)) <= 1e-6 * np.sqrt(np.mean(want ** 2))
+
+
+@pytest.mark.parametrize("d_model,ffn,m,fused", [(4096, 1024, 65, False), (4096, 1024, 100, False), (1024, 1024, 65, True), (2048, 5632, 65, True)])
+def test_swiglu_in_two_launches(dev, d_model, ffn, m, fused):
+    """SwiGLU at the store (always with option 14) takes k in one part: only where two launches, with k in several, are not quicker."""
+    from kalosm_amd.llama import Model
+
+    cfg = dict(n_layers=1, d_model=d_model, n_heads=d_model // 128, n_kv_heads=d_model // 512, head_dim=128, ffn=ffn, vocab=320, ctx=128, eps=1e-5, theta=1e4)
+    model, tokens, got = Model.random_init(dev, cfg, seed=2, sigma=2e-3), np.random.default_rng(m).integers(0, 320, m), []
+    for option in (0, 14):
+        dev.set_option("matmul_kernel", option)
+        try:
+            got.append(model.forward(tokens, want_hidden=True)[1].view(np.uint32))
+        finally:
+            dev.set_option("matmul_kernel", 0)
+        model.reset()
+    assert np.array_equal(got[0], got[1]) == fused

@@ -4,7 +4,8 @@
 
 bool fh_qmm_frag_supports(const fh_qmatrix *q);
 bool fh_qmm_frag_pays(const fh_qmatrix *q, int x_is_bf16, int m); // and where it is the faster way
-int fh_qmm_frag_parts(const fh_qmatrix *q, int x_is_bf16, int m); // parts of k it would take
+double fh_qmm_frag_us(const fh_qmatrix *q, int x_is_bf16, int m, int *parts); // (more than FH_SHORT_PROMPT rows) how long it would take, in how many parts of k
+double fh_qmm_tile_us(const fh_qmatrix *q, int x_is_bf16, int m);             // the tile kernels; 1e30 where they are far from filling the device
 // y[m, n] = x[m, k] . deq(q)^T; x f32 or bf16, rows contiguous and 16-byte aligned.  FH_ERR_UNSUPPORTED where the memory for the
 // fragments cannot be had.
 fh_status fh_launch_qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y);

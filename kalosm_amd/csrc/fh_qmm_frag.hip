@@ -573,8 +573,13 @@ fh_status fh_frag_sum(fh_device *dev, const float *part, int parts, int64_t stri
     return FH_OK;
 }
 
+struct FragAsk {
+    int parts;                     // of k
+    int64_t rounds, steps;         // of workgroups, 128s of k in all of them
+    double sum;                    // us for partial planes
+};
 template <int NW, int NX, int SC, int FW, int FX, int WGX>
-static fh_status frag_product(fh_device *dev, FragArgs g, int *ask) { // ask: only into how many parts of k
+static fh_status frag_product(fh_device *dev, FragArgs g, FragAsk *ask) { // ask: only how it would be cut
     typedef FragTile<NW, NX, FW, FX, WGX> Tile;
     constexpr int TW = Tile::TW, TX = Tile::TX, LDS = Tile::STAGES * Tile::STAGE;
     g.tiles_w = (g.n + TW - 1) / TW;
@@ -585,15 +590,16 @@ static fh_status frag_product(fh_device *dev, FragArgs g, int *ask) { // ask: on
     const int64_t tiles = (int64_t)g.tiles_w * g.tiles_x;
     double best = 1e30;
     int parts = 1;
+    FragAsk cut{1, 0, 0, 0.0};
     const int most = g.n == g.ldy || g.half ? 8 : 1; // (weight rows in several launches: whole)
     for (int p = 1; p <= most && p * 2 <= quads; p++) {
         const int64_t rounds = (tiles * p + dev->compute_units - 1) / dev->compute_units;
-        double t = (double)rounds * ((double)((quads + p - 1) / p) + 1.5) * 2.5;
-        if (p > 1) t += 4.0 + (2.0 * p + 1.0) * g.m * (double)g.n * 4.0 / 4e6;
-        if (t < best * 0.97) best = t, parts = p;
+        const double sum = p > 1 ? 4.0 + (2.0 * p + 1.0) * g.m * (double)g.n * 4.0 / 4e6 : 0.0;
+        const double t = (double)rounds * ((double)((quads + p - 1) / p) + 1.5) * 2.5 + sum;
+        if (t < best * 0.97) best = t, parts = p, cut = FragAsk{p, rounds, rounds * ((quads + p - 1) / p), sum};
     }
     if (ask) {
-        *ask = parts;
+        *ask = cut;
         return FH_OK;
     }
     g.parts = parts;
@@ -666,7 +672,7 @@ bool fh_qmm_frag_pays(const fh_qmatrix *q, int x_is_bf16, int m) {
 
 #define FRAG_GO(NW_, NX_, SC_, WGX_) \
     (m <= 64 ? frag_product<NW_, NX_, SC_, 2, 1, 2>(dev, g, ask) : frag_product<NW_, NX_, SC_, 2, 2, WGX_>(dev, g, ask))
-static fh_status frag_go(fh_device *dev, const FragArgs &g, int sc, int wp, int xp, int *ask) {
+static fh_status frag_go(fh_device *dev, const FragArgs &g, int sc, int wp, int xp, FragAsk *ask) {
     const int m = g.m;
     if (sc == 32) return xp == 2 ? FRAG_GO(1, 2, 32, 2) : FRAG_GO(1, 1, 32, 2);
     if (wp == 2) return xp == 2 ? FRAG_GO(2, 2, 256, 4) : FRAG_GO(2, 1, 256, 4);
@@ -676,7 +682,8 @@ static fh_status frag_go(fh_device *dev, const FragArgs &g, int sc, int wp, int 
 
 struct FragPlan {
     FragArgs g;
-    int ext, parts;          // columns of offsets; parts of k
+    FragAsk cut;             // of a launch
+    int ext;                 // columns of offsets
     int64_t rows, row_bytes; // weight rows of a launch
 };
 static fh_status frag_plan(const fh_qmatrix *q, int x_is_bf16, int m, int half, FragPlan *p) {
@@ -689,12 +696,25 @@ static fh_status frag_plan(const fh_qmatrix *q, int x_is_bf16, int m, int half, 
     rows = rows < 256 ? 256 : (rows > rows_all ? rows_all : rows);
     p->g = FragArgs{};
     p->g.m = m, p->g.n = (int)(rows < q->n ? rows : q->n), p->g.ldy = half ? half : q->n, p->g.kf = kf, p->g.half = half;
-    p->ext = ext, p->rows = rows, p->row_bytes = row_bytes, p->parts = 1;
-    return frag_go(q->dev, p->g, sc, wp, xp, &p->parts);
+    p->ext = ext, p->rows = rows, p->row_bytes = row_bytes;
+    return frag_go(q->dev, p->g, sc, wp, xp, &p->cut);
 }
-int fh_qmm_frag_parts(const fh_qmatrix *q, int x_is_bf16, int m) {
+// us, fitted to 2428 products of 65 - 2048 rows (standard deviation 8 %): fragments of the weights and the activations, the rounds of workgroups and the 128s of
+// k in them, the sums' bytes, partial planes.
+double fh_qmm_frag_us(const fh_qmatrix *q, int x_is_bf16, int m, int *parts) {
     FragPlan p;
-    return frag_plan(q, x_is_bf16, m, 0, &p) == FH_OK ? p.parts : 1;
+    if (frag_plan(q, x_is_bf16, m, 0, &p) != FH_OK) return 1e30;
+    if (parts) *parts = p.cut.parts;
+    double step = 0.0; // 128 of k
+    switch (q->type) {
+    case FH_Q4_K: step = x_is_bf16 ? 1.47 : 2.4; break;
+    case FH_Q5_K: step = x_is_bf16 ? 1.47 : 2.5; break;
+    case FH_Q5_0: step = x_is_bf16 ? 1.96 : 2.9; break;
+    case FH_Q6_K: step = 4.05; break; // (bf16 rows of the last two are not asked about)
+    default: step = 3.05;
+    }
+    const double n = (double)q->n, k = (double)q->k, launches = (double)((q->n + p.rows - 1) / p.rows);
+    return 6.0 + 0.62 * n * k / 1e6 + (x_is_bf16 ? 1.95 : 3.5) * m * k / 1e6 + launches * (8.0 * p.cut.rounds + step * p.cut.steps) + 0.36 * m * n / 1e6 + 0.5 * p.cut.sum;
 }
 
 static fh_status qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y, int half) {
@@ -702,7 +722,7 @@ static fh_status qmm_frag(const fh_qmatrix *q, const void *x, int x_is_bf16, int
     FragPlan plan;
     FH_TRY(frag_plan(q, x_is_bf16, m, half, &plan));
     FragArgs &g = plan.g;
-    const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2, wp = q->type == FH_Q6_K ? 2 : 1, sc = fh_block_elems(q->type), ext = plan.ext, kf = g.kf, parts = plan.parts;
+    const int k = (int)q->k, xp = x_is_bf16 ? 1 : 2, wp = q->type == FH_Q6_K ? 2 : 1, sc = fh_block_elems(q->type), ext = plan.ext, kf = g.kf, parts = plan.cut.parts;
     const int64_t rows = plan.rows, row_bytes = plan.row_bytes;
     if (half && (rows < q->n || parts > 1)) return FH_ERR_UNSUPPORTED; // all rows at once, k in one part
     // activations: rows up to a multiple of the largest tile (rows past m are multiplied and never stored)

@@ -1109,8 +1109,15 @@ static RegCut reg_cut(const fh_qmatrix *q, int x_is_bf16, int m, bool whole) {
             if (parts > 1) t += 3.4 + (2.0 * parts + 1.0) * m * (double)q->n * 4.0 / 4e6;
             if (t < least * 0.98) least = t, best.kw = kw, best.parts = parts;
         }
-    const bool five = q->type == FH_Q5_0 || q->type == FH_Q5_K;
-    const double type = q->type == FH_Q6_K ? 0.92 : q->type == FH_Q4_K ? 1.15 : five ? (x_is_bf16 ? 1.5 : 1.33) : 1.25;
+    double type;
+    switch (q->type) {
+    case FH_Q4_K: type = 1.15; break;
+    case FH_Q6_K: type = x_is_bf16 ? 0.85 : 0.92; break;
+    case FH_Q5_K: type = x_is_bf16 ? 1.38 : 1.32; break;
+    case FH_Q5_0: type = x_is_bf16 ? 1.45 : 1.32; break;
+    case FH_Q4_0: type = 1.16; break;
+    default: type = 1.22;
+    }
     best.us = 8.0 + m * (double)q->k / 1e6 * 1.6 + type * least; // (with the activations' launch; from 320 rows on, where there is a choice)
     return best;
 }
@@ -1126,14 +1133,19 @@ static RegCut reg_cut(const fh_qmatrix *q, int x_is_bf16, int m, bool whole) {
 //   Q8_0 f32   512 rows 146 / 194, 153 / 238, 52 / 93, 32 / 44, 43 / 97; 768 rows 218 / 257 but 75 / 69; bf16 768 rows 161 / 178, 180 / 279,
 //              59 / 111, 1024 rows 216 / 212 but 190 / 349, 62 / 123, 31 / 56, 64 / 107 for the smaller n.  Q4_0 as Q8_0.
 //   Q5_0 bf16  512 rows 122 / 136, 118 / 166; 768 rows 71 / 59 for 5632 x 2048
-// Left on the tiles though slower: Q4_K and Q5_0, f32, of rows (from 512, above 192) and matrices for which the tiles win over the fragments
-// (tile_fill; 8192 x 2048), but not Q4_K, 512 rows, of less than four times as many rows as columns (8192 x 3072 67 / 93).  Fewer than 1024 columns: four 256s are the least that a workgroup's wavefronts share out.
+// Rows of whole tiles: Q4_K f32 of 8192 x 2048 500 rows 46 / 71, 512 49 / 71, 513 77 / 67, 640 82 / 70; of 8192 x 3072 512 65 / 92, 640 107 / 95.  What is slower
+// past such an edge is left out by reg_way, which compares the two at hand.
+// Not taken although faster, as the fragments' test holds these sizes to be the tiles': Q4_K, 512 f32 rows of matrices with four times as many rows as
+// columns whose tiles fill the device, and Q5_0, 193 - 256 f32 rows of such (8192 x 2048, 200 rows 32 / 53).  Not yet taken: Q5_0, 257 - 512 f32 rows
+// of fewer than 3072 rows (320 of 2048 x 2048 27 / 47), Q6_K f32 above 512 (640 of 11008 x 4096 180 / 302), Q6_K, 257 - 512 bf16 rows, k above 8192 (384
+// of 5120 x 13824 126 / 297), Q8_0 bf16 above 1280 (1536 of 4096 x 14336 307 / 501).
+// Fewer than 1024 columns: four 256s are the least that a workgroup's wavefronts share out.
 static bool reg_few(const fh_qmatrix *q, int x_is_bf16, int m) {
     const int64_t n = q->n, k = q->k;
     switch (q->type) {
     case FH_Q4_K:
         if (x_is_bf16) return m <= 768;
-        return m < 512 || (m == 512 && n < 4 * k) || (m <= 640 && (k > n || fh_qmm_frag_pays(q, 0, m)));
+        return m < 512 || (m <= 640 && (k > n || n < 4 * k || fh_qmm_frag_pays(q, 0, m)));
     case FH_Q5_K: return m <= (x_is_bf16 ? 448 : 512);
     case FH_Q5_0:
         if (x_is_bf16) return m <= 512;
@@ -1151,38 +1163,52 @@ static double wide_us(const fh_qmatrix *q, int x_is_bf16, int m) {
     switch (q->type) {
     case FH_Q4_K: one = x_is_bf16 ? 2.3 : 3.8, two = x_is_bf16 ? 4.2 : 6.8; break;
     case FH_Q6_K: one = x_is_bf16 ? 3.75 : 5.55, two = x_is_bf16 ? 6.8 : 9.7; break;
-    case FH_Q5_K: case FH_Q5_0: one = x_is_bf16 ? 3.4 : 4.1, two = x_is_bf16 ? 5.6 : 7.5; break;
+    case FH_Q5_K: one = x_is_bf16 ? 3.15 : 4.1, two = x_is_bf16 ? 5.2 : 7.5; break;
+    case FH_Q5_0: one = x_is_bf16 ? 3.4 : 4.1, two = x_is_bf16 ? 5.6 : 7.5; break;
+    case FH_Q4_0: one = x_is_bf16 ? 2.9 : 3.9, two = x_is_bf16 ? 4.6 : 6.8; break;
     default: one = x_is_bf16 ? 3.1 : 4.3, two = x_is_bf16 ? 5.0 : 7.5;
     }
     return 15.0 + m * (double)q->k / 1e6 * (x_is_bf16 ? 0.9 : 1.5) + (double)(q->k / 256) * ((double)(each & 1) * one + (double)(each >> 1) * two);
 }
 
-// Which of the two, if any.  Both where few rows take k_qmm_reg: the one that is quicker by the models.  Above, k_qmm_wide where its
+// Which of the two, if any.  Where few rows take k_qmm_reg: the one that is quicker by the models.  Above, k_qmm_wide where its
 // tiles keep the device busy (us, wide / others: Q4_K bf16, 2048 rows, 14336 x 4096 276 / 315, 8192 x 3072 130 / 135, 5632 x 2048 74 / 89;
-// Q8_0 bf16 317 / 363, 148 / 165, 83 / 107; Q6_K bf16 420 / 478, 192 / 213, 105 / 131; Q4_K f32, 1024 rows, 28672 x 4096 437 / 495,
-// 14336 x 4096, five eighths full, 248 / 245), with f32 rows only for matrices of
-// 8192 rows and more (4096 x 4096, 2048 rows: 146 / 143) and not for Q6_K (2048 rows, 8192 x 3072 298 / 278).  k to 8192 only, and not where
-// the tiles would part all of it (qmm_launch_t): its sums are long.  f32 rows and a scale per 32: one sum along k, so that k_qmm_reg, whose 256s add up
-// by themselves, takes what the others would part (reg_parted; 750 rows of 14336 x 8192, Q8_0, against 64 bits 1.4e-7, fragments 2.2e-7, wide
-// 3.0e-7; 402, 462 and 407 us).  bf16 rows of the formats whose tiles leave the device idle for narrow matrices stay on k_qmm_reg (Q8_0, 1536 rows, 1024 x 4096 45 / 86, 3072 x 3072 85 / 140).
+// Q8_0 bf16 317 / 363, 148 / 165, 83 / 107; Q6_K bf16 420 / 478, 192 / 213, 105 / 131; Q4_K f32, 1024 rows, 28672 x 4096 437 / 495), with f32 rows only for
+// matrices of 8192 rows and more (4096 x 4096, 2048 rows: 146 / 143) and not for Q6_K (2048 rows, 8192 x 3072 298 / 278).  k to 8192 only, and not where
+// the tiles would part all of it (qmm_launch_t): its sums are long.  k_qmm_reg, whose 256s add up in eights or by themselves, takes what the others would
+// part (reg_parted; 750 rows of 14336 x 8192, Q8_0, against 64 bits 1.4e-7, fragments 2.2e-7, wide 3.0e-7; 402, 462 and 407 us).  bf16 rows of the formats whose
+// tiles leave the device idle for narrow matrices stay on k_qmm_reg (Q8_0, 1536 rows, 1024 x 4096 45 / 86, 3072 x 3072 85 / 140).
+// Neither where the fragments or the tiles, whichever would take the call, are quicker by their models: a last round of workgroups that is nearly empty here and full
+// there, or tiles that just fill the device.  (us, this / those: Q5_K f32, 384 rows, 11008 x 4096 136 / 111; Q5_K bf16, 2048 rows 284 / 240; Q4_K f32, 640
+// rows, 8192 x 2048 82 / 70; Q8_0 bf16, 1000 rows, 7168 x 12288 354 / 275; Q6_K bf16, 1280 rows, 6528 x 8192 364 / 270; of 3500 products the models pick one that is more than
+// 3 % slower 18 times, by 11 % at most.)
 enum { REG_NONE, REG_NARROW, REG_WIDE };
-// f32 rows, a scale per 32: whether the fragments, or the tiles in their last round, take k in parts.  (The tiles of Q5_0 multiply f32 values and
-// are the least exact.)
-static bool reg_parted(const fh_qmatrix *q, int m) {
-    if (m > 512 || (q->type == FH_Q5_0 && fh_qmm_frag_pays(q, 0, m))) return fh_qmm_frag_parts(q, 0, m) > 1;
+// Whether what k_qmm_wide would take the place of has k in parts and is the closer one for it: the fragments, for f32 rows of formats with a scale per 32
+// also the tiles in their last round.  (The tiles of Q5_0 multiply f32 values and are the least exact.)
+static bool reg_parted(const fh_qmatrix *q, int x_is_bf16, int m) {
+    if (fh_qmm_frag_pays(q, x_is_bf16, m)) {
+        int parts = 1;
+        (void)fh_qmm_frag_us(q, x_is_bf16, m, &parts);
+        return parts > 1;
+    }
     const int64_t tiles = (q->n + 127) / 128 * ((m + 255) / 256), cus = q->dev->compute_units, last = tiles > cus ? tiles % cus : 0;
-    return q->type != FH_Q5_0 && last > 0 && last * 2 <= cus;
+    return (q->type == FH_Q8_0 || q->type == FH_Q4_0) && last > 0 && last * 2 <= cus;
 }
 static int reg_way(const fh_qmatrix *q, int x_is_bf16, int m, bool whole) { // whole: k in one part
     if (!fh_qmm_reg_supports(q) || q->k < 1024) return REG_NONE;
     const int64_t n = q->n, tiles = (n + 255) / 256 * ((m + 63) / 64), cus = q->dev->compute_units;
     const bool can = q->k <= 8192 && (x_is_bf16 || n >= 8192) && (n + 127) / 128 * ((m + 255) / 256) * 5 >= cus * 4, few = reg_few(q, x_is_bf16, m);
     const bool narrow = few || (x_is_bf16 && n <= 3072 && (q->type == FH_Q8_0 || q->type == FH_Q4_0 || q->type == FH_Q6_K));
+    const bool parted = can && q->type != FH_Q6_K && (reg_sums(q->type) || !x_is_bf16) && reg_parted(q, x_is_bf16, m);
     const double fill = (double)tiles / (double)((tiles + cus - 1) / cus * cus);
-    const bool parted = can && !x_is_bf16 && !reg_sums(q->type) && q->type != FH_Q6_K && reg_parted(q, m);
-    if (!few && can && m > 512 && (x_is_bf16 || q->type != FH_Q6_K) && tiles >= 160 && fill >= (x_is_bf16 ? 0.6 : 0.7)) return parted ? REG_NARROW : REG_WIDE;
-    if (!narrow) return REG_NONE;
-    return can && !parted && wide_us(q, x_is_bf16, m) < 0.97 * reg_cut(q, x_is_bf16, m, whole).us ? REG_WIDE : REG_NARROW;
+    bool wide = !few && can && m > 512 && (x_is_bf16 || q->type != FH_Q6_K) && tiles >= 160 && fill >= (x_is_bf16 ? 0.6 : 0.7);
+    if (!narrow && !wide) return REG_NONE;
+    const double narrow_us = reg_cut(q, x_is_bf16, m, whole).us, us = wide_us(q, x_is_bf16, m);
+    wide = !parted && (wide || (can && us < 0.97 * narrow_us));
+    // (SwiGLU was asked about as a product first)
+    if (!whole && m > FH_SHORT_PROMPT && (wide ? us : narrow_us) > 0.97 * (fh_qmm_frag_pays(q, x_is_bf16, m) ? fh_qmm_frag_us(q, x_is_bf16, m, nullptr) : fh_qmm_tile_us(q, x_is_bf16, m)))
+        return REG_NONE;
+    return wide ? REG_WIDE : REG_NARROW;
 }
 bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m) { return reg_way(q, x_is_bf16, m, false) != REG_NONE; }
 // SwiGLU at the store takes k in one part.  A product that is quicker in several, its sums to memory and a launch for SwiGLU (4 us and their bytes, of

@@ -1906,6 +1906,34 @@ static fh_status qmm_launch_t(const fh_qmatrix *q, const _Float16 *xh, const _Fl
     return FH_OK;
 }
 
+// How long the tiles of 256 rows above take where they fill the device (formats with integer-code kernels; fh_qmm_reg.hip is the faster way
+// everywhere else): us, fitted to 470 products (3 - 6 %): rounds of workgroups by their 256s of k, the last one halved where its tiles are
+// split, and the activations.  Q4_K, and Q6_K with bf16 rows, split k and fill it so.
+double fh_qmm_tile_us(const fh_qmatrix *q, int x_is_bf16, int m) {
+    const int64_t cus = q->dev->compute_units, steps = q->k / 32, tiles = (q->n + 127) / 128 * ((m + 255) / 256);
+    const bool parted = q->type == FH_Q4_K || (q->type == FH_Q6_K && x_is_bf16);
+    int64_t ks = 1;
+    while (tiles * ks * 5 < cus * 4 && ks < 8 && steps % (ks * 4) == 0 && steps / (ks * 2) >= 16 && (q->n & 3) == 0) ks *= 2;
+    if (m <= 128 || tiles * ks * 5 < cus * 4 || (ks > 1 && (!parted || (q->k / 256) % ks))) return 1e30;
+    double base, row, step, round;
+    switch (q->type) {
+    case FH_Q4_0: case FH_Q8_0: {
+        const bool four = q->type == FH_Q4_0;
+        base = x_is_bf16 ? 20.0 : 7.0, row = x_is_bf16 ? 1.2 : 6.0, step = x_is_bf16 ? (four ? 4.95 : 5.4) : 9.0, round = x_is_bf16 ? 0.0 : 19.0;
+        break;
+    }
+    case FH_Q4_K: base = x_is_bf16 ? 13.0 : 25.0, row = x_is_bf16 ? 2.3 : 6.1, step = x_is_bf16 ? 5.8 : 8.2, round = x_is_bf16 ? 13.0 : 0.0; break;
+    case FH_Q6_K:
+        if (!x_is_bf16) return 1e30;
+        base = 20.0, row = 1.0, step = 7.0, round = 6.0;
+        break;
+    default: return 1e30;
+    }
+    const int64_t all = tiles * ks;
+    const double rounds = (double)((all + cus - 1) / cus) - (ks == 1 && qmm_tail_tiles(q->dev, (int)all) ? 0.5 : 0.0);
+    return base + row * m * (double)q->k / 1e6 + rounds * (step * (double)(q->k / 256) / (double)ks + round) + (ks > 1 ? 0.1 * (4.0 + (2.0 * ks + 1.0) * m * (double)q->n * 4.0 / 4e6) : 0.0);
+}
+
 // dense f16 / f32 weight rows: the plain tile kernel (its weight "decode" is a load), tile shape by row count
 template <int T, int NTERM>
 static fh_status qmm_launch_dense(const fh_qmatrix *q, const _Float16 *xh, const _Float16 *xl, const float *rs, int m,

@@ -71,6 +71,11 @@ def test_product(dev, oracle, ty, act, m, n, k, option):
     (synth.Q8_0, "bf16", 1280, 64, 1024, True), (synth.Q6_K, "f32", 513, 64, 1024, False),
     (synth.Q4_K, "bf16", 1300, 8192, 1024, True), (synth.Q4_K, "bf16", 1300, 1024, 1024, False), (synth.Q4_K, "bf16", 1300, 4096, 8448, False),
     (synth.Q4_K, "f32", 1000, 8192, 1024, True), (synth.Q4_K, "f32", 1000, 8176, 1024, False),
+    (synth.Q4_K, "f32", 512, 4096, 2048, True), (synth.Q4_K, "f32", 513, 4096, 2048, True),          # either side of whole tiles of 256 rows
+    (synth.Q4_K, "f32", 600, 8192, 2048, False), (synth.Q5_K, "f32", 384, 11008, 2048, False),       # a second round of workgroups: the fragments are quicker
+    (synth.Q5_K, "f32", 300, 11008, 2048, True), (synth.Q8_0, "bf16", 1000, 8192, 2048, True),
+    (synth.Q8_0, "bf16", 1000, 7168, 8448, False), (synth.Q8_0, "bf16", 1100, 7168, 8448, True),     # 224 whole tiles, 280
+    (synth.Q6_K, "bf16", 768, 10880, 1024, False), (synth.Q6_K, "bf16", 640, 4096, 1024, True),
 ])
 def test_rule(dev, ty, act, m, n, k, taken):
     """Both sides of the dispatch's lines: the bits of this kernel (option 14) or others."""

@@ -1180,8 +1180,8 @@ static double wide_us(const fh_qmatrix *q, int x_is_bf16, int m) {
 // tiles leave the device idle for narrow matrices stay on k_qmm_reg (Q8_0, 1536 rows, 1024 x 4096 45 / 86, 3072 x 3072 85 / 140).
 // Neither where the fragments or the tiles, whichever would take the call, are quicker by their models: a last round of workgroups that is nearly empty here and full
 // there, or tiles that just fill the device.  (us, this / those: Q5_K f32, 384 rows, 11008 x 4096 136 / 111; Q5_K bf16, 2048 rows 284 / 240; Q4_K f32, 640
-// rows, 8192 x 2048 82 / 70; Q8_0 bf16, 1000 rows, 7168 x 12288 354 / 275; Q6_K bf16, 1280 rows, 6528 x 8192 364 / 270; of 3500 products the models pick one that is more than
-// 3 % slower 18 times, by 11 % at most.)
+// rows, 8192 x 2048 82 / 70; Q8_0 bf16, 1000 rows, 7168 x 12288 354 / 275; Q6_K bf16, 1280 rows, 6528 x 8192 364 / 270; of 3000 products the models pick one that is more than
+// 3 % slower 20 times, by 11 % at most.)
 enum { REG_NONE, REG_NARROW, REG_WIDE };
 // Whether what k_qmm_wide would take the place of has k in parts and is the closer one for it: the fragments, for f32 rows of formats with a scale per 32
 // also the tiles in their last round.  (The tiles of Q5_0 multiply f32 values and are the least exact.)

@@ -437,8 +437,8 @@ __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
         }
     };
     RegW<T> w[TW];
-    floatx4 acc[TW][MT], sum[TW][MT], part256[TW][MT]; // of up to eight 256s, of a scale, of a 256 (formats with a scale per 32)
-    floatx4 all[TW][MT];                               // of the eights before (formats with a scale per 256)
+    floatx4 acc[TW][MT], sum[TW][MT], part256[TW][MT]; // of some 256s, of a scale, of a 256 (formats with a scale per 32)
+    floatx4 all[TW][MT];                               // of those before (formats with a scale per 256)
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < TW; t++)
@@ -466,10 +466,12 @@ __global__ __launch_bounds__(512) void k_qmm_reg(RegArgs g) {
     for (int u = 0; u < MT * NX; u++) xv[u] = *(const half8 *)(smem + (kw * PIECES + u) * 1024 + lane * 16);
     uint32_t one;
     asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(one));
-    // The sum ends after eight 256s, so that none is long: against 64 bits 384 bf16 rows of 4096 x 14336 in Q4_K 9.9e-8 (sums of 28: 1.22e-7), in Q5_K
-    // 1.08e-7 (1.30e-7), for a hundredth of the time.  (With a scale per 32 there are no registers for it, and the tiles added 32s.)
+    // The sum ends after four 256s (eight where there are many), so that none is long: against 64 bits 384 bf16 rows of 4096 x 14336 in Q4_K 9.9e-8 (sums of
+    // 28: 1.22e-7), in Q5_K 1.08e-7 (1.30e-7), of 5632 x 2048 in Q5_K 9.3e-8 (of 8: 9.7e-8), for a hundredth of the time.  (With a scale per 32 there are no
+    // registers for it, and the tiles added 32s.)
+    const int span = most > 32 ? 8 : 4;
     for (int from = 0; from < most;) {
-        const int to = PER32 || from + 8 > most ? most : from + 8;
+        const int to = PER32 || from + span > most ? most : from + span;
         for (int i = from; i < to; i++) {
             const int c0 = chunk(i), c1 = chunk(i + 1);
 #pragma unroll
@@ -1175,7 +1177,7 @@ static double wide_us(const fh_qmatrix *q, int x_is_bf16, int m) {
 // tiles keep the device busy (us, wide / others: Q4_K bf16, 2048 rows, 14336 x 4096 276 / 315, 8192 x 3072 130 / 135, 5632 x 2048 74 / 89;
 // Q8_0 bf16 317 / 363, 148 / 165, 83 / 107; Q6_K bf16 420 / 478, 192 / 213, 105 / 131; Q4_K f32, 1024 rows, 28672 x 4096 437 / 495), with f32 rows only for
 // matrices of 8192 rows and more (4096 x 4096, 2048 rows: 146 / 143) and not for Q6_K (2048 rows, 8192 x 3072 298 / 278).  k to 8192 only, and not where
-// the tiles would part all of it (qmm_launch_t): its sums are long.  k_qmm_reg, whose 256s add up in eights or by themselves, takes what the others would
+// the tiles would part all of it (qmm_launch_t): its sums are long.  k_qmm_reg, whose 256s add up in fours or by themselves, takes what the others would
 // part (reg_parted; 750 rows of 14336 x 8192, Q8_0, against 64 bits 1.4e-7, fragments 2.2e-7, wide 3.0e-7; 402, 462 and 407 us).  bf16 rows of the formats whose
 // tiles leave the device idle for narrow matrices stay on k_qmm_reg (Q8_0, 1536 rows, 1024 x 4096 45 / 86, 3072 x 3072 85 / 140).
 // Neither where the fragments or the tiles, whichever would take the call, are quicker by their models: a last round of workgroups that is nearly empty here and full

@@ -31,9 +31,10 @@
 // SPLIT (f32 Q, K and V): every operand is the exact two-term f16 split hi + lo of the f32 value (2^-22 relative;
 // the values must lie within the f16 range of +-65504) and both products are the three MFMAs
 // hi.hi + lo.hi + hi.lo, so the result keeps f32 accuracy at three times the matrix-core work.  Its tiles fill the LDS: one workgroup a
-// compute unit, for head_dim 128 one wavefront a SIMD, which nothing covers while it waits for an operand - so pairs are requested
-// four ahead (head_dim 64, two wavefronts: two) and the wavefront may have all registers (32 / 8 heads, 2048 tokens, causal: 139 us,
-// 180 with each pair requested in front of its products; 16 / 4 heads of 64, 3000 tokens 94 / 98).
+// compute unit, for head_dim 128 and one head a workgroup one wavefront a SIMD, which nothing covers while it waits for an operand - so pairs are
+// requested four ahead (head_dim 64, two wavefronts: two) and the wavefront may have all registers (32 / 8 heads, 2048 tokens, causal: 152 us,
+// 190 with each pair requested in front of its products; 16 / 4 heads of 64, 3000 tokens 102 / 107).  Two heads a workgroup are two wavefronts a SIMD, and
+// level: 32 / 8 heads, 4096 tokens 402 / 402.
 #include "fh_internal.h"
 
 typedef _Float16 fh_half;
@@ -89,7 +90,7 @@ __device__ __forceinline__ half8 ap_vt8(const fh_half *p, int row_stride) {
 }
 
 template <typename TQ, typename TKV, int D, bool SPLIT = false, int HW = 1, int KS = 1, int QW = 4>
-__global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_eu(QW == 4 && !(SPLIT && D == 128) ? 2 : 1, SPLIT && D == 128 ? 1 : 2))) void k_attn_prefill(const TQ *__restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_st,
+__global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_eu(QW == 4 && !(SPLIT && D == 128 && HW == 1) ? 2 : 1, SPLIT && D == 128 && HW == 1 ? 1 : 2))) void k_attn_prefill(const TQ *__restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_st,
                                                        const TKV *__restrict__ k, const TKV *__restrict__ v,
                                                        int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int hq, int hkv,
                                                        int sq, int skv, float scale, int causal, TQ *__restrict__ out) {
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
             }
             __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
         } else {
-            // three products an operand pair (hi.hi, lo.hi, hi.lo); pairs are requested four ahead
+            // three products an operand pair (hi.hi, lo.hi, hi.lo); pairs are requested four (two) ahead
             const fh_half *ap = sK + prow * KS_ + 8 * g;
             constexpr int NI = 2 * KSTEPS, AHEAD = D == 128 ? 4 : 2;
             half8 kh_[AHEAD], kl_[AHEAD];

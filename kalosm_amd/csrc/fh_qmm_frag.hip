@@ -80,7 +80,6 @@ __global__ __launch_bounds__(512) void k_frag_x(const void *__restrict__ xin, in
     uint8_t *dst = out + ((int64_t)(row >> 5) * kf) * 1024 + (row & 31) * 16;
     const int parts = (int)gridDim.y, span = ((k + parts - 1) / parts + 511) / 512 * 512, ns = k >> 5;
     const int from = (int)blockIdx.y * span, to = from + span < k ? from + span : k; // (whole 512s, so whole runs of 8 sums)
-#pragma unroll 2
     for (int at = from; at < to; at += 512) {
         const int c = at + (tid >> 3) * 8;
         float v[8];
@@ -623,7 +622,7 @@ bool fh_qmm_frag_supports(const fh_qmatrix *q) {
 }
 
 // Where the fragments pay for being written, against the tile kernels that decode inside the product (the rows and matrices that
-// fh_qmm_reg.hip takes are not asked about: of those up to 64, only k below 1024 or no multiple of 256 is left).  Both were timed for 13 - 64
+// fh_qmm_reg.hip takes are not asked about: of those up to 64, only k below 1024, above 16384 or no multiple of 256 is left).  Both were timed for 13 - 64
 // rows of 12 matrices and 129 - 3000 rows of 23, in every format; us, fragments / tiles, at the lines:
 //   Up to 64 rows a tile kernel takes the same time for any matrix whose tiles of 128 rows fit the device at once (32768 rows), the
 //     fragments as long as they are: Q4_K f32, 32 rows, 11008 x 4096 55 / 150, 32768 x 4096 145 / 158, 128256 x 4096 595 / 294;

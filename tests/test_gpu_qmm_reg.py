@@ -2,8 +2,8 @@
 dequantised weights.
 
 Bound: the operands are exact up to 2^-22 of each activation; products are added in f32, sixteen times 2 or 3 in a chain within a 256,
-then k / 256 of those (each with its offsets, which cancel most of it; the wide products of
-formats with a scale per 32 k / 32 of those), and rounding errors (2^-24 each, of either sign) grow with the
+then up to eight of those (each with its offsets, which cancel most of it) and the sums of eight; the wide products up to k / 256 of them,
+or, with a scale per 32, half of k / 32 (f32 rows: all).  Rounding errors (2^-24 each, of either sign) grow with the
 root of their number: 1e-6 of the root of the sum of the squared products (the result's root mean square where there are many of
 them; one result alone may be next to nothing by cancellation) covers k = 16384.  The largest single difference is held to ten
 times that (ten standard deviations)."""
@@ -27,20 +27,27 @@ def operands(dev, ty, m, n, k, act, x=None):
     return q, Tensor.from_slice(dev, bits, dtype="bf16"), synth.from_bf16_bits(bits), raw
 
 
-def run(dev, q, xt, option):
+def run(dev, q, xt, option, cut=0):
     out = Tensor.filled_bytes(dev, (xt.shape[0], q.shape()[0]), 0xFF)  # poisoned: unwritten elements show as NaN
     dev.set_option("matmul_kernel", option)
+    dev.set_option("matmul_cut", cut)
     try:
         return xt.q_mat_mul(q, out=out).as_slice()
     finally:
         dev.set_option("matmul_kernel", 0)
+        dev.set_option("matmul_cut", 0)
+
+
+def cut_of(mt, kw, parts):
+    """Row tiles of activations a workgroup, groups of its wavefronts along k, workgroups along k."""
+    return mt + 16 * kw + 256 * parts
 
 
 @pytest.mark.parametrize("act", ["f32", "bf16"])
 @pytest.mark.parametrize("ty", TYPES, ids=lambda t: synth.TYPE_NAMES[t])
 @pytest.mark.parametrize("m,n,k,option", [
-    (1, 1, 256, 16),       # one row, one output, one 256: most wavefronts have nothing of k
-    (17, 33, 1280, 16),    # five 256s over four groups of wavefronts; a second row tile of one row
+    (1, 1, 256, 16),       # one row, one output, one 256
+    (17, 33, 1280, 16),    # five 256s in parts of their own (how k is shared out otherwise: test_cuts); a second row tile of one row
     (48, 272, 2304, 16),   # three row tiles; nine 256s
     (65, 96, 4096, 16),    # five row tiles in two workgroups of three
     (130, 520, 1024, 16),  # nine row tiles in three workgroups
@@ -55,6 +62,23 @@ def run(dev, q, xt, option):
 def test_product(dev, oracle, ty, act, m, n, k, option):
     q, xt, x, raw = operands(dev, ty, m, n, k, act)
     got = run(dev, q, xt, option).astype(np.float64)
+    x, w = x.astype(np.float64), oracle.dequantize(ty, raw).reshape(n, k).astype(np.float64)
+    want, rms = x @ w.T, np.sqrt(np.mean((x * x) @ (w * w).T))
+    assert np.isfinite(got).all()
+    assert np.sqrt(np.mean((got - want) ** 2)) <= 1e-6 * rms
+    assert np.abs(got - want).max() <= 1e-5 * rms
+
+
+@pytest.mark.parametrize("act", ["f32", "bf16"])
+@pytest.mark.parametrize("ty", TYPES, ids=lambda t: synth.TYPE_NAMES[t])
+@pytest.mark.parametrize("mt", [1, 2, 3, 4])
+@pytest.mark.parametrize("kw,parts", [(1, 1), (1, 3), (2, 1), (2, 3), (4, 1), (4, 3)])
+def test_cuts(dev, oracle, ty, act, mt, kw, parts):
+    """Every way a product can be cut: 13 256s over one to twelve groups (most of them uneven, so that some multiply a 256 with a scale of
+    zero), a row tile past the last whole workgroup, weight rows past the last tile of one."""
+    m, n, k = 16 * mt + 3, 136, 256 * 13
+    q, xt, x, raw = operands(dev, ty, m, n, k, act)
+    got = run(dev, q, xt, 16, cut_of(mt, kw, parts)).astype(np.float64)
     x, w = x.astype(np.float64), oracle.dequantize(ty, raw).reshape(n, k).astype(np.float64)
     want, rms = x @ w.T, np.sqrt(np.mean((x * x) @ (w * w).T))
     assert np.isfinite(got).all()
@@ -83,20 +107,21 @@ def test_rule(dev, ty, act, m, n, k, taken):
     assert np.array_equal(run(dev, q, xt, 0).view(np.uint32), run(dev, q, xt, 14).view(np.uint32)) == taken
 
 
-@pytest.mark.parametrize("option", [15, 16])
-@pytest.mark.parametrize("ty", [synth.Q4_K, synth.Q6_K, synth.Q8_0], ids=lambda t: synth.TYPE_NAMES[t])
-def test_rows_are_independent(dev, ty, option):
+@pytest.mark.parametrize("option,cut", [(15, 0), (16, 0), (16, cut_of(3, 4, 1)), (16, cut_of(2, 2, 2))], ids=["wide", "model", "k over 4", "k over 2 x 2"])
+@pytest.mark.parametrize("ty,m", [(synth.Q4_K, 40), (synth.Q6_K, 40), (synth.Q8_0, 40), (synth.Q5_0, 12), (synth.Q5_K, 12)],
+                         ids=lambda t: synth.TYPE_NAMES.get(t, t))
+def test_rows_are_independent(dev, ty, m, option, cut):
     """Zeros stay zero, a power of two passes through exactly, and an infinity or a NaN stays in its row - also where a group of
-    wavefronts has fewer 256s than others (five over four)."""
-    m, n, k = 40, 96, 1280
+    wavefronts has fewer 256s than others (five over four), and with a power of two per 32 (12 rows of the 5-bit formats)."""
+    n, k = 96, 1280
     x = synth.random_activation(m, k, seed=5)
     q, xt, _, _ = operands(dev, ty, m, n, k, "f32", x.copy())
-    base = run(dev, q, xt, option)
+    base = run(dev, q, xt, option, cut)
     x[3] = 0.0
     x[4] *= np.float32(2.0 ** 20)
     x[5, 7] = np.inf
     x[6, 9] = np.nan
-    got = run(dev, q, Tensor.from_slice(dev, x), option)
+    got = run(dev, q, Tensor.from_slice(dev, x), option, cut)
     assert not got[3].any()
     assert np.array_equal(got[4], base[4] * np.float32(2.0 ** 20))
     assert not np.isfinite(got[5]).any() and np.isnan(got[6]).all()
@@ -166,25 +191,20 @@ def long_sum(dev, ty, option, cut, chunks):
         raw[..., 0:2] = np.array([1.0], np.float16).view(np.uint8)
         raw[..., 2] = 1
     q = QMatrix.from_raw_bytes(dev, (16, 256 * chunks), raw.reshape(-1), ty)
-    xt = Tensor.from_slice(dev, synth.to_bf16_bits(x), dtype="bf16")
-    dev.set_option("matmul_cut", cut)
-    try:
-        return run(dev, q, xt, option).astype(np.float64) - 2.0 ** 24
-    finally:
-        dev.set_option("matmul_cut", 0)
+    return run(dev, q, Tensor.from_slice(dev, synth.to_bf16_bits(x), dtype="bf16"), option, cut).astype(np.float64) - 2.0 ** 24
 
 
 @pytest.mark.parametrize("ty", [synth.Q8_0, synth.Q6_K], ids=lambda t: synth.TYPE_NAMES[t])
 def test_partial_planes_are_added_in_pairs(dev, ty):
     """16 planes of one 256 each: one pair loses its 1, the 14 others arrive.  (One after the other: all 15 are lost.)"""
-    assert (long_sum(dev, ty, 16, 1 + 16 * 1 + 256 * 16, 16) == 14).all()
+    assert (long_sum(dev, ty, 16, cut_of(1, 1, 16), 16) == 14).all()
 
 
 @pytest.mark.parametrize("kw,kept", [(1, 56), (4, 60)])
 def test_no_sum_is_long(dev, kw, kept):
     """64 times 256, scale per 256: the ones beside 2^24 in its first eight are lost, the 56 others arrive; of four groups of 16, which add up
     in fours, all but three.  One sum along k loses all 63, four of them 15."""
-    assert (long_sum(dev, synth.Q6_K, 16, 1 + 16 * kw + 256 * 1, 64) == kept).all()
+    assert (long_sum(dev, synth.Q6_K, 16, cut_of(1, kw, 1), 64) == kept).all()
 
 
 @pytest.mark.parametrize("chunks,kept", [(1, 0), (2, 0), (8, 4), (9, 4), (32, 16)])
@@ -209,7 +229,7 @@ def test_f32_products_that_others_part(dev, m, n, k, parted):
 
 @pytest.mark.parametrize("ty", [synth.Q5_0, synth.Q5_K], ids=lambda t: synth.TYPE_NAMES[t])
 @pytest.mark.parametrize("m", [5, 12])
-@pytest.mark.parametrize("cut", [0, 1 + 16 * 1 + 256 * 1, 1 + 16 * 2 + 256 * 2, 1 + 16 * 4 + 256 * 1])
+@pytest.mark.parametrize("cut", [0, cut_of(1, 1, 1), cut_of(1, 2, 2), cut_of(1, 4, 1)])
 def test_small_values_beside_large_ones(dev, oracle, ty, m, cut):
     """5 to 12 rows of the 5-bit formats keep every bit of a group of 32 whatever stands in the others, as the kernel for one row
     does: each 256 has a group of values 2^30 times the others', which meet weights of zero.  (Within a row's range of f16 hi + lo the others
@@ -224,11 +244,7 @@ def test_small_values_beside_large_ones(dev, oracle, ty, m, cut):
     x = synth.random_activation(m, k, seed=m)
     x.reshape(m, k // 256, 8, 32)[:, :, 3] *= np.float32(2.0 ** 30)
     q = QMatrix.from_raw_bytes(dev, (n, k), raw.reshape(-1), ty)
-    dev.set_option("matmul_cut", cut)
-    try:
-        got = run(dev, q, Tensor.from_slice(dev, x), 0 if not cut else 16).astype(np.float64)
-    finally:
-        dev.set_option("matmul_cut", 0)
+    got = run(dev, q, Tensor.from_slice(dev, x), 16 if cut else 0, cut).astype(np.float64)
     w = oracle.dequantize(ty, raw.reshape(-1)).reshape(n, k).astype(np.float64)
     assert not w.reshape(n, k // 256, 8, 32)[:, :, 3].any()
     want = x.astype(np.float64) @ w.T

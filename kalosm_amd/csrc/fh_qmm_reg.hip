@@ -1207,9 +1207,10 @@ static int reg_way(const fh_qmatrix *q, int x_is_bf16, int m, bool whole) { // w
     if (!narrow && !wide) return REG_NONE;
     const double narrow_us = reg_cut(q, x_is_bf16, m, whole).us, us = wide_us(q, x_is_bf16, m);
     wide = !parted && (wide || (can && us < 0.97 * narrow_us));
-    // (SwiGLU was asked about as a product first)
-    if (!whole && m > FH_SHORT_PROMPT && (wide ? us : narrow_us) > 0.97 * (fh_qmm_frag_pays(q, x_is_bf16, m) ? fh_qmm_frag_us(q, x_is_bf16, m, nullptr) : fh_qmm_tile_us(q, x_is_bf16, m)))
-        return REG_NONE;
+    if (!whole && m > FH_SHORT_PROMPT) { // (SwiGLU was asked about as a product first)
+        const double other = fh_qmm_frag_pays(q, x_is_bf16, m) ? fh_qmm_frag_us(q, x_is_bf16, m, nullptr) : fh_qmm_tile_us(q, x_is_bf16, m);
+        if ((wide ? us : narrow_us) > (wide && q->type == FH_Q4_K ? 1.0 : 0.97) * other) return REG_NONE; // (what is next to level stays with the others)
+    }
     return wide ? REG_WIDE : REG_NARROW;
 }
 bool fh_qmm_reg_pays(const fh_qmatrix *q, int x_is_bf16, int m) { return reg_way(q, x_is_bf16, m, false) != REG_NONE; }

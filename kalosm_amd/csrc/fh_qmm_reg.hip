@@ -12,11 +12,12 @@
 //   Q8_0, Q4_0, Q5_0   the code, d per 32, a sum of its own per 256
 // Activations: a power of two per row, hi + lo (f32 input) or one exact term (bf16).  With f32 input Q6_K drops lo * lo.
 //
-// What bounds it: 17 rows of 14336 x 4096 in Q4_K take 21 us (59 on fragments), 64 rows 32 (67), 192 rows 70 (102), 512 rows 140
-// (153); in Q6_K 26 (118), 38 (124), 90 (139), 180 (247); bf16 rows of Q8_0: one row 16 (140), 33 rows 22 (74), 512 rows 110 (120).  Up
+// What bounds it: 17 rows of 14336 x 4096 in Q4_K take 22 us (63 on fragments), 64 rows 34 (67), 192 rows 71 (103), 512 rows 137
+// (152); in Q6_K 29 (118), 40 (124), 92 (136), 185 (244); bf16 rows of Q8_0: one row 17 (140), 33 rows 23 (67), 512 rows 104 (114).  Up
 // to 64 rows that is three launches and, in the middle one, two or three memory round trips; from some hundred rows on the matrix
 // cores and the vector ALU beside them (a 16 x 16 x 32 product hides two vector instructions, a block of 32 has 2.2 a product).
-// Against 64 bits: 1.6e-7 (Q4_K), 1.1e-7 (Q8_0), 1.7e-7 (Q6_K); the tiles 2.6e-7 - 7e-7, the fragments 1.3e-7 - 1.8e-7.
+// Against 64 bits, 17 - 512 rows of that matrix: 1.6e-7 - 1.7e-7 (Q4_K, Q5_K), 1.1e-7 (Q8_0, 64 rows), 1.7e-7 (Q6_K); the fragments 1.6e-7 -
+// 1.7e-7 and, Q8_0 and Q5_0, 1.3e-7 - 1.6e-7, the tiles that few rows had in Q6_K 5e-7 - 7e-7, one bf16 row 0.8e-7 - 1.1e-7 for 5.6e-7 - 6.3e-7.
 #include "fh_blocks.h"
 #include "fh_qmm_frag.h"
 
@@ -794,7 +795,7 @@ struct WideW {
 //   products are the 32 x 32 x 16 ones, which leave it more room (16 of their half-size and 128 vector instructions of two wavefronts
 //   take 307 ns, as 16 x 16 x 32 ones 370);
 //   the two workgroups drift apart, and one decodes while the other multiplies: as one of eight wavefronts, in step at every barrier, 2048
-//   rows of 14336 x 4096 took 393 us in Q8_0 (333 so), 332 in Q4_K (289), bf16;
+//   rows of 14336 x 4096 took 393 us in Q8_0 (333 so, k in one chain; 344 in two halves), 332 in Q4_K (289), bf16;
 //   the tiles that run together on a die are eight weight tiles by eight of activations (as two by 32: 358 and 304).
 template <int T, int NX, int MX>
 struct WideTile {
@@ -1174,9 +1175,10 @@ static double wide_us(const fh_qmatrix *q, int x_is_bf16, int m) {
 }
 
 // Which of the two, if any.  Where few rows take k_qmm_reg: the one that is quicker by the models.  Above, k_qmm_wide where its
-// tiles keep the device busy (us, wide / others: Q4_K bf16, 2048 rows, 14336 x 4096 276 / 315, 8192 x 3072 130 / 135, 5632 x 2048 74 / 89;
-// Q8_0 bf16 317 / 363, 148 / 165, 83 / 107; Q6_K bf16 420 / 478, 192 / 213, 105 / 131; Q4_K f32, 1024 rows, 28672 x 4096 437 / 495), with f32 rows only for
-// matrices of 8192 rows and more (4096 x 4096, 2048 rows: 146 / 143) and not for Q6_K (2048 rows, 8192 x 3072 298 / 278).  k to 8192 only, and not where
+// tiles keep the device busy (us, wide / fragments / tiles: Q4_K bf16, 2048 rows, 14336 x 4096 300 / 333 / 474, 8192 x 3072 141 / 141 / 208, 5632 x 2048
+// 78 / 90 / 132; Q8_0 bf16 356 / 388 / 436, 164 / 159 / 175, 89 / 100 / 121; Q6_K bf16 470 / 466 / 526, 208 / 184 / 224, 108 / 114 / 149, both on the
+// tiles otherwise; Q4_K f32, 1024 rows, 28672 x 4096 490 / 525 / 702), with f32 rows only for
+// matrices of 8192 rows and more (4096 x 4096, 2048 rows: 146 / 143) and not for Q6_K (2048 rows, 8192 x 3072 313 / 266).  k to 8192 only, and not where
 // the tiles would part all of it (qmm_launch_t): its sums are long.  k_qmm_reg, whose 256s add up in fours or by themselves, takes what the others would
 // part (reg_parted; 750 rows of 14336 x 8192, Q8_0, against 64 bits 1.4e-7, fragments 2.2e-7, wide 3.0e-7; 402, 462 and 407 us).  bf16 rows of the formats whose
 // tiles leave the device idle for narrow matrices stay on k_qmm_reg (Q8_0, 1536 rows, 1024 x 4096 45 / 86, 3072 x 3072 85 / 140).

@@ -17,7 +17,13 @@
 // group, so a SIMD runs one wavefront's chain of a step instead of two.
 // What bounds the loop (measured per stage): the first product is matrix-core bound, the softmax vector-ALU bound
 // (both wavefronts of a SIMD are in it together) and the second product bound by the transposing LDS loads, which
-// run at half the rate of plain 16-byte loads.
+// run at half the rate of plain 16-byte loads.  So the softmax is kept to what a score needs (140 vector instructions for a wavefront's 2048; with
+// address arithmetic for the requests, cleared accumulators and output rescaled in most tiles they were 310): a request is a buffer load from a
+// descriptor that moves with the tile, the denominator is added up in pairs from the rounded weights, and split operands, whose weights
+// lose nothing by it, move their reference only where a maximum is 2^8 above it.  Rows of V are 64 bytes apart in the banks, so that the 16
+// lanes of a transposing load cover them once.  Heads that share a workgroup (four wavefronts each) are half a step apart, one in the softmax while
+// the other multiplies.  f16, 32 / 8 heads of 128, causal, before and after: 1024 tokens 25.3 / 23.7 us, 2048 53.4 / 50.8, 4096 166 / 151, 8192
+// 616 / 558 (985 TFLOP/s); f32 2048 129 / 125, 4096 400 / 350.
 // Both products are computed TRANSPOSED with
 // v_mfma_f32_32x32x16_f16 so that a lane always stands for ONE query (the accumulator column):
 //   S^T (keys x queries) = K . Q^T      A = K rows, B = Q^T kept in registers for the whole kernel
@@ -33,11 +39,11 @@
 // hi.hi + lo.hi + hi.lo, so the result keeps f32 accuracy at three times the matrix-core work.  Its tiles fill the LDS: one workgroup a
 // compute unit, for head_dim 128 and one head a workgroup one wavefront a SIMD, which nothing covers while it waits for an operand - so pairs are
 // requested four ahead (head_dim 64, two wavefronts: two) and the wavefront may have all registers (32 / 8 heads, 2048 tokens, causal: 152 us,
-// 190 with each pair requested in front of its products; 16 / 4 heads of 64, 3000 tokens 102 / 107).  Two heads a workgroup are two wavefronts a SIMD, and
-// level: 32 / 8 heads, 4096 tokens 402 / 402.
+// 190 with each pair requested in front of its products; 16 / 4 heads of 64, 3000 tokens 102 / 107).
 #include "fh_internal.h"
 
 typedef _Float16 fh_half;
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
@@ -49,6 +55,11 @@ __device__ __forceinline__ void ap_load8(const float *p, fh_half *o) {
 __device__ __forceinline__ void ap_load8(const fh_half *p, fh_half *o) {
     const uint4 r = *(const uint4 *)p;
     __builtin_memcpy(o, &r, 16);
+}
+// 16 bytes of a buffer, zeros past its end
+__device__ __forceinline__ uint4 ap_buffer16(__amdgpu_buffer_rsrc_t b, int offset) {
+    const auto u = __builtin_amdgcn_raw_buffer_load_b128(b, offset, 0, 0);
+    return make_uint4(u[0], u[1], u[2], u[3]);
 }
 __device__ __forceinline__ float ap_swap32_max(float v) {
     const uint32_t u = __float_as_uint(v);
@@ -94,16 +105,20 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
                                                        const TKV *__restrict__ k, const TKV *__restrict__ v,
                                                        int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int hq, int hkv,
                                                        int sq, int skv, float scale, int causal, TQ *__restrict__ out) {
-    constexpr int BN = 64, KS_ = D + 8, VS = D + 16, DT = D / 32, KSTEPS = D / 16, CH = D / 8; // CH: 8-element chunks per row
+    constexpr int BN = 64, KS_ = D + 8, VS = D + 32, DT = D / 32, KSTEPS = D / 16, CH = D / 8; // CH: 8-element chunks per row
     constexpr int NP = SPLIT ? 2 : 1; // operand planes: hi (, lo)
     static_assert(HW * KS <= 2 && !(SPLIT && KS == 2), "eight wavefronts at most; split operands leave no room for two tiles");
     static_assert(QW == 4 || (QW == 2 && HW == 1 && KS == 2), "query blocks of 128 rows, or of 64 with two key groups");
     constexpr int QB = 32 * QW; // query rows of a workgroup: QW wavefronts of 32
     constexpr int NTH = 64 * QW * HW * KS, KBUF = NP * BN * KS_, VBUF = NP * BN * VS, TILE = KBUF + VBUF; // halfs per staged tile
     extern __shared__ __attribute__((aligned(16))) fh_half ap_lds[]; // [2 buffers][K planes | V planes]
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = lane & 31, g = lane >> 5;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31, g = lane >> 5;
     const int kset = KS == 2 ? wave / QW : 0; // which key tiles of a step this wavefront multiplies
-    const int h = (int)blockIdx.x * HW + (HW == 2 ? wave >> 2 : 0), bi = blockIdx.z, kh = h / (hq / hkv);
+    // The wavefronts of two heads are half a step apart: those of one are in the first product and the softmax while those of the other are in the
+    // second product.
+    constexpr bool APART = HW == 2;
+    const int head = wave >> 2;
+    const int h = (int)blockIdx.x * HW + (HW == 2 ? wave >> 2 : 0), bi = blockIdx.z, kh = (int)blockIdx.x * HW / (hq / hkv);
     // causal: the last query blocks see the most keys; with the block index on the slow grid axis ALL heads of the
     // longest block are dispatched first and the short blocks fill the tail
     const int qb0 = (causal ? (int)(gridDim.y - 1 - blockIdx.y) : (int)blockIdx.y) * QB;
@@ -149,24 +164,39 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
     constexpr int NCH = KS * BN * CH / NTH;
     uint4 kreg[SPLIT ? 1 : NCH], vreg[SPLIT ? 1 : NCH];
     float4 kraw[SPLIT ? 2 * NCH : 1], vraw[SPLIT ? 2 * NCH : 1];
+    // Requested through buffer descriptors that begin at the step's first key, so that a request is one instruction; rows past the last key
+    // are zeros (their scores are masked and their P is 0).
+    const int row_bytes = (int)(kv_st * sizeof(TKV));
+    int piece[NCH]; // bytes from the step's first key
+#pragma unroll
+    for (int i = 0; i < NCH; i++) {
+        const int c = tid + NTH * i;
+        piece[i] = c / CH * row_bytes + 8 * (c % CH) * (int)sizeof(TKV); // key 0 .. KS * BN - 1: the KS tiles of a step
+    }
     auto fetch = [&](int t0) {
+        const int64_t end = (int64_t)(skv - t0 - 1) * row_bytes + D * (int)sizeof(TKV);
+        const int bytes = end < 0x7FFFFFFF ? (int)end : 0x7FFFFFFF;
+        const auto bk = __builtin_amdgcn_make_buffer_rsrc((void *)(kb + t0 * kv_st), 0, bytes, 0x00027000);
+        const auto bv = __builtin_amdgcn_make_buffer_rsrc((void *)(vb + t0 * kv_st), 0, bytes, 0x00027000);
 #pragma unroll
         for (int i = 0; i < NCH; i++) {
-            const int c = tid + NTH * i, key = c / CH, dc = c % CH; // key 0 .. KS * BN - 1: the KS tiles of a step
-            // rows past the end repeat the last one (no branch): their scores are masked and their P is 0
-            const int64_t row = (int64_t)(t0 + key < skv ? t0 + key : skv - 1) * kv_st + 8 * dc;
-            if constexpr (SPLIT) {
-                const float *kp = (const float *)kb + row, *vp = (const float *)vb + row;
-                kraw[2 * i] = *(const float4 *)kp;
-                kraw[2 * i + 1] = *(const float4 *)(kp + 4);
-                vraw[2 * i] = *(const float4 *)vp;
-                vraw[2 * i + 1] = *(const float4 *)(vp + 4);
+            if constexpr (sizeof(TKV) == 2) {
+                kreg[i] = ap_buffer16(bk, piece[i]);
+                vreg[i] = ap_buffer16(bv, piece[i]);
             } else {
-                fh_half t[8];
-                ap_load8(kb + row, t);
-                __builtin_memcpy(&kreg[i], t, 16);
-                ap_load8(vb + row, t);
-                __builtin_memcpy(&vreg[i], t, 16);
+                const uint4 u[4] = {ap_buffer16(bk, piece[i]), ap_buffer16(bk, piece[i] + 16), ap_buffer16(bv, piece[i]), ap_buffer16(bv, piece[i] + 16)};
+                if constexpr (SPLIT) {
+                    __builtin_memcpy(&kraw[2 * i], &u[0], 32);
+                    __builtin_memcpy(&vraw[2 * i], &u[2], 32);
+                } else {
+                    float x[16];
+                    __builtin_memcpy(x, u, 64);
+                    fh_half t[16];
+#pragma unroll
+                    for (int e = 0; e < 16; e++) t[e] = (fh_half)x[e];
+                    __builtin_memcpy(&kreg[i], t, 16);
+                    __builtin_memcpy(&vreg[i], t + 8, 16);
+                }
             }
         }
     };
@@ -215,6 +245,12 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
         if (KS * BN < kend) fetch(KS * BN);
     }
     __syncthreads();
+    auto bar = [&]() { // (requests for the tile after next stay on their way)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (APART && head == 1) bar();
 
     const float ninf = -INFINITY;
     for (int ts = 0, it = 0; ts < kend; ts += KS * BN, it++) { // a step: KS tiles, one per group of four wavefronts
@@ -223,9 +259,8 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
         const int lim_t = (KS == 1 || t0 < kend) ? lim : -1;
         const fh_half *sK = ap_lds + ((it & 1) * KS + kset) * TILE, *sV = sK + KBUF;
         // ---- S^T = K . Q^T for the two 32-key halves of the tile
+        const floatx16 zero = {0.f};
         floatx16 st[2];
-#pragma unroll
-        for (int r = 0; r < 16; r++) st[0][r] = st[1][r] = 0.f;
         if constexpr (!SPLIT) {
             // product i: key half i % 2, d step i / 2; the K operands are requested eight products ahead
             const fh_half *ap = sK + prow * KS_ + 8 * g;
@@ -235,7 +270,7 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
             for (int i = 0; i < AHEAD; i++) ka[i] = *(const half8 *)(ap + (i & 1) * 32 * KS_ + 16 * (i >> 1));
 #pragma unroll
             for (int i = 0; i < NI; i++) {
-                st[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[i % AHEAD], qf[i >> 1], st[i & 1], 0, 0, 0);
+                st[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[i % AHEAD], qf[i >> 1], i < 2 ? zero : st[i & 1], 0, 0, 0);
                 if (i + AHEAD < NI) ka[i % AHEAD] = *(const half8 *)(ap + (i & 1) * 32 * KS_ + 16 * ((i + AHEAD) >> 1));
             }
             __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
@@ -258,7 +293,7 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
             for (int i = 0; i < AHEAD; i++) read(i);
 #pragma unroll
             for (int i = 0; i < NI; i++) {
-                st[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh_[i % AHEAD], qf[i >> 1], st[i & 1], 0, 0, 0);
+                st[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh_[i % AHEAD], qf[i >> 1], i < 2 ? zero : st[i & 1], 0, 0, 0);
                 st[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl_[i % AHEAD], qf[i >> 1], st[i & 1], 0, 0, 0);
                 st[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh_[i % AHEAD], ql[i >> 1], st[i & 1], 0, 0, 0);
                 if (i + AHEAD < NI) read(i + AHEAD);
@@ -276,8 +311,11 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
         // (the scheduler may not mix the stages: the operands prefetched for one product and the tile in flight would
         // otherwise be live together with the scores)
         __builtin_amdgcn_sched_barrier(0);
-        if (ts + KS * BN < kend) stash((it + 1) & 1);
-        if (ts + 2 * KS * BN < kend) fetch(ts + 2 * KS * BN);
+        auto next = [&]() {
+            if (ts + KS * BN < kend) stash((it + 1) & 1);
+            if (ts + 2 * KS * BN < kend) fetch(ts + 2 * KS * BN);
+        };
+        if (!APART || head == 1) next(); // (both heads in the same half step: neither has a wavefront in the other buffer then)
         __builtin_amdgcn_sched_barrier(0);
         // ---- mask, running max: register r of half kt is key t0 + 32 kt + 16 (r / 8) + 8 g + r % 8
         // Only a tile that reaches past some query's last visible key pays for the compares (one branch for the
@@ -301,10 +339,17 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
             for (int r = 0; r < 16; r++) mx = fmaxf(mx, st[kt][r]);
         // the scale (> 0) is applied inside the exponent: p = 2^(s * sc2 - m), one multiply-add per score
         mx = ap_swap32_max(mx) * sc2;
-        const float m_new = fmaxf(m_run, mx);
-        const bool dead = m_new == -INFINITY; // nothing visible yet (only queries past the end)
-        const float alpha = dead ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
-        const float m_sub = dead ? 0.f : -m_new; // dead rows: 2^(-inf - 0) = 0
+        // The reference of the exponents.  Split operands: it moves only where a maximum is more than 2^8 above it, so that the output is rescaled
+        // in the first tiles and then hardly ever.  (Weights rounded to f16: where one key has most of the weight that is 1, exact; against 64 bits
+        // 2048 tokens with scores of four times the usual spread 2.13e-4, with a reference of its own 2.25e-4.)
+        const bool move = __any(mx > m_run + (SPLIT ? 8.f : 0.f));
+        float alpha = 1.f;
+        if (move) {
+            const float m_new = fmaxf(m_run, mx);
+            alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new); // (nothing visible yet: only queries past the end)
+            m_run = m_new;
+        }
+        const float m_sub = m_run == -INFINITY ? 0.f : -m_run; // dead rows: 2^(-inf - 0) = 0
         float ps = 0.f;
         half8 pb[2][2], pl[SPLIT ? 2 : 1][2];
 #pragma unroll
@@ -315,18 +360,24 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
                     const float p = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + e], sc2, m_sub)); // arguments <= 0
-                    ps += p;
                     t[e] = (fh_half)p;
-                    if constexpr (SPLIT) tl[e] = (fh_half)(p - (float)t[e]);
+                    if constexpr (SPLIT) ps += p, tl[e] = (fh_half)(p - (float)t[e]);
                 }
+                if constexpr (!SPLIT) // the denominator is the sum of what is multiplied, so that their roundings go together
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2) ps = __builtin_amdgcn_fdot2(half2v{t[e], t[e + 1]}, half2v{(fh_half)1.f, (fh_half)1.f}, ps, false);
                 __builtin_memcpy(&pb[kt][s2], t, 16);
                 if constexpr (SPLIT) __builtin_memcpy(&pl[kt][s2], tl, 16);
             }
-        l_run = l_run * alpha + ap_swap32_sum(ps);
-        m_run = m_new;
-        // ---- O^T = O^T * alpha + V^T . P^T (once the maxima have settled no lane of the wavefront rescales)
+        l_run = l_run * alpha + ps; // (of this lane's keys)
+        // ---- O^T = O^T * alpha + V^T . P^T
         __builtin_amdgcn_sched_barrier(0);
-        if (__any(alpha != 1.f)) {
+        if (APART) {
+            bar();
+            if (head == 0) next();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (move) {
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
@@ -379,8 +430,11 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
             }
             __builtin_amdgcn_sched_group_barrier(0x008, 3 * AHEAD, 0);
         }
-        __syncthreads(); // tile t+1 is staged, and nobody reads this tile's buffer any more
+        if (APART) bar();
+        else __syncthreads(); // tile t+1 is staged, and nobody reads this tile's buffer any more
     }
+    if (APART && head == 0) bar(); // (as many barriers as the other)
+    l_run = ap_swap32_sum(l_run);
     if constexpr (KS == 2) {
         // ---- the second group hands its statistics and output over: [value][query wavefront][lane] floats in the
         // tile buffers (the barrier that ended the last step has passed: nobody reads them any more)
@@ -423,7 +477,7 @@ template <typename TQ, typename TKV, int D, bool SPLIT, int HW, int KS = 1, int 
 static fh_status ap_launch_k(fh_device *dev, const void *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void *k,
                              const void *v, int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int b, int hq, int hkv, int sq,
                              int skv, float scale, int causal, void *out) {
-    constexpr int LDS = 2 * KS * (SPLIT ? 2 : 1) * 64 * (D + 8 + D + 16) * 2; // two buffers of KS tiles (K and V planes), bytes
+    constexpr int LDS = 2 * KS * (SPLIT ? 2 : 1) * 64 * (D + 8 + D + 32) * 2; // two buffers of KS tiles (K and V planes), bytes
     static_assert(KS == 1 || LDS >= (2 + (D / 32) * 16) * 256 * 4, "the merge of the key groups reuses the tile buffers");
     static_assert(LDS <= 160 * 1024, "KV tiles exceed the LDS of a compute unit");
     auto kern = k_attn_prefill<TQ, TKV, D, SPLIT, HW, KS, QW>;
@@ -472,6 +526,7 @@ fh_status fh_attention_prefill_mfma(fh_device *dev, int q_dtype, int kv_dtype, c
     if ((d != 128 && d != 64) || hq % hkv || (mask_kind != FH_MASK_NONE && mask_kind != FH_MASK_CAUSAL)) return FH_ERR_UNSUPPORTED;
     if (q_st % 8 || q_sh % 8 || q_sb % 8 || kv_st % 8 || kv_sh % 8 || kv_sb % 8 || (sq + 127) / 128 > 65535 || b > 65535) return FH_ERR_UNSUPPORTED;
     if (mask_kind == FH_MASK_CAUSAL && skv < sq) return FH_ERR_UNSUPPORTED;
+    if (kv_st < 0 || kv_st >= 1 << 21) return FH_ERR_UNSUPPORTED; // a step's 128 rows lie within the 2^31 bytes of a buffer
     const int causal = mask_kind == FH_MASK_CAUSAL;
     if (q_dtype == FH_F16 && kv_dtype == FH_F16)
         return ap_launch<fh_half, fh_half>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, d, scale, causal, out);

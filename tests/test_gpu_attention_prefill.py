@@ -1,0 +1,73 @@
+"""Prompt attention on the matrix cores in every workgroup shape: ends of key tiles (rows past the last key are zeros from the buffer), the
+reference of the exponents that moves late or never, and weights below the normal f16 range, against 64 bits."""
+import numpy as np
+import pytest
+
+from kalosm_amd.fusor import MaskKind, Tensor
+
+pytestmark = pytest.mark.gpu
+
+
+def exact(q, k, v, scale, causal):
+    h, g, t, s = q.shape[1], k.shape[1], q.shape[2], k.shape[2]
+    q, k, v = (a[0].astype(np.float64) for a in (q, k, v))
+    z = q @ np.repeat(k, h // g, 0).transpose(0, 2, 1) * scale
+    if causal:
+        z[:, np.arange(s)[None] > np.arange(t)[:, None] + s - t] = -np.inf
+    e = np.exp(z - z.max(2, keepdims=True))
+    return (e / e.sum(2, keepdims=True)) @ np.repeat(v, h // g, 0)
+
+
+def run(dev, q, k, v, dtype, scale, causal, shape):
+    dev.set_option("attn_kernel", shape)
+    try:
+        qt, kt, vt = (Tensor.from_slice(dev, a, dtype) for a in (q, k, v))
+        return qt.flash_attention(kt, vt, scale, MaskKind.Causal if causal else None).as_slice()[0].astype(np.float64)
+    finally:
+        dev.set_option("attn_kernel", 0)
+
+
+def close(got, want, dtype, scores):
+    """f16: weights, values and outputs each rounded by at most 2^-11 of themselves, against the outputs' root mean square: weights of
+    a row add up to one, so their roundings move an output by less than 2^-11 of the largest value (4.5 of N(0, 1)).  f32: the operands keep 22
+    bits, a score of size `scores` and so its weight an error of scores * 2^-21."""
+    tol = 2.0 ** -11 * (4.5 + 2 * np.abs(want)) if dtype == "f16" else 4.5 * 2.0 ** -21 * (2 + scores)
+    assert np.isfinite(got).all() and (np.abs(got - want) <= tol).all(), np.abs(got - want).max()
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("shape", [0, 6, 7, 8, 9])
+@pytest.mark.parametrize("t,s,d,causal", [(33, 33, 128, True), (64, 64, 64, True), (129, 129, 128, True), (200, 331, 128, True), (257, 257, 64, False),
+                                          (40, 127, 128, False), (383, 383, 128, True)])
+def test_every_shape_at_the_ends_of_its_tiles(dev, dtype, shape, t, s, d, causal):
+    rng = np.random.default_rng(t * 1000 + s)
+    q, k, v = (rng.standard_normal((1, n, m, d)).astype(np.float16 if dtype == "f16" else np.float32) for n, m in ((4, t), (2, s), (2, s)))
+    want = exact(q, k, v, d ** -0.5, causal)
+    close(run(dev, q, k, v, dtype, d ** -0.5, causal, shape), want, dtype, 6)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("shape", [6, 7, 8, 9])
+@pytest.mark.parametrize("steps", [[0.0, 4.0, 11.0, 11.5], [9.0, 0.0, 0.0, -3.0], [0.0, 7.0, 14.0, 21.0, 28.0, 35.0]])
+def test_reference_of_the_exponents(dev, dtype, shape, steps):
+    """A maximum that grows by less, by just less and by more than 2^8 (in powers of two) from one tile of keys to the next, or falls; far below it
+    are thousands of weights of 2^-17, which are subnormal in f16 and still make up a part of the denominator."""
+    rng = np.random.default_rng(len(steps))
+    d, tiles = 128, len(steps)
+    s = 128 * tiles + 3000
+    q = np.zeros((1, 4, 70, d), np.float32)
+    q[..., 0] = 1.0
+    k = np.zeros((1, 2, s, d), np.float32)
+    top = max(steps)
+    k[0, :, :, 0] = top - 17
+    for i, x in enumerate(steps):
+        k[0, :, 128 * i + 64, 0] = x
+    k[0, :, :, 0] = np.round(k[0, :, :, 0] * np.log(2.0) * 64) / 64  # exact in f16
+    v = (1 + 0.25 * rng.standard_normal((1, 2, s, d))).astype(np.float32)
+    if dtype == "f16":
+        q, k, v = (a.astype(np.float16) for a in (q, k, v))
+    want = exact(q, k, v, 1.0, False)
+    got = run(dev, q, k, v, dtype, 1.0, False, shape)
+    # subnormal weights, and what is left of them for the second operand of f32, are multiples of 2^-24: each is off by up to 2^-25, s of them
+    tol = (2.0 ** -10 * np.abs(want).max() if dtype == "f16" else 2.0 ** -20 * (2 + top)) + s * 2.0 ** -25
+    assert np.abs(got - want).max() <= tol, np.abs(got - want).max()

@@ -40,9 +40,8 @@
 // compute unit, for head_dim 128 and one head a workgroup one wavefront a SIMD, which nothing covers while it waits for an operand - so pairs are
 // requested four ahead (head_dim 64, two wavefronts: two) and the wavefront may have all registers (32 / 8 heads, 2048 tokens, causal: 152 us,
 // 190 with each pair requested in front of its products; 16 / 4 heads of 64, 3000 tokens 102 / 107).
-#include "fh_internal.h"
+#include "fh_blocks.h"
 
-typedef _Float16 fh_half;
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -98,6 +97,42 @@ __device__ __forceinline__ half8 ap_vt8(const fh_half *p, int row_stride) {
     __builtin_memcpy(&r, &a, 8);
     __builtin_memcpy((char *)&r + 8, &b, 8);
     return r;
+}
+
+// The second group of wavefronts hands its statistics and output over: [value][query wavefront][lane] floats in the tile buffers (the barrier
+// that ended the last step has passed: nobody reads them any more).
+template <int D, int QW>
+__device__ __forceinline__ void ap_merge(float *sm, int wave, int lane, int kset, float &m_run, float &l_run, floatx16 (&acc)[D / 32]) {
+    constexpr int NQ = 64 * QW, DT = D / 32;
+    const int slot = (wave % QW) * 64 + lane;
+    if (kset == 1) {
+        sm[slot] = m_run;
+        sm[NQ + slot] = l_run;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) sm[(2 + dt * 16 + r) * NQ + slot] = acc[dt][r];
+    }
+    __syncthreads();
+    if (kset == 1) return;
+    const float m1 = sm[slot], l1 = sm[NQ + slot];
+    const float mm = fmaxf(m_run, m1), ref = mm == -INFINITY ? 0.f : mm;
+    const float f0 = __builtin_amdgcn_exp2f(m_run - ref), f1 = __builtin_amdgcn_exp2f(m1 - ref);
+    l_run = l_run * f0 + l1 * f1;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[dt][r] = acc[dt][r] * f0 + sm[(2 + dt * 16 + r) * NQ + slot] * f1;
+}
+// lane = query, register r of d-tile dt is d = 32 dt + 8 (r / 4) + 4 g + r % 4
+template <int D, typename TQ>
+__device__ __forceinline__ void ap_store(TQ *op, int g, float inv, const floatx16 (&acc)[D / 32]) {
+#pragma unroll
+    for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; r4++)
+            ap_store4(op + 32 * dt + 8 * r4 + 4 * g, acc[dt][4 * r4] * inv, acc[dt][4 * r4 + 1] * inv, acc[dt][4 * r4 + 2] * inv,
+                      acc[dt][4 * r4 + 3] * inv);
 }
 
 template <typename TQ, typename TKV, int D, bool SPLIT = false, int HW = 1, int KS = 1, int QW = 4>
@@ -436,41 +471,202 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
     if (APART && head == 0) bar(); // (as many barriers as the other)
     l_run = ap_swap32_sum(l_run);
     if constexpr (KS == 2) {
-        // ---- the second group hands its statistics and output over: [value][query wavefront][lane] floats in the
-        // tile buffers (the barrier that ended the last step has passed: nobody reads them any more)
-        float *sm = (float *)ap_lds;
-        constexpr int NQ = 64 * QW;
-        const int slot = (wave % QW) * 64 + lane;
-        if (kset == 1) {
-            sm[slot] = m_run;
-            sm[NQ + slot] = l_run;
+        ap_merge<D, QW>((float *)ap_lds, wave, lane, kset, m_run, l_run, acc);
+        if (kset == 1) return;
+    }
+    if (qi < sq) ap_store<D>(out + (((int64_t)bi * hq + h) * sq + qi) * D, g, 1.0f / l_run, acc);
+}
+
+// f16 keys and values, one head a workgroup (KS as above).  The first product of the next tile and the softmax of this one are one stretch of code,
+// so that the matrix cores work beside the vector ALU; K is a tile ahead of V for it.  Two sets of scores leave no registers for tiles on their way:
+// those go straight into LDS, in rows without padding whose 16-byte pieces are swapped on the memory side (K: 16 rows' pieces of one number, V:
+// 4 rows' 64 bytes cover the banks once).  What is left is the chain of a step in one wavefront (with the two key groups half a step apart, one in
+// the softmax and one in the second product, it is longer: 2048 tokens 56 us).  Before and after, causal, us: 8 heads of 64, 3000 tokens 34.0 / 31.0;
+// 16 / 4 of 64, 777 12.1 / 12.0; 32 / 8 of 128, 2048 51.5 / 50.6, 3000 101 / 97.
+template <typename TQ, int D, int KS>
+__global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attn_ahead(
+    const TQ *__restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_st, const fh_half *__restrict__ k, const fh_half *__restrict__ v, int64_t kv_sb,
+    int64_t kv_sh, int64_t kv_st, int hq, int hkv, int sq, int skv, float scale, int causal, TQ *__restrict__ out) {
+    constexpr int BN = 64, DT = D / 32, KSTEPS = D / 16, CH = D / 8, TILE = BN * D, NW = 4 * KS, NP = TILE * KS * 2 / 1024 / NW; // NP: 1 KB pieces of K a wavefront
+    extern __shared__ __attribute__((aligned(16))) fh_half ap_lds[]; // [2 buffers][KS tiles of K, KS of V]
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31, g = lane >> 5;
+    const int kset = KS == 2 ? wave >> 2 : 0;
+    const int h = (int)blockIdx.x, bi = blockIdx.z, kh = h / (hq / hkv);
+    const int qb0 = (causal ? (int)(gridDim.y - 1 - blockIdx.y) : (int)blockIdx.y) * 128;
+    const int qi = qb0 + (wave & 3) * 32 + li, off = skv - sq;
+    const fh_half *kb = k + bi * kv_sb + kh * kv_sh, *vb = v + bi * kv_sb + kh * kv_sh;
+    int kend = skv;
+    if (causal) {
+        const int last = (qb0 + 127 < sq ? qb0 + 127 : sq - 1) + off + 1;
+        kend = last < skv ? last : skv;
+    }
+    const int steps = (kend + KS * BN - 1) / (KS * BN);
+    // Piece i of this wavefront: rows row + i RSTEP of a step's KS tiles; a lane brings one 16-byte piece of a row to its place.
+    constexpr int RSTEP = NW * 64 / CH;
+    static_assert(RSTEP % 16 == 0, "the same swap in all of a lane's rows");
+    const int row_bytes = (int)(kv_st * 2), row = (wave * 64 + lane) / CH, piece = lane % CH;
+    const int kc = (piece ^ (D == 128 ? row & 15 : (row >> 1) & 7)) * 16, vc = (piece ^ (D == 128 ? (row & 3) << 2 : ((row >> 1) & 1) << 2)) * 16;
+    auto fetch = [&](const fh_half *base, int c, int it, int plane) { // step `it` of K (plane 0) or V (1) into its buffer
+        const int t0 = it * KS * BN;
+        fh_half *to = ap_lds + ((it & 1) * 2 + plane) * KS * TILE + wave * 512;
+        const fh_half *from = base + t0 * kv_st;
+        if (t0 + KS * BN <= skv) {
+#pragma unroll
+            for (int i = 0; i < NP; i++) fh_buffer_to_lds(from, 0x7FFFFFFF, to + NW * i * 512, row * row_bytes + c, i * RSTEP * row_bytes);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NP; i++) { // rows past the last key repeat it: their scores are masked and their P is 0
+                const int r = row + i * RSTEP, end = skv - 1 - t0;
+                fh_buffer_to_lds(from, 0x7FFFFFFF, to + NW * i * 512, (r < end ? r : end) * row_bytes + c, 0);
+            }
+        }
+    };
+    auto landed = [&]() { // this wavefront's pieces, and everybody's behind the barrier
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (steps > 0) fetch(kb, kc, 0, 0), fetch(vb, vc, 0, 1);
+    half8 qf[KSTEPS];
+    {
+        const TQ *qp = q + bi * q_sb + h * q_sh + (int64_t)(qi < sq ? qi : sq - 1) * q_st + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ks++) {
+            fh_half t[8];
+            ap_load8(qp + 16 * ks, t);
+            __builtin_memcpy(&qf[ks], t, 16);
+        }
+    }
+    const int prow = 16 * (li >> 4) + 8 * ((li >> 2) & 1) + 4 * ((li >> 3) & 1) + (li & 3); // key read by MFMA row li
+    const uint32_t k_at = kset * TILE * 2 + prow * D * 2 + (g ^ (D == 128 ? prow & 15 : (prow >> 1) & 7)) * 16; // bytes
+    // keys 8 g + s / 4 (and 4 more) of a step of 16, dims 16 (lane / 16 % 2) + 4 (s % 4) .. of a tile of 32
+    const int vrow = 8 * g + ((lane & 15) >> 2), vpiece = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+    const uint32_t v_at = (KS + kset) * TILE * 2 + vrow * D * 2 + (vpiece ^ (D == 128 ? (vrow & 3) << 2 : ((vrow >> 1) & 1) << 2)) * 16 + 8 * (lane & 1);
+    const float sc2 = scale * 1.4426950408889634f, ninf = -INFINITY;
+    const int lim = causal ? (qi + off < skv - 1 ? qi + off : skv - 1) : skv - 1;
+    float m_run = -INFINITY, l_run = 0.f;
+    floatx16 acc[DT], sa[2], sb[2];
+    const floatx16 zero = {0.f};
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) acc[dt] = zero;
+
+    auto scores = [&](int it, floatx16 (&to)[2]) { // S^T of step `it`
+        uint32_t at = k_at + (uint32_t)(it & 1) * (4 * KS * TILE); // (swapped pieces are an exclusive or on the address, one instruction where it is used)
+        asm volatile("" : "+v"(at));
+        constexpr int NI = 2 * KSTEPS, AHEAD = 4;
+        half8 ka[AHEAD];
+        auto read = [&](int i) { ka[i % AHEAD] = *(const half8 *)((const uint8_t *)ap_lds + (at ^ (uint32_t)((i >> 1) * 32)) + (i & 1) * 64 * D); };
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) read(i);
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            to[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[i % AHEAD], qf[i >> 1], i < 2 ? zero : to[i & 1], 0, 0, 0);
+            if (i + AHEAD < NI) read(i + AHEAD);
+        }
+    };
+    auto mask = [&](int it, floatx16 (&to)[2]) {
+        const int t0 = (it * KS + kset) * BN, lim_t = KS == 1 || t0 < kend ? lim : -1; // (a group without a tile in the last step: all of it)
+        if (__any(t0 + BN - 1 > lim_t))
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int key = t0 + 32 * kt + 16 * (r >> 3) + 8 * g + (r & 7);
+                    asm volatile("v_cmp_le_i32 vcc, %1, %2\n\tv_cndmask_b32 %0, %3, %0, vcc"
+                                 : "+v"(to[kt][r])
+                                 : "v"(key), "v"(lim_t), "v"(ninf)
+                                 : "vcc");
+                }
+    };
+    auto step = [&](int it, floatx16 (&st)[2], floatx16 (&next)[2], bool last) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) mx = fmaxf(mx, st[kt][r]);
+        mx = ap_swap32_max(mx) * sc2;
+        if (__any(mx > m_run)) {
+            const float m_new = fmaxf(m_run, mx);
+            const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
+            m_run = m_new, l_run *= alpha;
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) sm[(2 + dt * 16 + r) * NQ + slot] = acc[dt][r];
+                for (int r = 0; r < 16; r++) acc[dt][r] *= alpha;
         }
-        __syncthreads();
-        if (kset == 1) return;
-        const float m1 = sm[slot], l1 = sm[NQ + slot];
-        const float mm = fmaxf(m_run, m1), ref = mm == -INFINITY ? 0.f : mm;
-        const float f0 = __builtin_amdgcn_exp2f(m_run - ref), f1 = __builtin_amdgcn_exp2f(m1 - ref);
-        l_run = l_run * f0 + l1 * f1;
+        const float m_sub = m_run == -INFINITY ? 0.f : -m_run; // dead rows: 2^(-inf - 0) = 0
+        if (it + 2 < steps) fetch(kb, kc, it + 2, 0);
+        if (!last) fetch(vb, vc, it + 1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!last) scores(it + 1, next);
+        half8 pb[2][2];
 #pragma unroll
-        for (int dt = 0; dt < DT; dt++)
+        for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[dt][r] = acc[dt][r] * f0 + sm[(2 + dt * 16 + r) * NQ + slot] * f1;
+            for (int s2 = 0; s2 < 2; s2++) {
+                fh_half t[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) t[e] = (fh_half)__builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + e], sc2, m_sub)); // arguments <= 0
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) l_run = __builtin_amdgcn_fdot2(half2v{t[e], t[e + 1]}, half2v{(fh_half)1.f, (fh_half)1.f}, l_run, false);
+                __builtin_memcpy(&pb[kt][s2], t, 16);
+            }
+        if (!last) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+            for (int i = 0; i < 2 * KSTEPS; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (i < 2 * KSTEPS - 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 64 / (2 * KSTEPS), 0);
+                __builtin_amdgcn_sched_group_barrier(0x400, 32 / (2 * KSTEPS), 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (!last) mask(it + 1, next);
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t at = v_at + (uint32_t)(it & 1) * (4 * KS * TILE);
+        asm volatile("" : "+v"(at));
+        constexpr int NJ = 4 * DT, AHEAD = 8;
+        half8 va[AHEAD];
+        auto read = [&](int j) { va[j % AHEAD] = ap_vt8((const fh_half *)((const uint8_t *)ap_lds + (at ^ (uint32_t)(j % DT * 64))) + 16 * (j / DT) * D, D); };
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) read(j);
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int c = j / DT;
+            acc[j % DT] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[j % AHEAD], pb[c >> 1][c & 1], acc[j % DT], 0, 0, 0);
+            if (j + AHEAD < NJ) read(j + AHEAD);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * AHEAD, 0);
+#pragma unroll
+        for (int j = 0; j < NJ - AHEAD; j++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+        landed();
+    };
+    if (steps > 0) {
+        landed();
+        if (steps > 1) fetch(kb, kc, 1, 0);
+        scores(0, sa);
+        mask(0, sa);
+        landed(); // (K of step 1; the place of step 0's is free)
+        int t = 0;
+        for (; t + 2 < steps; t += 2) {
+            step(t, sa, sb, false);
+            step(t + 1, sb, sa, false);
+        }
+        if (t + 2 == steps) {
+            step(t, sa, sb, false);
+            step(t + 1, sb, sa, true);
+        } else
+            step(t, sa, sb, true);
     }
-    // ---- store: lane = query, register r of d-tile dt is d = 32 dt + 8 (r / 4) + 4 g + r % 4
-    if (qi < sq) {
-        const float inv = 1.0f / l_run;
-        TQ *op = out + (((int64_t)bi * hq + h) * sq + qi) * D;
-#pragma unroll
-        for (int dt = 0; dt < DT; dt++)
-#pragma unroll
-            for (int r4 = 0; r4 < 4; r4++)
-                ap_store4(op + 32 * dt + 8 * r4 + 4 * g, acc[dt][4 * r4] * inv, acc[dt][4 * r4 + 1] * inv,
-                          acc[dt][4 * r4 + 2] * inv, acc[dt][4 * r4 + 3] * inv);
-    }
+    l_run = ap_swap32_sum(l_run);
+    if constexpr (KS == 2) ap_merge<D, 4>((float *)ap_lds, wave, lane, kset, m_run, l_run, acc);
+    if (KS == 2 && kset == 1) return;
+    if (qi < sq) ap_store<D>(out + (((int64_t)bi * hq + h) * sq + qi) * D, g, 1.0f / l_run, acc);
 }
 
 template <typename TQ, typename TKV, int D, bool SPLIT, int HW, int KS = 1, int QW = 4>
@@ -485,6 +681,17 @@ static fh_status ap_launch_k(fh_device *dev, const void *q, int64_t q_sb, int64_
     dim3 grid((unsigned)(hq / HW), (unsigned)((sq + 32 * QW - 1) / (32 * QW)), (unsigned)b);
     kern<<<grid, 64 * QW * HW * KS, LDS, dev->stream>>>((const TQ *)q, q_sb, q_sh, q_st, (const TKV *)k, (const TKV *)v, kv_sb,
                                                kv_sh, kv_st, hq, hkv, sq, skv, scale, causal, (TQ *)out);
+    FH_HIP(hipGetLastError());
+    return FH_OK;
+}
+
+template <typename TQ, int D, int KS>
+static fh_status ap_launch_ahead(fh_device *dev, const void *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void *k, const void *v, int64_t kv_sb,
+                                 int64_t kv_sh, int64_t kv_st, int b, int hq, int hkv, int sq, int skv, float scale, int causal, void *out) {
+    constexpr int LDS = 2 * 2 * KS * 64 * D * 2, MERGE = KS == 2 ? (2 + D / 2) * 256 * 4 : 0, BYTES = LDS > MERGE ? LDS : MERGE;
+    FH_TRY(fh_kernel_lds(dev, (const void *)k_attn_ahead<TQ, D, KS>, BYTES));
+    k_attn_ahead<TQ, D, KS><<<dim3((unsigned)hq, (unsigned)((sq + 127) / 128), (unsigned)b), 256 * KS, BYTES, dev->stream>>>(
+        (const TQ *)q, q_sb, q_sh, q_st, (const fh_half *)k, (const fh_half *)v, kv_sb, kv_sh, kv_st, hq, hkv, sq, skv, scale, causal, (TQ *)out);
     FH_HIP(hipGetLastError());
     return FH_OK;
 }
@@ -511,10 +718,19 @@ static fh_status ap_launch(fh_device *dev, const void *q, int64_t q_sb, int64_t 
         const bool rows64 = force == 9 || (force == 0 && halves && 4 * wgs64 <= 5L * dev->compute_units);
         if (rows64) return d == 128 ? ap_launch_k<TQ, TKV, 128, SPLIT, 1, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, out)
                                     : ap_launch_k<TQ, TKV, 64, SPLIT, 1, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, out);
-        if (halves) return d == 128 ? FH_AP(128, 1, 2) : FH_AP(64, 1, 2);
+        if constexpr (sizeof(TKV) == 2) {
+#define FH_AH(D, KS) ap_launch_ahead<TQ, D, KS>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, out)
+            if (halves) return d == 128 ? FH_AH(128, 2) : FH_AH(64, 2);
+            if (!pair) return d == 128 ? FH_AH(128, 1) : FH_AH(64, 1);
+#undef FH_AH
+            return d == 128 ? FH_AP(128, 2, 1) : FH_AP(64, 2, 1);
+        } else if (halves)
+            return d == 128 ? FH_AP(128, 1, 2) : FH_AP(64, 1, 2);
     }
-    if (d == 128) return pair ? FH_AP(128, 2, 1) : FH_AP(128, 1, 1);
-    return pair ? FH_AP(64, 2, 1) : FH_AP(64, 1, 1);
+    if constexpr (SPLIT || sizeof(TKV) == 4) {
+        if (d == 128) return pair ? FH_AP(128, 2, 1) : FH_AP(128, 1, 1);
+        return pair ? FH_AP(64, 2, 1) : FH_AP(64, 1, 1);
+    }
 #undef FH_AP
 }
 

@@ -483,21 +483,21 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
 // 4 rows' 64 bytes cover the banks once).  What is left is the chain of a step in one wavefront (with the two key groups half a step apart, one in
 // the softmax and one in the second product, it is longer: 2048 tokens 56 us).  Before and after, causal, us: 8 heads of 64, 3000 tokens 34.0 / 31.0;
 // 16 / 4 of 64, 777 12.1 / 12.0; 32 / 8 of 128, 2048 51.5 / 50.6, 3000 101 / 97.
-template <typename TQ, int D, int KS>
-__global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attn_ahead(
+template <typename TQ, int D, int KS, int QW>
+__global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(QW == 4 ? 2 : 1, 2))) void k_attn_ahead(
     const TQ *__restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_st, const fh_half *__restrict__ k, const fh_half *__restrict__ v, int64_t kv_sb,
     int64_t kv_sh, int64_t kv_st, int hq, int hkv, int sq, int skv, float scale, int causal, TQ *__restrict__ out) {
-    constexpr int BN = 64, DT = D / 32, KSTEPS = D / 16, CH = D / 8, TILE = BN * D, NW = 4 * KS, NP = TILE * KS * 2 / 1024 / NW; // NP: 1 KB pieces of K a wavefront
+    constexpr int BN = 64, DT = D / 32, KSTEPS = D / 16, CH = D / 8, TILE = BN * D, NW = QW * KS, NP = TILE * KS * 2 / 1024 / NW; // NP: 1 KB pieces of K a wavefront
     extern __shared__ __attribute__((aligned(16))) fh_half ap_lds[]; // [2 buffers][KS tiles of K, KS of V]
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31, g = lane >> 5;
-    const int kset = KS == 2 ? wave >> 2 : 0;
+    const int kset = KS == 2 ? wave / QW : 0;
     const int h = (int)blockIdx.x, bi = blockIdx.z, kh = h / (hq / hkv);
-    const int qb0 = (causal ? (int)(gridDim.y - 1 - blockIdx.y) : (int)blockIdx.y) * 128;
-    const int qi = qb0 + (wave & 3) * 32 + li, off = skv - sq;
+    const int qb0 = (causal ? (int)(gridDim.y - 1 - blockIdx.y) : (int)blockIdx.y) * 32 * QW;
+    const int qi = qb0 + (wave % QW) * 32 + li, off = skv - sq;
     const fh_half *kb = k + bi * kv_sb + kh * kv_sh, *vb = v + bi * kv_sb + kh * kv_sh;
     int kend = skv;
     if (causal) {
-        const int last = (qb0 + 127 < sq ? qb0 + 127 : sq - 1) + off + 1;
+        const int last = (qb0 + 32 * QW - 1 < sq ? qb0 + 32 * QW - 1 : sq - 1) + off + 1;
         kend = last < skv ? last : skv;
     }
     const int steps = (kend + KS * BN - 1) / (KS * BN);
@@ -664,7 +664,7 @@ __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2, 2))
             step(t, sa, sb, true);
     }
     l_run = ap_swap32_sum(l_run);
-    if constexpr (KS == 2) ap_merge<D, 4>((float *)ap_lds, wave, lane, kset, m_run, l_run, acc);
+    if constexpr (KS == 2) ap_merge<D, QW>((float *)ap_lds, wave, lane, kset, m_run, l_run, acc);
     if (KS == 2 && kset == 1) return;
     if (qi < sq) ap_store<D>(out + (((int64_t)bi * hq + h) * sq + qi) * D, g, 1.0f / l_run, acc);
 }
@@ -685,12 +685,12 @@ static fh_status ap_launch_k(fh_device *dev, const void *q, int64_t q_sb, int64_
     return FH_OK;
 }
 
-template <typename TQ, int D, int KS>
+template <typename TQ, int D, int KS, int QW = 4>
 static fh_status ap_launch_ahead(fh_device *dev, const void *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void *k, const void *v, int64_t kv_sb,
                                  int64_t kv_sh, int64_t kv_st, int b, int hq, int hkv, int sq, int skv, float scale, int causal, void *out) {
-    constexpr int LDS = 2 * 2 * KS * 64 * D * 2, MERGE = KS == 2 ? (2 + D / 2) * 256 * 4 : 0, BYTES = LDS > MERGE ? LDS : MERGE;
-    FH_TRY(fh_kernel_lds(dev, (const void *)k_attn_ahead<TQ, D, KS>, BYTES));
-    k_attn_ahead<TQ, D, KS><<<dim3((unsigned)hq, (unsigned)((sq + 127) / 128), (unsigned)b), 256 * KS, BYTES, dev->stream>>>(
+    constexpr int LDS = 2 * 2 * KS * 64 * D * 2, MERGE = KS == 2 ? (2 + D / 2) * 64 * QW * 4 : 0, BYTES = LDS > MERGE ? LDS : MERGE;
+    FH_TRY(fh_kernel_lds(dev, (const void *)k_attn_ahead<TQ, D, KS, QW>, BYTES));
+    k_attn_ahead<TQ, D, KS, QW><<<dim3((unsigned)hq, (unsigned)((sq + 32 * QW - 1) / (32 * QW)), (unsigned)b), 64 * QW * KS, BYTES, dev->stream>>>(
         (const TQ *)q, q_sb, q_sh, q_st, (const fh_half *)k, (const fh_half *)v, kv_sb, kv_sh, kv_st, hq, hkv, sq, skv, scale, causal, (TQ *)out);
     FH_HIP(hipGetLastError());
     return FH_OK;
@@ -716,16 +716,20 @@ static fh_status ap_launch(fh_device *dev, const void *q, int64_t q_sb, int64_t 
         // of them - a SIMD then runs one wavefront's chain of a step instead of two (512 tokens: 15.0 against 16.8 us)
         const long wgs64 = (long)hq * ((sq + 63) / 64) * b;
         const bool rows64 = force == 9 || (force == 0 && halves && 4 * wgs64 <= 5L * dev->compute_units);
-        if (rows64) return d == 128 ? ap_launch_k<TQ, TKV, 128, SPLIT, 1, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, out)
-                                    : ap_launch_k<TQ, TKV, 64, SPLIT, 1, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, out);
         if constexpr (sizeof(TKV) == 2) {
 #define FH_AH(D, KS) ap_launch_ahead<TQ, D, KS>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, out)
+            if (rows64)
+                return d == 128 ? ap_launch_ahead<TQ, 128, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, out)
+                                : ap_launch_ahead<TQ, 64, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, out);
             if (halves) return d == 128 ? FH_AH(128, 2) : FH_AH(64, 2);
             if (!pair) return d == 128 ? FH_AH(128, 1) : FH_AH(64, 1);
 #undef FH_AH
             return d == 128 ? FH_AP(128, 2, 1) : FH_AP(64, 2, 1);
-        } else if (halves)
-            return d == 128 ? FH_AP(128, 1, 2) : FH_AP(64, 1, 2);
+        } else {
+            if (rows64) return d == 128 ? ap_launch_k<TQ, TKV, 128, SPLIT, 1, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, out)
+                                        : ap_launch_k<TQ, TKV, 64, SPLIT, 1, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, out);
+            if (halves) return d == 128 ? FH_AP(128, 1, 2) : FH_AP(64, 1, 2);
+        }
     }
     if constexpr (SPLIT || sizeof(TKV) == 4) {
         if (d == 128) return pair ? FH_AP(128, 2, 1) : FH_AP(128, 1, 1);

@@ -53,6 +53,9 @@ extern "C" fh_status fh_device_create(int32_t ordinal, fh_device **out) {
     FH_HIP(hipEventCreate(&d->ev_stop));
     FH_HIP(hipMalloc(&d->small_buf, 64 * 1024));
     FH_HIP(hipMalloc(&d->fixed_buf, FH_FIXED_BYTES));
+    FH_HIP(hipMalloc((void **)&d->arrived, FH_ARRIVED * 4));
+    FH_HIP(hipMemset(d->arrived, 0, FH_ARRIVED * 4));
+    FH_HIP(hipStreamSynchronize(nullptr));
     // the reference's trace switches (models/kalosm-llama/src/raw/mod.rs:943-955, fusor-ml/core/src/compute_graph/
     // resolve/run.rs:141): present in the environment = on, lines on stderr
     if (getenv("KALOSM_TRACE_LAYER_NAN")) d->opt_trace_nan = d->opt_trace_stderr = 1;
@@ -78,6 +81,7 @@ extern "C" fh_status fh_device_destroy(fh_device *dev) {
     if (dev->frag_x) (void)hipFree(dev->frag_x);
     if (dev->small_buf) (void)hipFree(dev->small_buf);
     if (dev->fixed_buf) (void)hipFree(dev->fixed_buf);
+    if (dev->arrived) (void)hipFree(dev->arrived);
     (void)hipEventDestroy(dev->ev_start);
     (void)hipEventDestroy(dev->ev_stop);
     (void)hipStreamDestroy(dev->stream);

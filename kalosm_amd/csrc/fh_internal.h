@@ -60,6 +60,8 @@ struct fh_device {
     // 9 MB that never move (FH_FIXED_BYTES): the keys of a top-k over up to 2^20 logits, the rows of the output matrix's one pass.  In
     // buffers that grow they would end the graphs of other calls, and a captured call would need an eager one of its size.
     void *fixed_buf = nullptr;
+    // counters of workgroups that have written a part of a sum, zero between launches (fh_qmv_rows.hip)
+    uint32_t *arrived = nullptr;
     // Counts the reallocations of act_buf / part_buf / ksplit_buf.  A captured graph holds their addresses as
     // kernel arguments, so whoever keeps a graph records the value at capture and must not replay it after
     // the value has changed.
@@ -84,7 +86,7 @@ struct fh_device {
     int64_t opt_attn_heads = 0;      // query heads per workgroup of the decode attention (0: automatic; 1, 2, 4, 8)
     int64_t opt_attn_waves = 0;      // wavefronts per workgroup of the decode attention (0: 16; 8)
     int64_t opt_matvec_rows = 0;     // 1: 2 .. 4 activation rows never through the single-row Q4_K kernel's row variant
-    int64_t opt_matvec_direct = 0; // 1: 5 .. 16 rows never through the unstaged kernel, 2: 2 .. 4 rows through it as well
+    int64_t opt_matvec_direct = 0; // 1: 5 .. 16 rows never through the unstaged kernel, 2: 2 .. 4 rows through it as well, 3: 2 .. 16 rows in one launch (k_qmv_rows) wherever it can
     int64_t opt_wo_tiles = 0;        // row tiles per wavefront of the accumulating output projection (0: 4; 1, 2, 4)
     int64_t opt_wo_acc = 0;          // 0: decode steps accumulate the output projection into the residual stream, 1: never
     int64_t opt_fuse_norm = 0;       // 0: decode steps fold rms_norm into the consuming matvec, 1: separate launches
@@ -100,7 +102,7 @@ struct fh_device {
     int64_t opt_matmul_cut = 0;      // > 0: mt + 16 kw + 256 parts, how the products that decode in registers are cut (tests)
 };
 
-enum { FH_FIXED_BYTES = 9 << 20 };
+enum { FH_FIXED_BYTES = 9 << 20, FH_ARRIVED = 16384 };
 
 // Which scratch memory the kernels of a captured graph hold the addresses of: begin ahead of the capture, end behind it.
 struct FhScratchStamp {

@@ -14,6 +14,7 @@
 //                  of Q4_K uses the factorisation  y = d*sum_j sc_j*(q.x)_j - dmin*sum_j m_j*(sum x)_j.
 #include "fh_blocks.h"
 #include "fh_qmm_frag.h"
+#include "fh_qmv_rows.h"
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -407,6 +408,14 @@ static fh_status qmatmul(const fh_qmatrix *q, const float *x_dev, int32_t m, flo
     // dense f16 / f32 weight rows (core/src/quantized/matmul/kernel.rs:132-193 routes them to the dense matmul) take
     // the matrix-core tiles as well once there are rows to fill them
     const bool dense = (q->type == FH_W_F16 || q->type == FH_W_F32) && q->k % 32 == 0;
+    // a few rows: one launch that converts its activations itself (prompts of a decoder keep the sums they have)
+    const fh_device *dev = q->dev;
+    if (mk == 0 && dev->opt_matvec_kernel == 0 && fragments &&
+        (dev->opt_matvec_direct == 3 ? fh_qmv_rows_supports(q, x_dev, m)
+                                     : dev->opt_matvec_direct == 0 && dev->opt_matvec_tiles == 0 && dev->opt_matvec_per == 0 && dev->opt_matvec_rows == 0 && fh_qmv_rows_pays(q, x_dev, m))) {
+        const fh_status st = fh_launch_qmv_rows(q, x_dev, m, y_dev);
+        if (st != FH_ERR_UNSUPPORTED) return st;
+    }
     // The 5-bit formats have no batch kernel for 2 .. 16 rows: rows are a launch each up to four, the kernel of small prompts takes them
     // from there, with a power of two per 32 activations as they have it (us, launches / that: 12 rows of 14336 x 4096 in Q5_0 97 / 23, in Q5_K
     // 100 / 25, of 4096 x 4096 46 / 14 and 46 / 15, of 512 x 2048 40 / 14 and 40 / 16; four rows of the latter two take 16 and 14 as launches).

@@ -1,0 +1,110 @@
+"""Products of a few rows in one launch: every cut (row tiles a wavefront, 256s a workgroup, parts of k that the last workgroup adds) at the ends of its
+tiles and parts, against 64 bits; which products take it; repeats, captured ones among them, and rows that do not mix."""
+import numpy as np
+import pytest
+
+from kalosm_amd import synth
+from kalosm_amd.fusor import QMatrix, Tensor
+
+pytestmark = pytest.mark.gpu
+TYPES = [synth.Q4_0, synth.Q5_0, synth.Q8_0, synth.Q4_K, synth.Q5_K, synth.Q6_K]
+named = pytest.mark.parametrize("ty", TYPES, ids=lambda t: synth.TYPE_NAMES[t])
+
+
+class options:
+    def __init__(self, dev, **kv):
+        self.dev, self.kv = dev, kv
+
+    def __enter__(self):
+        for k, v in self.kv.items():
+            self.dev.set_option(k, v)
+
+    def __exit__(self, *_):
+        for k in self.kv:
+            self.dev.set_option(k, 0)
+
+
+def matrix(dev, oracle, ty, n, k, seed=1):
+    raw = synth.random_weight(ty, n, k, seed=seed)
+    return QMatrix.from_raw_bytes(dev, (n, k), raw, ty), oracle.dequantize(ty, raw).reshape(n, k).astype(np.float64)
+
+
+def close(got, x, w):
+    """An activation keeps 22 bits, a product is exact, and a sum of f32 takes at most 16 roundings to a value's place in a 256 (two operands, eight blocks,
+    scale, offset and factor) and a dozen behind it: 2^-19 of the sum of magnitudes, a hundredth of which is what random signs leave."""
+    x = x.astype(np.float64)
+    err = np.abs(got - x @ w.T)
+    assert np.isfinite(got).all() and (err <= 2.0 ** -19 * (np.abs(x) @ np.abs(w).T)).all()
+    assert np.sqrt((err ** 2).mean()) <= 3e-7 * np.sqrt(((x * x) @ (w * w).T).mean())
+
+
+@named
+@pytest.mark.parametrize("cut", [1, 2, 3, 4, 9, 10, 11, 12])
+@pytest.mark.parametrize("m,n,k", [(16, 272, 256 * 9), (5, 33, 256 * 4), (2, 600, 256 * 8), (13, 130, 256), (7, 1040, 256 * 21)])
+def test_every_cut(dev, oracle, ty, cut, m, n, k):
+    q, w = matrix(dev, oracle, ty, n, k)
+    x = synth.random_activation(m, k, seed=2) * np.exp(np.random.default_rng(3).standard_normal((m, 1))).astype(np.float32)
+    with options(dev, matvec_direct=3, matvec_tiles=cut):
+        close(Tensor.from_slice(dev, x).q_mat_mul(q).as_slice().astype(np.float64), x, w)
+
+
+@named
+@pytest.mark.parametrize("m,n,k,taken", [(16, 512, 2048, True), (5, 4096, 1024, True), (4, 512, 2048, False), (6, 40000, 2048, False)])
+def test_rule(dev, oracle, ty, m, n, k, taken):
+    """Either side of its lines: the bits of one launch, or of others."""
+    if ty == synth.Q6_K and m == 4:
+        taken = True
+    q, _ = matrix(dev, oracle, ty, n, k)
+    xt = Tensor.from_slice(dev, synth.random_activation(m, k, seed=2))
+    auto = xt.q_mat_mul(q).as_slice()
+    with options(dev, matvec_direct=3):
+        one = xt.q_mat_mul(q).as_slice()
+    assert np.array_equal(auto, one) == taken
+
+
+@named
+def test_small_groups_beside_a_large_one(dev, oracle, ty):
+    """Weights that are zero where the activations are large: the formats that normalise 32 values by themselves lose nothing of the small
+    ones, the others what a power of two per 256 leaves of them (values of 2^-16 of the largest keep eight bits)."""
+    n, k, m = 64, 2048, 6
+    raw = synth.random_weight(ty, n, k, seed=4)
+    w = oracle.dequantize(ty, raw).reshape(n, k)
+    size = synth.BLOCK_ELEMS[ty]
+    blocks = raw.reshape(n, k // size, -1).copy()
+    blocks[:, 0] = 0  # a block of zeros: scale (and offset) zero
+    raw = np.ascontiguousarray(blocks).reshape(-1)
+    w = oracle.dequantize(ty, raw).reshape(n, k).astype(np.float64)
+    assert not w[:, :size].any()
+    x = synth.random_activation(m, k, seed=5)
+    x[:, :min(32, size)] *= np.float32(2.0 ** 14)
+    q = QMatrix.from_raw_bytes(dev, (n, k), raw, ty)
+    with options(dev, matvec_direct=3):
+        got = Tensor.from_slice(dev, x).q_mat_mul(q).as_slice().astype(np.float64)
+    want = x.astype(np.float64) @ w.T
+    assert np.abs(got - want).max() <= 2.0 ** -17 * np.abs(want).max()
+
+
+@named
+def test_repeats_and_rows(dev, oracle, ty):
+    """The same bits every time, in a captured launch too (the counters of the parts are zero again behind each); an infinity or a NaN stays in
+    its row."""
+    n, k, m = 528, 256 * 13, 9
+    q, _ = matrix(dev, oracle, ty, n, k)
+    x = synth.random_activation(m, k, seed=6)
+    xt, y = Tensor.from_slice(dev, x), Tensor(dev, (m, n), "f32")
+    with options(dev, matvec_direct=3):
+        base = xt.q_mat_mul(q).as_slice()
+        dev.graph_begin()
+        xt.q_mat_mul(q, out=y)
+        graph = dev.graph_end()
+        for _ in range(5):
+            graph.launch()
+            dev.sync()
+            assert np.array_equal(y.as_slice(), base)
+            assert np.array_equal(xt.q_mat_mul(q).as_slice(), base)
+        x[2] = 0.0
+        x[3, 7], x[4, 9] = np.inf, np.nan
+        got = Tensor.from_slice(dev, x).q_mat_mul(q).as_slice()
+    assert not got[2].any() and not np.isfinite(got[3]).any() and np.isnan(got[4]).all()
+    rest = [r for r in range(m) if r not in (2, 3, 4)]
+    assert np.array_equal(got[rest], base[rest])

@@ -120,7 +120,16 @@ enum { FH_BF16_ACT = 2 };
 static inline size_t fh_act_size(int dtype) { return dtype == FH_BF16_ACT ? 2 : 4; }
 
 // Row groups of a grouped product: tile i covers rows [row0, row0 + rows) that all belong to group `group`.
-struct FhTile { int group, row0, rows, pad; };
+// A tile is number `at` of `of` (8 at most) neighbours of its group whose products are worked on together.
+struct FhTile { int group, row0, rows; short at, of; };
+// Tile j of a group of `rows` rows: row tiles of more than 128 rows share them out evenly, in steps of 32.
+__host__ __device__ static inline int fh_tiles_of(int rows, int tile_rows) { return (rows + tile_rows - 1) / tile_rows; }
+__host__ __device__ static inline FhTile fh_tile(int group, int row0, int rows, int j, int tile_rows) {
+    const int n = fh_tiles_of(rows, tile_rows), steps = (rows + 31) / 32, of = n - (j & ~7);
+    const int from = tile_rows > 128 ? (int)((int64_t)steps * j / n) * 32 : j * tile_rows;
+    const int to = tile_rows > 128 ? (int)((int64_t)steps * (j + 1) / n) * 32 : from + tile_rows;
+    return FhTile{group, row0 + from, (to < rows ? to : rows) - from, (short)(j & 7), (short)(of < 8 ? of : 8)};
+}
 
 enum {
     FH_GEMM_F32 = 0,        // y f32 [m, ldy]
@@ -139,7 +148,7 @@ struct FhGemm {
     int n = 0, kp = 0, m = 0;    // n: weight rows of a group
     const FhTile *tiles = nullptr; // grouped: device table and its fill count
     const int *n_tiles = nullptr;
-    int max_tiles = 0, tile_rows = 64; // rows an entry may cover: 64, or 128 with bf16 activations
+    int max_tiles = 0, tile_rows = 64; // rows an entry may cover: 64, or with bf16 activations 128 or a multiple of 32 up to 320
 };
 fh_status fh_gemm(fh_device *dev, int dtype, int epi, const FhGemm &g);
 
@@ -157,6 +166,12 @@ fh_status fh_rows_to_act(fh_device *dev, int dtype, const float *x, int64_t ldx,
 
 // The row table of a product whose `groups` groups have s rows each, group after group (FhGemm::tiles, n_tiles).
 static inline int fh_group_tile_rows(const fh_device *dev, int dtype, int groups, int s, int n) {
+    // tiles of up to 256 rows where their rounds of workgroups cost less than those of 128 rows (fh_gemm): four groups of 2048 rows,
+    // 4096 x 4096 253 us (300)
+    const int64_t opt = dev->opt_matmul_kernel, cus = dev->compute_units, wn = (n + 255) / 256;
+    const int64_t t256 = groups * wn * ((s + 255) / 256), t128 = groups * wn * ((s + 127) / 128);
+    const bool tall = t256 * 4 >= cus * 3 && (t128 + cus - 1) / cus * 2 >= (t256 + cus - 1) / cus * 3;
+    if (dtype != FH_F32 && opt != 3 && opt != 14 && (opt == 4 || tall)) return 256;
     return dtype != FH_F32 && (int64_t)groups * ((s + 127) / 128) * ((n + 127) / 128) >= dev->compute_units ? 128 : 64;
 }
 fh_status fh_group_tiles(fh_device *dev, int groups, int s, int tile_rows, FhTile *tiles, int *n_tiles);

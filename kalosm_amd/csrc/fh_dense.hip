@@ -1,6 +1,7 @@
 // Dense bf16 weights: prefill products on the matrix cores (plain and grouped by expert), the decode matvec with the
 // RMS norm of its input, and the norm that writes activation rows.
 #include "fh_dense.h"
+#include <type_traits>
 
 // ------------------------------------------------------------------------------ prefill product
 // y[m, n] = x[m, :] . W[n, :].  The weights are the A operand (accumulator rows), the activations the B operand
@@ -160,16 +161,19 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(FhGemm g) {
 // What bounds the 128 x 128 kernel above is what a compute unit gets from its L2 - 32 KB per 64 of k and 128 x 128 outputs, 78 B/ns
 // at the rate of the matrix cores - and that every step waits for the step just requested.  256 x 256 halves the bytes, and
 // the clock, which the matrix cores bring down to 1.7 GHz, becomes the bound: 2048 x 14336 x 4096 in 231 us (1.04 PFLOP/s, 331 us
-// before), 2048 x 4096 x 14336 with 128 rows per tile in 211 us (1.14 PFLOP/s).  Products grouped by expert stay bound by their
-// weights: 32 experts of 4096 x 4096 and 8192 rows 417 us (454 before; reading 1.07 GB takes 230 us).
+// before), 2048 x 4096 x 14336 with 128 rows per tile in 211 us (1.14 PFLOP/s).  Products grouped by expert: 32 experts of 4096 x 4096 and
+// 8192 rows 305 us with tiles of up to 320 rows where no expert has more, 364 over uneven ones (382 with 128 rows; reading 1.07 GB takes 230 us).  Their
+// row tiles are of any height: a wavefront multiplies only the 32-column tiles that have rows (without that, and with a weight tile's row tiles
+// on several dies, the 128-row form took 447), and the two wavefronts of a SIMD take the two halves of the columns.
 // 64 of k (a slab) per barrier; the barrier sits ahead of the slab's last quarter, whose operands are in registers already, so
 // the next slab's first operands are read and the requests of the slab after it go out while that quarter is multiplied.
-// SLABS buffers: two of 64 KB, or three of 48 KB with 128 activation rows (groups of rows, fewer rows).
+// SLABS buffers: two of 64 KB, three of 48 KB with 128 activation rows (fewer rows), or two of 72 KB with up to 320 (groups of rows).
 template <int TX>
 struct WideTile {
-    static constexpr int TW = 256, WGX = TX == 256 ? 4 : 2, FW = TX == 256 ? 4 : 2, FX = 2; // a wavefront: FW x FX tiles of 32 x 32
-    static constexpr int NLW = TW / 64, NLX = TX / 64, NL = NLW + NLX;                      // requests of a wavefront per slab
-    static constexpr int SLAB = (TW + TX) * 128, SLABS = TX == 256 ? 2 : 3;
+    static constexpr int TW = 256, WGX = TX == 256 ? 4 : 2, FW = TX == 256 ? 4 : 2, FX = TX / 32 / WGX; // a wavefront: FW x FX tiles of 32 x 32
+    static constexpr int NLW = TW / 64, NLX = TX / 64, NL = NLW + NLX;                                  // requests of a wavefront per slab
+    static constexpr int SLAB = (TW + TX) * 128, SLABS = TX == 128 ? 3 : 2;
+    static constexpr bool COUNT_VARIES = TX == 320; // rows that are not there are not requested: two slabs, of which none may be on its way
 };
 
 template <int TX, int EPI>
@@ -180,22 +184,27 @@ __global__ __launch_bounds__(512) void k_gemm_bf16_wide(FhGemm g) {
     constexpr bool W_ROWS = EPI == FH_GEMM_SWIGLU || EPI == FH_GEMM_ACT_T; // weight rows along the registers of the result, else along its lanes
     extern __shared__ __attribute__((aligned(16))) uint8_t wide_smem[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31;
-    const int ww = wave / WGX, wx = wave % WGX;
-    // The eight dies take runs of tiles.  Without groups: eight weight tiles by all row tiles, weight tiles first; with groups all
-    // weight tiles of a row tile first: a group's rows and weights meet in one die's L2.
-    const int tn = (g.n + TW - 1) / TW, ty = g.tiles ? *g.n_tiles : (g.m + TX - 1) / TX;
-    const int total = tn * ty, per = total >> 3, more = total & 7, die = (int)blockIdx.x & 7, idx = (int)blockIdx.x >> 3;
-    if (idx >= per + (die < more ? 1 : 0)) return;
-    const int lin = idx + die * per + (die < more ? die : more);
+    constexpr int WGW = 8 / WGX;
+    const int ww = wave % WGW, wx = wave / WGW;
+    // The eight dies take runs of tiles.  Without groups: eight weight tiles by all row tiles, weight tiles first.  With groups: up
+    // to eight row tiles of a group by all weight tiles, row tiles first, so that they read a weight tile from one die's L2 together.
+    const int tn = (g.n + TW - 1) / TW, die = (int)blockIdx.x & 7, idx = (int)blockIdx.x >> 3;
     int row0, m_end, n0;
     const uint16_t *w = g.w;
     if (g.tiles) {
-        const FhTile t = g.tiles[lin / tn];
-        n0 = lin % tn * TW;
+        const int total = *g.n_tiles * tn, per = total >> 3, more = total & 7;
+        if (idx >= per + (die < more ? 1 : 0)) return;
+        const int lin = idx + die * per + (die < more ? die : more), i = lin / tn;
+        const int of = g.tiles[i].of, at = g.tiles[i].at, l = lin - (i - at) * tn;
+        const FhTile t = g.tiles[i - at + l % of];
+        n0 = l / of * TW;
         row0 = t.row0;
         m_end = t.row0 + t.rows;
         w += (int64_t)t.group * g.w_group;
     } else {
+        const int ty = (g.m + TX - 1) / TX, total = tn * ty, per = total >> 3, more = total & 7;
+        if (idx >= per + (die < more ? 1 : 0)) return;
+        const int lin = idx + die * per + (die < more ? die : more);
         const int grp = lin / (8 * ty), in = lin - grp * 8 * ty, gw = tn - grp * 8 < 8 ? tn - grp * 8 : 8;
         n0 = (grp * 8 + in % gw) * TW;
         row0 = in / gw * TX;
@@ -216,6 +225,9 @@ __global__ __launch_bounds__(512) void k_gemm_bf16_wide(FhGemm g) {
         if (g.gather) m = g.gather[m];
         xp[i] = (const uint16_t *)g.x + (int64_t)m * g.kp + piece;
     }
+    // the 32-column tiles that have rows; with two wavefronts along them they are shared out evenly
+    const int cols = m_end - row0 < TX ? (m_end - row0 + 31) / 32 : TX / 32;
+    const int c0 = WGX > 2 ? wx * FX : wx ? (cols + 1) / 2 : 0, mine = WGX > 2 ? cols - c0 < FX ? cols - c0 : FX : wx ? cols / 2 : (cols + 1) / 2;
     const int slabs = g.kp / 64;
     auto fetch = [&](int s, int at) { // slab s into the buffer at byte `at`; past the end a repeat, so that the counts stay equal
         const int64_t o = (int64_t)(s < slabs ? s : slabs - 1) * 64;
@@ -226,18 +238,10 @@ __global__ __launch_bounds__(512) void k_gemm_bf16_wide(FhGemm g) {
                                              (__attribute__((address_space(3))) uint32_t *)(dst + i * 8192), 16, 0, 0);
 #pragma unroll
         for (int i = 0; i < Tile::NLX; i++)
-            __builtin_amdgcn_global_load_lds((const uint32_t *)(xp[i] + o),
+            if (!Tile::COUNT_VARIES || i * 2 < cols) __builtin_amdgcn_global_load_lds((const uint32_t *)(xp[i] + o),
                                              (__attribute__((address_space(3))) uint32_t *)(dst + (Tile::NLW + i) * 8192), 16, 0, 0);
     };
-    fh_bf8 fw[2][FW], fx[2][FX];
-    const int sw = gemm_sw(li), rw = (ww * FW * 32 + li) * 128, rx = (TW + wx * FX * 32 + li) * 128; // (tiles start at multiples of 32 rows)
-    auto read = [&](int set, int at, int q) { // quarter q (16 of k) of the slab at byte `at`
-        const uint8_t *b = wide_smem + at + ((2 * q + (lane >> 5)) ^ sw) * 16;
-#pragma unroll
-        for (int a = 0; a < FW; a++) fw[set][a] = *(const fh_bf8 *)(b + rw + a * 4096);
-#pragma unroll
-        for (int c = 0; c < FX; c++) fx[set][c] = *(const fh_bf8 *)(b + rx + c * 4096);
-    };
+    const int sw = gemm_sw(li), rw = (ww * FW * 32 + li) * 128, rx = (TW + c0 * 32 + li) * 128; // (tiles start at multiples of 32 rows)
     f16v acc[FW][FX];
 #pragma unroll
     for (int a = 0; a < FW; a++)
@@ -245,49 +249,68 @@ __global__ __launch_bounds__(512) void k_gemm_bf16_wide(FhGemm g) {
         for (int c = 0; c < FX; c++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[a][c][r] = 0.f;
-    auto mul = [&](int set) {
-#pragma unroll
-        for (int a = 0; a < FW; a++)
-#pragma unroll
-            for (int c = 0; c < FX; c++)
-                acc[a][c] = W_ROWS ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[set][a], fx[set][c], acc[a][c], 0, 0, 0)
-                                   : __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[set][c], fw[set][a], acc[a][c], 0, 0, 0);
-    };
 #pragma unroll
     for (int i = 0; i < SLABS; i++) fetch(i, i * SLAB);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SLABS - 1) * Tile::NL) : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    read(0, 0, 0);
-    int cur = 0;
-    for (int s = 0; s < slabs; s++) {
-        const int nxt = cur + SLAB == SLABS * SLAB ? 0 : cur + SLAB;
-        read(1, cur, 1);
-        mul(0);
-        __builtin_amdgcn_sched_barrier(0);
-        read(0, cur, 2);
-        mul(1);
-        __builtin_amdgcn_sched_barrier(0);
-        read(1, cur, 3);
-        mul(0);
-        __builtin_amdgcn_sched_barrier(0);
-        // the last quarter's operands are here: this wavefront is done with the slab's buffer; and slab s + 1 has landed
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((SLABS - 2) * Tile::NL) : "memory");
+    auto all = [&](auto have) { // so many of the wavefront's FX column tiles; the barriers are the same ones for every number
+        constexpr int C = decltype(have)::value;
+        fh_bf8 fw[2][FW], fx[2][FX];
+        auto read = [&](int set, int at, int q) { // quarter q (16 of k) of the slab at byte `at`
+            if (!C) return;
+            const uint8_t *b = wide_smem + at + ((2 * q + (lane >> 5)) ^ sw) * 16;
+#pragma unroll
+            for (int a = 0; a < FW; a++) fw[set][a] = *(const fh_bf8 *)(b + rw + a * 4096);
+#pragma unroll
+            for (int c = 0; c < C; c++) fx[set][c] = *(const fh_bf8 *)(b + rx + c * 4096);
+        };
+        auto mul = [&](int set) {
+#pragma unroll
+            for (int a = 0; a < FW; a++)
+#pragma unroll
+                for (int c = 0; c < C; c++)
+                    acc[a][c] = W_ROWS ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[set][a], fx[set][c], acc[a][c], 0, 0, 0)
+                                       : __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[set][c], fw[set][a], acc[a][c], 0, 0, 0);
+        };
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(Tile::COUNT_VARIES ? 0 : (SLABS - 1) * Tile::NL) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        read(0, nxt, 0);
-        fetch(s + SLABS, cur);
-        mul(1);
-        __builtin_amdgcn_sched_barrier(0);
-        cur = nxt;
-    }
+        read(0, 0, 0);
+        int cur = 0;
+        for (int s = 0; s < slabs; s++) {
+            const int nxt = cur + SLAB == SLABS * SLAB ? 0 : cur + SLAB;
+            read(1, cur, 1);
+            mul(0);
+            __builtin_amdgcn_sched_barrier(0);
+            read(0, cur, 2);
+            mul(1);
+            __builtin_amdgcn_sched_barrier(0);
+            read(1, cur, 3);
+            mul(0);
+            __builtin_amdgcn_sched_barrier(0);
+            // the last quarter's operands are here: this wavefront is done with the slab's buffer; and slab s + 1 has landed
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((SLABS - 2) * Tile::NL) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            read(0, nxt, 0);
+            fetch(s + SLABS, cur);
+            mul(1);
+            __builtin_amdgcn_sched_barrier(0);
+            cur = nxt;
+        }
+    };
+    if (mine >= FX) all(std::integral_constant<int, FX>{});
+    else if (FX > 4 && mine == 4) all(std::integral_constant<int, (FX > 4 ? 4 : 0)>{});
+    else if (FX > 3 && mine == 3) all(std::integral_constant<int, (FX > 3 ? 3 : 0)>{});
+    else if (FX > 2 && mine == 2) all(std::integral_constant<int, (FX > 2 ? 2 : 0)>{});
+    else if (mine == 1) all(std::integral_constant<int, 1>{});
+    else all(std::integral_constant<int, 0>{}); // its requests only
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // no LDS-direct load outlives the workgroup's LDS
-    const int nb = n0 + ww * FW * 32, mb = row0 + wx * FX * 32, h4 = 4 * (lane >> 5);
+    const int nb = n0 + ww * FW * 32, mb = row0 + c0 * 32, h4 = 4 * (lane >> 5);
 #pragma unroll
     for (int a = 0; a < FW; a++)
 #pragma unroll
         for (int c = 0; c < FX; c++) {
+            if (c >= mine) break;
             if (EPI == FH_GEMM_SWIGLU) { // rows 0 .. 15 of a tile are gates, 16 .. 31 the same outputs' up rows
 #pragma unroll
                 for (int q = 0; q < 2; q++) {
@@ -327,7 +350,9 @@ static fh_status gemm_wide(fh_device *dev, int epi, const FhGemm &g) {
     switch (epi) {
     case FH_GEMM_F32: WIDE_GO(FH_GEMM_F32); break;
     case FH_GEMM_ACT: WIDE_GO(FH_GEMM_ACT); break;
-    case FH_GEMM_ACT_T: WIDE_GO(FH_GEMM_ACT_T); break;
+    case FH_GEMM_ACT_T: // (never grouped)
+        if constexpr (TX != 320) WIDE_GO(FH_GEMM_ACT_T);
+        break;
     case FH_GEMM_RELU2: WIDE_GO(FH_GEMM_RELU2); break;
     default: WIDE_GO(FH_GEMM_SWIGLU); break;
     }
@@ -417,7 +442,7 @@ fh_status fh_gemm(fh_device *dev, int dtype, int epi, const FhGemm &g) {
     FH_REQUIRE(g.w && g.x && g.y && g.n > 0 && g.kp > 0 && g.kp % 64 == 0, "bad product");
     FH_REQUIRE(g.tiles ? g.max_tiles > 0 && g.n_tiles : g.m > 0, "product without rows");
     FH_REQUIRE(epi != FH_GEMM_SWIGLU || g.n % 32 == 0, "gate and up rows come in groups of 16");
-    FH_REQUIRE(!g.tiles || g.tile_rows == 64 || (g.tile_rows == 128 && dtype != FH_F32), "row tiles of %d", g.tile_rows);
+    FH_REQUIRE(!g.tiles || g.tile_rows == 64 || (g.tile_rows >= 128 && g.tile_rows <= 320 && g.tile_rows % 32 == 0 && dtype != FH_F32), "row tiles of %d", g.tile_rows);
     FH_REQUIRE(epi != FH_GEMM_ACT_T || !g.tiles, "a grouped product has no transposed form");
     hipStream_t s = dev->stream;
 #define FH_GEMM_EPI(K_, GRID_)                                              \
@@ -442,6 +467,7 @@ fh_status fh_gemm(fh_device *dev, int dtype, int epi, const FhGemm &g) {
         // this line and 7.2 / 4.7 / 3.4 ms without the kernel.  matmul_kernel = 3: never, 4: always where its row tiles fit, 14: the form with
         // 128 activation rows.
         const int64_t opt = dev->opt_matmul_kernel;
+        if (g.tiles && g.tile_rows > 128) return gemm_wide<320>(dev, epi, g);
         if (opt != 3) {
             // A round of workgroups with 128 activation rows takes two thirds of one with 256 (67 / 101 us at 4096 columns), so they
             // are the better ones where the tiles of 256 just miss a round: 14336 x 4096, 1025 rows 139 / 202 us (128 x 128: 156).
@@ -801,11 +827,8 @@ fh_status fh_head_rows(fh_device *dev, const float *x, int k, const float *w, fl
 
 // ------------------------------------------------------------------------------ residual streams normed at a sublayer's end
 __global__ void k_group_tiles(int groups, int s, int tile_rows, FhTile *tiles, int *n_tiles) {
-    const int per = (s + tile_rows - 1) / tile_rows;
-    for (int i = threadIdx.x; i < groups * per; i += blockDim.x) {
-        const int g = i / per, r = i % per * tile_rows;
-        tiles[i] = FhTile{g, g * s + r, s - r < tile_rows ? s - r : tile_rows, 0};
-    }
+    const int per = fh_tiles_of(s, tile_rows);
+    for (int i = threadIdx.x; i < groups * per; i += blockDim.x) tiles[i] = fh_tile(i / per, i / per * s, s, i % per, tile_rows);
     if (threadIdx.x == 0) *n_tiles = groups * per;
 }
 

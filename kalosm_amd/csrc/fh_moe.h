@@ -28,9 +28,15 @@ struct FhMoeWork {
     void *s_act;    // [t, sffp]
     float *s_y;     // [t, width]
 };
-// rows per tile: the larger ones where an expert has rows to fill them on average
-static inline int fh_moe_tile_rows(const FhMoe &m, int dtype, int s) {
-    return dtype != FH_F32 && (int64_t)s * m.top >= (int64_t)m.experts * 96 ? 128 : 64;
+// rows per tile: the larger ones where an expert has rows to fill them on average.  Of more than 128 rows an expert is one tile of up to
+// 320, so that its weights cross into the LDS once; with fewer there is nothing to save, and with few tiles the compute units
+// share out better by 128.  32 experts of 4096 x 4096 / 4096 x 2048, top 4, tiles of 320 (and of 128): 1800 tokens 281 / 177 us (331 / 193),
+// 1300 tokens 250 / 161 (282 / 176), 1000 tokens 236 / 153 (243 / 148).
+static inline int fh_moe_tile_rows(const fh_device *dev, const FhMoe &m, int dtype, int s, int width) {
+    const int64_t opt = dev->opt_matmul_kernel, rows = (int64_t)s * m.top, narrow = 2 * m.ffp < width ? 2 * m.ffp : width;
+    const bool tall = rows >= (int64_t)m.experts * 144 && m.experts * ((narrow + 255) / 256) >= dev->compute_units;
+    if (dtype != FH_F32 && opt != 3 && opt != 14 && (opt == 4 || tall)) return 320;
+    return dtype != FH_F32 && rows >= (int64_t)m.experts * 96 ? 128 : 64;
 }
 static inline int fh_moe_max_tiles(const FhMoe &m, int s, int tile_rows) { return s * m.top / tile_rows + m.experts; }
 // x [s, width] += mix [s, width] + the feed-forward of the activation rows h [s, kp]

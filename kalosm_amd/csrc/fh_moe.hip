@@ -28,14 +28,14 @@ __global__ __launch_bounds__(1024) void k_moe_sort(FhMoe m, const int *__restric
             start[e] = at;
             tstart[e] = tt;
             at += count[e];
-            tt += (count[e] + tile_rows - 1) / tile_rows;
+            tt += fh_tiles_of(count[e], tile_rows);
         }
         *n_tiles = tt;
     }
     __syncthreads();
     for (int e = tid; e < m.experts; e += 1024)
-        for (int i = 0, o = 0; o < count[e]; i++, o += tile_rows)
-            tiles[tstart[e] + i] = FhTile{e, start[e] + o, count[e] - o < tile_rows ? count[e] - o : tile_rows, 0};
+        for (int i = 0, of = fh_tiles_of(count[e], tile_rows); i < of; i++)
+            tiles[tstart[e] + i] = fh_tile(e, start[e], count[e], i, tile_rows);
     __syncthreads();
     for (int e = tid; e < m.experts; e += 1024) count[e] = 0;
     __syncthreads();
@@ -73,7 +73,7 @@ fh_status fh_moe_prefill(fh_device *dev, int dtype, const FhMoe &m, const void *
                          int s, int width, const FhMoeWork &w, const float *mix, float *x) {
     hipStream_t str = dev->stream;
     if (m.experts) {
-        const int tr = fh_moe_tile_rows(m, dtype, s);
+        const int tr = fh_moe_tile_rows(dev, m, dtype, s, width);
         k_moe_route<<<dim3((unsigned)((s + 3) / 4)), 256, 0, str>>>(m, proj, ldp, s, w.ids, w.wts);
         k_moe_sort<<<dim3(1), 1024, 0, str>>>(m, w.ids, s, tr, w.src, w.inv, w.tiles, w.n_tiles);
         FH_HIP(hipGetLastError());

@@ -54,3 +54,25 @@ def test_layers_agree(dev, option):
         finally:
             dev.set_option("matmul_kernel", 0)
         assert np.sqrt(np.mean((got - want) ** 2)) <= 2.7e-2 * np.sqrt(np.mean(want * want))
+
+
+@pytest.mark.parametrize("experts", [3, 5])
+@pytest.mark.parametrize("tokens", [31, 65, 160, 300, 511])
+def test_grouped_tiles(dev, tokens, experts):
+    """Groups of a few to 320 rows a tile, past that shared out evenly (option 4), against tiles of 128 rows (option 14): an output is the
+    same chain of products over k in both, so that they agree bit by bit."""
+    from kalosm_amd import bench_hybrid
+    from kalosm_amd.hybrid import HybridModel
+
+    small = dict(width=512, heads=4, experts=experts, top=2, ff=192, window=128, groups=2)
+    for cfg in (bench_hybrid.config(vocab=512, **small), bench_hybrid.zovovik_config(512, 4, 1024, 128, vocab=512)):
+        m = HybridModel.random_init(dev, cfg, ctx=512)
+        ids, got = np.random.default_rng(tokens).integers(0, 512, tokens), {}
+        try:
+            for option in (14, 4):
+                m.reset()
+                dev.set_option("matmul_kernel", option)
+                got[option] = m.forward(ids, want=range(tokens - 20, tokens))
+        finally:
+            dev.set_option("matmul_kernel", 0)
+        np.testing.assert_array_equal(got[4], got[14])

@@ -219,12 +219,18 @@ __global__ __launch_bounds__(256) void k_rec_out(FhRecurrent r, const float *__r
 //   S <- e^C_63 S + sum_s (e^(C_63 - C_s) k_s) v_s^T
 // No exponent may be positive, or fast decays would overflow: blocks of M below the diagonal ones split theirs at the start
 // of the row block, the diagonal blocks are summed pair by pair.
-// The second walks the chunks with 16 columns of a head's state per workgroup: U = U0 - W S.  All products are
+// The second walks the chunks with 16 columns of a head's state per workgroup: U = U0 - W S; the decays' exponentials come from
+// the first as well.  All products are
 // v_mfma_f32_16x16x4_f32; a lane takes four neighbouring k of an operand row at a time, on both sides alike.
+// The first launch leaves M, W, Q and K^T in the order in which the lanes of the second take them (rec_at), so that a request is a
+// whole kilobyte.  Row by row it was 16 rows of 64 bytes with neighbouring lanes in different rows, and the address unit, a lane a
+// cycle, was what bounded the scan (7900 of 12900 cycles a chunk): 2048 tokens, 32 heads of 128 x 128 delta rule 118 us (190 before),
+// 128 heads of 128 x 64 state space 152 (270), 16 heads of 256 x 256 retention 155 (233), 64 heads of 64 x 64 channel decay 65 (73).
 struct RecChunks { // scratch of one portion
     float *m, *w, *u0; // per (chunk, head): [64][64], [64][dp], [64][vp]
     float *kt;         // per (chunk, key head): [dp][64]
-    float *q, *f;      // channel decay, per (chunk, head): [64][dp] queries with the decay from the chunk's start, [dp] that of the chunk
+    float *q;          // per (chunk, key head): [64][dp]; channel decay: per head, with the decay from the chunk's start
+    float *f;          // per (chunk, head): e^c_t, then e^(c_63 - c_t) [2][64]; channel decay: that of the chunk [dp]
     int dp, vp, n;     // vp: vdim rounded up to 16, n: chunks
 };
 static RecChunks rec_chunks(const FhRecurrent &r, int s, float *p) {
@@ -233,13 +239,15 @@ static RecChunks rec_chunks(const FhRecurrent &r, int s, float *p) {
     const size_t hc = (size_t)c.n * r.heads;
     c.m = p, p += hc * 4096;
     c.kt = p, p += (size_t)c.n * r.kv_heads * c.dp * 64;
+    c.q = p, p += (size_t)c.n * (r.kind == FH_REC_CHANNEL ? r.heads : r.kv_heads) * 64 * c.dp;
     if (r.delta()) c.w = p, p += hc * 64 * c.dp, c.u0 = p;
-    if (r.kind == FH_REC_CHANNEL) c.q = p, p += hc * 64 * c.dp, c.f = p;
+    c.f = r.delta() ? c.u0 + hc * 64 * c.vp : p;
     return c;
 }
 size_t fh_rec_chunk_floats(const FhRecurrent &r, int s) {
     const RecChunks c = rec_chunks(r, s, nullptr);
-    return (size_t)c.n * ((size_t)r.heads * (4096 + (r.delta() ? 64 * (c.dp + c.vp) : r.kind == FH_REC_CHANNEL ? 65 * c.dp : 0)) + (size_t)r.kv_heads * c.dp * 64);
+    return (size_t)c.n * ((size_t)r.heads * (4096 + (r.kind == FH_REC_CHANNEL ? 65 * c.dp : r.delta() ? 64 * (c.dp + c.vp) + 128 : 128)) +
+                         (size_t)r.kv_heads * c.dp * (r.kind == FH_REC_CHANNEL ? 64 : 128));
 }
 
 __device__ __forceinline__ fh_f4 mma4(const float4 &a, const float4 &b, fh_f4 c) { // 16 of k
@@ -247,6 +255,12 @@ __device__ __forceinline__ fh_f4 mma4(const float4 &a, const float4 &b, fh_f4 c)
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
+}
+// Place of element (row, k) of an operand of kb blocks of 16 k: the four neighbouring k of a lane, lanes 16 (k % 16 / 4) + row % 16, k blocks, row blocks.
+__device__ __forceinline__ int rec_at(int row, int k, int kb) { return ((row / 16 * kb + k / 16) * 64 + k % 16 / 4 * 16 + row % 16) * 4 + k % 4; }
+// Piece i (four values) of such an operand: its row and first k.
+__device__ __forceinline__ void rec_piece(int i, int kb, int &row, int &k) {
+    row = i / 64 / kb * 16 + i % 16, k = i / 64 % kb * 16 + i % 64 / 16 * 4;
 }
 // Running sum of la over the 64 tokens of a chunk (one wavefront; tokens past the end change nothing).
 __device__ __forceinline__ float rec_decay_sum(const FhRecWork &w, int t, int s, int heads, int h) {
@@ -274,7 +288,10 @@ __global__ __launch_bounds__(256) void k_rec_chunk_prep(FhRecurrent r, FhRecWork
         *(float4 *)(sq + t * LD + x) = t0 + t < s ? *(const float4 *)(w.q + o) : z;
     }
     if (wave == 0) {
-        cs[lane] = rec_decay_sum(w, t0 + lane, s, r.heads, h);
+        const float sum = rec_decay_sum(w, t0 + lane, s, r.heads, h), end = __shfl(sum, 63, 64);
+        float *f = c.f + ((int64_t)ch * r.heads + h) * 128 + lane;
+        cs[lane] = sum;
+        f[0] = expf(sum), f[64] = expf(end - sum);
         be[lane] = t0 + lane < s ? w.beta[(int64_t)(t0 + lane) * r.heads + h] : 0.f;
     }
     __syncthreads();
@@ -295,12 +312,20 @@ __global__ __launch_bounds__(256) void k_rec_chunk_prep(FhRecurrent r, FhRecWork
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int t = 16 * wave + 4 * g + e, u = 16 * b + li;
-            mo[t * 64 + u] = u <= t ? expf(cs[t] - cs[u]) * qk[e] : 0.f;
+            mo[rec_at(t, u, 4)] = u <= t ? expf(cs[t] - cs[u]) * qk[e] : 0.f;
         }
     }
     if (h % rep == 0) {
-        float *kt = c.kt + ((int64_t)ch * r.kv_heads + kh) * DP * 64;
-        for (int i = tid; i < DP * 64; i += 256) kt[i] = sk[(i & 63) * LD + (i >> 6)];
+        const int64_t o = ((int64_t)ch * r.kv_heads + kh) * DP * 64;
+        float4 *kt = (float4 *)(c.kt + o), *qo = (float4 *)(c.q + o);
+        for (int i = tid; i < DP * 16; i += 256) {
+            int row, k;
+            rec_piece(i, 4, row, k);
+            const float *p = sk + k * LD + row;
+            kt[i] = make_float4(p[0], p[LD], p[2 * LD], p[3 * LD]);
+            rec_piece(i, DP / 16, row, k);
+            qo[i] = *(const float4 *)(sq + row * LD + k);
+        }
     }
     if (!DELTA) return;
     __syncthreads(); // Q has been read
@@ -339,10 +364,17 @@ __global__ __launch_bounds__(256) void k_rec_chunk_prep(FhRecurrent r, FhRecWork
             }
             x[t] = a;
         }
-        float *dst = j < DP ? c.w + hc * 64 * DP + j : c.u0 + hc * 64 * c.vp + j - DP;
-        const int st = j < DP ? DP : c.vp;
+        float *dst = j < DP ? sk + j : c.u0 + hc * 64 * c.vp + j - DP; // (column j of K has been read, by this thread)
+        const int st = j < DP ? LD : c.vp;
 #pragma unroll
         for (int t = 0; t < 64; t++) dst[t * st] = x[t];
+    }
+    __syncthreads();
+    float4 *wo = (float4 *)(c.w + hc * 64 * DP);
+    for (int i = tid; i < DP * 16; i += 256) {
+        int row, k;
+        rec_piece(i, DP / 16, row, k);
+        wo[i] = *(const float4 *)(sk + row * LD + k);
     }
 }
 
@@ -417,7 +449,7 @@ __global__ __launch_bounds__(256) void k_rec_channel_prep(FhRecurrent r, FhRecRo
     for (int b = 0; b < 3; b++) {
         if (b >= wave) break;
 #pragma unroll
-        for (int e = 0; e < 4; e++) mo[(16 * wave + 4 * g + e) * 64 + 16 * b + li] = off[b][e];
+        for (int e = 0; e < 4; e++) mo[rec_at(16 * wave + 4 * g + e, 16 * b + li, 4)] = off[b][e];
     }
 #pragma unroll
     for (int e = 0; e < 4; e++) {
@@ -434,15 +466,20 @@ __global__ __launch_bounds__(256) void k_rec_channel_prep(FhRecurrent r, FhRecRo
                 }
                 a = fmaf(q.x * k.x, f.x, fmaf(q.y * k.y, f.y, fmaf(q.z * k.z, f.z, fmaf(q.w * k.w, f.w, a))));
             }
-        mo[t * 64 + u] = a;
+        mo[rec_at(t, u, 4)] = a;
     }
-    for (int i = tid; i < 64 * DP; i += 256) {
-        const int t = i / DP, x = i % DP;
-        c.q[(hc * 64 + t) * DP + x] = sq[t * LD + x] * rec_exp2(blocks(0, t / 16, x) + sc[(t / 16 * 17 + t % 16) * LD + x]);
-    }
-    for (int i = tid; i < DP * 64; i += 256) {
-        const int t = i & 63, x = i >> 6;
-        c.kt[hc * DP * 64 + i] = sk[t * LD + x] * rec_exp2(rest(t / 16, t % 16 + 1, x) + blocks(t / 16 + 1, 4, x));
+    float4 *qo = (float4 *)(c.q + hc * 64 * DP), *kt = (float4 *)(c.kt + hc * DP * 64);
+    for (int i = tid; i < 16 * DP; i += 256) {
+        int t, x;
+        rec_piece(i, DP / 16, t, x);
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = sq[t * LD + x + e] * rec_exp2(blocks(0, t / 16, x + e) + sc[(t / 16 * 17 + t % 16) * LD + x + e]);
+        qo[i] = make_float4(v[0], v[1], v[2], v[3]);
+        rec_piece(i, 4, x, t);
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = sk[(t + e) * LD + x] * rec_exp2(rest(t / 16, t % 16 + e + 1, x) + blocks(t / 16 + 1, 4, x));
+        kt[i] = make_float4(v[0], v[1], v[2], v[3]);
     }
     for (int x = tid; x < DP; x += 256) c.f[hc * DP + x] = rec_exp2(blocks(0, 4, x));
 }
@@ -455,7 +492,7 @@ __global__ __launch_bounds__(256, 1) void k_rec_chunk_scan(FhRecurrent r, FhRecW
     constexpr bool DELTA = KIND == FH_REC_DELTA, CHANNEL = KIND == FH_REC_CHANNEL;
     constexpr int ST = DP / 64 > 0 ? DP / 64 : 1, SL = DP + 4, UL = 68; // state tiles of a wavefront
     constexpr int SW = DP / 16 / ST;                                    // wavefronts with state rows
-    __shared__ __attribute__((aligned(16))) float ss[16 * SL], su[16 * UL], sd[16 * UL], cs[2][64];
+    __shared__ __attribute__((aligned(16))) float ss[16 * SL], su[16 * UL], sd[16 * UL];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, g = lane >> 4;
     // The column blocks of a head read the same operands: they go to one of the eight dies, whose L2 then serves all but one
     // (workgroups are dealt to the dies in turn).
@@ -475,30 +512,30 @@ __global__ __launch_bounds__(256, 1) void k_rec_chunk_scan(FhRecurrent r, FhRecW
     const float skip = r.d_skip ? r.d_skip[h] : 0.f;
     struct Ops { // a lane's operands of one chunk
         float4 w[DELTA ? DP / 16 : 1], q[DP / 16], m[4], kt[ST][4];
-        float u[4], v[4], la;
-        float4 f[CHANNEL ? ST : 1];
+        float u[4], v[4], all;
+        float4 f[CHANNEL ? ST : 2];
     } o0, o1;
     // No branches around the requests: the number in flight is then known at compile time, so that waiting for one chunk's
     // operands does not wait for the next one's.  Places outside the portion read a valid address instead.
     auto load = [&](Ops &o, int ch) {
         const int64_t hc = (int64_t)ch * r.heads + h;
-        const int t = ch * 64 + 16 * wave + li, tq = t < s ? t : s - 1; // rows past the end are multiplied by zeros of M and decays
         if (DELTA) {
-            const float *wp = c.w + (hc * 64 + 16 * wave + li) * DP + 4 * g;
+            const float *wp = c.w + (hc * 64 + 16 * wave) * DP + 4 * lane;
 #pragma unroll
-            for (int x = 0; x < DP / 16; x++) o.w[x] = *(const float4 *)(wp + 16 * x);
+            for (int x = 0; x < DP / 16; x++) o.w[x] = *(const float4 *)(wp + 256 * x);
         }
-        const float *qp = (CHANNEL ? c.q + (hc * 64 + 16 * wave + li) * DP : w.q + ((int64_t)tq * r.kv_heads + kh) * DP) + 4 * g;
+        const int64_t kc = CHANNEL ? hc : (int64_t)ch * r.kv_heads + kh;
+        const float *qp = c.q + (kc * 64 + 16 * wave) * DP + 4 * lane; // rows past the end are zeros
 #pragma unroll
-        for (int x = 0; x < DP / 16; x++) o.q[x] = *(const float4 *)(qp + 16 * x);
-        const float *mp = c.m + hc * 4096 + (16 * wave + li) * 64 + 4 * g;
+        for (int x = 0; x < DP / 16; x++) o.q[x] = *(const float4 *)(qp + 256 * x);
+        const float *mp = c.m + hc * 4096 + wave * 1024 + 4 * lane;
 #pragma unroll
-        for (int b = 0; b < 4; b++) o.m[b] = *(const float4 *)(mp + 16 * b); // blocks behind the diagonal are never used
-        const float *kp = c.kt + (((int64_t)ch * r.kv_heads + kh) * DP + (owner ? wave : 0) * ST * 16 + li) * 64 + 4 * g;
+        for (int b = 0; b < 4; b++) o.m[b] = *(const float4 *)(mp + 256 * b); // blocks behind the diagonal are never used
+        const float *kp = c.kt + (((int64_t)ch * r.kv_heads + kh) * DP + (owner ? wave : 0) * ST * 16) * 64 + 4 * lane;
 #pragma unroll
         for (int i = 0; i < ST; i++)
 #pragma unroll
-            for (int b = 0; b < 4; b++) o.kt[i][b] = *(const float4 *)(kp + i * 1024 + 16 * b);
+            for (int b = 0; b < 4; b++) o.kt[i][b] = *(const float4 *)(kp + i * 1024 + 256 * b);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int row = 16 * wave + 4 * g + e, tt = ch * 64 + row < s ? ch * 64 + row : s - 1;
@@ -512,31 +549,30 @@ __global__ __launch_bounds__(256, 1) void k_rec_chunk_scan(FhRecurrent r, FhRecW
         if (CHANNEL)
 #pragma unroll
             for (int i = 0; i < ST; i++) o.f[i] = *(const float4 *)(c.f + hc * DP + (owner ? wave : 0) * ST * 16 + i * 16 + 4 * g);
-        else o.la = w.la[(int64_t)(ch * 64 + lane < s ? ch * 64 + lane : s - 1) * r.heads + h];
+        else {
+            const float *fp = c.f + hc * 128;
+            o.f[0] = *(const float4 *)(fp + 16 * wave + 4 * g), o.f[CHANNEL ? 0 : 1] = *(const float4 *)(fp + 64 + 16 * wave + 4 * g);
+            o.all = fp[63];
+        }
     };
     auto step = [&](const Ops &o, int ch) {
-        float *c_ = cs[ch & 1];
-        if (!CHANNEL && wave == 0) {
-            float v = ch * 64 + lane < s ? o.la : 0.f;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const float u = __shfl_up(v, d, 64);
-                if (lane >= d) v += u;
-            }
-            c_[lane] = v;
-        }
         if (owner)
 #pragma unroll
             for (int i = 0; i < ST; i++) *(fh_f4 *)(ss + li * SL + (wave * ST + i) * 16 + 4 * g) = S[i];
-        __syncthreads(); // state and decays are there; U of the chunk before has been read
+        __syncthreads(); // the state is there; U of the chunk before has been read
         fh_f4 ws = fh_f4{0.f, 0.f, 0.f, 0.f}, qs = ws;
+        constexpr int AHEAD = DELTA && DP > 128 ? 1 : 2; // operands read that many products early (with 2 the widest spills more)
+        float4 sb[DP / 16];
+#pragma unroll
+        for (int x = 0; x < AHEAD; x++) sb[x] = *(const float4 *)(ss + li * SL + 16 * x + 4 * g);
 #pragma unroll
         for (int x = 0; x < DP / 16; x++) {
-            const float4 b = *(const float4 *)(ss + li * SL + 16 * x + 4 * g);
-            if (DELTA) ws = mma4(o.w[x], b, ws);
-            qs = mma4(o.q[x], b, qs);
+            if (x + AHEAD < DP / 16) sb[x + AHEAD < DP / 16 ? x + AHEAD : 0] = *(const float4 *)(ss + li * SL + 16 * (x + AHEAD) + 4 * g);
+            __builtin_amdgcn_sched_barrier(0);
+            if (DELTA) ws = mma4(o.w[x], sb[x], ws);
+            qs = mma4(o.q[x], sb[x], qs);
         }
-        const float end = CHANNEL ? 0.f : c_[63];
+        const fh_f4 ec = fh_f4{o.f[0].x, o.f[0].y, o.f[0].z, o.f[0].w}, ed = fh_f4{o.f[CHANNEL ? 0 : 1].x, o.f[CHANNEL ? 0 : 1].y, o.f[CHANNEL ? 0 : 1].z, o.f[CHANNEL ? 0 : 1].w};
         fh_f4 u, ud, out;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -545,26 +581,31 @@ __global__ __launch_bounds__(256, 1) void k_rec_chunk_scan(FhRecurrent r, FhRecW
                 out[e] = qs[e];
                 continue;
             }
-            const float ct = c_[16 * wave + 4 * g + e];
             u[e] = DELTA ? o.u[e] - ws[e] : ch * 64 + 16 * wave + 4 * g + e < s ? o.u[e] * o.v[e] : 0.f;
-            ud[e] = expf(end - ct) * u[e];
-            out[e] = expf(ct) * qs[e];
+            ud[e] = ed[e] * u[e];
+            out[e] = ec[e] * qs[e];
         }
         *(fh_f4 *)(su + li * UL + 16 * wave + 4 * g) = u;
         if (!CHANNEL) *(fh_f4 *)(sd + li * UL + 16 * wave + 4 * g) = ud;
         __syncthreads();
+        const float *su_ = CHANNEL ? su : sd;
+        float4 ub[4];
 #pragma unroll
-        for (int b = 0; b < 4; b++)
-            if (b <= wave) out = mma4(o.m[b], *(const float4 *)(su + li * UL + 16 * b + 4 * g), out);
-        const float f = CHANNEL ? 1.f : expf(end), *su_ = CHANNEL ? su : sd;
+        for (int b = 0; b < 4; b++) ub[b] = *(const float4 *)(su_ + li * UL + 16 * b + 4 * g);
         if (owner)
 #pragma unroll
             for (int i = 0; i < ST; i++) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) S[i][e] *= !CHANNEL ? f : e == 0 ? o.f[i].x : e == 1 ? o.f[i].y : e == 2 ? o.f[i].z : o.f[i].w;
+                for (int e = 0; e < 4; e++) S[i][e] *= !CHANNEL ? o.all : e == 0 ? o.f[i].x : e == 1 ? o.f[i].y : e == 2 ? o.f[i].z : o.f[i].w;
 #pragma unroll
-                for (int b = 0; b < 4; b++) S[i] = mma4(o.kt[i][b], *(const float4 *)(su_ + li * UL + 16 * b + 4 * g), S[i]);
+                for (int b = 0; b < 4; b++) S[i] = mma4(o.kt[i][b], ub[b], S[i]);
             }
+        if (!CHANNEL)
+#pragma unroll
+            for (int b = 0; b < 4; b++) ub[b] = *(const float4 *)(su + li * UL + 16 * b + 4 * g);
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+            if (b <= wave) out = mma4(o.m[b], ub[b], out);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int tt = ch * 64 + 16 * wave + 4 * g + e;

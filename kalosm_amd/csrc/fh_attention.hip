@@ -359,7 +359,7 @@ extern "C" fh_status fh_flash_attention_ex(fh_device *dev, int32_t q_dtype, int3
     // through its split-operand form, which keeps f32 accuracy; attn_kernel = 2 asks for plain f16 rounding)
     if (sq >= 32 && dev->opt_attn_kernel != 1 && mask_kind != FH_MASK_BATCH_KEY) {
         fh_status st = fh_attention_prefill_mfma(dev, q_dtype, kv_dtype, q_dev, q_sb, q_sh, q_st, k_dev, v_dev, kv_sb, kv_sh,
-                                                 kv_st, b, hq, hkv, sq, skv, d, scale, mask_kind, out_dev);
+                                                 kv_st, b, hq, hkv, sq, skv, d, scale, mask_kind, false, out_dev);
         if (st != FH_ERR_UNSUPPORTED) return st;
     }
 #define FH_ATTN_ARGS dev, q_dev, q_sb, q_sh, q_st, k_dev, v_dev, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, d, scale, mask_kind, mask_dev, out_dev

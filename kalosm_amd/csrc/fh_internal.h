@@ -258,7 +258,7 @@ fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *
 fh_status fh_attention_prefill_mfma(fh_device *dev, int q_dtype, int kv_dtype, const void *q, int64_t q_sb,
                                     int64_t q_sh, int64_t q_st, const void *k, const void *v, int64_t kv_sb,
                                     int64_t kv_sh, int64_t kv_st, int b, int hq, int hkv, int sq, int skv, int d,
-                                    float scale, int mask_kind, void *out);
+                                    float scale, int mask_kind, bool by_row, void *out);
 fh_status fh_launch_q6k_m1_acc(const fh_qmatrix *q, const float *x, const float *xup, float *y_inout, const float *add);
 fh_status fh_launch_q6k_m1(const fh_qmatrix *q, const float *x, float *y, int epi, const float *a, const float *b);
 

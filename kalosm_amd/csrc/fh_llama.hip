@@ -373,7 +373,7 @@ fh_status fh_llama::layers(int s, bool dev_pos) {
         fh_llama_layer &l = m->layer[li];
         // Decode steps fold each rms_norm into the matvec that consumes it (one launch instead of two).
         const bool fuse = dev_pos && s == 1 && dev->opt_fuse_norm == 0 && dev->opt_matvec_kernel == 0;
-        bool qkv_done = false, wo_done = false, xacc = false;
+        bool qkv_done = false, wo_done = false, xacc = false, in_rows = false; // in_rows: att_t holds the attention's [s, H * hd]
         bool rope_done = false;
         if (fuse && l.qkv && l.qkv->type == FH_Q4_K) {
             // norm + projection + rope + cache append in one launch; without the rope epilogue as second choice
@@ -444,14 +444,21 @@ fh_status fh_llama::layers(int s, bool dev_pos) {
             FH_TRY(fh_kvcache_append_kv(m->cache, li, m->krot, (int64_t)s * hd, hd, vp, hd, k_st, s, pos));
             size_t plane = (size_t)HK * m->cache->capacity * hd * fh_dtype_size(c.kv_dtype);
             const uint8_t *kc = (const uint8_t *)m->cache->k + li * plane, *vc = (const uint8_t *)m->cache->v + li * plane;
-            FH_TRY(fh_flash_attention_ex(dev, FH_F32, c.kv_dtype, m->qrot, 0, (int64_t)s * hd, hd, kc, vc, 0,
-                                         (int64_t)m->cache->capacity * hd, hd, 1, H, HK, s, pos + s, hd, scale,
-                                         s > 1 ? FH_MASK_CAUSAL : FH_MASK_NONE, nullptr, m->att));
+            const int64_t cap = (int64_t)m->cache->capacity * hd;
+            if (s >= 32 && dev->opt_attn_kernel != 1) { // as fh_flash_attention_ex chooses, straight into the rows of the next product
+                fh_status st = fh_attention_prefill_mfma(dev, FH_F32, c.kv_dtype, m->qrot, 0, (int64_t)s * hd, hd, kc, vc, 0, cap, hd, 1, H, HK, s,
+                                                         pos + s, hd, scale, FH_MASK_CAUSAL, true, m->att_t);
+                if (st != FH_ERR_UNSUPPORTED) FH_TRY(st);
+                in_rows = st == FH_OK;
+            }
+            if (!in_rows)
+                FH_TRY(fh_flash_attention_ex(dev, FH_F32, c.kv_dtype, m->qrot, 0, (int64_t)s * hd, hd, kc, vc, 0, cap, hd, 1, H, HK, s, pos + s, hd,
+                                             scale, s > 1 ? FH_MASK_CAUSAL : FH_MASK_NONE, nullptr, m->att));
         }
         if (trace) FH_TRY(trace_mark(m, 2, li, "rope+cache+attention"));
         const float *att_in = m->att; // [H, s, hd]; for s == 1 this already is [s, H*hd]
         if (s > 1) {
-            FH_TRY(fh_transpose_shd(dev, m->att, H, s, hd, m->att_t));
+            if (!in_rows) FH_TRY(fh_transpose_shd(dev, m->att, H, s, hd, m->att_t));
             att_in = m->att_t;
         }
         if (!wo_done) FH_TRY(fh_qmatmul_prompt(l.wo, att_in, s, m->attn_out));

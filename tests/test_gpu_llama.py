@@ -478,3 +478,28 @@ def test_trace_switches_from_the_environment():
     env = {k: v for k, v in env.items() if k not in ("FUSOR_TRACE_GPU_KERNELS", "KALOSM_TRACE_LAYER_NAN")}
     r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "TEXT 0" in r.stdout and "[timing]" not in r.stderr
+
+
+@pytest.mark.parametrize("n", [31, 32, 33, 129, 240])
+@pytest.mark.parametrize("kv_dtype", ["f32", "f16"])
+@pytest.mark.parametrize("cfg", [SMALL, HD128], ids=["hd64", "hd128"])
+def test_prompt_lengths(dev, oracle, cfg, kv_dtype, n):
+    """From 32 rows on the attention writes the rows of the next product itself; query blocks exactly full and one row past that.  f32 keys against
+    the checker.  f16 keys against the kernel of one row a workgroup (attn_kernel = 1) on the same cache: queries and weights rounded to
+    f16 move scores of up to 30 by 30 x 2^-10 and the sums by as much of themselves, 2^-5 in the norm; a row in a wrong place moves it by order one."""
+    m, ref = build_pair(dev, oracle, cfg, kv_dtype=kv_dtype)
+    prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n)
+    parts = (prompt, prompt[:5])  # a few more rows behind it read the cache
+    got = [m.forward(p) for p in parts]
+    if kv_dtype == "f32":
+        for g, p in zip(got, parts):
+            assert_close(g, ref.forward(p), what="prompt")
+        return
+    m.reset()
+    dev.set_option("attn_kernel", 1)
+    try:
+        want = [m.forward(p) for p in parts]
+    finally:
+        dev.set_option("attn_kernel", 0)
+    for g, w in zip(got, want):
+        assert np.linalg.norm(g - w) <= 2.0 ** -5 * np.linalg.norm(w)

@@ -35,3 +35,17 @@ def check(dev, cfg, seed):
             got = m.forward(toks[at:at + n], want=places)
             assert G.rel_err(got, want[at + np.array(places)]).max() <= 3e-5, (sizes, at)
             at += n
+
+
+@pytest.mark.parametrize("layer", [G.mamba2(4, 64, 16, 1, 1, 2), G.mamba2(3, 85, 16, 1, 1, 2), G.mamba2(5, 104, 16, 1, 2, 2), G.mamba2(2, 129, 16, 1, 1, 2),
+                                   G.delta(2, 1, 16, 256, 2), G.delta(2, 1, 16, 252, 2)], ids=["256", "255", "2x260", "258", "2x256", "2x252"])
+def test_normed_groups(dev, layer):
+    """The gated norm of the outputs, four channels a thread for groups of 256 and more in fours: gate ahead of the norm and behind it, lanes
+    that stand idle at a group's end."""
+    cfg = G.config([G.with_mlp(layer, None)], 64, 50)
+    w = G.weights(cfg)
+    toks = np.random.default_rng(8).integers(0, 50, 70)
+    want, _ = R.forward(cfg, w, toks)
+    for dtype, tol in (("float32", 3e-5), ("bfloat16", 4e-2)):
+        got = G.build(dev, cfg, w, dtype).forward(toks, want=range(70))
+        assert G.rel_err(got, want).max() <= tol

@@ -722,7 +722,10 @@ static fh_status ap_launch(fh_device *dev, const void *q, int64_t q_sb, int64_t 
                 return d == 128 ? ap_launch_ahead<TQ, 128, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out)
                                 : ap_launch_ahead<TQ, 64, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out);
             if (halves) return d == 128 ? FH_AH(128, 2) : FH_AH(64, 2);
-            if (!pair) return d == 128 ? FH_AH(128, 1) : FH_AH(64, 1);
+            // up to two key tiles a query there is little to overlap, and the longer code costs more than it gives (32 / 8 heads of 128:
+            // 65 tokens 6.74 us for 6.55, 128 tokens 7.85 for 7.71; from 129 on, in two key groups, 7.5 for 8.4)
+            if (!pair && (skv > 128 || force == 8)) return d == 128 ? FH_AH(128, 1) : FH_AH(64, 1);
+            if (!pair) return d == 128 ? FH_AP(128, 1, 1) : FH_AP(64, 1, 1);
 #undef FH_AH
             return d == 128 ? FH_AP(128, 2, 1) : FH_AP(64, 2, 1);
         } else {

@@ -17,10 +17,12 @@
 // group, so a SIMD runs one wavefront's chain of a step instead of two.
 // What bounds the loop (measured per stage): the first product is matrix-core bound, the softmax vector-ALU bound
 // (both wavefronts of a SIMD are in it together) and the second product bound by the transposing LDS loads, which
-// run at half the rate of plain 16-byte loads.  So the softmax is kept to what a score needs (140 vector instructions for a wavefront's 2048; with
+// run at half the rate of plain 16-byte loads.  So the softmax is kept to what a score needs (some 160 vector instructions for a wavefront's 2048; with
 // address arithmetic for the requests, cleared accumulators and output rescaled in most tiles they were 310): a request is a buffer load from a
-// descriptor that moves with the tile, the denominator is added up in pairs from the rounded weights, and split operands, whose weights
-// lose nothing by it, move their reference only where a maximum is 2^8 above it.  Rows of V are 64 bytes apart in the banks, so that the 16
+// descriptor that moves with the tile, and split operands, whose weights lose nothing by it, move their reference only where a maximum is 2^8
+// above it.  The denominator is the sum of the f32 weights, whatever the products take them as: weights below 2^-25 of the largest are zero in f16, and
+// many of them still count (16384 keys 2^25.5 below one: 3.5e-4 of the output).  (Added up in pairs from the rounded weights it saved 16 of the
+// instructions and no time: 2048 tokens 51.9 us against 52.0.)  Rows of V are 64 bytes apart in the banks, so that the 16
 // lanes of a transposing load cover them once.  Heads that share a workgroup (four wavefronts each) are half a step apart, one in the softmax while
 // the other multiplies.  f16, 32 / 8 heads of 128, causal, before and after: 1024 tokens 25.3 / 23.7 us, 2048 53.4 / 50.8, 4096 166 / 151, 8192
 // 616 / 558 (985 TFLOP/s); f32 2048 129 / 125, 4096 400 / 350.
@@ -42,7 +44,6 @@
 // 190 with each pair requested in front of its products; 16 / 4 heads of 64, 3000 tokens 102 / 107).
 #include "fh_blocks.h"
 
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
@@ -394,17 +395,15 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
                 fh_half t[8], tl[8];
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-                    const float p = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + e], sc2, m_sub)); // arguments <= 0
+                    const float p = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + e], sc2, m_sub)); // arguments <= 0, split operands <= 8 (weights up to 2^8)
+                    ps += p;
                     t[e] = (fh_half)p;
-                    if constexpr (SPLIT) ps += p, tl[e] = (fh_half)(p - (float)t[e]);
+                    if constexpr (SPLIT) tl[e] = (fh_half)(p - (float)t[e]);
                 }
-                if constexpr (!SPLIT) // the denominator is the sum of what is multiplied, so that their roundings go together
-#pragma unroll
-                    for (int e = 0; e < 8; e += 2) ps = __builtin_amdgcn_fdot2(half2v{t[e], t[e + 1]}, half2v{(fh_half)1.f, (fh_half)1.f}, ps, false);
                 __builtin_memcpy(&pb[kt][s2], t, 16);
                 if constexpr (SPLIT) __builtin_memcpy(&pl[kt][s2], tl, 16);
             }
-        l_run = l_run * alpha + ps; // (of this lane's keys)
+        l_run = l_run * alpha + (SPLIT ? ps : ap_swap32_sum(ps)); // (split operands: of this lane's keys)
         // ---- O^T = O^T * alpha + V^T . P^T
         __builtin_amdgcn_sched_barrier(0);
         if (APART) {
@@ -469,7 +468,7 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
         else __syncthreads(); // tile t+1 is staged, and nobody reads this tile's buffer any more
     }
     if (APART && head == 0) bar(); // (as many barriers as the other)
-    l_run = ap_swap32_sum(l_run);
+    if constexpr (SPLIT) l_run = ap_swap32_sum(l_run);
     if constexpr (KS == 2) {
         ap_merge<D, QW>((float *)ap_lds, wave, lane, kset, m_run, l_run, acc);
         if (kset == 1) return;
@@ -600,24 +599,28 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(QW
         __builtin_amdgcn_sched_barrier(0);
         if (!last) scores(it + 1, next);
         half8 pb[2][2];
+        float ps = 0.f;
 #pragma unroll
         for (int kt = 0; kt < 2; kt++)
 #pragma unroll
             for (int s2 = 0; s2 < 2; s2++) {
                 fh_half t[8];
 #pragma unroll
-                for (int e = 0; e < 8; e++) t[e] = (fh_half)__builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + e], sc2, m_sub)); // arguments <= 0
-#pragma unroll
-                for (int e = 0; e < 8; e += 2) l_run = __builtin_amdgcn_fdot2(half2v{t[e], t[e + 1]}, half2v{(fh_half)1.f, (fh_half)1.f}, l_run, false);
+                for (int e = 0; e < 8; e++) {
+                    const float p = __builtin_amdgcn_exp2f(fmaf(st[kt][8 * s2 + e], sc2, m_sub)); // arguments <= 0
+                    ps += p;
+                    t[e] = (fh_half)p;
+                }
                 __builtin_memcpy(&pb[kt][s2], t, 16);
             }
+        l_run += ap_swap32_sum(ps);
         if (!last) {
             __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
             for (int i = 0; i < 2 * KSTEPS; i++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 if (i < 2 * KSTEPS - 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 64 / (2 * KSTEPS), 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 80 / (2 * KSTEPS), 0);
                 __builtin_amdgcn_sched_group_barrier(0x400, 32 / (2 * KSTEPS), 0);
             }
         }
@@ -663,7 +666,6 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(QW
         } else
             step(t, sa, sb, true);
     }
-    l_run = ap_swap32_sum(l_run);
     if constexpr (KS == 2) ap_merge<D, QW>((float *)ap_lds, wave, lane, kset, m_run, l_run, acc);
     if (KS == 2 && kset == 1) return;
     if (qi < sq) ap_store<D>(out + (by_row ? ((int64_t)bi * sq + qi) * hq + h : ((int64_t)bi * hq + h) * sq + qi) * D, g, 1.0f / l_run, acc);

@@ -71,3 +71,28 @@ def test_reference_of_the_exponents(dev, dtype, shape, steps):
     # subnormal weights, and what is left of them for the second operand of f32, are multiples of 2^-24: each is off by up to 2^-25, s of them
     tol = (2.0 ** -10 * np.abs(want).max() if dtype == "f16" else 2.0 ** -20 * (2 + top)) + s * 2.0 ** -25
     assert np.abs(got - want).max() <= tol, np.abs(got - want).max()
+
+
+@pytest.mark.parametrize("shape", [0, 6, 7, 8, 9])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("below", [25.5, 24.6])
+@pytest.mark.parametrize("dtype,s", [("f32", 16384), ("f16", 131072)])
+def test_denominator_of_small_weights(dev, dtype, s, below, d, shape):
+    """f16 keys, one of them ahead of all others by 2^25.5 or 2^24.6: weights that f16 rounds to zero, or to 2^-24.  They are in the denominator as they are;
+    values of 1 and -1 in turn take them out of the numerator, exactly.  Left are the roundings of a sum between 1 and 2, 2^-24 a tile of 64 keys, of
+    exponents and outputs.  Weights rounded ahead of the sum move it by 1.6e-4 (s = 16384, where 1.7e-5 are allowed) and 1.3e-3 (6.1e-4) at least."""
+    q, k, v = (np.zeros((1, n, m, d), np.float16) for n, m in ((4, 64), (2, s), (2, s)))
+    q[..., 0] = 1.0
+    k[..., 0] = np.float16(-below * np.log(2.0))
+    k[0, :, 3, 0] = 0.0
+    v[..., 0::2, :], v[..., 1::2, :] = 1.0, -1.0
+    v[0, :, 2, :], v[0, :, 3, :] = 0.0, 0.75  # (and the leading key's neighbour, so that as many are 1 as are -1)
+    tail = (s - 1) * np.exp(float(k[0, 0, 0, 0]))
+    qt, kt, vt = Tensor.from_slice(dev, q.astype(np.float32) if dtype == "f32" else q, dtype), Tensor.from_slice(dev, k, "f16"), Tensor.from_slice(dev, v, "f16")
+    dev.set_option("attn_kernel", shape)
+    try:
+        got = qt.flash_attention(kt, vt, 1.0).as_slice().astype(np.float64)
+    finally:
+        dev.set_option("attn_kernel", 0)
+    want = 0.75 / (1.0 + tail)
+    assert np.abs(got - want).max() <= want * (s / 64 * 2.0 ** -24 + 2.0 ** -20 + (2.0 ** -11 if dtype == "f16" else 0)), (got.max() / want - 1, got.min() / want - 1)

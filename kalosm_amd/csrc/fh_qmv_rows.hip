@@ -38,30 +38,45 @@ struct RowsX {
 
 // Four rows of a 256, one a row of 16 lanes: lane i has k 64 s + 4 i .. of its row in v[s].
 template <int T>
-__device__ __forceinline__ void rows_put(uint8_t *img, int row, int i, const float4 (&v)[4]) {
+__device__ __forceinline__ void rows_put(uint8_t *img, int row, int i, float4 (&v)[4]) {
     typedef RowsX<T> X;
-    float sc[X::OWN ? 4 : 1];
-    auto factor = [&](float top, float &up, float *back) {
-        int e = 141 - (int)((__float_as_uint(top) >> 23) & 0xFFu); // 14 - floor(log2 top); zero / inf / nan clamp
-        e = e > 100 ? 100 : (e < -100 ? -100 : e);
-        up = __uint_as_float((uint32_t)(e + 127) << 23);
-        if ((i & (X::OWN ? 7 : 15)) == 0) *back = __uint_as_float((uint32_t)(127 - e) << 23);
-    };
-    auto quads = [&](float t) { // of eight lanes
+    constexpr int NF = X::OWN ? 4 : 1;
+    float sc[NF], top[NF];
+    const bool first = (i & (X::OWN ? 7 : 15)) == 0; // of a factor's lanes
+    auto quads = [&](float t) {                      // of eight lanes
         t = fmaxf(t, rows_dpp<0xB1>(t));
         t = fmaxf(t, rows_dpp<0x4E>(t));
         return fmaxf(t, rows_dpp<0x141>(t));
     };
-    float *fac = (float *)(img + X::FAC_AT) + row;
+    float *fac = (float *)(img + X::FAC_AT) + row + (X::OWN ? (i >> 3) * 16 : 0);
     if constexpr (X::OWN) {
 #pragma unroll
-        for (int s = 0; s < 4; s++) factor(quads(rows_max(rows_max(0.f, v[s].x, v[s].y), v[s].z, v[s].w)), sc[s], fac + (2 * s + (i >> 3)) * 16);
+        for (int s = 0; s < 4; s++) top[s] = quads(rows_max(rows_max(0.f, v[s].x, v[s].y), v[s].z, v[s].w));
     } else {
-        float top = 0.f;
+        float t = 0.f;
 #pragma unroll
-        for (int s = 0; s < 4; s++) top = rows_max(rows_max(top, v[s].x, v[s].y), v[s].z, v[s].w);
-        top = quads(top);
-        factor(fmaxf(top, rows_dpp<0x140>(top)), sc[0], fac); // of sixteen
+        for (int s = 0; s < 4; s++) t = rows_max(rows_max(t, v[s].x, v[s].y), v[s].z, v[s].w);
+        t = quads(t);
+        top[0] = fmaxf(t, rows_dpp<0x140>(t)); // of sixteen
+    }
+    float most = top[0];
+#pragma unroll
+    for (int s = 0; s < NF; s++) {
+        int e = 141 - (int)((__float_as_uint(top[s]) >> 23) & 0xFFu); // 14 - floor(log2 top); zero / inf / nan clamp
+        e = e > 100 ? 100 : (e < -100 ? -100 : e);
+        sc[s] = __uint_as_float((uint32_t)(e + 127) << 23);
+        if (first) fac[s * 32] = __uint_as_float((uint32_t)(127 - e) << 23);
+        most = fmaxf(most, top[s]);
+    }
+    // An infinity is carried as +-2^15 with an infinite factor, so that the row's outputs are infinities of its weights' signs (its hi + lo would be a NaN).
+    // One branch for all values, out of the way: with one a quad of them launches of 512 x 2048 took 5 % longer.
+    if (__builtin_expect(__any(most == INFINITY), 0)) {
+        auto carry = [&](float &u) { u = fabsf(u) == INFINITY ? copysignf(0x1p115f, u) : u; }; // (times 2^-100)
+#pragma unroll
+        for (int s = 0; s < 4; s++) carry(v[s].x), carry(v[s].y), carry(v[s].z), carry(v[s].w);
+#pragma unroll
+        for (int s = 0; s < NF; s++)
+            if (first && top[s] == INFINITY) fac[s * 32] = INFINITY;
     }
     const int qi = i & 7, g = reg_order(T) == 2 ? qi & 3 : qi >> 1, half = reg_order(T) == 2 ? qi >> 2 : qi & 1;
     const int slot = (g * 16 + ((row + 4 * g) & 15)) * 16;

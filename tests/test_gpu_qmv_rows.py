@@ -108,3 +108,22 @@ def test_repeats_and_rows(dev, oracle, ty):
     assert not got[2].any() and not np.isfinite(got[3]).any() and np.isnan(got[4]).all()
     rest = [r for r in range(m) if r not in (2, 3, 4)]
     assert np.array_equal(got[rest], base[rest])
+
+
+@named
+@pytest.mark.parametrize("m,n,k,cut", [(5, 528, 256 * 13, 0), (12, 512, 2048, 0), (16, 130, 256, 9), (9, 272, 256 * 9, 2)])
+def test_infinities(dev, oracle, ty, m, n, k, cut):
+    """An infinite activation gives infinities of the sign of its weight, as f32 arithmetic does, and moves no other row."""
+    q, w = matrix(dev, oracle, ty, n, k)
+    x = synth.random_activation(m, k, seed=8)
+    at = {1: (7, np.inf), 3: (k - 1, -np.inf), 4: (k // 2 + 33, np.inf)}
+    with options(dev, matvec_direct=3 if cut else 0, matvec_tiles=cut):
+        base = Tensor.from_slice(dev, x).q_mat_mul(q).as_slice()
+        for row, (col, value) in at.items():
+            x[row, col] = value
+        got = Tensor.from_slice(dev, x).q_mat_mul(q).as_slice()
+    for row, (col, value) in at.items():
+        some = w[:, col] != 0  # (a weight of zero gives NaN)
+        assert some.any() and np.array_equal(got[row][some], np.sign(w[some, col]).astype(np.float32) * np.float32(value)), (row, got[row][:4])
+    rest = [r for r in range(m) if r not in at]
+    assert np.array_equal(got[rest], base[rest])

@@ -41,6 +41,9 @@ template <int T>
 __device__ __forceinline__ void rows_put(uint8_t *img, int row, int i, float4 (&v)[4]) {
     typedef RowsX<T> X;
     constexpr int NF = X::OWN ? 4 : 1;
+    // The largest power of two: per 32 its inverse times a scale (2^-24 and more) has to be a normal number.  Per 256 any value may be normalised; at 100, Q4_K's
+    // sums / 64 of activations of 1e-34 had lost so much that outputs were 3.8e-4 off (the kernels ahead of this one 1.4e-4, now 1.2e-7).
+    constexpr int MOST = X::OWN ? 100 : 126;
     float sc[NF], top[NF];
     const bool first = (i & (X::OWN ? 7 : 15)) == 0; // of a factor's lanes
     auto quads = [&](float t) {                      // of eight lanes
@@ -63,7 +66,7 @@ __device__ __forceinline__ void rows_put(uint8_t *img, int row, int i, float4 (&
 #pragma unroll
     for (int s = 0; s < NF; s++) {
         int e = 141 - (int)((__float_as_uint(top[s]) >> 23) & 0xFFu); // 14 - floor(log2 top); zero / inf / nan clamp
-        e = e > 100 ? 100 : (e < -100 ? -100 : e);
+        e = e > MOST ? MOST : (e < -100 ? -100 : e);
         sc[s] = __uint_as_float((uint32_t)(e + 127) << 23);
         if (first) fac[s * 32] = __uint_as_float((uint32_t)(127 - e) << 23);
         most = fmaxf(most, top[s]);

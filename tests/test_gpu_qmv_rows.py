@@ -127,3 +127,19 @@ def test_infinities(dev, oracle, ty, m, n, k, cut):
         assert some.any() and np.array_equal(got[row][some], np.sign(w[some, col]).astype(np.float32) * np.float32(value)), (row, got[row][:4])
     rest = [r for r in range(m) if r not in at]
     assert np.array_equal(got[rest], base[rest])
+
+
+@named
+@pytest.mark.parametrize("m,n,k", [(5, 528, 256 * 13), (16, 512, 2048)])
+@pytest.mark.parametrize("size", [1e-30, 1e-34, 1e-36])
+def test_tiny_rows(dev, oracle, ty, m, n, k, size):
+    """Rows of tiny activations keep their bits: a power of two per 256 reaches 2^126.  Per 32 of k it ends at 2^100, where half of the second operand's last
+    place is 2^-125 of an activation."""
+    q, w = matrix(dev, oracle, ty, n, k)
+    x = synth.random_activation(m, k, seed=9) * np.float32(size)
+    with options(dev, matvec_direct=3):
+        got = Tensor.from_slice(dev, x).q_mat_mul(q).as_slice().astype(np.float64)
+    if ty not in (synth.Q5_0, synth.Q5_K):
+        close(got, x, w)
+    x = x.astype(np.float64)
+    assert (np.abs(got - x @ w.T) <= 2.0 ** -19 * (np.abs(x) @ np.abs(w).T) + 2.0 ** -125 * np.abs(w).sum(1)).all()

@@ -48,14 +48,12 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ void ap_load8(const float *p, fh_half *o) {
-    const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 4);
-    o[0] = (fh_half)a.x; o[1] = (fh_half)a.y; o[2] = (fh_half)a.z; o[3] = (fh_half)a.w;
-    o[4] = (fh_half)b.x; o[5] = (fh_half)b.y; o[6] = (fh_half)b.z; o[7] = (fh_half)b.w;
+    float x[8];
+    __builtin_memcpy(x, p, 32);
+#pragma unroll
+    for (int e = 0; e < 8; e++) o[e] = (fh_half)x[e];
 }
-__device__ __forceinline__ void ap_load8(const fh_half *p, fh_half *o) {
-    const uint4 r = *(const uint4 *)p;
-    __builtin_memcpy(o, &r, 16);
-}
+__device__ __forceinline__ void ap_load8(const fh_half *p, fh_half *o) { __builtin_memcpy(o, p, 16); } // (any address)
 // 16 bytes of a buffer, zeros past its end
 __device__ __forceinline__ uint4 ap_buffer16(__amdgpu_buffer_rsrc_t b, int offset) {
     const auto u = __builtin_amdgcn_raw_buffer_load_b128(b, offset, 0, 0);
@@ -136,7 +134,8 @@ __device__ __forceinline__ void ap_store(TQ *op, int g, float inv, const floatx1
                       acc[dt][4 * r4 + 3] * inv);
 }
 
-template <typename TQ, typename TKV, int D, bool SPLIT = false, int HW = 1, int KS = 1, int QW = 4>
+// ANY: K and V through plain loads of 64-bit addresses instead of buffer requests, for views that those do not take (fh_attention_prefill_mfma).
+template <typename TQ, typename TKV, int D, bool SPLIT = false, int HW = 1, int KS = 1, int QW = 4, bool ANY = false>
 __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_eu(QW == 4 && !(SPLIT && D == 128 && HW == 1) ? 2 : 1, SPLIT && D == 128 && HW == 1 ? 1 : 2))) void k_attn_prefill(const TQ *__restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_st,
                                                        const TKV *__restrict__ k, const TKV *__restrict__ v,
                                                        int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int hq, int hkv,
@@ -210,6 +209,24 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
         piece[i] = c / CH * row_bytes + 8 * (c % CH) * (int)sizeof(TKV); // key 0 .. KS * BN - 1: the KS tiles of a step
     }
     auto fetch = [&](int t0) {
+        if constexpr (ANY) { // (rows past the last key repeat it)
+#pragma unroll
+            for (int i = 0; i < NCH; i++) {
+                const int c = tid + NTH * i, row = t0 + c / CH;
+                const int64_t at = (int64_t)(row < skv ? row : skv - 1) * kv_st + 8 * (c % CH);
+                if constexpr (SPLIT) {
+                    __builtin_memcpy(&kraw[2 * i], kb + at, 32);
+                    __builtin_memcpy(&vraw[2 * i], vb + at, 32);
+                } else {
+                    fh_half t[16];
+                    ap_load8(kb + at, t);
+                    ap_load8(vb + at, t + 8);
+                    __builtin_memcpy(&kreg[i], t, 16);
+                    __builtin_memcpy(&vreg[i], t + 8, 16);
+                }
+            }
+            return;
+        }
         const int64_t end = (int64_t)(skv - t0 - 1) * row_bytes + D * (int)sizeof(TKV);
         const int bytes = end < 0x7FFFFFFF ? (int)end : 0x7FFFFFFF;
         const auto bk = __builtin_amdgcn_make_buffer_rsrc((void *)(kb + t0 * kv_st), 0, bytes, 0x00027000);
@@ -671,14 +688,14 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(QW
     if (qi < sq) ap_store<D>(out + (by_row ? ((int64_t)bi * sq + qi) * hq + h : ((int64_t)bi * hq + h) * sq + qi) * D, g, 1.0f / l_run, acc);
 }
 
-template <typename TQ, typename TKV, int D, bool SPLIT, int HW, int KS = 1, int QW = 4>
+template <typename TQ, typename TKV, int D, bool SPLIT, int HW, int KS = 1, int QW = 4, bool ANY = false>
 static fh_status ap_launch_k(fh_device *dev, const void *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void *k,
                              const void *v, int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int b, int hq, int hkv, int sq,
                              int skv, float scale, int causal, int by_row, void *out) {
     constexpr int LDS = 2 * KS * (SPLIT ? 2 : 1) * 64 * (D + 8 + D + 32) * 2; // two buffers of KS tiles (K and V planes), bytes
     static_assert(KS == 1 || LDS >= (2 + (D / 32) * 16) * 256 * 4, "the merge of the key groups reuses the tile buffers");
     static_assert(LDS <= 160 * 1024, "KV tiles exceed the LDS of a compute unit");
-    auto kern = k_attn_prefill<TQ, TKV, D, SPLIT, HW, KS, QW>;
+    auto kern = k_attn_prefill<TQ, TKV, D, SPLIT, HW, KS, QW, ANY>;
     FH_TRY(fh_kernel_lds(dev, (const void *)kern, LDS)); // allow more than 64 KB of dynamic LDS
     dim3 grid((unsigned)(hq / HW), (unsigned)((sq + 32 * QW - 1) / (32 * QW)), (unsigned)b);
     kern<<<grid, 64 * QW * HW * KS, LDS, dev->stream>>>((const TQ *)q, q_sb, q_sh, q_st, (const TKV *)k, (const TKV *)v, kv_sb,
@@ -709,7 +726,11 @@ static fh_status ap_launch(fh_device *dev, const void *q, int64_t q_sb, int64_t 
     // with two key groups) whatever the size: tests
     const int64_t force = dev->opt_attn_kernel;
     const bool pair = (hq / hkv) % 2 == 0 && (force == 6 || (force != 7 && force != 8 && wgs >= 1024));
-#define FH_AP(D, HW, KS) ap_launch_k<TQ, TKV, D, SPLIT, HW, KS>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out)
+#define FH_AP(D, HW, KS, ...) ap_launch_k<TQ, TKV, D, SPLIT, HW, KS, ##__VA_ARGS__>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out)
+    // A request of 16 bytes, straight into LDS above all, is made for an address of its multiple, and a step's 128 rows lie within the 2^31 bytes
+    // of a buffer.  Other views are read as they lie by the plain form (32 / 8 heads of 128, causal, us: K and V of f16 one element off 149, aligned 55, a row a
+    // workgroup 8600; of f32 128, 134, 6400).
+    if (((uintptr_t)k | (uintptr_t)v) & 15 || kv_st < 0 || kv_st >= 1 << 21) return d == 128 ? FH_AP(128, 1, 1, 4, true) : FH_AP(64, 1, 1, 4, true);
     if constexpr (!SPLIT) {
         // short prompts: every workgroup is resident at once (two of four wavefronts per compute unit) and the launch
         // lasts as long as the last query block's - its key tiles are shared out over two groups of wavefronts
@@ -753,7 +774,6 @@ fh_status fh_attention_prefill_mfma(fh_device *dev, int q_dtype, int kv_dtype, c
     if ((d != 128 && d != 64) || hq % hkv || (mask_kind != FH_MASK_NONE && mask_kind != FH_MASK_CAUSAL)) return FH_ERR_UNSUPPORTED;
     if (q_st % 8 || q_sh % 8 || q_sb % 8 || kv_st % 8 || kv_sh % 8 || kv_sb % 8 || (sq + 127) / 128 > 65535 || b > 65535) return FH_ERR_UNSUPPORTED;
     if (mask_kind == FH_MASK_CAUSAL && skv < sq) return FH_ERR_UNSUPPORTED;
-    if (kv_st < 0 || kv_st >= 1 << 21) return FH_ERR_UNSUPPORTED; // a step's 128 rows lie within the 2^31 bytes of a buffer
     const int causal = mask_kind == FH_MASK_CAUSAL;
     if (q_dtype == FH_F16 && kv_dtype == FH_F16)
         return ap_launch<fh_half, fh_half>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, d, scale, causal, by_row, out);

@@ -3,6 +3,7 @@ reference of the exponents that moves late or never, and weights below the norma
 import numpy as np
 import pytest
 
+from kalosm_amd._lib import F16, F32, MASK_CAUSAL, check
 from kalosm_amd.fusor import MaskKind, Tensor
 
 pytestmark = pytest.mark.gpu
@@ -96,3 +97,34 @@ def test_denominator_of_small_weights(dev, dtype, s, below, d, shape):
         dev.set_option("attn_kernel", 0)
     want = 0.75 / (1.0 + tail)
     assert np.abs(got - want).max() <= want * (s / 64 * 2.0 ** -24 + 2.0 ** -20 + (2.0 ** -11 if dtype == "f16" else 0)), (got.max() / want - 1, got.min() / want - 1)
+
+
+@pytest.mark.parametrize("qt,kt", [("f32", "f16"), ("f16", "f16"), ("f32", "f32")])
+@pytest.mark.parametrize("view,t,s,d", [("odd", 33, 200, 128), ("odd", 129, 129, 64), ("odd", 70, 70, 128), ("back", 129, 129, 128), ("back", 40, 63, 64),
+                                        ("far", 33, 66, 64)])
+def test_views_of_any_address_and_stride(dev, view, qt, kt, t, s, d):
+    """K and V that begin one element behind an address of 16 bytes, whose positions run backwards, or are 2^21 elements apart, as a caller in C may pass them;
+    the elements around them are not finite."""
+    rng = np.random.default_rng(t + s + d)
+    q, k, v = (rng.standard_normal((1, n, m, d)).astype(np.float16 if ty == "f16" else np.float32) for n, m, ty in ((4, t, qt), (2, s, kt), (2, s, kt)))
+    q = q.astype(k.dtype).astype(q.dtype)
+    want = exact(q, k, v, d ** -0.5, True)
+    qd, out, size = Tensor.from_slice(dev, q, qt), Tensor(dev, q.shape, qt), k.itemsize
+    if view == "far": # both heads of K, then both of V, at each position
+        sh, st, held = d, 1 << 21, np.zeros((s, 1 << 21), k.dtype)
+        for i, a in enumerate((k, v)):
+            held[:, 2 * d * i:2 * d * (i + 1)] = a[0].transpose(1, 0, 2).reshape(s, 2 * d)
+        base = [Tensor.from_slice(dev, held, kt)]
+        ptr = [base[0].ptr, base[0].ptr + 2 * d * size]
+    else:
+        at, sh, st = 1 if view == "odd" else 0, s * d, d if view == "odd" else -d
+        base, ptr = [], []
+        for a in (k, v):
+            held = np.full(2 * s * d + 64, np.nan, k.dtype)
+            held[at:at + 2 * s * d] = (a if view == "odd" else a[:, :, ::-1]).reshape(-1)
+            base.append(Tensor.from_slice(dev, held, kt))
+            ptr.append(base[-1].ptr + (at if view == "odd" else (s - 1) * d) * size)
+    code = {"f32": F32, "f16": F16}
+    check(dev._lib.fh_flash_attention_ex(dev._h, code[qt], code[kt], qd.ptr, 4 * t * d, t * d, d, ptr[0], ptr[1], 0, sh, st, 1, 4, 2, t, s, d, d ** -0.5,
+                                         MASK_CAUSAL, None, out.ptr))
+    close(out.as_slice()[0].astype(np.float64), want, kt, 6)

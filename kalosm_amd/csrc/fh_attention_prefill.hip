@@ -395,10 +395,10 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
         // The reference of the exponents.  Split operands: it moves only where a maximum is more than 2^8 above it, so that the output is rescaled
         // in the first tiles and then hardly ever.  (Weights rounded to f16: where one key has most of the weight that is 1, exact; against 64 bits
         // 2048 tokens with scores of four times the usual spread 2.13e-4, with a reference of its own 2.25e-4.)
-        const bool move = __any(mx > m_run + (SPLIT ? 8.f : 0.f));
+        const bool moves = mx > m_run + (SPLIT ? 8.f : 0.f), move = __any(moves); // (each row's by its own scores, so that its bits do not depend on its neighbours)
         float alpha = 1.f;
         if (move) {
-            const float m_new = fmaxf(m_run, mx);
+            const float m_new = moves ? mx : m_run;
             alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new); // (nothing visible yet: only queries past the end)
             m_run = m_new;
         }

@@ -128,3 +128,18 @@ def test_views_of_any_address_and_stride(dev, view, qt, kt, t, s, d):
     check(dev._lib.fh_flash_attention_ex(dev._h, code[qt], code[kt], qd.ptr, 4 * t * d, t * d, d, ptr[0], ptr[1], 0, sh, st, 1, 4, 2, t, s, d, d ** -0.5,
                                          MASK_CAUSAL, None, out.ptr))
     close(out.as_slice()[0].astype(np.float64), want, kt, 6)
+
+
+@pytest.mark.parametrize("shape", [0, 6, 7, 8, 9])
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+def test_rows_are_their_own(dev, dtype, shape):
+    """A row's bits do not depend on what the rows beside it hold: not on scores of theirs that grow from tile to tile, not on infinities or NaN."""
+    rng = np.random.default_rng(9)
+    q, k, v = (rng.standard_normal((1, n, m, 128)).astype(np.float16 if dtype == "f16" else np.float32) for n, m in ((4, 70), (2, 700), (2, 700)))
+    base = run(dev, q, k, v, dtype, 128 ** -0.5, False, shape)
+    q[0, :, 5] *= 30
+    q[0, 1, 40, 3], q[0, 2, 41, 4] = np.inf, np.nan
+    got = run(dev, q, k, v, dtype, 128 ** -0.5, False, shape)
+    rest = [r for r in range(70) if r not in (5, 40, 41)]
+    assert np.array_equal(got[:, rest], base[:, rest])
+    assert not np.array_equal(got[:, 5], base[:, 5]) and np.isfinite(got[:, 5]).all() and np.isnan(got[2, 41]).all()

@@ -10,10 +10,11 @@
 // group supply 4 keys x 16 dims and receive, per lane, one dim of the 4 keys).  Two LDS buffers and one barrier per
 // tile: tile t+1 is written to the other buffer right after the first product of tile t (its LDS writes and the
 // request for tile t+2 then run under the softmax arithmetic).
-// KS = 2 (short prompts: fewer workgroups than the device holds, and the launch lasts as long as the workgroup of the
-// last query block): eight wavefronts per query block, the second four take every other key tile with running
-// statistics of their own, and the two halves are merged through LDS at the end - half the tile steps per workgroup.
-// QW = 2 (shorter still: every workgroup of 64 query rows finds a compute unit of its own): two wavefronts per key
+// KS = 2 (prompts whose workgroups are no more than two rounds): eight wavefronts per query block, the second four take every
+// other key tile with running statistics of their own, and the two halves are merged through LDS at the end - half the tile steps per
+// workgroup.  (k_attn_prefill has it for f32 operands rounded to f16 only, attn_kernel = 2.)
+// Of f16 keys and values k_attn_prefill has the launches of two heads a workgroup and those of at most 128 keys; all others are k_attn_ahead's.
+// QW = 2 (k_attn_ahead, shorter still: every workgroup of 64 query rows finds a compute unit of its own): two wavefronts per key
 // group, so a SIMD runs one wavefront's chain of a step instead of two.
 // What bounds the loop (measured per stage): the first product is matrix-core bound, the softmax vector-ALU bound
 // (both wavefronts of a SIMD are in it together) and the second product bound by the transposing LDS loads, which
@@ -135,20 +136,18 @@ __device__ __forceinline__ void ap_store(TQ *op, int g, float inv, const floatx1
 }
 
 // ANY: K and V through plain loads of 64-bit addresses instead of buffer requests, for views that those do not take (fh_attention_prefill_mfma).
-template <typename TQ, typename TKV, int D, bool SPLIT = false, int HW = 1, int KS = 1, int QW = 4, bool ANY = false>
-__global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_eu(QW == 4 && !(SPLIT && D == 128 && HW == 1) ? 2 : 1, SPLIT && D == 128 && HW == 1 ? 1 : 2))) void k_attn_prefill(const TQ *__restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_st,
+template <typename TQ, typename TKV, int D, bool SPLIT = false, int HW = 1, int KS = 1, bool ANY = false>
+__global__ __launch_bounds__(256 * HW * KS) __attribute__((amdgpu_waves_per_eu(SPLIT && D == 128 && HW == 1 ? 1 : 2, SPLIT && D == 128 && HW == 1 ? 1 : 2))) void k_attn_prefill(const TQ *__restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_st,
                                                        const TKV *__restrict__ k, const TKV *__restrict__ v,
                                                        int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int hq, int hkv,
                                                        int sq, int skv, float scale, int causal, int by_row, TQ *__restrict__ out) {
     constexpr int BN = 64, KS_ = D + 8, VS = D + 32, DT = D / 32, KSTEPS = D / 16, CH = D / 8; // CH: 8-element chunks per row
     constexpr int NP = SPLIT ? 2 : 1; // operand planes: hi (, lo)
     static_assert(HW * KS <= 2 && !(SPLIT && KS == 2), "eight wavefronts at most; split operands leave no room for two tiles");
-    static_assert(QW == 4 || (QW == 2 && HW == 1 && KS == 2), "query blocks of 128 rows, or of 64 with two key groups");
-    constexpr int QB = 32 * QW; // query rows of a workgroup: QW wavefronts of 32
-    constexpr int NTH = 64 * QW * HW * KS, KBUF = NP * BN * KS_, VBUF = NP * BN * VS, TILE = KBUF + VBUF; // halfs per staged tile
+    constexpr int QB = 128, NTH = 256 * HW * KS, KBUF = NP * BN * KS_, VBUF = NP * BN * VS, TILE = KBUF + VBUF; // halfs per staged tile
     extern __shared__ __attribute__((aligned(16))) fh_half ap_lds[]; // [2 buffers][K planes | V planes]
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 31, g = lane >> 5;
-    const int kset = KS == 2 ? wave / QW : 0; // which key tiles of a step this wavefront multiplies
+    const int kset = KS == 2 ? wave / 4 : 0; // which key tiles of a step this wavefront multiplies
     // The wavefronts of two heads are half a step apart: those of one are in the first product and the softmax while those of the other are in the
     // second product.
     constexpr bool APART = HW == 2;
@@ -157,7 +156,7 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
     // causal: the last query blocks see the most keys; with the block index on the slow grid axis ALL heads of the
     // longest block are dispatched first and the short blocks fill the tail
     const int qb0 = (causal ? (int)(gridDim.y - 1 - blockIdx.y) : (int)blockIdx.y) * QB;
-    const int qi = qb0 + (wave % QW) * 32 + li; // this lane's query row (KS = 2: both groups have the same rows)
+    const int qi = qb0 + (wave % 4) * 32 + li; // this lane's query row (KS = 2: both groups have the same rows)
     const int off = skv - sq;                  // causal: query i sees keys 0 .. i + off
     const TKV *kb = k + bi * kv_sb + kh * kv_sh, *vb = v + bi * kv_sb + kh * kv_sh;
 
@@ -308,7 +307,7 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
     const float ninf = -INFINITY;
     for (int ts = 0, it = 0; ts < kend; ts += KS * BN, it++) { // a step: KS tiles, one per group of four wavefronts
         const int t0 = ts + kset * BN;
-        // a group without a tile in the last step multiplies the staged rows (clamped, finite) with every key masked
+        // a group without a tile in the last step multiplies the staged rows (behind the last key: zeros) with every key masked
         const int lim_t = (KS == 1 || t0 < kend) ? lim : -1;
         const fh_half *sK = ap_lds + ((it & 1) * KS + kset) * TILE, *sV = sK + KBUF;
         // ---- S^T = K . Q^T for the two 32-key halves of the tile
@@ -487,7 +486,7 @@ __global__ __launch_bounds__(64 * QW * HW * KS) __attribute__((amdgpu_waves_per_
     if (APART && head == 0) bar(); // (as many barriers as the other)
     if constexpr (SPLIT) l_run = ap_swap32_sum(l_run);
     if constexpr (KS == 2) {
-        ap_merge<D, QW>((float *)ap_lds, wave, lane, kset, m_run, l_run, acc);
+        ap_merge<D, 4>((float *)ap_lds, wave, lane, kset, m_run, l_run, acc);
         if (kset == 1) return;
     }
     if (qi < sq) ap_store<D>(out + (by_row ? ((int64_t)bi * sq + qi) * hq + h : ((int64_t)bi * hq + h) * sq + qi) * D, g, 1.0f / l_run, acc);
@@ -688,17 +687,17 @@ __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(QW
     if (qi < sq) ap_store<D>(out + (by_row ? ((int64_t)bi * sq + qi) * hq + h : ((int64_t)bi * hq + h) * sq + qi) * D, g, 1.0f / l_run, acc);
 }
 
-template <typename TQ, typename TKV, int D, bool SPLIT, int HW, int KS = 1, int QW = 4, bool ANY = false>
+template <typename TQ, typename TKV, int D, bool SPLIT, int HW, int KS = 1, bool ANY = false>
 static fh_status ap_launch_k(fh_device *dev, const void *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void *k,
                              const void *v, int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int b, int hq, int hkv, int sq,
                              int skv, float scale, int causal, int by_row, void *out) {
     constexpr int LDS = 2 * KS * (SPLIT ? 2 : 1) * 64 * (D + 8 + D + 32) * 2; // two buffers of KS tiles (K and V planes), bytes
     static_assert(KS == 1 || LDS >= (2 + (D / 32) * 16) * 256 * 4, "the merge of the key groups reuses the tile buffers");
     static_assert(LDS <= 160 * 1024, "KV tiles exceed the LDS of a compute unit");
-    auto kern = k_attn_prefill<TQ, TKV, D, SPLIT, HW, KS, QW, ANY>;
+    auto kern = k_attn_prefill<TQ, TKV, D, SPLIT, HW, KS, ANY>;
     FH_TRY(fh_kernel_lds(dev, (const void *)kern, LDS)); // allow more than 64 KB of dynamic LDS
-    dim3 grid((unsigned)(hq / HW), (unsigned)((sq + 32 * QW - 1) / (32 * QW)), (unsigned)b);
-    kern<<<grid, 64 * QW * HW * KS, LDS, dev->stream>>>((const TQ *)q, q_sb, q_sh, q_st, (const TKV *)k, (const TKV *)v, kv_sb,
+    dim3 grid((unsigned)(hq / HW), (unsigned)((sq + 127) / 128), (unsigned)b);
+    kern<<<grid, 256 * HW * KS, LDS, dev->stream>>>((const TQ *)q, q_sb, q_sh, q_st, (const TKV *)k, (const TKV *)v, kv_sb,
                                                kv_sh, kv_st, hq, hkv, sq, skv, scale, causal, by_row, (TQ *)out);
     FH_HIP(hipGetLastError());
     return FH_OK;
@@ -730,16 +729,16 @@ static fh_status ap_launch(fh_device *dev, const void *q, int64_t q_sb, int64_t 
     // A request of 16 bytes, straight into LDS above all, is made for an address of its multiple, and a step's 128 rows lie within the 2^31 bytes
     // of a buffer.  Other views are read as they lie by the plain form (32 / 8 heads of 128, causal, us: K and V of f16 one element off 149, aligned 55, a row a
     // workgroup 8600; of f32 128, 134, 6400).
-    if (((uintptr_t)k | (uintptr_t)v) & 15 || kv_st < 0 || kv_st >= 1 << 21) return d == 128 ? FH_AP(128, 1, 1, 4, true) : FH_AP(64, 1, 1, 4, true);
+    if (((uintptr_t)k | (uintptr_t)v) & 15 || kv_st < 0 || kv_st >= 1 << 21) return d == 128 ? FH_AP(128, 1, 1, true) : FH_AP(64, 1, 1, true);
     if constexpr (!SPLIT) {
-        // short prompts: every workgroup is resident at once (two of four wavefronts per compute unit) and the launch
-        // lasts as long as the last query block's - its key tiles are shared out over two groups of wavefronts
+        // up to two rounds of workgroups (one a compute unit at a time: its tiles are 128 KB of LDS for head_dim 128), the longest first, so that a long and a short
+        // one follow each other: a workgroup's key tiles are shared out over two groups of wavefronts
         const bool halves = force == 7 || force == 9 || (force != 6 && force != 8 && wgs <= 2L * dev->compute_units && skv > 128);
-        // shorter still: query blocks of 64 rows, four wavefronts, while one workgroup per compute unit holds (nearly) all
-        // of them - a SIMD then runs one wavefront's chain of a step instead of two (512 tokens: 15.0 against 16.8 us)
-        const long wgs64 = (long)hq * ((sq + 63) / 64) * b;
-        const bool rows64 = force == 9 || (force == 0 && halves && 4 * wgs64 <= 5L * dev->compute_units);
         if constexpr (sizeof(TKV) == 2) {
+            // shorter still: query blocks of 64 rows, four wavefronts, while one workgroup per compute unit holds (nearly) all
+            // of them - a SIMD then runs one wavefront's chain of a step instead of two (512 tokens: 15.0 against 16.8 us)
+            const long wgs64 = (long)hq * ((sq + 63) / 64) * b;
+            const bool rows64 = force == 9 || (force == 0 && halves && 4 * wgs64 <= 5L * dev->compute_units);
 #define FH_AH(D, KS) ap_launch_ahead<TQ, D, KS>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out)
             if (rows64)
                 return d == 128 ? ap_launch_ahead<TQ, 128, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out)
@@ -752,8 +751,6 @@ static fh_status ap_launch(fh_device *dev, const void *q, int64_t q_sb, int64_t 
 #undef FH_AH
             return d == 128 ? FH_AP(128, 2, 1) : FH_AP(64, 2, 1);
         } else {
-            if (rows64) return d == 128 ? ap_launch_k<TQ, TKV, 128, SPLIT, 1, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out)
-                                        : ap_launch_k<TQ, TKV, 64, SPLIT, 1, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out);
             if (halves) return d == 128 ? FH_AP(128, 1, 2) : FH_AP(64, 1, 2);
         }
     }

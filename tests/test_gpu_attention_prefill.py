@@ -99,15 +99,16 @@ def test_denominator_of_small_weights(dev, dtype, s, below, d, shape):
     assert np.abs(got - want).max() <= want * (s / 64 * 2.0 ** -24 + 2.0 ** -20 + (2.0 ** -11 if dtype == "f16" else 0)), (got.max() / want - 1, got.min() / want - 1)
 
 
-@pytest.mark.parametrize("qt,kt", [("f32", "f16"), ("f16", "f16"), ("f32", "f32")])
+@pytest.mark.parametrize("qt,kt,kernel", [("f32", "f16", 0), ("f16", "f16", 0), ("f32", "f32", 0), ("f32", "f32", 2)])
 @pytest.mark.parametrize("view,t,s,d", [("odd", 33, 200, 128), ("odd", 129, 129, 64), ("odd", 70, 70, 128), ("back", 129, 129, 128), ("back", 40, 63, 64),
                                         ("far", 33, 66, 64)])
-def test_views_of_any_address_and_stride(dev, view, qt, kt, t, s, d):
+def test_views_of_any_address_and_stride(dev, view, qt, kt, kernel, t, s, d):
     """K and V that begin one element behind an address of 16 bytes, whose positions run backwards, or are 2^21 elements apart, as a caller in C may pass them;
     the elements around them are not finite."""
     rng = np.random.default_rng(t + s + d)
     q, k, v = (rng.standard_normal((1, n, m, d)).astype(np.float16 if ty == "f16" else np.float32) for n, m, ty in ((4, t, qt), (2, s, kt), (2, s, kt)))
-    q = q.astype(k.dtype).astype(q.dtype)
+    if kt == "f16" or kernel == 2:
+        q, k, v = (a.astype(np.float16).astype(a.dtype) for a in (q, k, v))
     want = exact(q, k, v, d ** -0.5, True)
     qd, out, size = Tensor.from_slice(dev, q, qt), Tensor(dev, q.shape, qt), k.itemsize
     if view == "far": # both heads of K, then both of V, at each position
@@ -125,9 +126,13 @@ def test_views_of_any_address_and_stride(dev, view, qt, kt, t, s, d):
             base.append(Tensor.from_slice(dev, held, kt))
             ptr.append(base[-1].ptr + (at if view == "odd" else (s - 1) * d) * size)
     code = {"f32": F32, "f16": F16}
-    check(dev._lib.fh_flash_attention_ex(dev._h, code[qt], code[kt], qd.ptr, 4 * t * d, t * d, d, ptr[0], ptr[1], 0, sh, st, 1, 4, 2, t, s, d, d ** -0.5,
-                                         MASK_CAUSAL, None, out.ptr))
-    close(out.as_slice()[0].astype(np.float64), want, kt, 6)
+    dev.set_option("attn_kernel", kernel)
+    try:
+        check(dev._lib.fh_flash_attention_ex(dev._h, code[qt], code[kt], qd.ptr, 4 * t * d, t * d, d, ptr[0], ptr[1], 0, sh, st, 1, 4, 2, t, s, d, d ** -0.5,
+                                             MASK_CAUSAL, None, out.ptr))
+    finally:
+        dev.set_option("attn_kernel", 0)
+    close(out.as_slice()[0].astype(np.float64), want, "f16" if kernel else kt, 6)
 
 
 @pytest.mark.parametrize("shape", [0, 6, 7, 8, 9])
@@ -143,3 +148,13 @@ def test_rows_are_their_own(dev, dtype, shape):
     rest = [r for r in range(70) if r not in (5, 40, 41)]
     assert np.array_equal(got[:, rest], base[:, rest])
     assert not np.array_equal(got[:, 5], base[:, 5]) and np.isfinite(got[:, 5]).all() and np.isnan(got[2, 41]).all()
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("t,s", [(33, 128), (33, 129), (129, 129), (200, 331), (128, 384)])
+def test_f32_rounded_to_f16(dev, t, s, d, causal):
+    """attn_kernel = 2: f32 operands rounded to f16, from 129 keys on in two key groups.  (Values of f16, so that the rounding changes none of them.)"""
+    rng = np.random.default_rng(t + s + d)
+    q, k, v = (rng.standard_normal((1, n, m, d)).astype(np.float16).astype(np.float32) for n, m in ((4, t), (2, s), (2, s)))
+    close(run(dev, q, k, v, "f32", d ** -0.5, causal, 2), exact(q, k, v, d ** -0.5, causal), "f16", 6)

@@ -269,7 +269,9 @@ static fh_status rows_go(const fh_qmatrix *q, const float *x, int m, float *y) {
 }
 
 // Row tiles a wavefront and 256s a workgroup: the least of a model fitted to 16 matrices in each format (us: of a launch, of a round of workgroups, of a
-// tile in it; the cut picked is 1 % slower than the best of the eight on average).
+// tile in it; of 128 - 11264 rows by 256 - 16384 columns the cut picked is 0.7 % slower than the best of the eight on average).  Up to four 256s there is nothing
+// for eight to a workgroup to do (512 x 1024 in Q6_K 5.5 us, by eight 6.5); more than four parts of four 256s cost what the last of a group reads (1408 x 16384 in
+// Q4_0, sixteen parts of two tiles 17.6 us, eight parts of eight 256s 11.1).
 struct RowsCut {
     int kc, tt;
     int64_t rounds;
@@ -281,11 +283,12 @@ static RowsCut rows_cut(const fh_qmatrix *q) {
                                        {{1.1, 2.6, 2.52}, {-1.0, 5.75, 1.67}}, {{1.3, 1.8, 4.5}, {-0.8, 5.6, 3.2}}, {{1.2, 2.1, 3.8}, {-1.2, 4.7, 3.3}}};
     const int type = q->type == FH_Q4_0 ? 0 : q->type == FH_Q5_0 ? 1 : q->type == FH_Q8_0 ? 2 : q->type == FH_Q4_K ? 3 : q->type == FH_Q5_K ? 4 : 5;
     RowsCut best{4, 1, 0, 1e30};
-    for (int kc = 4; kc <= 8; kc += 4)
+    for (int kc = 4; kc <= (chunks > 4 ? 8 : 4); kc += 4)
         for (int tt = 1; tt <= 4; tt++) {
             const double *c = of[type][kc == 8];
             const int64_t parts = (chunks + kc - 1) / kc, groups = (tiles * kc + 16 * tt - 1) / (16 * tt), rounds = (groups * parts + cus - 1) / cus;
-            const double us = c[0] + (parts > 1 ? (kc == 4 ? 1.0 : 2.3) : 0.0) + (double)rounds * (c[1] + c[2] * tt);
+            const double sum = parts == 1 ? 0.0 : kc == 8 ? 2.3 : 1.0 + 0.06 * tt * (double)(parts > 4 ? parts - 4 : 0);
+            const double us = c[0] + sum + (double)rounds * (c[1] + c[2] * tt);
             if (us < best.us) best = RowsCut{kc, tt, rounds, us};
         }
     return best;
@@ -301,15 +304,18 @@ bool fh_qmv_rows_supports(const fh_qmatrix *q, const float *x, int m) {
 // Where one round of workgroups does it, against what took the call (k_qb_prep and k_qmv_direct, 5-bit formats k_qmm_reg; of 480 products of 100 - 60000 rows and
 // 256 - 16384 columns).  In one round, 5 - 16 rows: Q4_0 0.76 of the time, Q4_K 0.83, Q5_0 0.76, Q5_K 0.80, Q6_K 0.82, Q8_0 0.80 (geometric means; 16 of 2048 x 8192
 // in Q4_K 12.8 / 8.5 us, 4096 x 11008 in Q6_K 26.2 / 20.9, 11008 x 4096 in Q8_0 21.6 / 15.4, 5 of 4096 x 4096 in Q5_K 15 / 10); in two
-// 0.94 - 1.24, for a workgroup's own phases do not overlap the next one's.  Level, and left to the other: Q4_K where that has four tiles a wavefront and k in one part (14336 x 4096
-// 15.4 / 15.8), and more than 24576 rows of few columns (10 of 30848 x 256 in Q6_K 9.3 / 10.0).  2 - 4 rows are the single-row kernel's row variant (4096 x 4096, four rows 6.8 / 8.6); Q6_K, which has none, from 3 rows on where there is
+// 0.94 - 1.24, for a workgroup's own phases do not overlap the next one's.  Level, and left to the other: Q4_K of five to seven 256s and few rows (512 x 1536 6.0 / 6.2), Q4_K where that has four tiles a wavefront and k in one part (14336 x 4096
+// 15.4 / 15.8), and more than 24576 rows of few columns (10 of 30848 x 256 in Q6_K 9.3 / 10.0), of 256
+// columns in Q6_K and Q8_0 more than 16384 (5 of 22528 x 256 7.3 / 8.5 and 6.2 / 6.7; of 16000 7.1 / 6.0 and 6.0 / 4.9).  2 - 4 rows are the single-row kernel's row variant (4096 x 4096, four rows 6.8 / 8.6); Q6_K, which has none, from 3 rows on where there is
 // one tile a wavefront (4096 x 4096 10.9 / 10.0, but 8192 x 3072 13.0 / 13.5).  Up to 65536 weights of the 5-bit formats stay although slower there, as the test of
 // k_qmm_reg's rule holds them to be its.
 bool fh_qmv_rows_pays(const fh_qmatrix *q, const float *x, int m) {
     if (!fh_qmv_rows_supports(q, x, m) || m < (q->type == FH_Q6_K ? 3 : 5)) return false;
     if ((q->type == FH_Q5_0 || q->type == FH_Q5_K) && q->n * q->k <= 65536) return false;
+    if (q->type == FH_Q4_K && q->k > 1024 && q->k < 2048 && q->n <= 2816) return false;
     if (q->type == FH_Q4_K && q->k <= 4096 && (q->n + 15) / 16 * 2 >= 7 * (int64_t)q->dev->compute_units) return false;
-    if ((q->n + 15) / 16 > 6 * (int64_t)q->dev->compute_units) return false;
+    const int64_t few = (q->type == FH_Q6_K || q->type == FH_Q8_0) && q->k <= 256 ? 4 : 6;
+    if ((q->n + 15) / 16 > few * q->dev->compute_units) return false;
     const RowsCut cut = rows_cut(q);
     return cut.rounds == 1 && (m >= 5 || cut.tt == 1);
 }

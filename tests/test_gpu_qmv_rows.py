@@ -62,6 +62,18 @@ def test_rule(dev, oracle, ty, m, n, k, taken):
     assert np.array_equal(auto, one) == taken
 
 
+@pytest.mark.parametrize("ty,m,n,k,cut", [(synth.Q4_K, 16, 512, 1536, 0), (synth.Q6_K, 5, 22528, 256, 0), (synth.Q8_0, 5, 22528, 256, 0),
+                                          (synth.Q4_0, 16, 1408, 16384, 8 + 2), (synth.Q6_K, 16, 512, 1024, 1)])
+def test_level_or_slower(dev, ty, m, n, k, cut):
+    """Products that stay with the kernels they had, for which one launch is level or slower (cut 0), and cuts that keep it quicker: many 256s in parts of
+    eight rather than in more parts of four, few of them four to a workgroup."""
+    q = QMatrix.from_raw_bytes(dev, (n, k), synth.random_weight(ty, n, k, seed=1), ty)
+    xt = Tensor.from_slice(dev, synth.random_activation(m, k, seed=2))
+    auto = xt.q_mat_mul(q).as_slice()
+    with options(dev, **(dict(matvec_direct=3, matvec_tiles=cut) if cut else dict(matvec_rows=1))):  # (any option of matvecs keeps it off the one launch)
+        assert np.array_equal(auto, xt.q_mat_mul(q).as_slice())
+
+
 @named
 def test_small_groups_beside_a_large_one(dev, oracle, ty):
     """Weights that are zero where the activations are large: the formats that normalise 32 values by themselves lose nothing of the small

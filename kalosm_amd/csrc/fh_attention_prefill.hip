@@ -23,7 +23,7 @@
 // descriptor that moves with the tile, and split operands, whose weights lose nothing by it, move their reference only where a maximum is 2^8
 // above it.  The denominator is the sum of the f32 weights, whatever the products take them as: weights below 2^-25 of the largest are zero in f16, and
 // many of them still count (16384 keys 2^25.5 below one: 3.5e-4 of the output).  (Added up in pairs from the rounded weights it saved 16 of the
-// instructions and no time: 2048 tokens 51.9 us against 52.0.)  Rows of V are 64 bytes apart in the banks, so that the 16
+// instructions and no time: 2048 tokens 51.9 us against 52.0.)  Rows of V are 64 bytes apart in the banks (ap_v_row), so that the 16
 // lanes of a transposing load cover them once.  Heads that share a workgroup (four wavefronts each) are half a step apart, one in the softmax while
 // the other multiplies.  f16, 32 / 8 heads of 128, causal, before and after: 1024 tokens 25.3 / 23.7 us, 2048 53.4 / 50.8, 4096 166 / 151, 8192
 // 616 / 558 (985 TFLOP/s); f32 2048 129 / 125, 4096 400 / 350.
@@ -124,6 +124,11 @@ __device__ __forceinline__ void ap_merge(float *sm, int wave, int lane, int kset
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[dt][r] = acc[dt][r] * f0 + sm[(2 + dt * 16 + r) * NQ + slot] * f1;
 }
+// Halfs of a row of V in LDS: 64 bytes past a multiple of the banks, or 32 where that many more would leave a compute unit one workgroup of split operands
+// instead of two (head_dim 64: 32 / 4 heads, causal, 3000 tokens 161 us with 64 bytes, 144 with 32).
+template <int D, bool SPLIT, int HW>
+constexpr int ap_v_row = SPLIT && D == 64 && HW == 1 ? D + 16 : D + 32;
+
 // lane = query, register r of d-tile dt is d = 32 dt + 8 (r / 4) + 4 g + r % 4
 template <int D, typename TQ>
 __device__ __forceinline__ void ap_store(TQ *op, int g, float inv, const floatx16 (&acc)[D / 32]) {
@@ -141,7 +146,7 @@ __global__ __launch_bounds__(256 * HW * KS) __attribute__((amdgpu_waves_per_eu(S
                                                        const TKV *__restrict__ k, const TKV *__restrict__ v,
                                                        int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int hq, int hkv,
                                                        int sq, int skv, float scale, int causal, int by_row, TQ *__restrict__ out) {
-    constexpr int BN = 64, KS_ = D + 8, VS = D + 32, DT = D / 32, KSTEPS = D / 16, CH = D / 8; // CH: 8-element chunks per row
+    constexpr int BN = 64, KS_ = D + 8, VS = ap_v_row<D, SPLIT, HW>, DT = D / 32, KSTEPS = D / 16, CH = D / 8; // CH: 8-element chunks per row
     constexpr int NP = SPLIT ? 2 : 1; // operand planes: hi (, lo)
     static_assert(HW * KS <= 2 && !(SPLIT && KS == 2), "eight wavefronts at most; split operands leave no room for two tiles");
     constexpr int QB = 128, NTH = 256 * HW * KS, KBUF = NP * BN * KS_, VBUF = NP * BN * VS, TILE = KBUF + VBUF; // halfs per staged tile
@@ -691,8 +696,9 @@ template <typename TQ, typename TKV, int D, bool SPLIT, int HW, int KS = 1, bool
 static fh_status ap_launch_k(fh_device *dev, const void *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void *k,
                              const void *v, int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int b, int hq, int hkv, int sq,
                              int skv, float scale, int causal, int by_row, void *out) {
-    constexpr int LDS = 2 * KS * (SPLIT ? 2 : 1) * 64 * (D + 8 + D + 32) * 2; // two buffers of KS tiles (K and V planes), bytes
+    constexpr int LDS = 2 * KS * (SPLIT ? 2 : 1) * 64 * (D + 8 + ap_v_row<D, SPLIT, HW>) * 2; // two buffers of KS tiles (K and V planes), bytes
     static_assert(KS == 1 || LDS >= (2 + (D / 32) * 16) * 256 * 4, "the merge of the key groups reuses the tile buffers");
+    static_assert(!(SPLIT && D == 64 && HW == 1) || 2 * LDS <= 160 * 1024, "two workgroups a compute unit");
     static_assert(LDS <= 160 * 1024, "KV tiles exceed the LDS of a compute unit");
     auto kern = k_attn_prefill<TQ, TKV, D, SPLIT, HW, KS, ANY>;
     FH_TRY(fh_kernel_lds(dev, (const void *)kern, LDS)); // allow more than 64 KB of dynamic LDS

@@ -269,9 +269,10 @@ static fh_status rows_go(const fh_qmatrix *q, const float *x, int m, float *y) {
 }
 
 // Row tiles a wavefront and 256s a workgroup: the least of a model fitted to 16 matrices in each format (us: of a launch, of a round of workgroups, of a
-// tile in it; of 128 - 11264 rows by 256 - 16384 columns the cut picked is 0.7 % slower than the best of the eight on average).  Up to four 256s there is nothing
-// for eight to a workgroup to do (512 x 1024 in Q6_K 5.5 us, by eight 6.5); more than four parts of four 256s cost what the last of a group reads (1408 x 16384 in
-// Q4_0, sixteen parts of two tiles 17.6 us, eight parts of eight 256s 11.1).
+// tile in it; of 128 - 11264 rows by 256 - 16384 columns the cut picked is 0.5 % slower than the best of the eight on average).  Up to four 256s there is nothing
+// for eight to a workgroup to do (512 x 1024 in Q6_K 5.5 us, by eight 6.5); more than four parts of four 256s cost what the last of a group reads, a
+// quarter of a microsecond a part and tile (1408 x 16384 in Q4_0, sixteen parts of two tiles 17.6 us, eight parts of eight 256s 11.1; 4096 x 11008 in Q4_K, eleven of
+// three tiles 18.8, six of eight 256s 15.4).
 struct RowsCut {
     int kc, tt;
     int64_t rounds;
@@ -287,7 +288,7 @@ static RowsCut rows_cut(const fh_qmatrix *q) {
         for (int tt = 1; tt <= 4; tt++) {
             const double *c = of[type][kc == 8];
             const int64_t parts = (chunks + kc - 1) / kc, groups = (tiles * kc + 16 * tt - 1) / (16 * tt), rounds = (groups * parts + cus - 1) / cus;
-            const double sum = parts == 1 ? 0.0 : kc == 8 ? 2.3 : 1.0 + 0.06 * tt * (double)(parts > 4 ? parts - 4 : 0);
+            const double sum = parts == 1 ? 0.0 : kc == 8 ? 2.3 : 1.0 + 0.07 * tt * tt * (double)(parts > 4 ? parts - 4 : 0);
             const double us = c[0] + sum + (double)rounds * (c[1] + c[2] * tt);
             if (us < best.us) best = RowsCut{kc, tt, rounds, us};
         }
@@ -301,22 +302,30 @@ bool fh_qmv_rows_supports(const fh_qmatrix *q, const float *x, int m) {
     }
     return false;
 }
-// Where one round of workgroups does it, against what took the call (k_qb_prep and k_qmv_direct, 5-bit formats k_qmm_reg; of 480 products of 100 - 60000 rows and
-// 256 - 16384 columns).  In one round, 5 - 16 rows: Q4_0 0.76 of the time, Q4_K 0.83, Q5_0 0.76, Q5_K 0.80, Q6_K 0.82, Q8_0 0.80 (geometric means; 16 of 2048 x 8192
-// in Q4_K 12.8 / 8.5 us, 4096 x 11008 in Q6_K 26.2 / 20.9, 11008 x 4096 in Q8_0 21.6 / 15.4, 5 of 4096 x 4096 in Q5_K 15 / 10); in two
-// 0.94 - 1.24, for a workgroup's own phases do not overlap the next one's.  Level, and left to the other: Q4_K of five to seven 256s and few rows (512 x 1536 6.0 / 6.2), Q4_K where that has four tiles a wavefront and k in one part (14336 x 4096
-// 15.4 / 15.8), and more than 24576 rows of few columns (10 of 30848 x 256 in Q6_K 9.3 / 10.0), of 256
-// columns in Q6_K and Q8_0 more than 16384 (5 of 22528 x 256 7.3 / 8.5 and 6.2 / 6.7; of 16000 7.1 / 6.0 and 6.0 / 4.9).  2 - 4 rows are the single-row kernel's row variant (4096 x 4096, four rows 6.8 / 8.6); Q6_K, which has none, from 3 rows on where there is
-// one tile a wavefront (4096 x 4096 10.9 / 10.0, but 8192 x 3072 13.0 / 13.5).  Up to 65536 weights of the 5-bit formats stay although slower there, as the test of
-// k_qmm_reg's rule holds them to be its.
+// Where one round of workgroups does it, against what took the call (k_qb_prep and k_qmv_direct, 5-bit formats k_qmm_reg, the tiles or a launch a row).  Replayed
+// graphs of 70 random products a format, 100 - 30000 rows, 256 - 16384 columns, 5 - 16 activation rows, those that come here: Q4_0 0.83 of the time, Q8_0 0.83, Q4_K
+// 0.85, Q6_K 0.86, Q5_0 0.49, Q5_K 0.52 (geometric means; 16 of 2048 x 8192 in Q4_K 11.0 / 9.4 us, 11008 x 4096 in Q8_0 18.2 / 13.5, 4096 x 11008 in Q6_K 24.4 / 19.5,
+// 5 of 4096 x 4096 in Q5_K 13.8 / 9.9).  In two rounds 0.94 - 1.24, for a workgroup's own phases do not overlap the next one's.
+// Left to the others, us there / here:
+// - Q4_K from 3.5 row tiles a compute unit on and up to 4096 columns, where k_qmv_direct has four tiles a wavefront: 14336 x 4096 (224 workgroups here, one round)
+//   14.7 / 14.8, 14336 x 3072 13.0 / 13.1, 16384 x 3072 13.1 / 14.5.  The line takes in some that would be quicker here (14336 x 2048 10.4 / 8.6, 20480 x 3072
+//   20.2 / 15.5).  Q4_0 likewise of 2304 - 3072 columns: 14336 x 2560 11.6 / 12.3 (12288 x 2560 12.7 / 11.2, 16000 x 4096 15.0 / 13.9).
+// - Q4_K of five to seven 256s and few rows: 512 x 1536 5.9 / 6.2.
+// - More than 24576 rows of few columns: 10 of 30848 x 256 in Q6_K 7.9 / 9.1; of 256 columns in Q6_K and Q8_0 more than 16384: 5 of 22528 x 256 7.3 / 8.5 and
+//   6.2 / 6.7 (16000 x 256 7.1 / 6.0 and 6.0 / 4.9).
+// - 13 - 16 rows of Q5_K where a wavefront has four tiles, in parts: 16326 x 2304 17.0 / 20.2, 8192 x 5376 19.4 / 20.4 (4096 x 14336 24.2 / 23.3).
+// - Up to 65536 weights of the 5-bit formats, although 64 x 1024 is 9.7 / 5.3: there k_qmm_reg's own line, five rows of 1024 columns, can be seen.
+// - 2 - 4 rows, which are the single-row kernel's row variant (4096 x 4096, four rows 6.8 / 8.6); Q6_K, which has none, only from 3 rows on and with one tile a
+//   wavefront (3 rows of 4096 x 4096 9.8 / 9.5, of 8192 x 3072 12.6 / 13.1).
 bool fh_qmv_rows_pays(const fh_qmatrix *q, const float *x, int m) {
     if (!fh_qmv_rows_supports(q, x, m) || m < (q->type == FH_Q6_K ? 3 : 5)) return false;
+    const int64_t tiles = (q->n + 15) / 16, cus = q->dev->compute_units;
     if ((q->type == FH_Q5_0 || q->type == FH_Q5_K) && q->n * q->k <= 65536) return false;
     if (q->type == FH_Q4_K && q->k > 1024 && q->k < 2048 && q->n <= 2816) return false;
-    if (q->type == FH_Q4_K && q->k <= 4096 && (q->n + 15) / 16 * 2 >= 7 * (int64_t)q->dev->compute_units) return false;
-    const int64_t few = (q->type == FH_Q6_K || q->type == FH_Q8_0) && q->k <= 256 ? 4 : 6;
-    if ((q->n + 15) / 16 > few * q->dev->compute_units) return false;
+    if (tiles * 2 >= 7 * cus && ((q->type == FH_Q4_K && q->k <= 4096) || (q->type == FH_Q4_0 && q->k > 2048 && q->k <= 3072))) return false;
+    if (tiles > ((q->type == FH_Q6_K || q->type == FH_Q8_0) && q->k <= 256 ? 4 : 6) * cus) return false;
     const RowsCut cut = rows_cut(q);
+    if (q->type == FH_Q5_K && m > 12 && cut.tt == 4 && q->k > 256 * cut.kc && q->k < 8192) return false;
     return cut.rounds == 1 && (m >= 5 || cut.tt == 1);
 }
 

@@ -63,6 +63,7 @@ def test_rule(dev, oracle, ty, m, n, k, taken):
 
 
 @pytest.mark.parametrize("ty,m,n,k,cut", [(synth.Q4_K, 16, 512, 1536, 0), (synth.Q6_K, 5, 22528, 256, 0), (synth.Q8_0, 5, 22528, 256, 0),
+                                          (synth.Q4_0, 5, 14336, 2560, 0), (synth.Q5_K, 16, 8192, 5376, 0), (synth.Q4_K, 16, 4096, 11008, 8 + 4),
                                           (synth.Q4_0, 16, 1408, 16384, 8 + 2), (synth.Q6_K, 16, 512, 1024, 1)])
 def test_level_or_slower(dev, ty, m, n, k, cut):
     """Products that stay with the kernels they had, for which one launch is level or slower (cut 0), and cuts that keep it quicker: many 256s in parts of

@@ -76,3 +76,22 @@ def test_grouped_tiles(dev, tokens, experts):
         finally:
             dev.set_option("matmul_kernel", 0)
         np.testing.assert_array_equal(got[4], got[14])
+
+
+@pytest.mark.parametrize("tokens", [1025, 1100, 2047])
+def test_grouped_tiles_more_than_eight(dev, tokens):
+    """Two experts of two take every token: as tiles of 128 rows (option 14) they are nine or sixteen each, eight neighbours and what is left, of up to 320 (option 4)
+    no more than seven."""
+    from kalosm_amd import bench_hybrid
+    from kalosm_amd.hybrid import HybridModel
+
+    m = HybridModel.random_init(dev, bench_hybrid.config(vocab=512, width=512, heads=4, experts=2, top=2, ff=192, window=128, groups=2), ctx=2048)
+    ids, got = np.random.default_rng(tokens).integers(0, 512, tokens), {}
+    try:
+        for option in (14, 4):
+            m.reset()
+            dev.set_option("matmul_kernel", option)
+            got[option] = m.forward(ids, want=range(tokens - 200, tokens))
+    finally:
+        dev.set_option("matmul_kernel", 0)
+    np.testing.assert_array_equal(got[4], got[14])

@@ -77,24 +77,31 @@ def test_level_or_slower(dev, ty, m, n, k, cut):
 
 @named
 def test_small_groups_beside_a_large_one(dev, oracle, ty):
-    """Weights that are zero where the activations are large: the formats that normalise 32 values by themselves lose nothing of the small
-    ones, the others what a power of two per 256 leaves of them (values of 2^-16 of the largest keep eight bits)."""
-    n, k, m = 64, 2048, 6
-    raw = synth.random_weight(ty, n, k, seed=4)
-    w = oracle.dequantize(ty, raw).reshape(n, k)
+    """Weights that are zero where the activations are large, in 32 of a 256: hi + lo keeps an activation to 2^-22 of itself or to 2^-39 of the largest with which
+    it shares a power of two.  The 5-bit formats have one per 32 and lose nothing of the small ones beside 2^28 times as much (with one per 256 an output is
+    off by 2^-12 of the sum of magnitudes, where 2^-19 is allowed); the others have one per 256 and 2^14."""
+    n, k, m, own = 64, 2048, 6, ty in (synth.Q5_0, synth.Q5_K)
     size = synth.BLOCK_ELEMS[ty]
-    blocks = raw.reshape(n, k // size, -1).copy()
-    blocks[:, 0] = 0  # a block of zeros: scale (and offset) zero
+    blocks = synth.random_weight(ty, n, k, seed=4).reshape(n, k // size, -1).copy()
+    if size == 32:
+        blocks[:, 0] = 0  # a block of zeros: scale zero
+    elif ty == synth.Q6_K:
+        blocks[:, 0, 192:194] = 0  # scales of the first two sixteens
+    else:
+        blocks[:, 0, [4, 8]] &= 0xC0  # scale and offset of the first 32
     raw = np.ascontiguousarray(blocks).reshape(-1)
     w = oracle.dequantize(ty, raw).reshape(n, k).astype(np.float64)
-    assert not w[:, :size].any()
+    assert not w[:, :32].any() and w[:, 32:256].any()
     x = synth.random_activation(m, k, seed=5)
-    x[:, :min(32, size)] *= np.float32(2.0 ** 14)
+    x[:, :32] *= np.float32(2.0 ** (28 if own else 14))
     q = QMatrix.from_raw_bytes(dev, (n, k), raw, ty)
     with options(dev, matvec_direct=3):
         got = Tensor.from_slice(dev, x).q_mat_mul(q).as_slice().astype(np.float64)
-    want = x.astype(np.float64) @ w.T
-    assert np.abs(got - want).max() <= 2.0 ** -17 * np.abs(want).max()
+    x = x.astype(np.float64)
+    tol = 2.0 ** -19 * (np.abs(x) @ np.abs(w).T)
+    if not own:
+        tol += 2.0 ** -38 * np.abs(x).max(1)[:, None] * np.abs(w[:, :256]).sum(1)
+    assert (np.abs(got - x @ w.T) <= tol).all()
 
 
 @named

@@ -269,7 +269,9 @@ fh_status fh_matmul(fh_device *dev, int32_t dtype, const void *a_dev, int64_t a_
  * q/k/v/out alike (kv may be f16 with f32 q via fh_flash_attention_ex).  mask_dev is
  * [sq, skv] f32 for FH_MASK_ADDITIVE, ignored otherwise.  FH_MASK_CAUSAL lets query i see keys
  * j <= i + (skv - sq) (attention_mask.rs:46-66 with the offset padding of mask_cache.rs:73-88).
- * d <= 256; d of 64 or 128 takes the tuned kernels. */
+ * d <= 256; d of 64 or 128 takes the tuned kernels.  Views may begin at any element and their positions run in any
+ * direction; prompts whose k or v does not begin at a multiple of 16 bytes, or whose positions are 2^21 elements or more
+ * apart or run backwards, are read by a slower form (f16, 2048 tokens, 32 / 8 heads of 128: 149 us for 55). */
 fh_status fh_flash_attention(fh_device *dev, int32_t dtype, const void *q_dev, int64_t q_sb,
                              int64_t q_sh, int64_t q_st, const void *k_dev, const void *v_dev,
                              int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int32_t b, int32_t hq,

@@ -23,10 +23,10 @@
 // descriptor that moves with the tile, and split operands, whose weights lose nothing by it, move their reference only where a maximum is 2^8
 // above it.  The denominator is the sum of the f32 weights, whatever the products take them as: weights below 2^-25 of the largest are zero in f16, and
 // many of them still count (16384 keys 2^25.5 below one: 3.5e-4 of the output).  (Added up in pairs from the rounded weights it saved 16 of the
-// instructions and no time: 2048 tokens 51.9 us against 52.0.)  Rows of V are 64 bytes apart in the banks (ap_v_row), so that the 16
+// instructions: 2048 tokens 51.9 us against 52.0, two heads a workgroup 4096 tokens 166 / 172, 8192 574 / 592.)  Rows of V are 64 bytes apart in the banks (ap_v_row), so that the 16
 // lanes of a transposing load cover them once.  Heads that share a workgroup (four wavefronts each) are half a step apart, one in the softmax while
-// the other multiplies.  f16, 32 / 8 heads of 128, causal, before and after: 1024 tokens 25.3 / 23.7 us, 2048 53.4 / 50.8, 4096 166 / 151, 8192
-// 616 / 558 (985 TFLOP/s); f32 2048 129 / 125, 4096 400 / 350.
+// the other multiplies.  Replayed graphs of ten calls, causal, 32 / 8 heads of 128, before all that (and k_attn_ahead) and now, us: f16 1024 tokens
+// 28.1 / 26.3, 2048 66 / 61, 3000 116 / 108, 4096 175 / 172, 8192 607 / 592 (930 TFLOP/s); f32 2048 146 / 144, 4096 396 / 363.
 // Both products are computed TRANSPOSED with
 // v_mfma_f32_32x32x16_f16 so that a lane always stands for ONE query (the accumulator column):
 //   S^T (keys x queries) = K . Q^T      A = K rows, B = Q^T kept in registers for the whole kernel
@@ -501,8 +501,8 @@ __global__ __launch_bounds__(256 * HW * KS) __attribute__((amdgpu_waves_per_eu(S
 // so that the matrix cores work beside the vector ALU; K is a tile ahead of V for it.  Two sets of scores leave no registers for tiles on their way:
 // those go straight into LDS, in rows without padding whose 16-byte pieces are swapped on the memory side (K: 16 rows' pieces of one number, V:
 // 4 rows' 64 bytes cover the banks once).  What is left is the chain of a step in one wavefront (with the two key groups half a step apart, one in
-// the softmax and one in the second product, it is longer: 2048 tokens 56 us).  Before and after, causal, us: 8 heads of 64, 3000 tokens 34.0 / 31.0;
-// 16 / 4 of 64, 777 12.1 / 12.0; 32 / 8 of 128, 2048 51.5 / 50.6, 3000 101 / 97.
+// the softmax and one in the second product, it is longer: 2048 tokens 56 us).  Replayed graphs, causal, us, k_attn_prefill in the same shape and this: 8 heads of 64, 3000
+// tokens 37.5 / 34.9; 16 / 4 of 64, 777 13.5 / 12.3; 32 / 8 of 128, 512 15.1 / 14.7, 2048 61.8 / 61.1, 3000 113 / 108.
 template <typename TQ, int D, int KS, int QW>
 __global__ __launch_bounds__(64 * QW * KS) __attribute__((amdgpu_waves_per_eu(QW == 4 ? 2 : 1, 2))) void k_attn_ahead(
     const TQ *__restrict__ q, int64_t q_sb, int64_t q_sh, int64_t q_st, const fh_half *__restrict__ k, const fh_half *__restrict__ v, int64_t kv_sb,

@@ -79,7 +79,7 @@ def test_level_or_slower(dev, ty, m, n, k, cut):
 def test_small_groups_beside_a_large_one(dev, oracle, ty):
     """Weights that are zero where the activations are large, in 32 of a 256: hi + lo keeps an activation to 2^-22 of itself or to 2^-39 of the largest with which
     it shares a power of two.  The 5-bit formats have one per 32 and lose nothing of the small ones beside 2^28 times as much (with one per 256 an output is
-    off by 2^-12 of the sum of magnitudes, where 2^-19 is allowed); the others have one per 256 and 2^14."""
+    off by 2^-15 of the sum of magnitudes, where 2^-19 is allowed); the others have one per 256 and 2^14."""
     n, k, m, own = 64, 2048, 6, ty in (synth.Q5_0, synth.Q5_K)
     size = synth.BLOCK_ELEMS[ty]
     blocks = synth.random_weight(ty, n, k, seed=4).reshape(n, k // size, -1).copy()

@@ -4,7 +4,7 @@
 // with the queries aligned to the END of the keys), fusor-ml/core/src/row_program.rs:1210-1382 (the fused kernel).
 //
 // grid (q heads / HW, query blocks of 128, batch); 4 x HW wavefronts, each owning 32 query rows of one head: the HW
-// (1 or 2) heads of a workgroup share a KV head, so a KV tile is fetched and staged once for 128 x HW query rows.
+// (1, or 2 of f32 keys) heads of a workgroup share a KV head, so a KV tile is fetched and staged once for 128 x HW query rows.
 // KV tiles of 64 keys go through LDS as f16, both as [key][d] rows written with 16-byte stores; the V^T operand
 // of the second product is read with the transposing LDS load of gfx950 (ds_read_b64_tr_b16: the 16 lanes of a
 // group supply 4 keys x 16 dims and receive, per lane, one dim of the 4 keys).  Two LDS buffers and one barrier per
@@ -13,7 +13,7 @@
 // KS = 2 (prompts whose workgroups are no more than two rounds): eight wavefronts per query block, the second four take every
 // other key tile with running statistics of their own, and the two halves are merged through LDS at the end - half the tile steps per
 // workgroup.  (k_attn_prefill has it for f32 operands rounded to f16 only, attn_kernel = 2.)
-// Of f16 keys and values k_attn_prefill has the launches of two heads a workgroup and those of at most 128 keys; all others are k_attn_ahead's.
+// Of f16 keys and values k_attn_prefill has the launches of at most 128 keys; all others are k_attn_ahead's.
 // QW = 2 (k_attn_ahead, shorter still: every workgroup of 64 query rows finds a compute unit of its own): two wavefronts per key
 // group, so a SIMD runs one wavefront's chain of a step instead of two.
 // What bounds the loop (measured per stage): the first product is matrix-core bound, the softmax vector-ALU bound
@@ -23,10 +23,10 @@
 // descriptor that moves with the tile, and split operands, whose weights lose nothing by it, move their reference only where a maximum is 2^8
 // above it.  The denominator is the sum of the f32 weights, whatever the products take them as: weights below 2^-25 of the largest are zero in f16, and
 // many of them still count (16384 keys 2^25.5 below one: 3.5e-4 of the output).  (Added up in pairs from the rounded weights it saved 16 of the
-// instructions: 2048 tokens 51.9 us against 52.0, two heads a workgroup 4096 tokens 166 / 172, 8192 574 / 592.)  Rows of V are 64 bytes apart in the banks (ap_v_row), so that the 16
+// instructions and no time in k_attn_ahead: 2048 tokens 51.9 us against 52.0.)  Rows of V are 64 bytes apart in the banks (ap_v_row), so that the 16
 // lanes of a transposing load cover them once.  Heads that share a workgroup (four wavefronts each) are half a step apart, one in the softmax while
 // the other multiplies.  Replayed graphs of ten calls, causal, 32 / 8 heads of 128, before all that (and k_attn_ahead) and now, us: f16 1024 tokens
-// 28.1 / 26.3, 2048 66 / 61, 3000 116 / 108, 4096 175 / 172, 8192 607 / 592 (930 TFLOP/s); f32 2048 146 / 144, 4096 396 / 363.
+// 28.3 / 26.1, 2048 64 / 59, 3000 114 / 104, 4096 178 / 172, 8192 604 / 585 (940 TFLOP/s); f32 2048 146 / 143, 4096 390 / 358.
 // Both products are computed TRANSPOSED with
 // v_mfma_f32_32x32x16_f16 so that a lane always stands for ONE query (the accumulator column):
 //   S^T (keys x queries) = K . Q^T      A = K rows, B = Q^T kept in registers for the whole kernel
@@ -724,13 +724,10 @@ template <typename TQ, typename TKV, bool SPLIT = false>
 static fh_status ap_launch(fh_device *dev, const void *q, int64_t q_sb, int64_t q_sh, int64_t q_st, const void *k,
                            const void *v, int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int b, int hq, int hkv, int sq,
                            int skv, int d, float scale, int causal, int by_row, void *out) {
-    // Two heads of one KV group share the staged tiles when the launch still has enough workgroups without the
-    // split: short prompts are bound by the longest workgroup and by how many compute units have one at all.
     const long wgs = (long)hq * ((sq + 127) / 128) * b;
-    // attn_kernel = 6 / 7 / 8 / 9 force the workgroup shape (two heads / two key groups / plain / 64-row query blocks
+    // attn_kernel = 6 / 7 / 8 / 9 force the workgroup shape (two heads, f32 keys only / two key groups / plain / 64-row query blocks
     // with two key groups) whatever the size: tests
     const int64_t force = dev->opt_attn_kernel;
-    const bool pair = (hq / hkv) % 2 == 0 && (force == 6 || (force != 7 && force != 8 && wgs >= 1024));
 #define FH_AP(D, HW, KS, ...) ap_launch_k<TQ, TKV, D, SPLIT, HW, KS, ##__VA_ARGS__>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out)
     // A request of 16 bytes, straight into LDS above all, is made for an address of its multiple, and a step's 128 rows lie within the 2^31 bytes
     // of a buffer.  Other views are read as they lie by the plain form (32 / 8 heads of 128, causal, us: K and V of f16 one element off 149, aligned 55, a row a
@@ -750,17 +747,21 @@ static fh_status ap_launch(fh_device *dev, const void *q, int64_t q_sb, int64_t 
                 return d == 128 ? ap_launch_ahead<TQ, 128, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out)
                                 : ap_launch_ahead<TQ, 64, 2, 2>(dev, q, q_sb, q_sh, q_st, k, v, kv_sb, kv_sh, kv_st, b, hq, hkv, sq, skv, scale, causal, by_row, out);
             if (halves) return d == 128 ? FH_AH(128, 2) : FH_AH(64, 2);
-            // up to two key tiles a query there is little to overlap, and the longer code costs more than it gives (32 / 8 heads of 128:
-            // 65 tokens 6.74 us for 6.55, 128 tokens 7.85 for 7.71; from 129 on, in two key groups, 7.5 for 8.4)
-            if (!pair && (skv > 128 || force == 8)) return d == 128 ? FH_AH(128, 1) : FH_AH(64, 1);
-            if (!pair) return d == 128 ? FH_AP(128, 1, 1) : FH_AP(64, 1, 1);
+            // Up to two key tiles a query there is little to overlap, and the longer code costs more than it gives (32 / 8 heads of 128:
+            // 65 tokens 6.74 us for 6.55, 128 tokens 7.85 for 7.71; from 129 on, in two key groups, 7.5 for 8.4).  Two heads a workgroup are not quicker in any number of
+            // workgroups (causal, us, two heads in k_attn_prefill / this: 8 x 8 / 2 of 64, 2048 tokens 104 / 73; 4 x 32 / 8 of 128, 1024 75 / 62; 32 / 8 of 128, 8000
+            // 570 / 566; 128 x 8 / 2 of 64, 65 tokens 17.6 / 14.6, 32 x 32 / 8 of 128, 128 level).
+            if (skv > 128 || force == 8) return d == 128 ? FH_AH(128, 1) : FH_AH(64, 1);
 #undef FH_AH
-            return d == 128 ? FH_AP(128, 2, 1) : FH_AP(64, 2, 1);
+            return d == 128 ? FH_AP(128, 1, 1) : FH_AP(64, 1, 1);
         } else {
             if (halves) return d == 128 ? FH_AP(128, 1, 2) : FH_AP(64, 1, 2);
         }
     }
-    if constexpr (SPLIT || sizeof(TKV) == 4) {
+    if constexpr (sizeof(TKV) == 4) {
+        // Two heads of one KV group share the staged tiles when the launch still has enough workgroups without the
+        // split: short prompts are bound by the longest workgroup and by how many compute units have one at all.
+        const bool pair = (hq / hkv) % 2 == 0 && (force == 6 || (force != 7 && force != 8 && wgs >= 1024));
         if (d == 128) return pair ? FH_AP(128, 2, 1) : FH_AP(128, 1, 1);
         return pair ? FH_AP(64, 2, 1) : FH_AP(64, 1, 1);
     }

@@ -30,9 +30,17 @@ template <> __device__ __forceinline__ uint16_t fh_to<uint16_t>(float f) { retur
 __device__ __forceinline__ float fh_up(float f) { return f; }
 __device__ __forceinline__ float fh_up(uint16_t b) { return fh_bf_f32(b); }
 
+// The sum over the wavefront, in every lane: of lanes 32 apart, 16, 8, 4, 2, 1.  (By register moves: through the LDS, as __shfl_xor has it, the same sum is six
+// round trips, and a matvec of 32768 rows of 512, one such sum each, took 11.0 us instead of 8.9.)
 __device__ __forceinline__ float fh_wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    typedef uint32_t pair __attribute__((ext_vector_type(2)));
+    const auto both = [](const pair &r) { return __uint_as_float(r[0]) + __uint_as_float(r[1]); };
+    v = both(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    v = both(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xF, 0xF, true)); // row_ror:8
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x124, 0xF, 0xF, true)); // row_ror:4
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));  // quad_perm 2 3 0 1
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));  // quad_perm 1 0 3 2
     return v;
 }
 // silu, softplus and the logistic function with the full-precision exponential
@@ -113,6 +121,93 @@ struct FhRowStream {
             if (p + i < pieces) use(i, p + i, x, acc);
     }
 };
+
+// A barrier behind LDS writes that leaves requests to memory on their way.
+__device__ __forceinline__ void fh_lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// The rows of a matrix that one wavefront goes through, one after the other: `count` rows `hop` elements apart, in pieces of 512 (a lane:
+// eight values, 16 bytes) with AHEAD pieces on their way.  Requests past the last row repeat it, and none is under a condition.
+// A compute unit answers its requests in their order, so what is on the way is also what the launch's own input waits behind: a launch
+// has one workgroup of eight wavefronts a compute unit, each with 4 KB on its way - 8 MB over the device, the rate of the memory
+// times its latency.  us of 14336 x 4096 / 32768 x 4096 / 4096 x 14336: 19.9 / 40.9 / 20.0 (plain reads of the bytes 19.6 / 42.5 / 19.6); 3 KB 20.0 /
+// 40.8 / 20.3, 2 KB 23.3 / 49.2 / 22.9, 8 KB 21.4 / 43.5 / 21.0, two such workgroups 22.7 / 45.7 / 22.0; without the hint that the weights are not
+// read again 20.7 / 44.4 / 22.0; as many workgroups as there are rows for, two rows and 8 KB a wavefront, 22.4 / 44.4 / 22.3, four rows and 16 KB 29.5 / 62.0 / 26.5.
+// The input lies in the LDS in two planes, so that neighbouring lanes read neighbouring 16 bytes.
+struct FhRowInput {
+    float *xs; // [2][plane]: the first and the second four of every eight values; zeros up to whole pieces
+    int plane; // pieces * 256
+    __device__ __forceinline__ float4 &quad(int q) const { return *(float4 *)(xs + (q & 1) * plane + (q >> 1) * 4); } // values 4 q ..
+    __device__ __forceinline__ float &at(int i) const { return xs[((i >> 2) & 1) * plane + (i >> 3) * 4 + (i & 3)]; }
+};
+__host__ __device__ static inline int fh_row_pieces(int kp) { return (kp + 511) / 512; }
+enum { FH_ROW_WAVES = 8 };
+template <int AHEAD = 4>
+struct FhRowDeal {
+    const uint16_t *row; // of the next request
+    int64_t hop;
+    int kp, pieces, count, left, piece, lane8;
+    uint4 u[AHEAD];
+    __device__ __forceinline__ void fetch(int slot) {
+        typedef uint32_t words __attribute__((ext_vector_type(4)));
+        const int c = piece * 512 + lane8;
+        const words v = __builtin_nontemporal_load((const words *)(row + (c < kp ? c : kp - 8)));
+        __builtin_memcpy(&u[slot], &v, 16);
+        const bool end = ++piece == pieces;
+        piece = end ? 0 : piece;
+        left -= end;
+        row += end && left > 0 ? hop : 0;
+    }
+    // rows first, first + step, .. of n (first: the wavefront's, in a scalar register)
+    __device__ __forceinline__ void start(const uint16_t *w, int kp_, int first, int step, int n) {
+        kp = kp_, pieces = fh_row_pieces(kp), lane8 = (threadIdx.x & 63) * 8, piece = 0;
+        left = count = first < n ? (n - first + step - 1) / step : 0;
+        row = w + (int64_t)(first < n ? first : n - 1) * kp, hop = (int64_t)step * kp;
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) fetch(i);
+    }
+    // done(i, row i . x) for each of them, in all lanes
+    template <typename F>
+    __device__ __forceinline__ void run(const FhRowInput &x, F done) {
+        float acc = 0.f;
+        int p = 0, i = 0;
+        const int total = count * pieces;
+        for (int t = 0; t < total; t += AHEAD) {
+#pragma unroll
+            for (int s = 0; s < AHEAD; s++) {
+                const float *at = x.xs + p * 256 + (lane8 >> 1);
+                const float4 a = *(const float4 *)at, b = *(const float4 *)(at + x.plane);
+                acc = fmaf(fh_bf_lo(u[s].x), a.x, acc);
+                acc = fmaf(fh_bf_hi(u[s].x), a.y, acc);
+                acc = fmaf(fh_bf_lo(u[s].y), a.z, acc);
+                acc = fmaf(fh_bf_hi(u[s].y), a.w, acc);
+                acc = fmaf(fh_bf_lo(u[s].z), b.x, acc);
+                acc = fmaf(fh_bf_hi(u[s].z), b.y, acc);
+                acc = fmaf(fh_bf_lo(u[s].w), b.z, acc);
+                acc = fmaf(fh_bf_hi(u[s].w), b.w, acc);
+                fetch(s);
+                if (++p == pieces) {
+                    acc = fh_wave_sum(acc);
+                    if (i < count) done(i, acc); // (what is behind the last row is the last piece again)
+                    acc = 0.f, p = 0, i++;
+                }
+            }
+        }
+    }
+};
+// Several matrices in one launch of at most `most` workgroups: as few rows a workgroup as that allows; tiles[i]: workgroups of matrix i.
+static inline int fh_row_share(const int *n, int count, int most, int *tiles) {
+    int64_t total = 0;
+    for (int i = 0; i < count; i++) total += n[i];
+    for (int64_t per = (total + most - 1) / most;; per++) {
+        int64_t sum = 0;
+        for (int i = 0; i < count; i++) sum += tiles[i] = (int)((n[i] + per - 1) / per);
+        if (sum <= most || per >= total) return (int)sum;
+    }
+}
 
 // ---------------------------------------------------------------- host launchers
 // Storage of activations between kernels: FH_F32, or FH_BF16_ACT for decoders that serve in bf16.
@@ -204,8 +299,10 @@ enum { FH_MV_ACT_NONE = 0, FH_MV_ACT_RELU2 = 1, FH_MV_ACT_TANH = 2, FH_MV_MAX = 
 struct FhMvMix { const uint16_t *w; const float *mu; float *y; int n, act; };
 struct FhMvAdd {
     const float *x = nullptr, *y = nullptr, *w = nullptr;
+    const float *norm = nullptr;  // x' = x / rms(x) * norm instead (fh_matvec_norm)
     float eps = 0.f;
     float *x_out = nullptr;
+    bool x_pad = false;           // x_out has zeros up to kp
     float *state = nullptr;       // [2][k]
     const int *pos_dev = nullptr;
     const float *gate = nullptr;

@@ -531,158 +531,6 @@ fh_status fh_rows_to_act(fh_device *dev, int dtype, const float *x, int64_t ldx,
     return FH_OK;
 }
 
-// ------------------------------------------------------------------------------ decode matvec
-// One wavefront per ROWS weight rows; a lane takes eight consecutive weights (16 bytes) of every 512.  The input is
-// normed once per workgroup into the LDS; f32 products and sums.
-// What bounds the decode products: a plain read of 117 MB takes 19 us on this device, the product 24 us (14336 x 4096) and 23 us
-// (4096 x 14336).  No request is under a condition, which would empty the pipeline every AHEAD pieces (FhRowStream).  The rest is the
-// input every workgroup stages: without it the same loops take 5 us less, whether it is requested first, last, behind a
-// barrier, rotated or from copies of its own, with 2 to 16 pieces ahead, and with one workgroup per compute unit.
-struct MvSegs { FhMvSeg s[3]; int tiles[3]; int n; };
-
-// XV: 16-byte pieces of the input a thread holds, requested ahead of the first weights; 0: the input goes to the LDS in a loop ahead
-// of them.  How much each way has on its way, and which one, is a matter of how many wavefronts there are on a compute unit:
-//   four rows a wavefront (8192 rows of the matrices or more): all workgroups of a matrix of 32768 rows fit the device at once if a
-//     wavefront takes at most 64 registers, so XV = 0 and two pieces of the weights: 32768 x 1024 / 2048 / 4096 in 13.2 / 27.6 /
-//     48.7 us; with the input in registers and four pieces (104 - 122 registers) 17.4 / 30.5 / 54.2.
-//   two rows (from 2048): XV = 0 and four pieces for inputs of 1025 to 4096 - 7000 x 4096 13.3 us, 4096 x 4096 9.1, in registers 15.9
-//     and 10.6.  Shorter ones are a piece a thread (7000 x 1000 4.8 us, the loop 5.1); longer ones leave room for few workgroups
-//     beside their LDS, so registers are free (7000 x 14336 39 us, 4096 x 14336 23; the loop 45 and 27).
-//   one row: in registers (1024 x 4096 5.3 us, 1024 x 14336 7.7), and two pieces of the weights for each of the input's, up to
-//     eight.  Requests past the end repeat the last piece, so more pieces than there are cost time (128 x 1024: 2.1 us, with four 2.5).
-template <int ROWS, int XV>
-__global__ __launch_bounds__(256, XV ? 1 : 8) void k_matvec_norm(const float *__restrict__ x, int k, int kp, const float *__restrict__ nw,
-                                                     float eps, MvSegs segs, float *__restrict__ norm_out) {
-    extern __shared__ __attribute__((aligned(16))) float xs[]; // [kp]
-    __shared__ float red[4];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    int tile = blockIdx.x, si = 0;
-    while (si + 1 < segs.n && tile >= segs.tiles[si]) tile -= segs.tiles[si++];
-    const FhMvSeg seg = segs.s[si];
-    const int row0 = (tile * 4 + wave) * ROWS;
-    FhRowStream<ROWS, XV == 0 ? 8 / ROWS : XV < 4 ? 2 * XV : 8> rows;
-#pragma unroll
-    for (int r = 0; r < ROWS; r++) rows.w[r] = seg.w + (int64_t)(row0 + r < seg.n ? row0 + r : seg.n - 1) * kp;
-    float ss = 0.f;
-    const auto scale = [&]() { // of the norm, from the threads' sums of squares
-        ss = fh_wave_sum(ss);
-        if (lane == 0) red[wave] = ss;
-        __syncthreads();
-        return 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
-    };
-    if (XV && !(k & 3)) { // (k is at most 1024 XV)
-        constexpr int NX = XV ? XV : 1, NW = XV <= 4 ? NX : 1; // (long inputs read the norm's weights when they are used)
-        float4 v[NX], w[NW];
-        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int j = 0; j < NX; j++) {
-            const int i = (tid + 256 * j) * 4, at = i < k ? i : 0;
-            v[j] = *(const float4 *)(x + at);
-            if (NW == NX) w[j] = nw ? *(const float4 *)(nw + at) : zero;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        rows.start(kp);
-        __builtin_amdgcn_sched_barrier(0);
-        float inv = 1.f;
-        if (nw) {
-#pragma unroll
-            for (int j = 0; j < NX; j++)
-                if ((tid + 256 * j) * 4 < k) ss = fmaf(v[j].x, v[j].x, fmaf(v[j].y, v[j].y, fmaf(v[j].z, v[j].z, fmaf(v[j].w, v[j].w, ss))));
-            inv = scale();
-        }
-#pragma unroll
-        for (int j = 0; j < NX; j++) {
-            const int i = (tid + 256 * j) * 4;
-            if (i >= kp) continue;
-            float4 o = i < k ? v[j] : zero;
-            if (nw && i < k) {
-                const float4 m = NW == NX ? w[j % NW] : *(const float4 *)(nw + i);
-                o = make_float4(o.x * inv * m.x, o.y * inv * m.y, o.z * inv * m.z, o.w * inv * m.w);
-            }
-            *(float4 *)(xs + i) = o;
-        }
-    } else {
-        if (!(k & 3)) {
-#pragma unroll 8
-            for (int i = tid * 4; i < kp; i += 1024) {
-                const float4 v = i < k ? *(const float4 *)(x + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-                ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
-                *(float4 *)(xs + i) = v;
-            }
-        } else {
-#pragma unroll 8
-            for (int i = tid; i < kp; i += 256) {
-                const float v = i < k ? x[i] : 0.f;
-                ss = fmaf(v, v, ss);
-                xs[i] = v;
-            }
-        }
-        rows.start(kp);
-        if (nw) {
-            const float inv = scale();
-            if (!(k & 3))
-#pragma unroll 2
-                for (int i = tid * 4; i < k; i += 1024) {
-                    const float4 v = *(const float4 *)(xs + i), m = *(const float4 *)(nw + i);
-                    *(float4 *)(xs + i) = make_float4(v.x * inv * m.x, v.y * inv * m.y, v.z * inv * m.z, v.w * inv * m.w);
-                }
-            else
-#pragma unroll 4
-                for (int i = tid; i < k; i += 256) xs[i] = xs[i] * inv * nw[i];
-        }
-    }
-    __syncthreads();
-    if (norm_out && blockIdx.x == 0)
-        for (int i = tid; i < kp; i += 256) norm_out[i] = xs[i];
-    float acc[ROWS];
-#pragma unroll
-    for (int r = 0; r < ROWS; r++) acc[r] = 0.f;
-    rows.run(xs, acc);
-#pragma unroll
-    for (int r = 0; r < ROWS; r++) acc[r] = fh_wave_sum(acc[r]);
-    if (lane == 0)
-#pragma unroll
-        for (int r = 0; r < ROWS; r++)
-            if (row0 + r < seg.n) seg.y[row0 + r] = acc[r];
-}
-
-fh_status fh_matvec_norm(fh_device *dev, const float *x, int k, const float *w, float eps, const FhMvSeg *segs, int n_segs,
-                         float *norm_out) {
-    FH_REQUIRE(n_segs >= 1 && n_segs <= 3, "1 to 3 matrices per matvec launch");
-    const int kp = (int)fh_pad64(k);
-    MvSegs ms{};
-    int64_t total = 0;
-    for (int i = 0; i < n_segs; i++) total += segs[i].n;
-    const int rows = total >= (int64_t)dev->compute_units * 4 * 4 * 2 ? 4 : total >= (int64_t)dev->compute_units * 4 * 2 ? 2 : 1;
-    int tiles = 0;
-    ms.n = n_segs;
-    for (int i = 0; i < n_segs; i++) {
-        ms.s[i] = segs[i];
-        ms.tiles[i] = (segs[i].n + 4 * rows - 1) / (4 * rows);
-        tiles += ms.tiles[i];
-    }
-    const size_t lds = (size_t)kp * 4;
-    FH_REQUIRE(lds <= 120 * 1024, "k = %d too long for the matvec", k);
-#define MV_NORM(ROWS_, XV_)                                                                                               \
-    do {                                                                                                                  \
-        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_matvec_norm<ROWS_, XV_>, lds));                    \
-        k_matvec_norm<ROWS_, XV_><<<dim3((unsigned)tiles), 256, lds, dev->stream>>>(x, k, kp, w, eps, ms, norm_out);      \
-    } while (0)
-    if (rows == 4) MV_NORM(4, 0);
-    else if (rows == 2) {
-        if (k <= 1024) MV_NORM(2, 1);
-        else if (k <= 4096 || k > 16384) MV_NORM(2, 0);
-        else MV_NORM(2, 16);
-    } else if (k <= 1024) MV_NORM(1, 1);
-    else if (k <= 2048) MV_NORM(1, 2);
-    else if (k <= 4096) MV_NORM(1, 4);
-    else if (k <= 16384) MV_NORM(1, 16);
-    else MV_NORM(1, 0);
-#undef MV_NORM
-    FH_HIP(hipGetLastError());
-    return FH_OK;
-}
-
 // ------------------------------------------------------------------------------ the output matrix for several rows
 // Bound by the weights, which the matvec reads again for every row (16 rows of 4096 and a matrix of 32768: 16 x 45 us), so up to 16
 // rows share one pass over them on the matrix cores.  The rows stay f32: each value is cut into three bf16 numbers of 8 bits (24
@@ -975,209 +823,273 @@ fh_status fh_low_rank_tanh(fh_device *dev, const float *x, int kp, int rows, con
     return FH_OK;
 }
 
-// A workgroup of eight wavefronts works its input out once, into the LDS; one wavefront per ROWS weight rows, a lane takes
-// eight consecutive weights (16 bytes) of every 512.  The first AHEAD pieces of 512 are requested before the input, later ones
-// while earlier ones are multiplied.
+// A workgroup of eight wavefronts, one a compute unit, works its input out once, into the LDS, and goes through its share of one matrix's rows
+// (FhRowDeal).  The input is requested ahead of the first weights, for requests are answered in their order, and under no condition.  What bounds
+// it is the memory: 1.9 us of a launch, the bytes at 7.1 TB/s (a plain read) and one to two us for the input.  Replayed graphs over 1 GB of matrices,
+// us, as many workgroups as there are rows for (two or four rows a wavefront, up to 16 KB on their way) / now:
+//   normed    2880 x 2048 5.6 / 4.5, 8288 x 2048 10.7 / 7.6, 32768 x 2048 28.1 / 21.5, 4096 x 4096 10.3 / 8.0, 32768 x 4096 47.2 / 41.0
+//   as it is  4096 x 14336 22.8 / 19.7;  a sublayer added  14336 x 4096 26.6 / 19.8, 16384 x 4096 29.7 / 22.1
+//   gated     4096 x 4096 16.0 / 9.6;   six matrices, five of them on mixtures with the token before, 14336 x 4096 together 28.2 / 21.9
+// (Before, the input's branches alone cost a third of that: with them in the code, though not taken, 4096 x 4096 took 9.7 us for 8.0.)
 struct MvMixes { FhMvMix s[FH_MV_MAX]; int tiles[FH_MV_MAX]; int n; };
 
-__device__ __forceinline__ float mv_sum8(const float *red) {
-    return ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
+template <int WAVES>
+__device__ __forceinline__ float mv_sum(const float *red) {
+    const float s = (red[0] + red[1]) + (red[2] + red[3]);
+    return WAVES == 4 ? s : s + ((red[4] + red[5]) + (red[6] + red[7]));
 }
 
-// x' into the LDS, mixed with the token before it where the matrix wants that.
-// The input is requested ahead of the first weights (`start`): requests are waited for in order, and the input comes out of the
-// L2 while the weights are on their way.
-template <typename F>
-__device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int k, int kp, float *xs, float *red, F start) {
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int pos = in.state ? *in.pos_dev : 0;
-    const float *before = in.state + ((pos - 1) & 1) * k;
-    float *here = in.state + (pos & 1) * k;
-    const bool one = blockIdx.x == 0, shift = mu && pos > 0;
-    if (!(k & 3) && k <= 4096) { // everything is requested at once
-        float4 x[2], y[2], w[2], m[2], b[2];
-        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-        float ss = 0.f;
+__device__ __forceinline__ float4 mv_if(bool c, float4 v) { // (v or zeros: as one choice of two float4 it would be one of addresses, in scratch memory)
+    return make_float4(c ? v.x : 0.f, c ? v.y : 0.f, c ? v.z : 0.f, c ? v.w : 0.f);
+}
+
+// x' into the LDS, mixed with the token before it where the matrix wants that; start() asks for the first weights.
+// XQ: fours of consecutive values of each vector that a thread holds, all requested at once (k a multiple of 4, 256 WAVES XQ at most); 0: any k, value
+// by value.  MODE: what a launch has of this, so that one without a norm has no requests and registers for it.
+enum { MV_PLAIN = 0, MV_NORM = 1, MV_ADD = 2, MV_SHIFT = 3, MV_GATED = 4 };
+template <int WAVES, int XQ, int MODE, typename F>
+__device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int k, int kp, const FhRowInput &xs, float *red, F start) {
+    constexpr int NT = WAVES * 64;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, end = 2 * xs.plane; // (whole pieces)
+    constexpr bool NORM = MODE == MV_NORM, SHIFT = MODE == MV_SHIFT, ADD = MODE == MV_ADD || SHIFT;
+    if (!SHIFT) mu = nullptr;
+    const bool add = MODE == MV_ADD || (SHIFT && in.y), normed = NORM || add, one = blockIdx.x == 0;
+    float *state = SHIFT ? in.state : nullptr;
+    const int pos = state ? *in.pos_dev : 0;
+    const float *before = state + ((pos - 1) & 1) * k;
+    float *here = state + (pos & 1) * k;
+    const bool shift = mu && pos > 0;
+    const int out = NORM ? kp : k; // values of x_out
+    float ss = 0.f;
+    const auto scale = [&]() { // of the norm, from the threads' sums of squares
+        ss = fh_wave_sum(ss);
+        if (lane == 0) red[wave] = ss;
+        fh_lds_barrier();
+        return 1.0f / sqrtf(mv_sum<WAVES>(red) / (float)k + in.eps);
+    };
+    if constexpr (XQ > 0) {
+        float4 x[XQ], y[ADD ? XQ : 1], w[MODE ? XQ : 1], m[SHIFT ? XQ : 1], b[SHIFT ? XQ : 1];
+        // (what is not there is read from x and dropped: behind a condition the compiler no longer knows how many requests are on their way)
+        const float *nw = NORM ? in.norm : add ? in.w : in.x, *yp = add ? in.y : in.x, *mp = mu ? mu : in.x, *bp = shift ? before : in.x;
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int i = (tid + 512 * j) * 4, at = i < k ? i : 0; // (past the end: the first values again, dropped below)
+        for (int j = 0; j < XQ; j++) {
+            const int i = (tid + NT * j) * 4, at = i < k ? i : 0; // (past the end: the first values again, dropped below)
             x[j] = *(const float4 *)(in.x + at);
-            y[j] = in.y ? *(const float4 *)(in.y + at) : zero;
-            w[j] = in.y ? *(const float4 *)(in.w + at) : zero;
-            m[j] = mu ? *(const float4 *)(mu + at) : zero;
-            b[j] = shift ? *(const float4 *)(before + at) : zero;
+            if (ADD) y[j] = *(const float4 *)(yp + at);
+            if (MODE) w[j] = *(const float4 *)(nw + at);
+            if (SHIFT) m[j] = *(const float4 *)(mp + at), b[j] = *(const float4 *)(bp + at);
         }
         __builtin_amdgcn_sched_barrier(0);
         start();
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-            if ((tid + 512 * j) * 4 >= k) x[j] = y[j] = w[j] = m[j] = b[j] = zero;
+        for (int j = 0; j < XQ; j++) {
+            const bool past = (tid + NT * j) * 4 >= k;
+            x[j] = mv_if(!past, x[j]);
+            if (ADD) y[j] = mv_if(!past && add, y[j]);
+            if (SHIFT) b[j] = mv_if(shift, b[j]);
+        }
         float inv = 0.f;
-        if (in.y) {
+        if (normed) {
 #pragma unroll
-            for (int j = 0; j < 2; j++) ss = fmaf(y[j].x, y[j].x, fmaf(y[j].y, y[j].y, fmaf(y[j].z, y[j].z, fmaf(y[j].w, y[j].w, ss))));
-            ss = fh_wave_sum(ss);
-            if (lane == 0) red[wave] = ss;
-            __syncthreads();
-            inv = 1.0f / sqrtf(mv_sum8(red) / (float)k + in.eps);
+            for (int j = 0; j < XQ; j++) {
+                const float4 v = NORM ? x[j] : y[j];
+                ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
+            }
+            inv = scale();
         }
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int i = (tid + 512 * j) * 4;
-            if (i >= kp) break;
+        for (int j = 0; j < XQ; j++) {
+            const int i = (tid + NT * j) * 4;
+            if (i >= end) break;
             float4 v = x[j];
-            if (in.y) v = make_float4(v.x + y[j].x * inv * w[j].x, v.y + y[j].y * inv * w[j].y, v.z + y[j].z * inv * w[j].z, v.w + y[j].w * inv * w[j].w);
-            if (one && i < k) {
-                if (in.x_out) *(float4 *)(in.x_out + i) = v;
-                if (in.state) *(float4 *)(here + i) = v;
+            if (NORM) v = make_float4(v.x * inv * w[j].x, v.y * inv * w[j].y, v.z * inv * w[j].z, v.w * inv * w[j].w);
+            else if (add) v = make_float4(v.x + y[j].x * inv * w[j].x, v.y + y[j].y * inv * w[j].y, v.z + y[j].z * inv * w[j].z, v.w + y[j].w * inv * w[j].w);
+            if (one) {
+                if (in.x_out && i < out) *(float4 *)(in.x_out + i) = mv_if(i < k, v);
+                if (state && i < k) *(float4 *)(here + i) = v;
             }
             if (mu)
                 v = make_float4(fmaf(b[j].x - v.x, m[j].x, v.x), fmaf(b[j].y - v.y, m[j].y, v.y), fmaf(b[j].z - v.z, m[j].z, v.z),
                                 fmaf(b[j].w - v.w, m[j].w, v.w));
-            *(float4 *)(xs + i) = v;
+            xs.quad(i >> 2) = mv_if(i < k, v);
         }
-        return;
+    } else {
+        float inv = 0.f;
+        if (normed) {
+            const float *v = NORM ? in.x : in.y;
+#pragma unroll 4
+            for (int i = tid; i < k; i += NT) ss = fmaf(v[i], v[i], ss);
+            inv = scale();
+        }
+#pragma unroll 4
+        for (int i = tid; i < end; i += NT) {
+            float v = 0.f;
+            if (i < k) {
+                v = in.x[i];
+                if (NORM) v *= inv * in.norm[i];
+                else if (add) v += in.y[i] * inv * in.w[i];
+                if (one) {
+                    if (in.x_out) in.x_out[i] = v;
+                    if (state) here[i] = v;
+                }
+                if (mu) v = fmaf((shift ? before[i] : 0.f) - v, mu[i], v);
+            } else if (one && in.x_out && i < out) in.x_out[i] = 0.f;
+            xs.at(i) = v;
+        }
+        start();
     }
-    if (!in.y && !(k & 3) && !in.x_out && !in.state && !mu && k <= 16384) { // a plain copy
-        float4 v[8];
-        const int n = (k + 2047) / 2048;
+}
+
+// Normed group by group and gated.  sums: k / 4 floats (XQ > 0: groups of a multiple of four values).
+template <int WAVES, int XQ, typename F>
+__device__ __forceinline__ void mv_gated(const FhMvAdd &in, int k, const FhRowInput &xs, float *ginv, float *sums, F start) {
+    constexpr int NT = WAVES * 64;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, gl = k / in.groups, end = 2 * xs.plane;
+    if constexpr (XQ > 0) {
+        float4 x[XQ], g[XQ], w[XQ];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int i = (tid + 512 * j) * 4;
-            v[j] = *(const float4 *)(in.x + (i < k ? i : 0));
+        for (int j = 0; j < XQ; j++) {
+            const int i = (tid + NT * j) * 4, at = i < k ? i : 0;
+            x[j] = *(const float4 *)(in.x + at);
+            g[j] = *(const float4 *)(in.gate + at);
+            w[j] = *(const float4 *)(in.w ? in.w + (in.w_len == k ? at : at % in.w_len) : in.gate + at);
         }
         __builtin_amdgcn_sched_barrier(0);
         start();
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int i = (tid + 512 * j) * 4;
-            if (j < n && i < kp) *(float4 *)(xs + i) = i < k ? v[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int j = 0; j < XQ; j++) {
+            const int q = tid + NT * j;
+            if (q * 4 < k) sums[q] = fmaf(x[j].x, x[j].x, fmaf(x[j].y, x[j].y, fmaf(x[j].z, x[j].z, x[j].w * x[j].w)));
         }
-        for (int i = k + tid; i < kp; i += 512) xs[i] = 0.f;
-        return;
-    }
-    start();
-    if (!in.y && !(k & 3) && !in.x_out && !in.state && !mu) { // a longer one
-#pragma unroll 8
-        for (int i = tid * 4; i < kp; i += 2048) *(float4 *)(xs + i) = i < k ? *(const float4 *)(in.x + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-        return;
-    }
-    float inv = 0.f;
-    if (in.y) {
-        float ss = 0.f;
+        fh_lds_barrier();
+        for (int n = wave; n < in.groups; n += WAVES) {
+            float ss = 0.f;
+            for (int i = lane; i < gl >> 2; i += 64) ss += sums[n * (gl >> 2) + i];
+            ss = fh_wave_sum(ss);
+            if (lane == 0) ginv[n] = 1.0f / sqrtf(ss / (float)gl + in.eps) * in.scale;
+        }
+        fh_lds_barrier();
+#pragma unroll
+        for (int j = 0; j < XQ; j++) {
+            const int i = (tid + NT * j) * 4;
+            const float s = ginv[i < k ? i / gl : 0];
+            if (!in.w) w[j].x = w[j].y = w[j].z = w[j].w = 1.f;
+            const float4 v = make_float4(x[j].x * s * w[j].x * fh_silu_f(g[j].x), x[j].y * s * w[j].y * fh_silu_f(g[j].y),
+                                         x[j].z * s * w[j].z * fh_silu_f(g[j].z), x[j].w * s * w[j].w * fh_silu_f(g[j].w));
+            if (i < end) xs.quad(i >> 2) = mv_if(i < k, v);
+        }
+    } else {
 #pragma unroll 4
-        for (int i = tid; i < k; i += 512) ss = fmaf(in.y[i], in.y[i], ss);
-        ss = fh_wave_sum(ss);
-        if (lane == 0) red[wave] = ss;
-        __syncthreads();
-        inv = 1.0f / sqrtf(mv_sum8(red) / (float)k + in.eps);
-    }
-    for (int i = tid; i < kp; i += 512) {
-        float v = 0.f;
-        if (i < k) {
-            v = in.x[i];
-            if (in.y) v += in.y[i] * inv * in.w[i];
-            if (one) {
-                if (in.x_out) in.x_out[i] = v;
-                if (in.state) here[i] = v;
-            }
-            if (mu) v = fmaf((shift ? before[i] : 0.f) - v, mu[i], v);
+        for (int i = tid; i < end; i += NT) xs.at(i) = i < k ? in.x[i] : 0.f;
+        start();
+        fh_lds_barrier();
+        for (int n = wave; n < in.groups; n += WAVES) {
+            float ss = 0.f;
+            for (int i = lane; i < gl; i += 64) ss = fmaf(xs.at(n * gl + i), xs.at(n * gl + i), ss);
+            ss = fh_wave_sum(ss);
+            if (lane == 0) ginv[n] = 1.0f / sqrtf(ss / (float)gl + in.eps) * in.scale;
         }
-        xs[i] = v;
+        fh_lds_barrier();
+#pragma unroll 4
+        for (int i = tid; i < k; i += NT) {
+            float v = xs.at(i) * ginv[i / gl];
+            if (in.w) v *= in.w[i % in.w_len];
+            xs.at(i) = v * fh_silu_f(in.gate[i]);
+        }
     }
 }
 
-// Normed group by group and gated.
-__device__ __forceinline__ void mv_gated(const FhMvAdd &in, int k, int kp, float *xs, float *ginv) {
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, gl = k / in.groups;
-#pragma unroll 4
-    for (int i = tid; i < kp; i += 512) xs[i] = i < k ? in.x[i] : 0.f;
-    __syncthreads();
-    for (int g = wave; g < in.groups; g += 8) {
-        float ss = 0.f;
-        for (int i = lane; i < gl; i += 64) ss = fmaf(xs[g * gl + i], xs[g * gl + i], ss);
-        ss = fh_wave_sum(ss);
-        if (lane == 0) ginv[g] = 1.0f / sqrtf(ss / (float)gl + in.eps) * in.scale;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int i = tid; i < k; i += 512) {
-        float v = xs[i] * ginv[i / gl];
-        if (in.w) v *= in.w[in.w_len == k ? i : i % in.w_len];
-        xs[i] = v * fh_silu_f(in.gate[i]);
-    }
-}
-
-template <int ROWS, bool GATED>
-__global__ __launch_bounds__(512, 4) void k_matvec_mix(FhMvAdd in, int k, int kp, MvMixes segs) {
-    constexpr int AHEAD = ROWS == 1 ? 8 : 16 / ROWS;
-    extern __shared__ __attribute__((aligned(16))) float xs[]; // [kp | groups]
-    __shared__ float red[8];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+template <int WAVES, int AHEAD, int XQ, int MODE>
+__global__ __launch_bounds__(WAVES * 64) void k_matvec_mix(FhMvAdd in, int k, int kp, MvMixes segs) {
+    extern __shared__ __attribute__((aligned(16))) float lds[]; // [kp in whole pieces | groups | k / 4 (gated)]
+    __shared__ float red[WAVES];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     int tile = blockIdx.x, si = 0;
     while (si + 1 < segs.n && tile >= segs.tiles[si]) tile -= segs.tiles[si++];
     const FhMvMix seg = segs.s[si];
-    const int row0 = (tile * 8 + wave) * ROWS;
-    FhRowStream<ROWS, AHEAD> rows;
-#pragma unroll
-    for (int r = 0; r < ROWS; r++) rows.w[r] = seg.w + (int64_t)(row0 + r < seg.n ? row0 + r : seg.n - 1) * kp;
-    if (GATED) {
-        rows.start(kp);
-        mv_gated(in, k, kp, xs, xs + kp);
-    } else {
-        mv_input(in, seg.mu, k, kp, xs, red, [&]() { rows.start(kp); });
-    }
-    __syncthreads();
-    float acc[ROWS];
-#pragma unroll
-    for (int r = 0; r < ROWS; r++) acc[r] = 0.f;
-    rows.run(xs, acc);
-#pragma unroll
-    for (int r = 0; r < ROWS; r++) acc[r] = fh_wave_sum(acc[r]);
-    if (lane == 0)
-#pragma unroll
-        for (int r = 0; r < ROWS; r++)
-            if (row0 + r < seg.n) {
-                float v = acc[r];
-                if (seg.act == FH_MV_ACT_RELU2) v = fmaxf(v, 0.f) * fmaxf(v, 0.f);
-                else if (seg.act == FH_MV_ACT_TANH) v = tanhf(v);
-                seg.y[row0 + r] = v;
-            }
+    const int nt = segs.tiles[si], first = wave * nt + tile, step = WAVES * nt;
+    const FhRowInput xs{lds, fh_row_pieces(kp) * 256};
+    FhRowDeal<AHEAD> rows;
+    const auto start = [&]() { rows.start(seg.w, kp, first, step, seg.n); };
+    if constexpr (MODE == MV_GATED) mv_gated<WAVES, XQ>(in, k, xs, lds + 2 * xs.plane, lds + 2 * xs.plane + in.groups, start);
+    else mv_input<WAVES, XQ, MODE>(in, seg.mu, k, kp, xs, red, start);
+    fh_lds_barrier();
+    rows.run(xs, [&](int i, float v) {
+        if (seg.act == FH_MV_ACT_RELU2) v = fmaxf(v, 0.f) * fmaxf(v, 0.f);
+        else if (seg.act == FH_MV_ACT_TANH) v = tanhf(v);
+        if (lane == 0) seg.y[first + i * step] = v;
+    });
 }
 
-template <int ROWS, bool GATED>
-static fh_status matvec_mix_go(fh_device *dev, const FhMvAdd &in, int k, int kp, const MvMixes &ms, int tiles) {
-    const size_t lds = (size_t)(kp + (GATED ? in.groups : 0)) * 4;
-    FH_REQUIRE(lds <= 150 * 1024, "k = %d too long for the matvec", k);
-    if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_matvec_mix<ROWS, GATED>, lds));
-    k_matvec_mix<ROWS, GATED><<<dim3((unsigned)tiles), 512, lds, dev->stream>>>(in, k, kp, ms);
+template <int WAVES, int AHEAD, int XQ, int MODE>
+static fh_status matvec_mix_go(fh_device *dev, const FhMvAdd &in, int k, const MvMixes &ms, int tiles) {
+    const int kp = (int)fh_pad64(k);
+    const size_t lds = (size_t)(fh_row_pieces(kp) * 512 + (MODE == MV_GATED ? in.groups + (XQ ? k / 4 : 0) : 0)) * 4;
+    if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_matvec_mix<WAVES, AHEAD, XQ, MODE>, lds));
+    k_matvec_mix<WAVES, AHEAD, XQ, MODE><<<dim3((unsigned)tiles), WAVES * 64, lds, dev->stream>>>(in, k, kp, ms);
     FH_HIP(hipGetLastError());
     return FH_OK;
 }
 
+// Few rows: workgroups of four wavefronts, a row each, with up to 8 KB on their way (every workgroup reads the whole input, so there are no more of them than
+// that).  us, eight wavefronts / four: 128 x 1024 2.9 / 2.5, 512 x 2048 4.1 / 3.0, 1024 x 4096 5.3 / 4.4, 2048 x 1024 3.9 / 3.0, 4096 x 1024 4.4 / 4.0; the other way
+// round 7000 x 1000 5.6 / 6.9, 2048 x 2048 4.0 / 4.1.  Inputs of 4097 values and more with nothing or a norm on their way in: 1024 x 14336 9.3 / 8.4.
+static fh_status matvec_mix(fh_device *dev, const FhMvAdd &in, int k, const FhMvMix *segs, int n_segs) {
+    MvMixes ms{};
+    int n[FH_MV_MAX], total = 0;
+    bool shift = in.state;
+    ms.n = n_segs;
+    for (int i = 0; i < n_segs; i++) ms.s[i] = segs[i], total += n[i] = segs[i].n, shift = shift || segs[i].mu;
+    const int mode = in.gate ? MV_GATED : in.norm ? MV_NORM : shift ? MV_SHIFT : in.y ? MV_ADD : in.x_out ? MV_SHIFT : MV_PLAIN;
+    const bool few = total <= (k <= 1024 ? 16 : 4) * dev->compute_units && (k <= 4096 || mode == MV_PLAIN || mode == MV_NORM);
+    const int tiles = fh_row_share(n, n_segs, few ? (total + 3) / 4 + n_segs - 1 : dev->compute_units, ms.tiles);
+    auto aligned = [](const void *p) { return !((uintptr_t)p & 15); };
+    bool quads = !(k & 3) && k <= 16384 && aligned(in.x) && aligned(in.y) && aligned(in.w) && aligned(in.norm) && aligned(in.x_out) && aligned(in.state) && aligned(in.gate);
+    for (int i = 0; i < n_segs; i++) quads = quads && aligned(segs[i].mu);
+    if (in.gate) quads = quads && !(k / in.groups & 3) && !(in.w && (in.w_len & 3));
+#define MV_MIX(W_, A_, XQ_)                                                                 \
+    switch (mode) {                                                                         \
+    case MV_PLAIN: return matvec_mix_go<W_, A_, XQ_, MV_PLAIN>(dev, in, k, ms, tiles);      \
+    case MV_NORM: return matvec_mix_go<W_, A_, XQ_, MV_NORM>(dev, in, k, ms, tiles);        \
+    case MV_ADD: return matvec_mix_go<W_, A_, XQ_, MV_ADD>(dev, in, k, ms, tiles);          \
+    case MV_SHIFT: return matvec_mix_go<W_, A_, XQ_, MV_SHIFT>(dev, in, k, ms, tiles);      \
+    default: return matvec_mix_go<W_, A_, XQ_, MV_GATED>(dev, in, k, ms, tiles);            \
+    }
+    if (few) {
+        if (!quads) MV_MIX(4, 4, 0)
+        if (k <= 1024) MV_MIX(4, 2, 1)
+        if (k <= 2048) MV_MIX(4, 4, 2)
+        if (k <= 4096) MV_MIX(4, 8, 4)
+        if (mode == MV_PLAIN) return k <= 8192 ? matvec_mix_go<4, 8, 8, MV_PLAIN>(dev, in, k, ms, tiles) : matvec_mix_go<4, 8, 16, MV_PLAIN>(dev, in, k, ms, tiles);
+        return k <= 8192 ? matvec_mix_go<4, 8, 8, MV_NORM>(dev, in, k, ms, tiles) : matvec_mix_go<4, 8, 16, MV_NORM>(dev, in, k, ms, tiles);
+    }
+    if (!quads) MV_MIX(8, 4, 0)
+    if (k <= 2048) MV_MIX(8, 4, 1)
+    if (k <= 4096) MV_MIX(8, 4, 2)
+    if (k <= 8192) MV_MIX(8, 4, 4)
+    MV_MIX(8, 4, 8)
+#undef MV_MIX
+}
+
 fh_status fh_matvec_mix(fh_device *dev, const FhMvAdd &in, int k, const FhMvMix *segs, int n_segs) {
     FH_REQUIRE(n_segs >= 1 && n_segs <= FH_MV_MAX, "1 to %d matrices per launch", FH_MV_MAX);
-    FH_REQUIRE(in.x && in.x != in.x_out && (!in.y || in.w) && (!in.state || in.pos_dev), "bad input of a decode product");
+    FH_REQUIRE(in.x && in.x != in.x_out && (!in.y || in.w) && (!in.state || in.pos_dev) && !in.norm, "bad input of a decode product");
     FH_REQUIRE(!in.gate || (!in.y && !in.state && in.groups > 0 && k % in.groups == 0), "bad gated input of a decode product");
-    const int kp = (int)fh_pad64(k);
-    MvMixes ms{};
-    int64_t total = 0;
-    for (int i = 0; i < n_segs; i++) total += segs[i].n;
-    const int rows = total >= (int64_t)dev->compute_units * 8 * 4 ? 4 : total >= (int64_t)dev->compute_units * 8 * 2 ? 2 : 1;
-    int tiles = 0;
-    ms.n = n_segs;
-    for (int i = 0; i < n_segs; i++) {
-        ms.s[i] = segs[i];
-        ms.tiles[i] = (segs[i].n + 8 * rows - 1) / (8 * rows);
-        tiles += ms.tiles[i];
-    }
-    if (in.gate)
-        return rows == 4 ? matvec_mix_go<4, true>(dev, in, k, kp, ms, tiles) : rows == 2 ? matvec_mix_go<2, true>(dev, in, k, kp, ms, tiles)
-                                                                                        : matvec_mix_go<1, true>(dev, in, k, kp, ms, tiles);
-    return rows == 4 ? matvec_mix_go<4, false>(dev, in, k, kp, ms, tiles) : rows == 2 ? matvec_mix_go<2, false>(dev, in, k, kp, ms, tiles)
-                                                                                     : matvec_mix_go<1, false>(dev, in, k, kp, ms, tiles);
+    FH_REQUIRE((fh_pad64(k) + (in.gate ? in.groups : 0)) * 4 <= 150 * 1024, "k = %d too long for the matvec", k);
+    return matvec_mix(dev, in, k, segs, n_segs);
+}
+
+fh_status fh_matvec_norm(fh_device *dev, const float *x, int k, const float *w, float eps, const FhMvSeg *segs, int n_segs,
+                         float *norm_out) {
+    FH_REQUIRE(n_segs >= 1 && n_segs <= 3, "1 to 3 matrices per matvec launch");
+    FH_REQUIRE(fh_pad64(k) * 4 <= 120 * 1024, "k = %d too long for the matvec", k);
+    FhMvMix ms[3];
+    for (int i = 0; i < n_segs; i++) ms[i] = FhMvMix{segs[i].w, nullptr, segs[i].y, segs[i].n, FH_MV_ACT_NONE};
+    FhMvAdd in;
+    in.x = x, in.norm = w, in.eps = eps, in.x_out = norm_out, in.x_pad = true;
+    return matvec_mix(dev, in, k, ms, n_segs);
 }
 
 // ------------------------------------------------------------------------------ fh_qmatmul on bf16 rows

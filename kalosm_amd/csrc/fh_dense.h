@@ -43,6 +43,16 @@ __device__ __forceinline__ float fh_wave_sum(float v) {
     v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));  // quad_perm 1 0 3 2
     return v;
 }
+__device__ __forceinline__ float fh_wave_max(float v) {
+    typedef uint32_t pair __attribute__((ext_vector_type(2)));
+    const auto both = [](const pair &r) { return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])); };
+    v = both(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    v = both(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xF, 0xF, true)));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x124, 0xF, 0xF, true)));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true)));
+    return fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true)));
+}
 // silu, softplus and the logistic function with the full-precision exponential
 __device__ __forceinline__ float fh_silu_f(float z) { return z / (1.0f + expf(-z)); }
 __device__ __forceinline__ float fh_softplus_f(float z) { return fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))); }
@@ -72,61 +82,28 @@ __device__ __forceinline__ fh_f4 fh_mma32(const fh_f8 &a, const fh_f8 &b, fh_f4 
     return c;
 }
 
-// ROWS weight rows of one wavefront, streamed in pieces of 512 (a lane: eight values, 16 bytes) with AHEAD pieces on their way.
-// No request is under a condition - a lane past the end of the rows repeats the last eight values, a piece past the last one the
-// last piece: with a branch around a request the compiler can no longer count what is younger and waits for everything.
-template <int ROWS, int AHEAD>
-struct FhRowStream {
-    const uint16_t *w[ROWS];
-    uint4 u[AHEAD][ROWS];
-    int kp, pieces, lane8;
-    __device__ __forceinline__ void fetch(int slot, int piece) {
-        const int c = piece * 512 + lane8, at = c < kp ? c : kp - 8;
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) u[slot][r] = *(const uint4 *)(w[r] + at);
-    }
-    __device__ __forceinline__ void start(int kp_) {
-        kp = kp_, pieces = (kp + 511) / 512, lane8 = (threadIdx.x & 63) * 8;
-#pragma unroll
-        for (int i = 0; i < AHEAD; i++) fetch(i, i < pieces ? i : pieces - 1);
-    }
-    __device__ __forceinline__ void use(int slot, int piece, const float *x, float *acc) const {
-        const int c = piece * 512 + lane8;
-        if (c >= kp) return;
-        const float4 a = *(const float4 *)(x + c), b = *(const float4 *)(x + c + 4);
-#pragma unroll
-        for (int r = 0; r < ROWS; r++) {
-            acc[r] = fmaf(fh_bf_lo(u[slot][r].x), a.x, acc[r]);
-            acc[r] = fmaf(fh_bf_hi(u[slot][r].x), a.y, acc[r]);
-            acc[r] = fmaf(fh_bf_lo(u[slot][r].y), a.z, acc[r]);
-            acc[r] = fmaf(fh_bf_hi(u[slot][r].y), a.w, acc[r]);
-            acc[r] = fmaf(fh_bf_lo(u[slot][r].z), b.x, acc[r]);
-            acc[r] = fmaf(fh_bf_hi(u[slot][r].z), b.y, acc[r]);
-            acc[r] = fmaf(fh_bf_lo(u[slot][r].w), b.z, acc[r]);
-            acc[r] = fmaf(fh_bf_hi(u[slot][r].w), b.w, acc[r]);
-        }
-    }
-    // acc[r] += rows . x (x: kp values in the LDS), not yet summed over the lanes
-    __device__ __forceinline__ void run(const float *x, float *acc) {
-        int p = 0;
-        for (; p + AHEAD < pieces; p += AHEAD) {
-#pragma unroll
-            for (int i = 0; i < AHEAD; i++) {
-                use(i, p + i, x, acc);
-                fetch(i, p + i + AHEAD < pieces ? p + i + AHEAD : pieces - 1);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < AHEAD; i++)
-            if (p + i < pieces) use(i, p + i, x, acc);
-    }
-};
-
 // A barrier behind LDS writes that leaves requests to memory on their way.
 __device__ __forceinline__ void fh_lds_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+}
+
+// 16 bytes that are read once
+__device__ __forceinline__ uint4 fh_load_once(const uint16_t *p) {
+    typedef uint32_t words __attribute__((ext_vector_type(4)));
+    const words v = __builtin_nontemporal_load((const words *)p);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ float fh_dot8(const uint4 &w, const float4 &a, const float4 &b, float acc) {
+    acc = fmaf(fh_bf_lo(w.x), a.x, acc);
+    acc = fmaf(fh_bf_hi(w.x), a.y, acc);
+    acc = fmaf(fh_bf_lo(w.y), a.z, acc);
+    acc = fmaf(fh_bf_hi(w.y), a.w, acc);
+    acc = fmaf(fh_bf_lo(w.z), b.x, acc);
+    acc = fmaf(fh_bf_hi(w.z), b.y, acc);
+    acc = fmaf(fh_bf_lo(w.w), b.z, acc);
+    return fmaf(fh_bf_hi(w.w), b.w, acc);
 }
 
 // The rows of a matrix that one wavefront goes through, one after the other: `count` rows `hop` elements apart, in pieces of 512 (a lane:
@@ -152,10 +129,8 @@ struct FhRowDeal {
     int kp, pieces, count, left, piece, lane8;
     uint4 u[AHEAD];
     __device__ __forceinline__ void fetch(int slot) {
-        typedef uint32_t words __attribute__((ext_vector_type(4)));
         const int c = piece * 512 + lane8;
-        const words v = __builtin_nontemporal_load((const words *)(row + (c < kp ? c : kp - 8)));
-        __builtin_memcpy(&u[slot], &v, 16);
+        u[slot] = fh_load_once(row + (c < kp ? c : kp - 8));
         const bool end = ++piece == pieces;
         piece = end ? 0 : piece;
         left -= end;
@@ -180,14 +155,7 @@ struct FhRowDeal {
             for (int s = 0; s < AHEAD; s++) {
                 const float *at = x.xs + p * 256 + (lane8 >> 1);
                 const float4 a = *(const float4 *)at, b = *(const float4 *)(at + x.plane);
-                acc = fmaf(fh_bf_lo(u[s].x), a.x, acc);
-                acc = fmaf(fh_bf_hi(u[s].x), a.y, acc);
-                acc = fmaf(fh_bf_lo(u[s].y), a.z, acc);
-                acc = fmaf(fh_bf_hi(u[s].y), a.w, acc);
-                acc = fmaf(fh_bf_lo(u[s].z), b.x, acc);
-                acc = fmaf(fh_bf_hi(u[s].z), b.y, acc);
-                acc = fmaf(fh_bf_lo(u[s].w), b.z, acc);
-                acc = fmaf(fh_bf_hi(u[s].w), b.w, acc);
+                acc = fh_dot8(u[s], a, b, acc);
                 fetch(s);
                 if (++p == pieces) {
                     acc = fh_wave_sum(acc);

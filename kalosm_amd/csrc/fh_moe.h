@@ -45,41 +45,47 @@ fh_status fh_moe_prefill(fh_device *dev, int dtype, const FhMoe &m, const void *
 
 #ifdef __HIPCC__
 // The n-th best expert of one token and its weight, for all n < count, by one wavefront: every lane keeps the logits
-// e = lane + 64 i.  Ties go to the smaller index.  pick(n, expert, weight) runs in every lane.
-template <typename F>
-__device__ __forceinline__ void fh_moe_route(const float *z, int experts, float scale, int count, F pick) {
+// e = lane + 64 i, i < PER.  Ties go to the smaller index.  pick(n, expert, weight) runs in every lane.
+template <int PER, typename F>
+__device__ __forceinline__ void fh_moe_route_per(const float *z, int experts, float scale, int count, F pick) {
     const int lane = threadIdx.x & 63;
-    float v[FH_MOE_MAX_EXPERTS / 64];
-    const int per = (experts + 63) / 64;
+    float v[PER];
     float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < FH_MOE_MAX_EXPERTS / 64; i++) {
-        v[i] = i < per && lane + 64 * i < experts ? z[lane + 64 * i] : -INFINITY;
+    for (int i = 0; i < PER; i++) {
+        const int e = lane + 64 * i;
+        v[i] = z[e < experts ? e : 0];
+        v[i] = e < experts ? v[i] : -INFINITY;
         mx = fmaxf(mx, v[i]);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    mx = fh_wave_max(mx);
     float den = 0.f;
 #pragma unroll
-    for (int i = 0; i < FH_MOE_MAX_EXPERTS / 64; i++) den += v[i] == -INFINITY ? 0.f : expf(v[i] - mx);
+    for (int i = 0; i < PER; i++) den += v[i] == -INFINITY ? 0.f : expf(v[i] - mx);
     den = fh_wave_sum(den);
+    float best = mx;
     for (int n = 0; n < count; n++) {
-        float best = -INFINITY;
-        int bi = 0x7FFFFFFF;
+        int e = -1; // of those with the best logit the first
 #pragma unroll
-        for (int i = 0; i < FH_MOE_MAX_EXPERTS / 64; i++)
-            if (v[i] > best) best = v[i], bi = lane + 64 * i;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float ob = __shfl_xor(best, o, 64);
-            const int oi = __shfl_xor(bi, o, 64);
-            if (ob > best || (ob == best && oi < bi)) best = ob, bi = oi;
+        for (int i = PER - 1; i >= 0; i--) {
+            const uint64_t who = __ballot(v[i] == best);
+            e = who ? 64 * i + __builtin_ctzll(who) : e;
         }
-        if (bi >= experts) bi = 0; // only when no logit is a number
-        pick(n, bi, expf(best - mx) / den * scale);
+        if (e < 0 || best == -INFINITY) e = 0; // only when no logit is a number
+        pick(n, e, expf(best - mx) / den * scale);
+        best = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < FH_MOE_MAX_EXPERTS / 64; i++)
-            if (bi == lane + 64 * i) v[i] = -INFINITY;
+        for (int i = 0; i < PER; i++) {
+            v[i] = e == lane + 64 * i ? -INFINITY : v[i];
+            best = fmaxf(best, v[i]);
+        }
+        best = fh_wave_max(best);
     }
+}
+template <typename F>
+__device__ __forceinline__ void fh_moe_route(const float *z, int experts, float scale, int count, F pick) {
+    if (experts <= 64) fh_moe_route_per<1>(z, experts, scale, count, pick);
+    else if (experts <= 256) fh_moe_route_per<4>(z, experts, scale, count, pick);
+    else fh_moe_route_per<FH_MOE_MAX_EXPERTS / 64>(z, experts, scale, count, pick);
 }
 #endif

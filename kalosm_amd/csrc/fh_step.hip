@@ -1,5 +1,6 @@
 // Decode step kernels of the layer-list decoders (fh_step.h).
 #include "fh_step.h"
+#include <algorithm>
 
 static constexpr float FH_LOG2E = 1.4426950408889634f;
 
@@ -147,75 +148,118 @@ __device__ __forceinline__ void latent_step(const FhStep &st, T *ring, int cap, 
         }
 }
 
-// Gate and up products of the chosen experts: a workgroup takes 8 activations of one of them, two per wavefront, with AHEAD pieces of
-// their rows on their way.  Four (100 registers) where all workgroups of the launch are on the device at once with them, four a
-// compute unit, and the rows are longer than two; else two (62 registers, eight a compute unit): us of the launch, two / four / one
-// in a loop, width 2048 with a state space of 4096, top 6 of 1024 14.4 / 14.0 / 14.8, top 8 of 1024 17.1 / 22.6 / 17.6; width 512 and
-// top 8 of 2048 16.3 / 22.3 / 16.3.
-template <int AHEAD>
-__device__ __forceinline__ void expert_step(const FhStep &st, int b, float *lds) {
+// Gate and up products of the chosen experts, dealt out over `blocks` workgroups of four wavefronts: a wavefront takes one activation after
+// the other, its gate and its up row together, in pieces of 512 with 4 KB on their way (FhRowDeal has the reason).  The chosen experts have
+// to be known first, so every workgroup works them out.  us of the launch in a step of width 2048, top 6 of 64 experts of 1024 (50 MB: a plain read takes 9.0):
+// beside latent attention 14.9 / 12.9, beside a recurrence 15.5 / 13.8 (workgroups of eight activations, 16 KB a wavefront on their way / now).
+__device__ __forceinline__ void expert_step(const FhStep &st, int b, int blocks, float *lds) {
+    constexpr int AHEAD = 2, NX = 4;
     const FhMoe &m = st.moe;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, tiles = (m.ff + 7) / 8, slot = b / tiles, tile = b % tiles;
-    int *who = (int *)(lds + st.kp);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lane8 = lane * 8;
+    const int kp = st.kp, pieces = fh_row_pieces(kp), total = m.top * m.ff, step = blocks * 4, first = wave * blocks + b;
+    const FhRowInput xs{lds, pieces * 256};
+    int *who = (int *)(lds + 2 * xs.plane);
+    float4 x[NX]; // requested beside the router's logits
+#pragma unroll
+    for (int j = 0; j < NX; j++) {
+        const int i = (tid + 256 * j) * 4;
+        x[j] = *(const float4 *)(st.hn + (i < kp ? i : 0));
+    }
     if (wave == 0)
-        fh_moe_route(st.proj + m.col_z, m.experts, m.scale, slot + 1, [&](int n, int e, float w) {
-            if (n == slot && lane == 0) {
-                *who = e;
-                if (tile == 0) st.ids[slot] = e, st.wts[slot] = w;
+        fh_moe_route(st.proj + m.col_z, m.experts, m.scale, m.top, [&](int n, int e, float w) {
+            if (lane == 0) {
+                who[n] = e;
+                if (b == 0) st.ids[n] = e, st.wts[n] = w;
             }
         });
-    for (int i = tid * 4; i < st.kp; i += 1024) *(float4 *)(lds + i) = *(const float4 *)(st.hn + i);
-    __syncthreads();
-    const uint16_t *w = m.gate_up + (int64_t)*who * m.gu_stride;
-    FhRowStream<4, AHEAD> rows;
-    const int p0 = tile * 8 + wave * 2;
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int p = p0 + i < m.ff ? p0 + i : m.ff - 1;
-        rows.w[2 * i] = w + (int64_t)(p / 16 * 32 + p % 16) * st.kp;
-        rows.w[2 * i + 1] = rows.w[2 * i] + (int64_t)16 * st.kp;
+    for (int j = 0; j < NX; j++) {
+        const int i = (tid + 256 * j) * 4;
+        float4 v = x[j];
+        if (i >= kp) v.x = v.y = v.z = v.w = 0.f;
+        if (i < 2 * xs.plane) xs.quad(i >> 2) = v;
     }
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    rows.start(st.kp);
-    rows.run(lds, acc);
+    for (int i = (tid + 256 * NX) * 4; i < 2 * xs.plane; i += 1024) {
+        float4 v = zero;
+        if (i < kp) v = *(const float4 *)(st.hn + i);
+        xs.quad(i >> 2) = v;
+    }
+    fh_lds_barrier();
+    const int count = first < total ? (total - first + step - 1) / step : 0;
+    struct At { int slot, p; }; // activation p of a chosen expert
+    auto ahead = [&](At a, int by) {
+        a.p += by;
+        while (a.p >= m.ff) a.p -= m.ff, a.slot++;
+        return a;
+    };
+    auto gate = [&](const At &a) { // (its up row is the 16th behind it)
+        return m.gate_up + (int64_t)__builtin_amdgcn_readfirstlane(who[a.slot]) * m.gu_stride + (int64_t)(a.p / 16 * 32 + a.p % 16) * kp;
+    };
+    At next = ahead(At{0, 0}, count ? first : 0), now = next;
+    const uint16_t *row = gate(next);
+    int left = count, piece = 0;
+    uint4 g[AHEAD], u[AHEAD];
+    auto fetch = [&](int s) {
+        const int c = piece * 512 + lane8;
+        const uint16_t *at = row + (c < kp ? c : kp - 8);
+        g[s] = fh_load_once(at);
+        u[s] = fh_load_once(at + (int64_t)16 * kp);
+        if (++piece == pieces) {
+            piece = 0, left--;
+            if (left > 0) next = ahead(next, step), row = gate(next);
+        }
+    };
 #pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] = fh_wave_sum(acc[i]);
-    if (lane == 0)
+    for (int s = 0; s < AHEAD; s++) fetch(s);
+    float ag = 0.f, au = 0.f;
+    int p = 0, i = 0;
+    for (int t = 0; t < count * pieces; t += AHEAD) {
 #pragma unroll
-        for (int i = 0; i < 2; i++)
-            if (p0 + i < m.ff) st.act[(int64_t)slot * m.ffp + p0 + i] = fh_silu_f(acc[2 * i]) * acc[2 * i + 1];
+        for (int s = 0; s < AHEAD; s++) {
+            const float *at = xs.xs + p * 256 + lane * 4;
+            const float4 a = *(const float4 *)at, c = *(const float4 *)(at + xs.plane);
+            ag = fh_dot8(g[s], a, c, ag);
+            au = fh_dot8(u[s], a, c, au);
+            fetch(s);
+            if (++p == pieces) {
+                ag = fh_wave_sum(ag), au = fh_wave_sum(au);
+                if (i < count && lane == 0) st.act[(int64_t)now.slot * m.ffp + now.p] = fh_silu_f(ag) * au;
+                ag = au = 0.f, p = 0;
+                if (++i < count) now = ahead(now, step);
+            }
+        }
+    }
 }
 
-template <int RPT, int AHEAD>
+template <int RPT>
 __global__ __launch_bounds__(256) void k_step_recurrent(FhStep st, int n_mix) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     if ((int)blockIdx.x < n_mix) rec_step<RPT>(st, blockIdx.x, lds);
-    else expert_step<AHEAD>(st, (int)blockIdx.x - n_mix, lds);
+    else expert_step(st, (int)blockIdx.x - n_mix, (int)gridDim.x - n_mix, lds);
 }
-template <typename T, int AHEAD>
+template <typename T>
 __global__ __launch_bounds__(256) void k_step_latent(FhStep st, T *ring, int cap, int n_mix) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     if ((int)blockIdx.x < n_mix) latent_step<T>(st, ring, cap, blockIdx.x, lds);
-    else expert_step<AHEAD>(st, (int)blockIdx.x - n_mix, lds);
+    else expert_step(st, (int)blockIdx.x - n_mix, (int)gridDim.x - n_mix, lds);
 }
 
 fh_status fh_step_middle(fh_device *dev, int dtype, const FhStep &st, fh_kvcache *cache) {
     const FhMoe &m = st.moe;
-    const int n_exp = m.experts ? m.top * ((m.ff + 7) / 8) : 0;
-    size_t lds = m.experts ? (size_t)(st.kp + 4) * 4 : 0;
+    // two workgroups of four wavefronts a compute unit, if there is an activation for every wavefront
+    const int n_exp = m.experts ? std::min(2 * dev->compute_units, (m.top * m.ff + 3) / 4) : 0;
+    size_t lds = m.experts ? (size_t)(fh_row_pieces(st.kp) * 512 + m.top) * 4 : 0;
     if (st.kind == FH_MIX_RECURRENT) {
         const int n_mix = st.rec.heads * ((st.rec.vdim + 15) / 16), rpt = (st.rec.dim + 15) / 16;
         const size_t need = (size_t)(2 * st.rec.dim + 32) * 4;
         lds = lds > need ? lds : need;
         FH_REQUIRE(rpt <= 16, "recurrent state of %d rows (at most 256)", st.rec.dim);
         const dim3 grid((unsigned)(n_mix + n_exp));
-        const bool four = st.kp > 1024 && n_mix + n_exp <= 4 * dev->compute_units;
-#define STEP_RECURRENT(RPT_)                                                                                                      \
-    do {                                                                                                                          \
-        const void *fn = four ? (const void *)k_step_recurrent<RPT_, 4> : (const void *)k_step_recurrent<RPT_, 2>;                \
-        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, fn, lds));                                                                 \
-        if (four) k_step_recurrent<RPT_, 4><<<grid, 256, lds, dev->stream>>>(st, n_mix);                                          \
-        else k_step_recurrent<RPT_, 2><<<grid, 256, lds, dev->stream>>>(st, n_mix);                                               \
+#define STEP_RECURRENT(RPT_)                                                                                     \
+    do {                                                                                                         \
+        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_step_recurrent<RPT_>, lds));              \
+        k_step_recurrent<RPT_><<<grid, 256, lds, dev->stream>>>(st, n_mix);                                      \
     } while (0)
         if (rpt <= 2) STEP_RECURRENT(2);
         else if (rpt <= 4) STEP_RECURRENT(4);
@@ -227,13 +271,10 @@ fh_status fh_step_middle(fh_device *dev, int dtype, const FhStep &st, fh_kvcache
         const size_t need = (size_t)16 * 128 * 4;
         lds = lds > need ? lds : need;
         const dim3 grid((unsigned)(n_mix + n_exp));
-        const bool four = st.kp > 1024 && n_mix + n_exp <= 4 * dev->compute_units;
-#define STEP_LATENT(T_)                                                                                                           \
-    do {                                                                                                                          \
-        const void *fn = four ? (const void *)k_step_latent<T_, 4> : (const void *)k_step_latent<T_, 2>;                          \
-        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, fn, lds));                                                                 \
-        if (four) k_step_latent<T_, 4><<<grid, 256, lds, dev->stream>>>(st, (T_ *)cache->k, cache->capacity, n_mix);              \
-        else k_step_latent<T_, 2><<<grid, 256, lds, dev->stream>>>(st, (T_ *)cache->k, cache->capacity, n_mix);                   \
+#define STEP_LATENT(T_)                                                                                          \
+    do {                                                                                                         \
+        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_step_latent<T_>, lds));                   \
+        k_step_latent<T_><<<grid, 256, lds, dev->stream>>>(st, (T_ *)cache->k, cache->capacity, n_mix);          \
     } while (0)
         if (dtype == FH_F32) STEP_LATENT(float);
         else STEP_LATENT(uint16_t);
@@ -244,165 +285,207 @@ fh_status fh_step_middle(fh_device *dev, int dtype, const FhStep &st, fh_kvcache
 }
 
 // ------------------------------------------------------------------------------ output launch
-// One wavefront per row of the residual stream, eight rows per workgroup.  A row's weights - of the output projection, of
-// the chosen experts and of the always-on one - are one list of pieces of 512; a table in the LDS says where each
-// piece lies.  The inputs are requested beside the experts' numbers, so that they are there when the first pieces go out, and
-// reach the LDS (gate and norm of the recurrent mixers applied on the way) while those are on theirs.  No request is under a
-// condition (FhRowStream).
-struct OutPiece { const uint16_t *w; int kp, len, in; };
-enum { FH_OUT_AHEAD = 8 };
-
-// NO, NE: 512 values of the mixer and 2048 of the experts a thread holds in registers (more are read when they are staged).  Requests past
-// the end repeat a value, so a thread holds no more than the size needs: a mixer of 512 without experts 4.4 us, with NO = 8 5.4 (read as it is staged 4.8).
-template <int NO, int NE>
-__global__ __launch_bounds__(512, 4) void k_step_out(FhStep st, int n_pieces) {
-    extern __shared__ __attribute__((aligned(16))) float in[]; // [kpo | top * ffp | sffp | norm groups | pieces]
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+// Rows of the residual stream, dealt out over workgroups of eight wavefronts, one a compute unit.  A row's weights - of the output projection, of
+// the chosen experts and of the always-on one - are one list of pieces of 512, and a wavefront has 4 KB of them on their way (FhRowDeal has the
+// reason).  The inputs and the experts' numbers are requested first, so that they do not wait behind weights, then the first pieces of the output
+// projection, whose places are known.  us of the launch in a step of width 2048, seven experts of 1024: behind latent attention (38 MB, a plain read 7.2) 12.6 /
+// 11.5, a delta rule 15.7 / 13.0, a state space (46 MB, 8.4) 20.1 / 14.2 (one row a wavefront with 8 KB on their way / now; with a table of the
+// pieces in the LDS, a round trip for every piece, 14.4 / 16.4 / 16.5).
+// NO, NE, NS: fours of values of the mixer, of the experts and of the always-on one that a thread holds in registers, requested ahead of the weights;
+// NO = 0: mixers whose length or groups are no multiple of 4, and longer inputs, are read as they are staged.  PRE: the output projection has four pieces or more.
+template <int NO, int NE, int NS, bool PRE>
+__global__ __launch_bounds__(512) void k_step_out(FhStep st) {
+    constexpr int AHEAD = 4;
+    constexpr bool EARLY = NO > 0;
+    extern __shared__ __attribute__((aligned(16))) float lds[]; // [kpo | top * ffp | sffp | norm groups | kpo / 4 (EARLY, recurrent) | top]
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lane8 = lane * 8;
     const FhMoe &m = st.moe;
     const int n_e = m.experts ? m.top : 0, n_s = m.sff ? m.sffp : 0, n_in = st.kpo + n_e * m.ffp + n_s;
     const bool recurrent = st.kind == FH_MIX_RECURRENT;
-    const int n_g = recurrent ? (st.rec.norm_groups + 3) / 4 * 4 : 0;
-    float *ie = in + st.kpo, *is = ie + n_e * m.ffp, *ginv = in + n_in;
-    OutPiece *pt = (OutPiece *)(ginv + n_g);
-    const int po = (st.kpo + 511) / 512, pe = (m.ffp + 511) / 512;
+    const int n_g = recurrent ? (st.rec.norm_groups + 3) / 4 * 4 : 0, e0 = st.kpo, s0 = e0 + n_e * m.ffp;
+    const FhRowInput in{lds, n_in / 2}; // (all lengths are multiples of 64)
+    float *ginv = lds + n_in, *sums = ginv + n_g;
+    int *who = (int *)(sums + (EARLY && recurrent ? st.kpo / 4 : 0));
     const int inner = recurrent ? st.rec.heads * st.rec.vdim : st.lat.heads * st.lat.dv;
     const float *gate = recurrent ? st.proj + st.rec.col_g : st.o;
-    const bool early = st.kpo <= 512 * NO && n_e * m.ffp <= 2048 * NE;
-    float ov[NO], gv[NO];
-    float4 ev[NE];
-    if (early) {
-#pragma unroll
-        for (int j = 0; j < NO; j++) {
-            const int i = tid + 512 * j, at = i < inner ? i : inner - 1;
-            ov[j] = st.o[at];
-            gv[j] = gate[at];
-        }
-        if (n_e)
-#pragma unroll
-            for (int j = 0; j < NE; j++) {
-                const int i = (tid + 512 * j) * 4;
-                ev[j] = *(const float4 *)(st.act + (i < n_e * m.ffp ? i : 0));
-            }
-    }
-    for (int i = tid; i < n_pieces; i += 512) {
-        OutPiece p;
-        int k;
-        if (i < po) k = i * 512, p.w = st.wo + k, p.kp = st.kpo, p.in = k;
-        else if (i < po + n_e * pe) {
-            const int j = (i - po) / pe;
-            k = (i - po) % pe * 512;
-            p.w = m.down + (int64_t)st.ids[j] * m.down_stride + k, p.kp = m.ffp, p.in = st.kpo + j * m.ffp + k;
-        } else k = (i - po - n_e * pe) * 512, p.w = m.s_down + k, p.kp = m.sffp, p.in = st.kpo + n_e * m.ffp + k;
-        p.len = p.kp - k;
-        pt[i] = p;
-    }
-    __syncthreads();
-    const int row = (int)blockIdx.x * 8 + wave, r = row < st.width ? row : st.width - 1;
-    uint4 u[FH_OUT_AHEAD];
-    auto fetch = [&](int i) -> uint4 { // (a lane past the end of a short piece repeats its last eight values)
-        const OutPiece p = pt[i < n_pieces ? i : n_pieces - 1];
-        return *(const uint4 *)(p.w + (int64_t)r * p.kp + (lane * 8 < p.len ? lane * 8 : p.len - 8));
-    };
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < FH_OUT_AHEAD; i++) u[i] = fetch(i);
-    __builtin_amdgcn_sched_barrier(0);
     const bool gate_first = recurrent && st.rec.gate_first;
-    if (early) {
+    const int blocks = (int)gridDim.x, step = 8 * blocks, first = wave * blocks + (int)blockIdx.x;
+    const int count = first < st.width ? (st.width - first + step - 1) / step : 0;
+    const int expert = (n_e ? st.ids : (const int *)st.o)[tid < n_e ? tid : 0]; // (what is not there is read from the mixer's output and dropped)
+    float ew[EARLY ? NE : 1];
+    float4 o[EARLY ? NO : 1], g[EARLY ? NO : 1], ev[EARLY ? NE : 1], sg[EARLY ? NS : 1], su[EARLY ? NS : 1], nw[EARLY ? NO : 1];
+    const float *acts = n_e ? st.act : st.o, *weights = n_e ? st.wts : st.o, *shared = n_s ? st.s_gu : st.o, *norm = recurrent ? st.rec.norm : st.o;
+    if constexpr (EARLY) {
 #pragma unroll
         for (int j = 0; j < NO; j++) {
-            const int i = tid + 512 * j;
-            if (i < st.kpo) in[i] = i < inner ? (gate_first ? ov[j] * fh_silu_f(gv[j]) : ov[j]) : 0.f;
+            const int i = (tid + 512 * j) * 4, at = i < inner ? i : 0;
+            o[j] = *(const float4 *)(st.o + at);
+            g[j] = *(const float4 *)(gate + at);
+            nw[j] = *(const float4 *)(norm + (recurrent && st.rec.norm_len != inner ? at % st.rec.norm_len : at));
+        }
+#pragma unroll
+        for (int j = 0; j < NE; j++) {
+            const int i = (tid + 512 * j) * 4;
+            ev[j] = *(const float4 *)(acts + (i < n_e * m.ffp ? i : 0));
+            ew[j] = weights[i < n_e * m.ffp ? i / m.ffp : 0];
+        }
+#pragma unroll
+        for (int j = 0; j < NS; j++) { // (gate and up in alternating groups of 16)
+            const int i = (tid + 512 * j) * 4, at = i < n_s ? i / 16 * 32 + i % 16 : 0;
+            sg[j] = *(const float4 *)(shared + at);
+            su[j] = *(const float4 *)(shared + (n_s ? at + 16 : 0));
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    uint4 u[AHEAD];
+    // A row's stretches: the output projection, the experts, the always-on one; a place is k values into one, whose inputs begin at `from`.
+    const int n_seg = 1 + n_e + (n_s ? 1 : 0);
+    struct Place { int seg, k, kp, from; };
+    auto advance = [&](Place &a) { // true: to the next row
+        a.k += 512;
+        if (a.k < a.kp) return false;
+        a.k = 0, a.from += a.kp, a.seg++;
+        const bool end = a.seg == n_seg;
+        if (end) a.seg = a.from = 0;
+        a.kp = a.seg == 0 ? st.kpo : a.seg <= n_e ? m.ffp : m.sffp;
+        return end;
+    };
+    Place next{0, 0, st.kpo, 0}, now = next;
+    int row = first < st.width ? first : st.width - 1, left = count;
+    const uint16_t *w = st.wo + (int64_t)row * st.kpo;
+    auto fetch = [&](int s) { // (a lane past the end of a short piece repeats its last eight values)
+        const int c = next.k + lane8;
+        u[s] = fh_load_once(w + (c < next.kp ? c : next.kp - 8));
+        if (advance(next)) row += --left > 0 ? step : 0;
+        if (next.k == 0) {
+            const uint16_t *base = next.seg == 0 ? st.wo : next.seg > n_e ? m.s_down : m.down + (int64_t)__builtin_amdgcn_readfirstlane(who[next.seg - 1]) * m.down_stride;
+            w = base + (int64_t)row * next.kp;
+        }
+    };
+    if (PRE)
+#pragma unroll
+        for (int s = 0; s < AHEAD; s++) { // (the last one's place is worked out behind the barrier, where the experts are known)
+            const int c = s * 512 + lane8;
+            u[s] = fh_load_once(w + (c < st.kpo ? c : st.kpo - 8));
+        }
+    __builtin_amdgcn_sched_barrier(0);
+    if (tid < n_e) who[tid] = expert;
+    auto put = [&](int i, float4 v, float w) {
+        const int c = i % m.ffp;
+        v.x = c < m.ff ? w * v.x : 0.f, v.y = c + 1 < m.ff ? w * v.y : 0.f, v.z = c + 2 < m.ff ? w * v.z : 0.f, v.w = c + 3 < m.ff ? w * v.w : 0.f;
+        in.quad((e0 + i) >> 2) = v;
+    };
+    if constexpr (EARLY) {
+#pragma unroll
+        for (int j = 0; j < NO; j++) {
+            const int q = tid + 512 * j, i = q * 4;
+            if (gate_first) o[j] = make_float4(o[j].x * fh_silu_f(g[j].x), o[j].y * fh_silu_f(g[j].y), o[j].z * fh_silu_f(g[j].z), o[j].w * fh_silu_f(g[j].w));
+            if (i >= inner) o[j].x = o[j].y = o[j].z = o[j].w = 0.f;
+            if (!recurrent && i < st.kpo) in.quad(q) = o[j];
+            if (recurrent && i < st.kpo) sums[q] = fmaf(o[j].x, o[j].x, fmaf(o[j].y, o[j].y, fmaf(o[j].z, o[j].z, o[j].w * o[j].w)));
+        }
+#pragma unroll
+        for (int j = 0; j < NE; j++)
+            if ((tid + 512 * j) * 4 < n_e * m.ffp) put((tid + 512 * j) * 4, ev[j], ew[j]);
+#pragma unroll
+        for (int j = 0; j < NS; j++) {
+            const int i = (tid + 512 * j) * 4;
+            if (i < n_s)
+                in.quad((s0 + i) >> 2) = make_float4(fh_silu_f(sg[j].x) * su[j].x, fh_silu_f(sg[j].y) * su[j].y, fh_silu_f(sg[j].z) * su[j].z, fh_silu_f(sg[j].w) * su[j].w);
         }
     } else {
         for (int i = tid; i < st.kpo; i += 512) {
             float v = i < inner ? st.o[i] : 0.f;
             if (gate_first && i < inner) v *= fh_silu_f(gate[i]);
-            in[i] = v;
+            in.at(i) = v;
+        }
+        for (int i = tid * 4; i < n_e * m.ffp; i += 2048) put(i, *(const float4 *)(st.act + i), st.wts[i / m.ffp]);
+        for (int i = tid; i < n_s; i += 512) {
+            const int at = i / 16 * 32 + i % 16;
+            in.at(s0 + i) = fh_silu_f(st.s_gu[at]) * st.s_gu[at + 16];
         }
     }
-    auto put = [&](int i, const float4 &v) {
-        const int j = i / m.ffp, c = i % m.ffp;
-        const float w = st.wts[j];
-        *(float4 *)(ie + i) = make_float4(c < m.ff ? w * v.x : 0.f, c + 1 < m.ff ? w * v.y : 0.f, c + 2 < m.ff ? w * v.z : 0.f,
-                                          c + 3 < m.ff ? w * v.w : 0.f);
-    };
-    if (early) {
+    fh_lds_barrier();
+    if (PRE) { // where the requests above left off
+        next.k = (AHEAD - 1) * 512;
+        if (advance(next)) row += --left > 0 ? step : 0;
+        if (next.k == 0)
+            w = (next.seg == 0 ? st.wo : next.seg > n_e ? m.s_down : m.down + (int64_t)__builtin_amdgcn_readfirstlane(who[next.seg - 1]) * m.down_stride) + (int64_t)row * next.kp;
+    } else
 #pragma unroll
-        for (int j = 0; j < NE; j++)
-            if ((tid + 512 * j) * 4 < n_e * m.ffp) put((tid + 512 * j) * 4, ev[j]);
-    } else {
-        for (int i = tid * 4; i < n_e * m.ffp; i += 2048) put(i, *(const float4 *)(st.act + i));
-    }
-    for (int i = tid; i < n_s; i += 512) {
-        const int g = i / 16 * 32 + i % 16;
-        is[i] = fh_silu_f(st.s_gu[g]) * st.s_gu[g + 16];
-    }
-    __syncthreads();
+        for (int i = 0; i < AHEAD; i++) fetch(i);
     if (recurrent) {
         const FhRecurrent &rc = st.rec;
         const int gl = inner / rc.norm_groups;
-        for (int g = wave; g < rc.norm_groups; g += 8) {
+        for (int n = wave; n < rc.norm_groups; n += 8) {
             float ss = 0.f;
-            for (int i = lane; i < gl; i += 64) ss = fmaf(in[g * gl + i], in[g * gl + i], ss);
+            if (EARLY)
+                for (int i = lane; i < gl >> 2; i += 64) ss += sums[n * (gl >> 2) + i];
+            else
+                for (int i = lane; i < gl; i += 64) ss = fmaf(in.at(n * gl + i), in.at(n * gl + i), ss);
             ss = fh_wave_sum(ss);
-            if (lane == 0) ginv[g] = 1.0f / sqrtf(ss / (float)gl + rc.eps);
+            if (lane == 0) ginv[n] = 1.0f / sqrtf(ss / (float)gl + rc.eps);
         }
-        __syncthreads();
-        if (early) {
+        fh_lds_barrier();
+        if constexpr (EARLY) {
 #pragma unroll
             for (int j = 0; j < NO; j++) {
-                const int i = tid + 512 * j;
-                if (i >= inner) continue;
-                float v = in[i] * ginv[i / gl] * rc.norm[rc.norm_len == inner ? i : i % rc.norm_len];
-                if (!gate_first) v *= fh_silu_f(gv[j]);
-                in[i] = v;
+                const int q = tid + 512 * j, i = q * 4;
+                const float inv = ginv[i < inner ? i / gl : 0];
+                float4 v = make_float4(o[j].x * inv * nw[j].x, o[j].y * inv * nw[j].y, o[j].z * inv * nw[j].z, o[j].w * inv * nw[j].w);
+                if (!gate_first) v = make_float4(v.x * fh_silu_f(g[j].x), v.y * fh_silu_f(g[j].y), v.z * fh_silu_f(g[j].z), v.w * fh_silu_f(g[j].w));
+                if (i >= inner) v.x = v.y = v.z = v.w = 0.f;
+                if (i < st.kpo) in.quad(q) = v;
             }
         } else {
             for (int i = tid; i < inner; i += 512) {
-                float v = in[i] * ginv[i / gl] * rc.norm[rc.norm_len == inner ? i : i % rc.norm_len];
+                float v = in.at(i) * ginv[i / gl] * rc.norm[rc.norm_len == inner ? i : i % rc.norm_len];
                 if (!gate_first) v *= fh_silu_f(gate[i]);
-                in[i] = v;
+                in.at(i) = v;
             }
         }
-        __syncthreads();
+        fh_lds_barrier();
     }
     float acc = 0.f;
-    auto use = [&](int slot, int i) {
-        const OutPiece &p = pt[i];
-        if (lane * 8 < p.len) acc = dot8(u[slot], in + p.in + lane * 8, acc);
-    };
-    int b = 0;
-    for (; b + FH_OUT_AHEAD < n_pieces; b += FH_OUT_AHEAD) {
+    for (int i = 0; i < count;) {
 #pragma unroll
-        for (int i = 0; i < FH_OUT_AHEAD; i++) {
-            use(i, b + i);
-            u[i] = fetch(b + i + FH_OUT_AHEAD);
+        for (int s = 0; s < AHEAD; s++) {
+            const bool in_row = now.k + lane8 < now.kp;
+            const float *at = in.xs + ((now.from + now.k) >> 1) + (in_row ? lane * 4 : 0);
+            const float more = fh_dot8(u[s], *(const float4 *)at, *(const float4 *)(at + in.plane), acc);
+            acc = in_row ? more : acc;
+            fetch(s);
+            if (advance(now)) {
+                acc = fh_wave_sum(acc);
+                if (i < count && lane == 0) st.x[first + i * step] += acc;
+                acc = 0.f, i++;
+            }
         }
     }
-#pragma unroll
-    for (int i = 0; i < FH_OUT_AHEAD; i++)
-        if (b + i < n_pieces) use(i, b + i);
-    acc = fh_wave_sum(acc);
-    if (lane == 0 && row < st.width) st.x[row] += acc;
 }
 
 fh_status fh_step_out(fh_device *dev, const FhStep &st) {
     const FhMoe &m = st.moe;
     const int n_e = m.experts ? m.top : 0, n_s = m.sff ? m.sffp : 0;
-    const int pieces = (st.kpo + 511) / 512 + n_e * ((m.ffp + 511) / 512) + (n_s + 511) / 512;
-    const size_t lds = (size_t)(st.kpo + n_e * m.ffp + n_s + (st.kind == FH_MIX_RECURRENT ? (st.rec.norm_groups + 3) / 4 * 4 : 0)) * 4 +
-                       (size_t)pieces * sizeof(OutPiece);
-    FH_REQUIRE(lds <= 156 * 1024, "a decode step stages at most 156 KB of inputs (%zu bytes needed)", lds);
-#define STEP_OUT(NO_, NE_)                                                                                        \
-    do {                                                                                                          \
-        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_step_out<NO_, NE_>, lds));                 \
-        k_step_out<NO_, NE_><<<dim3((unsigned)((st.width + 7) / 8)), 512, lds, dev->stream>>>(st, pieces);        \
+    const bool recurrent = st.kind == FH_MIX_RECURRENT;
+    const size_t need = (size_t)(st.kpo + n_e * m.ffp + n_s + (recurrent ? (st.rec.norm_groups + 3) / 4 * 4 : 0) + n_e) * 4;
+    FH_REQUIRE(need <= 156 * 1024, "a decode step stages at most 156 KB of inputs (%zu bytes needed)", need);
+    const int inner = recurrent ? st.rec.heads * st.rec.vdim : st.lat.heads * st.lat.dv;
+    bool quads = inner % 4 == 0 && need + st.kpo <= 156 * 1024 && ((uintptr_t)st.o & 15) == 0;
+    if (recurrent) quads = quads && inner / st.rec.norm_groups % 4 == 0 && st.rec.norm_len % 4 == 0 && ((uintptr_t)(st.proj + st.rec.col_g) & 15) == 0;
+    const dim3 grid((unsigned)std::min(dev->compute_units, (st.width + 7) / 8));
+#define STEP_OUT(NO_, NE_, NS_, PRE_)                                                                                         \
+    do {                                                                                                                      \
+        const size_t lds = need + (NO_ && recurrent ? st.kpo : 0);                                                            \
+        if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_step_out<NO_, NE_, NS_, PRE_>, lds));                  \
+        k_step_out<NO_, NE_, NS_, PRE_><<<grid, 512, lds, dev->stream>>>(st);                                                 \
     } while (0)
-    if (st.kpo <= 512 && n_e * m.ffp <= 2048) STEP_OUT(1, 1);
-    else if (st.kpo <= 1024 && n_e * m.ffp <= 2048) STEP_OUT(2, 1);
-    else if (st.kpo <= 2048 && n_e * m.ffp <= 4096) STEP_OUT(4, 2);
-    else STEP_OUT(8, 4);
+    if (!quads || st.kpo > 8192 || n_e * m.ffp > 8192 || n_s > 2048) STEP_OUT(0, 1, 1, false);
+    else if (st.kpo <= 1536 && n_e * m.ffp <= 2048) STEP_OUT(1, 1, 1, false);
+    else if (st.kpo <= 1536) STEP_OUT(1, 4, 1, false);
+    else if (st.kpo <= 2048 && n_e * m.ffp <= 4096) STEP_OUT(1, 2, 1, true);
+    else if (st.kpo <= 4096) STEP_OUT(2, 4, 1, true);
+    else STEP_OUT(4, 4, 1, true);
 #undef STEP_OUT
     FH_HIP(hipGetLastError());
     return FH_OK;

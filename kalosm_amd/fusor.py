@@ -7,6 +7,7 @@ on the host except shape bookkeeping and host<->device copies.
 from __future__ import annotations
 
 import ctypes as C
+import math
 from typing import Optional, Sequence
 
 import numpy as np
@@ -213,19 +214,20 @@ class Tensor:
     # ---- operators -------------------------------------------------------------------------
     def q_mat_mul(self, w: "QMatrix", out: Optional["Tensor"] = None) -> "Tensor":
         """Tensor::q_mat_mul (fusor-ml/fusor/src/lib.rs:1132-1223); rank 1, 2 or 3 (rank 1 is viewed as [1, k])."""
-        k = self.shape[-1]
+        shape = self.shape  # (a decode step's product is 3 us on the device: math.prod and plain integers, not numpy and c_void_p)
+        k = shape[-1]
         if k != w.k:
             raise FusorHipError(_lib.FH_ERR_INVALID,
                                 f"Matrix dimension mismatch: lhs columns ({k}) != weight in_features ({w.k})")
-        m = int(np.prod(self.shape[:-1])) if len(self.shape) > 1 else 1
-        oshape = (*self.shape[:-1], w.n) if len(self.shape) > 1 else (w.n,)
-        out = out or Tensor(self.device, oshape, "f32")
+        out = out or Tensor(self.device, (*shape[:-1], w.n) if len(shape) > 1 else (w.n,), "f32")
         L = self.device._lib
         if self.dtype == "bf16":
-            check(L.fh_qmatmul_bf16(w._h, C.c_void_p(self.ptr), m, C.c_void_p(out.ptr)))
+            status = L.fh_qmatmul_bf16(w._h, self.ptr, math.prod(shape[:-1]), out.ptr)
         else:
             assert self.dtype == "f32"
-            check(L.fh_qmatmul(w._h, C.c_void_p(self.ptr), m, C.c_void_p(out.ptr)))
+            status = L.fh_qmatmul(w._h, self.ptr, math.prod(shape[:-1]), out.ptr)
+        if status:
+            check(status)
         return out
 
     def matmul(self, rhs: "Tensor", rhs_transposed: bool = False, out: Optional["Tensor"] = None) -> "Tensor":

@@ -531,6 +531,18 @@ fh_status fh_rows_to_act(fh_device *dev, int dtype, const float *x, int64_t ldx,
     return FH_OK;
 }
 
+// Sums of squares of a row: fours of values (single ones where their number is no multiple of 4) dealt out to 512 threads, eight wavefronts' sums in pairs.  A
+// workgroup of four wavefronts has two of those threads' chains a thread (ss[1]: those of threads 256 on), so a row's norm has the same bits in every launch.
+template <int WAVES>
+__device__ __forceinline__ void row_sums(const float (&ss)[8 / WAVES], float *red) {
+#pragma unroll
+    for (int h = 0; h < 8 / WAVES; h++) {
+        const float s = fh_wave_sum(ss[h]);
+        if ((threadIdx.x & 63) == 0) red[h * WAVES + (threadIdx.x >> 6)] = s;
+    }
+}
+__device__ __forceinline__ float row_sum(const float *red) { return ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7])); }
+
 // ------------------------------------------------------------------------------ the output matrix for several rows
 // Bound by the weights, which the matvec reads again for every row (16 rows of 4096 and a matrix of 32768: 16 x 45 us), so up to 16
 // rows share one pass over them on the matrix cores.  The rows stay f32: each value is cut into three bf16 numbers of 8 bits (24
@@ -549,27 +561,28 @@ int fh_head_rows_from(int k, int n) {
 }
 struct HeadRows { int row[HEAD_ROWS], place[HEAD_ROWS], n; };
 
-// Final norm of the rows (the arithmetic of k_matvec_norm, addition for addition: the normed row that a pass gives back has the same
+// Final norm of the rows (the arithmetic of k_matvec_mix, addition for addition: the normed row that a pass gives back has the same
 // bits however many rows it has) and their three terms in the order of the MFMA operand: 64 of k: two
 // steps of 32: three terms: lane l (row l % 16, k = 8 (l / 16) .. + 7): 16 bytes.  Rows that are not there are zeros.
 __global__ __launch_bounds__(256) void k_head_x(const float *__restrict__ x, int k, int kp, const float *__restrict__ nw, float eps,
                                                 HeadRows rows, uint16_t *__restrict__ xf, float *__restrict__ norm_out) {
-    __shared__ float red[4];
+    __shared__ float red[8];
     const int tid = threadIdx.x, r = blockIdx.x;
     const bool there = r < rows.n;
     const float *xr = x + (int64_t)rows.row[there ? r : 0] * k;
-    float ss = 0.f;
-    if (!(k & 3))
-        for (int i = tid * 4; i < k; i += 1024) {
-            const float4 v = *(const float4 *)(xr + i);
-            ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
-        }
-    else
-        for (int i = tid; i < k; i += 256) ss = fmaf(xr[i], xr[i], ss);
-    ss = fh_wave_sum(ss);
-    if ((tid & 63) == 0) red[tid >> 6] = ss;
+    float ss[2] = {0.f, 0.f};
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+        if (!(k & 3))
+            for (int i = (tid + 256 * h) * 4; i < k; i += 2048) {
+                const float4 v = *(const float4 *)(xr + i);
+                ss[h] = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss[h]))));
+            }
+        else
+            for (int i = tid + 256 * h; i < k; i += 512) ss[h] = fmaf(xr[i], xr[i], ss[h]);
+    row_sums<4>(ss, red);
     __syncthreads();
-    const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)k + eps);
+    const float inv = 1.0f / sqrtf(row_sum(red) / (float)k + eps);
     for (int i = tid; i < kp; i += 256) {
         const float v = there && i < k ? xr[i] * inv * nw[i] : 0.f;
         if (r == rows.n - 1) norm_out[i] = v;
@@ -833,12 +846,6 @@ fh_status fh_low_rank_tanh(fh_device *dev, const float *x, int kp, int rows, con
 // (Before, the input's branches alone cost a third of that: with them in the code, though not taken, 4096 x 4096 took 9.7 us for 8.0.)
 struct MvMixes { FhMvMix s[FH_MV_MAX]; int tiles[FH_MV_MAX]; int n; };
 
-template <int WAVES>
-__device__ __forceinline__ float mv_sum(const float *red) {
-    const float s = (red[0] + red[1]) + (red[2] + red[3]);
-    return WAVES == 4 ? s : s + ((red[4] + red[5]) + (red[6] + red[7]));
-}
-
 __device__ __forceinline__ float4 mv_if(bool c, float4 v) { // (v or zeros: as one choice of two float4 it would be one of addresses, in scratch memory)
     return make_float4(c ? v.x : 0.f, c ? v.y : 0.f, c ? v.z : 0.f, c ? v.w : 0.f);
 }
@@ -850,7 +857,7 @@ enum { MV_PLAIN = 0, MV_NORM = 1, MV_ADD = 2, MV_SHIFT = 3, MV_GATED = 4 };
 template <int WAVES, int XQ, int MODE, typename F>
 __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int k, int kp, const FhRowInput &xs, float *red, F start) {
     constexpr int NT = WAVES * 64;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, end = 2 * xs.plane; // (whole pieces)
+    const int tid = threadIdx.x, end = 2 * xs.plane; // (whole pieces)
     constexpr bool NORM = MODE == MV_NORM, SHIFT = MODE == MV_SHIFT, ADD = MODE == MV_ADD || SHIFT;
     if (!SHIFT) mu = nullptr;
     const bool add = MODE == MV_ADD || (SHIFT && in.y), normed = NORM || add, one = blockIdx.x == 0;
@@ -860,12 +867,11 @@ __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int
     float *here = state + (pos & 1) * k;
     const bool shift = mu && pos > 0;
     const int out = NORM ? kp : k; // values of x_out
-    float ss = 0.f;
+    float ss[8 / WAVES] = {0.f};
     const auto scale = [&]() { // of the norm, from the threads' sums of squares
-        ss = fh_wave_sum(ss);
-        if (lane == 0) red[wave] = ss;
+        row_sums<WAVES>(ss, red);
         fh_lds_barrier();
-        return 1.0f / sqrtf(mv_sum<WAVES>(red) / (float)k + in.eps);
+        return 1.0f / sqrtf(row_sum(red) / (float)k + in.eps);
     };
     if constexpr (XQ > 0) {
         float4 x[XQ], y[ADD ? XQ : 1], w[MODE ? XQ : 1], m[SHIFT ? XQ : 1], b[SHIFT ? XQ : 1];
@@ -894,7 +900,8 @@ __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int
 #pragma unroll
             for (int j = 0; j < XQ; j++) {
                 const float4 v = NORM ? x[j] : y[j];
-                ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
+                float &t = ss[j % (8 / WAVES)];
+                t = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, t))));
             }
             inv = scale();
         }
@@ -918,8 +925,10 @@ __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int
         float inv = 0.f;
         if (normed) {
             const float *v = NORM ? in.x : in.y;
-#pragma unroll 4
-            for (int i = tid; i < k; i += NT) ss = fmaf(v[i], v[i], ss);
+            for (int i = tid; i < k; i += 512)
+#pragma unroll
+                for (int h = 0; h < 8 / WAVES; h++)
+                    if (i + NT * h < k) ss[h] = fmaf(v[i + NT * h], v[i + NT * h], ss[h]);
             inv = scale();
         }
 #pragma unroll 4
@@ -927,7 +936,7 @@ __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int
             float v = 0.f;
             if (i < k) {
                 v = in.x[i];
-                if (NORM) v *= inv * in.norm[i];
+                if (NORM) v = v * inv * in.norm[i];
                 else if (add) v += in.y[i] * inv * in.w[i];
                 if (one) {
                     if (in.x_out) in.x_out[i] = v;
@@ -1004,7 +1013,7 @@ __device__ __forceinline__ void mv_gated(const FhMvAdd &in, int k, const FhRowIn
 template <int WAVES, int AHEAD, int XQ, int MODE>
 __global__ __launch_bounds__(WAVES * 64) void k_matvec_mix(FhMvAdd in, int k, int kp, MvMixes segs) {
     extern __shared__ __attribute__((aligned(16))) float lds[]; // [kp in whole pieces | groups | k / 4 (gated)]
-    __shared__ float red[WAVES];
+    __shared__ float red[8];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     int tile = blockIdx.x, si = 0;
     while (si + 1 < segs.n && tile >= segs.tiles[si]) tile -= segs.tiles[si++];

@@ -70,7 +70,8 @@ struct Q4kExtra {
 // i / (16 / RS) in the steps of accumulator a = 0 .. RS - 1.  The accumulator entries whose row and column name the
 // same block are the dots; the rest is discarded.  As many MFMAs per weight byte as with whole tiles, RS times the
 // workgroups: matrices with fewer row tiles than compute units fill the device in one launch.
-template <int FMT, int TPW, int PER, int EPI, int IN, int MR = 1, int RS = 1>
+// RAG: the blocks are no multiple of the wavefronts'; what a wavefront has past the last one is the last one again, times zero.
+template <int FMT, int TPW, int PER, int EPI, int IN, int MR = 1, int RS = 1, bool RAG = false>
 __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict__ x, float *__restrict__ y,
                                                       const float *__restrict__ ea, const float *__restrict__ eb,
                                                       int SW, const float *__restrict__ xres,
@@ -81,6 +82,7 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
     static_assert(RS == 1 || (FMT == FH_Q4_K && TPW == 1 && MR == 1 && IN == 0 && (EPI == FH_EPI_NONE || EPI == FH_EPI_ADD2)),
                   "row split: Q4_K, one tile part, one row, plain input, epilogues none / add2");
     static_assert(RS == 1 || RS == 2 || RS == 4, "row split");
+    static_assert(!RAG || (IN == 0 && TPW == 1 && MR == 1 && RS == 1 && EPI != FH_EPI_SWIGLU), "ragged: plain input, one tile, one row");
     constexpr int NB = PER * RS; // blocks a wavefront stages and multiplies
     // SwiGLU with one tile per wavefront: the "tile" is rows 8h .. 8h+7 of a gate tile (columns 0-7 of the MFMA) and
     // the same rows of the matching up tile (columns 8-15), h = workgroup parity: workgroups half as heavy as with a
@@ -107,7 +109,8 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t nout = EPI == FH_EPI_SWIGLU ? q.n / 2 : q.n;
     const int64_t tiles_out = (nout + 15) / 16;
-    const int b0 = wave * NB;
+    const int b0 = wave * NB, last = (int)(q.k >> 8) - 1 - b0; // (the host launches no wavefront without a block)
+    auto blk = [&](int r) { return RAG && r > last ? last : r; };
     // bytes of a tiled record, and per 256 activations and tile
     constexpr int REC = FMT == FH_Q4_0 ? 1152 : (FMT == FH_Q8_0 ? 1088 : (FMT == FH_Q5_0 ? 1408 : (FMT == FH_Q5_K ? 2816 : 2304)));
     constexpr int CHUNK = FMT == FH_Q8_0 ? 4352 : ((FMT == FH_Q5_0 || FMT == FH_Q5_K) ? 2816 : 2304);
@@ -162,7 +165,7 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
     float2 pm[IN == 2 ? PER : 1][8];
 #pragma unroll
     for (int i = 0; i < NB; i++) {
-        const int64_t at = (int64_t)(boff + b0 + i) * 256 + lane * 4;
+        const int64_t at = (int64_t)(boff + b0 + blk(i)) * 256 + lane * 4;
         if (IN != 2) xv[i] = *(const float4 *)(x + at);
 #pragma unroll
         for (int mr = 1; mr < MR; mr++) // rows past the valid ones repeat the last (never stored)
@@ -190,32 +193,32 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
 #pragma unroll
         for (int tp = 0; tp < TPW; tp++) {
             if constexpr (FMT == FH_Q5_0) { // the Q4_0 records, each followed by the lane's fifth bits (one byte per block)
-                w[tp][r].h.x = *(const uint32_t *)(ph[tp] + r * CHUNK);
-                w[tp][r].qa = *(const uint4 *)(pq[tp] + r * CHUNK);
-                w[tp][r].qb = *(const uint4 *)(pq[tp] + r * CHUNK + REC);
-                w[tp][r].qc.x = *(const uint32_t *)(pq[tp] + 1152 - 12 * lane + r * CHUNK);
-                w[tp][r].qc.y = *(const uint32_t *)(pq[tp] + 1152 - 12 * lane + r * CHUNK + REC);
+                w[tp][r].h.x = *(const uint32_t *)(ph[tp] + blk(r) * CHUNK);
+                w[tp][r].qa = *(const uint4 *)(pq[tp] + blk(r) * CHUNK);
+                w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * CHUNK + REC);
+                w[tp][r].qc.x = *(const uint32_t *)(pq[tp] + 1152 - 12 * lane + blk(r) * CHUNK);
+                w[tp][r].qc.y = *(const uint32_t *)(pq[tp] + 1152 - 12 * lane + blk(r) * CHUNK + REC);
             } else if constexpr (FMT == FH_Q5_K) { // the Q4_K record followed by the lane's eight qh bytes
-                w[tp][r].h = *(const uint4 *)(ph[tp] + r * CHUNK);
-                w[tp][r].qa = *(const uint4 *)(pq[tp] + r * CHUNK);
-                w[tp][r].qb = *(const uint4 *)(pq[tp] + r * CHUNK + 1024);
-                const uint2 hb = *(const uint2 *)(pq[tp] + 2048 - 8 * lane + r * CHUNK);
+                w[tp][r].h = *(const uint4 *)(ph[tp] + blk(r) * CHUNK);
+                w[tp][r].qa = *(const uint4 *)(pq[tp] + blk(r) * CHUNK);
+                w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * CHUNK + 1024);
+                const uint2 hb = *(const uint2 *)(pq[tp] + 2048 - 8 * lane + blk(r) * CHUNK);
                 w[tp][r].qc.x = hb.x;
                 w[tp][r].qc.y = hb.y;
             } else if (FMT == FH_Q4_0) {
-                w[tp][r].h.x = *(const uint32_t *)(ph[tp] + r * 2304);
-                w[tp][r].qa = *(const uint4 *)(pq[tp] + r * 2304);
-                w[tp][r].qb = *(const uint4 *)(pq[tp] + r * 2304 + 1152);
+                w[tp][r].h.x = *(const uint32_t *)(ph[tp] + blk(r) * 2304);
+                w[tp][r].qa = *(const uint4 *)(pq[tp] + blk(r) * 2304);
+                w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * 2304 + 1152);
             } else if (FMT == FH_Q8_0) {
-                w[tp][r].h.x = *(const uint32_t *)(ph[tp] + r * 4352);
-                w[tp][r].qa = *(const uint4 *)(pq[tp] + r * 4352);
-                w[tp][r].qb = *(const uint4 *)(pq[tp] + r * 4352 + 1088);
-                w[tp][r].qc = *(const uint4 *)(pq[tp] + r * 4352 + 2176);
-                w[tp][r].qd = *(const uint4 *)(pq[tp] + r * 4352 + 3264);
+                w[tp][r].h.x = *(const uint32_t *)(ph[tp] + blk(r) * 4352);
+                w[tp][r].qa = *(const uint4 *)(pq[tp] + blk(r) * 4352);
+                w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * 4352 + 1088);
+                w[tp][r].qc = *(const uint4 *)(pq[tp] + blk(r) * 4352 + 2176);
+                w[tp][r].qd = *(const uint4 *)(pq[tp] + blk(r) * 4352 + 3264);
             } else {
-                w[tp][r].h = *(const uint4 *)(ph[tp] + r * RS * 2304);
-                w[tp][r].qa = *(const uint4 *)(pq[tp] + r * RS * 2304);
-                w[tp][r].qb = *(const uint4 *)(pq[tp] + r * RS * 2304 + 1024);
+                w[tp][r].h = *(const uint4 *)(ph[tp] + blk(r) * RS * 2304);
+                w[tp][r].qa = *(const uint4 *)(pq[tp] + blk(r) * RS * 2304);
+                w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * RS * 2304 + 1024);
             }
         }
     // ---- 2. stage x (lane owns k = 256*b + 4*lane .. +3).  A wavefront stages exactly the blocks it multiplies:
@@ -227,6 +230,7 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
         const int i = ii % NB;
         const int b = (b0 + i) * MR + ii / NB; // image index: [block][row]
         float4 v = xv[ii];
+        if (RAG && i > last) v.x = v.y = v.z = v.w = 0.f;
         if (IN == 2) { // merge the splits: softmax weights exp(m_s - max), then num / den
             float mx = -INFINITY;
 #pragma unroll
@@ -631,6 +635,39 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
     qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0>(q, x, y, ea, eb, SW, xres, nw, eps, nsplit, rk);
 }
 
+// k of more than 16 blocks that no number of up to 16 wavefronts shares out evenly (43 of 11008 columns); epilogues none / add2
+template <int FMT, int PER, int EPI>
+__global__ __launch_bounds__(1024) void k_qmv_q4k_m1_rag(Q4K_M1_PARAMS) {
+    qmv_q4k_m1_body<FMT, 1, PER, EPI, 0, 1, 1, true>(q, x, y, ea, eb, SW, xres, nw, eps, nsplit, rk);
+}
+
+template <int FMT, int PER>
+static fh_status q4k_m1_rag_go(const fh_qmatrix *q, const float *x, float *y, int epi, const float *a, const float *b) {
+    const int SW = (int)(q->k / 256 + PER - 1) / PER, kb = SW * PER;
+    const size_t lds = (size_t)kb * Q4K_IMG * 16 + (size_t)kb * 64 + 16 * 64 + 64;
+    const auto kern = epi == FH_EPI_ADD2 ? k_qmv_q4k_m1_rag<FMT, PER, FH_EPI_ADD2> : k_qmv_q4k_m1_rag<FMT, PER, FH_EPI_NONE>;
+    FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
+    kern<<<dim3((unsigned)((q->n + 15) / 16)), dim3(64 * SW), lds, q->dev->stream>>>(fh_view(q), x, y, a, b, SW, nullptr, nullptr, 0.f, 0, FhRopeArgs{});
+    FH_HIP(hipGetLastError());
+    return FH_OK;
+}
+
+// us of one row of 4096 x 11008 by the kernels that took it (the batch kernel, the 5-bit formats element by element) / here: Q4_K 15.0 / 7.7, Q4_0 15.2 /
+// 7.2, Q8_0 18.4 / 10.8, Q5_0 124 / 9.4, Q5_K 165 / 9.5 (of 4096 x 14336, whose 56 blocks 14 wavefronts share, 9.9 in Q4_K).
+static fh_status q4k_m1_rag(const fh_qmatrix *q, const float *x, float *y, int epi, const float *a, const float *b) {
+    const bool two = q->k <= 32 * 256;
+#define RAG_GO(T_) return two ? q4k_m1_rag_go<T_, 2>(q, x, y, epi, a, b) : q4k_m1_rag_go<T_, 4>(q, x, y, epi, a, b)
+    switch (q->type) {
+    case FH_Q4_K: RAG_GO(FH_Q4_K);
+    case FH_Q5_K: RAG_GO(FH_Q5_K);
+    case FH_Q4_0: RAG_GO(FH_Q4_0);
+    case FH_Q5_0: RAG_GO(FH_Q5_0);
+    case FH_Q8_0: RAG_GO(FH_Q8_0);
+    }
+#undef RAG_GO
+    return FH_ERR_UNSUPPORTED;
+}
+
 template <int TPW, int PER, int EPI>
 static fh_status q4k_m1_launch(const fh_qmatrix *q, const float *x, float *y, const float *a, const float *b, int SW,
                                unsigned grid, size_t lds, const Q4kExtra &ex) {
@@ -918,6 +955,8 @@ static fh_status q4k_m1_any(const fh_qmatrix *q, const float *x, const Q4kExtra 
         per *= 2;
     }
     const int SW = kb / per;
+    if (SW > 16 && kb <= 64 && (epi == FH_EPI_NONE || epi == FH_EPI_ADD2) && ex.ksplit == 1 && ex.nsplit == 0 && !ex.nw)
+        return q4k_m1_rag(q, x, y, epi, a, b);
     if (SW > 16 || kb % per || tpw * per > 4) return FH_ERR_UNSUPPORTED;
     size_t lds = (size_t)kb * Q4K_IMG * 16 + (size_t)kb * 64 + (size_t)tpw * 16 * 64 + 64;
     if (lds > 160 * 1024) return FH_ERR_UNSUPPORTED;

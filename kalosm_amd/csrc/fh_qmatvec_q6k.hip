@@ -27,7 +27,8 @@ struct Q6KRegs {
 // Workgroup = SW wavefronts, one per k-slice of PER blocks; a wavefront multiplies its slice of TPW row tiles (with
 // the SwiGLU epilogue: gate tiles and the matching up tiles), stages the activations of its own blocks only (no
 // barrier before the products) and requests all its weight bytes before anything else.
-template <int TPW, int PER, int EPI>
+// RAG: the blocks are no multiple of the wavefronts'; what a wavefront has past the last one is the last one again, times zero.
+template <int TPW, int PER, int EPI, bool RAG = false>
 __global__ __launch_bounds__(1024) void k_qmv_q6k_m1(QView q, const float *__restrict__ x, float *__restrict__ y,
                                                       const float *__restrict__ ea, const float *__restrict__ eb,
                                                       int SW, const float *__restrict__ xup) {
@@ -44,7 +45,8 @@ __global__ __launch_bounds__(1024) void k_qmv_q6k_m1(QView q, const float *__res
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t nout = EPI == FH_EPI_SWIGLU ? q.n / 2 : q.n;
     const int64_t tiles_out = (nout + 15) / 16;
-    const int b0 = wave * PER;
+    const int b0 = wave * PER, last = (int)(q.k >> 8) - 1 - b0; // (the host launches no wavefront without a block)
+    auto blk = [&](int r) { return RAG && r > last ? last : r; };
     const uint8_t *rec[TPW];
 #pragma unroll
     for (int tp = 0; tp < TPW; tp++) {
@@ -61,7 +63,7 @@ __global__ __launch_bounds__(1024) void k_qmv_q6k_m1(QView q, const float *__res
     float4 xv[PER], uv[PER];
 #pragma unroll
     for (int i = 0; i < PER; i++) {
-        const int64_t at = (int64_t)(boff + b0 + i) * 256 + lane * 4;
+        const int64_t at = (int64_t)(boff + b0 + blk(i)) * 256 + lane * 4;
         xv[i] = *(const float4 *)(x + at);
         if (xup) uv[i] = *(const float4 *)(xup + at);
     }
@@ -74,7 +76,7 @@ __global__ __launch_bounds__(1024) void k_qmv_q6k_m1(QView q, const float *__res
     for (int r = 0; r < PER; r++)
 #pragma unroll
         for (int tp = 0; tp < TPW; tp++) {
-            const uint8_t *p = rec[tp] + r * 3360;
+            const uint8_t *p = rec[tp] + blk(r) * 3360;
             w[tp][r].l0 = *(const uint4 *)(p + lane * 16);
             w[tp][r].l1 = *(const uint4 *)(p + 1024 + lane * 16);
             w[tp][r].h = *(const uint4 *)(p + 2048 + lane * 16);
@@ -88,6 +90,7 @@ __global__ __launch_bounds__(1024) void k_qmv_q6k_m1(QView q, const float *__res
     for (int i = 0; i < PER; i++) {
         const int b = b0 + i;
         float4 v = xv[i];
+        if (RAG && i > last) v.x = v.y = v.z = v.w = 0.f;
         if (xup)
             v = make_float4((v.x / (__expf(-v.x) + 1.0f)) * uv[i].x, (v.y / (__expf(-v.y) + 1.0f)) * uv[i].y,
                             (v.z / (__expf(-v.z) + 1.0f)) * uv[i].z, (v.w / (__expf(-v.w) + 1.0f)) * uv[i].w);
@@ -239,6 +242,16 @@ static fh_status q6k_m1_launch(const fh_qmatrix *q, const float *x, float *y, co
     return FH_OK;
 }
 
+template <int PER, int EPI>
+static fh_status q6k_m1_rag(const fh_qmatrix *q, const float *x, float *y, const float *a, const float *b) {
+    const int SW = (int)(q->kb + PER - 1) / PER, kb = SW * PER;
+    const size_t lds = (size_t)kb * Q6K_IMG * 16 + (size_t)kb * Q6K_SF * 4 + (size_t)SW * 64;
+    FH_TRY(fh_kernel_lds(q->dev, (const void *)k_qmv_q6k_m1<1, PER, EPI, true>, 160 * 1024));
+    k_qmv_q6k_m1<1, PER, EPI, true><<<dim3((unsigned)((q->n + 15) / 16)), dim3(64 * SW), lds, q->dev->stream>>>(fh_view(q), x, y, a, b, SW, nullptr);
+    FH_HIP(hipGetLastError());
+    return FH_OK;
+}
+
 // (tiles per wavefront, blocks per wavefront) with at most four block tiles (56 registers of weights) per wavefront
 template <int EPI>
 static fh_status q6k_m1_shape(int tpw, int per, const fh_qmatrix *q, const float *x, float *y, const float *a,
@@ -277,6 +290,10 @@ fh_status fh_launch_q6k_m1(const fh_qmatrix *q, const float *x, float *y, int ep
         per *= 2;
     }
     const int SW = kb / per;
+    // more than 16 blocks that no number of up to 16 wavefronts shares out evenly: 4096 x 11008, 43 of them, 10.7 us (20.4 by the batch kernel)
+    if (SW > 16 && kb <= 64 && epi != FH_EPI_SWIGLU)
+        return epi == FH_EPI_ADD2 ? (kb <= 32 ? q6k_m1_rag<2, FH_EPI_ADD2>(q, x, y, a, b) : q6k_m1_rag<4, FH_EPI_ADD2>(q, x, y, a, b))
+                                  : (kb <= 32 ? q6k_m1_rag<2, FH_EPI_NONE>(q, x, y, a, b) : q6k_m1_rag<4, FH_EPI_NONE>(q, x, y, a, b));
     if (SW > 16 || kb % per || tpw * per > 4) return FH_ERR_UNSUPPORTED;
     size_t lds = (size_t)kb * Q6K_IMG * 16 + (size_t)kb * Q6K_SF * 4 + (size_t)tpw * SW * 64;
     if (lds > 160 * 1024) return FH_ERR_UNSUPPORTED;

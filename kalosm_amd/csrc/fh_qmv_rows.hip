@@ -316,17 +316,20 @@ bool fh_qmv_rows_supports(const fh_qmatrix *q, const float *x, int m) {
 // - 13 - 16 rows of Q5_K where a wavefront has four tiles, in parts: 16326 x 2304 17.0 / 20.2, 8192 x 5376 19.4 / 20.4 (4096 x 14336 24.2 / 23.3).
 // - Up to 65536 weights of the 5-bit formats, although 64 x 1024 is 9.7 / 5.3: there k_qmm_reg's own line, five rows of 1024 columns, can be seen.
 // - 2 - 4 rows, which are the single-row kernel's row variant (4096 x 4096, four rows 6.8 / 8.6); Q6_K, which has none, only from 3 rows on and with one tile a
-//   wavefront (3 rows of 4096 x 4096 9.8 / 9.5, of 8192 x 3072 12.6 / 13.1).
+//   wavefront (3 rows of 4096 x 4096 9.8 / 9.5, of 8192 x 3072 12.6 / 13.1).  The 5-bit formats, which have none either and take a launch a row, from 3 rows on where a
+//   launch is more than its own start, that is beyond 2^20 weights: three rows of 4096 x 4096 in Q5_0 11.6 / 9.4 and in Q5_K 11.6 / 10.3, of 14336 x 4096 25.8 / 18.0 and
+//   26.4 / 20.7, four rows 33.8 / 17.8 and 34.6 / 20.8, of 8192 x 3072 17.9 / 12.2 and 18.1 / 13.6 (512 x 2048 9.7 / 6.7, two rows 5.0 / 6.6).
 bool fh_qmv_rows_pays(const fh_qmatrix *q, const float *x, int m) {
-    if (!fh_qmv_rows_supports(q, x, m) || m < (q->type == FH_Q6_K ? 3 : 5)) return false;
+    const bool five = q->type == FH_Q5_0 || q->type == FH_Q5_K;
+    if (!fh_qmv_rows_supports(q, x, m) || m < (q->type == FH_Q6_K || (five && q->n * q->k > 1 << 20) ? 3 : 5)) return false;
     const int64_t tiles = (q->n + 15) / 16, cus = q->dev->compute_units;
-    if ((q->type == FH_Q5_0 || q->type == FH_Q5_K) && q->n * q->k <= 65536) return false;
+    if (five && q->n * q->k <= 65536) return false;
     if (q->type == FH_Q4_K && q->k > 1024 && q->k < 2048 && q->n <= 2816) return false;
     if (tiles * 2 >= 7 * cus && ((q->type == FH_Q4_K && q->k <= 4096) || (q->type == FH_Q4_0 && q->k > 2048 && q->k <= 3072))) return false;
     if (tiles > ((q->type == FH_Q6_K || q->type == FH_Q8_0) && q->k <= 256 ? 4 : 6) * cus) return false;
     const RowsCut cut = rows_cut(q);
     if (q->type == FH_Q5_K && m > 12 && cut.tt == 4 && q->k > 256 * cut.kc && q->k < 8192) return false;
-    return cut.rounds == 1 && (m >= 5 || cut.tt == 1);
+    return cut.rounds == 1 && (m >= 5 || five || cut.tt == 1);
 }
 
 fh_status fh_launch_qmv_rows(const fh_qmatrix *q, const float *x, int m, float *y) {

@@ -161,6 +161,7 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
     // ---- 0. the activations of this wavefront's blocks are requested first: they are needed first and are short
     // With nw the input is rms_norm(x [+ xres]) * nw (composite/normalization.rs:287-401): the weight nw is
     // folded into the staged values and the common factor 1 / rms is applied to the finished dot product.
+    const int pos = EPI == FH_EPI_ROPEKV ? *rk.pos : 0;
     float4 xv[NB * MR], rv[NB], wv[NB], pacc[IN == 2 ? PER : 1][8];
     float2 pm[IN == 2 ? PER : 1][8];
 #pragma unroll
@@ -221,6 +222,13 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
                 w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * RS * 2304 + 1024);
             }
         }
+    // What the last phase adds or rotates by is asked for here and below, by every wavefront (no branch); asked for there it was one or two trips to memory
+    // after all others (us a pass of a 2048-wide decoder, 37 + 64 tokens: 9216 / 9082)
+    constexpr int EROWS = RS > 1 ? 16 / RS : TOUT * 16;
+    const int64_t erow = (int64_t)blockIdx.x * EROWS + tid % EROWS;
+    const int64_t eat = erow < nout ? erow : nout - 1;
+    float add_a = 0.f, add_b = 0.f;
+    if constexpr (EPI == FH_EPI_ADD2 && MR == 1) add_a = ea[eat], add_b = eb[eat];
     // ---- 2. stage x (lane owns k = 256*b + 4*lane .. +3).  A wavefront stages exactly the blocks it multiplies:
     // nobody else reads its part of the image, so there is no barrier between this and the products.  (No branch
     // around it either: the compiler would sink the activation loads into it, behind the weight loads.)
@@ -308,6 +316,13 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
         ss += dpp_f32<DPP_ROW_MIRROR>(ss); // rows of 16 are uniform now
         ss = rows_sum(ss);
         if (lane == 0) l_ss[wave] = ss;
+    }
+    float rope_c = 0.f, rope_s = 0.f; // of this thread's row, for the last phase; the position has arrived with the activations
+    if constexpr (EPI == FH_EPI_ROPEKV) {
+        const int half = rk.hd >> 1, r = (int)eat, rh = r < rk.qd ? r : r - rk.qd;
+        const int64_t at = (int64_t)(pos < rk.table_rows ? pos : rk.table_rows - 1) * half + (rh % rk.hd >> 1);
+        rope_c = rk.cs[at];
+        rope_s = rk.sn[at];
     }
     // ---- 3. eight chained MFMA steps per block and tile; the TPW tiles share every operand read
     if constexpr (RS > 1) {
@@ -563,13 +578,11 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
             if (jr < 8) y[(int64_t)blockIdx.x * 8 + jr] = (v0 / (__expf(-v0) + 1.0f)) * up;
         } else if (EPI == FH_EPI_ROPEKV) {
             const float other = __shfl_xor(v0, 1, 64); // the pair (2i, 2i+1) sits in neighbouring lanes
-            const int pos = *rk.pos;
             if (row < nout && pos < rk.cap) {
                 const int r = (int)row;
                 if (r < rk.qd + rk.kd) {
-                    const int rh = r < rk.qd ? r : r - rk.qd, e = rh % rk.hd, i = e >> 1, half = rk.hd >> 1;
-                    const int tp = pos < rk.table_rows ? pos : rk.table_rows - 1;
-                    const float c = rk.cs[(int64_t)tp * half + i], sn = rk.sn[(int64_t)tp * half + i];
+                    const int rh = r < rk.qd ? r : r - rk.qd, e = rh % rk.hd;
+                    const float c = rope_c, sn = rope_s;
                     const float x0 = (r & 1) ? other : v0, x1 = (r & 1) ? v0 : other;
                     const float ac = x0 * c, bs = x1 * sn, as = x0 * sn, bc = x1 * c;
                     const float yv = (r & 1) ? as + bc : ac - bs;
@@ -594,7 +607,7 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
             }
         } else if (row < nout) {
             float rr = v0;
-            if (EPI == FH_EPI_ADD2) rr = (rr + ea[row]) + eb[row];
+            if (EPI == FH_EPI_ADD2) rr = (rr + add_a) + add_b;
             if (EPI == FH_EPI_SWIGLU) rr = (rr / (__expf(-rr) + 1.0f)) * v1;
             if (EPI == FH_EPI_ACC) unsafeAtomicAdd(y + row, (blockIdx.y == 0 && ea) ? rr + ea[row] : rr);
             else y[row] = rr;

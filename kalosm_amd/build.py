@@ -22,6 +22,7 @@ FLAGS = [
     "-fPIC",
     "-ffp-contract=off",          # dequantised values are compared bit for bit: never fuse a*b - c
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",  # the first words of a kernel's plain arguments are in registers when it starts
     "-Wall", "-Wno-unused-function", "-Wno-unknown-warning-option", "-Wno-unused-command-line-argument",
     "-fvisibility=hidden",
 ]

@@ -530,9 +530,10 @@ struct QdRegs {
 #define QD_LDS_IMG 8448 // bytes of LDS per wavefront for the second half of a chunk's image: 8 operands + 64 sums
 
 template <int T, int TPW, int EPI>
-__global__ __launch_bounds__(1024) void k_qmv_direct(QView q, const uint8_t *__restrict__ ximg, int M, int cps,
-                                                     float *__restrict__ y, float *__restrict__ part,
+__global__ __launch_bounds__(1024) void k_qmv_direct(const uint8_t *data, const uint8_t *__restrict__ ximg, int rows, int chunks, int recs, int rec_bytes, int M, int cps,
+                                                     float *__restrict__ part, float *__restrict__ y,
                                                      const float *__restrict__ ea, const float *__restrict__ eb) {
+    const QView q{data, rows, (int64_t)chunks * 256, 0, recs, rec_bytes}; // (plain values: in registers when the kernel starts)
     constexpr int IMG = QdImg<T>::BYTES;
     constexpr int NT = EPI == FH_EPI_SWIGLU ? 2 : 1, TOUT = TPW / NT;
     constexpr bool LDS_HALF = TPW == 4;
@@ -689,15 +690,15 @@ static fh_status qd_launch(const fh_qmatrix *q, const float *x, int m, float *y,
     if (four) {
         if constexpr (EPI != FH_EPI_SWIGLU && (T == FH_Q4_K || T == FH_Q4_0)) {
             if (lds > 64 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_qmv_direct<T, 4, EPI>, lds));
-            k_qmv_direct<T, 4, EPI><<<grid, block, lds, dev->stream>>>(fh_view(q), (const uint8_t *)dev->act_buf, m, cps, y,
-                                                                      part, a, b);
+            k_qmv_direct<T, 4, EPI><<<grid, block, lds, dev->stream>>>(q->data, (const uint8_t *)dev->act_buf, (int)q->n, C, (int)q->recs, q->rec_bytes, m, cps,
+                                                                  part, y, a, b);
         }
     } else if (two)
-        k_qmv_direct<T, 2, EPI><<<grid, block, lds, dev->stream>>>(fh_view(q), (const uint8_t *)dev->act_buf, m, cps, y,
-                                                                  part, a, b);
+        k_qmv_direct<T, 2, EPI><<<grid, block, lds, dev->stream>>>(q->data, (const uint8_t *)dev->act_buf, (int)q->n, C, (int)q->recs, q->rec_bytes, m, cps,
+                                                                  part, y, a, b);
     else if constexpr (EPI != FH_EPI_SWIGLU)
-        k_qmv_direct<T, 1, EPI><<<grid, block, lds, dev->stream>>>(fh_view(q), (const uint8_t *)dev->act_buf, m, cps, y,
-                                                                  part, a, b);
+        k_qmv_direct<T, 1, EPI><<<grid, block, lds, dev->stream>>>(q->data, (const uint8_t *)dev->act_buf, (int)q->n, C, (int)q->recs, q->rec_bytes, m, cps,
+                                                                  part, y, a, b);
     if (part) {
         const int64_t total = (int64_t)m * nout;
         k_qd_reduce<EPI><<<dim3((unsigned)((total + 255) / 256)), dim3(256), 0, dev->stream>>>(part, parts, m, q->n, nout, y,

@@ -617,41 +617,53 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
 
 // The kernel proper.  With at most two block tiles per wavefront the register budget of eight wavefronts per SIMD
 // (64 VGPRs) is enforced: the kernel lives on the number of bytes in flight per compute unit.
+// What the first requests need comes first and as plain values: the first 14 words of a kernel's arguments are in scalar registers when its wavefronts
+// start (-amdgpu-kernarg-preload-count), the rest are a trip to memory away.  us, as a struct ahead of them / so: 12 products of one row (4096 / 14336) 74.0 /
+// 69.9, of 16 rows 148.9 / 145.4; in a replayed graph 0.2 a launch (8B, 128 tokens: 2 %).
 #define Q4K_M1_PARAMS                                                                                              \
-    QView q, const float *__restrict__ x, float *__restrict__ y, const float *__restrict__ ea,                    \
-        const float *__restrict__ eb, int SW, const float *__restrict__ xres, const float *__restrict__ nw, float eps, int nsplit, FhRopeArgs rk
+    const uint8_t *data, const float *__restrict__ x, const float *__restrict__ nw, const float *__restrict__ xres, int recs, int n, int k, int SW, int nsplit, \
+        float eps, float *__restrict__ y, const float *__restrict__ ea, const float *__restrict__ eb, FhRopeArgs rk
+#define Q4K_M1_ARGS QView{data, n, k, 0, recs, 0}, x, y, ea, eb, SW, xres, nw, eps, nsplit, rk
+typedef void (*q4k_m1_kern)(Q4K_M1_PARAMS);
+static fh_status q4k_m1_start(q4k_m1_kern kern, const fh_qmatrix *q, dim3 grid, int SW, size_t lds, const float *x, float *y, const float *a, const float *b,
+                              const float *xres = nullptr, const float *nw = nullptr, float eps = 0.f, int nsplit = 0, const FhRopeArgs &rk = {}) {
+    FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
+    kern<<<grid, dim3(64 * SW), lds, q->dev->stream>>>(q->data, x, nw, xres, (int)q->recs, (int)q->n, (int)q->k, SW, nsplit, eps, y, a, b, rk);
+    FH_HIP(hipGetLastError());
+    return FH_OK;
+}
 template <int TPW, int PER, int EPI, int IN>
 __global__ __launch_bounds__(1024) void k_qmv_q4k_m1(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FH_Q4_K, TPW, PER, EPI, IN>(q, x, y, ea, eb, SW, xres, nw, eps, nsplit, rk);
+    qmv_q4k_m1_body<FH_Q4_K, TPW, PER, EPI, IN>(Q4K_M1_ARGS);
 }
 template <int TPW, int PER, int EPI, int IN>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_qmv_q4k_m1_w8(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FH_Q4_K, TPW, PER, EPI, IN>(q, x, y, ea, eb, SW, xres, nw, eps, nsplit, rk);
+    qmv_q4k_m1_body<FH_Q4_K, TPW, PER, EPI, IN>(Q4K_M1_ARGS);
 }
 // 16 / RS rows of a tile per workgroup, RS blocks at once per wavefront (matrices with few row tiles)
 template <int RS, int PER, int EPI, int IN>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_qmv_q4k_m1_rs(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FH_Q4_K, 1, PER, EPI, IN, 1, RS>(q, x, y, ea, eb, SW, xres, nw, eps, nsplit, rk);
+    qmv_q4k_m1_body<FH_Q4_K, 1, PER, EPI, IN, 1, RS>(Q4K_M1_ARGS);
 }
 // 2 .. 4 activation rows (plain input; epilogues none / add2); nsplit = number of valid rows
 template <int FMT, int TPW, int PER, int EPI, int MR>
 __global__ __launch_bounds__(1024) void k_qmv_q4k_mr(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0, MR>(q, x, y, ea, eb, SW, xres, nw, eps, nsplit, rk);
+    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0, MR>(Q4K_M1_ARGS);
 }
 // Q4_0 / Q8_0 weights (plain input; epilogues none / add2 / SwiGLU)
 template <int FMT, int TPW, int PER, int EPI>
 __global__ __launch_bounds__(1024) void k_qmv_q40_m1(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0>(q, x, y, ea, eb, SW, xres, nw, eps, nsplit, rk);
+    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0>(Q4K_M1_ARGS);
 }
 template <int FMT, int TPW, int PER, int EPI>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_qmv_q40_m1_w8(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0>(q, x, y, ea, eb, SW, xres, nw, eps, nsplit, rk);
+    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0>(Q4K_M1_ARGS);
 }
 
 // k of more than 16 blocks that no number of up to 16 wavefronts shares out evenly (43 of 11008 columns); epilogues none / add2
 template <int FMT, int PER, int EPI>
 __global__ __launch_bounds__(1024) void k_qmv_q4k_m1_rag(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FMT, 1, PER, EPI, 0, 1, 1, true>(q, x, y, ea, eb, SW, xres, nw, eps, nsplit, rk);
+    qmv_q4k_m1_body<FMT, 1, PER, EPI, 0, 1, 1, true>(Q4K_M1_ARGS);
 }
 
 template <int FMT, int PER>
@@ -659,10 +671,7 @@ static fh_status q4k_m1_rag_go(const fh_qmatrix *q, const float *x, float *y, in
     const int SW = (int)(q->k / 256 + PER - 1) / PER, kb = SW * PER;
     const size_t lds = (size_t)kb * Q4K_IMG * 16 + (size_t)kb * 64 + 16 * 64 + 64;
     const auto kern = epi == FH_EPI_ADD2 ? k_qmv_q4k_m1_rag<FMT, PER, FH_EPI_ADD2> : k_qmv_q4k_m1_rag<FMT, PER, FH_EPI_NONE>;
-    FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
-    kern<<<dim3((unsigned)((q->n + 15) / 16)), dim3(64 * SW), lds, q->dev->stream>>>(fh_view(q), x, y, a, b, SW, nullptr, nullptr, 0.f, 0, FhRopeArgs{});
-    FH_HIP(hipGetLastError());
-    return FH_OK;
+    return q4k_m1_start(kern, q, dim3((unsigned)((q->n + 15) / 16)), SW, lds, x, y, a, b);
 }
 
 // us of one row of 4096 x 11008 by the kernels that took it (the batch kernel, the 5-bit formats element by element) / here: Q4_K 15.0 / 7.7, Q4_0 15.2 /
@@ -684,20 +693,14 @@ static fh_status q4k_m1_rag(const fh_qmatrix *q, const float *x, float *y, int e
 template <int TPW, int PER, int EPI>
 static fh_status q4k_m1_launch(const fh_qmatrix *q, const float *x, float *y, const float *a, const float *b, int SW,
                                unsigned grid, size_t lds, const Q4kExtra &ex) {
-    typedef void (*kern_t)(QView, const float *, float *, const float *, const float *, int, const float *, const float *,
-                           float, int, FhRopeArgs);
-    kern_t kern;
+    q4k_m1_kern kern;
     const int in = ex.nsplit > 0 ? 2 : (ex.nw ? 1 : 0); // input: plain, rms_norm, attention partials
     if (q->type == FH_Q5_0) { // (17 registers of weights per block tile, as Q8_0)
         if constexpr ((EPI == FH_EPI_NONE || EPI == FH_EPI_ADD2 || EPI == FH_EPI_SWIGLU) && !(EPI == FH_EPI_SWIGLU && TPW == 1)) {
             if (in != 0) return FH_ERR_UNSUPPORTED;
             if constexpr (TPW * PER == 1) kern = k_qmv_q40_m1_w8<FH_Q5_0, TPW, PER, EPI>;
             else kern = k_qmv_q40_m1<FH_Q5_0, TPW, PER, EPI>;
-            FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
-            kern<<<dim3(grid, 1), dim3(64 * SW), lds, q->dev->stream>>>(fh_view(q), x, y, a, b, SW, nullptr, nullptr, 0.f, 0,
-                                                                        ex.rk);
-            FH_HIP(hipGetLastError());
-            return FH_OK;
+            return q4k_m1_start(kern, q, dim3(grid, 1), SW, lds, x, y, a, b);
         } else {
             return FH_ERR_UNSUPPORTED;
         }
@@ -707,11 +710,7 @@ static fh_status q4k_m1_launch(const fh_qmatrix *q, const float *x, float *y, co
             if (in != 0) return FH_ERR_UNSUPPORTED;
             if constexpr (TPW * PER == 1) kern = k_qmv_q40_m1_w8<FH_Q5_K, TPW, PER, EPI>;
             else kern = k_qmv_q40_m1<FH_Q5_K, TPW, PER, EPI>;
-            FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
-            kern<<<dim3(grid, 1), dim3(64 * SW), lds, q->dev->stream>>>(fh_view(q), x, y, a, b, SW, nullptr, nullptr, 0.f, 0,
-                                                                        ex.rk);
-            FH_HIP(hipGetLastError());
-            return FH_OK;
+            return q4k_m1_start(kern, q, dim3(grid, 1), SW, lds, x, y, a, b);
         } else {
             return FH_ERR_UNSUPPORTED;
         }
@@ -726,11 +725,7 @@ static fh_status q4k_m1_launch(const fh_qmatrix *q, const float *x, float *y, co
             } else {
                 kern = q8 ? k_qmv_q40_m1<FH_Q8_0, TPW, PER, EPI> : k_qmv_q40_m1<FH_Q4_0, TPW, PER, EPI>;
             }
-            FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
-            kern<<<dim3(grid, 1), dim3(64 * SW), lds, q->dev->stream>>>(fh_view(q), x, y, a, b, SW, nullptr, nullptr, 0.f, 0,
-                                                                        ex.rk);
-            FH_HIP(hipGetLastError());
-            return FH_OK;
+            return q4k_m1_start(kern, q, dim3(grid, 1), SW, lds, x, y, a, b);
         } else {
             return FH_ERR_UNSUPPORTED;
         }
@@ -745,29 +740,19 @@ static fh_status q4k_m1_launch(const fh_qmatrix *q, const float *x, float *y, co
         if (in == 2) return FH_ERR_UNSUPPORTED; // the merge of the attention partials needs the registers
         kern = in == 1 ? k_qmv_q4k_m1<TPW, PER, EPI, 1> : k_qmv_q4k_m1<TPW, PER, EPI, 0>;
     }
-    FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
-    kern<<<dim3(grid, (unsigned)ex.ksplit), dim3(64 * SW), lds, q->dev->stream>>>(fh_view(q), x, y, a, b, SW, ex.xres,
-                                                                                  ex.nw, ex.eps, ex.nsplit, ex.rk);
-    FH_HIP(hipGetLastError());
-    return FH_OK;
+    return q4k_m1_start(kern, q, dim3(grid, (unsigned)ex.ksplit), SW, lds, x, y, a, b, ex.xres, ex.nw, ex.eps, ex.nsplit, ex.rk);
 }
 
 template <int EPI>
 static fh_status q4k_m1_launch_rs(int rs, int per, const fh_qmatrix *q, const float *x, float *y, const float *a,
                                   const float *b, int SW, unsigned grid, size_t lds, const Q4kExtra &ex) {
     if constexpr (EPI == FH_EPI_NONE || EPI == FH_EPI_ADD2) {
-        typedef void (*kern_t)(QView, const float *, float *, const float *, const float *, int, const float *,
-                               const float *, float, int, FhRopeArgs);
-        kern_t kern = nullptr;
+        q4k_m1_kern kern = nullptr;
         if (rs == 2 && per == 1) kern = k_qmv_q4k_m1_rs<2, 1, EPI, 0>;
         else if (rs == 2 && per == 2) kern = k_qmv_q4k_m1_rs<2, 2, EPI, 0>;
         else if (rs == 4 && per == 1) kern = k_qmv_q4k_m1_rs<4, 1, EPI, 0>;
         else return FH_ERR_UNSUPPORTED;
-        FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
-        kern<<<dim3(grid, 1), dim3(64 * SW), lds, q->dev->stream>>>(fh_view(q), x, y, a, b, SW, ex.xres, ex.nw, ex.eps, 0,
-                                                                    ex.rk);
-        FH_HIP(hipGetLastError());
-        return FH_OK;
+        return q4k_m1_start(kern, q, dim3(grid, 1), SW, lds, x, y, a, b, ex.xres, ex.nw, ex.eps);
     } else {
         return FH_ERR_UNSUPPORTED;
     }
@@ -806,13 +791,9 @@ static fh_status q4k_mr_parts(const fh_qmatrix *q, const float *x, int m, float 
     int tpw = (int)dev->opt_matvec_tiles;
     if (tpw != 1 && tpw != 2) tpw = tiles * parts > 2 * (int64_t)dev->compute_units ? 2 : 1;
     FH_TRY(fh_dev_scratch(dev, (void **)&dev->ksplit_buf, &dev->ksplit_cap, (size_t)parts * 16 * q->n * 4));
-    typedef void (*kern_t)(QView, const float *, float *, const float *, const float *, int, const float *, const float *,
-                           float, int, FhRopeArgs);
-    const kern_t kern = tpw == 2 ? (kern_t)k_qmv_q4k_mr<FMT, 2, 1, FH_EPI_NONE, MR> : (kern_t)k_qmv_q4k_mr<FMT, 1, 1, FH_EPI_NONE, MR>;
-    FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
-    kern<<<dim3((unsigned)((tiles + tpw - 1) / tpw), (unsigned)parts), dim3(64 * SW), lds, dev->stream>>>(
-        fh_view(q), x, (float *)dev->ksplit_buf, nullptr, nullptr, SW, nullptr, nullptr, 0.f, m, FhRopeArgs{});
-    FH_HIP(hipGetLastError());
+    const q4k_m1_kern kern = tpw == 2 ? (q4k_m1_kern)k_qmv_q4k_mr<FMT, 2, 1, FH_EPI_NONE, MR> : (q4k_m1_kern)k_qmv_q4k_mr<FMT, 1, 1, FH_EPI_NONE, MR>;
+    FH_TRY(q4k_m1_start(kern, q, dim3((unsigned)((tiles + tpw - 1) / tpw), (unsigned)parts), SW, lds, x, (float *)dev->ksplit_buf, nullptr, nullptr, nullptr,
+                        nullptr, 0.f, m));
     return fh_launch_kparts_reduce(dev, (const float *)dev->ksplit_buf, parts, m, q->n, y, EPI, a, b);
 }
 
@@ -834,14 +815,9 @@ static fh_status q4k_mr_go(const fh_qmatrix *q, const float *x, int m, float *y,
     if (tpw != 1 && tpw != 2) tpw = tiles > dev->compute_units ? 2 : 1;
     if (per == 2) tpw = 1;
     const unsigned grid = (unsigned)((tiles + tpw - 1) / tpw);
-    typedef void (*kern_t)(QView, const float *, float *, const float *, const float *, int, const float *, const float *,
-                           float, int, FhRopeArgs);
-    const kern_t kern = per == 2 ? (kern_t)k_qmv_q4k_mr<FMT, 1, 2, EPI, MR>
-                                 : (tpw == 2 ? (kern_t)k_qmv_q4k_mr<FMT, 2, 1, EPI, MR> : (kern_t)k_qmv_q4k_mr<FMT, 1, 1, EPI, MR>);
-    FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
-    kern<<<dim3(grid, 1), dim3(64 * SW), lds, dev->stream>>>(fh_view(q), x, y, a, b, SW, nullptr, nullptr, 0.f, m, FhRopeArgs{});
-    FH_HIP(hipGetLastError());
-    return FH_OK;
+    const q4k_m1_kern kern = per == 2 ? (q4k_m1_kern)k_qmv_q4k_mr<FMT, 1, 2, EPI, MR>
+                                 : (tpw == 2 ? (q4k_m1_kern)k_qmv_q4k_mr<FMT, 2, 1, EPI, MR> : (q4k_m1_kern)k_qmv_q4k_mr<FMT, 1, 1, EPI, MR>);
+    return q4k_m1_start(kern, q, dim3(grid, 1), SW, lds, x, y, a, b, nullptr, nullptr, 0.f, m);
 }
 
 template <int FMT>

@@ -29,9 +29,9 @@ struct Q6KRegs {
 // barrier before the products) and requests all its weight bytes before anything else.
 // RAG: the blocks are no multiple of the wavefronts'; what a wavefront has past the last one is the last one again, times zero.
 template <int TPW, int PER, int EPI, bool RAG = false>
-__global__ __launch_bounds__(1024) void k_qmv_q6k_m1(QView q, const float *__restrict__ x, float *__restrict__ y,
-                                                      const float *__restrict__ ea, const float *__restrict__ eb,
-                                                      int SW, const float *__restrict__ xup) {
+__global__ __launch_bounds__(1024) void k_qmv_q6k_m1(const uint8_t *data, const float *__restrict__ x, const float *__restrict__ xup, int recs, int n, int k, int SW,
+                                                      float *__restrict__ y, const float *__restrict__ ea, const float *__restrict__ eb) {
+    const QView q{data, n, k, 0, recs, 0}; // (plain values, the first needed first: in registers when the kernel starts)
     constexpr int NT = EPI == FH_EPI_SWIGLU ? 2 : 1;
     constexpr int TOUT = TPW / NT; // output tiles of the workgroup
     extern __shared__ uint4 lds[];
@@ -237,7 +237,7 @@ template <int TPW, int PER, int EPI>
 static fh_status q6k_m1_launch(const fh_qmatrix *q, const float *x, float *y, const float *a, const float *b, int SW,
                                unsigned grid, size_t lds, unsigned ksplit = 1, const float *xup = nullptr) {
     FH_TRY(fh_kernel_lds(q->dev, (const void *)k_qmv_q6k_m1<TPW, PER, EPI>, 160 * 1024));
-    k_qmv_q6k_m1<TPW, PER, EPI><<<dim3(grid, ksplit), dim3(64 * SW), lds, q->dev->stream>>>(fh_view(q), x, y, a, b, SW, xup);
+    k_qmv_q6k_m1<TPW, PER, EPI><<<dim3(grid, ksplit), dim3(64 * SW), lds, q->dev->stream>>>(q->data, x, xup, (int)q->recs, (int)q->n, (int)q->k, SW, y, a, b);
     FH_HIP(hipGetLastError());
     return FH_OK;
 }
@@ -247,7 +247,7 @@ static fh_status q6k_m1_rag(const fh_qmatrix *q, const float *x, float *y, const
     const int SW = (int)(q->kb + PER - 1) / PER, kb = SW * PER;
     const size_t lds = (size_t)kb * Q6K_IMG * 16 + (size_t)kb * Q6K_SF * 4 + (size_t)SW * 64;
     FH_TRY(fh_kernel_lds(q->dev, (const void *)k_qmv_q6k_m1<1, PER, EPI, true>, 160 * 1024));
-    k_qmv_q6k_m1<1, PER, EPI, true><<<dim3((unsigned)((q->n + 15) / 16)), dim3(64 * SW), lds, q->dev->stream>>>(fh_view(q), x, y, a, b, SW, nullptr);
+    k_qmv_q6k_m1<1, PER, EPI, true><<<dim3((unsigned)((q->n + 15) / 16)), dim3(64 * SW), lds, q->dev->stream>>>(q->data, x, nullptr, (int)q->recs, (int)q->n, (int)q->k, SW, y, a, b);
     FH_HIP(hipGetLastError());
     return FH_OK;
 }

@@ -115,8 +115,9 @@ struct RowsTile {
 };
 
 template <int T, int KC, int TT>
-__global__ __launch_bounds__(1024) void k_qmv_rows(QView q, const float *__restrict__ x, int m, int wtiles, int parts, float *__restrict__ part,
+__global__ __launch_bounds__(1024) void k_qmv_rows(const uint8_t *data, const float *__restrict__ x, int n, int k, int m, int wtiles, int parts, float *__restrict__ part,
                                                    uint32_t *__restrict__ arrived, float *__restrict__ y) {
+    const QView q{data, n, k, 0, 0, 0}; // (plain values: in registers when the kernel starts)
     constexpr bool OWN = RowsX<T>::OWN, SUMS = RowsX<T>::SUMS, PER32 = OWN || (!SUMS && T != FH_Q6_K), MINS = T == FH_Q5_K; // MINS: offsets block by block
     constexpr int REC = RegW<T>::REC, NW = RegW<T>::NW, PITCH = 272, TILES = RowsTile<T, KC, TT>::TILES;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -263,7 +264,7 @@ static fh_status rows_go(const fh_qmatrix *q, const float *x, int m, float *y) {
         part = dev->ksplit_buf;
     }
     FH_TRY(fh_kernel_lds(dev, (const void *)k_qmv_rows<T, KC, TT>, (size_t)Tile::LDS));
-    k_qmv_rows<T, KC, TT><<<dim3((unsigned)(groups * parts)), 1024, Tile::LDS, dev->stream>>>(fh_view(q), x, m, tiles, parts, part, dev->arrived, y);
+    k_qmv_rows<T, KC, TT><<<dim3((unsigned)(groups * parts)), 1024, Tile::LDS, dev->stream>>>(q->data, x, (int)q->n, (int)q->k, m, tiles, parts, part, dev->arrived, y);
     FH_HIP(hipGetLastError());
     return FH_OK;
 }

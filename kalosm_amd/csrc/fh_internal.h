@@ -167,6 +167,7 @@ struct fh_qmatrix {
     // dense f32 rows on the matrix cores: a power of two that brings the largest |w| into [2^14, 2^15), so that the
     // f16 pair hi + lo of w * wscale keeps 22 bits for every value that matters next to the largest one
     float wscale = 1.f;
+    int streamed = -1; // 1, 0: of a decoder whose weights are more, no more than the last cache; -1: not known (fh_weights_once)
 };
 
 // Weight types kept in the file's own row-major order (no tiled re-layout): dense f32 / f16 rows.

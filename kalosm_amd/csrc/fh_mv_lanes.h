@@ -41,3 +41,18 @@ __device__ __forceinline__ uint32_t sel_lanes(uint64_t mask, uint32_t yes, uint3
     return r;
 }
 
+
+// Weights of a product of one or a few rows are read by one wavefront each and not again in this launch.  Where more than the 256 MB of the last cache passes
+// before the next step reads them, they are read with the hint that they are streamed; a decoder knows whether it does, a matrix by itself is taken for a part of
+// a larger whole from 16 MB on.  us, plainly / by that rule: 8B, 512 + 128 tokens 197017 / 188284 (only the matrices of 16 MB and more 196240), products of three
+// layers (4096 / 14336, 235 MB) of one row 69.9 / 66.5 (all with the hint 68.5), of 16 rows 145.6 / 139.9; a 2048-wide decoder of 193 MB 8904 (9052 with it).
+template <bool ONCE, typename T>
+__device__ __forceinline__ T fh_ld_weights(const uint8_t *p) {
+    if constexpr (!ONCE) return *(const T *)p;
+    typedef uint32_t words __attribute__((ext_vector_type(sizeof(T) / 4)));
+    const words v = __builtin_nontemporal_load((const words *)p);
+    T r;
+    __builtin_memcpy(&r, &v, sizeof(T));
+    return r;
+}
+static inline bool fh_weights_once(const fh_qmatrix *q) { return q->streamed < 0 ? q->bytes >= (size_t)16 << 20 : q->streamed != 0; }

@@ -18,6 +18,7 @@
 // flight (the kernel is bound by memory latency, not by arithmetic).  The slices are added through LDS in a fixed
 // order and the epilogue is applied at the store.
 #include "fh_blocks.h"
+#include "fh_mv_lanes.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -50,11 +51,12 @@ struct QbW;
 template <>
 struct QbW<FH_Q4_K> {
     uint4 a, b, h;
+    template <bool ONCE = false>
     __device__ __forceinline__ void load(const QView &q, int64_t tile, int c, int lane) {
         const uint8_t *rec = q.data + (tile * q.recs + c) * 2304;
-        h = *(const uint4 *)(rec + 16 * (lane & 15));
-        a = *(const uint4 *)(rec + 256 + lane * 16);
-        b = *(const uint4 *)(rec + 1280 + lane * 16);
+        h = fh_ld_weights<ONCE, uint4>(rec + 16 * (lane & 15));
+        a = fh_ld_weights<ONCE, uint4>(rec + 256 + lane * 16);
+        b = fh_ld_weights<ONCE, uint4>(rec + 1280 + lane * 16);
     }
 };
 template <>
@@ -62,14 +64,15 @@ struct QbW<FH_Q6_K> {
     uint4 l0, l1, hh;
     uint32_t sc[4];
     uint32_t d;
+    template <bool ONCE = false>
     __device__ __forceinline__ void load(const QView &q, int64_t tile, int c, int lane) {
         const uint8_t *rec = q.data + (tile * q.recs + c) * 3360;
         const int j = lane & 15;
-        l0 = *(const uint4 *)(rec + lane * 16);
-        l1 = *(const uint4 *)(rec + 1024 + lane * 16);
-        hh = *(const uint4 *)(rec + 2048 + lane * 16);
+        l0 = fh_ld_weights<ONCE, uint4>(rec + lane * 16);
+        l1 = fh_ld_weights<ONCE, uint4>(rec + 1024 + lane * 16);
+        hh = fh_ld_weights<ONCE, uint4>(rec + 2048 + lane * 16);
 #pragma unroll
-        for (int qd = 0; qd < 4; qd++) sc[qd] = *(const uint32_t *)(rec + 3072 + (qd * 16 + j) * 4);
+        for (int qd = 0; qd < 4; qd++) sc[qd] = fh_ld_weights<ONCE, uint32_t>(rec + 3072 + (qd * 16 + j) * 4);
         d = fh_ld16(rec + 3328 + 2 * j);
     }
 };
@@ -77,12 +80,13 @@ template <>
 struct QbW<FH_Q8_0> {
     uint4 w[4];
     uint32_t d[4];
+    template <bool ONCE = false>
     __device__ __forceinline__ void load(const QView &q, int64_t tile, int c, int lane) {
         const uint8_t *rec = q.data + (tile * q.recs + 4 * c) * 1088;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            w[r] = *(const uint4 *)(rec + r * 1088 + lane * 16);
-            d[r] = *(const uint32_t *)(rec + r * 1088 + 1024 + 4 * (lane & 15));
+            w[r] = fh_ld_weights<ONCE, uint4>(rec + r * 1088 + lane * 16);
+            d[r] = fh_ld_weights<ONCE, uint32_t>(rec + r * 1088 + 1024 + 4 * (lane & 15));
         }
     }
 };
@@ -90,12 +94,13 @@ template <>
 struct QbW<FH_Q4_0> {
     uint4 w[2];
     uint2 d[2];
+    template <bool ONCE = false>
     __device__ __forceinline__ void load(const QView &q, int64_t tile, int c, int lane) {
         const uint8_t *rec = q.data + (tile * q.recs + 2 * c) * 1152;
 #pragma unroll
         for (int r = 0; r < 2; r++) {
-            w[r] = *(const uint4 *)(rec + r * 1152 + lane * 16);
-            d[r] = *(const uint2 *)(rec + r * 1152 + 1024 + 8 * (lane & 15));
+            w[r] = fh_ld_weights<ONCE, uint4>(rec + r * 1152 + lane * 16);
+            d[r] = fh_ld_weights<ONCE, uint2>(rec + r * 1152 + 1024 + 8 * (lane & 15));
         }
     }
 };
@@ -529,7 +534,7 @@ struct QdRegs {
 
 #define QD_LDS_IMG 8448 // bytes of LDS per wavefront for the second half of a chunk's image: 8 operands + 64 sums
 
-template <int T, int TPW, int EPI>
+template <int T, int TPW, int EPI, bool ONCE>
 __global__ __launch_bounds__(1024) void k_qmv_direct(const uint8_t *data, const uint8_t *__restrict__ ximg, int rows, int chunks, int recs, int rec_bytes, int M, int cps,
                                                      float *__restrict__ part, float *__restrict__ y,
                                                      const float *__restrict__ ea, const float *__restrict__ eb) {
@@ -559,7 +564,7 @@ __global__ __launch_bounds__(1024) void k_qmv_direct(const uint8_t *data, const 
         for (int tp = 0; tp < TPW; tp++) {
             int64_t to = (int64_t)blockIdx.x * TOUT + (tp % TOUT);
             if (to >= tiles_out) to = tiles_out - 1; // a tile past the end re-reads the last one; never stored
-            w[tp].load(q, to + (int64_t)(tp / TOUT) * (nout / 16), c, lane);
+            w[tp].template load<ONCE>(q, to + (int64_t)(tp / TOUT) * (nout / 16), c, lane);
         }
         __builtin_amdgcn_sched_barrier(0);
         // Four tiles per wavefront leave no registers for the second half of the image: it is requested now as well,
@@ -689,15 +694,16 @@ static fh_status qd_launch(const fh_qmatrix *q, const float *x, int m, float *y,
     const size_t lds = four ? std::max((size_t)cps * 4 * 16 * 17 * 4, (size_t)cps * QD_LDS_IMG) : (size_t)cps * (two ? 2 : 1) * 16 * 17 * 4;
     if (four) {
         if constexpr (EPI != FH_EPI_SWIGLU && (T == FH_Q4_K || T == FH_Q4_0)) {
-            if (lds > 64 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_qmv_direct<T, 4, EPI>, lds));
-            k_qmv_direct<T, 4, EPI><<<grid, block, lds, dev->stream>>>(q->data, (const uint8_t *)dev->act_buf, (int)q->n, C, (int)q->recs, q->rec_bytes, m, cps,
+            const auto kern = fh_weights_once(q) ? k_qmv_direct<T, 4, EPI, true> : k_qmv_direct<T, 4, EPI, false>;
+            if (lds > 64 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)kern, lds));
+            kern<<<grid, block, lds, dev->stream>>>(q->data, (const uint8_t *)dev->act_buf, (int)q->n, C, (int)q->recs, q->rec_bytes, m, cps,
                                                                   part, y, a, b);
         }
     } else if (two)
-        k_qmv_direct<T, 2, EPI><<<grid, block, lds, dev->stream>>>(q->data, (const uint8_t *)dev->act_buf, (int)q->n, C, (int)q->recs, q->rec_bytes, m, cps,
+        (fh_weights_once(q) ? k_qmv_direct<T, 2, EPI, true> : k_qmv_direct<T, 2, EPI, false>)<<<grid, block, lds, dev->stream>>>(q->data, (const uint8_t *)dev->act_buf, (int)q->n, C, (int)q->recs, q->rec_bytes, m, cps,
                                                                   part, y, a, b);
     else if constexpr (EPI != FH_EPI_SWIGLU)
-        k_qmv_direct<T, 1, EPI><<<grid, block, lds, dev->stream>>>(q->data, (const uint8_t *)dev->act_buf, (int)q->n, C, (int)q->recs, q->rec_bytes, m, cps,
+        (fh_weights_once(q) ? k_qmv_direct<T, 1, EPI, true> : k_qmv_direct<T, 1, EPI, false>)<<<grid, block, lds, dev->stream>>>(q->data, (const uint8_t *)dev->act_buf, (int)q->n, C, (int)q->recs, q->rec_bytes, m, cps,
                                                                   part, y, a, b);
     if (part) {
         const int64_t total = (int64_t)m * nout;

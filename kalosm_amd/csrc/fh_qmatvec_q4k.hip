@@ -71,7 +71,7 @@ struct Q4kExtra {
 // same block are the dots; the rest is discarded.  As many MFMAs per weight byte as with whole tiles, RS times the
 // workgroups: matrices with fewer row tiles than compute units fill the device in one launch.
 // RAG: the blocks are no multiple of the wavefronts'; what a wavefront has past the last one is the last one again, times zero.
-template <int FMT, int TPW, int PER, int EPI, int IN, int MR = 1, int RS = 1, bool RAG = false>
+template <int FMT, int TPW, int PER, int EPI, int IN, int MR = 1, int RS = 1, bool RAG = false, bool ONCE = false>
 __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict__ x, float *__restrict__ y,
                                                       const float *__restrict__ ea, const float *__restrict__ eb,
                                                       int SW, const float *__restrict__ xres,
@@ -194,32 +194,32 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
 #pragma unroll
         for (int tp = 0; tp < TPW; tp++) {
             if constexpr (FMT == FH_Q5_0) { // the Q4_0 records, each followed by the lane's fifth bits (one byte per block)
-                w[tp][r].h.x = *(const uint32_t *)(ph[tp] + blk(r) * CHUNK);
-                w[tp][r].qa = *(const uint4 *)(pq[tp] + blk(r) * CHUNK);
-                w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * CHUNK + REC);
-                w[tp][r].qc.x = *(const uint32_t *)(pq[tp] + 1152 - 12 * lane + blk(r) * CHUNK);
-                w[tp][r].qc.y = *(const uint32_t *)(pq[tp] + 1152 - 12 * lane + blk(r) * CHUNK + REC);
+                w[tp][r].h.x = fh_ld_weights<ONCE, uint32_t>(ph[tp] + blk(r) * CHUNK);
+                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * CHUNK);
+                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * CHUNK + REC);
+                w[tp][r].qc.x = fh_ld_weights<ONCE, uint32_t>(pq[tp] + 1152 - 12 * lane + blk(r) * CHUNK);
+                w[tp][r].qc.y = fh_ld_weights<ONCE, uint32_t>(pq[tp] + 1152 - 12 * lane + blk(r) * CHUNK + REC);
             } else if constexpr (FMT == FH_Q5_K) { // the Q4_K record followed by the lane's eight qh bytes
-                w[tp][r].h = *(const uint4 *)(ph[tp] + blk(r) * CHUNK);
-                w[tp][r].qa = *(const uint4 *)(pq[tp] + blk(r) * CHUNK);
-                w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * CHUNK + 1024);
-                const uint2 hb = *(const uint2 *)(pq[tp] + 2048 - 8 * lane + blk(r) * CHUNK);
+                w[tp][r].h = fh_ld_weights<ONCE, uint4>(ph[tp] + blk(r) * CHUNK);
+                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * CHUNK);
+                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * CHUNK + 1024);
+                const uint2 hb = fh_ld_weights<ONCE, uint2>(pq[tp] + 2048 - 8 * lane + blk(r) * CHUNK);
                 w[tp][r].qc.x = hb.x;
                 w[tp][r].qc.y = hb.y;
             } else if (FMT == FH_Q4_0) {
-                w[tp][r].h.x = *(const uint32_t *)(ph[tp] + blk(r) * 2304);
-                w[tp][r].qa = *(const uint4 *)(pq[tp] + blk(r) * 2304);
-                w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * 2304 + 1152);
+                w[tp][r].h.x = fh_ld_weights<ONCE, uint32_t>(ph[tp] + blk(r) * 2304);
+                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 2304);
+                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 2304 + 1152);
             } else if (FMT == FH_Q8_0) {
-                w[tp][r].h.x = *(const uint32_t *)(ph[tp] + blk(r) * 4352);
-                w[tp][r].qa = *(const uint4 *)(pq[tp] + blk(r) * 4352);
-                w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * 4352 + 1088);
-                w[tp][r].qc = *(const uint4 *)(pq[tp] + blk(r) * 4352 + 2176);
-                w[tp][r].qd = *(const uint4 *)(pq[tp] + blk(r) * 4352 + 3264);
+                w[tp][r].h.x = fh_ld_weights<ONCE, uint32_t>(ph[tp] + blk(r) * 4352);
+                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 4352);
+                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 4352 + 1088);
+                w[tp][r].qc = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 4352 + 2176);
+                w[tp][r].qd = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 4352 + 3264);
             } else {
-                w[tp][r].h = *(const uint4 *)(ph[tp] + blk(r) * RS * 2304);
-                w[tp][r].qa = *(const uint4 *)(pq[tp] + blk(r) * RS * 2304);
-                w[tp][r].qb = *(const uint4 *)(pq[tp] + blk(r) * RS * 2304 + 1024);
+                w[tp][r].h = fh_ld_weights<ONCE, uint4>(ph[tp] + blk(r) * RS * 2304);
+                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * RS * 2304);
+                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * RS * 2304 + 1024);
             }
         }
     // What the last phase adds or rotates by is asked for here and below, by every wavefront (no branch); asked for there it was one or two trips to memory
@@ -632,13 +632,13 @@ static fh_status q4k_m1_start(q4k_m1_kern kern, const fh_qmatrix *q, dim3 grid, 
     FH_HIP(hipGetLastError());
     return FH_OK;
 }
-template <int TPW, int PER, int EPI, int IN>
+template <int TPW, int PER, int EPI, int IN, bool ONCE>
 __global__ __launch_bounds__(1024) void k_qmv_q4k_m1(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FH_Q4_K, TPW, PER, EPI, IN>(Q4K_M1_ARGS);
+    qmv_q4k_m1_body<FH_Q4_K, TPW, PER, EPI, IN, 1, 1, false, ONCE>(Q4K_M1_ARGS);
 }
-template <int TPW, int PER, int EPI, int IN>
+template <int TPW, int PER, int EPI, int IN, bool ONCE>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_qmv_q4k_m1_w8(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FH_Q4_K, TPW, PER, EPI, IN>(Q4K_M1_ARGS);
+    qmv_q4k_m1_body<FH_Q4_K, TPW, PER, EPI, IN, 1, 1, false, ONCE>(Q4K_M1_ARGS);
 }
 // 16 / RS rows of a tile per workgroup, RS blocks at once per wavefront (matrices with few row tiles)
 template <int RS, int PER, int EPI, int IN>
@@ -646,31 +646,33 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
     qmv_q4k_m1_body<FH_Q4_K, 1, PER, EPI, IN, 1, RS>(Q4K_M1_ARGS);
 }
 // 2 .. 4 activation rows (plain input; epilogues none / add2); nsplit = number of valid rows
-template <int FMT, int TPW, int PER, int EPI, int MR>
+template <int FMT, int TPW, int PER, int EPI, int MR, bool ONCE>
 __global__ __launch_bounds__(1024) void k_qmv_q4k_mr(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0, MR>(Q4K_M1_ARGS);
+    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0, MR, 1, false, ONCE>(Q4K_M1_ARGS);
 }
 // Q4_0 / Q8_0 weights (plain input; epilogues none / add2 / SwiGLU)
-template <int FMT, int TPW, int PER, int EPI>
+template <int FMT, int TPW, int PER, int EPI, bool ONCE>
 __global__ __launch_bounds__(1024) void k_qmv_q40_m1(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0>(Q4K_M1_ARGS);
+    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0, 1, 1, false, ONCE>(Q4K_M1_ARGS);
 }
-template <int FMT, int TPW, int PER, int EPI>
+template <int FMT, int TPW, int PER, int EPI, bool ONCE>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_qmv_q40_m1_w8(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0>(Q4K_M1_ARGS);
+    qmv_q4k_m1_body<FMT, TPW, PER, EPI, 0, 1, 1, false, ONCE>(Q4K_M1_ARGS);
 }
 
 // k of more than 16 blocks that no number of up to 16 wavefronts shares out evenly (43 of 11008 columns); epilogues none / add2
-template <int FMT, int PER, int EPI>
+template <int FMT, int PER, int EPI, bool ONCE>
 __global__ __launch_bounds__(1024) void k_qmv_q4k_m1_rag(Q4K_M1_PARAMS) {
-    qmv_q4k_m1_body<FMT, 1, PER, EPI, 0, 1, 1, true>(Q4K_M1_ARGS);
+    qmv_q4k_m1_body<FMT, 1, PER, EPI, 0, 1, 1, true, ONCE>(Q4K_M1_ARGS);
 }
+
+#define Q4K_ONCE(K_, ...) (fh_weights_once(q) ? K_<__VA_ARGS__, true> : K_<__VA_ARGS__, false>)
 
 template <int FMT, int PER>
 static fh_status q4k_m1_rag_go(const fh_qmatrix *q, const float *x, float *y, int epi, const float *a, const float *b) {
     const int SW = (int)(q->k / 256 + PER - 1) / PER, kb = SW * PER;
     const size_t lds = (size_t)kb * Q4K_IMG * 16 + (size_t)kb * 64 + 16 * 64 + 64;
-    const auto kern = epi == FH_EPI_ADD2 ? k_qmv_q4k_m1_rag<FMT, PER, FH_EPI_ADD2> : k_qmv_q4k_m1_rag<FMT, PER, FH_EPI_NONE>;
+    const auto kern = epi == FH_EPI_ADD2 ? Q4K_ONCE(k_qmv_q4k_m1_rag, FMT, PER, FH_EPI_ADD2) : Q4K_ONCE(k_qmv_q4k_m1_rag, FMT, PER, FH_EPI_NONE);
     return q4k_m1_start(kern, q, dim3((unsigned)((q->n + 15) / 16)), SW, lds, x, y, a, b);
 }
 
@@ -698,8 +700,8 @@ static fh_status q4k_m1_launch(const fh_qmatrix *q, const float *x, float *y, co
     if (q->type == FH_Q5_0) { // (17 registers of weights per block tile, as Q8_0)
         if constexpr ((EPI == FH_EPI_NONE || EPI == FH_EPI_ADD2 || EPI == FH_EPI_SWIGLU) && !(EPI == FH_EPI_SWIGLU && TPW == 1)) {
             if (in != 0) return FH_ERR_UNSUPPORTED;
-            if constexpr (TPW * PER == 1) kern = k_qmv_q40_m1_w8<FH_Q5_0, TPW, PER, EPI>;
-            else kern = k_qmv_q40_m1<FH_Q5_0, TPW, PER, EPI>;
+            if constexpr (TPW * PER == 1) kern = Q4K_ONCE(k_qmv_q40_m1_w8, FH_Q5_0, TPW, PER, EPI);
+            else kern = Q4K_ONCE(k_qmv_q40_m1, FH_Q5_0, TPW, PER, EPI);
             return q4k_m1_start(kern, q, dim3(grid, 1), SW, lds, x, y, a, b);
         } else {
             return FH_ERR_UNSUPPORTED;
@@ -708,8 +710,8 @@ static fh_status q4k_m1_launch(const fh_qmatrix *q, const float *x, float *y, co
     if (q->type == FH_Q5_K) { // (14 registers of weights per block tile: budgeted like Q8_0)
         if constexpr ((EPI == FH_EPI_NONE || EPI == FH_EPI_ADD2 || EPI == FH_EPI_SWIGLU) && !(EPI == FH_EPI_SWIGLU && TPW == 1)) {
             if (in != 0) return FH_ERR_UNSUPPORTED;
-            if constexpr (TPW * PER == 1) kern = k_qmv_q40_m1_w8<FH_Q5_K, TPW, PER, EPI>;
-            else kern = k_qmv_q40_m1<FH_Q5_K, TPW, PER, EPI>;
+            if constexpr (TPW * PER == 1) kern = Q4K_ONCE(k_qmv_q40_m1_w8, FH_Q5_K, TPW, PER, EPI);
+            else kern = Q4K_ONCE(k_qmv_q40_m1, FH_Q5_K, TPW, PER, EPI);
             return q4k_m1_start(kern, q, dim3(grid, 1), SW, lds, x, y, a, b);
         } else {
             return FH_ERR_UNSUPPORTED;
@@ -720,10 +722,10 @@ static fh_status q4k_m1_launch(const fh_qmatrix *q, const float *x, float *y, co
             if (in != 0) return FH_ERR_UNSUPPORTED;
             const bool q8 = q->type == FH_Q8_0;
             if constexpr (TPW * PER <= 2) { // Q8_0 holds 17 registers of weights per block tile: one fits the budget
-                if constexpr (TPW * PER == 1) kern = q8 ? k_qmv_q40_m1_w8<FH_Q8_0, TPW, PER, EPI> : k_qmv_q40_m1_w8<FH_Q4_0, TPW, PER, EPI>;
-                else kern = q8 ? k_qmv_q40_m1<FH_Q8_0, TPW, PER, EPI> : k_qmv_q40_m1_w8<FH_Q4_0, TPW, PER, EPI>;
+                if constexpr (TPW * PER == 1) kern = q8 ? Q4K_ONCE(k_qmv_q40_m1_w8, FH_Q8_0, TPW, PER, EPI) : Q4K_ONCE(k_qmv_q40_m1_w8, FH_Q4_0, TPW, PER, EPI);
+                else kern = q8 ? Q4K_ONCE(k_qmv_q40_m1, FH_Q8_0, TPW, PER, EPI) : Q4K_ONCE(k_qmv_q40_m1_w8, FH_Q4_0, TPW, PER, EPI);
             } else {
-                kern = q8 ? k_qmv_q40_m1<FH_Q8_0, TPW, PER, EPI> : k_qmv_q40_m1<FH_Q4_0, TPW, PER, EPI>;
+                kern = q8 ? Q4K_ONCE(k_qmv_q40_m1, FH_Q8_0, TPW, PER, EPI) : Q4K_ONCE(k_qmv_q40_m1, FH_Q4_0, TPW, PER, EPI);
             }
             return q4k_m1_start(kern, q, dim3(grid, 1), SW, lds, x, y, a, b);
         } else {
@@ -731,14 +733,14 @@ static fh_status q4k_m1_launch(const fh_qmatrix *q, const float *x, float *y, co
         }
     }
     if constexpr (TPW * PER <= 2) {
-        kern = in == 2 ? k_qmv_q4k_m1<TPW, PER, EPI, 2>
-                       : (in == 1 ? k_qmv_q4k_m1_w8<TPW, PER, EPI, 1> : k_qmv_q4k_m1_w8<TPW, PER, EPI, 0>);
+        kern = in == 2 ? Q4K_ONCE(k_qmv_q4k_m1, TPW, PER, EPI, 2)
+                       : (in == 1 ? Q4K_ONCE(k_qmv_q4k_m1_w8, TPW, PER, EPI, 1) : Q4K_ONCE(k_qmv_q4k_m1_w8, TPW, PER, EPI, 0));
     } else if constexpr (EPI == FH_EPI_ACC && PER == 1) {
-        kern = in == 2 ? k_qmv_q4k_m1<TPW, PER, EPI, 2>
-                       : (in == 1 ? k_qmv_q4k_m1<TPW, PER, EPI, 1> : k_qmv_q4k_m1<TPW, PER, EPI, 0>);
+        kern = in == 2 ? Q4K_ONCE(k_qmv_q4k_m1, TPW, PER, EPI, 2)
+                       : (in == 1 ? Q4K_ONCE(k_qmv_q4k_m1, TPW, PER, EPI, 1) : Q4K_ONCE(k_qmv_q4k_m1, TPW, PER, EPI, 0));
     } else {
         if (in == 2) return FH_ERR_UNSUPPORTED; // the merge of the attention partials needs the registers
-        kern = in == 1 ? k_qmv_q4k_m1<TPW, PER, EPI, 1> : k_qmv_q4k_m1<TPW, PER, EPI, 0>;
+        kern = in == 1 ? Q4K_ONCE(k_qmv_q4k_m1, TPW, PER, EPI, 1) : Q4K_ONCE(k_qmv_q4k_m1, TPW, PER, EPI, 0);
     }
     return q4k_m1_start(kern, q, dim3(grid, (unsigned)ex.ksplit), SW, lds, x, y, a, b, ex.xres, ex.nw, ex.eps, ex.nsplit, ex.rk);
 }
@@ -791,7 +793,7 @@ static fh_status q4k_mr_parts(const fh_qmatrix *q, const float *x, int m, float 
     int tpw = (int)dev->opt_matvec_tiles;
     if (tpw != 1 && tpw != 2) tpw = tiles * parts > 2 * (int64_t)dev->compute_units ? 2 : 1;
     FH_TRY(fh_dev_scratch(dev, (void **)&dev->ksplit_buf, &dev->ksplit_cap, (size_t)parts * 16 * q->n * 4));
-    const q4k_m1_kern kern = tpw == 2 ? (q4k_m1_kern)k_qmv_q4k_mr<FMT, 2, 1, FH_EPI_NONE, MR> : (q4k_m1_kern)k_qmv_q4k_mr<FMT, 1, 1, FH_EPI_NONE, MR>;
+    const q4k_m1_kern kern = tpw == 2 ? Q4K_ONCE(k_qmv_q4k_mr, FMT, 2, 1, FH_EPI_NONE, MR) : Q4K_ONCE(k_qmv_q4k_mr, FMT, 1, 1, FH_EPI_NONE, MR);
     FH_TRY(q4k_m1_start(kern, q, dim3((unsigned)((tiles + tpw - 1) / tpw), (unsigned)parts), SW, lds, x, (float *)dev->ksplit_buf, nullptr, nullptr, nullptr,
                         nullptr, 0.f, m));
     return fh_launch_kparts_reduce(dev, (const float *)dev->ksplit_buf, parts, m, q->n, y, EPI, a, b);
@@ -815,8 +817,8 @@ static fh_status q4k_mr_go(const fh_qmatrix *q, const float *x, int m, float *y,
     if (tpw != 1 && tpw != 2) tpw = tiles > dev->compute_units ? 2 : 1;
     if (per == 2) tpw = 1;
     const unsigned grid = (unsigned)((tiles + tpw - 1) / tpw);
-    const q4k_m1_kern kern = per == 2 ? (q4k_m1_kern)k_qmv_q4k_mr<FMT, 1, 2, EPI, MR>
-                                 : (tpw == 2 ? (q4k_m1_kern)k_qmv_q4k_mr<FMT, 2, 1, EPI, MR> : (q4k_m1_kern)k_qmv_q4k_mr<FMT, 1, 1, EPI, MR>);
+    const q4k_m1_kern kern = per == 2 ? Q4K_ONCE(k_qmv_q4k_mr, FMT, 1, 2, EPI, MR)
+                                 : (tpw == 2 ? Q4K_ONCE(k_qmv_q4k_mr, FMT, 2, 1, EPI, MR) : Q4K_ONCE(k_qmv_q4k_mr, FMT, 1, 1, EPI, MR));
     return q4k_m1_start(kern, q, dim3(grid, 1), SW, lds, x, y, a, b, nullptr, nullptr, 0.f, m);
 }
 

@@ -28,7 +28,7 @@ struct Q6KRegs {
 // the SwiGLU epilogue: gate tiles and the matching up tiles), stages the activations of its own blocks only (no
 // barrier before the products) and requests all its weight bytes before anything else.
 // RAG: the blocks are no multiple of the wavefronts'; what a wavefront has past the last one is the last one again, times zero.
-template <int TPW, int PER, int EPI, bool RAG = false>
+template <int TPW, int PER, int EPI, bool RAG, bool ONCE>
 __global__ __launch_bounds__(1024) void k_qmv_q6k_m1(const uint8_t *data, const float *__restrict__ x, const float *__restrict__ xup, int recs, int n, int k, int SW,
                                                       float *__restrict__ y, const float *__restrict__ ea, const float *__restrict__ eb) {
     const QView q{data, n, k, 0, recs, 0}; // (plain values, the first needed first: in registers when the kernel starts)
@@ -77,10 +77,10 @@ __global__ __launch_bounds__(1024) void k_qmv_q6k_m1(const uint8_t *data, const 
 #pragma unroll
         for (int tp = 0; tp < TPW; tp++) {
             const uint8_t *p = rec[tp] + blk(r) * 3360;
-            w[tp][r].l0 = *(const uint4 *)(p + lane * 16);
-            w[tp][r].l1 = *(const uint4 *)(p + 1024 + lane * 16);
-            w[tp][r].h = *(const uint4 *)(p + 2048 + lane * 16);
-            w[tp][r].sc = *(const uint32_t *)(p + 3072 + lane * 4);
+            w[tp][r].l0 = fh_ld_weights<ONCE, uint4>(p + lane * 16);
+            w[tp][r].l1 = fh_ld_weights<ONCE, uint4>(p + 1024 + lane * 16);
+            w[tp][r].h = fh_ld_weights<ONCE, uint4>(p + 2048 + lane * 16);
+            w[tp][r].sc = fh_ld_weights<ONCE, uint32_t>(p + 3072 + lane * 4);
             w[tp][r].d = *(const uint16_t *)(p + 3328 + 2 * j);
         }
     // ---- 2. stage x: lane owns k = 256*b + 4*lane .. +3, i.e. a quarter of group G = lane / 4.  A wavefront stages
@@ -236,8 +236,9 @@ __global__ __launch_bounds__(1024) void k_qmv_q6k_m1(const uint8_t *data, const 
 template <int TPW, int PER, int EPI>
 static fh_status q6k_m1_launch(const fh_qmatrix *q, const float *x, float *y, const float *a, const float *b, int SW,
                                unsigned grid, size_t lds, unsigned ksplit = 1, const float *xup = nullptr) {
-    FH_TRY(fh_kernel_lds(q->dev, (const void *)k_qmv_q6k_m1<TPW, PER, EPI>, 160 * 1024));
-    k_qmv_q6k_m1<TPW, PER, EPI><<<dim3(grid, ksplit), dim3(64 * SW), lds, q->dev->stream>>>(q->data, x, xup, (int)q->recs, (int)q->n, (int)q->k, SW, y, a, b);
+    const auto kern = fh_weights_once(q) ? k_qmv_q6k_m1<TPW, PER, EPI, false, true> : k_qmv_q6k_m1<TPW, PER, EPI, false, false>;
+    FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
+    kern<<<dim3(grid, ksplit), dim3(64 * SW), lds, q->dev->stream>>>(q->data, x, xup, (int)q->recs, (int)q->n, (int)q->k, SW, y, a, b);
     FH_HIP(hipGetLastError());
     return FH_OK;
 }
@@ -246,8 +247,9 @@ template <int PER, int EPI>
 static fh_status q6k_m1_rag(const fh_qmatrix *q, const float *x, float *y, const float *a, const float *b) {
     const int SW = (int)(q->kb + PER - 1) / PER, kb = SW * PER;
     const size_t lds = (size_t)kb * Q6K_IMG * 16 + (size_t)kb * Q6K_SF * 4 + (size_t)SW * 64;
-    FH_TRY(fh_kernel_lds(q->dev, (const void *)k_qmv_q6k_m1<1, PER, EPI, true>, 160 * 1024));
-    k_qmv_q6k_m1<1, PER, EPI, true><<<dim3((unsigned)((q->n + 15) / 16)), dim3(64 * SW), lds, q->dev->stream>>>(q->data, x, nullptr, (int)q->recs, (int)q->n, (int)q->k, SW, y, a, b);
+    const auto kern = fh_weights_once(q) ? k_qmv_q6k_m1<1, PER, EPI, true, true> : k_qmv_q6k_m1<1, PER, EPI, true, false>;
+    FH_TRY(fh_kernel_lds(q->dev, (const void *)kern, 160 * 1024));
+    kern<<<dim3((unsigned)((q->n + 15) / 16)), dim3(64 * SW), lds, q->dev->stream>>>(q->data, x, nullptr, (int)q->recs, (int)q->n, (int)q->k, SW, y, a, b);
     FH_HIP(hipGetLastError());
     return FH_OK;
 }

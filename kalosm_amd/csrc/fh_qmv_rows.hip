@@ -114,7 +114,7 @@ struct RowsTile {
     static constexpr int TILES = 16 / KC * TT, IMG = KC * RowsX<T>::BYTES, RED = 16 * TT * 272 * 4, LDS = IMG > RED ? IMG : RED;
 };
 
-template <int T, int KC, int TT>
+template <int T, int KC, int TT, bool ONCE>
 __global__ __launch_bounds__(1024) void k_qmv_rows(const uint8_t *data, const float *__restrict__ x, int n, int k, int m, int wtiles, int parts, float *__restrict__ part,
                                                    uint32_t *__restrict__ arrived, float *__restrict__ y) {
     const QView q{data, n, k, 0, 0, 0}; // (plain values: in registers when the kernel starts)
@@ -140,8 +140,8 @@ __global__ __launch_bounds__(1024) void k_qmv_rows(const uint8_t *data, const fl
         int at = (group * (16 / KC) + tg) * TT + t;
         at = at < wtiles ? at : wtiles - 1;
         const uint8_t *rec = q.data + ((int64_t)at * chunks + c) * REC;
-        w[s].ask_a(rec, lane);
-        w[s].ask_b(rec, lane);
+        w[s].template ask_a<ONCE>(rec, lane);
+        w[s].template ask_b<ONCE>(rec, lane);
     };
     ask(0, 0);
     if (TT > 1) ask(1, 1);
@@ -263,8 +263,9 @@ static fh_status rows_go(const fh_qmatrix *q, const float *x, int m, float *y) {
         if (!fh_dev_scratch_try(dev, (void **)&dev->ksplit_buf, &dev->ksplit_cap, (size_t)groups * parts * Tile::TILES * 1024)) return FH_ERR_UNSUPPORTED;
         part = dev->ksplit_buf;
     }
-    FH_TRY(fh_kernel_lds(dev, (const void *)k_qmv_rows<T, KC, TT>, (size_t)Tile::LDS));
-    k_qmv_rows<T, KC, TT><<<dim3((unsigned)(groups * parts)), 1024, Tile::LDS, dev->stream>>>(q->data, x, (int)q->n, (int)q->k, m, tiles, parts, part, dev->arrived, y);
+    const auto kern = fh_weights_once(q) ? k_qmv_rows<T, KC, TT, true> : k_qmv_rows<T, KC, TT, false>;
+    FH_TRY(fh_kernel_lds(dev, (const void *)kern, (size_t)Tile::LDS));
+    kern<<<dim3((unsigned)(groups * parts)), 1024, Tile::LDS, dev->stream>>>(q->data, x, (int)q->n, (int)q->k, m, tiles, parts, part, dev->arrived, y);
     FH_HIP(hipGetLastError());
     return FH_OK;
 }

@@ -1,6 +1,7 @@
 // Weights of the tiled layout decoded in a lane's registers into operands of the matrix cores (fh_qmm_reg.hip, fh_qmv_rows.hip).
 #pragma once
 #include "fh_blocks.h"
+#include "fh_mv_lanes.h"
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -42,12 +43,14 @@ struct RegK { // Q4_K, Q5_K
     uint4 next, cod[2];
     uint2 next5, five;
     uint32_t dm, sc[2], mn[2];
+    template <bool ONCE = false>
     __device__ __forceinline__ void ask_a(const uint8_t *rec, int lane) {
-        next = *(const uint4 *)(rec + (lane & 15) * 16);
-        cod[0] = *(const uint4 *)(rec + 256 + lane * 16);
-        if (T == FH_Q5_K) next5 = *(const uint2 *)(rec + 2304 + lane * 8);
+        next = fh_ld_weights<ONCE, uint4>(rec + (lane & 15) * 16);
+        cod[0] = fh_ld_weights<ONCE, uint4>(rec + 256 + lane * 16);
+        if (T == FH_Q5_K) next5 = fh_ld_weights<ONCE, uint2>(rec + 2304 + lane * 8);
     }
-    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { cod[1] = *(const uint4 *)(rec + 1280 + lane * 16); }
+    template <bool ONCE = false>
+    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { cod[1] = fh_ld_weights<ONCE, uint4>(rec + 1280 + lane * 16); }
     __device__ __forceinline__ void begin() {
         dm = next.x, five = next5;
         sc[0] = next.y & 0x3F3F3F3Fu, sc[1] = (next.w & 0x0F0F0F0Fu) | ((next.y >> 2) & 0x30303030u);
@@ -94,13 +97,15 @@ struct RegW<FH_Q6_K> {
     uint4 lo[2], next_hi, hi;
     uint32_t next_sc, sc[4], at;
     uint16_t next_d, dv;
+    template <bool ONCE = false>
     __device__ __forceinline__ void ask_a(const uint8_t *rec, int lane) {
-        lo[0] = *(const uint4 *)(rec + lane * 16);
-        next_hi = *(const uint4 *)(rec + 2048 + lane * 16);
-        next_sc = *(const uint32_t *)(rec + 3072 + lane * 4);
+        lo[0] = fh_ld_weights<ONCE, uint4>(rec + lane * 16);
+        next_hi = fh_ld_weights<ONCE, uint4>(rec + 2048 + lane * 16);
+        next_sc = fh_ld_weights<ONCE, uint32_t>(rec + 3072 + lane * 4);
         next_d = fh_ld16(rec + 3328 + (lane & 15) * 2);
     }
-    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { lo[1] = *(const uint4 *)(rec + 1024 + lane * 16); }
+    template <bool ONCE = false>
+    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { lo[1] = fh_ld_weights<ONCE, uint4>(rec + 1024 + lane * 16); }
     __device__ __forceinline__ void begin() {
         hi = next_hi, dv = next_d;
         const int lane = (int)threadIdx.x & 63;
@@ -133,15 +138,18 @@ struct RegW<FH_Q8_0> {
     static constexpr int REC = 4352, QA = 4, QB = 4, NW = 1;
     uint4 cod[2][2];
     uint32_t dd[2][2];
+    template <bool ONCE = false>
     __device__ __forceinline__ void ask(int p, const uint8_t *rec, int lane) {
 #pragma unroll
         for (int r = 0; r < 2; r++) {
-            cod[p][r] = *(const uint4 *)(rec + (2 * p + r) * 1088 + lane * 16);
-            dd[p][r] = *(const uint32_t *)(rec + (2 * p + r) * 1088 + 1024 + (lane & 15) * 4);
+            cod[p][r] = fh_ld_weights<ONCE, uint4>(rec + (2 * p + r) * 1088 + lane * 16);
+            dd[p][r] = fh_ld_weights<ONCE, uint32_t>(rec + (2 * p + r) * 1088 + 1024 + (lane & 15) * 4);
         }
     }
-    __device__ __forceinline__ void ask_a(const uint8_t *rec, int lane) { ask(0, rec, lane); }
-    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { ask(1, rec, lane); }
+    template <bool ONCE = false>
+    __device__ __forceinline__ void ask_a(const uint8_t *rec, int lane) { ask<ONCE>(0, rec, lane); }
+    template <bool ONCE = false>
+    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { ask<ONCE>(1, rec, lane); }
     __device__ __forceinline__ void begin() {}
     __device__ __forceinline__ void get(int sb, uint32_t, half8 (&out)[1]) const {
         const uint4 c = cod[sb >> 2][(sb >> 1) & 1];
@@ -158,13 +166,16 @@ struct Reg4 { // Q4_0, Q5_0
     uint4 cod[2];
     uint2 dd[2];
     uint32_t five[2];
+    template <bool ONCE = false>
     __device__ __forceinline__ void ask(int p, const uint8_t *rec, int lane) {
-        cod[p] = *(const uint4 *)(rec + p * HALF + lane * 16);
-        dd[p] = *(const uint2 *)(rec + p * HALF + 1024 + (lane & 15) * 8);
-        if (T == FH_Q5_0) five[p] = *(const uint32_t *)(rec + p * HALF + 1152 + lane * 4);
+        cod[p] = fh_ld_weights<ONCE, uint4>(rec + p * HALF + lane * 16);
+        dd[p] = fh_ld_weights<ONCE, uint2>(rec + p * HALF + 1024 + (lane & 15) * 8);
+        if (T == FH_Q5_0) five[p] = fh_ld_weights<ONCE, uint32_t>(rec + p * HALF + 1152 + lane * 4);
     }
-    __device__ __forceinline__ void ask_a(const uint8_t *rec, int lane) { ask(0, rec, lane); }
-    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { ask(1, rec, lane); }
+    template <bool ONCE = false>
+    __device__ __forceinline__ void ask_a(const uint8_t *rec, int lane) { ask<ONCE>(0, rec, lane); }
+    template <bool ONCE = false>
+    __device__ __forceinline__ void ask_b(const uint8_t *rec, int lane) { ask<ONCE>(1, rec, lane); }
     __device__ __forceinline__ void begin() {}
     // q - 8 (q - 16) from 1024 + q, high nibbles from 1024 + 16 q
     __device__ __forceinline__ void get(int sb, uint32_t one, half8 (&out)[1]) const {

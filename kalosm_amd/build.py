@@ -22,15 +22,19 @@ FLAGS = [
     "-fPIC",
     "-ffp-contract=off",          # dequantised values are compared bit for bit: never fuse a*b - c
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    "-mllvm", "-amdgpu-kernarg-preload-count=14",  # the first words of a kernel's plain arguments are in registers when it starts
     "-Wall", "-Wno-unused-function", "-Wno-unknown-warning-option", "-Wno-unused-command-line-argument",
     "-fvisibility=hidden",
 ]
+AHEAD = ["-mllvm", "-amdgpu-kernarg-preload-count=14"]  # the first words of a kernel's plain arguments are in registers when it starts
+# Arguments are loaded ahead only where the first requests need no others: prompt attention's need three pointers and nine strides
+# (8 heads of 128, 300 tokens: 10.18 us without, 10.25 with).
+LOADS_ARGUMENTS = {"fh_attention_prefill.hip"}
 
 
 def _compile(src: str) -> str:
     obj = os.path.join(OBJ, os.path.basename(src) + ".o")
-    cmd = [HIPCC, *FLAGS, "-c", src, "-o", obj]
+    ahead = [] if os.path.basename(src) in LOADS_ARGUMENTS else AHEAD
+    cmd = [HIPCC, *FLAGS, *ahead, "-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stdout}\n{r.stderr}")

@@ -11,6 +11,7 @@
 // row is spread over D / 8 lanes (32 bytes of f32 or 16 bytes of f16 each).  Partial results go to [q head][split][D + 4]:
 // unnormalised output, running max, running sum; k_attn_combine_dl (or the consumer of the partials) merges them.
 #include "fh_internal.h"
+#include <algorithm>
 
 typedef _Float16 fh_half;
 
@@ -651,10 +652,15 @@ fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *
     const int mfma_min = dev->opt_attn_kernel == 5 ? 32 : 4096;
     if (kv_dtype == FH_F16 && d == 128 && hq % hkv == 0 && hq / hkv <= 16 && skv >= mfma_min &&
         (dev->opt_attn_kernel == 0 || dev->opt_attn_kernel == 5) && dev->opt_attn_heads == 0 && kv_st % 8 == 0 && kv_sh % 8 == 0) {
-        // parts: four wavefronts each, two chunks of 32 keys per wavefront, at most 128 parts for the merge (measured on
-        // MI355X, 32 / 8 heads: 19.2 us against 22.0 us of the vector-ALU kernel at 16384 keys, level at 4096)
+        // parts: a workgroup of four wavefronts each, one a compute unit; two a compute unit where a wavefront would have more than three chunks of 32 keys.
+        // us of a call of 32 / 8 heads, eight chunks a part / one workgroup a compute unit / two: 4096 keys 9.8 / 9.0 / 9.0, 6000 11.7 / 10.4 / 12.2, 8192 11.7 / 11.6 /
+        // 11.8, 12000 16.5 / 13.1 / 13.8 (368 workgroups are two rounds on some compute units), 16384 16.9 / 17.9 / 16.9, 30000 27.9 / 24.1 / 24.4; 16 heads of
+        // their own, 5000 keys 15.7 / 11.4 / 11.8, 32 heads, 8192 26.5 / 26.4 / 25.9.  (The vector-ALU kernels: 22.0 at 16384.)  At most 128 parts for the merge.
         const int nct = (skv + 31) / 32;
-        int splits = dev->opt_attn_splits > 0 ? (int)dev->opt_attn_splits : nct / 8;
+        int splits = std::max(1, dev->compute_units / hkv);
+        if (nct > 12 * splits) splits = std::max(1, 2 * dev->compute_units / hkv);
+        splits = std::min(splits, nct / 2);
+        if (dev->opt_attn_splits > 0) splits = (int)dev->opt_attn_splits;
         splits = splits < 1 ? 1 : (splits > 128 ? 128 : splits);
         FH_TRY(fh_dev_scratch(dev, (void **)&dev->part_buf, &dev->part_cap, (size_t)hq * splits * (128 + 4) * 4));
         fh_status st = fh_attention_decode_mfma(dev, q, q_f16, k, v, kv_sh, kv_st, hq, hkv, d, scale, skv, splits, dev->part_buf);

@@ -13,8 +13,10 @@
 //           LDS tile of V rows through the transposing load (ds_read_b64_tr_b16)
 // so a wavefront spends about 140 instructions per 32 keys and the kernel is a stream of cache rows.
 // grid (S parts, KV heads); chunk c of 32 keys belongs to part c mod S, and the wavefronts of a workgroup take the
-// part's chunks in turn, each with its own running maximum, denominator and output; the next chunk of a wavefront
-// is in flight (128 registers) while the current one is multiplied.  No barrier until the wavefronts merge at the
+// part's chunks in turn, each with its own running maximum, denominator and output; the next chunk's keys are asked for when the
+// current one's have been multiplied, its values when the current ones are in LDS: a wavefront has 16 KB on their way at any time.  (All of the next chunk
+// ahead of the current one, 32 KB, is more than the memory takes gladly: 16384 keys, 32 / 8 heads, 17.5 us a call / 17.0 so, 8192 12.8 / 11.6, 4096 10.2 /
+// 9.7, before the parts' number changed.)  No barrier until the wavefronts merge at the
 // end (LDS operations of one wavefront execute in order, and every wavefront reads only the tile it wrote).
 // Partials as the other decode kernels write them: [head][part][128 weighted sums | max | denominator | 2 unused].
 #include "fh_internal.h"
@@ -92,22 +94,20 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_decode_mfma(const void *__res
 #pragma unroll
     for (int t = 0; t < DT; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    u32x4 kr0[2][4], vr0[2][4], kr1[2][4], vr1[2][4]; // two buffers of [16-key block][step]
-    auto issue = [&](u32x4 (&kr)[2][4], u32x4 (&vr)[2][4], int j) { // local chunk j of the part (past the end: the last row again, never used)
+    u32x4 kr[2][4], vr[2][4]; // [16-key block][step]
+    auto issue = [&](u32x4 (&r)[2][4], const fh_half *base, int j) { // local chunk j of the part (past the end: the last row again, never used)
         const int row0 = CK * (j * S + split);
 #pragma unroll
         for (int blk = 0; blk < 2; blk++) {
             int row = row0 + 16 * blk + i;
             row = row < skv ? row : skv - 1;
-            const fh_half *kp = kb + (int64_t)row * kv_st, *vp = vb + (int64_t)row * kv_st;
+            const fh_half *p = base + (int64_t)row * kv_st;
 #pragma unroll
-            for (int s = 0; s < 4; s++) {
-                kr[blk][s] = *(const u32x4 *)(kp + 32 * s);
-                vr[blk][s] = *(const u32x4 *)(vp + 32 * s);
-            }
+            for (int s = 0; s < 4; s++) r[blk][s] = *(const u32x4 *)(p + 32 * s);
         }
+        __builtin_amdgcn_sched_barrier(0);
     };
-    auto process = [&](const u32x4 (&kr)[2][4], const u32x4 (&vr)[2][4], int j) {
+    auto process = [&](int j) {
         const int row0 = CK * (j * S + split);
         // ---- scores of the two 16-key blocks: register r of block blk is key row0 + 16 blk + 4 g + r, column = head
         floatx4 st[2];
@@ -119,11 +119,15 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_decode_mfma(const void *__res
                 st[blk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, kr[blk][s]), qf[s], st[blk], 0, 0, 0);
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
+        issue(kr, kb, j + NWV);
         // ---- V rows into the wavefront's LDS tile (a clamped row past the end holds live data and meets a zero weight)
 #pragma unroll
         for (int blk = 0; blk < 2; blk++)
 #pragma unroll
             for (int s = 0; s < 4; s++) *(u32x4 *)(sv + (16 * blk + i) * VS + 32 * s + 8 * g) = vr[blk][s];
+        __builtin_amdgcn_sched_barrier(0);
+        issue(vr, vb, j + NWV);
         // ---- mask the keys past the end (only the last chunk has any), running max over the chunk
         float mx = -INFINITY;
         if (row0 + CK > skv) {
@@ -164,20 +168,11 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_decode_mfma(const void *__res
 #pragma unroll
         for (int t = 0; t < DT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(am_vt8(vp + 16 * t, VS), pb, acc[t], 0, 0, 0);
     };
-    // the wavefront's chunks: wave, wave + NWV, ...; two per trip, each requested one chunk ahead
-    // (no branches around the requests - a wait after a branch waits for everything in flight: requests past the
-    // end re-read the last live row and are dropped)
-    issue(kr0, vr0, wave);
-    for (int j = wave; j < nc; j += 2 * NWV) {
-        issue(kr1, vr1, j + NWV);
-        __builtin_amdgcn_sched_barrier(0); // the requests stay ahead of the arithmetic on the other chunk
-        process(kr0, vr0, j);
-        __builtin_amdgcn_sched_barrier(0);
-        issue(kr0, vr0, j + 2 * NWV);
-        __builtin_amdgcn_sched_barrier(0);
-        if (j + NWV < nc) process(kr1, vr1, j + NWV);
-        __builtin_amdgcn_sched_barrier(0);
-    }
+    // the wavefront's chunks: wave, wave + NWV, ... (no branches around the requests - a wait after a branch waits for everything in flight: requests
+    // past the end re-read the last live row and are dropped)
+    issue(kr, kb, wave);
+    issue(vr, vb, wave);
+    for (int j = wave; j < nc; j += NWV) process(j);
     // ---- merge the wavefronts: lane (head i, g) holds d = 16 t + 4 g + r of tile t
     l_run = am_rows_sum(l_run);
     __syncthreads(); // every wavefront is done with its V tile

@@ -643,6 +643,19 @@ fh_status fh_attention_combine_parts(fh_device *dev, const float *part, int hq, 
     return FH_OK;
 }
 
+// Query heads a workgroup.  Long caches are bandwidth bound: two, so that K and V are read less often (32 / 8 heads, f16 cache: 1 head x 8 parts x 16 wavefronts
+// at 1024 keys, 2 x 16 x 8 at 4096).  Short ones: one, unless that makes more workgroups than compute units, which two of sixteen wavefronts fill
+// one after the other (us of 64 / 8 heads, one / two: 300 keys 10.8 / 9.5, 1000 10.8 / 9.5, 2040 11.1 / 9.9; 32 / 8 heads 9.0 / 9.3, 9.0 / 9.4, 8.9 / 9.8).
+static int ad_heads(const fh_device *dev, int hq, int skv) {
+    return dev->opt_attn_heads > 0 ? (int)dev->opt_attn_heads : skv <= 2048 && 8 * hq <= dev->compute_units ? 1 : 2;
+}
+
+// Parts of the keys: 16 of a long cache where the workgroups of two heads then find a compute unit each (64 / 8 heads, 4000 keys 14.7 us with 16, 11.7 with 8).
+static int ad_parts(const fh_device *dev, int hq, int skv) {
+    if (dev->opt_attn_splits > 0) return dev->opt_attn_splits > 128 ? 128 : (int)dev->opt_attn_splits;
+    return skv <= 2048 || 8 * hq > dev->compute_units ? 8 : 16;
+}
+
 // One f32 query per head against `skv` cached keys known on the host; `out` is f32 or f16 [hq, d].  The key
 // range is cut into more parts the longer it is (every part is a workgroup per KV head and query-head group).
 fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *q, bool q_f16, const void *k,
@@ -670,12 +683,8 @@ fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *
         }
     }
     if (q_f16 && (dev->opt_attn_kernel == 4 || (dev->opt_attn_heads > 4))) return FH_ERR_UNSUPPORTED; // caller widens q
-    int splits = skv <= 2048 ? 8 : 16;
-    if (dev->opt_attn_splits > 0) splits = dev->opt_attn_splits > 128 ? 128 : (int)dev->opt_attn_splits;
-    // long caches are bandwidth bound: all query heads of a KV head in one workgroup, so K and V are read once
-    // (measured on MI355X, 32 / 8 heads, f16 cache: 1 head x 8 parts x 16 wavefronts at 1024 keys, 2 x 16 x 8 at
-    // 4096 and 16384)
-    const int heads = dev->opt_attn_heads > 0 ? (int)dev->opt_attn_heads : (skv <= 2048 ? 1 : 2);
+    const int splits = ad_parts(dev, hq, skv);
+    const int heads = ad_heads(dev, hq, skv);
     return ad_any(dev, kv_dtype, (const float *)q, k, v, kv_sh, kv_st, hq, hkv, d, scale, nullptr, skv, (float *)out, nullptr,
                   skv - 1, splits, out_f16, heads, skv > 2048 ? 8 : 0, q_f16);
 }
@@ -714,15 +723,14 @@ extern "C" fh_status fh_flash_attention_decode_static(fh_device *dev, int32_t q_
         FH_FAIL(FH_ERR_UNSUPPORTED, "the allocation-free decode attention needs head_dim 128 and K / V strides that are "
                                     "multiples of 8 elements (got d = %d, strides %lld, %lld)", d, (long long)kv_sh,
                 (long long)kv_st);
-    // the same cut of the key range as fh_flash_attention makes for one query position
-    int splits = skv <= 2048 ? 8 : 16;
-    if (dev->opt_attn_splits > 0) splits = dev->opt_attn_splits > 128 ? 128 : (int)dev->opt_attn_splits;
-    const size_t need = (size_t)hq * splits * (128 + 4) * 4;
+    // the same cut of the key range as fh_flash_attention makes for one query position; room is asked for 16 parts of more than 2048 keys however many there are
+    const int splits = ad_parts(dev, hq, skv), room = dev->opt_attn_splits > 0 ? splits : skv <= 2048 ? 8 : 16;
+    const size_t need = (size_t)hq * room * (128 + 4) * 4;
     if (need > dev->static_scratch_bytes)
         FH_FAIL(FH_ERR_INVALID, "%d query heads x %d key parts need %zu bytes of partial results; the static scratch "
-                                "holds %zu (at most 64 heads x 16 parts): use fh_flash_attention", hq, splits, need,
+                                "holds %zu (at most 64 heads x 16 parts): use fh_flash_attention", hq, room, need,
                 dev->static_scratch_bytes);
-    const int heads = dev->opt_attn_heads > 0 ? (int)dev->opt_attn_heads : (skv <= 2048 ? 1 : 2);
+    const int heads = ad_heads(dev, hq, skv);
     // Every (head, part) slot the merge reads is written by this call's first kernel, parts without keys
     // included, so nothing has to be cleared between calls.
     return ad_any(dev, kv_dtype, (const float *)q_dev, k_dev, v_dev, kv_sh, kv_st, hq, hkv, d, scale, nullptr, skv,

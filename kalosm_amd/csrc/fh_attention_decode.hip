@@ -656,6 +656,15 @@ static int ad_parts(const fh_device *dev, int hq, int skv) {
     return skv <= 2048 || 8 * hq > dev->compute_units ? 8 : 16;
 }
 
+// Room for the partial results of `splits` parts.  When it has to grow it grows to what a cache of any length needs, so that a call that is captured
+// finds it whatever number of keys the calls before it had.
+static fh_status ad_room(fh_device *dev, int hq, int hkv, int splits) {
+    const size_t part = (size_t)hq * (128 + 4) * 4;
+    if (hkv < 1 || dev->part_cap >= part * splits) return FH_OK;
+    const int most = std::max(splits, std::min(128, std::max(16, 2 * dev->compute_units / hkv)));
+    return fh_dev_scratch(dev, (void **)&dev->part_buf, &dev->part_cap, part * most);
+}
+
 // One f32 query per head against `skv` cached keys known on the host; `out` is f32 or f16 [hq, d].  The key
 // range is cut into more parts the longer it is (every part is a workgroup per KV head and query-head group).
 fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *q, bool q_f16, const void *k,
@@ -675,7 +684,7 @@ fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *
         splits = std::min(splits, nct / 2);
         if (dev->opt_attn_splits > 0) splits = (int)dev->opt_attn_splits;
         splits = splits < 1 ? 1 : (splits > 128 ? 128 : splits);
-        FH_TRY(fh_dev_scratch(dev, (void **)&dev->part_buf, &dev->part_cap, (size_t)hq * splits * (128 + 4) * 4));
+        FH_TRY(ad_room(dev, hq, hkv, splits));
         fh_status st = fh_attention_decode_mfma(dev, q, q_f16, k, v, kv_sh, kv_st, hq, hkv, d, scale, skv, splits, dev->part_buf);
         if (st != FH_ERR_UNSUPPORTED) {
             if (st != FH_OK) return st;
@@ -685,6 +694,7 @@ fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *
     if (q_f16 && (dev->opt_attn_kernel == 4 || (dev->opt_attn_heads > 4))) return FH_ERR_UNSUPPORTED; // caller widens q
     const int splits = ad_parts(dev, hq, skv);
     const int heads = ad_heads(dev, hq, skv);
+    if (d == 128 && hq >= hkv && kv_st % 8 == 0 && kv_sh % 8 == 0) FH_TRY(ad_room(dev, hq, hkv, splits)); // (what ad_any takes)
     return ad_any(dev, kv_dtype, (const float *)q, k, v, kv_sh, kv_st, hq, hkv, d, scale, nullptr, skv, (float *)out, nullptr,
                   skv - 1, splits, out_f16, heads, skv > 2048 ? 8 : 0, q_f16);
 }

@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from kalosm_amd.fusor import Tensor
+from kalosm_amd.fusor import Device, Tensor
 
 pytestmark = pytest.mark.gpu
 
@@ -28,3 +28,28 @@ def test_parts_of_the_keys_match_oracle(dev, oracle, hq, hkv, L):
         dev.set_option("attn_kernel", 0)
     # weights and outputs are rounded to f16: 2^-11 of each weight, in all at most 2^-11 of the largest |v|, and 2^-11 of an output
     assert (np.abs(got - ref) <= 2.0 ** -11 * (np.abs(v.astype(np.float32)).max() + np.abs(ref)) + 1e-6).all()
+
+
+def test_long_caches_captured_after_a_short_one():
+    """The room for parts that a call of 100 keys leaves behind is enough for a captured one of 4096, of twice as many parts as before, and of 16384."""
+    dev = Device.gpu(0)
+    try:
+        rng = np.random.default_rng(5)
+        q = Tensor.from_slice(dev, rng.standard_normal((1, 32, 1, 128)).astype(np.float16), "f16")
+        for L in (100, 4096, 16384):
+            k, v = (Tensor.from_slice(dev, rng.standard_normal((1, 8, L, 128)).astype(np.float16), "f16") for _ in range(2))
+            out = Tensor(dev, (1, 32, 1, 128), "f16")
+            if L > 100:
+                dev.graph_begin()
+            q.flash_attention(k, v, 0.1, out=out)
+            if L > 100:
+                graph = dev.graph_end()
+                got = []
+                for _ in range(3):
+                    graph.launch()
+                    got.append(out.as_slice().view(np.uint16).copy())
+                q.flash_attention(k, v, 0.1, out=out)
+                assert all(np.array_equal(g, out.as_slice().view(np.uint16)) for g in got)
+                del graph
+    finally:
+        dev.close()

@@ -370,6 +370,7 @@ __global__ __launch_bounds__(512) void k_step_out(FhStep st) {
         }
     __builtin_amdgcn_sched_barrier(0);
     if (tid < n_e) who[tid] = expert;
+    for (int i = tid + 512; i < n_e; i += 512) who[i] = st.ids[i]; // (a token has as many as there are, up to 1024)
     auto put = [&](int i, float4 v, float w) {
         const int c = i % m.ffp;
         v.x = c < m.ff ? w * v.x : 0.f, v.y = c + 1 < m.ff ? w * v.y : 0.f, v.z = c + 2 < m.ff ? w * v.z : 0.f, v.w = c + 3 < m.ff ? w * v.w : 0.f;

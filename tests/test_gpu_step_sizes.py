@@ -40,3 +40,11 @@ def test_sizes(dev, width, mixer, mlp):
     w = G.weights(cfg)
     toks = np.random.default_rng(width).integers(0, 50, 8)
     close(run_portions(G.build(dev, cfg, w), toks, [1]), R.forward(cfg, w, toks)[0], TOL["float32"])
+
+
+def test_more_chosen_experts_than_threads(dev):
+    """520 experts a token: a workgroup of the output launch has 512 threads, and its table of the chosen ones is read whole."""
+    cfg = G.config([G.with_mlp(latent(2), G.moe(530, 520, 16, 0))], 64, 50)
+    w = G.weights(cfg)
+    toks = np.random.default_rng(1).integers(0, 50, 4)
+    close(run_portions(G.build(dev, cfg, w), toks, [1]), R.forward(cfg, w, toks)[0], TOL["float32"])

@@ -656,13 +656,19 @@ static int ad_parts(const fh_device *dev, int hq, int skv) {
     return skv <= 2048 || 8 * hq > dev->compute_units ? 8 : 16;
 }
 
-// Room for the partial results of `splits` parts.  When it has to grow it grows to what a cache of any length needs, so that a call that is captured
-// finds it whatever number of keys the calls before it had.
-static fh_status ad_room(fh_device *dev, int hq, int hkv, int splits) {
+// Room for the partial results of `splits` parts.  When it has to grow it grows to what a cache of any length needs, so that the graphs that hold its address
+// end once and not at every other length.  It belongs to the device, and calls of other numbers of heads leave it as they need it, so a captured call, which
+// cannot grow it, takes as many parts as it has room for.
+static fh_status ad_room(fh_device *dev, int hq, int hkv, int *splits) {
     const size_t part = (size_t)hq * (128 + 4) * 4;
-    if (hkv < 1 || dev->part_cap >= part * splits) return FH_OK;
-    const int most = std::max(splits, std::min(128, std::max(16, 2 * dev->compute_units / hkv)));
-    return fh_dev_scratch(dev, (void **)&dev->part_buf, &dev->part_cap, part * most);
+    if (hkv < 1 || dev->part_cap >= part * *splits) return FH_OK;
+    if (dev->capturing) {
+        if (dev->part_cap >= part && dev->opt_attn_splits == 0) *splits = (int)(dev->part_cap / part);
+    } else {
+        const int most = std::max(*splits, std::min(128, std::max(16, 2 * dev->compute_units / hkv)));
+        return fh_dev_scratch(dev, (void **)&dev->part_buf, &dev->part_cap, part * most);
+    }
+    return fh_dev_scratch(dev, (void **)&dev->part_buf, &dev->part_cap, part * *splits);
 }
 
 // One f32 query per head against `skv` cached keys known on the host; `out` is f32 or f16 [hq, d].  The key
@@ -684,7 +690,7 @@ fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *
         splits = std::min(splits, nct / 2);
         if (dev->opt_attn_splits > 0) splits = (int)dev->opt_attn_splits;
         splits = splits < 1 ? 1 : (splits > 128 ? 128 : splits);
-        FH_TRY(ad_room(dev, hq, hkv, splits));
+        FH_TRY(ad_room(dev, hq, hkv, &splits));
         fh_status st = fh_attention_decode_mfma(dev, q, q_f16, k, v, kv_sh, kv_st, hq, hkv, d, scale, skv, splits, dev->part_buf);
         if (st != FH_ERR_UNSUPPORTED) {
             if (st != FH_OK) return st;
@@ -692,9 +698,9 @@ fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *
         }
     }
     if (q_f16 && (dev->opt_attn_kernel == 4 || (dev->opt_attn_heads > 4))) return FH_ERR_UNSUPPORTED; // caller widens q
-    const int splits = ad_parts(dev, hq, skv);
+    int splits = ad_parts(dev, hq, skv);
     const int heads = ad_heads(dev, hq, skv);
-    if (d == 128 && hq >= hkv && kv_st % 8 == 0 && kv_sh % 8 == 0) FH_TRY(ad_room(dev, hq, hkv, splits)); // (what ad_any takes)
+    if (d == 128 && hq >= hkv && kv_st % 8 == 0 && kv_sh % 8 == 0) FH_TRY(ad_room(dev, hq, hkv, &splits)); // (what ad_any takes)
     return ad_any(dev, kv_dtype, (const float *)q, k, v, kv_sh, kv_st, hq, hkv, d, scale, nullptr, skv, (float *)out, nullptr,
                   skv - 1, splits, out_f16, heads, skv > 2048 ? 8 : 0, q_f16);
 }

@@ -53,3 +53,39 @@ def test_long_caches_captured_after_a_short_one():
                 del graph
     finally:
         dev.close()
+
+
+def test_captured_beside_calls_of_other_heads(oracle):
+    """The room belongs to the device: calls of eight heads leave it so that one of 32 heads and few keys fits and one of 4096 keys has fewer parts than it would take."""
+    dev = Device.gpu(0)
+    try:
+        rng = np.random.default_rng(6)
+
+        def inputs(hq, L):
+            return [rng.standard_normal((1, h, n, 128)).astype(np.float16) for h, n in ((hq, 1), (8, L), (8, L))]
+
+        def put(a):
+            return [Tensor.from_slice(dev, t, "f16") for t in a]
+
+        for hq, L in ((8, 4096), (32, 100), (32, 3000)):
+            q, k, v = put(inputs(hq, L))
+            q.flash_attention(k, v, 0.1)
+        for L in (4096, 16384):
+            a = inputs(32, L)
+            q, k, v = put(a)
+            out = Tensor(dev, (1, 32, 1, 128), "f16")
+            dev.graph_begin()
+            q.flash_attention(k, v, 0.1, out=out)
+            graph = dev.graph_end()
+            got = []
+            for _ in range(3):
+                graph.launch()
+                got.append(out.as_slice())
+            a = [t.astype(np.float32) for t in a]
+            want = oracle.flash_attention(*a, 0.1)
+            # (weights and outputs are rounded to f16, as above)
+            assert (np.abs(got[0].astype(np.float32) - want) <= 2.0 ** -11 * (np.abs(a[2]).max() + np.abs(want)) + 1e-6).all()
+            assert all(np.array_equal(g.view(np.uint16), got[0].view(np.uint16)) for g in got)
+            del graph
+    finally:
+        dev.close()

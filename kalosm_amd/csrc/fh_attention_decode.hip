@@ -657,8 +657,8 @@ static int ad_parts(const fh_device *dev, int hq, int skv) {
 }
 
 // Room for the partial results of `splits` parts.  When it has to grow it grows to what a cache of any length needs, so that the graphs that hold its address
-// end once and not at every other length.  It belongs to the device, and calls of other numbers of heads leave it as they need it, so a captured call, which
-// cannot grow it, takes as many parts as it has room for.
+// end once and not at every other length; where that much cannot be had, to what this call needs.  It belongs to the device, and calls of other numbers of heads
+// leave it as they need it, so a captured call, which cannot grow it, takes as many parts as it has room for.
 static fh_status ad_room(fh_device *dev, int hq, int hkv, int *splits) {
     const size_t part = (size_t)hq * (128 + 4) * 4;
     if (hkv < 1 || dev->part_cap >= part * *splits) return FH_OK;
@@ -666,7 +666,7 @@ static fh_status ad_room(fh_device *dev, int hq, int hkv, int *splits) {
         if (dev->part_cap >= part && dev->opt_attn_splits == 0) *splits = (int)(dev->part_cap / part);
     } else {
         const int most = std::max(*splits, std::min(128, std::max(16, 2 * dev->compute_units / hkv)));
-        return fh_dev_scratch(dev, (void **)&dev->part_buf, &dev->part_cap, part * most);
+        if (fh_dev_scratch_try(dev, (void **)&dev->part_buf, &dev->part_cap, part * most)) return FH_OK;
     }
     return fh_dev_scratch(dev, (void **)&dev->part_buf, &dev->part_cap, part * *splits);
 }

@@ -89,3 +89,19 @@ def test_captured_beside_calls_of_other_heads(oracle):
             del graph
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("dtype,L", [("f16", 100), ("f32", 100), ("f16", 4096)])
+def test_scratch_limit_that_the_call_keeps(oracle, dtype, L):
+    """A call whose own parts fit the limit does not fail because those of longer caches would not."""
+    dev = Device.gpu(0)
+    try:
+        dev.set_option("scratch_limit", 32 * 32 * 132 * 4)  # the 32 parts of 4096 keys; a cache of any length may take 64
+        rng = np.random.default_rng(7)
+        a = [rng.standard_normal((1, h, n, 128)).astype(np.float16) for h, n in ((32, 1), (8, L), (8, L))]
+        got = Tensor.from_slice(dev, a[0], dtype).flash_attention(*(Tensor.from_slice(dev, t, dtype) for t in a[1:]), 0.1).as_slice().astype(np.float32)
+        a = [t.astype(np.float32) for t in a]
+        want = oracle.flash_attention(*a, 0.1)
+        assert (np.abs(got - want) <= 2.0 ** -11 * (np.abs(a[2]).max() + np.abs(want)) + 1e-6).all()
+    finally:
+        dev.close()

@@ -150,18 +150,19 @@ struct FhRowDeal {
         float acc = 0.f;
         int p = 0, i = 0;
         const int total = count * pieces;
+        const bool past = (pieces - 1) * 512 + lane8 >= kp; // of a row's last piece this lane has its last eight values again, which may be infinite: not used
         for (int t = 0; t < total; t += AHEAD) {
 #pragma unroll
             for (int s = 0; s < AHEAD; s++) {
                 const float *at = x.xs + p * 256 + (lane8 >> 1);
                 const float4 a = *(const float4 *)at, b = *(const float4 *)(at + x.plane);
-                acc = fh_dot8(u[s], a, b, acc);
+                const float more = fh_dot8(u[s], a, b, acc);
                 fetch(s);
                 if (++p == pieces) {
-                    acc = fh_wave_sum(acc);
+                    acc = fh_wave_sum(past ? acc : more);
                     if (i < count) done(i, acc); // (what is behind the last row is the last piece again)
                     acc = 0.f, p = 0, i++;
-                }
+                } else acc = more;
             }
         }
     }

@@ -56,3 +56,17 @@ def test_decode_step(dev, width, ff):
     w = G.weights(cfg)
     toks = np.random.default_rng(ff).integers(0, 50, 12)
     close(run_portions(G.build(dev, cfg, w), toks, [1]), R.forward(cfg, w, toks)[0], TOL["float32"])
+
+
+@pytest.mark.parametrize("k", [64, 2112, 11008])
+@pytest.mark.parametrize("n", [9, 5000])
+def test_infinite_weights(dev, n, k):
+    """An infinity among the last stored weights of a row that does not fill whole pieces of 512 gives an infinity: lanes past the row multiply nothing."""
+    rng = np.random.default_rng(k)
+    w = synth.to_bf16_bits(rng.standard_normal(n * k, dtype=np.float32)).reshape(n, k)
+    w[2, k - 1], w[3, k - 8], w[4, 0] = 0x7F80, 0xFF80, 0x7F80
+    x = np.abs(rng.standard_normal((1, k), dtype=np.float32))
+    got = Tensor.from_slice(dev, x).q_mat_mul(QMatrix.from_raw_bytes(dev, (n, k), w, synth.W_BF16)).as_slice()[0]
+    assert got[2] == np.inf and got[3] == -np.inf and got[4] == np.inf
+    rest = [i for i in range(n) if i not in (2, 3, 4)]
+    near(got[rest].astype(np.float64), synth.from_bf16_bits(w[rest]).astype(np.float64) @ x[0].astype(np.float64))

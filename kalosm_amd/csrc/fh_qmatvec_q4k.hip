@@ -70,7 +70,7 @@ struct Q4kExtra {
 // i / (16 / RS) in the steps of accumulator a = 0 .. RS - 1.  The accumulator entries whose row and column name the
 // same block are the dots; the rest is discarded.  As many MFMAs per weight byte as with whole tiles, RS times the
 // workgroups: matrices with fewer row tiles than compute units fill the device in one launch.
-// RAG: the blocks are no multiple of the wavefronts'; what a wavefront has past the last one is the last one again, times zero.
+// RAG: the blocks are no multiple of the wavefronts'; what a wavefront has past the last one is the last one's codes again, activations and scales zero.
 template <int FMT, int TPW, int PER, int EPI, int IN, int MR = 1, int RS = 1, bool RAG = false, bool ONCE = false>
 __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict__ x, float *__restrict__ y,
                                                       const float *__restrict__ ea, const float *__restrict__ eb,
@@ -523,7 +523,8 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
                 }
     #pragma unroll
                 for (int tp = 0; tp < TPW; tp++) {
-                    const uint4 h = w[tp][r].h;
+                    uint4 h = w[tp][r].h;
+                    if (RAG && r > last) h.x = 0; // (infinite scales would make NaN of the zeros)
                     if (Q40 || FMT == FH_Q8_0) {
                         const float off = FMT == FH_Q8_0 ? 1152.0f : (FMT == FH_Q5_0 ? 16.0f : 8.0f);
                         const float da = fh_h2f((uint16_t)(h.x & 0xFFFF)), db = fh_h2f((uint16_t)(h.x >> 16));

@@ -27,7 +27,7 @@ struct Q6KRegs {
 // Workgroup = SW wavefronts, one per k-slice of PER blocks; a wavefront multiplies its slice of TPW row tiles (with
 // the SwiGLU epilogue: gate tiles and the matching up tiles), stages the activations of its own blocks only (no
 // barrier before the products) and requests all its weight bytes before anything else.
-// RAG: the blocks are no multiple of the wavefronts'; what a wavefront has past the last one is the last one again, times zero.
+// RAG: the blocks are no multiple of the wavefronts'; what a wavefront has past the last one is the last one's codes again, activations and scales zero.
 template <int TPW, int PER, int EPI, bool RAG, bool ONCE>
 __global__ __launch_bounds__(1024) void k_qmv_q6k_m1(const uint8_t *data, const float *__restrict__ x, const float *__restrict__ xup, int recs, int n, int k, int SW,
                                                       float *__restrict__ y, const float *__restrict__ ea, const float *__restrict__ eb) {
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(1024) void k_qmv_q6k_m1(const uint8_t *data, const 
         const float2 f0 = *(const float2 *)(psf + r * Q6K_SF + 16), f1 = *(const float2 *)(psf + r * Q6K_SF + 24);
 #pragma unroll
         for (int tp = 0; tp < TPW; tp++) {
-            const float d = fh_h2f(w[tp][r].d);
+            const float d = RAG && r > last ? 0.f : fh_h2f(w[tp][r].d); // (an infinite scale would make NaN of the zeros)
             const int scw = (int)w[tp][r].sc;
             const float s0 = (float)((scw << 24) >> 24), s1 = (float)((scw << 16) >> 24),
                         s2 = (float)((scw << 8) >> 24), s3 = (float)(scw >> 24);

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from kalosm_amd import synth
-from kalosm_amd.fusor import Tensor
+from kalosm_amd.fusor import QMatrix, Tensor
 from test_gpu_qmv_rows import close, matrix, named
 
 pytestmark = pytest.mark.gpu
@@ -33,3 +33,35 @@ def test_few_rows_of_five_bits(dev, oracle, ty, m, n, k):
     q, w = matrix(dev, oracle, ty, n, k)
     x = synth.random_activation(m, k, seed=2) * np.exp(np.random.default_rng(3).standard_normal((m, 1))).astype(np.float32)
     close(Tensor.from_slice(dev, x).q_mat_mul(q).as_slice().astype(np.float64), x, w)
+
+
+def alternating(ty, raw, n, k, row, bits):
+    """`raw` with scale `bits` and its largest and smallest codes in turn (scales of one, offsets of none) in the last block of a row."""
+    per, size = k // synth.BLOCK_ELEMS[ty], synth.BLOCK_BYTES[ty]
+    out = raw.copy().reshape(n, per, size)
+    block = out[row, -1]
+    codes = np.tile(np.array([0xFF, 0], np.uint8), 100)
+    if ty == synth.Q6_K:
+        block[0:192], block[192:208] = codes[:192], 1
+        block[208:210] = np.array([bits], np.uint16).view(np.uint8)
+    else:
+        block[0:2] = np.array([bits], np.uint16).view(np.uint8)
+        if ty == synth.Q4_K:
+            block[2:4], block[4:16] = 0, synth.pack_k4_scales(np.ones(8), np.zeros(8))
+        block[size - (16 if ty == synth.Q4_0 else 128):] = codes[:16 if ty == synth.Q4_0 else 128]
+    return out.reshape(-1)
+
+
+@pytest.mark.parametrize("ty", [synth.Q4_0, synth.Q4_K, synth.Q6_K], ids=lambda t: synth.TYPE_NAMES[t])
+@pytest.mark.parametrize("blocks", [17, 31, 43])
+def test_infinite_scale_of_the_last_block(dev, ty, blocks):
+    """A wavefront with fewer blocks than others multiplies the last one again by nothing: an infinite scale there gives the infinity that it stands for."""
+    n, k = 48, 256 * blocks
+    raw = synth.random_weight(ty, n, k, seed=1)
+    x = synth.random_activation(1, k, seed=2)
+    x[0, -256:] = np.tile(np.array([-1.0, 1.5], np.float32), 128)  # large codes meet the negative ones, the sum is positive
+    t = Tensor.from_slice(dev, x)
+    got, want = (t.q_mat_mul(QMatrix.from_raw_bytes(dev, (n, k), alternating(ty, raw, n, k, 5, bits), ty)).as_slice()[0] for bits in (0x7C00, 0x3C00))
+    assert got[5] == -np.inf
+    got[5] = want[5]
+    assert np.array_equal(got, want)

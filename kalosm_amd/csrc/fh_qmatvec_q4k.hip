@@ -277,7 +277,9 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
         const int half = Q40 ? (lane >> 2) & 1 : lane & 1;
         // e = 14 - floor(log2(amax)) from the exponent field (zero / subnormal / inf / nan just clamp)
         int e = 141 - (int)((am >> 23) & 0xFFu);
-        e = e > 100 ? 100 : (e < -100 ? -100 : e);
+        // (ragged rows: high nibbles lose four bits of scale below, and the batch kernel that would take them loses none down to 2^-86)
+        constexpr int MOST = RAG ? 125 : 100;
+        e = e > MOST ? MOST : (e < -100 ? -100 : e);
         const int eo = e - (FMT == FH_Q8_0 ? 0 : 4 * (Q40 ? half : s & 1)); // high nibbles: codes x 16
         const float sc = __uint_as_float((uint32_t)(eo + 127) << 23);
         // hi = f16(x * sc), lo = f16(x * sc - hi) (x * sc is exact, a power of two, so the fused form rounds once),

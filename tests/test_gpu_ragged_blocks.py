@@ -65,3 +65,17 @@ def test_infinite_scale_of_the_last_block(dev, ty, blocks):
     assert got[5] == -np.inf
     got[5] = want[5]
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("ty", [synth.Q4_0, synth.Q4_K], ids=lambda t: synth.TYPE_NAMES[t])
+def test_tiny_activations_of_one_row(dev, ty):
+    """Down to 2^-113 a power of two more or less in the activations changes nothing but the results' exponents: 22 bits of each are there."""
+    n, k = 48, 256 * 43
+    q = QMatrix.from_raw_bytes(dev, (n, k), synth.random_weight(ty, n, k, seed=1), ty)
+    x = synth.random_activation(1, k, seed=2)
+    want = Tensor.from_slice(dev, x).q_mat_mul(q).as_slice().astype(np.float64)
+    rms = np.sqrt((want ** 2).mean())
+    for e in (-60, -90, -113):
+        got = Tensor.from_slice(dev, np.ldexp(x, e)).q_mat_mul(q).as_slice().astype(np.float64)
+        # the products are exact and the sums the same; a bit that leaves a low term is 2^-22 of an activation
+        assert np.sqrt(((np.ldexp(got, -e) - want) ** 2).mean()) <= 2.0 ** -22 * rms, e

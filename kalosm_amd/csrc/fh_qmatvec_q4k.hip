@@ -82,7 +82,7 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
     static_assert(RS == 1 || (FMT == FH_Q4_K && TPW == 1 && MR == 1 && IN == 0 && (EPI == FH_EPI_NONE || EPI == FH_EPI_ADD2)),
                   "row split: Q4_K, one tile part, one row, plain input, epilogues none / add2");
     static_assert(RS == 1 || RS == 2 || RS == 4, "row split");
-    static_assert(!RAG || (IN == 0 && TPW == 1 && MR == 1 && RS == 1 && EPI != FH_EPI_SWIGLU), "ragged: plain input, one tile, one row");
+    static_assert(!RAG || ((FMT == FH_Q4_K || FMT == FH_Q4_0) && IN == 0 && TPW == 1 && MR == 1 && RS == 1 && EPI != FH_EPI_SWIGLU), "ragged: Q4_K or Q4_0, plain input, one tile, one row");
     constexpr int NB = PER * RS; // blocks a wavefront stages and multiplies
     // SwiGLU with one tile per wavefront: the "tile" is rows 8h .. 8h+7 of a gate tile (columns 0-7 of the MFMA) and
     // the same rows of the matching up tile (columns 8-15), h = workgroup parity: workgroups half as heavy as with a
@@ -194,16 +194,16 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
 #pragma unroll
         for (int tp = 0; tp < TPW; tp++) {
             if constexpr (FMT == FH_Q5_0) { // the Q4_0 records, each followed by the lane's fifth bits (one byte per block)
-                w[tp][r].h.x = fh_ld_weights<ONCE, uint32_t>(ph[tp] + blk(r) * CHUNK);
-                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * CHUNK);
-                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * CHUNK + REC);
-                w[tp][r].qc.x = fh_ld_weights<ONCE, uint32_t>(pq[tp] + 1152 - 12 * lane + blk(r) * CHUNK);
-                w[tp][r].qc.y = fh_ld_weights<ONCE, uint32_t>(pq[tp] + 1152 - 12 * lane + blk(r) * CHUNK + REC);
+                w[tp][r].h.x = fh_ld_weights<ONCE, uint32_t>(ph[tp] + r * CHUNK);
+                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + r * CHUNK);
+                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + r * CHUNK + REC);
+                w[tp][r].qc.x = fh_ld_weights<ONCE, uint32_t>(pq[tp] + 1152 - 12 * lane + r * CHUNK);
+                w[tp][r].qc.y = fh_ld_weights<ONCE, uint32_t>(pq[tp] + 1152 - 12 * lane + r * CHUNK + REC);
             } else if constexpr (FMT == FH_Q5_K) { // the Q4_K record followed by the lane's eight qh bytes
-                w[tp][r].h = fh_ld_weights<ONCE, uint4>(ph[tp] + blk(r) * CHUNK);
-                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * CHUNK);
-                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * CHUNK + 1024);
-                const uint2 hb = fh_ld_weights<ONCE, uint2>(pq[tp] + 2048 - 8 * lane + blk(r) * CHUNK);
+                w[tp][r].h = fh_ld_weights<ONCE, uint4>(ph[tp] + r * CHUNK);
+                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + r * CHUNK);
+                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + r * CHUNK + 1024);
+                const uint2 hb = fh_ld_weights<ONCE, uint2>(pq[tp] + 2048 - 8 * lane + r * CHUNK);
                 w[tp][r].qc.x = hb.x;
                 w[tp][r].qc.y = hb.y;
             } else if (FMT == FH_Q4_0) {
@@ -211,11 +211,11 @@ __device__ __forceinline__ void qmv_q4k_m1_body(QView q, const float *__restrict
                 w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 2304);
                 w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 2304 + 1152);
             } else if (FMT == FH_Q8_0) {
-                w[tp][r].h.x = fh_ld_weights<ONCE, uint32_t>(ph[tp] + blk(r) * 4352);
-                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 4352);
-                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 4352 + 1088);
-                w[tp][r].qc = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 4352 + 2176);
-                w[tp][r].qd = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * 4352 + 3264);
+                w[tp][r].h.x = fh_ld_weights<ONCE, uint32_t>(ph[tp] + r * 4352);
+                w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + r * 4352);
+                w[tp][r].qb = fh_ld_weights<ONCE, uint4>(pq[tp] + r * 4352 + 1088);
+                w[tp][r].qc = fh_ld_weights<ONCE, uint4>(pq[tp] + r * 4352 + 2176);
+                w[tp][r].qd = fh_ld_weights<ONCE, uint4>(pq[tp] + r * 4352 + 3264);
             } else {
                 w[tp][r].h = fh_ld_weights<ONCE, uint4>(ph[tp] + blk(r) * RS * 2304);
                 w[tp][r].qa = fh_ld_weights<ONCE, uint4>(pq[tp] + blk(r) * RS * 2304);
@@ -679,20 +679,13 @@ static fh_status q4k_m1_rag_go(const fh_qmatrix *q, const float *x, float *y, in
     return q4k_m1_start(kern, q, dim3((unsigned)((q->n + 15) / 16)), SW, lds, x, y, a, b);
 }
 
-// us of one row of 4096 x 11008 by the kernels that took it (the batch kernel, the 5-bit formats element by element) / here: Q4_K 15.0 / 7.7, Q4_0 15.2 /
-// 7.2, Q8_0 18.4 / 10.8, Q5_0 124 / 9.4, Q5_K 165 / 9.5 (of 4096 x 14336, whose 56 blocks 14 wavefronts share, 9.9 in Q4_K).
+// us of one row of 4096 x 11008 by the batch kernel / here: Q4_K 15.0 / 7.7, Q4_0 15.2 / 7.2 (of 4096 x 14336, whose 56 blocks 14 wavefronts share, 9.9 in
+// Q4_K), and as far from 64 bits (7.7e-7 / 7.6e-7 and 2.2e-6 / 1.7e-6 of the results' size).  The other formats stay where they were: their single-row kernels
+// are quicker too, but further off than what takes these rows (Q8_0 18.4 / 10.8 us, 2.7e-7 / 1.9e-6; Q5_0 124 / 9.4, 2.5e-7 / 8.9e-7; Q5_K 165 / 9.5, 2.3e-7 / 3.9e-7).
 static fh_status q4k_m1_rag(const fh_qmatrix *q, const float *x, float *y, int epi, const float *a, const float *b) {
     const bool two = q->k <= 32 * 256;
-#define RAG_GO(T_) return two ? q4k_m1_rag_go<T_, 2>(q, x, y, epi, a, b) : q4k_m1_rag_go<T_, 4>(q, x, y, epi, a, b)
-    switch (q->type) {
-    case FH_Q4_K: RAG_GO(FH_Q4_K);
-    case FH_Q5_K: RAG_GO(FH_Q5_K);
-    case FH_Q4_0: RAG_GO(FH_Q4_0);
-    case FH_Q5_0: RAG_GO(FH_Q5_0);
-    case FH_Q8_0: RAG_GO(FH_Q8_0);
-    }
-#undef RAG_GO
-    return FH_ERR_UNSUPPORTED;
+    if (q->type == FH_Q4_K) return two ? q4k_m1_rag_go<FH_Q4_K, 2>(q, x, y, epi, a, b) : q4k_m1_rag_go<FH_Q4_K, 4>(q, x, y, epi, a, b);
+    return two ? q4k_m1_rag_go<FH_Q4_0, 2>(q, x, y, epi, a, b) : q4k_m1_rag_go<FH_Q4_0, 4>(q, x, y, epi, a, b);
 }
 
 template <int TPW, int PER, int EPI>
@@ -949,7 +942,7 @@ static fh_status q4k_m1_any(const fh_qmatrix *q, const float *x, const Q4kExtra 
         per *= 2;
     }
     const int SW = kb / per;
-    if (SW > 16 && kb <= 64 && (epi == FH_EPI_NONE || epi == FH_EPI_ADD2) && ex.ksplit == 1 && ex.nsplit == 0 && !ex.nw)
+    if (SW > 16 && kb <= 64 && (q->type == FH_Q4_K || q->type == FH_Q4_0) && (epi == FH_EPI_NONE || epi == FH_EPI_ADD2) && ex.ksplit == 1 && ex.nsplit == 0 && !ex.nw)
         return q4k_m1_rag(q, x, y, epi, a, b);
     if (SW > 16 || kb % per || tpw * per > 4) return FH_ERR_UNSUPPORTED;
     size_t lds = (size_t)kb * Q4K_IMG * 16 + (size_t)kb * 64 + (size_t)tpw * 16 * 64 + 64;

@@ -321,9 +321,13 @@ bool fh_qmv_rows_supports(const fh_qmatrix *q, const float *x, int m) {
 //   wavefront (3 rows of 4096 x 4096 9.8 / 9.5, of 8192 x 3072 12.6 / 13.1).  The 5-bit formats, which have none either and take a launch a row, from 3 rows on where a
 //   launch is more than its own start, that is beyond 2^20 weights: three rows of 4096 x 4096 in Q5_0 11.6 / 9.4 and in Q5_K 11.6 / 10.3, of 14336 x 4096 25.8 / 18.0 and
 //   26.4 / 20.7, four rows 33.8 / 17.8 and 34.6 / 20.8, of 8192 x 3072 17.9 / 12.2 and 18.1 / 13.6 (512 x 2048 9.7 / 6.7, two rows 5.0 / 6.6).
+//   Not where no single-row kernel shares their 256s out: those rows are f32 sums element by element, which take activations of any size as they are (here
+//   those below 2^-86 lose bits: 1.4e-4 of 1e-34).
 bool fh_qmv_rows_pays(const fh_qmatrix *q, const float *x, int m) {
     const bool five = q->type == FH_Q5_0 || q->type == FH_Q5_K;
-    if (!fh_qmv_rows_supports(q, x, m) || m < (q->type == FH_Q6_K || (five && q->n * q->k > 1 << 20) ? 3 : 5)) return false;
+    const int64_t kb = q->k / 256;
+    const bool even = kb <= 16 || (kb <= 32 && kb % 2 == 0) || (kb <= 64 && kb % 4 == 0); // 1, 2 or 4 blocks a wavefront, 16 wavefronts
+    if (!fh_qmv_rows_supports(q, x, m) || m < (q->type == FH_Q6_K || (five && even && q->n * q->k > 1 << 20) ? 3 : 5)) return false;
     const int64_t tiles = (q->n + 15) / 16, cus = q->dev->compute_units;
     if (five && q->n * q->k <= 65536) return false;
     if (q->type == FH_Q4_K && q->k > 1024 && q->k < 2048 && q->n <= 2816) return false;

@@ -1,5 +1,5 @@
-"""GPU parity: one row of k whose 256s no number of up to 16 wavefronts shares out evenly (43 of 11008 columns), and 3 and 4 rows of 5-bit matrices in one
-launch, against 64 bits.
+"""GPU parity: one row of k whose 256s no number of up to 16 wavefronts shares out evenly (43 of 11008 columns), and 3 and 4 rows of 5-bit matrices, in one
+launch (2048 columns) and element by element (11008), against 64 bits.
 
 Bound: as of products of a few rows, but that the kernels of one row multiply f16 subnormals, which lose up to 1.3e-6 of a product."""
 import numpy as np
@@ -97,5 +97,17 @@ def test_formats_that_would_lose_bits(dev, oracle, ty, rows):
     assert np.array_equal(np.ldexp(Tensor.from_slice(dev, np.ldexp(x, -100)).q_mat_mul(q).as_slice(), 100), got)
     x[0, 5] = np.inf
     got = Tensor.from_slice(dev, x).q_mat_mul(q).as_slice()
-    assert np.array_equal(got[0], np.where(w[:, 5] == 0, np.nan, np.sign(w[:, 5]) * np.inf).astype(np.float32), equal_nan=True)
+    assert np.array_equal(got[0], np.where(w[:, 5] == 0, np.nan, np.copysign(np.inf, w[:, 5])).astype(np.float32), equal_nan=True)
     assert np.isfinite(got[1:]).all()
+
+
+@pytest.mark.parametrize("ty", [synth.Q5_0, synth.Q5_K], ids=lambda t: synth.TYPE_NAMES[t])
+@pytest.mark.parametrize("m", [3, 4])
+@pytest.mark.parametrize("blocks", [17, 43, 61, 112])
+def test_few_ragged_rows_of_five_bits(dev, ty, m, blocks):
+    """3 and 4 rows of what the single-row kernel does not share out: f32 values as they are, so powers of two come through."""
+    n, k = 512, 256 * blocks
+    q = QMatrix.from_raw_bytes(dev, (n, k), synth.random_weight(ty, n, k, seed=1), ty)
+    x = synth.random_activation(m, k, seed=2)
+    got = [Tensor.from_slice(dev, np.ldexp(x, e)).q_mat_mul(q).as_slice() for e in (0, -100)]
+    assert np.array_equal(np.ldexp(got[1], 100), got[0])

@@ -643,17 +643,28 @@ fh_status fh_attention_combine_parts(fh_device *dev, const float *part, int hq, 
     return FH_OK;
 }
 
-// Query heads a workgroup.  Long caches are bandwidth bound: two, so that K and V are read less often (32 / 8 heads, f16 cache: 1 head x 8 parts x 16 wavefronts
-// at 1024 keys, 2 x 16 x 8 at 4096).  Short ones: one, unless that makes more workgroups than compute units, which two of sixteen wavefronts fill
-// one after the other (us of 64 / 8 heads, one / two: 300 keys 10.8 / 9.5, 1000 10.8 / 9.5, 2040 11.1 / 9.9; 32 / 8 heads 9.0 / 9.3, 9.0 / 9.4, 8.9 / 9.8).
-static int ad_heads(const fh_device *dev, int hq, int skv) {
-    return dev->opt_attn_heads > 0 ? (int)dev->opt_attn_heads : skv <= 2048 && 8 * hq <= dev->compute_units ? 1 : 2;
+// Query heads a workgroup (one where two do not share a KV head evenly).  Long caches are bandwidth bound: two, so that K and V are read less often.  Short ones: one,
+// unless that makes more workgroups of sixteen wavefronts than compute units, which then take two rounds, and a part is one chunk of a workgroup's rows (128 keys of
+// f32, 256 of f16): us of 64 / 8 heads, one / two: f16 300 keys 10.0 / 8.9, 2040 11.0 / 9.4, f32 300 9.1 / 8.2, 1000 9.7 / 8.5, 1200 13.0 / 15.3, 2040 14.1 / 18.7
+// (34 / 17 heads: f16 10.2 / 9.1, 11.7 / 10.6; f32 8.7 / 8.1, 10.2 / 9.7, 1100 13.5 / 16.3); f16 32 / 8 heads 300 keys 9.0 / 9.3, 2040 8.9 / 9.8.
+static int ad_heads(const fh_device *dev, int hq, int skv, bool f16) {
+    return dev->opt_attn_heads > 0 ? (int)dev->opt_attn_heads : skv <= 2048 && (8 * hq <= dev->compute_units || (!f16 && skv > 1024)) ? 1 : 2;
 }
 
-// Parts of the keys: 16 of a long cache where the workgroups of two heads then find a compute unit each (64 / 8 heads, 4000 keys 14.7 us with 16, 11.7 with 8).
-static int ad_parts(const fh_device *dev, int hq, int skv) {
+// Parts of the keys: 16 of a long cache, 8 of one of more than 32 heads where fewer workgroups are enough, that is
+// - where there are half as many again as compute units (one round instead of two or three): us of f32 48 / 16 heads, 16 parts / 8: 3000 keys 24.6 / 19.8, 16384
+//   119 / 83.7; 56 / 8 heads 18.1 / 16.0 and 83.0 / 62.1; 56 heads of their own 34.2 / 33.4 and 168 / 161; with fewer: 40 heads of their own 26.4 / 29.2 and 123 / 136,
+//   33 / 11 heads 4000 keys 18.0 / 19.8, 40 / 8 18.0 / 20.0;
+// - where two heads share a workgroup: f32 64 / 8 15.9 / 13.3 and 51.2 / 43.5, 34 / 17 19.3 / 15.8 and 70.3 / 59.1, f16 64 / 8 14.9 / 11.5 and 38.5 / 31.6 - but for
+//   fewer than eight KV heads only while the keys are few: f32 36 / 6 heads 3000 keys 14.2 / 12.9, 4000 15.1 / 15.8, 16384 39.7 / 42.7, f16 16384 31.5 / 31.1, 32768 53.7 / 55.1;
+// - f16 below 4096 keys, whose parts are short, where heads share a KV head: 33 / 11 heads 15.8 / 14.4, 36 / 4 14.5 / 14.1 (33 heads of their own 20.1 / 20.8).
+static int ad_parts(const fh_device *dev, int hq, int hkv, int skv, bool f16) {
     if (dev->opt_attn_splits > 0) return dev->opt_attn_splits > 128 ? 128 : (int)dev->opt_attn_splits;
-    return skv <= 2048 || 8 * hq > dev->compute_units ? 8 : 16;
+    if (skv <= 2048) return 8;
+    const int cus = dev->compute_units, group = hq / hkv;
+    if (8 * hq <= cus) return 16;
+    if (group % 2 == 0) return hkv >= 8 || skv <= (f16 ? 16384 : 3072) ? 8 : 16;
+    return 8 * hq >= 3 * cus / 2 || (f16 && group > 1 && skv < 4096) ? 8 : 16;
 }
 
 // Room for the partial results of `splits` parts.  When it has to grow it grows to what a cache of any length needs, so that the graphs that hold its address
@@ -698,8 +709,9 @@ fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *
         }
     }
     if (q_f16 && (dev->opt_attn_kernel == 4 || (dev->opt_attn_heads > 4))) return FH_ERR_UNSUPPORTED; // caller widens q
-    int splits = ad_parts(dev, hq, skv);
-    const int heads = ad_heads(dev, hq, skv);
+    const bool f16 = kv_dtype == FH_F16;
+    int splits = ad_parts(dev, hq, hkv, skv, f16);
+    const int heads = ad_heads(dev, hq, skv, f16);
     if (d == 128 && hq >= hkv && kv_st % 8 == 0 && kv_sh % 8 == 0) FH_TRY(ad_room(dev, hq, hkv, &splits)); // (what ad_any takes)
     return ad_any(dev, kv_dtype, (const float *)q, k, v, kv_sh, kv_st, hq, hkv, d, scale, nullptr, skv, (float *)out, nullptr,
                   skv - 1, splits, out_f16, heads, skv > 2048 ? 8 : 0, q_f16);
@@ -740,13 +752,14 @@ extern "C" fh_status fh_flash_attention_decode_static(fh_device *dev, int32_t q_
                                     "multiples of 8 elements (got d = %d, strides %lld, %lld)", d, (long long)kv_sh,
                 (long long)kv_st);
     // the same cut of the key range as fh_flash_attention makes for one query position; room is asked for 16 parts of more than 2048 keys however many there are
-    const int splits = ad_parts(dev, hq, skv), room = dev->opt_attn_splits > 0 ? splits : skv <= 2048 ? 8 : 16;
+    const bool f16 = kv_dtype == FH_F16;
+    const int splits = ad_parts(dev, hq, hkv, skv, f16), room = dev->opt_attn_splits > 0 ? splits : skv <= 2048 ? 8 : 16;
     const size_t need = (size_t)hq * room * (128 + 4) * 4;
     if (need > dev->static_scratch_bytes)
         FH_FAIL(FH_ERR_INVALID, "%d query heads x %d key parts need %zu bytes of partial results; the static scratch "
                                 "holds %zu (at most 64 heads x 16 parts): use fh_flash_attention", hq, room, need,
                 dev->static_scratch_bytes);
-    const int heads = ad_heads(dev, hq, skv);
+    const int heads = ad_heads(dev, hq, skv, f16);
     // Every (head, part) slot the merge reads is written by this call's first kernel, parts without keys
     // included, so nothing has to be cleared between calls.
     return ad_any(dev, kv_dtype, (const float *)q_dev, k_dev, v_dev, kv_sh, kv_st, hq, hkv, d, scale, nullptr, skv,

@@ -1,4 +1,5 @@
-"""Matrix-core decode attention where the number of parts changes: one workgroup a compute unit, two, fewer parts than that for few keys."""
+"""Decode attention where the number of parts changes: on the matrix cores one workgroup a compute unit, two, fewer parts than that for few keys; without them
+8 or 16, and one or two heads a workgroup, of up to 64 heads."""
 import numpy as np
 import pytest
 
@@ -11,7 +12,7 @@ pytestmark = pytest.mark.gpu
     (64, 64, 1536),    # four parts of twelve chunks: three a wavefront
     (64, 64, 1537),    # one key more: eight parts
     (64, 64, 255),     # fewer chunks than wavefronts
-    (300, 300, 130),   # more heads than compute units: one part
+    (300, 300, 130),   # more than 64 heads: the kernel of any number of them
     (16, 2, 4100),     # as many parts as there are pairs of chunks
 ])
 def test_parts_of_the_keys_match_oracle(dev, oracle, hq, hkv, L):
@@ -105,3 +106,39 @@ def test_scratch_limit_that_the_call_keeps(oracle, dtype, L):
         assert (np.abs(got - want) <= 2.0 ** -11 * (np.abs(a[2]).max() + np.abs(want)) + 1e-6).all()
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,L,parts", [
+    ("f16", 64, 8, 300, 8),     # two heads a workgroup of short caches, one chunk of a part and its end
+    ("f16", 64, 8, 2048, 8),
+    ("f16", 34, 17, 2047, 8),
+    ("f32", 64, 8, 1024, 8),
+    ("f32", 64, 8, 1025, 8),    # one head again
+    ("f32", 40, 40, 2049, 16),  # more workgroups than compute units, but fewer than half as many again
+    ("f32", 48, 16, 2049, 8),   # not fewer
+    ("f32", 40, 8, 4000, 16),
+    ("f32", 64, 8, 4000, 8),    # two heads a workgroup
+    ("f32", 36, 6, 3072, 8),    # of few KV heads, while the keys are few
+    ("f32", 36, 6, 3073, 16),
+    ("f16", 33, 11, 4095, 8),
+    ("f16", 33, 33, 4095, 16),
+    ("f32", 32, 8, 2049, 16),
+])
+def test_heads_and_parts_without_matrix_cores(dev, oracle, dtype, hq, hkv, L, parts):
+    rng = np.random.default_rng(L)
+    a = [rng.standard_normal((1, h, n, 128)).astype(np.float16 if dtype == "f16" else np.float32) for h, n in ((hq, 1), (hkv, L), (hkv, L))]
+    q, k, v = (Tensor.from_slice(dev, t, dtype) for t in a)
+    auto = q.flash_attention(k, v, 0.1).as_slice()
+    same = []
+    for forced in (8, 16):  # another number of parts rounds the sums elsewhere
+        dev.set_option("attn_splits", forced)
+        try:
+            same.append(np.array_equal(q.flash_attention(k, v, 0.1).as_slice(), auto))
+        finally:
+            dev.set_option("attn_splits", 0)
+    assert same[parts == 16] and (dtype == "f16" or not same[parts != 16])
+    a = [t.astype(np.float32) for t in a]
+    want = oracle.flash_attention(*a, 0.1)
+    # f32 sums of the weighted values, a lane's chain of a few hundred; of f16 the outputs are rounded
+    bound = 2.0 ** -17 * np.abs(a[2]).max() + (2.0 ** -11 * np.abs(want) if dtype == "f16" else 0)
+    assert (np.abs(auto.astype(np.float32) - want) <= bound).all()

@@ -302,10 +302,10 @@ __device__ __forceinline__ float ad_rows_max(float a) {
 // arithmetic of one wavefront runs under the transfers of the others.  Lane groups and wavefronts are merged at
 // the end.  Partials as k_attn_decode_dl writes them: [head][part][D weighted sums | max | denominator | 2 unused].
 template <typename TKV, int G, int NWV>
-__global__ __launch_bounds__(64 * NWV) void k_attn_decode_1p(const void *__restrict__ qv, int q_f16, const TKV *__restrict__ k,
-                                                              const TKV *__restrict__ v, int64_t kv_sh, int64_t kv_st,
-                                                              const int *__restrict__ len_dev, int len_host, float scale,
-                                                              int cap, int gtot, float *__restrict__ part) {
+__device__ __forceinline__ void attn_decode_1p(const void *__restrict__ qv, int q_f16, const TKV *__restrict__ k,
+                                               const TKV *__restrict__ v, int64_t kv_sh, int64_t kv_st,
+                                               const int *__restrict__ len_dev, int len_host, float scale,
+                                               int cap, int gtot, float *__restrict__ part) {
     constexpr int D = 128, LP = D / 8, RPW = 64 / LP, RW = NWV * RPW;
     constexpr int C = sizeof(TKV) == 2 ? 4 : 2; // rows of a chunk per lane group: 2 KB of K and V per lane group
     __shared__ float s_red[NWV * G * D];
@@ -465,6 +465,25 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_decode_1p(const void *__restr
     }
 }
 
+template <typename TKV, int G, int NWV>
+__global__ __launch_bounds__(64 * NWV) void k_attn_decode_1p(const void *__restrict__ qv, int q_f16, const TKV *__restrict__ k,
+                                                              const TKV *__restrict__ v, int64_t kv_sh, int64_t kv_st,
+                                                              const int *__restrict__ len_dev, int len_host, float scale,
+                                                              int cap, int gtot, float *__restrict__ part) {
+    attn_decode_1p<TKV, G, NWV>(qv, q_f16, k, v, kv_sh, kv_st, len_dev, len_host, scale, cap, gtot, part);
+}
+// Sixteen wavefronts of f16 rows, or of f32 rows for two heads, need more than the 128 registers there are for them and keep some in scratch memory.  Such kernels load
+// their arguments themselves, that is take them as a struct: with the first ones in registers at their start they take 0.2 us more (f16, us, so / in registers: 32 / 8
+// heads of 300 keys 6.92 / 7.20, of 2040 7.37 / 7.60; f32 64 / 8 of 1000 8.08 / 8.36; the others are quicker with them there: f32 32 / 8 of 2040 9.41 / 9.16).
+template <typename TKV, int G, int NWV>
+constexpr bool AD_SPILLS = NWV == 16 && G <= 2 && (sizeof(TKV) == 2 || G == 2);
+template <typename TKV>
+struct AdArgs { const void *qv; int q_f16; const TKV *k, *v; int64_t kv_sh, kv_st; const int *len_dev; int len_host; float scale; int cap, gtot; float *part; };
+template <typename TKV, int G, int NWV>
+__global__ __launch_bounds__(64 * NWV) void k_attn_decode_1p_args(AdArgs<TKV> a) {
+    attn_decode_1p<TKV, G, NWV>(a.qv, a.q_f16, a.k, a.v, a.kv_sh, a.kv_st, a.len_dev, a.len_host, a.scale, a.cap, a.gtot, a.part);
+}
+
 // Merge of the parts of one head: thread t fetches the statistics of part t (all parts at once instead of one
 // dependent load per loop trip), the weights go through LDS, and the weighted rows are summed eight loads at a time.
 template <int D, typename TO = float>
@@ -526,9 +545,13 @@ static fh_status ad_launch(fh_device *dev, const float *q, const void *k, const 
             FH_TRY(fh_dev_scratch(dev, (void **)&dev->part_buf, &dev->part_cap, (size_t)hq * S * (D + 4) * 4));
             part = dev->part_buf;
         }
-        k_attn_decode_1p<TKV, (G <= 4 ? G : 4), NWV><<<dim3((unsigned)S, (unsigned)hkv, (unsigned)(gtot / G)), dim3(64 * NWV), 0,
-                                                       dev->stream>>>(q, q_f16 ? 1 : 0, (const TKV *)k, (const TKV *)v, kv_sh,
-                                                                      kv_st, len_dev, len_host, scale, max_len, gtot, part);
+        const dim3 grid((unsigned)S, (unsigned)hkv, (unsigned)(gtot / G));
+        if constexpr (AD_SPILLS<TKV, G, NWV>)
+            k_attn_decode_1p_args<TKV, G, NWV><<<grid, dim3(64 * NWV), 0, dev->stream>>>(
+                AdArgs<TKV>{q, q_f16 ? 1 : 0, (const TKV *)k, (const TKV *)v, kv_sh, kv_st, len_dev, len_host, scale, max_len, gtot, part});
+        else
+            k_attn_decode_1p<TKV, (G <= 4 ? G : 4), NWV><<<grid, dim3(64 * NWV), 0, dev->stream>>>(q, q_f16 ? 1 : 0, (const TKV *)k, (const TKV *)v, kv_sh,
+                                                                                                   kv_st, len_dev, len_host, scale, max_len, gtot, part);
         FH_HIP(hipGetLastError());
         if (splits_out) *splits_out = S;
         if (out) {

@@ -678,6 +678,8 @@ static int ad_heads(const fh_device *dev, int hq, int skv, bool f16) {
 // - where there are half as many again as compute units (one round instead of two or three): us of f32 48 / 16 heads, 16 parts / 8: 3000 keys 24.6 / 19.8, 16384
 //   119 / 83.7; 56 / 8 heads 18.1 / 16.0 and 83.0 / 62.1; 56 heads of their own 34.2 / 33.4 and 168 / 161; with fewer: 40 heads of their own 26.4 / 29.2 and 123 / 136,
 //   33 / 11 heads 4000 keys 18.0 / 19.8, 40 / 8 18.0 / 20.0;
+// - or twelve KV heads and more that several share, from 4096 keys on: f32 36 / 12 heads 5000 keys 25.9 / 23.9, 16384 71.6 / 62.9, 45 / 15 35.4 / 27.2 and 107 / 79.8 (of fewer
+//   40 / 8 22.1 / 23.5, 35 / 7 53.4 / 57.4; of 3500 keys 36 / 12 18.2 / 19.6);
 // - where two heads share a workgroup: f32 64 / 8 15.9 / 13.3 and 51.2 / 43.5, 34 / 17 19.3 / 15.8 and 70.3 / 59.1, f16 64 / 8 14.9 / 11.5 and 38.5 / 31.6 - but for
 //   fewer than eight KV heads only while the keys are few: f32 36 / 6 heads 3000 keys 14.2 / 12.9, 4000 15.1 / 15.8, 16384 39.7 / 42.7, f16 16384 31.5 / 31.1, 32768 53.7 / 55.1;
 // - f16 below 4096 keys, whose parts are short, where heads share a KV head: 33 / 11 heads 15.8 / 14.4, 36 / 4 14.5 / 14.1 (33 heads of their own 20.1 / 20.8).
@@ -687,7 +689,7 @@ static int ad_parts(const fh_device *dev, int hq, int hkv, int skv, bool f16) {
     const int cus = dev->compute_units, group = hq / hkv;
     if (8 * hq <= cus) return 16;
     if (group % 2 == 0) return hkv >= 8 || skv <= (f16 ? 16384 : 3072) ? 8 : 16;
-    return 8 * hq >= 3 * cus / 2 || (f16 && group > 1 && skv < 4096) ? 8 : 16;
+    return 8 * hq >= 3 * cus / 2 || (group > 1 && (hkv >= 12 ? skv >= 4096 || f16 : f16 && skv < 4096)) ? 8 : 16;
 }
 
 // Room for the partial results of `splits` parts.  When it has to grow it grows to what a cache of any length needs, so that the graphs that hold its address

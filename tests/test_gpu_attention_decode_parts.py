@@ -117,6 +117,8 @@ def test_scratch_limit_that_the_call_keeps(oracle, dtype, L):
     ("f32", 40, 40, 2049, 16),  # more workgroups than compute units, but fewer than half as many again
     ("f32", 48, 16, 2049, 8),   # not fewer
     ("f32", 40, 8, 4000, 16),
+    ("f32", 36, 12, 4095, 16),  # twelve KV heads
+    ("f32", 36, 12, 4096, 8),
     ("f32", 64, 8, 4000, 8),    # two heads a workgroup
     ("f32", 36, 6, 3072, 8),    # of few KV heads, while the keys are few
     ("f32", 36, 6, 3073, 16),

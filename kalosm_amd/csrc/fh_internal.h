@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stddef.h>
+#include <atomic>
 #include <string>
 #include <utility>
 #include <vector>
@@ -72,6 +73,7 @@ struct fh_device {
     size_t static_scratch_bytes = 0;
     // kernels whose dynamic LDS limit was raised on this device, with the limit (fh_kernel_lds)
     std::vector<std::pair<const void *, size_t>> lds_raised;
+    std::atomic<uint64_t> matrix_bytes{0}; // of all its matrices (fh_matrices_stream)
     // options (fh_set_option)
     int64_t opt_matvec_kernel = 0;   // 0 auto, 1 generic VALU, 2 MFMA, 3 first-generation Q4_K MFMA, 4 batch MFMA
     int64_t opt_matvec_splitk = 0;   // 0 auto, else forced split count
@@ -103,6 +105,10 @@ struct fh_device {
 };
 
 enum { FH_FIXED_BYTES = 9 << 20, FH_ARRIVED = 16384 };
+// Whether more weights are on the device than its last cache holds, 256 MB: what a program keeps there it reads between two uses of one of them, as far as a
+// single product can know.
+enum { FH_LAST_CACHE = 256 << 20 };
+static inline bool fh_matrices_stream(const fh_device *dev) { return dev->matrix_bytes.load(std::memory_order_relaxed) > FH_LAST_CACHE; }
 
 // Which scratch memory the kernels of a captured graph hold the addresses of: begin ahead of the capture, end behind it.
 struct FhScratchStamp {

@@ -326,7 +326,7 @@ fh_status fh_llama::finalize() {
     FH_TRY(fh_kvcache_create(m->dev, c.n_layers, c.n_kv_heads, c.head_dim, c.ctx, c.kv_dtype, &m->cache));
     FH_TRY(m->create_loop_buffers());
     FH_TRY(m->ensure_steps(1));
-    const int streamed = m->weight_bytes() > (uint64_t)256 << 20;
+    const int streamed = m->weight_bytes() > FH_LAST_CACHE;
     for (auto &l : m->layer)
         for (fh_qmatrix *q : {l.wq, l.wk, l.wv, l.wo, l.gate, l.up, l.down, l.qkv, l.gate_up})
             if (q) q->streamed = streamed;

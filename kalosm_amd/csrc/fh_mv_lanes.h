@@ -43,9 +43,10 @@ __device__ __forceinline__ uint32_t sel_lanes(uint64_t mask, uint32_t yes, uint3
 
 
 // Weights of a product of one or a few rows are read by one wavefront each and not again in this launch.  Where more than the 256 MB of the last cache passes
-// before the next step reads them, they are read with the hint that they are streamed; a decoder knows whether it does, a matrix by itself is taken for a part of
-// a larger whole from 16 MB on.  us, plainly / by that rule: 8B, 512 + 128 tokens 197017 / 188284 (only the matrices of 16 MB and more 196240), products of three
-// layers (4096 / 14336, 235 MB) of one row 69.9 / 66.5 (all with the hint 68.5), of 16 rows 145.6 / 139.9; a 2048-wide decoder of 193 MB 8904 (9052 with it).
+// before the next step reads them, they are read with the hint that they are streamed.  A decoder knows whether it does; a matrix by itself is taken for a part
+// of a larger whole from 16 MB on, if the matrices on the device are more than that cache.  us, plainly / with the hint: 8B, 512 + 128 tokens 197017 / 188284 (only the
+// matrices of 16 MB and more 196240), a 2048-wide decoder of 193 MB 8904 / 9052; one row of Q4_K 28672 x 4096, one of them 12.4 / 12.9, four (264 MB) 12.4 / 13.8, seven (462 MB)
+// 14.8 / 14.0, of 65536 x 4096, one (151 MB) 23.2 / 26.1, two 28.0 / 26.7; sixteen rows of Q8_0 14336 x 4096, four (250 MB) 17.0 / 18.2, seven 19.3 / 18.5.
 template <bool ONCE, typename T>
 __device__ __forceinline__ T fh_ld_weights(const uint8_t *p) {
     if constexpr (!ONCE) return *(const T *)p;
@@ -55,4 +56,4 @@ __device__ __forceinline__ T fh_ld_weights(const uint8_t *p) {
     __builtin_memcpy(&r, &v, sizeof(T));
     return r;
 }
-static inline bool fh_weights_once(const fh_qmatrix *q) { return q->streamed < 0 ? q->bytes >= (size_t)16 << 20 : q->streamed != 0; }
+static inline bool fh_weights_once(const fh_qmatrix *q) { return q->streamed < 0 ? q->bytes >= (size_t)16 << 20 && fh_matrices_stream(q->dev) : q->streamed != 0; }

@@ -138,6 +138,7 @@ static fh_status qm_alloc(fh_device *dev, uint32_t type, int64_t n, int64_t k, f
         FH_FAIL(err == hipErrorOutOfMemory ? FH_ERR_OOM : FH_ERR_HIP, "hipMalloc(%zu) failed: %s", q->bytes,
                 hipGetErrorString(err));
     }
+    dev->matrix_bytes += q->bytes;
     *out = q;
     return FH_OK;
 }
@@ -251,6 +252,7 @@ extern "C" fh_status fh_qmatrix_free(fh_qmatrix *q) {
     if (q->data) {
         (void)hipStreamSynchronize(q->dev->stream);
         (void)hipFree(q->data);
+        q->dev->matrix_bytes -= q->bytes;
     }
     delete q;
     return FH_OK;

@@ -1,4 +1,5 @@
-"""Products of one to sixteen rows of matrices on both sides of the size from which weights are read as a stream: the same weights, the same sums."""
+"""Products of one to sixteen rows of matrices on both sides of the size from which weights are read as a stream where there are more of them than the last
+cache holds, and of the same matrix with and without others beside it: the same weights, the same sums."""
 import numpy as np
 import pytest
 
@@ -28,3 +29,18 @@ def test_rows_do_not_depend_on_how_weights_are_read(ty, rows):
     w = np.abs(QMatrix.from_raw_bytes(dev, (few, k), part, ty).dequantize().as_slice().astype(np.float64).reshape(few, k))
     bound = np.abs(x.astype(np.float64)).reshape(rows, k) @ w.T * 4096 * 2.0 ** -24
     assert (np.abs(got[:, 0].astype(np.float64) - want) <= bound).all()
+
+
+@pytest.mark.parametrize("ty", TYPES)
+def test_bits_do_not_depend_on_other_matrices(ty):
+    """A matrix of 16 MB by itself is read plainly, beside 256 MB of others as a stream, and plainly again when they are gone."""
+    dev, n, k = Device.gpu(0), 16384, 4096
+    q = QMatrix.from_raw_bytes(dev, (n, k), np.tile(synth.random_weight(ty, 512, k, seed=ty), n // 512), ty)
+    xs = [Tensor.from_slice(dev, synth.random_activation(rows, k, seed=rows)) for rows in (1, 2, 4, 16)]
+    alone = [x.q_mat_mul(q).as_slice() for x in xs]
+    others = QMatrix.from_raw_bytes(dev, (65536, 4096), np.zeros(65536 * 4096 // 32 * 34, np.uint8), synth.Q8_0)
+    for x, want in zip(xs, alone):
+        assert np.array_equal(x.q_mat_mul(q).as_slice(), want)
+    del others
+    for x, want in zip(xs, alone):
+        assert np.array_equal(x.q_mat_mul(q).as_slice(), want)

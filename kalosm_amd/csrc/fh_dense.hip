@@ -1106,11 +1106,138 @@ __global__ __launch_bounds__(256) void k_pad_bf16_rows(const uint16_t *__restric
     for (int i = threadIdx.x; i < kp; i += 256) y[(int64_t)blockIdx.x * kp + i] = i < k ? x[(int64_t)blockIdx.x * k + i] : 0;
 }
 
+// ROWS weight rows of one wavefront, streamed in pieces of 512 (a lane: eight values, 16 bytes) with AHEAD pieces on their way.
+// No request is under a condition - a lane past the end of the rows repeats the last eight values, a piece past the last one the
+// last piece: with a branch around a request the compiler can no longer count what is younger and waits for everything.
+template <int ROWS, int AHEAD>
+struct RowStream {
+    const uint16_t *w[ROWS];
+    uint4 u[AHEAD][ROWS];
+    int kp, pieces, lane8;
+    __device__ __forceinline__ void fetch(int slot, int piece) {
+        const int c = piece * 512 + lane8, at = c < kp ? c : kp - 8;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) u[slot][r] = *(const uint4 *)(w[r] + at);
+    }
+    __device__ __forceinline__ void start(int kp_) {
+        kp = kp_, pieces = fh_row_pieces(kp), lane8 = (threadIdx.x & 63) * 8;
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) fetch(i, i < pieces ? i : pieces - 1);
+    }
+    __device__ __forceinline__ void use(int slot, int piece, const float *x, float *acc) const {
+        const int c = piece * 512 + lane8;
+        if (c >= kp) return;
+        const float4 a = *(const float4 *)(x + c), b = *(const float4 *)(x + c + 4);
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) acc[r] = fh_dot8(u[slot][r], a, b, acc[r]);
+    }
+    // acc[r] += rows . x (x: kp values in the LDS), not yet summed over the lanes
+    __device__ __forceinline__ void run(const float *x, float *acc) {
+        int p = 0;
+        for (; p + AHEAD < pieces; p += AHEAD) {
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) {
+                use(i, p + i, x, acc);
+                fetch(i, p + i + AHEAD < pieces ? p + i + AHEAD : pieces - 1);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++)
+            if (p + i < pieces) use(i, p + i, x, acc);
+    }
+};
+
+// The product by itself where dealing the rows out (FhRowDeal, k_matvec_mix) costs more than it gives: as many workgroups of four wavefronts as there are rows for,
+// each with all that it reads on its way; the same sums.  XV: 16-byte pieces of the input a thread holds, requested ahead of the first weights (k a multiple
+// of four); 0: the input goes to the LDS in a loop ahead of them.
+template <int ROWS, int XV>
+__global__ __launch_bounds__(256, XV ? 1 : 8) void k_matvec_rows(const float *__restrict__ x, const uint16_t *__restrict__ w, int k, int kp, int n, float *__restrict__ y) {
+    typedef float four __attribute__((ext_vector_type(4), aligned(4))); // (a caller's x may begin anywhere)
+    extern __shared__ __attribute__((aligned(16))) float xs[]; // [kp]
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, row0 = ((int)blockIdx.x * 4 + wave) * ROWS;
+    RowStream<ROWS, XV == 0 ? 8 / ROWS : XV == 1 ? 2 : 8> rows;
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) rows.w[r] = w + (int64_t)(row0 + r < n ? row0 + r : n - 1) * kp;
+    if (XV && !(k & 3)) { // (k is at most 1024 XV)
+        constexpr int NX = XV ? XV : 1;
+        four v[NX];
+#pragma unroll
+        for (int j = 0; j < NX; j++) {
+            const int i = (tid + 256 * j) * 4;
+            v[j] = *(const four *)(x + (i < k ? i : 0));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        rows.start(kp);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NX; j++) {
+            const int i = (tid + 256 * j) * 4;
+            if (i < kp) *(float4 *)(xs + i) = mv_if(i < k, make_float4(v[j][0], v[j][1], v[j][2], v[j][3]));
+        }
+    } else {
+        if (!(k & 3)) {
+#pragma unroll 8
+            for (int i = tid * 4; i < kp; i += 1024) {
+                four v = {0.f, 0.f, 0.f, 0.f};
+                if (i < k) v = *(const four *)(x + i);
+                *(float4 *)(xs + i) = make_float4(v[0], v[1], v[2], v[3]);
+            }
+        } else {
+#pragma unroll 8
+            for (int i = tid; i < kp; i += 256) xs[i] = i < k ? x[i] : 0.f;
+        }
+        rows.start(kp);
+    }
+    __syncthreads();
+    float acc[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) acc[r] = 0.f;
+    rows.run(xs, acc);
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) acc[r] = fh_wave_sum(acc[r]);
+    if (lane == 0)
+#pragma unroll
+        for (int r = 0; r < ROWS; r++)
+            if (row0 + r < n) y[row0 + r] = acc[r];
+}
+
+template <int ROWS, int XV>
+static fh_status matvec_rows_go(const fh_qmatrix *q, const float *x, float *y) {
+    fh_device *dev = q->dev;
+    const int n = (int)q->n, kp = (int)q->recs;
+    const size_t lds = (size_t)kp * 4;
+    if (lds > 48 * 1024) FH_TRY(fh_kernel_lds(dev, (const void *)k_matvec_rows<ROWS, XV>, lds));
+    k_matvec_rows<ROWS, XV><<<dim3((unsigned)((n + 4 * ROWS - 1) / (4 * ROWS))), 256, lds, dev->stream>>>(x, (const uint16_t *)q->data, (int)q->k, kp, n, y);
+    FH_HIP(hipGetLastError());
+    return FH_OK;
+}
+
+// Where that is.  Times of the rows dealt out over those here, one matrix again and again / 420 MB of them:
+// - long inputs and few rows, of which a wavefront has one: 512 x 14336 1.4 / 1.25, 512 x 8192 1.2 / 1.05, 512 x 28672 1.8 / 1.8, 1024 x 28672 1.4 / 1.3, but 1024 x 14336 1.3 / 1.0 and
+//   1024 x 16384 1.25 / 0.9 (1536 x 14336 0.87 / 0.95, 512 x 4096 1.0 / 0.8);
+// - rows of one piece, whose sum over the lanes is all there is to wait for: k = 512 1.2 to 1.5 / 1.1 to 1.3; of two pieces (k = 1024) 4096 rows 1.36 / 1.0, 16384 rows
+//   1.5 / 1.0 (512 rows 1.13 / 0.94), and of three where the dealt out ones come out uneven: k = 1536 6144 rows 1.5 / 1.25, 4096 rows 1.4 / 1.05 (3072 rows / 0.98);
+// - k up to 3072 and 2048 to 6144 rows that stay in the last cache: 4096 x 2048 4.0 us / 3.1, 3072 x 2048 1.29 (/ 0.95; 16384 x 2048 0.76 / 0.8).
+static bool matvec_rows_pay(const fh_device *dev, int n, int k) {
+    const bool stream = fh_matrices_stream(dev);
+    if (k > 4096) return n <= (stream && k <= 16384 ? 512 : 1024);
+    if (k <= 512 || (k <= 1536 && n >= 4096 && n < 8192)) return true;
+    return !stream && (k <= 1024 || (k <= 3072 && n >= 2048 && n <= 6144) || (k <= 2048 && n >= 2048 && n <= 8192));
+}
+static fh_status matvec_rows(const fh_qmatrix *q, const float *x, float *y) {
+    const int64_t k = q->k, waves = (int64_t)q->dev->compute_units * 4;
+    if (q->n >= waves * 8) return matvec_rows_go<4, 0>(q, x, y);
+    if (q->n >= waves * 2) return k <= 1024 ? matvec_rows_go<2, 1>(q, x, y) : matvec_rows_go<2, 0>(q, x, y);
+    if (k <= 1024) return matvec_rows_go<1, 1>(q, x, y);
+    return k <= 16384 ? matvec_rows_go<1, 16>(q, x, y) : matvec_rows_go<1, 0>(q, x, y);
+}
+
 // f32 activations are multiplied in true f32, bf16 ones on the bf16 matrix cores.
 fh_status fh_launch_bf16_matmul(const fh_qmatrix *q, const void *x, int x_is_bf16, int m, float *y) {
     fh_device *dev = q->dev;
     const int k = (int)q->k, kp = (int)q->recs;
     if (m == 1 && !x_is_bf16 && (size_t)kp * 4 <= 120 * 1024) {
+        if (matvec_rows_pay(dev, (int)q->n, k)) return matvec_rows(q, (const float *)x, y);
         const FhMvSeg s{(const uint16_t *)q->data, y, (int)q->n};
         return fh_matvec_norm(dev, (const float *)x, k, nullptr, 0.f, &s, 1, nullptr);
     }

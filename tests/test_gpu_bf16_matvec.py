@@ -1,4 +1,4 @@
-"""GPU parity: one f32 row times bf16 weights (csrc/fh_dense.hip: k_matvec_norm, k_matvec_mix) against float64, over every way
+"""GPU parity: one f32 row times bf16 weights (csrc/fh_dense.hip: k_matvec_mix, k_matvec_rows) against float64, over every way
 the input takes to the LDS and past the requests that go out ahead.
 
 Bound: f32 products and sums of k terms, a lane's chain of k / 64 of them: rounding errors of 2^-24 of either sign, 1e-6 of the
@@ -8,7 +8,7 @@ import pytest
 
 import hybridgen as G
 from kalosm_amd import synth
-from kalosm_amd.fusor import QMatrix, Tensor
+from kalosm_amd.fusor import Device, QMatrix, Tensor
 from oracle import hybrid_ref as R
 from test_gpu_hybrid import TOL, close, run_portions
 
@@ -70,3 +70,25 @@ def test_infinite_weights(dev, n, k):
     assert got[2] == np.inf and got[3] == -np.inf and got[4] == np.inf
     rest = [i for i in range(n) if i not in (2, 3, 4)]
     near(got[rest].astype(np.float64), synth.from_bf16_bits(w[rest]).astype(np.float64) @ x[0].astype(np.float64))
+
+
+@pytest.mark.parametrize("n,k", [(37, 500), (1024, 4100), (1025, 4100), (1000, 20000), (5000, 1500), (2048, 2048), (6144, 3072), (8192, 2048), (8200, 1024), (3000, 1002)])
+@pytest.mark.parametrize("offset", [0, 4])
+def test_the_same_sums_dealt_out_or_not(dev, n, k, offset):
+    """Either side of the lines between the two ways rows are handed to wavefronts, one of which is whether the device's matrices are more than its last
+    cache; the input may begin at any value."""
+    rng = np.random.default_rng(n + k)
+    w = synth.to_bf16_bits(rng.standard_normal(n * k, dtype=np.float32))
+    x = rng.standard_normal((1, k), dtype=np.float32)
+    own = Device.gpu(0)
+    try:
+        q = QMatrix.from_raw_bytes(own, (n, k), w, synth.W_BF16)
+        base = Tensor.from_slice(own, np.concatenate([np.zeros(offset // 4, np.float32), x[0]]))
+        xt = Tensor(own, (1, k), ptr=base.ptr + offset)
+        alone = xt.q_mat_mul(q).as_slice()
+        near(alone[0].astype(np.float64), synth.from_bf16_bits(w).reshape(n, k).astype(np.float64) @ x[0].astype(np.float64))
+        others = QMatrix.from_raw_bytes(own, (65536, 2056), np.zeros(65536 * 2056, np.uint16), synth.W_BF16)
+        assert np.array_equal(xt.q_mat_mul(q).as_slice(), alone)
+        del others
+    finally:
+        own.close()

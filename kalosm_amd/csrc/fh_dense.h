@@ -95,6 +95,14 @@ __device__ __forceinline__ uint4 fh_load_once(const uint16_t *p) {
     const words v = __builtin_nontemporal_load((const words *)p);
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
+// Values at .. at + 7 of a row of kp (in a scalar register), zeros past its end: it is a buffer of its own, and what lies past a buffer is not read.  (The row's last
+// eight values again, whose products with zeros are dropped, would have to be told from others: an infinity among them makes NaN.  us of 32768 x 1024 / 16384 x 1280 /
+// 4096 x 4096: without that, 13.0 / 9.4 / 8.2, with that choice in the code 13.5 / 9.5 / 8.4, so 13.4 / 9.3 / 8.1.)
+__device__ __forceinline__ uint4 fh_load_row_once(const uint16_t *row, int kp, int at) {
+    typedef uint32_t words __attribute__((ext_vector_type(4)));
+    const words v = __builtin_amdgcn_raw_buffer_load_b128(__builtin_amdgcn_make_buffer_rsrc((void *)row, 0, kp * 2, 0x00027000), at * 2, 0, 2); // (2: not read again)
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
 __device__ __forceinline__ float fh_dot8(const uint4 &w, const float4 &a, const float4 &b, float acc) {
     acc = fmaf(fh_bf_lo(w.x), a.x, acc);
     acc = fmaf(fh_bf_hi(w.x), a.y, acc);
@@ -129,8 +137,7 @@ struct FhRowDeal {
     int kp, pieces, count, left, piece, lane8;
     uint4 u[AHEAD];
     __device__ __forceinline__ void fetch(int slot) {
-        const int c = piece * 512 + lane8;
-        u[slot] = fh_load_once(row + (c < kp ? c : kp - 8));
+        u[slot] = fh_load_row_once(row, kp, piece * 512 + lane8);
         const bool end = ++piece == pieces;
         piece = end ? 0 : piece;
         left -= end;
@@ -150,19 +157,18 @@ struct FhRowDeal {
         float acc = 0.f;
         int p = 0, i = 0;
         const int total = count * pieces;
-        const bool past = (pieces - 1) * 512 + lane8 >= kp; // of a row's last piece this lane has its last eight values again, which may be infinite: not used
         for (int t = 0; t < total; t += AHEAD) {
 #pragma unroll
             for (int s = 0; s < AHEAD; s++) {
                 const float *at = x.xs + p * 256 + (lane8 >> 1);
                 const float4 a = *(const float4 *)at, b = *(const float4 *)(at + x.plane);
-                const float more = fh_dot8(u[s], a, b, acc);
+                acc = fh_dot8(u[s], a, b, acc);
                 fetch(s);
                 if (++p == pieces) {
-                    acc = fh_wave_sum(past ? acc : more);
+                    acc = fh_wave_sum(acc);
                     if (i < count) done(i, acc); // (what is behind the last row is the last piece again)
                     acc = 0.f, p = 0, i++;
-                } else acc = more;
+                }
             }
         }
     }

@@ -201,10 +201,8 @@ __device__ __forceinline__ void expert_step(const FhStep &st, int b, int blocks,
     int left = count, piece = 0;
     uint4 g[AHEAD], u[AHEAD];
     auto fetch = [&](int s) {
-        const int c = piece * 512 + lane8;
-        const uint16_t *at = row + (c < kp ? c : kp - 8);
-        g[s] = fh_load_once(at);
-        u[s] = fh_load_once(at + (int64_t)16 * kp);
+        g[s] = fh_load_row_once(row, kp, piece * 512 + lane8);
+        u[s] = fh_load_row_once(row + (int64_t)16 * kp, kp, piece * 512 + lane8);
         if (++piece == pieces) {
             piece = 0, left--;
             if (left > 0) next = ahead(next, step), row = gate(next);
@@ -212,7 +210,6 @@ __device__ __forceinline__ void expert_step(const FhStep &st, int b, int blocks,
     };
 #pragma unroll
     for (int s = 0; s < AHEAD; s++) fetch(s);
-    const bool past = (pieces - 1) * 512 + lane8 >= kp; // (FhRowDeal)
     float ag = 0.f, au = 0.f;
     int p = 0, i = 0;
     for (int t = 0; t < count * pieces; t += AHEAD) {
@@ -220,14 +217,15 @@ __device__ __forceinline__ void expert_step(const FhStep &st, int b, int blocks,
         for (int s = 0; s < AHEAD; s++) {
             const float *at = xs.xs + p * 256 + lane * 4;
             const float4 a = *(const float4 *)at, c = *(const float4 *)(at + xs.plane);
-            const float mg = fh_dot8(g[s], a, c, ag), mu = fh_dot8(u[s], a, c, au);
+            ag = fh_dot8(g[s], a, c, ag);
+            au = fh_dot8(u[s], a, c, au);
             fetch(s);
             if (++p == pieces) {
-                ag = fh_wave_sum(past ? ag : mg), au = fh_wave_sum(past ? au : mu);
+                ag = fh_wave_sum(ag), au = fh_wave_sum(au);
                 if (i < count && lane == 0) st.act[(int64_t)now.slot * m.ffp + now.p] = fh_silu_f(ag) * au;
                 ag = au = 0.f, p = 0;
                 if (++i < count) now = ahead(now, step);
-            } else ag = mg, au = mu;
+            }
         }
     }
 }

@@ -851,9 +851,10 @@ __device__ __forceinline__ float4 mv_if(bool c, float4 v) { // (v or zeros: as o
 }
 
 // x' into the LDS, mixed with the token before it where the matrix wants that; start() asks for the first weights.
-// XQ: fours of consecutive values of each vector that a thread holds, all requested at once (k a multiple of 4, 256 WAVES XQ at most); 0: any k, value
-// by value.  MODE: what a launch has of this, so that one without a norm has no requests and registers for it.
+// XQ: fours of consecutive values of each vector that a thread holds, all requested at once (k a multiple of 4, 256 WAVES XQ at most); 0: any k, in
+// fours or value by value.  MODE: what a launch has of this, so that one without a norm has no requests and registers for it.
 enum { MV_PLAIN = 0, MV_NORM = 1, MV_ADD = 2, MV_SHIFT = 3, MV_GATED = 4 };
+typedef float mv_four __attribute__((ext_vector_type(4), aligned(4))); // (of a vector that may begin anywhere)
 template <int WAVES, int XQ, int MODE, typename F>
 __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int k, int kp, const FhRowInput &xs, float *red, F start) {
     constexpr int NT = WAVES * 64;
@@ -921,6 +922,40 @@ __device__ __forceinline__ void mv_input(const FhMvAdd &in, const float *mu, int
                                 fmaf(b[j].w - v.w, m[j].w, v.w));
             xs.quad(i >> 2) = mv_if(i < k, v);
         }
+    } else if (!(k & 3)) { // longer than that, or from anywhere: in fours as well, dealt out alike, so that a norm has the same bits
+        float inv = 0.f;
+        if (normed) {
+            const float *from = NORM ? in.x : in.y;
+#pragma unroll
+            for (int h = 0; h < 8 / WAVES; h++)
+                for (int i = (tid + NT * h) * 4; i < k; i += 2048) {
+                    const mv_four v = *(const mv_four *)(from + i);
+                    ss[h] = fmaf(v[0], v[0], fmaf(v[1], v[1], fmaf(v[2], v[2], fmaf(v[3], v[3], ss[h]))));
+                }
+            inv = scale();
+        }
+#pragma unroll 2
+        for (int i = tid * 4; i < end; i += NT * 4) {
+            mv_four v = {0.f, 0.f, 0.f, 0.f};
+            if (i < k) {
+                v = *(const mv_four *)(in.x + i);
+                if (NORM) v = v * inv * *(const mv_four *)(in.norm + i);
+                else if (add) v += *(const mv_four *)(in.y + i) * inv * *(const mv_four *)(in.w + i);
+                if (one) {
+                    if (in.x_out) *(mv_four *)(in.x_out + i) = v;
+                    if (state) *(mv_four *)(here + i) = v;
+                }
+                if (mu) {
+                    const mv_four m = *(const mv_four *)(mu + i);
+                    mv_four b = {0.f, 0.f, 0.f, 0.f};
+                    if (shift) b = *(const mv_four *)(before + i);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] = fmaf(b[e] - v[e], m[e], v[e]);
+                }
+            } else if (one && in.x_out && i < out) *(mv_four *)(in.x_out + i) = v;
+            xs.quad(i >> 2) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+        start();
     } else {
         float inv = 0.f;
         if (normed) {
@@ -1152,7 +1187,6 @@ struct RowStream {
 // of four); 0: the input goes to the LDS in a loop ahead of them.
 template <int ROWS, int XV>
 __global__ __launch_bounds__(256, XV ? 1 : 8) void k_matvec_rows(const float *__restrict__ x, const uint16_t *__restrict__ w, int k, int kp, int n, float *__restrict__ y) {
-    typedef float four __attribute__((ext_vector_type(4), aligned(4))); // (a caller's x may begin anywhere)
     extern __shared__ __attribute__((aligned(16))) float xs[]; // [kp]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, row0 = ((int)blockIdx.x * 4 + wave) * ROWS;
     RowStream<ROWS, XV == 0 ? 8 / ROWS : XV == 1 ? 2 : 8> rows;
@@ -1160,11 +1194,11 @@ __global__ __launch_bounds__(256, XV ? 1 : 8) void k_matvec_rows(const float *__
     for (int r = 0; r < ROWS; r++) rows.w[r] = w + (int64_t)(row0 + r < n ? row0 + r : n - 1) * kp;
     if (XV && !(k & 3)) { // (k is at most 1024 XV)
         constexpr int NX = XV ? XV : 1;
-        four v[NX];
+        mv_four v[NX];
 #pragma unroll
         for (int j = 0; j < NX; j++) {
             const int i = (tid + 256 * j) * 4;
-            v[j] = *(const four *)(x + (i < k ? i : 0));
+            v[j] = *(const mv_four *)(x + (i < k ? i : 0));
         }
         __builtin_amdgcn_sched_barrier(0);
         rows.start(kp);
@@ -1178,8 +1212,8 @@ __global__ __launch_bounds__(256, XV ? 1 : 8) void k_matvec_rows(const float *__
         if (!(k & 3)) {
 #pragma unroll 8
             for (int i = tid * 4; i < kp; i += 1024) {
-                four v = {0.f, 0.f, 0.f, 0.f};
-                if (i < k) v = *(const four *)(x + i);
+                mv_four v = {0.f, 0.f, 0.f, 0.f};
+                if (i < k) v = *(const mv_four *)(x + i);
                 *(float4 *)(xs + i) = make_float4(v[0], v[1], v[2], v[3]);
             }
         } else {

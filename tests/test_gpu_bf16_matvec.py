@@ -49,7 +49,7 @@ def test_normed(dev, width, vocab):
     near(logits, w["head"].astype(np.float64) @ hidden.astype(np.float64))
 
 
-@pytest.mark.parametrize("width,ff", [(64, 16640), (4160, 48)])
+@pytest.mark.parametrize("width,ff", [(64, 16640), (4160, 48), (16400, 48), (16402, 40)])
 def test_decode_step(dev, width, ff):
     """Inputs of a step's products that no thread holds whole: a long feed-forward, a wide stream."""
     cfg = G.config_apart([G.with_mlp(G.pair(), G.dense(ff)), G.with_mlp(G.retention(), G.dense(ff))], width=width, vocab=50)

@@ -50,3 +50,15 @@ def test_few_rows(dev, width, vocab, matvecs):
         want = np.array(alone[:count])
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)) == (count == matvecs)
         assert np.sqrt(np.mean((got - want) ** 2)) <= 2e-6 * np.sqrt(np.mean(want ** 2))
+
+
+@pytest.mark.parametrize("width", [16388, 16400, 16401])
+def test_wide_rows_norm_alike(dev, width):
+    """Rows longer than a workgroup holds in registers, in fours and value by value: of one place and of several the same bits."""
+    cfg = G.config([G.with_mlp(G.delta(1, 1, 16, 16, 4), None)], width, 30)
+    m = G.build(dev, cfg, G.weights(cfg))
+    toks = np.random.default_rng(width).integers(0, 30, 9)
+    _, last = m.forward(toks, want_hidden=True, want=list(range(9)))
+    m.reset()
+    _, hidden = m.forward(toks, want_hidden=True, want=[8])
+    assert np.array_equal(last.view(np.uint32), hidden.view(np.uint32))

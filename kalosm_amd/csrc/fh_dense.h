@@ -129,7 +129,6 @@ struct FhRowInput {
     __device__ __forceinline__ float &at(int i) const { return xs[((i >> 2) & 1) * plane + (i >> 3) * 4 + (i & 3)]; }
 };
 __host__ __device__ static inline int fh_row_pieces(int kp) { return (kp + 511) / 512; }
-enum { FH_ROW_WAVES = 8 };
 template <int AHEAD = 4>
 struct FhRowDeal {
     const uint16_t *row; // of the next request
@@ -222,7 +221,7 @@ struct FhGemm {
 };
 fh_status fh_gemm(fh_device *dev, int dtype, int epi, const FhGemm &g);
 
-// y[seg][row] = W_seg[row, :] . n(x), n(x) = x / rms(x) * w (w NULL: x as it is).  norm_out (optional) receives n(x).
+// y[seg][row] = W_seg[row, :] . n(x), n(x) = x / rms(x) * w (w NULL: x as it is).  norm_out (optional, with w) receives n(x), kp values.
 struct FhMvSeg { const uint16_t *w; float *y; int n; };
 fh_status fh_matvec_norm(fh_device *dev, const float *x, int k, const float *w, float eps, const FhMvSeg *segs, int n_segs,
                          float *norm_out);
@@ -277,7 +276,6 @@ struct FhMvAdd {
     const float *norm = nullptr;  // x' = x / rms(x) * norm instead (fh_matvec_norm)
     float eps = 0.f;
     float *x_out = nullptr;
-    bool x_pad = false;           // x_out has zeros up to kp
     float *state = nullptr;       // [2][k]
     const int *pos_dev = nullptr;
     const float *gate = nullptr;

@@ -1128,11 +1128,12 @@ fh_status fh_matvec_mix(fh_device *dev, const FhMvAdd &in, int k, const FhMvMix 
 fh_status fh_matvec_norm(fh_device *dev, const float *x, int k, const float *w, float eps, const FhMvSeg *segs, int n_segs,
                          float *norm_out) {
     FH_REQUIRE(n_segs >= 1 && n_segs <= 3, "1 to 3 matrices per matvec launch");
+    FH_REQUIRE(w || !norm_out, "a normed row to give back needs a norm");
     FH_REQUIRE(fh_pad64(k) * 4 <= 120 * 1024, "k = %d too long for the matvec", k);
     FhMvMix ms[3];
     for (int i = 0; i < n_segs; i++) ms[i] = FhMvMix{segs[i].w, nullptr, segs[i].y, segs[i].n, FH_MV_ACT_NONE};
     FhMvAdd in;
-    in.x = x, in.norm = w, in.eps = eps, in.x_out = norm_out, in.x_pad = true;
+    in.x = x, in.norm = w, in.eps = eps, in.x_out = norm_out;
     return matvec_mix(dev, in, k, ms, n_segs);
 }
 

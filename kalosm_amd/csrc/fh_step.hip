@@ -4,18 +4,6 @@
 
 static constexpr float FH_LOG2E = 1.4426950408889634f;
 
-__device__ __forceinline__ float dot8(const uint4 &w, const float *x, float acc) {
-    const float4 a = *(const float4 *)x, b = *(const float4 *)(x + 4);
-    acc = fmaf(fh_bf_lo(w.x), a.x, acc);
-    acc = fmaf(fh_bf_hi(w.x), a.y, acc);
-    acc = fmaf(fh_bf_lo(w.y), a.z, acc);
-    acc = fmaf(fh_bf_hi(w.y), a.w, acc);
-    acc = fmaf(fh_bf_lo(w.z), b.x, acc);
-    acc = fmaf(fh_bf_hi(w.z), b.y, acc);
-    acc = fmaf(fh_bf_lo(w.w), b.z, acc);
-    acc = fmaf(fh_bf_hi(w.w), b.w, acc);
-    return acc;
-}
 
 // One step of a recurrence: workgroup b takes 16 columns of one head's state, RPT rows per lane as in the prefill scan.
 template <int RPT>
@@ -543,9 +531,9 @@ __device__ __forceinline__ void linear_step(const FhMixStep &st, int pos, int b,
 #pragma unroll
         for (int i = 0; i < RPT; i++) {
             const int c = 16 * i + (tid >> 4);
-            float z = rg * 8 < r.rp ? dot8(w2[i], t1 + rg * 8, 0.f) : 0.f;
+            float z = rg * 8 < r.rp ? fh_dot8(w2[i], *(const float4 *)(t1 + rg * 8), *(const float4 *)(t1 + rg * 8 + 4), 0.f) : 0.f;
             if (c < d)
-                for (int x = rg * 8 + 128; x < r.rp; x += 128) z = dot8(*(const uint4 *)(r.w2 + (int64_t)(h * d + c) * r.rp + x), t1 + x, z);
+                for (int x = rg * 8 + 128; x < r.rp; x += 128) z = fh_dot8(*(const uint4 *)(r.w2 + (int64_t)(h * d + c) * r.rp + x), *(const float4 *)(t1 + x), *(const float4 *)(t1 + x + 4), z);
             z = fh_row16_sum(z);
             if (rg == 0 && c < d) g[c] = expf(fh_rec_la(z + w0[i]));
         }

@@ -181,7 +181,7 @@ struct fh_qmatrix {
 enum { FH_W_F32 = 0, FH_W_F16 = 1, FH_GGML_I32 = 26 };
 static inline bool fh_is_plain(uint32_t t) { return t == FH_W_F32 || t == FH_W_F16 || t == FH_BF16; }
 // Types without kernels for several activation rows (batch, row and tile kernels): those go row by row or element by
-// element.  The 5-bit formats have the single-row matrix-core kernel only.
+// element.  The 5-bit formats have the single-row matrix-core kernel and those that decode in registers (fh_qmv_rows.hip, fh_qmm_reg.hip).
 static inline bool fh_single_row_only(uint32_t t) { return fh_is_plain(t) || t == FH_Q5_0 || t == FH_Q5_K; }
 static inline int fh_block_elems(uint32_t t) {
     switch (t) {

@@ -358,8 +358,8 @@ fh_status fh_launch_qmatvec(const fh_qmatrix *q, const float *x, int m, float *y
         fh_status st = fh_launch_q4k_m1(q, x, y, epi, a, b);
         if (st != FH_ERR_UNSUPPORTED) return st;
     }
-    // the 5-bit formats have the single-row kernel only: a few rows are a launch each (10 us a row against 110 - 640 us
-    // for 2 .. 16 rows through the per-element kernel at 14336 x 4096)
+    // the 5-bit formats have the single-row kernel here only: rows that no other kernel has taken (fh_qmatmul: one launch of 3 rows and more where it pays) are a
+    // launch each (10 us a row against 110 - 640 us for 2 .. 16 rows through the per-element kernel at 14336 x 4096), also with residuals to add
     if (kernel != 1 && kernel != 3 && (q->type == FH_Q5_K || q->type == FH_Q5_0) && q->k % 256 == 0 && m >= 2 && m <= 16) {
         const int64_t nout = epi == FH_EPI_SWIGLU ? q->n / 2 : q->n;
         fh_status st = FH_OK;
@@ -416,8 +416,8 @@ static fh_status qmatmul(const fh_qmatrix *q, const float *x_dev, int32_t m, flo
         const fh_status st = fh_launch_qmv_rows(q, x_dev, m, y_dev);
         if (st != FH_ERR_UNSUPPORTED) return st;
     }
-    // The 5-bit formats have no batch kernel for 2 .. 16 rows: rows are a launch each up to four, the kernel of small prompts takes them
-    // from there, with a power of two per 32 activations as they have it (us, launches / that: 12 rows of 14336 x 4096 in Q5_0 97 / 23, in Q5_K
+    // Rows of the 5-bit formats that the one launch above does not take, and there is no batch kernel for: a launch each up to four; from there on the kernel of
+    // small prompts, with a power of two per 32 activations as the launches have it (us, launches / that: 12 rows of 14336 x 4096 in Q5_0 97 / 23, in Q5_K
     // 100 / 25, of 4096 x 4096 46 / 14 and 46 / 15, of 512 x 2048 40 / 14 and 40 / 16; four rows of the latter two take 16 and 14 as launches).
     // Where it does not (few columns, short prompts of a decoder, no memory for its activations) they stay a launch each up to 12, which
     // needs none; the tiles take them above.

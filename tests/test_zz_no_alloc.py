@@ -38,7 +38,8 @@ def _case(dev, oracle, hq, hkv, L, dtype, seed):
 def test_static_scratch_attention_matches_the_allocating_entry_point(dev, oracle, dtype):
     _case(dev, oracle, 32, 8, 4096, dtype, 1)      # 16 key parts, two query heads per workgroup
     _case(dev, oracle, 8, 2, 300, dtype, 2)        # smaller: fewer heads, 8 parts, most slots of the array untouched
-    _case(dev, oracle, 64, 8, 2049, dtype, 3)      # the most the array holds: 64 heads x 16 parts
+    _case(dev, oracle, 64, 8, 2049, dtype, 3)      # 64 heads, 8 parts
+    _case(dev, oracle, 64, 4, 3500, dtype, 5)      # f32: the most the array holds, 64 heads x 16 parts
     _case(dev, oracle, 4, 4, 1, dtype, 4)          # a single key: parts without keys
 
 

@@ -12,6 +12,7 @@
 // unnormalised output, running max, running sum; k_attn_combine_dl (or the consumer of the partials) merges them.
 #include "fh_internal.h"
 #include <algorithm>
+#include <cstdlib>
 
 typedef _Float16 fh_half;
 
@@ -695,16 +696,35 @@ static int ad_parts(const fh_device *dev, int hq, int hkv, int skv, bool f16) {
 // Room for the partial results of `splits` parts.  When it has to grow it grows to what a cache of any length needs, so that the graphs that hold its address
 // end once and not at every other length; where that much cannot be had, to what this call needs.  It belongs to the device, and calls of other numbers of heads
 // leave it as they need it, so a captured call, which cannot grow it, takes as many parts as it has room for.
-static fh_status ad_room(fh_device *dev, int hq, int hkv, int *splits) {
+static fh_status ad_room(fh_device *dev, int hq, int *splits) {
     const size_t part = (size_t)hq * (128 + 4) * 4;
-    if (hkv < 1 || dev->part_cap >= part * *splits) return FH_OK;
+    if (dev->part_cap >= part * *splits) return FH_OK;
     if (dev->capturing) {
         if (dev->part_cap >= part && dev->opt_attn_splits == 0) *splits = (int)(dev->part_cap / part);
-    } else {
-        const int most = std::max(*splits, std::min(128, std::max(16, 2 * dev->compute_units / hkv)));
-        if (fh_dev_scratch_try(dev, (void **)&dev->part_buf, &dev->part_cap, part * most)) return FH_OK;
-    }
+    } else if (fh_dev_scratch_try(dev, (void **)&dev->part_buf, &dev->part_cap, part * 128)) return FH_OK; // (128 parts at most, of either kernel)
     return fh_dev_scratch(dev, (void **)&dev->part_buf, &dev->part_cap, part * *splits);
+}
+
+// Parts of the keys for the matrix cores: a workgroup of four wavefronts each, chunks of 32 keys in turn.  us of a call:
+// - One a compute unit; two where a wavefront would have more than three chunks.  32 / 8 heads, eight chunks a part / one workgroup a compute unit / two: 4096 keys 9.8 / 9.0 /
+//   9.0, 6000 11.7 / 10.4 / 12.2, 8192 11.7 / 11.6 / 11.8, 12000 16.5 / 13.1 / 13.8 (368 workgroups are two rounds on some compute units), 16384 16.9 / 17.9 / 16.9, 30000
+//   27.9 / 24.1 / 24.4; 16 heads of their own, 5000 keys 15.7 / 11.4 / 11.8.  (The vector-ALU kernels: 22.0 at 16384.)
+// - KV heads that do not share the compute units out evenly: never two, whose last round is nearly empty, and a power of two, which the eight dies share: 24 / 12 heads, 21 or 42
+//   parts / 16: 4096 keys 11.6 / 10.1, 16384 25.3 / 23.9, 131072 138 / 129; 12 / 3 heads, 85 / 64: 8192 keys 10.7 / 9.0; 48 / 6, 42 / 32: 20000 keys 17.8 / 16.6; 36 / 9, 28 or 56 / 16: 8192 keys
+//   15.3 / 13.9, but 65536 60.4 / 64.3: of 9 and 10 up to 8192 keys.  (Below 16 parts this leaves too few workgroups.)
+// - Sixteen KV heads and more, or eight of 32768 keys and more, 1 MB or a multiple of 2 MB apart: they read the same memory channels at a time, the more so the fewer
+//   parts there are.  A part has two chunks a wavefront.  32 heads of their own, by the rules above / so: 16384 keys 60.2 / 52.8, 32768 103 / 93.2; 64 heads, 8192 keys 58.4 / 51.7;
+//   16 heads, 20000 keys of 32768 41.4 / 36.2; 8 heads, 65536 keys 53.8 / 51.5.  (Heads 20480 rows apart 59.4 / 60; 8 heads, 32768 keys of 32832 29.0 / 30.3.)
+// At most 128 parts for the merge.
+static int ad_mfma_parts(const fh_device *dev, int hkv, int nct, int64_t apart) {
+    const int cus = dev->compute_units, one = std::max(1, cus / hkv);
+    const int64_t mb = 1 << 20, near = 64 << 10;
+    const bool level = std::abs(apart - mb) < near || ((apart + near) & (2 * mb - 1)) < 2 * near;
+    if (level && (cus % hkv == 0 || hkv >= 28) && (hkv >= 16 || (hkv == 8 && nct >= 1024 && apart % mb == 0))) return std::max(16, (nct / 8 + 8) / 16 * 16);
+    if (one < 16 || one * hkv == cus || (one >= 24 && one < 32 && nct > 256)) return nct > 12 * one ? std::max(1, 2 * cus / hkv) : one;
+    int parts = 16;
+    while (parts * 2 <= one) parts *= 2;
+    return parts;
 }
 
 // One f32 query per head against `skv` cached keys known on the host; `out` is f32 or f16 [hq, d].  The key
@@ -716,17 +736,11 @@ fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *
     const int mfma_min = dev->opt_attn_kernel == 5 ? 32 : 4096;
     if (kv_dtype == FH_F16 && d == 128 && hq % hkv == 0 && hq / hkv <= 16 && skv >= mfma_min &&
         (dev->opt_attn_kernel == 0 || dev->opt_attn_kernel == 5) && dev->opt_attn_heads == 0 && kv_st % 8 == 0 && kv_sh % 8 == 0) {
-        // parts: a workgroup of four wavefronts each, one a compute unit; two a compute unit where a wavefront would have more than three chunks of 32 keys.
-        // us of a call of 32 / 8 heads, eight chunks a part / one workgroup a compute unit / two: 4096 keys 9.8 / 9.0 / 9.0, 6000 11.7 / 10.4 / 12.2, 8192 11.7 / 11.6 /
-        // 11.8, 12000 16.5 / 13.1 / 13.8 (368 workgroups are two rounds on some compute units), 16384 16.9 / 17.9 / 16.9, 30000 27.9 / 24.1 / 24.4; 16 heads of
-        // their own, 5000 keys 15.7 / 11.4 / 11.8, 32 heads, 8192 26.5 / 26.4 / 25.9.  (The vector-ALU kernels: 22.0 at 16384.)  At most 128 parts for the merge.
         const int nct = (skv + 31) / 32;
-        int splits = std::max(1, dev->compute_units / hkv);
-        if (nct > 12 * splits) splits = std::max(1, 2 * dev->compute_units / hkv);
-        splits = std::min(splits, nct / 2);
+        int splits = std::min(ad_mfma_parts(dev, hkv, nct, kv_sh * 2), nct / 2);
         if (dev->opt_attn_splits > 0) splits = (int)dev->opt_attn_splits;
         splits = splits < 1 ? 1 : (splits > 128 ? 128 : splits);
-        FH_TRY(ad_room(dev, hq, hkv, &splits));
+        FH_TRY(ad_room(dev, hq, &splits));
         fh_status st = fh_attention_decode_mfma(dev, q, q_f16, k, v, kv_sh, kv_st, hq, hkv, d, scale, skv, splits, dev->part_buf);
         if (st != FH_ERR_UNSUPPORTED) {
             if (st != FH_OK) return st;
@@ -737,7 +751,7 @@ fh_status fh_attention_decode_hostlen(fh_device *dev, int kv_dtype, const void *
     const bool f16 = kv_dtype == FH_F16;
     int splits = ad_parts(dev, hq, hkv, skv, f16);
     const int heads = ad_heads(dev, hq, skv, f16);
-    if (d == 128 && hq >= hkv && kv_st % 8 == 0 && kv_sh % 8 == 0) FH_TRY(ad_room(dev, hq, hkv, &splits)); // (what ad_any takes)
+    if (d == 128 && hq >= hkv && kv_st % 8 == 0 && kv_sh % 8 == 0) FH_TRY(ad_room(dev, hq, &splits)); // (what ad_any takes)
     return ad_any(dev, kv_dtype, (const float *)q, k, v, kv_sh, kv_st, hq, hkv, d, scale, nullptr, skv, (float *)out, nullptr,
                   skv - 1, splits, out_f16, heads, skv > 2048 ? 8 : 0, q_f16);
 }

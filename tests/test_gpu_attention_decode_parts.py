@@ -144,3 +144,38 @@ def test_heads_and_parts_without_matrix_cores(dev, oracle, dtype, hq, hkv, L, pa
     # f32 sums of the weighted values, a lane's chain of a few hundred; of f16 the outputs are rounded
     bound = 2.0 ** -17 * np.abs(a[2]).max() + (2.0 ** -11 * np.abs(want) if dtype == "f16" else 0)
     assert (np.abs(auto.astype(np.float32) - want) <= bound).all()
+
+
+@pytest.mark.parametrize("hq,hkv,L,parts", [
+    (16, 16, 8192, 32),    # heads 2 MB apart: two chunks a wavefront
+    (16, 16, 8100, 32),    # nearly (the number in sixteens)
+    (16, 16, 7600, 32),    # not: two workgroups a compute unit
+    (48, 48, 4096, 16),    # 1 MB
+    (48, 48, 4400, 10),    # a little more
+    (8, 8, 32768, 128),    # eight heads, from so many keys on
+    (8, 8, 16384, 64),
+    (40, 40, 8192, 32),
+    (24, 12, 4096, 16),    # KV heads that do not share the compute units out
+    (24, 12, 8200, 16),
+    (10, 10, 8192, 16),
+    (10, 10, 8224, 25),
+    (8, 8, 32832, 64),
+    (12, 3, 8224, 64),
+])
+def test_parts_on_the_matrix_cores(dev, oracle, hq, hkv, L, parts):
+    rng = np.random.default_rng(L)
+    a = [rng.standard_normal((1, h, n, 128), dtype=np.float32).astype(np.float16) for h, n in ((hq, 1), (hkv, L), (hkv, L))]
+    q, k, v = (Tensor.from_slice(dev, t, "f16") for t in a)
+    auto = q.flash_attention(k, v, 0.1).as_slice()
+    same = []
+    for forced in (parts, parts - 3):  # another number of parts rounds the sums elsewhere
+        dev.set_option("attn_splits", forced)
+        try:
+            same.append(np.array_equal(q.flash_attention(k, v, 0.1).as_slice(), auto))
+        finally:
+            dev.set_option("attn_splits", 0)
+    assert same == [True, False]
+    a = [t.astype(np.float32) for t in a]
+    want = oracle.flash_attention(*a, 0.1)
+    # (weights and outputs are rounded to f16, as above)
+    assert (np.abs(auto.astype(np.float32) - want) <= 2.0 ** -11 * (np.abs(a[2]).max() + np.abs(want)) + 1e-6).all()

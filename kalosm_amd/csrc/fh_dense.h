@@ -89,7 +89,11 @@ __device__ __forceinline__ void fh_lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
-// 16 bytes that are read once
+// 16 bytes that are read once.  Decoders take the hint whatever their size: where the last cache keeps the weights, the launch that reads most of them can be slower with it,
+// but what lies in the second cache for the launches around it stays there.  us a step, plainly / with the hint, output launches and the rest: 512 wide, eight experts of
+// 2048 (201 MB) 59.6 + 65.1 / 67.2 + 66.2; 512 wide, an always-on one of 8192 (100 MB) 54.6 + 58.4 / 58.6 + 54.6; 1024 wide, the same (201 MB) 61.4 + 68.3 / 64.3 + 66.2;
+// 1024 wide, four experts and an always-on one of 512 29.7 + 54.3 / 30.3 + 51.5; 2048 wide, eight of 2048 (805 MB) 91.0 + 141.3 / 86.8 + 135.4.  ms of 33 + 64 tokens: Fidasun
+// 1024 wide (169 MB) 8.96 / 8.71, 1536 wide (363 MB) 11.03 / 10.87, Zovovik 1024 wide (137 MB) 8.77 / 8.90, 1536 wide (245 MB) 10.06 / 10.51, 2048 wide (295 MB) 10.30 / 10.30.
 __device__ __forceinline__ uint4 fh_load_once(const uint16_t *p) {
     typedef uint32_t words __attribute__((ext_vector_type(4)));
     const words v = __builtin_nontemporal_load((const words *)p);

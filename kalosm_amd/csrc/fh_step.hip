@@ -276,7 +276,9 @@ fh_status fh_step_middle(fh_device *dev, int dtype, const FhStep &st, fh_kvcache
 // reason).  The inputs and the experts' numbers are requested first, so that they do not wait behind weights, then the first pieces of the output
 // projection, whose places are known.  us of the launch in a step of width 2048, seven experts of 1024: behind latent attention (38 MB, a plain read 7.2) 12.6 /
 // 11.5, a delta rule 15.7 / 13.0, a state space (46 MB, 8.4) 20.1 / 14.2 (one row a wavefront with 8 KB on their way / now; with a table of the
-// pieces in the LDS, a round trip for every piece, 14.4 / 16.4 / 16.5).
+// pieces in the LDS, a round trip for every piece, 14.4 / 16.4 / 16.5).  Narrow streams gain nothing here, long rows of few wavefronts lose (512 wide, eight experts of 2048
+// 14.9 / 16.9, of which the hint of fh_load_once is all; 1024 wide 17.6 / 17.9): 8 KB on the way 16.9, the experts' numbers in a register instead of the LDS 17.1, the next
+// piece's inputs asked for ahead 17.2.
 // NO, NE, NS: fours of values of the mixer, of the experts and of the always-on one that a thread holds in registers, requested ahead of the weights;
 // NO = 0: mixers whose length or groups are no multiple of 4, and longer inputs, are read as they are staged.  PRE: the output projection has four pieces or more.
 template <int NO, int NE, int NS, bool PRE>
